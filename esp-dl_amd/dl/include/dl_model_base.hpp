@@ -60,7 +60,8 @@ public:
     /// Enqueue only; pair with synchronize().  Uses the captured HIP graph when enable_graph() succeeded.
     void run_async(runtime_mode_t mode = RUNTIME_MODE_SINGLE_CORE);
     void synchronize();
-    /// Capture the plan into a HIP graph (after one eager run has created every module's device state).
+    /// Capture the plan into a HIP graph (after one eager run has created every module's device state).  A short
+    /// chain of kernels that the host keeps ahead of is replayed as plain launches, anything else as the graph.
     bool enable_graph();
     void disable_graph();
     bool graph_enabled() const { return m_graph_exec != nullptr; }
@@ -97,6 +98,7 @@ private:
     void fuse_dw_project();
     void fuse_conv_add();
     void fuse_conv_gap();
+    size_t plan_bytes();
 
     fbs::FbsModel *m_fbs_model = nullptr;
     std::vector<dl::module::Module *> m_execution_plan;
@@ -110,6 +112,7 @@ private:
     bool m_own_stream = false;
     void *m_graph = nullptr;      // hipGraph_t
     void *m_graph_exec = nullptr; // hipGraphExec_t
+    void *m_launches = nullptr;   // the captured kernels of a short plan, replayed without the graph
     bool m_built = false;
     bool m_failed = false;
     long m_errors_at_start = 0;

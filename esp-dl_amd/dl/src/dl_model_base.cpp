@@ -36,6 +36,61 @@ dtype_t dtype_of(quant_type_t q)
     }
 }
 
+// Which captured plans are replayed as plain kernel launches instead of as a HIP graph.  A graph replay costs the
+// stream about 8 us in which no kernel runs and the host 15 to 20 us, whatever the number of nodes (one 3x3
+// convolution at batch 1: 14.9 us per graph replay, 6.1 us per launch).  A plain launch costs the host 3 to 4 us and,
+// with its own release of the caches, the stream a few tenths of a microsecond more than a graph node does.  So a plan
+// of up to kDirectAlways launches is always replayed plainly, and one of up to kDirectLaunches when its modules
+// move kDirectBytes or more on average: such kernels take long enough for the host to stay ahead of the stream
+// (MobileNetV2 at batch 256, 19 launches of 33 us: 651 against 646 us; the attention block over 7 x 7 maps, 15 launches
+// of 3.6 us: 62 us as a graph, 63 us launched one by one; MobileNetV2 on one image: 348 against 354 us).
+constexpr size_t kDirectAlways = 4;
+constexpr size_t kDirectLaunches = 24;
+constexpr size_t kDirectBytes = 1 << 20;
+
+// The kernel launches of a captured plan in stream order.  The parameter blocks belong to the graph.
+struct LaunchList {
+    std::vector<hipKernelNodeParams> launches;
+};
+
+// Launch list of a graph that is one chain of kernel nodes; null for any other graph.
+LaunchList *chain_of_kernels(hipGraph_t graph)
+{
+    size_t n_nodes = 0, n_edges = 0;
+    if (hipGraphGetNodes(graph, nullptr, &n_nodes) != hipSuccess || n_nodes == 0 || n_nodes > kDirectLaunches ||
+        hipGraphGetEdges(graph, nullptr, nullptr, &n_edges) != hipSuccess || n_edges != n_nodes - 1)
+        return nullptr;
+    std::vector<hipGraphNode_t> nodes(n_nodes), from(n_edges + 1), to(n_edges + 1);
+    if (hipGraphGetNodes(graph, nodes.data(), &n_nodes) != hipSuccess ||
+        (n_edges != 0 && hipGraphGetEdges(graph, from.data(), to.data(), &n_edges) != hipSuccess))
+        return nullptr;
+    std::map<hipGraphNode_t, hipGraphNode_t> next;
+    std::set<hipGraphNode_t> heads(nodes.begin(), nodes.end());
+    for (size_t i = 0; i < n_edges; i++) {
+        if (!next.emplace(from[i], to[i]).second) // two successors: not a chain
+            return nullptr;
+        heads.erase(to[i]);
+    }
+    if (heads.size() != 1)
+        return nullptr;
+    LaunchList list;
+    hipGraphNode_t node = *heads.begin();
+    for (size_t i = 0; i < n_nodes; i++) {
+        hipGraphNodeType type;
+        hipKernelNodeParams params;
+        if (hipGraphNodeGetType(node, &type) != hipSuccess || type != hipGraphNodeTypeKernel ||
+            hipGraphKernelNodeGetParams(node, &params) != hipSuccess || params.kernelParams == nullptr)
+            return nullptr;
+        list.launches.push_back(params);
+        const auto it = next.find(node);
+        if ((it == next.end()) != (i + 1 == n_nodes))
+            return nullptr;
+        if (it != next.end())
+            node = it->second;
+    }
+    return new LaunchList(list);
+}
+
 // One block of the activation arena.
 struct Block {
     size_t offset, bytes;
@@ -978,6 +1033,16 @@ void Model::run_async(runtime_mode_t mode)
         m_failed = true;
         return;
     }
+    if (m_launches) {
+        for (const hipKernelNodeParams &p : static_cast<LaunchList *>(m_launches)->launches)
+            if (!hip_ok(hipLaunchKernel(p.func, p.gridDim, p.blockDim, p.kernelParams, p.sharedMemBytes,
+                                        static_cast<hipStream_t>(m_stream)),
+                        "hipLaunchKernel")) {
+                m_failed = true;
+                return;
+            }
+        return;
+    }
     if (m_graph_exec) {
         (void)hip_ok(hipGraphLaunch(static_cast<hipGraphExec_t>(m_graph_exec), static_cast<hipStream_t>(m_stream)),
                      "hipGraphLaunch");
@@ -1086,11 +1151,32 @@ bool Model::enable_graph()
     }
     m_graph = graph;
     m_graph_exec = exec;
+    LaunchList *list = chain_of_kernels(graph);
+    (void)hipGetLastError(); // a refused query must not surface as the error of a later launch
+    if (list != nullptr && list->launches.size() > kDirectAlways && plan_bytes() < kDirectBytes * list->launches.size()) {
+        delete list;
+        list = nullptr;
+    }
+    m_launches = list;
     return true;
+}
+
+// Bytes of the tensors the modules of the plan read and write.
+size_t Model::plan_bytes()
+{
+    size_t bytes = 0;
+    for (auto *module : m_execution_plan)
+        for (const auto *ids : {&module->m_inputs_index, &module->m_outputs_index})
+            for (int idx : *ids)
+                if (TensorBase *t = m_model_context->get_tensor(idx))
+                    bytes += t->get_bytes();
+    return bytes;
 }
 
 void Model::disable_graph()
 {
+    delete static_cast<LaunchList *>(m_launches);
+    m_launches = nullptr;
     if (m_graph_exec) {
         (void)hipStreamSynchronize(static_cast<hipStream_t>(m_stream));
         (void)hipGraphExecDestroy(static_cast<hipGraphExec_t>(m_graph_exec));
