@@ -41,15 +41,7 @@ hipError_t launch_conv2d_s8_mfma(const ConvGeom &g, const int8_t *in, const int8
         bmode = B_POINT;
     else if ((g.in_c & 15) == 0 && (g.in_pitch & 15) == 0 && aligned16)
         bmode = B_VEC16;
-    else if (g.dil_w == 1 && g.in_pitch == g.in_c) // a filter row's bytes are contiguous in a dense input only
-        bmode = B_ROWSEG;
-    a.seg_len = a.seg_pad = 0;
     a.K = g.k_h * g.k_w * g.in_c;
-    if (bmode == B_ROWSEG) {
-        a.seg_len = g.k_w * g.in_c;
-        a.seg_pad = (a.seg_len + 15) & ~15;
-        a.K = g.k_h * a.seg_pad;
-    }
     a.ksteps = (a.K + 63) / 64;
     a.n_groups = (g.out_c + 63) / 64;
     const uintptr_t out_addr = reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(residual);
@@ -101,7 +93,6 @@ hipError_t launch_conv2d_s8_mfma(const ConvGeom &g, const int8_t *in, const int8
     a.fd_out_w = make_fastdiv((unsigned)g.out_w);
     a.fd_in_c = make_fastdiv((unsigned)g.in_c);
     a.fd_k_w = make_fastdiv((unsigned)g.k_w);
-    a.fd_seg_pad = make_fastdiv((unsigned)(a.seg_pad > 0 ? a.seg_pad : 1));
 
     // persistent grid: sized by launch_variant from the residency of the chosen kernel variant
     const GridPlan grid{cus, n_chunks};
@@ -111,8 +102,6 @@ hipError_t launch_conv2d_s8_mfma(const ConvGeom &g, const int8_t *in, const int8
         return launch_vec16(a, pt, ksc, grid, lds, stream);
     case B_POINT:
         return launch_point(a, pt, ksc, grid, lds, stream);
-    case B_ROWSEG:
-        return launch_rowseg(a, pt, ksc, grid, lds, stream);
     default:
         return launch_gather(a, pt, ksc, grid, lds, stream);
     }

@@ -22,11 +22,8 @@
 //             aligned 16-byte load, or zeros when the tap falls into the padding;
 //   B_POINT   1x1 filter without padding: k is the channel index; one (possibly unaligned) 16-byte
 //             load that may run past in_c into the next pixel (those positions meet zero weights);
-//   B_ROWSEG  dilation_w == 1: the k_w * in_c bytes of one filter row are contiguous in the input, so
-//             the reduction axis is re-ordered as (ky, j) with every row segment padded to a
-//             multiple of 16; a lane's chunk is one unaligned 16-byte load, masked at the left and
-//             right image borders (the 3-channel stem convolutions run this way);
-//   B_GATHER  anything else: byte gather.
+//   B_GATHER  anything else: byte gather (the dispatcher sends such layers to conv2d_s8_pwgemm.hip and
+//             conv2d_s8_narrow.hip; this form is left for tensors of fewer than 16 bytes or images over 2 GiB).
 // Epilogue.  When every shift of the workgroup's filters lies in 1..31, rounding is half-up and
 // |bias + 2^(s-1)| + K * 2^14 cannot overflow, the accumulator starts at bias + 2^(s-1) and a value
 // costs about three VALU instructions: t = (acc << max(0, 8-s)) >> max(0, s-8) carries the result in
@@ -47,7 +44,7 @@
 namespace espdl {
 namespace mfma_conv {
 
-enum { B_VEC16 = 0, B_POINT = 1, B_GATHER = 2, B_ROWSEG = 3 };
+enum { B_VEC16 = 0, B_POINT = 1, B_GATHER = 2 };
 
 constexpr int kThreads = 256; // 4 wavefronts
 
@@ -60,9 +57,7 @@ struct MfmaConvArgs {
     const int8_t *res; // tensor of the output's shape added with saturation to the stored value, or nullptr
     int8_t *out;
     ConvGeom g;
-    int K;                // length of the reduction axis as the MFMA sees it (k_h * seg_pad for B_ROWSEG)
-    int seg_len;          // B_ROWSEG: k_w * in_c, bytes of one filter row
-    int seg_pad;          // B_ROWSEG: seg_len rounded up to a multiple of 16
+    int K;                // length of the reduction axis
     int ksteps;           // ceil(K / 64)
     int ks_per_chunk;     // k steps resident in LDS at a time (== ksteps when everything fits)
     int n_kchunks;        // ceil(ksteps / ks_per_chunk)
@@ -72,7 +67,7 @@ struct MfmaConvArgs {
     long long npix;       // batch * out_h * out_w
     long long in_bytes;   // size of the input tensor
     int out_vec;          // widest store the output allows: 16, 4 or 1 bytes
-    FastDiv fd_out_hw, fd_out_w, fd_in_c, fd_k_w, fd_seg_pad; // launch-invariant divisors
+    FastDiv fd_out_hw, fd_out_w, fd_in_c, fd_k_w; // launch-invariant divisors
     int stage_out;        // 1: a wave collects its 16*PT x out_c outputs in LDS and writes them as one
                           //    contiguous block (needs every filter group resident, i.e. one chunk)
 };
@@ -95,16 +90,6 @@ __device__ __forceinline__ v4i weight_unit(const MfmaConvArgs &a, int gbase, int
     const int oc = gbase + 4 * nt * (i >> 2) + 4 * t + (i & 3);
     if (oc >= OC || k >= K)
         return val;
-    if (a.seg_pad > 0) {
-        // (ky, j) ordering: filter row ky starts at k = ky * seg_pad and holds seg_len bytes
-        const int ky = k / a.seg_pad, j0 = k - ky * a.seg_pad;
-        const int8_t *src = a.w + ((size_t)oc * a.g.k_h + ky) * a.seg_len + j0;
-        unsigned int words[4] = {0, 0, 0, 0};
-        const int n = min(16, a.seg_len - j0);
-        for (int b = 0; b < n; b++)
-            words[b >> 2] |= (unsigned int)(unsigned char)src[b] << ((b & 3) * 8);
-        return v4i{(int)words[0], (int)words[1], (int)words[2], (int)words[3]};
-    }
     const int8_t *src = a.w + (size_t)oc * K + k;
     if ((K & 15) == 0 && (reinterpret_cast<uintptr_t>(a.w) & 15) == 0)
         return *reinterpret_cast<const v4i *>(src);
@@ -178,37 +163,6 @@ __device__ __forceinline__ v4i load_b(const MfmaConvArgs &a, bool valid, long lo
         const int iy = iy0 + ky * g.dil_h, ix = ix0 + kx * g.dil_w;
         if ((unsigned)iy < (unsigned)g.in_h && (unsigned)ix < (unsigned)g.in_w)
             r = *reinterpret_cast<const v4i *>(a.in + img_off + ((long long)iy * g.in_w + ix) * g.in_pitch + c0);
-        return r;
-    }
-    if (BMODE == B_ROWSEG) {
-        const int ky = (int)fastdiv((unsigned)k, a.fd_seg_pad), j0 = k - ky * a.seg_pad;
-        const int iy = iy0 + ky * g.dil_h;
-        if ((unsigned)iy >= (unsigned)g.in_h)
-            return r;
-        // valid bytes of this chunk: those whose input column lies inside the image
-        const int row_lo = -ix0 * g.in_c, row_hi = (g.in_w - ix0) * g.in_c; // j range inside the image
-        const int nlo = min(max(row_lo - j0, 0), 16), nhi = min(max(row_hi - j0, 0), 16);
-        if (nlo >= nhi)
-            return r;
-        const long long off = img_off + ((long long)iy * g.in_w + ix0) * g.in_c + j0;
-        if (off >= 0 && off + 16 <= a.in_bytes) {
-            __builtin_memcpy(&r, a.in + off, 16);
-            if (nlo > 0 || nhi < 16) {
-#pragma unroll
-                for (int w = 0; w < 4; w++) {
-                    const int hi_n = min(max(nhi - 4 * w, 0), 4), lo_n = min(max(nlo - 4 * w, 0), 4);
-                    const unsigned hi_m = hi_n >= 4 ? 0xffffffffu : ((1u << (8 * hi_n)) - 1u);
-                    const unsigned lo_m = lo_n >= 4 ? 0xffffffffu : ((1u << (8 * lo_n)) - 1u);
-                    r[w] = (int)((unsigned)r[w] & hi_m & ~lo_m);
-                }
-            }
-        } else {
-            unsigned int words[4] = {0, 0, 0, 0};
-            const int stop = min(nhi, a.seg_len - j0);
-            for (int b = nlo; b < stop; b++)
-                words[b >> 2] |= (unsigned int)(unsigned char)a.in[off + b] << ((b & 3) * 8);
-            r = v4i{(int)words[0], (int)words[1], (int)words[2], (int)words[3]};
-        }
         return r;
     }
     // B_GATHER
@@ -727,7 +681,6 @@ hipError_t launch_ksc(const MfmaConvArgs &a, int ksc, GridPlan grid, size_t lds,
 // Per operand-B mode entry points, each compiled in its own translation unit.
 hipError_t launch_vec16(const MfmaConvArgs &a, int pt, int ksc, GridPlan grid, size_t lds, hipStream_t stream);
 hipError_t launch_point(const MfmaConvArgs &a, int pt, int ksc, GridPlan grid, size_t lds, hipStream_t stream);
-hipError_t launch_rowseg(const MfmaConvArgs &a, int pt, int ksc, GridPlan grid, size_t lds, hipStream_t stream);
 hipError_t launch_gather(const MfmaConvArgs &a, int pt, int ksc, GridPlan grid, size_t lds, hipStream_t stream);
 
 } // namespace mfma_conv

@@ -20,12 +20,13 @@
 // leaves every lane with 16 consecutive output channels per pixel: one 16-byte store.
 #include <type_traits>
 
-#include "espdl_device.h"
-#include "espdl_kernels.h"
+#include "conv_window.h"
 
 namespace espdl {
 
 namespace {
+
+using namespace window;
 
 constexpr int kThreads = 256;
 // LDS row of a tile: 64 k bytes + padding.  96 where LDS capacity allows it (conflict-free operand reads, see the
@@ -47,10 +48,9 @@ struct PwArgs {
     int ksteps;
     int relu, half_even, n_shift;
     int out_vec; // 16, 4 or 1
-    // WIN builds: a convolution with a window as the same product over gathered rows (im2col on the fly): row m is
-    // output pixel m, its k bytes [tap][channel] come from the input pixels under the window (zeros outside the image)
-    int w_in_h, w_in_w, w_in_c, w_k_w, w_stride_h, w_stride_w, w_dil_h, w_dil_w, w_pad_top, w_pad_left;
-    FastDiv fd_ohw, fd_ow, fd_inc, fd_kw;
+    // UNITS builds: a convolution with a window as the same product over gathered rows (im2col on the fly): row m is
+    // output pixel m, its k bytes are the units of conv_window.h (zeros outside the image)
+    WindowArgs win;
     int hw;          // GAP builds: pixels per image (at most 64)
     float gap_scale; // GAP builds: 2^in_exp / (h w) * 2^-out_exp of the pooling operator
 };
@@ -61,12 +61,12 @@ struct PwArgs {
 // results (requantized, activation applied, exactly what the separate operator would have stored) are summed
 // over the image's pixels - over the 16 lanes of a pixel tile by rotations inside the row, over the four
 // wavefronts through LDS - and the sum goes through the pooling operator's float scale and rounding.
-// WIN: rows are gathered from under a convolution window (channels a multiple of 64, so that a k step of 64 lies
-// inside one tap): what conv2d_33cn / conv2d_hwcn compute (esp-dl/dl/base/dl_base_conv2d.cpp:35-163) under
-// conv_operation_shell's window clipping (esp-dl/dl/base/dl_base.hpp:940-1191).  For layers with few output pixels
-// and a long reduction axis (the strided 3 x 3 convolutions deep in a detector's backbone), where a workgroup of
-// the other kernels spends its time staging filters it uses for a handful of pixel sets.
-template <int NG, int PT, bool GAP = false, bool K16 = true, bool WIN = false>
+// UNITS: rows are gathered from under a convolution window, a k step being four 16-channel units of conv_window.h:
+// what conv2d_33cn / conv2d_hwcn compute (esp-dl/dl/base/dl_base_conv2d.cpp:35-163) under conv_operation_shell's
+// window clipping (esp-dl/dl/base/dl_base.hpp:940-1191), for any channel count (K16: whole aligned units).  A unit's
+// tap costs a thread about ten instructions per k step, next to 512 matrix cycles; an earlier form that took its tap
+// from a scalar (channels a multiple of 64) was 2 to 10 % slower for its 64-bit addresses and selects.
+template <int NG, int PT, bool GAP = false, bool K16 = true, bool UNITS = false>
 __global__ __launch_bounds__(kThreads) void conv2d_s8_pwgemm_kernel(const PwArgs a)
 {
     constexpr int TN = 64 * NG;
@@ -127,49 +127,40 @@ __global__ __launch_bounds__(kThreads) void conv2d_s8_pwgemm_kernel(const PwArgs
         }
         return r;
     };
-    // WIN: where the window of this thread's rows starts in the input (row of piece slot j: (tid + j * kThreads) / 4)
-    long long win_base[WIN ? kPiecesB : 1];
-    int win_iy[WIN ? kPiecesB : 1], win_ix[WIN ? kPiecesB : 1];
-    if constexpr (WIN) {
+    // UNITS: the windows of this thread's rows; a thread's pieces of a k step are the same unit (tid % 4) of each
+    [[maybe_unused]] PixelWindow px[UNITS ? kPiecesB : 1];
+    [[maybe_unused]] __amdgpu_buffer_rsrc_t in_rsrc = tensor_rsrc(a.in, a.win.in_bytes);
+    [[maybe_unused]] __amdgpu_buffer_rsrc_t w_rsrc = tensor_rsrc(a.w, a.win.w_bytes);
+    if constexpr (UNITS) {
 #pragma unroll
-        for (int j = 0; j < kPiecesB; j++) {
-            const long long m = row_pixel((tid + j * kThreads) >> 2);
-            win_iy[j] = -0x40000000; // a row past the last: every tap is outside
-            win_ix[j] = 0;
-            win_base[j] = 0;
-            if (m >= 0) {
-                const unsigned n = fastdiv((unsigned)m, a.fd_ohw);
-                const unsigned rem = (unsigned)m - n * a.fd_ohw.d;
-                const unsigned oy = fastdiv(rem, a.fd_ow);
-                const unsigned ox = rem - oy * a.fd_ow.d;
-                win_iy[j] = (int)oy * a.w_stride_h - a.w_pad_top;
-                win_ix[j] = (int)ox * a.w_stride_w - a.w_pad_left;
-                win_base[j] = (((long long)n * a.w_in_h + win_iy[j]) * a.w_in_w + win_ix[j]) * a.in_pitch;
-            }
-        }
+        for (int j = 0; j < kPiecesB; j++)
+            px[j] = pixel_window(a.win, (int)m0 + ((tid + j * kThreads) >> 2), (int)a.M);
     }
+    // (UNITS) channels the thread's unit of k step ks holds
+    auto unit_channels = [&](int ks) {
+        const int u = 4 * ks + (tid & 3);
+        return a.win.in_c - 16 * (u - (int)(fastdiv((unsigned)u, a.win.fd_upt) * a.win.fd_upt.d));
+    };
     auto fetch = [&](int ks, v4i(&pb)[kPiecesB], v4i(&pa)[kPiecesA]) {
         const int k0 = 64 * ks;
-        if constexpr (WIN) {
-            // the tap and first channel of this k step (uniform)
-            const unsigned tap = fastdiv((unsigned)k0, a.fd_inc);
-            const int c0 = k0 - (int)tap * a.w_in_c;
-            const unsigned ky = fastdiv(tap, a.fd_kw);
-            const int dy = (int)ky * a.w_dil_h, dx = (int)(tap - ky * a.fd_kw.d) * a.w_dil_w;
-            const long long tap_off = ((long long)dy * a.w_in_w + dx) * a.in_pitch + c0;
+        if constexpr (UNITS) {
+            const Unit u = locate_unit(a.win, 4 * ks + (tid & 3));
 #pragma unroll
-            for (int j = 0; j < kPiecesB; j++) {
-                const int p = tid + j * kThreads;
-                const bool ok = (unsigned)(win_iy[j] + dy) < (unsigned)a.w_in_h && (unsigned)(win_ix[j] + dx) < (unsigned)a.w_in_w;
-                pb[j] = ok ? *reinterpret_cast<const v4i *>(a.in + win_base[j] + tap_off + 16 * (p & 3)) : v4i{0, 0, 0, 0};
-            }
-        } else {
+            for (int j = 0; j < kPiecesB; j++)
+                pb[j] = load_pixel_unit<K16>(a.win, in_rsrc, px[j], u);
 #pragma unroll
-            for (int j = 0; j < kPiecesB; j++) {
-                const int p = tid + j * kThreads;
-                const long long m = row_pixel(p >> 2);
-                pb[j] = m >= 0 ? piece(a.in + m * a.in_pitch, k0 + 16 * (p & 3)) : v4i{0, 0, 0, 0};
+            for (int j = 0; j < kPiecesA; j++) {
+                // (a filter past the last one reads the last one again: its results are not stored)
+                const int n = min(n0 + ((tid + j * kThreads) >> 2), a.N - 1);
+                pa[j] = load_filter_unit<K16>(a.win, w_rsrc, n * a.win.w_len, u);
             }
+            return;
+        }
+#pragma unroll
+        for (int j = 0; j < kPiecesB; j++) {
+            const int p = tid + j * kThreads;
+            const long long m = row_pixel(p >> 2);
+            pb[j] = m >= 0 ? piece(a.in + m * a.in_pitch, k0 + 16 * (p & 3)) : v4i{0, 0, 0, 0};
         }
 #pragma unroll
         for (int j = 0; j < kPiecesA; j++) {
@@ -178,7 +169,7 @@ __global__ __launch_bounds__(kThreads) void conv2d_s8_pwgemm_kernel(const PwArgs
             pa[j] = n < a.N ? piece(a.w + (long long)n * a.K, k0 + 16 * (p & 3)) : v4i{0, 0, 0, 0};
         }
     };
-    auto stash = [&](int buf, const v4i(&pb)[kPiecesB], const v4i(&pa)[kPiecesA]) {
+    auto stash = [&](int buf, [[maybe_unused]] int ks, const v4i(&pb)[kPiecesB], const v4i(&pa)[kPiecesA]) {
 #pragma unroll
         for (int j = 0; j < kPiecesB; j++) {
             const int p = tid + j * kThreads;
@@ -187,7 +178,10 @@ __global__ __launch_bounds__(kThreads) void conv2d_s8_pwgemm_kernel(const PwArgs
 #pragma unroll
         for (int j = 0; j < kPiecesA; j++) {
             const int p = tid + j * kThreads;
-            *reinterpret_cast<v4i *>(&a_l[buf][(p >> 2) * kRow + 16 * (p & 3)]) = pa[j];
+            v4i v = pa[j];
+            if constexpr (UNITS && !K16)
+                v = mask_unit<false>(v, unit_channels(ks));
+            *reinterpret_cast<v4i *>(&a_l[buf][(p >> 2) * kRow + 16 * (p & 3)]) = v;
         }
     };
 
@@ -226,7 +220,7 @@ __global__ __launch_bounds__(kThreads) void conv2d_s8_pwgemm_kernel(const PwArgs
         cst[1][tid] = fast ? max(0, my_s - 8) : my_s;
         cst[2][tid] = fast ? max(0, 8 - my_s) : 0;
     }
-    stash(0, pb, pa);
+    stash(0, 0, pb, pa);
     if (a.ksteps > 2)
         fetch(2, pb, pa);
     __syncthreads();
@@ -276,13 +270,13 @@ __global__ __launch_bounds__(kThreads) void conv2d_s8_pwgemm_kernel(const PwArgs
     for (int ks = 0; ks < a.ksteps; ks += 2) {
         products(0);
         if (ks + 1 < a.ksteps) {
-            stash(1, pb2, pa2);
+            stash(1, ks + 1, pb2, pa2);
             if (ks + 3 < a.ksteps)
                 fetch(ks + 3, pb2, pa2);
             __syncthreads();
             products(1);
             if (ks + 2 < a.ksteps) {
-                stash(0, pb, pa);
+                stash(0, ks + 2, pb, pa);
                 if (ks + 4 < a.ksteps)
                     fetch(ks + 4, pb, pa);
                 __syncthreads();
@@ -449,80 +443,6 @@ __global__ __launch_bounds__(kThreads) void conv2d_s8_pwgemm_kernel(const PwArgs
     }
 }
 
-// The same product for a handful of rows (a classifier Gemm over one batch: 256 x 1280 x 1000): the tiled kernel
-// above would run on a few dozen compute units and spend its time in twenty barrier-separated k steps.  Here a
-// wavefront owns a 16-row x 16-filter tile for the whole reduction and reads both operands straight from
-// global memory / L2 in the MFMA operand layout (lane (col, quad): 16 bytes of row col at k = 64 step + 16 quad),
-// G k steps per batch of loads, the next batch in flight under the current one's MFMAs; a workgroup is four row
-// tiles under one filter tile, so N / 16 x M / 64 workgroups fill the device and a workgroup's time is a few memory
-// round trips.  K must be a multiple of 64.  The epilogue is the general one (any shift, either rounding).
-template <int G>
-__global__ __launch_bounds__(kThreads) void conv2d_s8_rows_kernel(const PwArgs a)
-{
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int col = lane & 15, quad = lane >> 4;
-    const long long m0 = ((long long)blockIdx.x * 4 + wave) * 16;
-    const int n0 = blockIdx.y * 16;
-    if (m0 >= a.M) // uniform per wavefront; the kernel has no barrier
-        return;
-    const long long row = min(m0 + col, a.M - 1);
-    const int flt = min(n0 + col, a.N - 1);
-    const v4i *pa = reinterpret_cast<const v4i *>(a.w + (long long)flt * a.K + 16 * quad);
-    const v4i *pb = reinterpret_cast<const v4i *>(a.in + row * a.in_pitch + 16 * quad);
-    v4i ca[G], cb[G], na[G], nb[G];
-#pragma unroll
-    for (int i = 0; i < G; i++) {
-        const int ks = min(i, a.ksteps - 1);
-        ca[i] = pa[4 * ks];
-        cb[i] = pb[4 * ks];
-    }
-    v4i acc = {0, 0, 0, 0};
-    for (int g0 = 0; g0 < a.ksteps; g0 += G) {
-        const bool more = g0 + G < a.ksteps; // uniform
-        if (more) {
-#pragma unroll
-            for (int i = 0; i < G; i++) {
-                const int ks = min(g0 + G + i, a.ksteps - 1);
-                na[i] = pa[4 * ks];
-                nb[i] = pb[4 * ks];
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < G; i++)
-            if (g0 + i < a.ksteps) // uniform
-                acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(ca[i], cb[i], acc, 0, 0, 0);
-        if (more) {
-#pragma unroll
-            for (int i = 0; i < G; i++) {
-                ca[i] = na[i];
-                cb[i] = nb[i];
-            }
-        }
-    }
-    // lane (col, quad) holds filters n0 + 4 quad + [0, 4) of row m0 + col
-    const long long m = m0 + col;
-    const int n = n0 + 4 * quad;
-    const bool relu = a.relu != 0, half_even = a.half_even != 0;
-    int q[4];
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-        const int nn = min(n + r, a.N - 1);
-        const int b = a.bias != nullptr ? a.bias[nn] : 0;
-        q[r] = requant_s8(acc[r] + b, a.shift[a.n_shift == 1 ? 0 : nn], relu, half_even);
-    }
-    if (m >= a.M || n >= a.N)
-        return;
-    int8_t *dst = a.out + m * a.out_pitch + n;
-    if (a.out_vec >= 4 && n + 4 <= a.N) {
-        *reinterpret_cast<int *>(dst) = pack4_s8(q[0], q[1], q[2], q[3]);
-    } else {
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-            if (n + r < a.N)
-                dst[r] = (int8_t)q[r];
-    }
-}
-
 } // namespace
 
 // Flat pointwise geometry; worth it when a workgroup of the implicit-GEMM
@@ -545,20 +465,6 @@ bool conv2d_s8_pwgemm_supports(const ConvGeom &g, const void *in, const void *fi
     if (g.in_c <= 128 && g.out_c >= 2048 && npix >= 64ll * cus)
         return false;
     return npix > 0 && (npix + 63) / 64 < (long long)cus * 16 && (npix + 63) / 64 <= 0x7fffffffll;
-}
-
-// The one-wavefront-per-tile kernel on its own: any filter count (a classifier with a handful of classes), K a
-// multiple of 64, fewer 64 x 64 tiles than compute units.
-bool conv2d_s8_rows_supports(const ConvGeom &g, const void *in, const void *filter, int cu_count)
-{
-    const bool flat = g.k_h == 1 && g.k_w == 1 && g.stride_h == 1 && g.stride_w == 1 && g.pad_top == 0 &&
-        g.pad_left == 0 && g.out_h == g.in_h && g.out_w == g.in_w;
-    if (!flat || (g.in_c & 63) != 0 || g.out_c < 1 || (g.in_pitch & 15) != 0 ||
-        ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(filter)) & 15) != 0)
-        return false;
-    const long long npix = (long long)g.batch * g.out_h * g.out_w;
-    const int cus = cu_count > 0 ? cu_count : 256;
-    return npix > 0 && (npix + 63) / 64 * ((g.out_c + 63) / 64) < cus;
 }
 
 hipError_t launch_conv2d_s8_pwgemm(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,
@@ -595,12 +501,6 @@ hipError_t launch_conv2d_s8_pwgemm(const ConvGeom &g, const int8_t *in, const in
     const unsigned gy = (unsigned)((a.N + 63) / 64);
     const long long tiles128 = (a.M + 127) / 128;
     const int cus = cu_count > 0 ? cu_count : 256;
-    // fewer 64 x 64 tiles than compute units: one wavefront per 16 x 16 tile, operands straight from global memory
-    if (lut == nullptr && residual == nullptr && (a.K & 63) == 0 && (a.in_pitch & 15) == 0 && (a.M + 63) / 64 * gy < cus) {
-        hipLaunchKernelGGL((conv2d_s8_rows_kernel<10>), dim3((unsigned)((a.M + 63) / 64), (unsigned)((a.N + 15) / 16)),
-                           dim3(kThreads), 0, stream, a);
-        return hipGetLastError();
-    }
     const bool k16 = (a.K & 15) == 0 && (a.in_pitch & 15) == 0;
     if (tiles128 * gy * 2 < 3ll * cus) {
         if (k16)
@@ -616,23 +516,31 @@ hipError_t launch_conv2d_s8_pwgemm(const ConvGeom &g, const int8_t *in, const in
     return hipGetLastError();
 }
 
-// A convolution with a window through the same kernel, rows gathered from under the window: channels a multiple of
-// 64, few output pixels per compute unit and a long reduction axis.
-bool conv2d_s8_wingemm_supports(const ConvGeom &g, const void *in, const void *filter, int cu_count)
+// A convolution (window or not) over any channel count through the same kernel, a k step being four 16-channel units.
+bool conv2d_s8_units_support(const ConvGeom &g)
 {
-    if (g.k_h * g.k_w < 2 || (g.in_c & 63) != 0 || (g.in_pitch & 15) != 0 || g.out_c < 64 ||
-        ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(filter)) & 15) != 0)
-        return false;
-    const long long npix = (long long)g.batch * g.out_h * g.out_w;
-    const int cus = cu_count > 0 ? cu_count : 256;
-    // the workgroups of the other kernels stage a filter group for every few pixel sets here: at most sixteen
-    // 64-pixel tiles per compute unit, and a reduction axis of nine k steps or more
-    return npix > 0 && npix < 0x7fffffffll && (npix + 63) / 64 < (long long)cus * 32 && g.k_h * g.k_w * g.in_c >= 576;
+    return window_supports(g);
 }
 
-hipError_t launch_conv2d_s8_wingemm(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,
-                                    const int32_t *shift, const int8_t *lut, const int8_t *residual, int8_t *out,
-                                    int cu_count, hipStream_t stream)
+bool conv2d_s8_units_aligned(const ConvGeom &g, const void *in, const void *filter)
+{
+    return window_aligned(g, in, filter);
+}
+
+// Expected time (see dense_s8_route): launch, reduction steps of a workgroup, tiles in flight over the device.
+float conv2d_s8_unitgemm_us(const ConvGeom &g, const void *in, const void *filter, long long *tile_steps)
+{
+    const long long tiles = (((long long)g.batch * g.out_h * g.out_w + 63) / 64) * ((g.out_c + 63) / 64);
+    const int ksteps = (g.k_h * g.k_w * ((g.in_c + 15) / 16) + 3) / 4;
+    *tile_steps = tiles * ksteps;
+    if (window_aligned(g, in, filter))
+        return 2.9f + 0.26f * (float)ksteps + 0.32e-3f * (float)*tile_steps + 1.47e-3f * (float)tiles;
+    return 3.2f + 0.39f * (float)ksteps + 0.45e-3f * (float)*tile_steps + 1.95e-3f * (float)tiles;
+}
+
+hipError_t launch_conv2d_s8_unitgemm(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,
+                                     const int32_t *shift, const int8_t *lut, const int8_t *residual, int8_t *out,
+                                     int cu_count, hipStream_t stream)
 {
     PwArgs a = {};
     a.in = in;
@@ -648,24 +556,11 @@ hipError_t launch_conv2d_s8_wingemm(const ConvGeom &g, const int8_t *in, const i
     a.in_pitch = g.in_pitch;
     a.out_pitch = g.out_pitch;
     a.res_pitch = g.res_pitch;
-    a.ksteps = a.K / 64;
+    a.win = window_args(g, in, filter);
+    a.ksteps = (a.win.n_units + 3) / 4;
     a.relu = g.relu;
     a.half_even = g.half_even;
     a.n_shift = g.n_shift;
-    a.w_in_h = g.in_h;
-    a.w_in_w = g.in_w;
-    a.w_in_c = g.in_c;
-    a.w_k_w = g.k_w;
-    a.w_stride_h = g.stride_h;
-    a.w_stride_w = g.stride_w;
-    a.w_dil_h = g.dil_h;
-    a.w_dil_w = g.dil_w;
-    a.w_pad_top = g.pad_top;
-    a.w_pad_left = g.pad_left;
-    a.fd_ohw = make_fastdiv((unsigned)(g.out_h * g.out_w));
-    a.fd_ow = make_fastdiv((unsigned)g.out_w);
-    a.fd_inc = make_fastdiv((unsigned)g.in_c);
-    a.fd_kw = make_fastdiv((unsigned)g.k_w);
     const uintptr_t oaddr = reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(residual);
     a.out_vec = ((a.N & 15) == 0 && (oaddr & 15) == 0 && (a.out_pitch & 15) == 0) ? 16
         : (((a.N & 3) == 0 && (oaddr & 3) == 0 && (a.out_pitch & 3) == 0) ? 4 : 1);
@@ -674,10 +569,17 @@ hipError_t launch_conv2d_s8_wingemm(const ConvGeom &g, const int8_t *in, const i
     const unsigned gy = (unsigned)((a.N + 63) / 64);
     const long long tiles128 = (a.M + 127) / 128;
     const int cus = cu_count > 0 ? cu_count : 256;
-    if (tiles128 * gy * 2 < 3ll * cus)
-        hipLaunchKernelGGL((conv2d_s8_pwgemm_kernel<1, 1, false, true, true>), dim3((unsigned)((a.M + 63) / 64), gy), dim3(kThreads), 0, stream, a);
+    const bool k16 = window_aligned(g, in, filter);
+    const bool small = tiles128 * gy * 2 < 3ll * cus;
+    const dim3 grid(small ? (unsigned)((a.M + 63) / 64) : (unsigned)tiles128, gy);
+    if (small && k16)
+        hipLaunchKernelGGL((conv2d_s8_pwgemm_kernel<1, 1, false, true, true>), grid, dim3(kThreads), 0, stream, a);
+    else if (small)
+        hipLaunchKernelGGL((conv2d_s8_pwgemm_kernel<1, 1, false, false, true>), grid, dim3(kThreads), 0, stream, a);
+    else if (k16)
+        hipLaunchKernelGGL((conv2d_s8_pwgemm_kernel<1, 2, false, true, true>), grid, dim3(kThreads), 0, stream, a);
     else
-        hipLaunchKernelGGL((conv2d_s8_pwgemm_kernel<1, 2, false, true, true>), dim3((unsigned)tiles128, gy), dim3(kThreads), 0, stream, a);
+        hipLaunchKernelGGL((conv2d_s8_pwgemm_kernel<1, 2, false, false, true>), grid, dim3(kThreads), 0, stream, a);
     return hipGetLastError();
 }
 

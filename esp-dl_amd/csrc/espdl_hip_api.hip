@@ -124,6 +124,61 @@ bool misaligned(const void *p, uintptr_t a)
     return (reinterpret_cast<uintptr_t>(p) & (a - 1)) != 0;
 }
 
+// Images of a layer that one launch of the unit-reading kernels takes: their offsets into the input are 31-bit.
+int images_per_unit_launch(const espdl::ConvGeom &g)
+{
+    espdl::ConvGeom part = g;
+    while (part.batch > 1 && !espdl::conv2d_s8_units_support(part))
+        part.batch = (part.batch + 1) / 2;
+    return espdl::conv2d_s8_units_support(part) ? part.batch : 0;
+}
+
+enum DenseRoute { DENSE_STEM, DENSE_NARROW, DENSE_UNITGEMM, DENSE_PWGEMM, DENSE_TILED, DENSE_DIRECT };
+
+// Kernel of a dense int8 convolution.  The two kernels that read windows as 16-channel units take any layer; their
+// times, measured over 128 layers of 1 to 600 K output pixels, are straight lines in their work (within 15 %), so the
+// choice between them compares those lines.  Where the other kernels begin:
+//   * window rows of at most 16 bytes (RGB input): the first-layer kernel, which never takes less than 5.2 us;
+//   * 1x1 over flat rows: the pointwise GEMM kernel where it applies (two reads less address arithmetic), the direct
+//     kernel where pixels are many and channels few (its wavefronts keep their pixels in registers and write whole
+//     rows: 640 K pixels and up at 32 channels, 43 against 34 us);
+//   * a window over whole aligned units at stride 1 with many outputs: the tiled kernel, which reads every input byte
+//     once instead of once per tap (80 x 80 x 32 -> 32, 3 x 3, batch 64: 17.0 against 24.7 us; batch 8: 8.2 against 6.5 us,
+//     for it stages its filters in every workgroup).  It computes filter tiles of 16, the unit kernel 64, so the line
+//     moves with the share of the last 64 filters in use;
+//   * strided windows of fewer than five reduction steps with many outputs: the direct kernel (320 x 320 x 16 -> 32 at
+//     stride 2, batch 32: 35.5 against 38.3 us).
+// A channel count that is not a multiple of 16 under a window has no other kernel worth taking: 31 x 101 x 61 -> 16,
+// 5 x 5, batch 142: 509 -> 111 us; 45 x 99 x 162 -> 87, 5 x 5 at stride 2, batch 3: 312 -> 33 us.
+DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *filter, const void *residual, int cus)
+{
+    const bool units = images_per_unit_launch(g) > 0;
+    float narrow = 0.f, gemm = 0.f;
+    long long tile_steps = 0; // 64-pixel x 64-filter tiles times reduction steps
+    if (units) {
+        narrow = espdl::conv2d_s8_narrow_us(g, in, filter, cus);
+        gemm = espdl::conv2d_s8_unitgemm_us(g, in, filter, &tile_steps);
+    }
+    if (espdl::conv2d_s8_stem_supports(g, residual))
+        return units && narrow < 5.2f ? DENSE_NARROW : DENSE_STEM;
+    const bool flat = g.k_h == 1 && g.k_w == 1 && g.stride_h == 1 && g.stride_w == 1 && g.pad_top == 0 &&
+        g.pad_left == 0 && g.out_h == g.in_h && g.out_w == g.in_w;
+    const DenseRoute few = narrow < gemm ? DENSE_NARROW : DENSE_UNITGEMM;
+    if (flat) {
+        if (espdl::conv2d_s8_pwgemm_supports(g, in, filter, cus))
+            return units && narrow < 0.97f * gemm ? DENSE_NARROW : DENSE_PWGEMM;
+        return units && tile_steps <= 3500 ? few : DENSE_DIRECT;
+    }
+    if (!espdl::conv2d_s8_units_aligned(g, in, filter))
+        return units ? few : DENSE_DIRECT;
+    const int filter_tiles = (g.out_c + 15) / 16, filter_groups = (g.out_c + 63) / 64;
+    const long long unit_limit = 2500 + 3500ll * filter_tiles / filter_groups;
+    const bool strided = g.stride_h != 1 || g.stride_w != 1;
+    if (units && (tile_steps <= unit_limit || (strided && g.k_h * g.k_w * g.in_c > 256) || g.k_h * g.k_w * g.in_c >= 2048))
+        return few;
+    return espdl::conv2d_s8_tiled_supports(g, in, filter, cus) ? DENSE_TILED : DENSE_DIRECT;
+}
+
 } // namespace
 
 extern "C" {
@@ -195,29 +250,40 @@ int espdl_hip_conv2d_add(const espdl_hip_conv_desc *desc, const void *in, const 
                                      "depthwise_s8_mfma");
             return device_status(espdl::launch_depthwise_s8(g, i8, f8, b32, shift, lut, o8, s), "depthwise_s8");
         }
-        if (espdl::conv2d_s8_stem_supports(g, residual))
-            return device_status(espdl::launch_conv2d_s8_stem(g, i8, f8, b32, shift, lut, o8, cu_count_cached(), s),
-                                 "conv2d_s8_stem");
-        // (the second test admits products with fewer than 32 filters, which only the few-rows kernel inside takes)
-        if (espdl::conv2d_s8_pwgemm_supports(g, in, filter, cu_count_cached()) ||
-            (lut == nullptr && residual == nullptr && espdl::conv2d_s8_rows_supports(g, in, filter, cu_count_cached())))
-            return device_status(espdl::launch_conv2d_s8_pwgemm(g, i8, f8, b32, shift, lut, residual, o8, cu_count_cached(), s),
-                                 "conv2d_s8_pwgemm");
-        // Windows over 64 channels or more on few pixels: the pointwise GEMM kernel over gathered rows.  Strided
-        // windows (80 x 80 x 128 -> 128 at stride 2, batch 64: 91 -> 41 us); at stride 1 up to 128 K output pixels
-        // (40 x 40 x 128 -> 64, batch 64: 26 -> 22 us; 20 x 20 x 256 -> 256: 93 -> 38 us) or with a reduction axis of
-        // 2048 or more, whose filters the LDS-tiled kernel below cannot keep resident (80 x 80 x 256 -> 256: 732 ->
-        // 472 us); with more pixels and fewer channels that kernel is faster (80 x 80 x 64 -> 64: 30 against 41 us).
-        const bool few_pixels = (long long)g.batch * g.out_h * g.out_w <= 128 * 1024;
-        if ((g.stride_h != 1 || g.stride_w != 1 || few_pixels || g.k_h * g.k_w * g.in_c >= 2048) &&
-            espdl::conv2d_s8_wingemm_supports(g, in, filter, cu_count_cached()))
-            return device_status(espdl::launch_conv2d_s8_wingemm(g, i8, f8, b32, shift, lut, residual, o8, cu_count_cached(), s),
-                                 "conv2d_s8_wingemm");
-        if (espdl::conv2d_s8_tiled_supports(g, in, filter, cu_count_cached()))
-            return device_status(espdl::launch_conv2d_s8_tiled(g, i8, f8, b32, shift, lut, residual, o8, cu_count_cached(), s),
-                                 "conv2d_s8_tiled");
-        return device_status(espdl::launch_conv2d_s8_mfma(g, i8, f8, b32, shift, lut, residual, o8, cu_count_cached(), s),
-                             "conv2d_s8");
+        const int cus = cu_count_cached();
+        const auto run = [&](auto launch, const char *name) {
+            return device_status(launch(g, i8, f8, b32, shift, lut, residual, o8, cus, s), name);
+        };
+        // in parts of the batch where the input is larger than a launch's offsets reach
+        const auto run_units = [&](auto launch, const char *name) {
+            espdl::ConvGeom part = g;
+            const int most = images_per_unit_launch(g);
+            const size_t in_img = (size_t)g.in_h * g.in_w * g.in_pitch, out_pix = (size_t)g.out_h * g.out_w;
+            for (int n = 0; n < g.batch; n += most) {
+                part.batch = g.batch - n < most ? g.batch - n : most;
+                const hipError_t e = launch(part, i8 + n * in_img, f8, b32, shift, lut,
+                                            residual ? residual + n * out_pix * g.res_pitch : nullptr,
+                                            o8 + n * out_pix * g.out_pitch, cus, s);
+                if (e != hipSuccess)
+                    return device_status(e, name);
+            }
+            return (int)ESPDL_HIP_OK;
+        };
+        switch (dense_s8_route(g, in, filter, residual, cus)) {
+        case DENSE_STEM:
+            return device_status(espdl::launch_conv2d_s8_stem(g, i8, f8, b32, shift, lut, o8, cus, s), "conv2d_s8_stem");
+        case DENSE_NARROW:
+            return run_units(espdl::launch_conv2d_s8_narrow, "conv2d_s8_narrow");
+        case DENSE_UNITGEMM:
+            return run_units(espdl::launch_conv2d_s8_unitgemm, "conv2d_s8_unitgemm");
+        case DENSE_PWGEMM:
+            return run(espdl::launch_conv2d_s8_pwgemm, "conv2d_s8_pwgemm");
+        case DENSE_TILED:
+            return run(espdl::launch_conv2d_s8_tiled, "conv2d_s8_tiled");
+        case DENSE_DIRECT:
+            break;
+        }
+        return run(espdl::launch_conv2d_s8_mfma, "conv2d_s8");
     }
     if (lut != nullptr || residual != nullptr)
         return fail(ESPDL_HIP_ENOTSUP, "the fused LUT / residual epilogues exist for ESPDL_HIP_S8 only");

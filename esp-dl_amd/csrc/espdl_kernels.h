@@ -31,16 +31,23 @@ hipError_t launch_conv2d_s8_mfma(const ConvGeom &g, const int8_t *in, const int8
 // Pointwise int8 convolution / Gemm as a tiled GEMM with both operands streamed through LDS; for layers
 // with few pixels per compute unit, where the implicit-GEMM kernel's filter staging dominates.
 bool conv2d_s8_pwgemm_supports(const ConvGeom &g, const void *in, const void *filter, int cu_count);
-bool conv2d_s8_rows_supports(const ConvGeom &g, const void *in, const void *filter, int cu_count);
 hipError_t launch_conv2d_s8_pwgemm(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,
                                    const int32_t *shift, const int8_t *lut, const int8_t *residual, int8_t *out,
                                    int cu_count, hipStream_t stream);
-// A convolution with a window through the pointwise GEMM kernel, rows gathered from under the window (channels a
-// multiple of 64, few output pixels per compute unit, a long reduction axis).
-bool conv2d_s8_wingemm_supports(const ConvGeom &g, const void *in, const void *filter, int cu_count);
-hipError_t launch_conv2d_s8_wingemm(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,
-                                    const int32_t *shift, const int8_t *lut, const int8_t *residual, int8_t *out,
-                                    int cu_count, hipStream_t stream);
+// A convolution through the pointwise GEMM kernel whatever its channel count, each 16-byte unit of a k step with a tap
+// of its own.
+bool conv2d_s8_units_support(const ConvGeom &g); // tensors of 16 bytes to 2 GiB: this kernel and the narrow one
+bool conv2d_s8_units_aligned(const ConvGeom &g, const void *in, const void *filter);
+float conv2d_s8_unitgemm_us(const ConvGeom &g, const void *in, const void *filter, long long *tile_steps);
+hipError_t launch_conv2d_s8_unitgemm(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,
+                                     const int32_t *shift, const int8_t *lut, const int8_t *residual, int8_t *out,
+                                     int cu_count, hipStream_t stream);
+// Dense int8 convolution / Gemm with few outputs, any channel count: 16 pixels x 16 to 64 filters per workgroup, the
+// reduction axis split over its wavefronts (conv2d_s8_narrow.hip).
+float conv2d_s8_narrow_us(const ConvGeom &g, const void *in, const void *filter, int cu_count);
+hipError_t launch_conv2d_s8_narrow(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,
+                                   const int32_t *shift, const int8_t *lut, const int8_t *residual, int8_t *out,
+                                   int cu_count, hipStream_t stream);
 // Dense int8 convolution with a window, input tile and filters staged in LDS (conv2d_s8_tiled.hip): channel
 // count a multiple of 16, 16-byte aligned input and filter.
 bool conv2d_s8_tiled_supports(const ConvGeom &g, const void *in, const void *filter, int cu_count);

@@ -120,6 +120,21 @@ TILED_MANY_PIXELS = [
     ("tm64_50x60_k3d2p2_oc72", (50, 60, 64), 72, (3, 3), (1, 1), (2, 2), (2, 2, 2, 2), False, True),
 ]
 
+# Windows over channel counts around the 16-channel units the two unit-reading kernels work in (one less, one more, a
+# single channel, several units), with the batch each needs to reach the one kernel or the other: (case, images).
+UNIT_CASES = [
+    (("u17_5x7_k3p1_oc1", (5, 7, 17), 1, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True), 1),
+    (("u15_9x9_k3s2p1_oc31", (9, 9, 15), 31, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), True, False), 2),
+    (("u33_13x11_k5p2_oc65", (13, 11, 33), 65, (5, 5), (1, 1), (1, 1), (2, 2, 2, 2), True, True), 3),
+    (("u1_6x8_k5s2_oc3", (6, 8, 1), 3, (5, 5), (2, 2), (1, 1), (0, 0, 0, 0), False, False), 1),
+    (("u137_8x9_k3d2p2_oc50", (8, 9, 137), 50, (3, 3), (1, 1), (2, 2), (2, 2, 2, 2), True, True), 2),
+    (("u160_6x6_k3p1_oc17", (6, 6, 160), 17, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, False), 1),
+    (("u17_40x41_k3p1_oc33", (40, 41, 17), 33, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True), 40),
+    (("u31_30x31_k5s2p2_oc64", (30, 31, 31), 64, (5, 5), (2, 2), (1, 1), (2, 2, 2, 2), True, False), 80),
+    (("u48_30x30_k3p1_oc70", (30, 30, 48), 70, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True), 30),
+    (("u61_50x50_k1_oc20", (50, 50, 61), 20, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, True), 20),
+]
+
 CONFIG1 = ("config1_56x56x64_k3p1_relu", (56, 56, 64), 64, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)
 
 DW_CASES = [

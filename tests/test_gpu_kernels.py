@@ -5,7 +5,7 @@ import ctypes
 import numpy as np
 import pytest
 
-from cases import CONFIG1, CONV_CASES, DW_CASES, GEMM_CASES, POINTWISE_MANY_PIXELS, WIDE_ROWS, WINDOW_GEMM_CASES, TILED_MANY_PIXELS, STEM_CASES, TILED_CASES, every_sum_image, rng_int8, typical_shift
+from cases import CONFIG1, CONV_CASES, DW_CASES, GEMM_CASES, POINTWISE_MANY_PIXELS, WIDE_ROWS, WINDOW_GEMM_CASES, TILED_MANY_PIXELS, STEM_CASES, TILED_CASES, UNIT_CASES, every_sum_image, rng_int8, typical_shift
 from gpu_util import announce, espdl, to_dev, to_host
 
 pytestmark = pytest.mark.gpu
@@ -166,6 +166,27 @@ def test_conv2d_s8_window_on_many_pixels(oracle, case, flavour):
         kw["half_even"] = True
     if flavour == "residual":
         kw["residual_seed"] = 11
+    oracle.set_threads(16)
+    got, want = _run_conv_s8(oracle, x, f, bias, shift, k, stride, dil, pads, relu, **kw)
+    np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("case", UNIT_CASES, ids=lambda c: c[0][0])
+@pytest.mark.parametrize("flavour", ["per_channel", "half_even", "lut_residual", "general_epilogue"])
+def test_conv2d_s8_channel_units(oracle, case, flavour):
+    """Channel counts that end inside a 16-channel unit, through both kernels that read windows as units."""
+    announce(f"conv2d_s8 channel units {case[0][0]} {flavour}")
+    x, f, bias, shift, k, stride, dil, pads, relu = _conv_inputs(case[0], 251, case[1], True)
+    kw = {}
+    if flavour == "half_even":
+        kw["half_even"] = True
+    if flavour == "lut_residual":
+        kw["lut"] = np.array([(i * 109 + 37) & 0xFF for i in range(256)], dtype=np.uint8).view(np.int8)
+        kw["residual_seed"] = 13
+    if flavour == "general_epilogue":
+        shift = np.array(shift, dtype=np.int32)
+        shift[::3] = 0
+        shift[1::5] = 33
     oracle.set_threads(16)
     got, want = _run_conv_s8(oracle, x, f, bias, shift, k, stride, dil, pads, relu, **kw)
     np.testing.assert_array_equal(got, want)
