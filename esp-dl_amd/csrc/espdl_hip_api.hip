@@ -125,12 +125,12 @@ bool misaligned(const void *p, uintptr_t a)
 }
 
 // Images of a layer that one launch of the unit-reading kernels takes: their offsets into the input are 31-bit.
-int images_per_unit_launch(const espdl::ConvGeom &g)
+int images_per_launch(const espdl::ConvGeom &g, bool (*supports)(const espdl::ConvGeom &))
 {
     espdl::ConvGeom part = g;
-    while (part.batch > 1 && !espdl::conv2d_s8_units_support(part))
+    while (part.batch > 1 && !supports(part))
         part.batch = (part.batch + 1) / 2;
-    return espdl::conv2d_s8_units_support(part) ? part.batch : 0;
+    return supports(part) ? part.batch : 0;
 }
 
 enum DenseRoute { DENSE_STEM, DENSE_NARROW, DENSE_UNITGEMM, DENSE_PWGEMM, DENSE_TILED, DENSE_DIRECT };
@@ -152,7 +152,7 @@ enum DenseRoute { DENSE_STEM, DENSE_NARROW, DENSE_UNITGEMM, DENSE_PWGEMM, DENSE_
 // 5 x 5, batch 142: 509 -> 111 us; 45 x 99 x 162 -> 87, 5 x 5 at stride 2, batch 3: 312 -> 33 us.
 DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *filter, const void *residual, int cus)
 {
-    const bool units = images_per_unit_launch(g) > 0;
+    const bool units = images_per_launch(g, espdl::conv2d_s8_units_support) > 0;
     float narrow = 0.f, gemm = 0.f;
     long long tile_steps = 0; // 64-pixel x 64-filter tiles times reduction steps
     if (units) {
@@ -257,7 +257,7 @@ int espdl_hip_conv2d_add(const espdl_hip_conv_desc *desc, const void *in, const 
         // in parts of the batch where the input is larger than a launch's offsets reach
         const auto run_units = [&](auto launch, const char *name) {
             espdl::ConvGeom part = g;
-            const int most = images_per_unit_launch(g);
+            const int most = images_per_launch(g, espdl::conv2d_s8_units_support);
             const size_t in_img = (size_t)g.in_h * g.in_w * g.in_pitch, out_pix = (size_t)g.out_h * g.out_w;
             for (int n = 0; n < g.batch; n += most) {
                 part.batch = g.batch - n < most ? g.batch - n : most;
@@ -295,6 +295,22 @@ int espdl_hip_conv2d_add(const espdl_hip_conv_desc *desc, const void *in, const 
     int16_t *o16 = static_cast<int16_t *>(out);
     if (depthwise)
         return device_status(espdl::launch_depthwise_s16(g, i16, f16, b64, shift, o16, s), "depthwise_s16");
+    // The earlier kernel walks pixel tiles under filters it keeps in LDS: still the better one for a short reduction
+    // under few filters over many pixels (80 x 80 x 16 -> 16, 1 x 1, batch 64: 17 against 22 us).
+    const long long k_steps = ((long long)g.k_h * g.k_w * g.in_c + 63) / 64;
+    const bool many_pixels = k_steps <= 3 && g.out_c <= 48 && (long long)g.batch * g.out_h * g.out_w >= 60000;
+    const int most = images_per_launch(g, espdl::conv2d_s16_units_supports);
+    if (most > 0 && !(many_pixels && espdl::conv2d_s16_mfma_supports(g, i16, f16, o16))) {
+        espdl::ConvGeom part = g;
+        for (int n = 0; n < g.batch; n += most) {
+            part.batch = g.batch - n < most ? g.batch - n : most;
+            const hipError_t e = espdl::launch_conv2d_s16_units(part, i16 + (size_t)n * g.in_h * g.in_w * g.in_c, f16, b64, shift,
+                                                                o16 + (size_t)n * g.out_h * g.out_w * g.out_c, cu_count_cached(), s);
+            if (e != hipSuccess)
+                return device_status(e, "conv2d_s16_units");
+        }
+        return ESPDL_HIP_OK;
+    }
     if (espdl::conv2d_s16_mfma_supports(g, i16, f16, o16))
         return device_status(espdl::launch_conv2d_s16_mfma(g, i16, f16, b64, shift, o16, cu_count_cached(), s),
                              "conv2d_s16_mfma");

@@ -170,7 +170,12 @@ bool conv2d_s8_stem_supports(const ConvGeom &g, const void *residual);
 hipError_t launch_conv2d_s8_stem(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,
                                  const int32_t *shift, const int8_t *lut, int8_t *out, int cu_count, hipStream_t stream);
 
-// Dense int16 convolution on the int8 matrix pipe (two signed bytes per operand); in_c % 16 == 0, reduction length <= 36000.
+// Dense int16 convolution on the int8 matrix pipe (two signed bytes per operand), any channel count, reductions under
+// 65536 (conv_s16_units.hip); and the same with the filters resident in LDS, in_c % 16 == 0, reduction length <= 36000
+// (conv_s16_mfma.hip).
+bool conv2d_s16_units_supports(const ConvGeom &g);
+hipError_t launch_conv2d_s16_units(const ConvGeom &g, const int16_t *in, const int16_t *filter, const int64_t *bias,
+                                   const int32_t *shift, int16_t *out, int cu_count, hipStream_t stream);
 bool conv2d_s16_mfma_supports(const ConvGeom &g, const void *in, const void *filter, const void *out);
 hipError_t launch_conv2d_s16_mfma(const ConvGeom &g, const int16_t *in, const int16_t *filter, const int64_t *bias,
                                   const int32_t *shift, int16_t *out, int cu_count, hipStream_t stream);

@@ -626,6 +626,48 @@ def test_conv2d_s16_matrix_pipe(oracle, case):
     assert want.min() < want.max()
 
 
+S16_UNIT_CASES = [
+    # (name, (n, h, w, c), out_c, k, stride, dil, pads, relu, half_even, lowest and highest shift, values): channel counts
+    # around the 16-channel units, one to four filter tiles and tails of each, few pixels (narrow kernel) and many
+    # (tiled kernel, 64 and 128 pixels), shifts on both sides of 16 and outside the short epilogue's 1 .. 44
+    ("n_17_33", (1, 7, 9, 17), 33, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, False, 24, 28, "random"),
+    ("n_1_5", (2, 6, 5, 1), 5, (5, 5), (2, 2), (1, 1), (2, 2, 2, 2), False, False, 18, 22, "random"),
+    ("n_137_7_halfeven", (1, 9, 8, 137), 7, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), False, True, 27, 30, "random"),
+    ("n_8_20_bias_only_tail", (1, 3, 3, 8), 20, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, False, 19, 22, "random"),
+    ("t_31_16", (24, 30, 31, 31), 16, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, False, 24, 27, "random"),
+    ("t_16_13", (40, 30, 30, 16), 13, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), False, False, 22, 26, "random"),
+    ("t_48_32", (12, 30, 30, 48), 32, (3, 3), (1, 1), (2, 2), (2, 2, 2, 2), True, False, 25, 28, "random"),
+    ("t_33_70", (12, 28, 29, 33), 70, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), True, False, 24, 28, "random"),
+    ("t_64_64_halfeven", (8, 20, 21, 64), 64, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), False, True, 25, 28, "random"),
+    ("t_12_100_mixed_shifts", (30, 20, 20, 12), 100, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), False, False, 9, 20, "random"),
+    ("t_16_40_shifts_16_17", (60, 20, 20, 16), 40, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, False, 16, 17, "random"),
+    ("t_16_40_general", (60, 20, 20, 16), 40, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, False, -3, 60, "random"),
+    ("t_64_64_min", (10, 24, 24, 64), 64, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), False, False, 24, 28, "min"),
+    ("t_64_64_max_low_shifts", (10, 24, 24, 64), 64, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), False, False, 1, 20, "max"),
+]
+
+
+@pytest.mark.parametrize("case", S16_UNIT_CASES, ids=lambda c: c[0])
+def test_conv2d_s16_channel_units(oracle, case):
+    """int16 convolutions over any channel count through the two unit-reading kernels and their epilogues."""
+    announce(f"conv2d_s16 units {case[0]}")
+    name, (n, h, w, c), oc, k, stride, dil, pads, relu, half_even, s_lo, s_hi, values = case
+    rng = np.random.default_rng(0x517 + len(name))
+    fill = {"min": (-32768, -32767), "max": (32767, 32768), "random": (-32768, 32768)}[values]
+    x = rng.integers(*fill, size=(n, h, w, c)).astype(np.int16)
+    f = rng.integers(*fill, size=(oc, k[0], k[1], c)).astype(np.int16)
+    bias = rng.integers(-2**40, 2**40, size=oc).astype(np.int64)
+    shift = rng.integers(s_lo, s_hi + 1, size=oc).astype(np.int32)
+    m = espdl()
+    oracle.set_threads(16)
+    got = m.conv2d(to_dev(x), to_dev(f), to_dev(bias), to_dev(shift), k, stride, dil, pads,
+                   activation=m.capi.RELU if relu else m.capi.LINEAR,
+                   round_mode=m.capi.ROUND_HALF_EVEN if half_even else m.capi.ROUND_HALF_UP)
+    want = oracle.conv2d_s16(x, f, bias, shift, k, stride, dil, pads, oracle.RELU if relu else oracle.LINEAR,
+                             oracle.ROUND_HALF_EVEN if half_even else oracle.ROUND_HALF_UP)
+    np.testing.assert_array_equal(to_host(got), want)
+
+
 @pytest.mark.parametrize("case", DW_TILE_CASES, ids=lambda c: c[0])
 def test_depthwise_s8_tiles(oracle, case):
     announce(f"depthwise_s8 tiles {case[0]}")
