@@ -133,6 +133,10 @@ def lib():
         L.espdl_hip_mbconv_s8_supported.argtypes = [mp]
         L.espdl_hip_mbconv_s8.argtypes = [mp, vp, ctypes.POINTER(MbconvWeights), vp, vp, vp]
         L.espdl_hip_mbconv_s8_staged.argtypes = L.espdl_hip_mbconv_s8.argtypes
+        L.espdl_hip_mbconv_s8_ws.argtypes = [mp, vp, ctypes.POINTER(MbconvWeights), vp, vp, vp, vp]
+        L.espdl_hip_mbconv_s8_ws.restype = ctypes.c_int
+        L.espdl_hip_mbconv_s8_workspace.argtypes = [mp]
+        L.espdl_hip_mbconv_s8_workspace.restype = i64
         L.espdl_hip_mbconv_s8_preferred.argtypes = [mp]
         for name in ("mbconv_out_shape", "mbconv_s8_supported", "mbconv_s8_preferred", "mbconv_s8", "mbconv_s8_staged"):
             getattr(L, "espdl_hip_" + name).restype = ctypes.c_int
@@ -223,10 +227,11 @@ def conv2d_gap_s8(x, filt, bias, shift, conv_out_exp, pool_out_exp, activation=L
 
 def mbconv_s8(x, expand, dw, project, k, stride=(1, 1), dilation=(1, 1), pads=(0, 0, 0, 0), relus=(True, True, False),
               residual=None, round_mode=ROUND_HALF_UP, out=None, stream=None, staged=False, expand_conv=None,
-              residual_shift=0, clip_expand=None, clip_dw=None):
+              residual_shift=0, clip_expand=None, clip_dw=None, workspace=None):
     """Fused inverted-residual block (staged=True: espdl_hip_mbconv_s8_staged, the separate stages with the
     intermediates in the library's own device array; `out` must then be given, nothing is allocated).  expand / dw / project are (filter, bias, shift) triples of CUDA
     tensors (expand may be None); filters as for conv2d: [E][C], [kH][kW][E], [OC][E].
+    workspace: device tensor of [N][out_h][out_w][E] bytes; the block then runs as two launches where that form exists.
     expand_conv = (kernel, stride, pads) makes the expand stage a dense convolution with a window over the
     block input (filter [E][kH][kW][C]); the depthwise stage then works on that convolution's output."""
     import torch
@@ -254,6 +259,10 @@ def mbconv_s8(x, expand, dw, project, k, stride=(1, 1), dilation=(1, 1), pads=(0
     if out is None:
         out = torch.empty((n, oh.value, ow.value, out_c), dtype=torch.int8, device=x.device)
     wts = MbconvWeights(_p(we), _p(be), _p(se), _p(wd), _p(bd), _p(sd), _p(wp), _p(bp), _p(sp))
+    if workspace is not None:
+        _check(lib().espdl_hip_mbconv_s8_ws(ctypes.byref(desc), _p(x), ctypes.byref(wts), _p(residual), _p(workspace), _p(out),
+                                            _stream(stream)))
+        return out
     fn = lib().espdl_hip_mbconv_s8_staged if staged else lib().espdl_hip_mbconv_s8
     _check(fn(ctypes.byref(desc), _p(x), ctypes.byref(wts), _p(residual), _p(out), _stream(stream)))
     return out

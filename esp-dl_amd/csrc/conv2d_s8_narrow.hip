@@ -33,7 +33,7 @@ struct NarrowArgs {
     const int8_t *lut, *res;
     int8_t *out;
     int n_pix, out_c, out_pitch, res_pitch;
-    int ksteps, relu, half_even, n_shift;
+    int ksteps, relu, half_even, n_shift, res_shift;
 };
 
 template <int NT, bool SPLIT, bool ALIGNED>
@@ -137,13 +137,14 @@ __global__ __launch_bounds__(kThreads) void conv2d_s8_narrow_kernel(const Narrow
             sum = part[0][wave][lane] + part[1][wave][lane] + part[2][wave][lane] + part[3][wave][lane];
         const int f = n0 + 4 * NT * quad + 4 * (SPLIT ? wave : t);
         int q[4];
+        const int word = a.res_shift != 0 ? requant4_s8(res[t], make_requant4(a.res_shift)) : res[t];
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             q[r] = requant_s8(sum[r] + bias[t][r], shift[t][r], relu, half_even);
             if (a.lut != nullptr)
                 q[r] = lut_l[q[r] + 128];
             if (a.res != nullptr)
-                q[r] = clamp_s8(q[r] + (int)(int8_t)(res[t] >> (8 * r)));
+                q[r] = clamp_s8(q[r] + (int)(int8_t)(word >> (8 * r)));
         }
         if (m >= a.n_pix || f >= a.out_c)
             continue;
@@ -230,6 +231,7 @@ hipError_t launch_conv2d_s8_narrow(const ConvGeom &g, const int8_t *in, const in
     a.relu = g.relu;
     a.half_even = g.half_even;
     a.n_shift = g.n_shift;
+    a.res_shift = g.res_shift;
     if (a.n_pix == 0)
         return hipSuccess;
     const NarrowPlan p = narrow_plan(g, cu_count);

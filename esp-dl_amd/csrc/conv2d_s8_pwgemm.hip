@@ -46,7 +46,7 @@ struct PwArgs {
     int K, N;
     int in_pitch, out_pitch, res_pitch; // bytes between consecutive rows of in, out and res (K, N, N when dense)
     int ksteps;
-    int relu, half_even, n_shift;
+    int relu, half_even, n_shift, res_shift;
     int out_vec; // 16, 4 or 1
     // UNITS builds: a convolution with a window as the same product over gathered rows (im2col on the fly): row m is
     // output pixel m, its k bytes are the units of conv_window.h (zeros outside the image)
@@ -286,6 +286,8 @@ __global__ __launch_bounds__(kThreads) void conv2d_s8_pwgemm_kernel(const PwArgs
 
     // epilogue: lane (col, quad) holds, per pixel tile and group, filters 64*g + 16*quad + [0, 16)
     const int floor_pk = relu ? 0 : (int)0x80008000u;
+    const Requant4 res_q = make_requant4(a.res_shift);
+    auto rescaled = [&](int word) { return a.res_shift != 0 ? requant4_s8(word, res_q) : word; };
     // one straight-line copy per rounding mode (pack_fast4 mode 1: half up, 5: half even)
     auto epilogue = [&](auto mode) {
     #pragma unroll
@@ -325,7 +327,7 @@ __global__ __launch_bounds__(kThreads) void conv2d_s8_pwgemm_kernel(const PwArgs
                         const v4i r = *reinterpret_cast<const v4i_unaligned *>(a.res + roff);
     #pragma unroll
                         for (int d = 0; d < 4; d++)
-                            v[d] = sat_add4_s8(v[d], r[d]);
+                            v[d] = sat_add4_s8(v[d], rescaled(r[d]));
                     }
                     if (a.out_vec == 16)
                         __builtin_nontemporal_store(v, reinterpret_cast<v4i *>(a.out + goff));
@@ -337,14 +339,14 @@ __global__ __launch_bounds__(kThreads) void conv2d_s8_pwgemm_kernel(const PwArgs
                         if (n + 4 * t + 4 <= a.N) {
                             int v = words[t];
                             if (a.res != nullptr)
-                                v = sat_add4_s8(v, *reinterpret_cast<const int_unaligned *>(a.res + roff + 4 * t));
+                                v = sat_add4_s8(v, rescaled(*reinterpret_cast<const int_unaligned *>(a.res + roff + 4 * t)));
                             *reinterpret_cast<int_unaligned *>(a.out + goff + 4 * t) = v;
                         } else {
                             for (int r = 0; r < 4; r++)
                                 if (n + 4 * t + r < a.N) {
                                     int v = (int)(int8_t)(words[t] >> (8 * r));
                                     if (a.res != nullptr)
-                                        v = clamp_s8(v + (int)a.res[roff + 4 * t + r]);
+                                        v = clamp_s8(v + (int)(int8_t)rescaled((int)(unsigned char)a.res[roff + 4 * t + r]));
                                     a.out[goff + 4 * t + r] = (int8_t)v;
                                 }
                         }
@@ -489,6 +491,7 @@ hipError_t launch_conv2d_s8_pwgemm(const ConvGeom &g, const int8_t *in, const in
     a.relu = g.relu;
     a.half_even = g.half_even;
     a.n_shift = g.n_shift;
+    a.res_shift = g.res_shift;
     a.hw = 0;
     a.gap_scale = 0.f;
     const uintptr_t oaddr = reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(residual);
@@ -561,6 +564,7 @@ hipError_t launch_conv2d_s8_unitgemm(const ConvGeom &g, const int8_t *in, const 
     a.relu = g.relu;
     a.half_even = g.half_even;
     a.n_shift = g.n_shift;
+    a.res_shift = g.res_shift;
     const uintptr_t oaddr = reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(residual);
     a.out_vec = ((a.N & 15) == 0 && (oaddr & 15) == 0 && (a.out_pitch & 15) == 0) ? 16
         : (((a.N & 3) == 0 && (oaddr & 3) == 0 && (a.out_pitch & 3) == 0) ? 4 : 1);
@@ -614,6 +618,7 @@ hipError_t launch_conv2d_gap_s8(const ConvGeom &g, const int8_t *in, const int8_
     a.relu = g.relu;
     a.half_even = g.half_even;
     a.n_shift = g.n_shift;
+    a.res_shift = g.res_shift;
     a.out_vec = 1;
     a.gap_scale = gap_scale;
     if (a.M == 0)

@@ -1126,15 +1126,14 @@ int espdl_hip_mbconv_s8_preferred(const espdl_hip_mbconv_desc *desc)
     return (kind == 5 ? espdl::mbconv_s8_group_has_fast_build(p) : espdl::mbconv_s8_wave_has_fast_build(p)) ? 1 : 0;
 }
 
-int espdl_hip_mbconv_s8(const espdl_hip_mbconv_desc *desc, const int8_t *in, const espdl_hip_mbconv_weights *w,
-                        const int8_t *residual, int8_t *out, void *stream)
+// Checks a block's operands and puts them next to its geometry.
+static int mbconv_params(const espdl_hip_mbconv_desc *desc, const int8_t *in, const espdl_hip_mbconv_weights *w,
+                         const int8_t *residual, int8_t *out, espdl::MbconvParams *params)
 {
-    espdl::MbconvParams p = {};
+    espdl::MbconvParams &p = *params;
     const int rc = mbconv_geometry(desc, &p);
-    if (rc != ESPDL_HIP_OK)
+    if (rc != ESPDL_HIP_OK || p.batch == 0)
         return rc;
-    if (p.batch == 0)
-        return ESPDL_HIP_OK;
     if (in == nullptr || out == nullptr || w == nullptr || w->w_dw == nullptr || w->s_dw == nullptr ||
         w->w_project == nullptr || w->s_project == nullptr || (desc->has_expand && (w->w_expand == nullptr || w->s_expand == nullptr)))
         return fail(ESPDL_HIP_EINVAL, "in, out, filters and shifts must not be NULL");
@@ -1154,6 +1153,16 @@ int espdl_hip_mbconv_s8(const espdl_hip_mbconv_desc *desc, const int8_t *in, con
     p.w_project = w->w_project;
     p.b_project = w->b_project;
     p.s_project = w->s_project;
+    return ESPDL_HIP_OK;
+}
+
+int espdl_hip_mbconv_s8(const espdl_hip_mbconv_desc *desc, const int8_t *in, const espdl_hip_mbconv_weights *w,
+                        const int8_t *residual, int8_t *out, void *stream)
+{
+    espdl::MbconvParams p = {};
+    const int rc = mbconv_params(desc, in, w, residual, out, &p);
+    if (rc != ESPDL_HIP_OK || p.batch == 0)
+        return rc;
     if (espdl::mbconv_has_clip(p)) {
         if (!desc->has_expand || !espdl::mbconv_s8_wave_has_fast_build(p))
             return fail(ESPDL_HIP_ENOTSUP, "a Clip between the stages is covered for the block shapes with a guard-free build of the one-wavefront-per-tile kernel, round half up");
@@ -1200,6 +1209,85 @@ int espdl_hip_mbconv_s8(const espdl_hip_mbconv_desc *desc, const int8_t *in, con
         return fail(ESPDL_HIP_ENOTSUP, "this block shape is not covered by the fused kernel");
     return device_status(espdl::launch_mbconv_s8_fused(p, cu_count_cached(), reinterpret_cast<hipStream_t>(stream)),
                          "mbconv_s8_fused");
+}
+
+// The project convolution of a block as a dense convolution over the depthwise result.
+static espdl::ConvGeom project_geometry(const espdl::MbconvParams &p)
+{
+    espdl::ConvGeom g = {};
+    g.batch = p.batch;
+    g.in_h = g.out_h = p.out_h;
+    g.in_w = g.out_w = p.out_w;
+    g.in_c = g.in_pitch = p.exp_c;
+    g.out_c = g.out_pitch = g.res_pitch = p.out_c;
+    g.k_h = g.k_w = g.stride_h = g.stride_w = g.dil_h = g.dil_w = 1;
+    g.relu = p.relu_project;
+    g.half_even = p.half_even;
+    g.n_shift = p.n_s_project;
+    g.res_shift = p.residual_shift;
+    return g;
+}
+
+// Dense kernel of the project convolution and its expected time.
+static auto project_launch(const espdl::ConvGeom &g, const void *in, const void *filter, int cus, float *us)
+{
+    long long tile_steps;
+    const bool flat = espdl::conv2d_s8_pwgemm_supports(g, in, filter, cus);
+    const float gemm = espdl::conv2d_s8_unitgemm_us(g, in, filter, &tile_steps) * (flat ? 0.97f : 1.f);
+    const float narrow = espdl::conv2d_s8_narrow_us(g, in, filter, cus);
+    *us = narrow < gemm ? narrow : gemm;
+    return narrow < gemm ? espdl::launch_conv2d_s8_narrow : (flat ? espdl::launch_conv2d_s8_pwgemm : espdl::launch_conv2d_s8_unitgemm);
+}
+
+// The single launch is a chain of 10 to 25 us through all expanded channels of a tile, whatever the batch, until the
+// device is full; the two launches start at 7 us and grow with the work (MobileNetV2 at 224 x 224: one image 282 -> 155 us,
+// 16 images 296 -> 221 us; the blocks of batch 256 stay single launches).  Where no single-launch kernel has a fast build
+// the alternative is three launches, of which the depthwise one alone takes 9 us.
+int64_t espdl_hip_mbconv_s8_workspace(const espdl_hip_mbconv_desc *desc)
+{
+    espdl::MbconvParams p = {};
+    if (mbconv_geometry(desc, &p) != ESPDL_HIP_OK || !desc->has_expand || p.batch == 0)
+        return 0;
+    static const int8_t *const aligned = reinterpret_cast<const int8_t *>(uintptr_t(256));
+    p.in = aligned;
+    p.w_expand = aligned;
+    const espdl::ConvGeom g = project_geometry(p);
+    if (!espdl::mbconv_s8_split_supports(p) || !espdl::conv2d_s8_units_support(g))
+        return 0;
+    const int cus = cu_count_cached();
+    float project = 0.f;
+    (void)project_launch(g, aligned, aligned, cus, &project);
+    const float expand_dw = espdl::mbconv_s8_expand_dw_us(p);
+    float other = 9.f + 1.25f * expand_dw + project;
+    if (espdl_hip_mbconv_s8_supported(desc) == 0)
+        other = 1e30f; // a Clip between the stages in half-even mode: no single launch
+    else if (espdl_hip_mbconv_s8_preferred(desc) == 1)
+        other = espdl_hip_mbconv_s8_supported(desc) == 5 ? espdl::mbconv_s8_group_us(p, cus) : espdl::mbconv_s8_wave_us(p);
+    return expand_dw + project < other ? (int64_t)p.batch * p.out_h * p.out_w * p.exp_c : 0;
+}
+
+int espdl_hip_mbconv_s8_ws(const espdl_hip_mbconv_desc *desc, const int8_t *in, const espdl_hip_mbconv_weights *w,
+                           const int8_t *residual, void *workspace, int8_t *out, void *stream)
+{
+    if (workspace == nullptr)
+        return espdl_hip_mbconv_s8(desc, in, w, residual, out, stream);
+    espdl::MbconvParams p = {};
+    const int rc = mbconv_params(desc, in, w, residual, out, &p);
+    if (rc != ESPDL_HIP_OK || p.batch == 0)
+        return rc;
+    const espdl::ConvGeom g = project_geometry(p);
+    if (!desc->has_expand || misaligned(workspace, 16) || !espdl::mbconv_s8_split_supports(p) || !espdl::conv2d_s8_units_support(g))
+        return espdl_hip_mbconv_s8(desc, in, w, residual, out, stream);
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    const int cus = cu_count_cached();
+    int8_t *mid = static_cast<int8_t *>(workspace);
+    hipError_t e = espdl::launch_mbconv_s8_expand_dw(p, mid, cus, s);
+    if (e == hipSuccess) {
+        float us;
+        const auto launch = project_launch(g, mid, p.w_project, cus, &us);
+        e = launch(g, mid, p.w_project, p.b_project, p.s_project, nullptr, p.residual, p.out, cus, s);
+    }
+    return device_status(e, "mbconv_s8_ws");
 }
 
 static int binary_s16(int op, const int32_t out_dims[4], const int64_t in0_strides[4], const int64_t in1_strides[4],

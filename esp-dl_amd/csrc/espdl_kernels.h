@@ -17,6 +17,9 @@ struct ConvGeom {
     int relu, half_even, n_shift;
     // channel pitches of input, output and residual operand in elements (>= the channel count; equal: dense)
     int in_pitch, out_pitch, res_pitch;
+    // the residual operand is requantized by 2^res_shift (-7 .. 7) before the Add; only the narrow kernel and the
+    // pointwise GEMM kernel take a value other than 0
+    int res_shift = 0;
 };
 inline bool conv_is_dense(const ConvGeom &g)
 {
@@ -129,6 +132,12 @@ inline bool mbconv_has_clip(const MbconvParams &p)
 {
     return p.clip_e != 0 || p.clip_d != 0;
 }
+// Expand -> depthwise of a block as one launch that writes the depthwise result ([batch][out_h][out_w][exp_c]) to `mid`;
+// p.w_project and p.out are not used (mbconv_s8_split.hip).
+bool mbconv_s8_split_supports(const struct MbconvParams &p);
+float mbconv_s8_expand_dw_us(const struct MbconvParams &p);
+hipError_t launch_mbconv_s8_expand_dw(const struct MbconvParams &p, int8_t *mid, int cu_count, hipStream_t stream);
+
 inline bool mbconv_expand_is_pointwise(const MbconvParams &p)
 {
     return p.ek_h == 1 && p.ek_w == 1 && p.es_h == 1 && p.es_w == 1 && p.epad_top == 0 && p.epad_left == 0 &&
@@ -143,12 +152,14 @@ bool mbconv_s8_wave_supports(const MbconvParams &p);
 // Does the launch take one of the guard-free builds (compiled for the tile plans of MobileNetV2-style blocks)?
 // The guarded builds cover every supported shape but do not beat the separate launches.
 bool mbconv_s8_wave_has_fast_build(const MbconvParams &p);
+float mbconv_s8_wave_us(const MbconvParams &p); // expected time of a guard-free build
 hipError_t launch_mbconv_s8_wave(const MbconvParams &p, int cu_count, hipStream_t stream);
 
 // The same block for small images (output at most 16 pixels wide): a workgroup of eight wavefronts per tile
 // splits the expanded channels (mbconv_s8_group.hip); block-input channels a multiple of 16, at most 192.
 bool mbconv_s8_group_supports(const MbconvParams &p);
 bool mbconv_s8_group_has_fast_build(const MbconvParams &p);
+float mbconv_s8_group_us(const MbconvParams &p, int cu_count); // expected time of a guard-free build
 hipError_t launch_mbconv_s8_group(const MbconvParams &p, int cu_count, hipStream_t stream);
 
 // Depthwise -> 1x1 project [-> Add] in one launch of the LDS-tile depthwise kernel: the depthwise

@@ -21,6 +21,7 @@
 // Two barriers per tile in all; between them eight independent instruction streams per workgroup keep the
 // matrix pipe, the vector ALU and LDS busy.
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <type_traits>
@@ -606,6 +607,20 @@ hipError_t launch_mbconv_s8_group(const MbconvParams &p, int cu_count, hipStream
                       : launch_group_one<9, 3, kGroupPtMax, 2, false, false>(plan, stream);
     return s == 1 ? launch_group_one<9, 3, kGroupPtMax, 1, true, false>(plan, stream)
                   : launch_group_one<9, 3, kGroupPtMax, 2, true, false>(plan, stream);
+}
+
+// A wavefront's share of the expanded channels, then rounds over the device: two workgroups per compute unit for up to
+// 64 input channels, else one (MobileNetV2's blocks at batch 1 to 256, within 15 %).
+float mbconv_s8_group_us(const MbconvParams &p, int cu_count)
+{
+    const GroupPlan plan = group_plan(p);
+    const float chunks = (float)((plan.a.n_sub + kGroupWaves - 1) / kGroupWaves);
+    const float chain = (6.2f + (p.stride_h == 1 ? 1.55f : 0.95f) * chunks) * (1.f + 0.05f * (float)(plan.a.kse - 1)) *
+        (p.half_even ? 1.25f : 1.f);
+    const float fill = (float)((long long)p.batch * plan.a.tiles_y) / (float)(cu_count > 0 ? cu_count : 256);
+    if (fill <= 1.f)
+        return chain;
+    return chain * (plan.a.kse == 1 ? (fill <= 2.f ? 0.5f + 0.5f * fill : 0.75f * fill) : std::ceil(fill));
 }
 
 bool mbconv_s8_group_has_fast_build(const MbconvParams &p)

@@ -50,6 +50,10 @@ public:
     void *get_device_root() { return m_device_root; }
     size_t get_device_size() { return m_device_size; }
     void root_free();
+    /// Scratch memory of at least `bytes` for one launch sequence on the stream (modules use it one after the other), or
+    /// nullptr in the temporary context of Module::run.  It grows during the first pass over a plan and stays.
+    void *workspace(size_t bytes);
+    size_t get_workspace_size() { return m_workspace_size; }
     size_t get_parameter_memory_size();
     size_t get_variable_memory_size();
     void clear();
@@ -57,6 +61,8 @@ public:
 private:
     void *m_device_root = nullptr;
     size_t m_device_size = 0;
+    void *m_workspace = nullptr;
+    size_t m_workspace_size = 0;
     std::map<std::string, int> m_name2index;
 };
 

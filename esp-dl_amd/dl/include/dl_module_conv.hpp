@@ -168,7 +168,7 @@ public:
              m_expand_pads != std::vector<int>{0, 0, 0, 0});
     }
     /// answer of espdl_hip_mbconv_s8_supported for the fused form at its last forward (0 before the first):
-    /// which single-launch kernel runs it
+    /// which single-launch kernel runs it; 6 when it ran as two launches (espdl_hip_mbconv_s8_ws)
     int fused_kernel() const { return m_fused_kernel; }
     /// Absorb the Add that follows a dense Conv: `residual_index` is the Add's other operand and
     /// `own_out_exponent` the exponent of the tensor the Conv used to write.  The Add sums stored integers
@@ -461,9 +461,14 @@ public:
         w.w_project = static_cast<const int8_t *>(pfilter->data);
         w.b_project = pbias ? static_cast<const int32_t *>(pbias->data) : nullptr;
         w.s_project = m_shift_project.sync(s_pj);
-        const int rc = espdl_hip_mbconv_s8(&d, static_cast<const int8_t *>(input->data), &w,
-                                           residual ? static_cast<const int8_t *>(residual->data) : nullptr,
-                                           static_cast<int8_t *>(output->data), context->stream);
+        // few images: expand -> depthwise and project as two launches with the depthwise result in a workspace
+        const int64_t ws_bytes = espdl_hip_mbconv_s8_workspace(&d);
+        void *ws = ws_bytes > 0 ? context->workspace((size_t)ws_bytes) : nullptr;
+        if (ws)
+            m_fused_kernel = 6;
+        const int rc = espdl_hip_mbconv_s8_ws(&d, static_cast<const int8_t *>(input->data), &w,
+                                              residual ? static_cast<const int8_t *>(residual->data) : nullptr, ws,
+                                              static_cast<int8_t *>(output->data), context->stream);
         if (rc != ESPDL_HIP_OK)
             DL_LOGE("Conv", "%s: %s", name.c_str(), espdl_hip_last_error());
     }

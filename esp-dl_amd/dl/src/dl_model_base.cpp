@@ -396,6 +396,7 @@ void Model::fuse_dw_project()
         dl::module::Conv *ex = nullptr;
         dl::module::Clip *clip_e = nullptr;
         int ex_kernel[2] = {1, 1};
+        bool two_launches = false;
         espdl_hip_mbconv_desc de = d; // the whole block, when a Conv in front joins
         {
             int dw_in = dw->m_inputs_index[0];
@@ -466,8 +467,12 @@ void Model::fuse_dw_project()
                     de.exp_pad_left = ex->get_pads()[2];
                     de.exp_pad_right = ex->get_pads()[3];
                 }
-                if (espdl_hip_mbconv_s8_preferred(&de) != 1)
-                    ex = nullptr;
+                // one launch, or two (expand + depthwise, project) where that beats separate launches
+                if (espdl_hip_mbconv_s8_preferred(&de) != 1) {
+                    two_launches = espdl_hip_mbconv_s8_supported(&de) != 0 && espdl_hip_mbconv_s8_workspace(&de) > 0;
+                    if (!two_launches)
+                        ex = nullptr;
+                }
             }
             if (!ex)
                 clip_e = nullptr; // a Clip in front of a depthwise Conv that stays on its own stays too
@@ -480,7 +485,8 @@ void Model::fuse_dw_project()
         int residual = -1;
         size_t add_pos = 0;
         dl::module::Add *add = nullptr;
-        if (single_reader(out_index, &add_pos) && add_pos > pj_pos) {
+        // (in the two-launch form the Add belongs to the project convolution's epilogue)
+        if ((!two_launches || (m_fuse & FUSE_CONV_ADD) != 0) && single_reader(out_index, &add_pos) && add_pos > pj_pos) {
             add = plain_add(m_execution_plan[add_pos]);
             if (add && add->quant_type == QUANT_TYPE_SYMM_8BIT && add->m_inputs_index.size() == 2 &&
                 add->m_inputs_index[0] != add->m_inputs_index[1]) {
@@ -1302,10 +1308,10 @@ std::vector<module_info> Model::get_module_info(int repeats)
         mi.type = m_fbs_model->get_operation_type(module->name);
         if (auto *conv = dynamic_cast<dl::module::Conv *>(module)) {
             // a Conv that absorbed its neighbours reports what it runs
-            // and, after a colon, which single-launch kernel took it (the espdl_hip_mbconv_s8_supported answer)
-            static const char *const kKernel[] = {"", ":fused", ":lds", ":lds", ":wave", ":group"};
+            // and, after a colon, which single-launch kernel took it (the espdl_hip_mbconv_s8_supported answer; split: two launches)
+            static const char *const kKernel[] = {"", ":fused", ":lds", ":lds", ":wave", ":group", ":split"};
             const int k = conv->fused_kernel();
-            const char *suffix = k >= 0 && k <= 5 ? kKernel[k] : "";
+            const char *suffix = k >= 0 && k <= 6 ? kKernel[k] : "";
             if (conv->has_fused_expand())
                 mi.type = std::string("Conv>DepthwiseConv>Conv") + suffix;
             else if (conv->has_fused_project())

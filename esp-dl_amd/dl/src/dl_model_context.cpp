@@ -104,6 +104,25 @@ void ModelContext::root_free()
     }
 }
 
+void *ModelContext::workspace(size_t bytes)
+{
+    if (!owns_tensors)
+        return nullptr;
+    if (bytes > m_workspace_size) {
+        void *grown = nullptr;
+        // launches that use the smaller one may still be running
+        if (hipStreamSynchronize(static_cast<hipStream_t>(stream)) != hipSuccess || hipMalloc(&grown, bytes) != hipSuccess) {
+            (void)hipGetLastError(); // the caller does without
+            return nullptr;
+        }
+        if (m_workspace)
+            (void)hipFree(m_workspace);
+        m_workspace = grown;
+        m_workspace_size = bytes;
+    }
+    return m_workspace;
+}
+
 size_t ModelContext::get_parameter_memory_size()
 {
     size_t total = 0;
@@ -127,6 +146,10 @@ void ModelContext::clear()
             delete t;
     }
     root_free();
+    if (m_workspace)
+        (void)hipFree(m_workspace);
+    m_workspace = nullptr;
+    m_workspace_size = 0;
     m_variables.assign(1, nullptr);
     m_parameters.assign(1, nullptr);
     m_name2index.clear();

@@ -440,6 +440,18 @@ int espdl_hip_mbconv_s8(const espdl_hip_mbconv_desc *desc, const int8_t *in, con
                         const int8_t *residual, int8_t *out, void *stream);
 
 /*
+ * The same block in one or two launches, whichever is expected to be faster: with few images (or few tiles) the single
+ * launch leaves most of the device idle, and expand + depthwise as one launch, project (+ Add) as another, with the
+ * depthwise result in `workspace`, take half of its time.  espdl_hip_mbconv_s8_workspace() answers the workspace bytes
+ * of the two-launch form (16-byte aligned device memory, free between calls that are ordered on a stream) where that
+ * form is the faster one, 0 elsewhere; with workspace NULL espdl_hip_mbconv_s8_ws() is espdl_hip_mbconv_s8().
+ * Results are bit-identical.
+ */
+int64_t espdl_hip_mbconv_s8_workspace(const espdl_hip_mbconv_desc *desc);
+int espdl_hip_mbconv_s8_ws(const espdl_hip_mbconv_desc *desc, const int8_t *in, const espdl_hip_mbconv_weights *weights,
+                           const int8_t *residual, void *workspace, int8_t *out, void *stream);
+
+/*
  * The same block as espdl_hip_mbconv_s8, run as its separate stages ([1x1 Conv] -> depthwise Conv ->
  * 1x1 Conv [+ Add]: espdl_hip_conv2d, espdl_hip_conv2d, espdl_hip_conv2d_add on `stream`) with the two
  * intermediate activations in device memory that belongs to the library.  It has no counterpart in the

@@ -1209,6 +1209,67 @@ def test_mbconv_s8_guard_free_builds_ragged_tiles(oracle, case):
     np.testing.assert_array_equal(to_host(got), cur)
 
 
+# The block as two launches (expand + depthwise, then project): tiles of 7 x 14, 7 x 7 and, at stride 2, 4 x 7 outputs with
+# ragged last rows and columns, one to three reduction steps of block-input channels (also 4 and 20: units that end
+# inside a pixel), expanded channels that leave a group of 64 unfinished, Clips, a requantized residual operand, shifts
+# outside the short epilogue.  (name, (N, H, W, Cin), Ce, Cout, stride, residual, half_even, extra)
+TWO_LAUNCHES = [
+    ("14x14_64_384_64_res", (2, 14, 14, 64), 384, 64, 1, True, False, ""),
+    ("14x14_96_576_96_halfeven", (1, 14, 14, 96), 576, 96, 1, True, True, ""),
+    ("7x7_160_960_160_res", (3, 7, 7, 160), 960, 160, 1, True, False, ""),
+    ("5x6_160_960_320", (2, 5, 6, 160), 960, 320, 1, False, False, ""),
+    ("56x56_24_144_24_res", (1, 56, 56, 24), 144, 24, 1, True, False, ""),
+    ("30x37_16_96_24_s2", (2, 30, 37, 16), 96, 24, 2, False, False, ""),
+    ("15x13_96_576_160_s2_halfeven", (2, 15, 13, 96), 576, 160, 2, False, True, ""),
+    ("9x23_20_16_4", (1, 9, 23, 20), 16, 4, 1, False, False, ""),
+    ("1x1_4_48_12", (5, 1, 1, 4), 48, 12, 1, False, False, ""),
+    ("14x15_192_80_36", (1, 14, 15, 192), 80, 36, 1, False, False, "general"),
+    ("8x8_32_192_32_clips", (2, 8, 8, 32), 192, 32, 1, True, False, "clip"),
+    ("20x20_24_144_24_clips_halfeven", (2, 20, 20, 24), 144, 24, 1, True, True, "clip"),
+    ("14x14_64_384_64_residual_shift", (2, 14, 14, 64), 384, 64, 1, True, False, "shift-3"),
+    ("12x12_32_192_32_residual_shift", (60, 12, 12, 32), 192, 32, 1, True, False, "shift2"),
+]
+
+
+@pytest.mark.parametrize("case", TWO_LAUNCHES, ids=lambda c: c[0])
+def test_mbconv_s8_two_launches(oracle, case):
+    announce(f"mbconv_s8 as two launches: {case[0]}")
+    import torch
+    name, (n, h, w, cin), ce, cout, stride, with_res, half_even, extra = case
+    m = espdl()
+    rng = np.random.default_rng(0x2A + len(name))
+    rm_o = oracle.ROUND_HALF_EVEN if half_even else oracle.ROUND_HALF_UP
+    oracle.set_threads(16)
+
+    def stage(oc, kk, fshape):
+        shift = (typical_shift(kk) + rng.integers(-2, 3, size=oc)).astype(np.int32)
+        if extra == "general":
+            shift[::5] = 0
+        return rng_int8(rng, fshape), rng.integers(-4096, 4097, size=oc).astype(np.int32), shift
+
+    x = rng_int8(rng, (n, h, w, cin))
+    ex, dw, pj = stage(ce, cin, (ce, 1, 1, cin)), stage(ce, 9, (3, 3, ce)), stage(cout, ce, (cout, 1, 1, ce))
+    pads = (1, 1, 1, 1)
+    clips = ((-5, 90), (0, 77)) if extra == "clip" else (None, None)
+    one = ((1, 1), (1, 1), (1, 1), (0, 0, 0, 0))
+    cur = oracle.conv2d_s8(x, ex[0], ex[1], ex[2], *one, oracle.LINEAR if clips[0] else oracle.RELU, rm_o)
+    cur = oracle.clip_s8(cur, *clips[0]) if clips[0] else cur
+    cur = oracle.depthwise_s8(cur, dw[0], dw[1], dw[2], (3, 3), (stride, stride), (1, 1), pads, oracle.RELU, rm_o)
+    cur = oracle.clip_s8(cur, *clips[1]) if clips[1] else cur
+    ws = torch.empty(cur.size, dtype=torch.int8, device="cuda")
+    want = oracle.conv2d_s8(cur, pj[0], pj[1], pj[2], *one, oracle.LINEAR, rm_o)
+    res, d = None, int(extra[5:]) if extra.startswith("shift") else 0
+    if with_res:
+        res = rng_int8(rng, want.shape)
+        want = oracle.add_s8(want, oracle.requantize_s8(res, d, 0) if d else res)
+    dev = lambda t: tuple(to_dev(a) for a in t)  # noqa: E731
+    got = m.mbconv_s8(to_dev(x), dev(ex), dev(dw), dev(pj), (3, 3), (stride, stride), (1, 1), pads, (not clips[0], True, False),
+                      residual=to_dev(res), round_mode=m.capi.ROUND_HALF_EVEN if half_even else m.capi.ROUND_HALF_UP,
+                      residual_shift=d, clip_expand=clips[0], clip_dw=clips[1], workspace=ws)
+    np.testing.assert_array_equal(to_host(ws).reshape(cur.shape), cur)  # the workspace holds the depthwise result
+    np.testing.assert_array_equal(to_host(got), want)
+
+
 # 1x1 convolution followed by GlobalAveragePool in one launch against the two operators of the oracle: the head of
 # MobileNetV2 (7 x 7 x 320 -> 1280), an image of 64 pixels, one of 1 pixel, a filter count that is no multiple of
 # 64, both rounding modes, a linear convolution, shifts outside the short epilogue's range, and a batch large
