@@ -38,6 +38,13 @@ class MbconvDesc(ctypes.Structure):
         "clip_dw_min", "clip_dw_max")]
 
 
+class AttentionDesc(ctypes.Structure):
+    """espdl_hip_attention_desc"""
+    _fields_ = [(n, ctypes.c_int32) for n in (
+        "batch", "heads", "positions", "channels", "head_pitch", "key_dim", "head_dim", "q_offset", "k_offset", "v_offset",
+        "qk_shift", "qk_activation", "mul_shift", "softmax_exp", "prob_exp", "av_shift", "av_activation", "round_mode")]
+
+
 class MbconvWeights(ctypes.Structure):
     """espdl_hip_mbconv_weights"""
     _fields_ = [(n, ctypes.c_void_p) for n in (
@@ -124,6 +131,8 @@ def lib():
         L.espdl_hip_softmax_s8.argtypes = [vp, i64, i64, i64, i32, vp, vp]
         L.espdl_hip_quantize_f32.argtypes = [vp, i64, i32, i32, vp, vp]
         L.espdl_hip_dequantize_f32.argtypes = [vp, i64, i32, i32, vp, vp]
+        L.espdl_hip_attention_s8.argtypes = [ctypes.POINTER(AttentionDesc), vp, vp, vp, vp, vp]
+        L.espdl_hip_attention_s8.restype = ctypes.c_int
         L.espdl_hip_matmul_s8.argtypes = [vp, vp, i32, i32, i32, vp, vp, vp, i32, i32, i32, vp, vp]
         for name in ("concat", "copy_rows", "transpose", "resize_nearest_s8", "max_pool", "avg_pool_s8", "slice",
                      "reduce_mean_s8", "softmax_s8", "quantize_f32", "dequantize_f32", "matmul_s8"):
@@ -544,6 +553,20 @@ def matmul_s8(a, b, shift, activation=0, round_mode=0, stream=None):
                                      (ctypes.c_int64 * 2)(*strides(la, m * k)), (ctypes.c_int64 * 2)(*strides(lb, k * n)),
                                      shift, activation, round_mode, _p(out), _stream(stream)))
     return out
+
+
+def attention_s8(qkv, heads, key_dim, head_dim, qk_shift, softmax_exp, prob_exp, av_shift, mul_constant=None, mul_shift=0,
+                 activations=(0, 0), round_mode=0, stream=None):
+    """qkv [N, H, W, heads * (2 key_dim + head_dim)] -> (feature map, v), both [N, H, W, heads * head_dim]
+    (espdl_hip_attention_s8; a head's channels are q, k, v in this order)."""
+    import torch
+    n, h, w, c = (int(d) for d in qkv.shape)
+    d = AttentionDesc(n, heads, h * w, c, 2 * key_dim + head_dim, key_dim, head_dim, 0, key_dim, 2 * key_dim, qk_shift,
+                      activations[0], mul_shift, softmax_exp, prob_exp, av_shift, activations[1], round_mode)
+    out = torch.empty((n, h, w, heads * head_dim), dtype=torch.int8, device=qkv.device)
+    v = torch.empty_like(out)
+    _check(lib().espdl_hip_attention_s8(ctypes.byref(d), _p(qkv), _p(mul_constant), _p(out), _p(v), _stream(stream)))
+    return out, v
 
 
 def lut_s16(x, table, round_mode=0, stream=None):

@@ -1562,4 +1562,70 @@ int espdl_hip_matmul_s8(const int8_t *a, const int8_t *b, int32_t m, int32_t k, 
                          "matmul_s8");
 }
 
+static espdl::AttentionParams attention_params(const espdl_hip_attention_desc &d)
+{
+    espdl::AttentionParams p = {};
+    p.batch = d.batch;
+    p.heads = d.heads;
+    p.positions = d.positions;
+    p.channels = d.channels;
+    p.head_pitch = d.head_pitch;
+    p.key_dim = d.key_dim;
+    p.head_dim = d.head_dim;
+    p.q_offset = d.q_offset;
+    p.k_offset = d.k_offset;
+    p.v_offset = d.v_offset;
+    p.qk_shift = d.qk_shift;
+    p.qk_relu = d.qk_activation == ESPDL_HIP_RELU;
+    p.mul_shift = d.mul_shift;
+    p.softmax_exp = d.softmax_exp;
+    p.prob_exp = d.prob_exp;
+    p.av_shift = d.av_shift;
+    p.av_relu = d.av_activation == ESPDL_HIP_RELU;
+    p.half_even = d.round_mode == ESPDL_HIP_ROUND_HALF_EVEN;
+    return p;
+}
+
+int espdl_hip_attention_s8_supported(const espdl_hip_attention_desc *desc)
+{
+    return desc != nullptr && desc->q_offset >= 0 && desc->k_offset >= 0 && desc->v_offset >= 0 &&
+        espdl::attention_s8_supports(attention_params(*desc));
+}
+
+int espdl_hip_attention_s8(const espdl_hip_attention_desc *desc, const int8_t *qkv, const int8_t *mul_constant, int8_t *out,
+                           int8_t *v_out, void *stream)
+{
+    if (desc == nullptr)
+        return fail(ESPDL_HIP_EINVAL, "desc must not be NULL");
+    const espdl_hip_attention_desc &d = *desc;
+    if (d.batch < 0)
+        return fail(ESPDL_HIP_EINVAL, "negative extent");
+    for (int act : {d.qk_activation, d.av_activation})
+        if (act != ESPDL_HIP_LINEAR && act != ESPDL_HIP_RELU)
+            return fail(ESPDL_HIP_EINVAL, "activations must be ESPDL_HIP_LINEAR or ESPDL_HIP_RELU");
+    if (d.round_mode != ESPDL_HIP_ROUND_HALF_UP && d.round_mode != ESPDL_HIP_ROUND_HALF_EVEN)
+        return fail(ESPDL_HIP_EINVAL, "unknown round mode %d", d.round_mode);
+    for (int shift : {d.qk_shift, d.av_shift})
+        if (shift < -31 || shift > 62)
+            return fail(ESPDL_HIP_EINVAL, "shift %d outside [-31, 62]", shift);
+    if (mul_constant != nullptr && (d.mul_shift < -60 || d.mul_shift > 60))
+        return fail(ESPDL_HIP_EINVAL, "mul_shift %d outside [-60, 60]", d.mul_shift);
+    if (check_exps(d.softmax_exp, d.prob_exp) != ESPDL_HIP_OK)
+        return ESPDL_HIP_EINVAL;
+    if (!espdl_hip_attention_s8_supported(desc))
+        return fail(ESPDL_HIP_ENOTSUP, "no attention kernel for these sizes");
+    if (d.batch == 0)
+        return ESPDL_HIP_OK;
+    if (qkv == nullptr || out == nullptr)
+        return fail(ESPDL_HIP_EINVAL, "qkv and out must not be NULL");
+    if (misaligned(qkv, 16) || misaligned(out, 16) || (v_out && misaligned(v_out, 16)))
+        return fail(ESPDL_HIP_EINVAL, "qkv, out and v_out must be 16-byte aligned");
+    espdl::AttentionParams p = attention_params(d);
+    p.qkv = qkv;
+    p.mul_constant = mul_constant;
+    p.out = out;
+    p.v_out = v_out;
+    return device_status(espdl::launch_attention_s8(p, reinterpret_cast<hipStream_t>(stream)), "attention_s8");
+}
+
 } // extern "C"

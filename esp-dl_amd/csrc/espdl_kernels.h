@@ -282,4 +282,17 @@ hipError_t launch_matmul_s8(const int8_t *a, const int8_t *b, int m, int k, int 
                             const long long a_stride[2], const long long b_stride[2], int shift, bool relu, bool half_even,
                             int8_t *out, hipStream_t stream);
 
+// attention_s8.hip
+struct AttentionParams {
+    int batch, heads, positions;
+    int channels, head_pitch;         // of qkv per position, of one head's q, k and v together
+    int key_dim, head_dim;
+    int q_offset, k_offset, v_offset; // inside a head's channels
+    int qk_shift, qk_relu, mul_shift, softmax_exp, prob_exp, av_shift, av_relu, half_even;
+    const int8_t *qkv, *mul_constant; // mul_constant may be nullptr
+    int8_t *out, *v_out;              // v_out may be nullptr
+};
+bool attention_s8_supports(const AttentionParams &p);
+hipError_t launch_attention_s8(const AttentionParams &p, hipStream_t stream);
+
 } // namespace espdl

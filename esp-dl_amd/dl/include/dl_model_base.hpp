@@ -27,7 +27,8 @@ struct module_info {
     int64_t bytes;    ///< bytes of the tensors it reads and writes (each counted once)
 };
 
-enum { FUSE_CONV_LUT = 1, FUSE_DW_PROJECT = 2, FUSE_CONV_ADD = 4, FUSE_CONV_GAP = 8, FUSE_CHANNEL_SLICES = 16 };
+enum { FUSE_CONV_LUT = 1, FUSE_DW_PROJECT = 2, FUSE_CONV_ADD = 4, FUSE_CONV_GAP = 8, FUSE_CHANNEL_SLICES = 16,
+       FUSE_ATTENTION = 32 };
 
 class Model {
 public:
@@ -37,10 +38,12 @@ public:
     /// FUSE_CONV_ADD folds the Add behind a dense Conv into its epilogue, FUSE_CONV_GAP runs a 1x1 Conv and the
     /// GlobalAveragePool behind it as one kernel that writes the pooled tensor only, FUSE_CHANNEL_SLICES leaves the
     /// outputs of a Split along the last axis inside its input and lets dense 8-bit Convs write straight into the
-    /// output of a Concat along the last axis (the modules stay in the plan and copy only what is not in place).
+    /// output of a Concat along the last axis (the modules stay in the plan and copy only what is not in place),
+    /// FUSE_ATTENTION runs an attention block between its convolutions as one kernel.
     /// All are exact and on by default.
     Model(fbs::FbsModel *fbs_model, int batch = 1, round_mode_t round_mode = ROUND_MODE_HALF_UP, void *stream = nullptr,
-          int fuse = FUSE_CONV_LUT | FUSE_DW_PROJECT | FUSE_CONV_ADD | FUSE_CONV_GAP | FUSE_CHANNEL_SLICES);
+          int fuse = FUSE_CONV_LUT | FUSE_DW_PROJECT | FUSE_CONV_ADD | FUSE_CONV_GAP | FUSE_CHANNEL_SLICES |
+              FUSE_ATTENTION);
     virtual ~Model();
     Model(const Model &) = delete;
     Model &operator=(const Model &) = delete;
@@ -98,6 +101,7 @@ private:
     void fuse_dw_project();
     void fuse_conv_add();
     void fuse_conv_gap();
+    void fuse_attention();
     size_t plan_bytes();
 
     fbs::FbsModel *m_fbs_model = nullptr;
@@ -107,7 +111,8 @@ private:
     std::string m_name, m_doc_string;
     int64_t m_version = 0;
     int m_batch = 1;
-    int m_fuse = FUSE_CONV_LUT | FUSE_DW_PROJECT | FUSE_CONV_ADD | FUSE_CONV_GAP | FUSE_CHANNEL_SLICES;
+    int m_fuse = FUSE_CONV_LUT | FUSE_DW_PROJECT | FUSE_CONV_ADD | FUSE_CONV_GAP | FUSE_CHANNEL_SLICES |
+        FUSE_ATTENTION;
     void *m_stream = nullptr;
     bool m_own_stream = false;
     void *m_graph = nullptr;      // hipGraph_t

@@ -224,6 +224,8 @@ public:
             DL_LOGE("MatMul", "%s: %s", name.c_str(), espdl_hip_last_error());
     }
 
+    activation_type_t get_activation() const { return m_activation; }
+
     static Module *deserialize(fbs::FbsModel *fbs_model, std::string node_name)
     {
         activation_type_t activation_type = Linear;

@@ -296,6 +296,7 @@ public:
         if (rc != ESPDL_HIP_OK)
             DL_LOGE("Transpose", "%s: %s", name.c_str(), espdl_hip_last_error());
     }
+    const std::vector<int> &get_perm() const { return m_perm; }
     static Module *deserialize(fbs::FbsModel *fbs_model, std::string node_name)
     {
         quant_type_t quant_type = QUANT_TYPE_NONE;
@@ -1259,6 +1260,7 @@ public:
         if (rc != ESPDL_HIP_OK)
             DL_LOGE("Softmax", "%s: %s", name.c_str(), espdl_hip_last_error());
     }
+    int get_axis() const { return m_axis; }
     static Module *deserialize(fbs::FbsModel *fbs_model, std::string node_name)
     {
         quant_type_t quant_type = QUANT_TYPE_NONE;

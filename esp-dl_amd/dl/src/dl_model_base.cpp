@@ -8,6 +8,7 @@
 #include <set>
 #include <typeinfo>
 
+#include "dl_module_attention.hpp"
 #include "dl_module_creator.hpp"
 
 namespace dl {
@@ -243,6 +244,8 @@ esp_err_t Model::load(fbs::FbsModel *fbs_model)
         fuse_conv_add();
     if (ret == ESP_OK && (m_fuse & FUSE_CONV_GAP))
         fuse_conv_gap();
+    if (ret == ESP_OK && (m_fuse & FUSE_ATTENTION))
+        fuse_attention();
     return ret;
 }
 
@@ -679,6 +682,187 @@ void Model::fuse_conv_add()
         m_execution_plan[add_pos] = conv;
         m_execution_plan.erase(m_execution_plan.begin() + i);
         i--;
+    }
+}
+
+// The chain between the 1x1 Conv that leaves q, k and v of an attention block and the block's feature map:
+//   qkv -> Transpose to channels first -> Reshape [1, heads, ., n] -> Split into q, k, v along the channels
+//   Transpose(q) x k -> [Mul by one constant] -> Softmax -> QuantizeLinear -> Transpose, v x that -> Reshape ->
+//   Transpose to channels last, and beside it possibly v -> Reshape -> Transpose to channels last
+// Found from its Softmax.  When every tensor in between has no other reader and nobody asks for it, one module with the
+// same results takes the place of the chain's first module: all it needs, qkv and a constant, exists there.
+void Model::fuse_attention()
+{
+    using namespace dl::module;
+    std::set<std::string> pinned;
+    for (auto &n : m_fbs_model->get_graph_outputs())
+        pinned.insert(n);
+    for (auto &n : m_fbs_model->get_test_outputs_name())
+        pinned.insert(n);
+    const auto name_of = [&](int tensor) { return m_model_context->get_tensor_name(tensor); };
+    const auto shape_of = [&](int tensor) { return m_fbs_model->get_value_info_shape(name_of(tensor)); };
+    const auto exp_of = [&](int tensor) { return m_fbs_model->get_value_info_exponent(name_of(tensor)); };
+    const auto producer = [&](int tensor) -> Module * {
+        for (Module *m : m_execution_plan)
+            if (std::count(m->m_outputs_index.begin(), m->m_outputs_index.end(), tensor))
+                return m;
+        return nullptr;
+    };
+    // the modules that read a tensor; none when it has to stay
+    const auto readers = [&](int tensor) {
+        std::vector<Module *> all;
+        if (pinned.count(name_of(tensor)) || !m_fbs_model->has_value_info(name_of(tensor)))
+            return all;
+        for (Module *m : m_execution_plan)
+            for (int in : m->m_inputs_index)
+                if (in == tensor)
+                    all.push_back(m);
+        return all;
+    };
+    const auto sole_reader = [&](int tensor) -> Module * {
+        const std::vector<Module *> all = readers(tensor);
+        return all.size() == 1 ? all[0] : nullptr;
+    };
+    const auto transposes = [&](Module *m, const std::vector<int> &perm) {
+        auto *t = dynamic_cast<Transpose *>(m);
+        return t && t->get_perm() == perm;
+    };
+    // v or the product as [1, heads, head_dim, n] -> Reshape -> Transpose to [1, H, W, heads * head_dim]: the two modules
+    const auto to_map = [&](Module *m, const std::vector<int> &qkv_shape, int channels, std::vector<Module *> *taken) {
+        if (!dynamic_cast<ShapeView *>(m) || shape_of(m->m_outputs_index[0]) != std::vector<int>{1, channels, qkv_shape[1], qkv_shape[2]})
+            return -1;
+        Module *t = sole_reader(m->m_outputs_index[0]);
+        if (!transposes(t, {0, 2, 3, 1}) || !m_fbs_model->has_value_info(name_of(t->m_outputs_index[0])))
+            return -1;
+        taken->push_back(m);
+        taken->push_back(t);
+        return t->m_outputs_index[0];
+    };
+    const std::vector<int> swap_last = {0, 1, 3, 2};
+    for (size_t at = 0; at < m_execution_plan.size(); at++) {
+        auto *softmax = dynamic_cast<Softmax *>(m_execution_plan[at]);
+        if (!softmax || softmax->quant_type != QUANT_TYPE_SYMM_8BIT)
+            continue;
+        std::vector<Module *> taken = {softmax};
+        const int x = softmax->m_inputs_index[0];
+        const std::vector<int> score_shape = shape_of(x);
+        if (score_shape.size() != 4 || (softmax->get_axis() != 3 && softmax->get_axis() != -1) || sole_reader(x) != softmax)
+            continue;
+        // in front: [Mul by a one-element constant], MatMul
+        int score = x, constant = -1;
+        Module *m = producer(x);
+        if (m && typeid(*m) == typeid(Mul) && m->m_inputs_index.size() == 2 && m->quant_type == QUANT_TYPE_SYMM_8BIT) {
+            taken.push_back(m);
+            const int side = m->m_inputs_index[0] >= CONTEXT_PARAMETER_OFFSET ? 0 : 1;
+            constant = m->m_inputs_index[side];
+            score = m->m_inputs_index[1 - side];
+            TensorBase *c = constant >= CONTEXT_PARAMETER_OFFSET ? m_model_context->get_tensor(constant) : nullptr;
+            if (!c || c->dtype != DATA_TYPE_INT8 || c->get_size() != 1 || score >= CONTEXT_PARAMETER_OFFSET || sole_reader(score) != m)
+                continue;
+            m = producer(score);
+        }
+        auto *qk = dynamic_cast<MatMul *>(m);
+        if (!qk || qk->quant_type != QUANT_TYPE_SYMM_8BIT || shape_of(score) != score_shape)
+            continue;
+        taken.push_back(qk);
+        const int qt = qk->m_inputs_index[0], k = qk->m_inputs_index[1];
+        Module *q_transpose = producer(qt);
+        if (!transposes(q_transpose, swap_last) || sole_reader(qt) != qk || sole_reader(k) != qk)
+            continue;
+        taken.push_back(q_transpose);
+        const int q = q_transpose->m_inputs_index[0];
+        // behind: QuantizeLinear, Transpose, MatMul, Reshape, Transpose
+        const int f = softmax->m_outputs_index[0];
+        Module *quantize = sole_reader(f);
+        if (!quantize || typeid(*quantize) != typeid(RequantizeLinear) ||
+            m_fbs_model->get_value_info_dtype(name_of(quantize->m_outputs_index[0])) != DATA_TYPE_INT8)
+            continue;
+        taken.push_back(quantize);
+        const int prob = quantize->m_outputs_index[0];
+        Module *p_transpose = sole_reader(prob);
+        if (!transposes(p_transpose, swap_last))
+            continue;
+        taken.push_back(p_transpose);
+        const int pt = p_transpose->m_outputs_index[0];
+        auto *av = dynamic_cast<MatMul *>(sole_reader(pt));
+        if (!av || av->quant_type != QUANT_TYPE_SYMM_8BIT || av->m_inputs_index[1] != pt || av->m_inputs_index[0] == pt)
+            continue;
+        taken.push_back(av);
+        const int v = av->m_inputs_index[0], product = av->m_outputs_index[0];
+        // q, k and v are the pieces of one Split of the channels-first tensor
+        auto *split = dynamic_cast<Split *>(producer(q));
+        if (!split || split != producer(k) || split != producer(v) || split->m_outputs_index.size() != 3 || q == k || q == v || k == v ||
+            sole_reader(q) != q_transpose)
+            continue;
+        taken.push_back(split);
+        const std::vector<int> heads_shape = shape_of(split->m_inputs_index[0]);
+        Module *view = producer(split->m_inputs_index[0]);
+        if (heads_shape.size() != 4 || (split->get_axis() != 2 && split->get_axis() != -2) || !dynamic_cast<ShapeView *>(view) ||
+            sole_reader(split->m_inputs_index[0]) != split)
+            continue;
+        taken.push_back(view);
+        Module *nchw = producer(view->m_inputs_index[0]);
+        if (!transposes(nchw, {0, 3, 1, 2}) || sole_reader(view->m_inputs_index[0]) != view)
+            continue;
+        taken.push_back(nchw);
+        const int qkv = nchw->m_inputs_index[0];
+        const std::vector<int> in = shape_of(qkv);
+        if (qkv >= CONTEXT_PARAMETER_OFFSET || !m_fbs_model->has_value_info(name_of(qkv)) || in.size() != 4 || in[0] != 1 ||
+            m_fbs_model->get_value_info_dtype(name_of(qkv)) != DATA_TYPE_INT8)
+            continue;
+        espdl_hip_attention_desc d = {};
+        d.batch = 1;
+        d.heads = heads_shape[1];
+        d.positions = in[1] * in[2];
+        d.channels = in[3];
+        d.head_pitch = heads_shape[2];
+        if (heads_shape[0] != 1 || heads_shape[3] != d.positions || d.heads * d.head_pitch != d.channels ||
+            score_shape != std::vector<int>{1, d.heads, d.positions, d.positions})
+            continue;
+        int channel = 0;
+        for (int piece : split->m_outputs_index) {
+            (piece == q ? d.q_offset : piece == k ? d.k_offset : d.v_offset) = channel;
+            channel += shape_of(piece).size() == 4 ? shape_of(piece)[2] : 0;
+        }
+        d.key_dim = shape_of(q).size() == 4 ? shape_of(q)[2] : 0;
+        d.head_dim = shape_of(v).size() == 4 ? shape_of(v)[2] : 0;
+        if (channel != d.head_pitch || shape_of(k) != shape_of(q))
+            continue;
+        const int out = [&] {
+            Module *reshape = sole_reader(product);
+            return reshape ? to_map(reshape, in, d.heads * d.head_dim, &taken) : -1;
+        }();
+        if (out < 0)
+            continue;
+        const std::vector<Module *> v_readers = readers(v);
+        int v_map = -1;
+        if (v_readers.size() == 2)
+            v_map = to_map(v_readers[v_readers[0] == av ? 1 : 0], in, d.heads * d.head_dim, &taken);
+        if (v_readers.empty() || v_readers.size() > 2 || (v_readers.size() == 2 && v_map < 0))
+            continue;
+        d.qk_shift = exp_of(score) - exp_of(qt) - exp_of(k);
+        d.qk_activation = qk->get_activation() == ReLU ? ESPDL_HIP_RELU : ESPDL_HIP_LINEAR;
+        if (constant >= 0)
+            d.mul_shift = exp_of(x) - exp_of(score) - m_model_context->get_tensor(constant)->exponent.get();
+        d.softmax_exp = exp_of(x);
+        d.prob_exp = exp_of(prob);
+        d.av_shift = exp_of(product) - exp_of(v) - exp_of(pt);
+        d.av_activation = av->get_activation() == ReLU ? ESPDL_HIP_RELU : ESPDL_HIP_LINEAR;
+        if (espdl_hip_attention_s8_supported(&d) != 1)
+            continue;
+        auto *fused = new Attention(softmax->name.c_str(), d);
+        fused->m_inputs_index.push_back(qkv);
+        if (constant >= 0)
+            fused->m_inputs_index.push_back(constant);
+        fused->m_outputs_index.push_back(out);
+        if (v_map >= 0)
+            fused->m_outputs_index.push_back(v_map);
+        *std::find(m_execution_plan.begin(), m_execution_plan.end(), nchw) = fused;
+        for (Module *t : taken) {
+            m_execution_plan.erase(std::remove(m_execution_plan.begin(), m_execution_plan.end(), t), m_execution_plan.end());
+            delete t;
+        }
+        at = 0; // positions have moved
     }
 }
 
@@ -1316,6 +1500,8 @@ std::vector<module_info> Model::get_module_info(int repeats)
                 mi.type = std::string("Conv>DepthwiseConv>Conv") + suffix;
             else if (conv->has_fused_project())
                 mi.type = std::string("DepthwiseConv>Conv") + suffix;
+        } else if (dynamic_cast<dl::module::Attention *>(module)) {
+            mi.type = "Attention";
         }
         mi.latency_us = (float)std::max(0.0, (total_ms[i] / repeats - gap_ms) * 1000.0);
         std::vector<std::vector<int>> in_shapes;

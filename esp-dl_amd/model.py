@@ -196,11 +196,12 @@ class Model:
     """dl::Model handle.  `stream` is a raw hipStream_t value (e.g. torch.cuda.Stream().cuda_stream) or None."""
 
     def __init__(self, graph, batch, round_mode=0, stream=None, fuse_lut=True, fuse_blocks=True, fuse_add=True,
-                 fuse_gap=True, channel_slices=True):
+                 fuse_gap=True, channel_slices=True, fuse_attention=True):
         self.graph = graph  # keep alive: the native model references it
         self.h = lib().espdl_model_create(graph.h, batch, round_mode, ctypes.c_void_p(stream) if stream else None,
                                           (1 if fuse_lut else 0) | (2 if fuse_blocks else 0) | (4 if fuse_add else 0) |
-                                          (8 if fuse_gap else 0) | (16 if channel_slices else 0))
+                                          (8 if fuse_gap else 0) | (16 if channel_slices else 0) |
+                                          (32 if fuse_attention else 0))
         if not self.h:
             raise EspdlModelError("espdl_model_create failed (see stderr)")
         self.batch = batch

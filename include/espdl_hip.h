@@ -357,6 +357,33 @@ int espdl_hip_matmul_s8(const int8_t *a, const int8_t *b, int32_t m, int32_t k, 
                         const int64_t a_stride[2], const int64_t b_stride[2], int32_t shift, int32_t activation,
                         int32_t round_mode, int8_t *out, void *stream);
 
+/* The core of an attention block on int8 in one launch: what MatMul (q^T x k), Mul by a one-element constant, Softmax,
+ * QuantizeLinear and MatMul (v x attn^T) give one after the other, with the layout changes and the Split around them.
+ * qkv is [batch][positions][channels]; head h owns the channels [h * head_pitch, (h + 1) * head_pitch) of a position, its
+ * q (key_dim channels), k (key_dim) and v (head_dim) at the given offsets inside them.  With n, m positions:
+ *   score[n][m] = MatMul with qk_shift = score_exp - q_exp - k_exp and qk_activation
+ *   x = mul_constant ? requantize(score * *mul_constant, mul_shift) : score     (mul_constant on the device)
+ *   prob = QuantizeLinear(Softmax over m of x * 2^softmax_exp) at exponent prob_exp
+ *   out[batch][n][h * head_dim + d] = MatMul over m of v and prob, with av_shift and av_activation
+ * v_out (or NULL) receives v as [batch][positions][heads * head_dim].  The shifts have the bounds of the
+ * separate operators.
+ * espdl_hip_attention_s8_supported: 1 when the sizes have this kernel (key_dim up to 64, head_dim up to 128, all channel
+ * counts and offsets multiples of 16, at most 1024 positions), 0 when not. */
+typedef struct {
+    int32_t batch, heads, positions;
+    int32_t channels, head_pitch;
+    int32_t key_dim, head_dim;
+    int32_t q_offset, k_offset, v_offset;
+    int32_t qk_shift, qk_activation;
+    int32_t mul_shift;
+    int32_t softmax_exp, prob_exp;
+    int32_t av_shift, av_activation;
+    int32_t round_mode;
+} espdl_hip_attention_desc;
+int espdl_hip_attention_s8_supported(const espdl_hip_attention_desc *desc);
+int espdl_hip_attention_s8(const espdl_hip_attention_desc *desc, const int8_t *qkv, const int8_t *mul_constant, int8_t *out,
+                           int8_t *v_out, void *stream);
+
 /* TensorBase::slice for positive steps (esp-dl/dl/base/dl_base_shape.cpp:68-120 gives the shape rule):
  * out[i0, i1, ...] = in[start[0] + i0 * step[0], start[1] + i1 * step[1], ...].  The caller passes
  * normalized values per dim (0 <= start, step >= 1, out_shape) for all `dims` dims of the input;

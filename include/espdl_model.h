@@ -81,7 +81,8 @@ int espdl_graph_add_test_output(espdl_graph *g, const char *name, const int32_t 
  * depthwise Conv -> 1x1 Conv [-> Add] chains as one kernel, 4 folds the Add behind a dense Conv into the
  * conv epilogue, 8 runs a 1x1 Conv and the GlobalAveragePool behind it as one kernel, 16 keeps the outputs of a
  * Split along the last axis inside its input and lets dense 8-bit Convs write straight into the output of a
- * Concat along the last axis, so that neither copies (31 = all).  The graph must outlive the model. */
+ * Concat along the last axis, so that neither copies, 32 runs an attention block between its convolutions as one
+ * kernel (63 = all).  The graph must outlive the model. */
 espdl_model *espdl_model_create(espdl_graph *g, int32_t batch, int32_t round_mode, void *stream, int32_t fuse);
 void espdl_model_destroy(espdl_model *m);
 /* Module::forward returns void, as in the reference, so a module whose launch is rejected (an operand

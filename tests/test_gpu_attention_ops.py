@@ -291,3 +291,39 @@ def test_div_s8_one_element_operands(oracle):
     assert got[0] == -128
     z16 = np.array([0], np.int16)
     assert to_host(espdl().div_s16(to_dev(z16), to_dev(z16), 0))[0] == 0
+
+
+ATTENTION_CASES = [
+    # (batch, h, w, heads, key_dim, head_dim, qk_shift, mul shift or None, softmax exp, prob exp, av_shift, activations)
+    (2, 20, 20, 2, 32, 64, 9, 7, -3, -8, 8, (0, 0)),
+    (1, 7, 7, 1, 16, 16, 8, None, -4, -9, 7, (0, 0)),      # less than one chunk of keys
+    (3, 8, 8, 3, 32, 48, 9, 6, -3, -7, 8, (0, 1)),         # whole chunks, value tiles partly empty
+    (2, 5, 13, 1, 64, 128, 10, 7, -5, -10, 6, (1, 0)),     # one key and one query past a tile; the widest head
+    (1, 19, 27, 1, 32, 16, 9, 7, -3, -8, 8, (0, 0)),       # one key past eight chunks
+    (1, 1, 3, 2, 48, 32, 0, -1, -4, -7, -2, (0, 0)),       # left shifts: the general epilogue
+    (1, 32, 32, 1, 16, 32, 5, 9, -2, -8, 3, (0, 0)),       # the longest row; small scores, quotients on ties
+]
+
+
+@pytest.mark.parametrize("round_mode", [0, 1], ids=["half_up", "half_even"])
+@pytest.mark.parametrize("case", ATTENTION_CASES, ids=lambda c: f"{c[0]}x{c[1]}x{c[2]}_h{c[3]}_{c[4]}_{c[5]}")
+def test_attention_s8(oracle, case, round_mode):
+    """One launch against the operators it stands for."""
+    n, h, w, heads, kd, hd, qk_shift, mul_shift, e, prob_exp, av_shift, acts = case
+    announce(f"attention_s8 {case} round_mode={round_mode}")
+    rng = np.random.default_rng(47)
+    x = _rand(rng, (n, h, w, heads * (2 * kd + hd)))
+    t = np.ascontiguousarray(np.moveaxis(x.reshape(n, h * w, heads, -1), 1, -1))
+    q, k, v = (np.ascontiguousarray(p) for p in np.split(t, [kd, 2 * kd], axis=2))
+    scores = oracle.matmul_s8(np.ascontiguousarray(np.swapaxes(q, 2, 3)), k, qk_shift, acts[0], round_mode)
+    scores = scores.reshape(n, heads, h * w, h * w)
+    c = np.array([91], np.int8)
+    if mul_shift is not None:
+        scores = oracle.mul_s8(scores, c, mul_shift, round_mode)
+    prob = oracle.quantize_f32(oracle.softmax_s8(scores, -1, e), prob_exp)
+    want = oracle.matmul_s8(v, np.ascontiguousarray(np.swapaxes(prob, 2, 3)), av_shift, acts[1], round_mode)
+    to_map = lambda y: np.moveaxis(y.reshape(n, heads * hd, h, w), 1, -1)
+    out, v_out = espdl().attention_s8(to_dev(x), heads, kd, hd, qk_shift, e, prob_exp, av_shift,
+                                      to_dev(c) if mul_shift is not None else None, mul_shift or 0, acts, round_mode)
+    np.testing.assert_array_equal(to_host(out), to_map(want))
+    np.testing.assert_array_equal(to_host(v_out), to_map(v))

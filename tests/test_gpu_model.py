@@ -390,6 +390,24 @@ def test_attention_block(oracle, round_mode):
     mdl.close()
 
 
+def test_attention_block_is_one_module(oracle):
+    """The modules between the block's convolutions become one; the separate ones give the same bytes."""
+    announce("model attention_block fused and not")
+    _, zoo, model, _ = _mods()
+    spec = zoo.attention_block(hw=9, heads=3)
+    x = spec.make_input(np.random.default_rng(36), 2)
+    outs, counts = [], []
+    for fuse in (False, True):
+        mdl = model.Model(model.Graph.from_spec(spec), 2, fuse_attention=fuse)
+        mdl.set_input(spec.inputs[0], x)
+        mdl.run()
+        outs.append(mdl.get_tensor(spec.outputs[0]))
+        counts.append(mdl.module_count())
+        mdl.close()
+    np.testing.assert_array_equal(outs[0], outs[1])
+    assert counts == [18, 5]
+
+
 @pytest.mark.parametrize("round_mode", [0, 1], ids=["half_up", "half_even"])
 def test_int16_tail(oracle, round_mode):
     """int16 table, Add, Mul by a constant, AveragePool and ReduceMean behind an int8 -> int16 requantize."""
