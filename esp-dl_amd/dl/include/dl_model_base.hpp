@@ -10,6 +10,7 @@
 #pragma once
 
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -79,6 +80,10 @@ public:
     void profile(bool sort_module_by_latency = false);
     mem_info_t get_memory_info();
 
+    /// Copy a whole dense device tensor from / to host memory on the model's stream; done on return.
+    bool write_tensor(TensorBase *tensor, const void *host);
+    bool read_tensor(const TensorBase *tensor, void *host);
+
     virtual std::map<std::string, TensorBase *> &get_inputs() { return m_inputs; }
     virtual TensorBase *get_input();
     virtual TensorBase *get_input(const std::string &name);
@@ -103,6 +108,7 @@ private:
     void fuse_conv_gap();
     void fuse_attention();
     size_t plan_bytes();
+    char *staging(size_t bytes);
 
     fbs::FbsModel *m_fbs_model = nullptr;
     std::vector<dl::module::Module *> m_execution_plan;
@@ -118,6 +124,9 @@ private:
     void *m_graph = nullptr;      // hipGraph_t
     void *m_graph_exec = nullptr; // hipGraphExec_t
     void *m_launches = nullptr;   // the captured kernels of a short plan, replayed without the graph
+    char *m_staging = nullptr;    // pinned host memory of read_tensor / write_tensor
+    size_t m_staging_bytes = 0;
+    std::mutex m_staging_mutex;
     bool m_built = false;
     bool m_failed = false;
     long m_errors_at_start = 0;

@@ -183,6 +183,8 @@ Model::~Model()
         delete m;
     m_execution_plan.clear();
     delete m_model_context;
+    if (m_staging)
+        (void)hipHostFree(m_staging);
     if (m_own_stream && m_stream)
         (void)hipStreamDestroy(static_cast<hipStream_t>(m_stream));
 }
@@ -1251,6 +1253,68 @@ void Model::run(runtime_mode_t mode)
 {
     run_async(mode);
     synchronize();
+}
+
+// Host copies through pinned memory of the model's own, moved by a kernel, where that is faster than what the runtime
+// does with pageable memory.  Reading: the thousand bytes of a classifier's result take 12.6 us instead of 21 us; large
+// results stay with the runtime, which then streams.  Writing: up to 1 MiB the runtime stages the copy itself (12 us for
+// 150 KB, 38 us for 900 KB), above it pins the caller's pages first (61 us for 1.05 MB, 93 us for 2.4 MB); in pieces of
+// 512 KiB, the next one copied while the kernel fetches the last, these take 46 and 75 us.  At 4 MB the two meet.
+static constexpr size_t kReadStaging = 64 << 10;
+static constexpr size_t kWriteFrom = 1 << 20, kWritePiece = 512 << 10, kWriteStaging = 4 << 20;
+
+char *Model::staging(size_t bytes)
+{
+    if (bytes > m_staging_bytes) {
+        if (m_staging)
+            (void)hipHostFree(m_staging);
+        m_staging = nullptr;
+        m_staging_bytes = 0;
+        const size_t size = std::max(bytes, kReadStaging);
+        void *p = nullptr;
+        if (hipHostMalloc(&p, size, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        m_staging = static_cast<char *>(p);
+        m_staging_bytes = size;
+    }
+    return m_staging;
+}
+
+bool Model::read_tensor(const TensorBase *tensor, void *host)
+{
+    const size_t bytes = tensor ? tensor->get_bytes() : 0;
+    if (host && tensor && tensor->on_device() && tensor->is_dense() && bytes <= kReadStaging) {
+        std::lock_guard<std::mutex> lock(m_staging_mutex);
+        if (char *p = staging(bytes)) {
+            if (espdl_hip_copy_rows(tensor->data, (int64_t)bytes, p, (int64_t)bytes, (int64_t)bytes, 1, m_stream) != ESPDL_HIP_OK ||
+                !hip_ok(hipStreamSynchronize(static_cast<hipStream_t>(m_stream)), "hipStreamSynchronize"))
+                return false;
+            memcpy(host, p, bytes);
+            return true;
+        }
+    }
+    return tensor && tensor->copy_to_host(host, bytes, m_stream);
+}
+
+bool Model::write_tensor(TensorBase *tensor, const void *host)
+{
+    const size_t bytes = tensor ? tensor->get_bytes() : 0;
+    if (host && tensor && tensor->on_device() && tensor->is_dense() && bytes > kWriteFrom && bytes <= kWriteStaging) {
+        std::lock_guard<std::mutex> lock(m_staging_mutex);
+        if (char *p = staging(bytes)) {
+            for (size_t at = 0; at < bytes; at += kWritePiece) {
+                const size_t n = std::min(kWritePiece, bytes - at);
+                memcpy(p + at, static_cast<const char *>(host) + at, n);
+                if (espdl_hip_copy_rows(p + at, (int64_t)n, static_cast<char *>(tensor->data) + at, (int64_t)n, (int64_t)n, 1,
+                                        m_stream) != ESPDL_HIP_OK)
+                    return false;
+            }
+            return hip_ok(hipStreamSynchronize(static_cast<hipStream_t>(m_stream)), "hipStreamSynchronize");
+        }
+    }
+    return tensor && tensor->copy_from_host(host, bytes, m_stream);
 }
 
 void Model::run(TensorBase *input, runtime_mode_t mode)

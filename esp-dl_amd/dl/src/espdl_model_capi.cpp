@@ -395,7 +395,7 @@ int espdl_model_set_input(espdl_model *m, const char *name, const void *host_dat
     dl::TensorBase *t = (m && name) ? m->model->get_input(name) : nullptr;
     if (!t || bytes != (int64_t)t->get_bytes())
         return -1;
-    return t->copy_from_host(host_data, (size_t)bytes, m->model->get_stream()) ? 0 : -1;
+    return m->model->write_tensor(t, host_data) ? 0 : -1;
 }
 
 int espdl_model_get_tensor(espdl_model *m, const char *name, void *host_data, int64_t bytes)
@@ -403,7 +403,7 @@ int espdl_model_get_tensor(espdl_model *m, const char *name, void *host_data, in
     dl::TensorBase *t = (m && name) ? m->model->get_intermediate(name) : nullptr;
     if (!t || bytes != (int64_t)t->get_bytes())
         return -1;
-    return t->copy_to_host(host_data, (size_t)bytes, m->model->get_stream()) ? 0 : -1;
+    return m->model->read_tensor(t, host_data) ? 0 : -1;
 }
 
 int64_t espdl_model_device_bytes(espdl_model *m)

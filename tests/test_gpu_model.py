@@ -390,6 +390,23 @@ def test_attention_block(oracle, round_mode):
     mdl.close()
 
 
+@pytest.mark.parametrize("size", [1, 65536, 65537, 1 << 20, (1 << 20) + 3, 3 << 19, 4 << 20, (4 << 20) + 1])
+def test_host_copies(size):
+    """set_input and get_tensor on both sides of the sizes where the copy takes another way."""
+    announce(f"model host copies {size}")
+    _, zoo, model, _ = _mods()
+    g = zoo.GraphSpec("view")
+    b = zoo.Builder(g, 1)
+    b.output(b.reshape(b.input("input", [1, 1, 1, size], 0), [1, size]))
+    mdl = model.Model(model.Graph.from_spec(g), 1)
+    for seed in (1, 2):
+        x = np.random.default_rng(seed).integers(-128, 128, (1, 1, 1, size), dtype=np.int8)
+        mdl.set_input("input", x)
+        mdl.run()
+        np.testing.assert_array_equal(mdl.get_tensor(g.outputs[0]).ravel(), x.ravel())
+    mdl.close()
+
+
 def test_attention_block_is_one_module(oracle):
     """The modules between the block's convolutions become one; the separate ones give the same bytes."""
     announce("model attention_block fused and not")
