@@ -242,6 +242,9 @@ int espdl_hip_conv2d_add(const espdl_hip_conv_desc *desc, const void *in, const 
         if (residual != nullptr && depthwise)
             return fail(ESPDL_HIP_ENOTSUP, "the fused residual Add exists for dense int8 convolutions only");
         if (depthwise) {
+            if (espdl::depthwise_s8_strip_supports(g))
+                return device_status(espdl::launch_depthwise_s8_strip(g, i8, f8, b32, shift, lut, o8, cu_count_cached(), s),
+                                     "depthwise_s8_strip");
             if (espdl::depthwise_s8_lds_supports(g, in, out))
                 return device_status(espdl::launch_depthwise_s8_lds(g, i8, f8, b32, shift, lut, o8, cu_count_cached(), s),
                                      "depthwise_s8_lds");

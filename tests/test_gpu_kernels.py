@@ -683,6 +683,29 @@ def test_depthwise_s8_tiles(oracle, case):
     np.testing.assert_array_equal(got, want)
 
 
+@pytest.mark.parametrize("half_even", [False, True], ids=["half_up", "half_even"])
+@pytest.mark.parametrize("case", [
+    # (n, h, w, c), stride, pads, lowest and highest shift, lut: channels around the threads' four, output columns around
+    # their four, strips of one row and of many, both strides on either axis, left shifts and the general epilogue
+    ((2, 5, 4, 4), (1, 1), (1, 1, 1, 1), 7, 11, False), ((1, 9, 5, 5), (2, 2), (1, 1, 1, 1), 7, 11, True),
+    ((3, 8, 9, 7), (1, 2), (0, 1, 1, 0), 3, 9, False), ((2, 7, 11, 18), (2, 1), (1, 0, 0, 2), 7, 11, False),
+    ((1, 3, 3, 67), (1, 1), (0, 0, 0, 0), 0, 32, False), ((40, 61, 30, 33), (1, 1), (1, 1, 1, 1), 7, 11, True),
+    ((30, 40, 57, 130), (2, 2), (0, 1, 0, 1), 7, 11, False), ((1, 1, 1, 9), (1, 1), (1, 1, 1, 1), 6, 8, False)],
+    ids=lambda c: "x".join(map(str, c[0])) + "_s%d%d" % c[1])
+def test_depthwise_s8_strips(oracle, case, half_even):
+    shape, stride, pads, s_lo, s_hi, with_lut = case
+    announce(f"depthwise_s8 strips {case} half_even={half_even}")
+    rng = np.random.default_rng(0xD7)
+    c = shape[3]
+    x, f = rng_int8(rng, shape), rng_int8(rng, (3, 3, c))
+    bias = rng.integers(-4096, 4097, size=c).astype(np.int32)
+    shift = rng.integers(s_lo, s_hi + 1, size=c).astype(np.int32)
+    lut = np.array([(i * 109 + 37) & 0xFF for i in range(256)], dtype=np.uint8).view(np.int8) if with_lut else None
+    got, want = _run_conv_s8(oracle, x, f, bias, shift, (3, 3), stride, (1, 1), pads, not with_lut, depthwise=True,
+                             half_even=half_even, lut=lut)
+    np.testing.assert_array_equal(got, want)
+
+
 def _run_conv_s16(oracle, x, f, bias, shift, k, stride, dil, pads, relu, depthwise):
     m = espdl()
     act = m.capi.RELU if relu else m.capi.LINEAR
