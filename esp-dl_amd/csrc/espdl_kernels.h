@@ -239,9 +239,8 @@ hipError_t launch_max_pool(const void *in, int elem_size, int batch, int h, int 
                            int stride_w, int pad_top, int pad_left, int out_h, int out_w, long long in_pitch,
                            long long out_pitch, void *out, int cu_count, hipStream_t stream);
 // int8, square windows of 2 / 3 / 5 at stride 1, channels and pitches in multiples of 16 (max_pool_s8.hip)
-bool max_pool_s8_window_supports(const void *in, int h, int w, int c, int k_h, int k_w, int stride_h, int stride_w,
-                                 int pad_top, int pad_left, int out_h, int out_w, long long in_pitch, long long out_pitch,
-                                 const void *out);
+bool max_pool_s8_window_supports(int h, int w, int c, int k_h, int k_w, int stride_h, int stride_w, int pad_top,
+                                 int pad_left, int out_h, int out_w);
 hipError_t launch_max_pool_s8_window(const void *in, int batch, int h, int w, int c, int k, int pad_top, int pad_left,
                                      int out_h, int out_w, long long in_pitch, long long out_pitch, void *out,
                                      int cu_count, hipStream_t stream);

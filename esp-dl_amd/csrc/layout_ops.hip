@@ -52,8 +52,9 @@ __global__ __launch_bounds__(kBlock) void copy_rows_kernel(const RowCopyArgs a)
             r = i / s.per_row.d;
             c = (unsigned)(i - r * s.per_row.d);
         }
-        sp = s.src + r * s.src_pitch + (long long)c * s.vec;
-        dp = s.dst + r * s.dst_pitch + (long long)c * s.vec;
+        const long long at = min((long long)c * s.vec, s.row_bytes - s.vec);
+        sp = s.src + r * s.src_pitch + at;
+        dp = s.dst + r * s.dst_pitch + at;
     };
     for (long long i0 = (long long)blockIdx.x * kBlock + threadIdx.x; i0 < total; i0 += 4 * stride) {
         if (s.vec == 16) {
@@ -64,12 +65,12 @@ __global__ __launch_bounds__(kBlock) void copy_rows_kernel(const RowCopyArgs a)
                 const long long i = i0 + j * stride;
                 const char *sp;
                 locate(i < total ? i : i0, sp, dp[j]);
-                v[j] = *reinterpret_cast<const v4i *>(sp);
+                v[j] = *reinterpret_cast<const v4i_unaligned *>(sp);
             }
 #pragma unroll
             for (int j = 0; j < 4; j++)
                 if (i0 + j * stride < total)
-                    *reinterpret_cast<v4i *>(dp[j]) = v[j];
+                    *reinterpret_cast<v4i_unaligned *>(dp[j]) = v[j];
         } else {
             for (int j = 0; j < 4; j++) {
                 const long long i = i0 + j * stride;
@@ -91,7 +92,7 @@ inline int widest_access(const void *a, const void *b, long long p0, long long p
 {
     const uintptr_t m = reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | (uintptr_t)p0 | (uintptr_t)p1 |
         (uintptr_t)n;
-    return (m & 15) == 0 ? 16 : ((m & 3) == 0 ? 4 : 1);
+    return (m & 3) == 0 ? 4 : 1;
 }
 
 inline bool fill_seg(RowSeg &s, const void *src, long long src_pitch, void *dst, long long dst_pitch, long long row_bytes)
@@ -101,8 +102,10 @@ inline bool fill_seg(RowSeg &s, const void *src, long long src_pitch, void *dst,
     s.src_pitch = src_pitch;
     s.dst_pitch = dst_pitch;
     s.row_bytes = row_bytes;
-    s.vec = widest_access(src, dst, src_pitch, dst_pitch, row_bytes);
-    const long long per_row = row_bytes / s.vec;
+    // 16 bytes at any address; the last access of a row that is no multiple of 16 long reaches back over bytes its
+    // neighbour copies too
+    s.vec = row_bytes >= 16 ? 16 : widest_access(src, dst, src_pitch, dst_pitch, row_bytes);
+    const long long per_row = (row_bytes + s.vec - 1) / s.vec;
     if (per_row > 0x7fffffffll)
         return false;
     s.per_row = make_fastdiv((unsigned)std::max<long long>(per_row, 1));
@@ -517,13 +520,17 @@ namespace {
 // Concat walked in OUTPUT order: piece o of the output (16 bytes) lies in row o / per_row at column o % per_row,
 // and the column says which input it comes from.  Every store of a wavefront is then a run of whole cache lines;
 // with one pass per input the two halves of a 128-byte line arrive from different workgroups at different times
-// (measured on 64 + 64 channels: 4.2 TB/s per-input, see the table in the kernel list for this form).
+// (measured on 64 + 64 channels: 4.2 TB/s per-input, see the table in the kernel list for this form).  The last piece of
+// an input whose rows are no multiple of 16 bytes long reaches back over bytes its neighbour copies too; addresses need no
+// alignment (194 + 194 channels, 36864 rows: 7.5 us, byte by byte 20 us).
 struct ConcatArgs {
     const char *src[kMaxSeg];
     unsigned first[kMaxSeg + 1]; // first output piece (of a row) of input j; first[n] = pieces per row
-    unsigned pieces[kMaxSeg];    // pieces per row of input j
+    unsigned bytes[kMaxSeg];     // bytes per row of input j, at least 16
+    unsigned at[kMaxSeg];        // where they start in a row of the output
     int n;
     char *dst;
+    unsigned row_bytes;
     long long rows;
     FastDiv per_row;
 };
@@ -534,6 +541,7 @@ __global__ __launch_bounds__(kBlock) void concat_rows_kernel(const ConcatArgs a)
     const long long stride = (long long)gridDim.x * kBlock;
     for (long long i0 = (long long)blockIdx.x * kBlock + threadIdx.x; i0 < total; i0 += 4 * stride) {
         v4i v[4];
+        char *to[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const long long i = i0 + j * stride < total ? i0 + j * stride : i0;
@@ -543,12 +551,14 @@ __global__ __launch_bounds__(kBlock) void concat_rows_kernel(const ConcatArgs a)
 #pragma unroll
             for (int k = 1; k < kMaxSeg; k++)
                 seg += (k < a.n && c >= a.first[k]) ? 1 : 0;
-            v[j] = *reinterpret_cast<const v4i *>(a.src[seg] + ((long long)r * a.pieces[seg] + (c - a.first[seg])) * 16);
+            const unsigned bytes = a.bytes[seg], off = min((c - a.first[seg]) * 16, bytes - 16);
+            v[j] = *reinterpret_cast<const v4i_unaligned *>(a.src[seg] + (long long)r * bytes + off);
+            to[j] = a.dst + (long long)r * a.row_bytes + a.at[seg] + off;
         }
 #pragma unroll
         for (int j = 0; j < 4; j++)
             if (i0 + j * stride < total)
-                reinterpret_cast<v4i *>(a.dst)[i0 + j * stride] = v[j];
+                *reinterpret_cast<v4i_unaligned *>(to[j]) = v[j];
     }
 }
 
@@ -558,7 +568,8 @@ __global__ __launch_bounds__(kBlock) void concat_rows_kernel(const ConcatArgs a)
 struct SplitArgs {
     char *dst[kMaxSeg];
     unsigned first[kMaxSeg + 1]; // first input piece (of a row) of output j; first[n] = pieces per row
-    unsigned pieces[kMaxSeg];    // pieces per row of output j
+    unsigned bytes[kMaxSeg];     // bytes per row of output j, at least 16
+    unsigned at[kMaxSeg];        // where they start in a row of the input
     int n;
     const char *src;
     long long src_pitch; // bytes from row to row of the input
@@ -572,25 +583,25 @@ __global__ __launch_bounds__(kBlock) void split_rows_kernel(const SplitArgs a)
     const long long stride = (long long)gridDim.x * kBlock;
     for (long long i0 = (long long)blockIdx.x * kBlock + threadIdx.x; i0 < total; i0 += 4 * stride) {
         v4i v[4];
-        unsigned rr[4], cc[4];
+        char *to[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const long long i = i0 + j * stride < total ? i0 + j * stride : i0;
-            rr[j] = fastdiv((unsigned)i, a.per_row);
-            cc[j] = (unsigned)i - rr[j] * a.per_row.d;
-            v[j] = *reinterpret_cast<const v4i *>(a.src + (long long)rr[j] * a.src_pitch + (long long)cc[j] * 16);
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            if (i0 + j * stride >= total)
-                continue;
+            const unsigned r = fastdiv((unsigned)i, a.per_row);
+            const unsigned c = (unsigned)i - r * a.per_row.d;
             int seg = 0;
 #pragma unroll
             for (int k = 1; k < kMaxSeg; k++)
-                seg += (k < a.n && cc[j] >= a.first[k]) ? 1 : 0;
-            if (a.dst[seg] != nullptr) // an output that already lies in the input is not written
-                *reinterpret_cast<v4i *>(a.dst[seg] + ((long long)rr[j] * a.pieces[seg] + (cc[j] - a.first[seg])) * 16) = v[j];
+                seg += (k < a.n && c >= a.first[k]) ? 1 : 0;
+            const unsigned bytes = a.bytes[seg], off = min((c - a.first[seg]) * 16, bytes - 16);
+            v[j] = *reinterpret_cast<const v4i_unaligned *>(a.src + (long long)r * a.src_pitch + a.at[seg] + off);
+            // an output that already lies in the input is not written
+            to[j] = a.dst[seg] != nullptr ? a.dst[seg] + (long long)r * bytes + off : nullptr;
         }
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (i0 + j * stride < total && to[j] != nullptr)
+                *reinterpret_cast<v4i_unaligned *>(to[j]) = v[j];
     }
 }
 } // namespace
@@ -603,17 +614,19 @@ hipError_t launch_split(const void *in, long long in_pitch, int n_outputs, void 
         total += copy_bytes[j];
     if (rows <= 0 || total <= 0)
         return hipSuccess;
-    // input-order form: up to kMaxSeg outputs, everything in whole aligned 16-byte pieces
-    bool ok = n_outputs <= kMaxSeg && (reinterpret_cast<uintptr_t>(in) & 15) == 0 && (in_pitch & 15) == 0 &&
-        rows * (total / 16) <= 0x7fffffffll;
+    // input-order form: up to kMaxSeg outputs of at least 16 bytes per row (the last piece of each may reach back, see
+    // the Concat above)
+    bool ok = n_outputs <= kMaxSeg && total < (1ll << 31) && rows * (total / 16 + kMaxSeg) <= 0x7fffffffll;
     SplitArgs a = {};
-    unsigned first = 0;
+    unsigned first = 0, at = 0;
     for (int j = 0; ok && j < n_outputs; j++) {
-        ok = (copy_bytes[j] & 15) == 0 && copy_bytes[j] > 0 && (reinterpret_cast<uintptr_t>(outputs[j]) & 15) == 0;
+        ok = copy_bytes[j] >= 16;
         a.dst[j] = static_cast<char *>(outputs[j]);
         a.first[j] = first;
-        a.pieces[j] = (unsigned)(copy_bytes[j] / 16);
-        first += a.pieces[j];
+        a.bytes[j] = (unsigned)copy_bytes[j];
+        a.at[j] = at;
+        at += a.bytes[j];
+        first += (a.bytes[j] + 15) / 16;
     }
     if (ok) {
         for (int k = n_outputs; k <= kMaxSeg; k++)
@@ -649,20 +662,21 @@ hipError_t launch_concat(int n_inputs, const void *const *inputs, const long lon
     if (loop_times <= 0 || total <= 0)
         return hipSuccess;
     {
-        // output-order form: up to kMaxSeg inputs, everything in whole aligned 16-byte pieces
-        bool ok = n_inputs <= kMaxSeg && (reinterpret_cast<uintptr_t>(out) & 15) == 0 && (total & 15) == 0 &&
-            loop_times * (total / 16) <= 0x7fffffffll;
+        // output-order form: up to kMaxSeg inputs of at least 16 bytes per row
+        bool ok = n_inputs <= kMaxSeg && total < (1ll << 31) && loop_times * (total / 16 + kMaxSeg) <= 0x7fffffffll;
         ConcatArgs a = {};
         unsigned first = 0;
         int n = 0;
         for (int j = 0; ok && j < n_inputs; j++) {
             if (copy_bytes[j] == 0)
                 continue;
-            ok = (copy_bytes[j] & 15) == 0 && (reinterpret_cast<uintptr_t>(inputs[j]) & 15) == 0;
+            ok = copy_bytes[j] >= 16;
             a.src[n] = static_cast<const char *>(inputs[j]);
             a.first[n] = first;
-            a.pieces[n] = (unsigned)(copy_bytes[j] / 16);
-            first += a.pieces[n];
+            a.bytes[n] = (unsigned)copy_bytes[j];
+            a.at[n] = a.row_bytes;
+            a.row_bytes += a.bytes[n];
+            first += (a.bytes[n] + 15) / 16;
             n++;
         }
         if (ok && n > 0) {
@@ -898,8 +912,7 @@ hipError_t launch_max_pool(const void *in, int elem_size, int batch, int h, int 
                            int stride_w, int pad_top, int pad_left, int out_h, int out_w, long long in_pitch,
                            long long out_pitch, void *out, int cu_count, hipStream_t stream)
 {
-    if (elem_size == 1 && max_pool_s8_window_supports(in, h, w, c, k_h, k_w, stride_h, stride_w, pad_top, pad_left, out_h,
-                                                      out_w, in_pitch, out_pitch, out))
+    if (elem_size == 1 && max_pool_s8_window_supports(h, w, c, k_h, k_w, stride_h, stride_w, pad_top, pad_left, out_h, out_w))
         return launch_max_pool_s8_window(in, batch, h, w, c, k_h, pad_top, pad_left, out_h, out_w, in_pitch, out_pitch, out,
                                          cu_count, stream);
     PoolArgs a;

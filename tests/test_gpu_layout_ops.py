@@ -216,6 +216,25 @@ def test_max_pool_window_kernel(oracle, shape, k, pads, fill):
     np.testing.assert_array_equal(got, oracle.max_pool(x, (k, k), (1, 1), pads))
 
 
+@pytest.mark.parametrize("shape,k", [((2, 9, 7, 9), 5), ((1, 6, 5, 15), 2), ((3, 8, 9, 17), 3), ((2, 13, 6, 31), 5), ((5, 36, 8, 194), 5)])
+def test_max_pool_window_odd_channels(oracle, shape, k):
+    """Channel counts whose last vector reaches back, also as a slice at odd addresses; the bytes beside it stay."""
+    import torch
+    announce(f"max_pool window odd channels {shape} k{k}")
+    x = _rand(np.random.default_rng(29), shape)
+    pads = ((k - 1) // 2, k // 2) * 2
+    want = oracle.max_pool(x, (k, k), (1, 1), pads)
+    np.testing.assert_array_equal(to_host(espdl().max_pool(to_dev(x), (k, k), (1, 1), pads)), want)
+    n, h, w, c = shape
+    wide = torch.full((n, h, w, c + 6), 77, dtype=torch.int8, device="cuda")
+    wide_in = torch.zeros_like(wide)
+    wide_in[..., 1:c + 1] = to_dev(x)
+    espdl().max_pool(wide_in[..., 1:c + 1], (k, k), (1, 1), pads, out=wide[..., 5:c + 5])
+    got = to_host(wide)
+    np.testing.assert_array_equal(got[..., 5:c + 5], want)
+    assert (got[..., :5] == 77).all() and (got[..., c + 5:] == 77).all()
+
+
 @pytest.mark.parametrize("c,wide_in,wide_out,at", [(16, 64, 48, 16), (32, 32, 128, 96), (16, 40, 16, 0), (24, 72, 48, 24)])
 def test_max_pool_channel_slices(oracle, c, wide_in, wide_out, at):
     """Input and output as channel slices of wider tensors (pitches that are and are not multiples of 16 bytes);
