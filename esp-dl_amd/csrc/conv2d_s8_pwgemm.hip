@@ -463,7 +463,7 @@ bool conv2d_s8_pwgemm_supports(const ConvGeom &g, const void *in, const void *fi
     const int cus = cu_count > 0 ? cu_count : 256;
     // A short reduction under thousands of filters (a recognizer's 120 -> 6625 classifier) is bound by writing
     // the output: the implicit-GEMM kernel, whose wavefronts keep their pixels' operands in registers and write
-    // several hundred contiguous bytes per pixel, does that faster (76 against 112 us on 20480 x 120 x 6625).
+    // several hundred contiguous bytes per pixel, does that faster (rows of an odd length: conv2d_s8_wide.hip).
     if (g.in_c <= 128 && g.out_c >= 2048 && npix >= 64ll * cus)
         return false;
     return npix > 0 && (npix + 63) / 64 < (long long)cus * 16 && (npix + 63) / 64 <= 0x7fffffffll;

@@ -1,0 +1,288 @@
+// Pointwise int8 convolution / Gemm with a short reduction under thousands of filters (a recognizer's 120 -> 6625
+// classifier over every position): bound by writing the result, which is fifty times the size of the input.
+//
+// A wavefront keeps 64 pixels in registers as operand B for its whole walk and takes the filters 64 at a time, which it
+// reads as operand A straight from L2 in operand order, a step ahead.  The four wavefronts of a workgroup take
+// neighbouring groups of 64 filters of the same pixels, so a step makes 256 neighbouring bytes of each of 64 rows.  (Row i
+// of tile t is filter 16 (i / 4) + 4 t + i % 4 of the group: a lane ends with 16 neighbouring filters of one pixel.)
+// Rows of an odd length start at any address.  Writing them as the lanes hold them, 16 bytes at odd addresses, ran at
+// 1.9 TB/s; so a step's bytes pass through LDS and leave as whole aligned 16-byte pieces of memory, cut out of the bytes
+// of this step and the last 16 of the step before, and only the two ends of a row's walk are written by the byte.
+//
+// 20480 pixels x 120 -> 6625 (136 MB written, 26 us at the copy rate): 50 us, where the kernel that keeps filters in LDS
+// took 75 us.  A third of that is the start of a walk (its pixels and constants), of which every compute unit does four.
+//
+// Restates conv2d_11cn (esp-dl/dl/base/dl_base_conv2d.cpp:9-33) with the n_wise epilogue
+// (esp-dl/dl/base/dl_base_activate_buffer.hpp:27-36, 61-72, 173-181, 201-210).
+#include <type_traits>
+
+#include "conv_window.h"
+
+namespace espdl {
+namespace {
+
+using namespace window;
+
+typedef unsigned v4u __attribute__((ext_vector_type(4)));
+
+constexpr int kThreads = 256;
+constexpr int kRow = 16 + 256; // a row of the output tile in LDS: the 16 bytes in front, then those of the step
+
+struct WideArgs {
+    const int8_t *in, *w;
+    const int32_t *bias, *shift;
+    int8_t *out;
+    int in_bytes, w_bytes;
+    int M, K, N, in_pitch, out_pitch;
+    int per_walk; // filters of a workgroup, a multiple of 256
+    int relu, half_even, n_shift;
+};
+
+template <int KS>
+__global__ __launch_bounds__(kThreads, 2) void conv2d_s8_wide_kernel(const WideArgs a)
+{
+    __shared__ __align__(16) unsigned char tile[2][64 * kRow + 16];
+    extern __shared__ __align__(16) int cst[]; // per filter of the walk: start value | right shift | left shift
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int col = lane & 15, quad = lane >> 4;
+    const int m0 = blockIdx.x * 64, n_begin = blockIdx.y * a.per_walk, n_end = min(a.N, n_begin + a.per_walk);
+    int *const c_start = cst, *const c_rsh = cst + a.per_walk, *const c_lsh = cst + 2 * a.per_walk;
+    const __amdgpu_buffer_rsrc_t in = tensor_rsrc(a.in, a.in_bytes), w = tensor_rsrc(a.w, a.w_bytes);
+
+    // the wavefront's pixels, zeros behind the last channel (operand A may then hold anything there)
+    v4i b[4][KS];
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+        for (int k = 0; k < KS; k++) {
+            const int at = 64 * k + 16 * quad, m = m0 + 16 * c + col;
+            b[c][k] = load16<false>(in, m < a.M && at < a.K ? m * a.in_pitch + at : kParked, a.in_bytes);
+        }
+    // Operand A of step n: rows in lane order, a filter past the last one reads the last one again.  Away from the last
+    // filters every piece is whole and the lane's one offset serves all of them.
+    const int row_in_group = 16 * (col >> 2) + (col & 3);
+    const auto fetch = [&](int n, v4i (&p)[4][KS]) {
+        if (n + 64 < a.N) {
+            const int row = (n + row_in_group) * a.K + 16 * quad;
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int k = 0; k < KS; k++)
+                    p[t][k] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(w, row, 4 * t * a.K + 64 * k, 0));
+            return;
+        }
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const int row = min(n + row_in_group + 4 * t, a.N - 1) * a.K + 16 * quad;
+#pragma unroll
+            for (int k = 0; k < KS; k++)
+                p[t][k] = load16<false>(w, 64 * k + 16 * quad < a.K ? row + 64 * k : kParked, a.w_bytes);
+        }
+    };
+    v4i fa[4][KS];
+    fetch(n_begin + 64 * wave, fa);
+
+    int ok = 1; // the short epilogue is exact
+    for (int i0 = tid; i0 < a.per_walk; i0 += 6 * kThreads) { // six at a time: their loads are in flight together
+        int sh[6], bias[6];
+#pragma unroll
+        for (int u = 0; u < 6; u++) {
+            const int n = min(n_begin + i0 + u * kThreads, a.N - 1);
+            sh[u] = a.shift[a.n_shift == 1 ? 0 : n];
+            bias[u] = a.bias != nullptr ? a.bias[n] : 0;
+        }
+#pragma unroll
+        for (int u = 0; u < 6; u++) {
+            const int i = i0 + u * kThreads, s = min(max(sh[u], 1), 31);
+            const long long start = (long long)bias[u] + (1ll << (s - 1));
+            if (sh[u] != s || (start < 0 ? -start : start) + (long long)a.K * 16384 >= 1ll << (31 - max(0, 8 - s)))
+                ok = 0;
+            if (i < a.per_walk) {
+                c_start[i] = (int)start - (a.half_even ? 1 : 0);
+                c_rsh[i] = max(0, s - 8);
+                c_lsh[i] = max(0, 8 - s);
+            }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+        for (int k = 0; k < KS; k++)
+            b[c][k] = mask_unit<false>(b[c][k], max(a.K - (64 * k + 16 * quad), 0));
+    const bool fast = __syncthreads_and(ok) != 0;
+
+    const int floor_pk = a.relu ? 0 : (int)0x80008000u;
+    // The walk's bytes of row r start lead(r) bytes into a 16-byte piece of memory.
+    int8_t *const out0 = a.out + (long long)m0 * a.out_pitch + n_begin;
+    const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(out0 - 16, (short)0, 0x7ffffff0, 0x00020000);
+    const auto lead = [&](int r) { return (int)((reinterpret_cast<uintptr_t>(out0) + (unsigned)(r * a.out_pitch)) & 15); };
+    const int len = n_end - n_begin;
+    // Pieces of the rows this lane writes: row (tid / 16) + 16 i, piece tid % 16 of a step.
+    int from[4], to[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int r = (tid >> 4) + 16 * i, at = 16 * (tid & 15) - lead(r);
+        from[i] = r * kRow + 16 + at;
+        to[i] = m0 + r < a.M ? 16 + r * a.out_pitch + at : kParked;
+    }
+    const auto walk = [&](auto mode) {
+        constexpr int MODE = decltype(mode)::value; // of pack_fast4, -1: the general epilogue
+        for (int step = 0; 256 * step < len; step++) {
+            const int n = n_begin + 256 * step + 64 * wave;
+            unsigned char *buf = tile[step & 1], *next = tile[~step & 1];
+            v4i acc[4][4]; // [pixel tile][filter tile]
+            const int at = n - n_begin + 16 * quad;
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                v4i start;
+                if constexpr (MODE >= 0) {
+                    start = *reinterpret_cast<const v4i *>(&c_start[at + 4 * t]);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        start[r] = a.bias != nullptr ? a.bias[min(n_begin + at + 4 * t + r, a.N - 1)] : 0;
+                }
+#pragma unroll
+                for (int c = 0; c < 4; c++)
+                    acc[c][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[t][0], b[c][0], start, 0, 0, 0);
+            }
+#pragma unroll
+            for (int k = 1; k < KS; k++)
+#pragma unroll
+                for (int t = 0; t < 4; t++)
+#pragma unroll
+                    for (int c = 0; c < 4; c++)
+                        acc[c][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fa[t][k], b[c][k], acc[c][t], 0, 0, 0);
+            if (256 * (step + 1) < len)
+                fetch(n + 256, fa);
+            int words[4][4];
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const v4i rsh = *reinterpret_cast<const v4i *>(&c_rsh[at + 4 * t]);
+                const v4i lsh = *reinterpret_cast<const v4i *>(&c_lsh[at + 4 * t]);
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    if constexpr (MODE >= 0) {
+                        words[c][t] = pack_fast4<MODE>(acc[c][t], lsh, rsh, floor_pk);
+                    } else {
+                        int q[4];
+#pragma unroll
+                        for (int r = 0; r < 4; r++)
+                            q[r] = requant_s8(acc[c][t][r], a.shift[a.n_shift == 1 ? 0 : min(n_begin + at + 4 * t + r, a.N - 1)], a.relu != 0, a.half_even != 0);
+                        words[c][t] = pack4_s8(q[0], q[1], q[2], q[3]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                *reinterpret_cast<v4i *>(buf + (16 * c + col) * kRow + 16 + 64 * wave + 16 * quad) =
+                    v4i{words[c][0], words[c][1], words[c][2], words[c][3]};
+            __syncthreads(); // one barrier per step: the other buffer was read before this one
+            // Out in whole 16-byte pieces of memory: a piece ends lead(r) bytes short of where 16 bytes of the step end, so
+            // the first of a step begins with bytes of the step before.
+            const bool last = 256 * (step + 1) >= len;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int *src = reinterpret_cast<const int *>(buf + (from[i] & ~3));
+                int d[5];
+#pragma unroll
+                for (int k = 0; k < 5; k++)
+                    d[k] = src[k];
+                v4i v;
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    v[k] = (int)__builtin_amdgcn_alignbyte((unsigned)d[k + 1], (unsigned)d[k], (unsigned)(from[i] & 3));
+                int at = to[i];
+                if (step == 0 || last) { // pieces of which the walk only has a part
+                    const int r = (tid >> 4) + 16 * i, off = lead(r), first = 256 * step + 16 * (tid & 15);
+                    if (first < off || first + 16 > off + len)
+                        at = kParked;
+                }
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, v), out, at, 256 * step, 0);
+            }
+            // those parts, a byte per lane: in front and behind
+            if (step == 0 || last) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int r = (tid >> 4) + 16 * i, byte = tid & 15, off = lead(r), end = off + len, tail = end & ~15;
+                    if (m0 + r >= a.M)
+                        continue;
+                    int8_t *row = out0 + (long long)r * a.out_pitch - off;
+                    const unsigned char *bytes = buf + r * kRow + 16 - off;
+                    if (step == 0 && byte >= off && byte < end && (off != 0 || end < 16))
+                        row[byte] = (int8_t)bytes[byte];
+                    if (last && tail != 0 && tail + byte < end)
+                        row[tail + byte] = (int8_t)bytes[tail + byte - 256 * step];
+                }
+            }
+            if (tid < 64) // what the next step's first pieces start with
+                *reinterpret_cast<v4i *>(next + tid * kRow) = *reinterpret_cast<const v4i *>(buf + tid * kRow + 256);
+        }
+    };
+    if (!fast)
+        walk(std::integral_constant<int, -1>{});
+    else if (a.half_even)
+        walk(std::integral_constant<int, 5>{});
+    else
+        walk(std::integral_constant<int, 1>{});
+}
+
+} // namespace
+
+// Rows of the result that are no multiple of 16 bytes long, which the other kernels write in pieces at odd addresses, and
+// enough of them: 640 rows of 6625 take 8.5 us either way, 1280 rows 10 against 15 us.  (3000 rows of 2048 from 128: 8.7
+// against 6.6 us, 20480 rows of 4096 from 64: 28 against 30 us.)
+bool conv2d_s8_wide_supports(const ConvGeom &g, const int8_t *lut, const int8_t *residual)
+{
+    const bool flat = g.k_h == 1 && g.k_w == 1 && g.stride_h == 1 && g.stride_w == 1 && g.pad_top == 0 && g.pad_left == 0 &&
+        g.out_h == g.in_h && g.out_w == g.in_w;
+    return flat && lut == nullptr && residual == nullptr && g.in_c >= 16 && g.in_c <= 128 && g.out_c >= 2048 &&
+        (g.out_pitch & 15) != 0 && g.out_pitch < (1 << 24) && (long long)g.batch * g.out_h * g.out_w >= 1024 && window_supports(g);
+}
+
+hipError_t launch_conv2d_s8_wide(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,
+                                 const int32_t *shift, int8_t *out, int cu_count, hipStream_t stream)
+{
+    const WindowArgs wa = window_args(g, in, filter);
+    WideArgs a;
+    a.in = in;
+    a.w = filter;
+    a.bias = bias;
+    a.shift = shift;
+    a.out = out;
+    a.in_bytes = wa.in_bytes;
+    a.w_bytes = wa.w_bytes;
+    a.M = g.batch * g.out_h * g.out_w;
+    a.K = g.in_c;
+    a.N = g.out_c;
+    a.in_pitch = g.in_pitch;
+    a.out_pitch = g.out_pitch;
+    a.relu = g.relu;
+    a.half_even = g.half_even;
+    a.n_shift = g.n_shift;
+    if (a.M == 0)
+        return hipSuccess;
+    // Steps per walk: rounds of workgroups (two fit a compute unit) times a walk and its start, which costs about four
+    // steps; twelve steps' constants at most lie in LDS.
+    const int tiles = (a.M + 63) / 64, steps = (a.N + 255) / 256;
+    const long long slots = 2ll * std::max(1, cu_count);
+    int per = 1;
+    long long best = 0;
+    for (int p = 1; p <= std::min(steps, 12); p++) {
+        const long long cost = ((long long)tiles * ((steps + p - 1) / p) + slots - 1) / slots * (p + 4);
+        if (p == 1 || cost < best) {
+            best = cost;
+            per = p;
+        }
+    }
+    a.per_walk = 256 * per;
+    const dim3 grid((unsigned)tiles, (unsigned)((steps + per - 1) / per));
+    const size_t lds = (size_t)3 * sizeof(int) * a.per_walk;
+    if (a.K <= 64)
+        hipLaunchKernelGGL(conv2d_s8_wide_kernel<1>, grid, dim3(kThreads), lds, stream, a);
+    else
+        hipLaunchKernelGGL(conv2d_s8_wide_kernel<2>, grid, dim3(kThreads), lds, stream, a);
+    return hipGetLastError();
+}
+
+} // namespace espdl

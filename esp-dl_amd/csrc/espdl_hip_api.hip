@@ -272,6 +272,8 @@ int espdl_hip_conv2d_add(const espdl_hip_conv_desc *desc, const void *in, const 
             }
             return (int)ESPDL_HIP_OK;
         };
+        if (espdl::conv2d_s8_wide_supports(g, lut, residual))
+            return device_status(espdl::launch_conv2d_s8_wide(g, i8, f8, b32, shift, o8, cus, s), "conv2d_s8_wide");
         switch (dense_s8_route(g, in, filter, residual, cus)) {
         case DENSE_STEM:
             return device_status(espdl::launch_conv2d_s8_stem(g, i8, f8, b32, shift, lut, o8, cus, s), "conv2d_s8_stem");

@@ -93,6 +93,10 @@ struct DwExpand {
 
 // Depthwise with the input tile staged in LDS (contiguous global reads and writes) and the products
 // on the matrix pipe; same shape limits as the direct form.
+// conv2d_s8_wide.hip
+bool conv2d_s8_wide_supports(const ConvGeom &g, const int8_t *lut, const int8_t *residual);
+hipError_t launch_conv2d_s8_wide(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,
+                                 const int32_t *shift, int8_t *out, int cu_count, hipStream_t stream);
 // depthwise_s8_strip.hip
 bool depthwise_s8_strip_supports(const ConvGeom &g);
 hipError_t launch_depthwise_s8_strip(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,

@@ -483,6 +483,33 @@ def test_gemm_s8(oracle, m, k, n, has_bias, relu):
     np.testing.assert_array_equal(got, want)
 
 
+# A short reduction under thousands of filters with rows of an odd length: channel counts on both sides of one and two
+# k steps, rows and filters past whole tiles, walks of one step and of many, an output inside wider rows.
+@pytest.mark.parametrize("m,k,n,pad", [(1024, 16, 2049, 0), (1031, 17, 2303, 0), (1100, 64, 2305, 0), (5000, 65, 2055, 0),
+                                       (1400, 128, 6625, 0), (40000, 120, 2119, 0), (1025, 33, 2064, 5)])
+@pytest.mark.parametrize("variant", ["per_channel", "per_tensor", "half_even", "wide_shifts"])
+def test_conv2d_s8_wide_rows(oracle, m, k, n, pad, variant):
+    import torch
+    announce(f"conv2d_s8 wide rows M={m} K={k} N={n} pad={pad} {variant}")
+    rng = np.random.default_rng(0xF5 + m + n)
+    x, f = rng_int8(rng, (m, 1, 1, k)), rng_int8(rng, (n, 1, 1, k))
+    bias = None if variant == "per_tensor" else rng.integers(-4096, 4097, size=n).astype(np.int32)
+    lo, hi = (-2, 34) if variant == "wide_shifts" else (6, 12)
+    shift = np.array([9], np.int32) if variant == "per_tensor" else rng.integers(lo, hi, size=n).astype(np.int32)
+    mod, relu, even = espdl(), variant == "per_channel", variant == "half_even"
+    out = torch.full((m, 1, 1, n + pad), 77, dtype=torch.int8, device="cuda")
+    lo_c = pad // 2
+    mod.conv2d(to_dev(x), to_dev(f), None if bias is None else to_dev(bias), to_dev(shift), (1, 1),
+               activation=mod.capi.RELU if relu else mod.capi.LINEAR, out=out[..., lo_c:lo_c + n],
+               round_mode=mod.capi.ROUND_HALF_EVEN if even else mod.capi.ROUND_HALF_UP)
+    got = to_host(out)
+    oracle.set_threads(16)
+    want = oracle.conv2d_s8(x, f, bias, shift, (1, 1), activation=oracle.RELU if relu else oracle.LINEAR,
+                            round_mode=oracle.ROUND_HALF_EVEN if even else oracle.ROUND_HALF_UP)
+    np.testing.assert_array_equal(got[..., lo_c:lo_c + n], want)
+    assert (np.delete(got, np.s_[lo_c:lo_c + n], axis=3) == 77).all()
+
+
 # Products with so few rows that the tiled kernels would leave most of the device idle go to a kernel with one
 # wavefront per 16 x 16 tile: ragged row and filter counts, byte stores (N not a multiple of 4), one shift for all
 # filters, shifts outside 1..31, both roundings.
