@@ -132,6 +132,8 @@ def lib():
         L.espdl_hip_softmax_s8.argtypes = [vp, i64, i64, i64, i32, vp, vp]
         L.espdl_hip_quantize_f32.argtypes = [vp, i64, i32, i32, vp, vp]
         L.espdl_hip_dequantize_f32.argtypes = [vp, i64, i32, i32, vp, vp]
+        L.espdl_hip_conv2d_s16_x8.argtypes = [dp, vp, vp, vp, vp, vp, i32, vp, vp]
+        L.espdl_hip_conv2d_s16_x8.restype = ctypes.c_int
         L.espdl_hip_attention_s8.argtypes = [ctypes.POINTER(AttentionDesc), vp, vp, vp, vp, vp]
         L.espdl_hip_attention_s8.restype = ctypes.c_int
         L.espdl_hip_matmul_s8.argtypes = [vp, vp, i32, i32, i32, vp, vp, vp, i32, i32, i32, vp, vp]
@@ -227,6 +229,18 @@ def conv2d(x, filt, bias, shift, k, stride=(1, 1), dilation=(1, 1), pads=(0, 0, 
         out = torch.empty(out_shape, dtype=x.dtype, device=x.device)
     _check(lib().espdl_hip_conv2d_add(desc, _p(x), _p(filt), _p(bias), _p(shift), _p(lut), _p(residual), _p(out),
                                       _stream(stream)))
+    return out
+
+
+def conv2d_s16_x8(x, filt, bias, shift, k, stride=(1, 1), dilation=(1, 1), pads=(0, 0, 0, 0), activation=LINEAR,
+                  round_mode=ROUND_HALF_UP, table=None, stream=None):
+    """int16 convolution of 256 * x for an int8 x, with an int16 table behind it (espdl_hip_conv2d_s16_x8)."""
+    import torch
+    desc, out_shape = _conv_plan(x.shape, filt.numel(), tuple(k), tuple(stride), tuple(dilation), tuple(pads), False, activation,
+                                 round_mode, shift.numel(), S16, 0, 0, 0)
+    out = torch.empty(out_shape, dtype=torch.int16, device=x.device)
+    _check(lib().espdl_hip_conv2d_s16_x8(desc, _p(x), _p(filt), _p(bias), _p(shift), _p(table),
+                                         0 if table is None else table.numel(), _p(out), _stream(stream)))
     return out
 
 

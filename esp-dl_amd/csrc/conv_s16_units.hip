@@ -20,6 +20,12 @@
 // like any other product (where w = 0, x may be anything).  So nothing is special but the filter's bytes behind a
 // tap's last channel, which are cleared.
 //
+// X8 builds: the input is an int8 tensor that a RequantizeLinear would have multiplied by 256, so its low bytes are zero
+// and its high bytes the int8 values themselves:  sum_k x w = 65536 sum x8 wh + 256 sum x8 l + 32768 sum x8 (l as above).
+// Two products per step instead of four, no cutting of pixels, half the input, no RequantizeLinear and no int16 copy.
+// They also take an int16 table behind the result (the nearest-entry LUT of esp-dl/dl/base/dl_base_lut.cpp:49-77).
+// 80 x 80 x 64 -> 64, 3 x 3, batch 64: 78 us where the three operators took 135 us.
+//
 // Two kernels, chosen by their measured cost (see the launch).  Against the one-wavefront-per-pixel-tile kernel
 // (conv_s16_mfma.hip) and the 64-bit multiply-add kernel (conv_s16.hip): 80 x 80 x 64 -> 64, 3 x 3, batch 64 98 -> 92 us,
 // batch 8 22 -> 17 us, one image 13.4 -> 8.4 us; 40 x 40 x 128 -> 128, batch 64 147 -> 89 us; 22 x 12 x 122 -> 252, 3 x 3,
@@ -47,7 +53,17 @@ struct S16Args {
     int16_t *out;
     int n_pix, out_c, ksteps;
     int relu, half_even, n_shift;
+    const int16_t *table; // X8: applied to the result, or nullptr
+    int table_size, table_shift;
 };
+constexpr int kMostTable = 4097; // entries
+
+// The table's entry nearest to sample point v; ties as the rounding mode has them.
+__device__ __forceinline__ int nearest_entry(int v, int shift, bool half_even)
+{
+    const int x = (v & 0xffff) ^ 0x8000, half = 1 << (shift - 1);
+    return (half_even ? x + half - 1 + ((x >> shift) & 1) : x + half) >> shift;
+}
 
 // The 16 values of a unit: two 16-byte loads through the descriptor, zeros where nothing exists.
 struct Unit16 {
@@ -87,6 +103,28 @@ __device__ __forceinline__ Unit locate_unit16(const WindowArgs &a, int u)
     r.w_off = (int)tap * a.in_c + 32 * j;
     r.n = u < a.n_units ? a.in_c - 32 * j : 0; // bytes
     return r;
+}
+
+// X8: a unit is 16 bytes of the input and 32 of the filter (in_c and the pitch count int8 channels).
+__device__ __forceinline__ Unit locate_unit_x8(const WindowArgs &a, int u)
+{
+    const unsigned tap = fastdiv((unsigned)u, a.fd_upt);
+    const int j = u - (int)(tap * a.fd_upt.d);
+    const unsigned ky = fastdiv(tap, a.fd_kw);
+    Unit r;
+    r.dy = (int)ky * a.dil_h;
+    r.dx = (int)(tap - ky * a.fd_kw.d) * a.dil_w;
+    r.in_off = (r.dy * a.in_w + r.dx) * a.in_pitch + 16 * j;
+    r.w_off = 2 * (int)tap * a.in_c + 32 * j;
+    r.n = u < a.n_units ? 2 * (a.in_c - 16 * j) : 0; // filter bytes
+    return r;
+}
+__device__ __forceinline__ int byte_sum(const v4i &v, int sum)
+{
+#pragma unroll
+    for (int d = 0; d < 4; d++)
+        sum = __builtin_amdgcn_sdot4(v[d], 0x01010101, sum, false);
+    return sum;
 }
 
 // High bytes and low bytes xor 0x80 of half a unit or a unit, in k order, and the running sums of both.
@@ -134,11 +172,13 @@ __device__ __forceinline__ long long combine(int hh, int mid, int ll)
 }
 
 // PT: pixel tiles of 16 per wavefront; FT: filter tiles of 16 per workgroup.
-template <int PT, int FT, bool ALIGNED>
+template <int PT, int FT, bool ALIGNED, bool X8 = false>
 __global__ __launch_bounds__(kThreads) void conv2d_s16_gemm_kernel(const S16Args a)
 {
     constexpr int kTileM = 64 * PT;
-    __shared__ __align__(16) unsigned char b_l[2][2][kTileM * kRow]; // [buffer][high, low]
+    constexpr int kSums = X8 ? 2 : 3; // accumulators of a value
+    __shared__ __align__(16) unsigned char b_l[2][X8 ? 1 : 2][kTileM * kRow]; // [buffer][high, low]
+    [[maybe_unused]] __shared__ __align__(16) int16_t table_l[X8 ? kMostTable + 7 : 1];
     __shared__ __align__(16) unsigned char a_l[2][2][16 * FT * kRow];
     __shared__ long long pix_term[kTileM];
     __shared__ long long cst[16 * FT];
@@ -161,15 +201,20 @@ __global__ __launch_bounds__(kThreads) void conv2d_s16_gemm_kernel(const S16Args
     const int w_row = min(n0 + my_row, a.out_c - 1) * a.win.w_len;
 
     struct Pieces {
-        Unit16 b[PT], w;
+        std::conditional_t<X8, v4i, Unit16> b[PT];
+        Unit16 w;
         int n;
     };
     auto fetch = [&](int ks, Pieces &p) {
-        const Unit u = locate_unit16(a.win, 4 * ks + q4);
+        const Unit u = X8 ? locate_unit_x8(a.win, 4 * ks + q4) : locate_unit16(a.win, 4 * ks + q4);
         p.n = u.n;
 #pragma unroll
-        for (int j = 0; j < PT; j++)
-            p.b[j] = load_pixel16<ALIGNED>(a.win, in_rsrc, px[j], u);
+        for (int j = 0; j < PT; j++) {
+            if constexpr (X8)
+                p.b[j] = load_pixel_unit<ALIGNED>(a.win, in_rsrc, px[j], u);
+            else
+                p.b[j] = load_pixel16<ALIGNED>(a.win, in_rsrc, px[j], u);
+        }
         if (FT == 4 || my_row < 16 * FT)
             p.w = load_filter16<ALIGNED>(a.win, w_rsrc, w_row, u);
     };
@@ -178,9 +223,14 @@ __global__ __launch_bounds__(kThreads) void conv2d_s16_gemm_kernel(const S16Args
         const int at = my_row * kRow + 16 * q4;
 #pragma unroll
         for (int j = 0; j < PT; j++) {
-            const Planes c = cut(p.b[j], bsum_h[j], bsum_l[j]);
-            *reinterpret_cast<v4i *>(&b_l[buf][0][at + 64 * j * kRow]) = c.h;
-            *reinterpret_cast<v4i *>(&b_l[buf][1][at + 64 * j * kRow]) = c.l;
+            if constexpr (X8) {
+                bsum_h[j] = byte_sum(p.b[j], bsum_h[j]);
+                *reinterpret_cast<v4i *>(&b_l[buf][0][at + 64 * j * kRow]) = p.b[j];
+            } else {
+                const Planes c = cut(p.b[j], bsum_h[j], bsum_l[j]);
+                *reinterpret_cast<v4i *>(&b_l[buf][0][at + 64 * j * kRow]) = c.h;
+                *reinterpret_cast<v4i *>(&b_l[buf][1][at + 64 * j * kRow]) = c.l;
+            }
         }
         if (FT == 4 || my_row < 16 * FT) {
             const Planes c = cut_filter<ALIGNED>(p.w, p.n, wsum_h, wsum_l);
@@ -195,21 +245,26 @@ __global__ __launch_bounds__(kThreads) void conv2d_s16_gemm_kernel(const S16Args
         fetch(1, p1);
     if (tid < 16 * FT) {
         const int n = min(n0 + tid, a.out_c - 1);
-        cst[tid] = (a.bias != nullptr ? a.bias[n] : 0) + 16384ll * 64 * a.ksteps;
+        cst[tid] = (a.bias != nullptr ? a.bias[n] : 0) + (X8 ? 0 : 16384ll * 64 * a.ksteps);
         shf[tid] = a.shift[a.n_shift == 1 ? 0 : n];
+    }
+    if constexpr (X8) {
+        if (a.table != nullptr)
+            for (int i = tid; i < a.table_size; i += kThreads)
+                table_l[i] = a.table[i];
     }
     stash(0, p0);
     if (a.ksteps > 2)
         fetch(2, p0);
     __syncthreads();
 
-    v4i acc[PT][FT][3]; // HH, HL + LH, LL
+    v4i acc[PT][FT][kSums]; // HH, HL + LH, LL
 #pragma unroll
     for (int c = 0; c < PT; c++)
 #pragma unroll
         for (int t = 0; t < FT; t++)
 #pragma unroll
-            for (int s = 0; s < 3; s++)
+            for (int s = 0; s < kSums; s++)
                 acc[c][t][s] = v4i{0, 0, 0, 0};
     // row i of filter tile t is filter 4 FT (i / 4) + 4 t + i % 4: a lane ends up with 4 FT consecutive channels
     const int a_row0 = 4 * FT * (col >> 2) + (col & 3);
@@ -219,7 +274,8 @@ __global__ __launch_bounds__(kThreads) void conv2d_s16_gemm_kernel(const S16Args
         for (int c = 0; c < PT; c++) {
             const int at = (16 * PT * wave + 16 * c + col) * kRow + 16 * quad;
             xh[c] = *reinterpret_cast<const v4i *>(&b_l[buf][0][at]);
-            xl[c] = *reinterpret_cast<const v4i *>(&b_l[buf][1][at]);
+            if constexpr (!X8)
+                xl[c] = *reinterpret_cast<const v4i *>(&b_l[buf][1][at]);
         }
 #pragma unroll
         for (int t = 0; t < FT; t++) {
@@ -230,8 +286,10 @@ __global__ __launch_bounds__(kThreads) void conv2d_s16_gemm_kernel(const S16Args
             for (int c = 0; c < PT; c++) {
                 acc[c][t][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wh, xh[c], acc[c][t][0], 0, 0, 0);
                 acc[c][t][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wl, xh[c], acc[c][t][1], 0, 0, 0);
-                acc[c][t][2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wl, xl[c], acc[c][t][2], 0, 0, 0);
-                acc[c][t][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wh, xl[c], acc[c][t][1], 0, 0, 0);
+                if constexpr (!X8) {
+                    acc[c][t][2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wl, xl[c], acc[c][t][2], 0, 0, 0);
+                    acc[c][t][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wh, xl[c], acc[c][t][1], 0, 0, 0);
+                }
             }
         }
     };
@@ -268,7 +326,7 @@ __global__ __launch_bounds__(kThreads) void conv2d_s16_gemm_kernel(const S16Args
         if (q4 == 0)
             pix_term[64 * j + my_row] = t;
     }
-    {
+    if constexpr (!X8) {
         const long long t = row_term(wsum_h, wsum_l);
         if (q4 == 0 && my_row < 16 * FT)
             cst[my_row] += t; // (the first barrier lies behind the start value)
@@ -296,7 +354,17 @@ __global__ __launch_bounds__(kThreads) void conv2d_s16_gemm_kernel(const S16Args
     const bool fast = __syncthreads_and(fine) != 0;
     const bool any_low = __syncthreads_or(low) != 0;
     const int n = n0 + 4 * FT * quad; // this lane: channels n .. n + 4 FT - 1
-    auto write = [&](int c, const int(&words)[2 * FT]) {
+    auto write = [&](int c, int(&words)[2 * FT]) {
+        if constexpr (X8) {
+            if (a.table != nullptr) {
+#pragma unroll
+                for (int i = 0; i < 2 * FT; i++) {
+                    const int lo = nearest_entry(words[i], a.table_shift, a.half_even != 0);
+                    const int hi = nearest_entry(words[i] >> 16, a.table_shift, a.half_even != 0);
+                    words[i] = (int)(unsigned short)table_l[lo] | (table_l[hi] << 16);
+                }
+            }
+        }
         const int row = 16 * PT * wave + 16 * c + col;
         if (m0 + row >= a.n_pix || n >= a.out_c)
             return;
@@ -338,7 +406,7 @@ __global__ __launch_bounds__(kThreads) void conv2d_s16_gemm_kernel(const S16Args
                 const int s = shf[f];
 #pragma unroll
                 for (int c = 0; c < PT; c++) {
-                    const int l = acc[c][t][2][r] + fl + pl[c];
+                    const int l = (X8 ? 0 : acc[c][t][kSums - 1][r]) + fl + pl[c];
                     const int mid = acc[c][t][1][r] + (l >> 8);
                     const int x = acc[c][t][0][r] + fh + ph[c] + (mid >> 8);
                     if constexpr (LOW) {
@@ -379,7 +447,7 @@ __global__ __launch_bounds__(kThreads) void conv2d_s16_gemm_kernel(const S16Args
             for (int r = 0; r < 4; r++) {
                 const int f = 4 * FT * quad + 4 * t + r;
                 const int s = shf[f];
-                const long long v = cst[f] + pt + combine(acc[c][t][0][r], acc[c][t][1][r], acc[c][t][2][r]);
+                const long long v = cst[f] + pt + combine(acc[c][t][0][r], acc[c][t][1][r], X8 ? 0 : acc[c][t][kSums - 1][r]);
                 q[r] = requant_s16(v, s, relu, half_even);
             }
             words[2 * t] = (q[0] & 0xffff) | (q[1] << 16);
@@ -389,11 +457,12 @@ __global__ __launch_bounds__(kThreads) void conv2d_s16_gemm_kernel(const S16Args
     }
 }
 
-template <int NT, bool ALIGNED>
+template <int NT, bool ALIGNED, bool X8 = false>
 __global__ __launch_bounds__(kThreads) void conv2d_s16_narrow_kernel(const S16Args a)
 {
     constexpr int G = 2; // steps per batch of loads
-    __shared__ v4i part[4][NT][3][64];
+    constexpr int kSums = X8 ? 2 : 3;
+    __shared__ v4i part[4][NT][kSums][64];
     __shared__ long long pix_part[4][16], flt_part[4][NT][16];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -410,15 +479,20 @@ __global__ __launch_bounds__(kThreads) void conv2d_s16_narrow_kernel(const S16Ar
         row[t] = min(n0 + 4 * NT * (col >> 2) + 4 * t + (col & 3), a.out_c - 1) * a.win.w_len;
 
     struct Batch {
-        Unit16 b[G], w[G][NT];
+        std::conditional_t<X8, v4i, Unit16> b[G];
+        Unit16 w[G][NT];
         int n[G];
     };
     auto request = [&](int s0, Batch &t) {
 #pragma unroll
         for (int i = 0; i < G; i++) {
-            const Unit u = locate_unit16(a.win, 4 * (wave + 4 * (s0 + i)) + quad);
+            const int at = 4 * (wave + 4 * (s0 + i)) + quad;
+            const Unit u = X8 ? locate_unit_x8(a.win, at) : locate_unit16(a.win, at);
             t.n[i] = u.n;
-            t.b[i] = load_pixel16<ALIGNED>(a.win, in_rsrc, px, u);
+            if constexpr (X8)
+                t.b[i] = load_pixel_unit<ALIGNED>(a.win, in_rsrc, px, u);
+            else
+                t.b[i] = load_pixel16<ALIGNED>(a.win, in_rsrc, px, u);
 #pragma unroll
             for (int f = 0; f < NT; f++)
                 t.w[i][f] = load_filter16<ALIGNED>(a.win, w_rsrc, row[f], u);
@@ -440,25 +514,35 @@ __global__ __launch_bounds__(kThreads) void conv2d_s16_narrow_kernel(const S16Ar
         shift[r] = finisher ? a.shift[a.n_shift == 1 ? 0 : n] : 0;
     }
 
-    v4i acc[NT][3];
+    v4i acc[NT][kSums];
     int bh = 0, bl = 0, wh_s[NT] = {}, wl_s[NT] = {};
 #pragma unroll
     for (int t = 0; t < NT; t++)
 #pragma unroll
-        for (int s = 0; s < 3; s++)
+        for (int s = 0; s < kSums; s++)
             acc[t][s] = v4i{0, 0, 0, 0};
     auto products = [&](const Batch &t, int left) {
 #pragma unroll
         for (int i = 0; i < G; i++)
             if (i < left) { // uniform
-                const Planes x = cut(t.b[i], bh, bl);
+                v4i xh, xl;
+                if constexpr (X8) {
+                    xh = t.b[i];
+                    bh = byte_sum(xh, bh);
+                } else {
+                    const Planes x = cut(t.b[i], bh, bl);
+                    xh = x.h;
+                    xl = x.l;
+                }
 #pragma unroll
                 for (int f = 0; f < NT; f++) {
                     const Planes w = cut_filter<ALIGNED>(t.w[i][f], t.n[i], wh_s[f], wl_s[f]);
-                    acc[f][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w.h, x.h, acc[f][0], 0, 0, 0);
-                    acc[f][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w.l, x.h, acc[f][1], 0, 0, 0);
-                    acc[f][2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w.l, x.l, acc[f][2], 0, 0, 0);
-                    acc[f][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w.h, x.l, acc[f][1], 0, 0, 0);
+                    acc[f][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w.h, xh, acc[f][0], 0, 0, 0);
+                    acc[f][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w.l, xh, acc[f][1], 0, 0, 0);
+                    if constexpr (!X8) {
+                        acc[f][2] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w.l, xl, acc[f][2], 0, 0, 0);
+                        acc[f][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(w.h, xl, acc[f][1], 0, 0, 0);
+                    }
                 }
             }
     };
@@ -489,25 +573,30 @@ __global__ __launch_bounds__(kThreads) void conv2d_s16_narrow_kernel(const S16Ar
         if (quad == 0)
             flt_part[wave][t][col] = byte_term(h, l);
 #pragma unroll
-        for (int s = 0; s < 3; s++)
+        for (int s = 0; s < kSums; s++)
             part[wave][t][s][lane] = acc[t][s];
     }
     __syncthreads();
     if (!finisher || m >= a.n_pix || f0 >= a.out_c)
         return;
     v4i sum[3];
+    sum[2] = v4i{0, 0, 0, 0};
 #pragma unroll
-    for (int s = 0; s < 3; s++)
+    for (int s = 0; s < kSums; s++)
         sum[s] = part[0][wave][s][lane] + part[1][wave][s][lane] + part[2][wave][s][lane] + part[3][wave][s][lane];
     // every wavefront counted its own steps: 64 positions each
-    const long long common = pix_part[0][col] + pix_part[1][col] + pix_part[2][col] + pix_part[3][col] + 16384ll * 64 * a.ksteps;
+    const long long common = pix_part[0][col] + pix_part[1][col] + pix_part[2][col] + pix_part[3][col] +
+        (X8 ? 0 : 16384ll * 64 * a.ksteps);
     int q[4];
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         const int i = 4 * quad + r; // filter row of the tile
-        const long long flt = flt_part[0][wave][i] + flt_part[1][wave][i] + flt_part[2][wave][i] + flt_part[3][wave][i];
+        const long long flt =
+            X8 ? 0 : flt_part[0][wave][i] + flt_part[1][wave][i] + flt_part[2][wave][i] + flt_part[3][wave][i];
         q[r] = requant_s16(bias[r] + common + flt + combine(sum[0][r], sum[1][r], sum[2][r]), shift[r], a.relu != 0,
                            a.half_even != 0);
+        if (X8 && a.table != nullptr)
+            q[r] = a.table[nearest_entry(q[r], a.table_shift, a.half_even != 0)];
     }
     int16_t *dst = a.out + (long long)m * a.out_c + f0;
     if (f0 + 4 <= a.out_c) {
@@ -520,7 +609,7 @@ __global__ __launch_bounds__(kThreads) void conv2d_s16_narrow_kernel(const S16Ar
     }
 }
 
-template <int FT>
+template <int FT, bool X8>
 void launch_gemm(const S16Args &a, bool aligned, int cus, hipStream_t stream)
 {
     // 128-pixel tiles unless that leaves fewer than 1.5 workgroups per compute unit
@@ -529,13 +618,13 @@ void launch_gemm(const S16Args &a, bool aligned, int cus, hipStream_t stream)
     const bool small = tiles128 * gy * 2 < 3ll * cus;
     const dim3 grid(small ? (unsigned)((a.n_pix + 63) / 64) : (unsigned)tiles128, gy);
     if (small && aligned)
-        hipLaunchKernelGGL((conv2d_s16_gemm_kernel<1, FT, true>), grid, dim3(kThreads), 0, stream, a);
+        hipLaunchKernelGGL((conv2d_s16_gemm_kernel<1, FT, true, X8>), grid, dim3(kThreads), 0, stream, a);
     else if (small)
-        hipLaunchKernelGGL((conv2d_s16_gemm_kernel<1, FT, false>), grid, dim3(kThreads), 0, stream, a);
+        hipLaunchKernelGGL((conv2d_s16_gemm_kernel<1, FT, false, X8>), grid, dim3(kThreads), 0, stream, a);
     else if (aligned)
-        hipLaunchKernelGGL((conv2d_s16_gemm_kernel<2, FT, true>), grid, dim3(kThreads), 0, stream, a);
+        hipLaunchKernelGGL((conv2d_s16_gemm_kernel<2, FT, true, X8>), grid, dim3(kThreads), 0, stream, a);
     else
-        hipLaunchKernelGGL((conv2d_s16_gemm_kernel<2, FT, false>), grid, dim3(kThreads), 0, stream, a);
+        hipLaunchKernelGGL((conv2d_s16_gemm_kernel<2, FT, false, X8>), grid, dim3(kThreads), 0, stream, a);
 }
 
 // The geometry in bytes, as conv_window.h counts: a pixel of in_c channels is 2 in_c bytes.
@@ -551,20 +640,12 @@ int steps_of(const ConvGeom &g)
     return (g.k_h * g.k_w * ((g.in_c + 15) / 16) + 3) / 4;
 }
 
-} // namespace
-
-bool conv2d_s16_units_supports(const ConvGeom &g)
+// The kernel for a layer and its launch; a.win holds the input and the filter.
+template <bool X8>
+hipError_t launch_units(const ConvGeom &g, S16Args &a, const int64_t *bias, const int32_t *shift, int16_t *out, int cu_count,
+                        hipStream_t stream)
 {
-    return steps_of(g) < 1024 && window_supports(byte_geometry(g)); // K = 64 steps: the int32 accumulators stay exact
-}
-
-hipError_t launch_conv2d_s16_units(const ConvGeom &g, const int16_t *in, const int16_t *filter, const int64_t *bias,
-                                   const int32_t *shift, int16_t *out, int cu_count, hipStream_t stream)
-{
-    S16Args a;
-    const ConvGeom b = byte_geometry(g);
-    a.win = window_args(b, reinterpret_cast<const int8_t *>(in), reinterpret_cast<const int8_t *>(filter));
-    a.win.upt = (g.in_c + 15) / 16; // units of 32 bytes
+    a.win.upt = (g.in_c + 15) / 16; // units of 16 channels
     a.win.n_units = g.k_h * g.k_w * a.win.upt;
     a.win.fd_upt = make_fastdiv((unsigned)a.win.upt);
     a.bias = bias;
@@ -579,7 +660,7 @@ hipError_t launch_conv2d_s16_units(const ConvGeom &g, const int16_t *in, const i
     if (a.n_pix == 0)
         return hipSuccess;
     const bool aligned = (g.in_c & 15) == 0 &&
-        ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(filter)) & 15) == 0;
+        ((reinterpret_cast<uintptr_t>(a.win.in) | reinterpret_cast<uintptr_t>(a.win.w)) & 15) == 0;
     const int cus = cu_count > 0 ? cu_count : 256;
     // Expected times of the two kernels, straight lines in their work fitted to 97 layers of 56 to 720 K output pixels
     // (within 10 to 17 %): launch, the steps of one wavefront or workgroup, all of them over the device.
@@ -597,21 +678,56 @@ hipError_t launch_conv2d_s16_units(const ConvGeom &g, const int16_t *in, const i
     if (narrow_us < gemm_us) {
         const dim3 grid(tiles16, ny);
         if (two && aligned)
-            hipLaunchKernelGGL((conv2d_s16_narrow_kernel<2, true>), grid, dim3(kThreads), 0, stream, a);
+            hipLaunchKernelGGL((conv2d_s16_narrow_kernel<2, true, X8>), grid, dim3(kThreads), 0, stream, a);
         else if (two)
-            hipLaunchKernelGGL((conv2d_s16_narrow_kernel<2, false>), grid, dim3(kThreads), 0, stream, a);
+            hipLaunchKernelGGL((conv2d_s16_narrow_kernel<2, false, X8>), grid, dim3(kThreads), 0, stream, a);
         else if (aligned)
-            hipLaunchKernelGGL((conv2d_s16_narrow_kernel<1, true>), grid, dim3(kThreads), 0, stream, a);
+            hipLaunchKernelGGL((conv2d_s16_narrow_kernel<1, true, X8>), grid, dim3(kThreads), 0, stream, a);
         else
-            hipLaunchKernelGGL((conv2d_s16_narrow_kernel<1, false>), grid, dim3(kThreads), 0, stream, a);
+            hipLaunchKernelGGL((conv2d_s16_narrow_kernel<1, false, X8>), grid, dim3(kThreads), 0, stream, a);
     } else if (ft == 1) {
-        launch_gemm<1>(a, aligned, cus, stream);
+        launch_gemm<1, X8>(a, aligned, cus, stream);
     } else if (ft == 2) {
-        launch_gemm<2>(a, aligned, cus, stream);
+        launch_gemm<2, X8>(a, aligned, cus, stream);
     } else {
-        launch_gemm<4>(a, aligned, cus, stream);
+        launch_gemm<4, X8>(a, aligned, cus, stream);
     }
     return hipGetLastError();
+}
+
+} // namespace
+
+bool conv2d_s16_units_supports(const ConvGeom &g)
+{
+    return steps_of(g) < 1024 && window_supports(byte_geometry(g)); // K = 64 steps: the int32 accumulators stay exact
+}
+
+hipError_t launch_conv2d_s16_units(const ConvGeom &g, const int16_t *in, const int16_t *filter, const int64_t *bias,
+                                   const int32_t *shift, int16_t *out, int cu_count, hipStream_t stream)
+{
+    S16Args a = {};
+    a.win = window_args(byte_geometry(g), reinterpret_cast<const int8_t *>(in), reinterpret_cast<const int8_t *>(filter));
+    return launch_units<false>(g, a, bias, shift, out, cu_count, stream);
+}
+
+bool conv2d_s16_x8_supports(const ConvGeom &g, int table_size)
+{
+    return conv2d_s16_units_supports(g) && window_supports(g) && table_size <= kMostTable;
+}
+
+hipError_t launch_conv2d_s16_x8(const ConvGeom &g, const int8_t *in, const int16_t *filter, const int64_t *bias,
+                                const int32_t *shift, const int16_t *table, int table_size, int16_t *out, int cu_count,
+                                hipStream_t stream)
+{
+    S16Args a = {};
+    a.win = window_args(g, in, reinterpret_cast<const int8_t *>(filter));
+    a.win.w_len *= 2;
+    a.win.w_bytes *= 2;
+    a.table = table;
+    a.table_size = table_size;
+    for (a.table_shift = 0; table != nullptr && ((table_size - 1) << a.table_shift) < 65536;)
+        a.table_shift++;
+    return launch_units<true>(g, a, bias, shift, out, cu_count, stream);
 }
 
 } // namespace espdl

@@ -1458,6 +1458,17 @@ int espdl_hip_insert_zeros(const void *in, int32_t elem_size, int32_t batch, int
                          "insert_zeros");
 }
 
+// log2 of the input steps between a 16-bit table's entries, -1 for a size no table has
+static int table_step(int32_t table_size)
+{
+    if (table_size == 65536)
+        return 0;
+    for (int s = 0; s <= 15; s++)
+        if (table_size == (65536 >> s) + 1)
+            return s;
+    return -1;
+}
+
 int espdl_hip_lut_s16(const int16_t *in, int64_t size, const int16_t *table, int32_t table_size, int32_t round_mode,
                       int16_t *out, void *stream)
 {
@@ -1465,12 +1476,7 @@ int espdl_hip_lut_s16(const int16_t *in, int64_t size, const int16_t *table, int
         return fail(ESPDL_HIP_EINVAL, "negative size");
     if (round_mode != ESPDL_HIP_ROUND_HALF_UP && round_mode != ESPDL_HIP_ROUND_HALF_EVEN)
         return fail(ESPDL_HIP_EINVAL, "unknown round mode %d", round_mode);
-    int shift = -1;
-    if (table_size == 65536)
-        shift = 0;
-    for (int s = 0; s <= 15 && shift < 0; s++)
-        if (table_size == (65536 >> s) + 1)
-            shift = s;
+    const int shift = table_step(table_size);
     if (shift < 0)
         return fail(ESPDL_HIP_EINVAL, "table of %d entries: need 65536 / 2^n + 1 (n = 0..15) or 65536", table_size);
     if (size == 0)
@@ -1480,6 +1486,53 @@ int espdl_hip_lut_s16(const int16_t *in, int64_t size, const int16_t *table, int
     return device_status(espdl::launch_lut_s16(in, size, table, table_size, shift, round_mode == ESPDL_HIP_ROUND_HALF_EVEN,
                                                out, cu_count_cached(), reinterpret_cast<hipStream_t>(stream)),
                          "lut_s16");
+}
+
+static bool x8_layer(const espdl::ConvGeom &g)
+{
+    return espdl::conv2d_s16_x8_supports(g, 0);
+}
+
+int espdl_hip_conv2d_s16_x8_supported(const espdl_hip_conv_desc *desc, int32_t table_size)
+{
+    espdl::ConvGeom g;
+    if (desc == nullptr || desc->dtype != ESPDL_HIP_S16 || desc->group != 1 || derive_geometry(desc, &g) != ESPDL_HIP_OK ||
+        !espdl::conv_is_dense(g) || (table_size != 0 && table_step(table_size) < 0))
+        return 0;
+    const int most = images_per_launch(g, x8_layer);
+    g.batch = most;
+    return most > 0 && espdl::conv2d_s16_x8_supports(g, table_size) ? 1 : 0;
+}
+
+int espdl_hip_conv2d_s16_x8(const espdl_hip_conv_desc *desc, const int8_t *in, const int16_t *filter, const int64_t *bias,
+                            const int32_t *shift, const int16_t *table, int32_t table_size, int16_t *out, void *stream)
+{
+    espdl::ConvGeom g;
+    const int rc = derive_geometry(desc, &g);
+    if (rc != ESPDL_HIP_OK)
+        return rc;
+    if (table == nullptr)
+        table_size = 0;
+    if (!espdl_hip_conv2d_s16_x8_supported(desc, table_size))
+        return fail(ESPDL_HIP_ENOTSUP, "no kernel for this layer on an int8 input");
+    if (g.batch == 0)
+        return ESPDL_HIP_OK;
+    if (in == nullptr || filter == nullptr || shift == nullptr || out == nullptr)
+        return fail(ESPDL_HIP_EINVAL, "in, filter, shift and out must not be NULL");
+    if (misaligned(filter, 2) || misaligned(out, 2) || misaligned(table, 2) || misaligned(bias, 8) || misaligned(shift, 4))
+        return fail(ESPDL_HIP_EINVAL, "int16 tensors must be 2-byte aligned, int64 bias 8-byte aligned");
+    // in parts of the batch where a tensor is larger than a launch's offsets reach
+    espdl::ConvGeom part = g;
+    const int most = images_per_launch(g, x8_layer);
+    for (int n = 0; n < g.batch; n += most) {
+        part.batch = g.batch - n < most ? g.batch - n : most;
+        const hipError_t e = espdl::launch_conv2d_s16_x8(part, in + (size_t)n * g.in_h * g.in_w * g.in_c, filter, bias, shift, table,
+                                                         table_size, out + (size_t)n * g.out_h * g.out_w * g.out_c,
+                                                         cu_count_cached(), reinterpret_cast<hipStream_t>(stream));
+        if (e != hipSuccess)
+            return device_status(e, "conv2d_s16_x8");
+    }
+    return ESPDL_HIP_OK;
 }
 
 int espdl_hip_softmax_s8(const int8_t *in, int64_t outer, int64_t len, int64_t inner, int32_t in_exp, float *out,

@@ -195,6 +195,11 @@ hipError_t launch_conv2d_s8_stem(const ConvGeom &g, const int8_t *in, const int8
 bool conv2d_s16_units_supports(const ConvGeom &g);
 hipError_t launch_conv2d_s16_units(const ConvGeom &g, const int16_t *in, const int16_t *filter, const int64_t *bias,
                                    const int32_t *shift, int16_t *out, int cu_count, hipStream_t stream);
+// the same on an int8 input times 256, with an int16 table behind it (table_size 0: none)
+bool conv2d_s16_x8_supports(const ConvGeom &g, int table_size);
+hipError_t launch_conv2d_s16_x8(const ConvGeom &g, const int8_t *in, const int16_t *filter, const int64_t *bias,
+                                const int32_t *shift, const int16_t *table, int table_size, int16_t *out, int cu_count,
+                                hipStream_t stream);
 bool conv2d_s16_mfma_supports(const ConvGeom &g, const void *in, const void *filter, const void *out);
 hipError_t launch_conv2d_s16_mfma(const ConvGeom &g, const int16_t *in, const int16_t *filter, const int64_t *bias,
                                   const int32_t *shift, int16_t *out, int cu_count, hipStream_t stream);

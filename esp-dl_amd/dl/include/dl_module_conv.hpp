@@ -52,6 +52,8 @@ private:
     int m_lut_in_exponent = 0;   ///< exponent of the conv result that indexes a fused LUT
     int m_project_filter_pos = -1, m_project_bias_pos = -1, m_residual_pos = -1;
     int m_residual_shift = 0;
+    bool m_x8 = false;           ///< int16 convolution on an int8 input
+    int m_x8_in_exponent = 0;
     bool m_has_gap = false;      // a GlobalAveragePool behind this (1x1) convolution runs in its launch
     int m_gap_in_exponent = 0;   // exponent of the tensor the convolution used to write
     int m_own_inputs = 0; ///< inputs of the Conv itself when a plain residual Add was absorbed
@@ -100,6 +102,15 @@ public:
         m_lut_in_exponent = table_in_exponent;
     }
     bool has_fused_lut() const { return m_fused_lut != nullptr; }
+    /// int16 only: take the int8 tensor that a RequantizeLinear multiplied by 256 (its output is eight exponents finer)
+    /// as the input.  `in_exponent` is the exponent of the int16 tensor this convolution used to read.
+    void fuse_requantize(int int8_index, int in_exponent)
+    {
+        m_inputs_index[0] = int8_index;
+        m_x8 = true;
+        m_x8_in_exponent = in_exponent;
+    }
+    bool has_fused_requantize() const { return m_x8; }
     bool has_fused_project() const { return m_has_project; }
     const std::vector<int> &get_pads() const { return m_pads; }
     const std::vector<int> &get_strides() const { return m_strides; }
@@ -341,16 +352,27 @@ public:
                 DL_LOGE("Conv", "%s: %s", name.c_str(), espdl_hip_last_error());
             return;
         }
+        const int out_exponent =
+            m_fused_lut ? m_lut_in_exponent : (m_has_pre_add_exponent ? m_pre_add_exponent : output->exponent.get());
+        // (x8: the shifts belong to the int16 input that is no longer there)
         const std::vector<int32_t> shifts =
-            conv_shifts(m_fused_lut ? m_lut_in_exponent
-                                    : (m_has_pre_add_exponent ? m_pre_add_exponent : output->exponent.get()),
-                        input, filter, d.out_c);
+            conv_shifts(m_x8 ? out_exponent + input->exponent.get() - m_x8_in_exponent : out_exponent, input, filter, d.out_c);
         d.n_shift = (int32_t)shifts.size();
         const int32_t *shift_dev = m_shift.sync(shifts);
         if (m_fused_lut && !m_fused_lut->on_device()) {
             TensorBase *dev = m_fused_lut->to_device(context->stream);
             delete m_fused_lut;
             m_fused_lut = dev;
+        }
+        if (m_x8) {
+            const int rc = espdl_hip_conv2d_s16_x8(
+                &d, static_cast<const int8_t *>(input->data), static_cast<const int16_t *>(filter->data),
+                bias ? static_cast<const int64_t *>(bias->data) : nullptr, shift_dev,
+                m_fused_lut ? static_cast<const int16_t *>(m_fused_lut->data) : nullptr, m_fused_lut ? m_fused_lut->get_size() : 0,
+                static_cast<int16_t *>(output->data), context->stream);
+            if (rc != ESPDL_HIP_OK)
+                DL_LOGE("Conv", "%s: %s", name.c_str(), espdl_hip_last_error());
+            return;
         }
         TensorBase *residual = m_residual_pos >= 0 ? context->get_tensor(m_inputs_index[m_residual_pos]) : nullptr;
         if (residual && !residual->on_device()) {

@@ -248,6 +248,8 @@ esp_err_t Model::load(fbs::FbsModel *fbs_model)
         fuse_conv_gap();
     if (ret == ESP_OK && (m_fuse & FUSE_ATTENTION))
         fuse_attention();
+    if (ret == ESP_OK && (m_fuse & FUSE_CONV_LUT))
+        fuse_s16_input();
     return ret;
 }
 
@@ -865,6 +867,85 @@ void Model::fuse_attention()
             delete t;
         }
         at = 0; // positions have moved
+    }
+}
+
+// RequantizeLinear (int8 to an int16 tensor eight exponents finer: the values times 256) -> int16 Conv [-> LUT]: where
+// nobody else reads the tensors in between, the Conv reads the int8 tensor and applies the table
+// (espdl_hip_conv2d_s16_x8).
+void Model::fuse_s16_input()
+{
+    std::set<std::string> pinned;
+    for (auto &n : m_fbs_model->get_graph_outputs())
+        pinned.insert(n);
+    for (auto &n : m_fbs_model->get_test_outputs_name())
+        pinned.insert(n);
+    // position of the only reader of a tensor that may go, -1 otherwise
+    const auto sole_reader = [&](int tensor) {
+        int pos = -1, readers = 0;
+        for (size_t j = 0; j < m_execution_plan.size(); j++)
+            for (int in : m_execution_plan[j]->m_inputs_index)
+                if (in == tensor) {
+                    readers++;
+                    pos = (int)j;
+                }
+        const std::string name = m_model_context->get_tensor_name(tensor);
+        return readers == 1 && !pinned.count(name) && m_fbs_model->has_value_info(name) ? pos : -1;
+    };
+    for (size_t i = 0; i < m_execution_plan.size(); i++) {
+        auto *rq = m_execution_plan[i];
+        if (typeid(*rq) != typeid(dl::module::RequantizeLinear) || rq->m_inputs_index[0] >= CONTEXT_PARAMETER_OFFSET)
+            continue;
+        const std::string src = m_model_context->get_tensor_name(rq->m_inputs_index[0]);
+        const std::string dst = m_model_context->get_tensor_name(rq->m_outputs_index[0]);
+        const int at = sole_reader(rq->m_outputs_index[0]);
+        if (at <= (int)i || !m_fbs_model->has_value_info(src) || m_fbs_model->get_value_info_dtype(src) != DATA_TYPE_INT8 ||
+            m_fbs_model->get_value_info_dtype(dst) != DATA_TYPE_INT16 ||
+            m_fbs_model->get_value_info_exponent(dst) != m_fbs_model->get_value_info_exponent(src) - 8)
+            continue;
+        auto *conv = dynamic_cast<dl::module::Conv *>(m_execution_plan[at]);
+        const std::vector<int> shape = m_fbs_model->get_value_info_shape(src);
+        if (!conv || conv->quant_type != QUANT_TYPE_SYMM_16BIT || conv->get_group() != 1 || conv->has_fused_lut() ||
+            conv->get_pads().size() != 4 || shape.size() != 4 || conv->m_inputs_index[0] != rq->m_outputs_index[0] ||
+            (conv->get_activation() != Linear && conv->get_activation() != ReLU))
+            continue;
+        TensorBase *filter = m_model_context->get_tensor(conv->m_inputs_index[1]);
+        if (!filter || filter->shape.size() != 4)
+            continue;
+        espdl_hip_conv_desc d = {};
+        d.dtype = ESPDL_HIP_S16;
+        d.batch = 1;
+        d.in_h = shape[1];
+        d.in_w = shape[2];
+        d.in_c = shape[3];
+        d.out_c = filter->shape[3];
+        d.k_h = filter->shape[0];
+        d.k_w = filter->shape[1];
+        d.stride_h = conv->get_strides()[0];
+        d.stride_w = conv->get_strides()[1];
+        d.dil_h = conv->get_dilations()[0];
+        d.dil_w = conv->get_dilations()[1];
+        d.pad_top = conv->get_pads()[0];
+        d.pad_bottom = conv->get_pads()[1];
+        d.pad_left = conv->get_pads()[2];
+        d.pad_right = conv->get_pads()[3];
+        d.group = 1;
+        d.n_shift = 1;
+        if (espdl_hip_conv2d_s16_x8_supported(&d, 0) != 1)
+            continue;
+        conv->fuse_requantize(rq->m_inputs_index[0], m_fbs_model->get_value_info_exponent(dst));
+        const int mid = conv->m_outputs_index[0], lut_at = sole_reader(mid);
+        auto *lut = lut_at > at ? dynamic_cast<dl::module::LUT *>(m_execution_plan[lut_at]) : nullptr;
+        if (lut && lut->quant_type == QUANT_TYPE_SYMM_16BIT && lut->get_table() && lut->get_table()->dtype == DATA_TYPE_INT16 &&
+            espdl_hip_conv2d_s16_x8_supported(&d, (int32_t)lut->get_table()->get_size()) == 1) {
+            conv->fuse_lut(lut->release_table(), m_fbs_model->get_value_info_exponent(m_model_context->get_tensor_name(mid)));
+            conv->m_outputs_index[0] = lut->m_outputs_index[0];
+            delete lut;
+            m_execution_plan.erase(m_execution_plan.begin() + lut_at);
+        }
+        delete rq;
+        m_execution_plan.erase(m_execution_plan.begin() + i);
+        i--;
     }
 }
 

@@ -332,6 +332,14 @@ int espdl_hip_pad(const void *in, const int32_t *shape, int32_t dims, const int3
 int espdl_hip_lut_s16(const int16_t *in, int64_t size, const int16_t *table, int32_t table_size, int32_t round_mode,
                       int16_t *out, void *stream);
 
+/* espdl_hip_conv2d for ESPDL_HIP_S16 (group 1, dense) on an int8 input whose values stand for 256 times themselves: what
+ * RequantizeLinear to an int16 tensor eight exponents finer, Conv and (with a table) LUT give one after the other.  The
+ * shifts are those of the int16 layer, `table` as for espdl_hip_lut_s16, at most 4097 entries, or NULL; out is int16.
+ * espdl_hip_conv2d_s16_x8_supported: 1 when a kernel takes the layer with a table of that size (0: none), 0 when not. */
+int espdl_hip_conv2d_s16_x8_supported(const espdl_hip_conv_desc *desc, int32_t table_size);
+int espdl_hip_conv2d_s16_x8(const espdl_hip_conv_desc *desc, const int8_t *in, const int16_t *filter, const int64_t *bias,
+                            const int32_t *shift, const int16_t *table, int32_t table_size, int16_t *out, void *stream);
+
 /* module::Softmax on an int8 tensor (Softmax::forward_lut, esp-dl/dl/module/include/dl_module_softmax.hpp:148-217):
  * the tensor is viewed as [outer][len][inner] and normalized along len; out is float32 of the same
  * layout, out = T[q] / sum_i T[q_i] with T[q] = expf(2^in_exp * q), the sum taken in float32 in index

@@ -77,7 +77,8 @@ int espdl_graph_add_test_output(espdl_graph *g, const char *name, const int32_t 
                                 const void *data, int32_t exponent);
 
 /* round_mode: 0 half-up (portable C path), 1 half-even.  stream: hipStream_t or NULL (own stream).
- * fuse: bit mask of graph fusions, all exact: 1 folds Conv -> LUT pairs into the conv epilogue, 2 runs
+ * fuse: bit mask of graph fusions, all exact: 1 folds Conv -> LUT pairs into the conv epilogue (int16
+ * pairs together with a RequantizeLinear from int8 in front of them), 2 runs
  * depthwise Conv -> 1x1 Conv [-> Add] chains as one kernel, 4 folds the Add behind a dense Conv into the
  * conv epilogue, 8 runs a 1x1 Conv and the GlobalAveragePool behind it as one kernel, 16 keeps the outputs of a
  * Split along the last axis inside its input and lets dense 8-bit Convs write straight into the output of a

@@ -695,6 +695,33 @@ def test_conv2d_s16_channel_units(oracle, case):
     np.testing.assert_array_equal(to_host(got), want)
 
 
+@pytest.mark.parametrize("table_size", [0, 257, 4097])
+@pytest.mark.parametrize("case", S16_UNIT_CASES, ids=lambda c: c[0])
+def test_conv2d_s16_on_int8(oracle, case, table_size):
+    """The same layers on an int8 input that stands for 256 times itself, with a table behind them."""
+    announce(f"conv2d_s16_x8 {case[0]} table {table_size}")
+    name, (n, h, w, c), oc, k, stride, dil, pads, relu, half_even, s_lo, s_hi, values = case
+    rng = np.random.default_rng(0x518 + len(name))
+    lo, hi = {"min": (-128, -127), "max": (127, 128), "random": (-128, 128)}[values]
+    x = rng.integers(lo, hi, size=(n, h, w, c)).astype(np.int8)
+    f = rng.integers(256 * lo, 256 * hi, size=(oc, k[0], k[1], c)).astype(np.int16)
+    bias = rng.integers(-2**40, 2**40, size=oc).astype(np.int64)
+    shift = rng.integers(s_lo, s_hi + 1, size=oc).astype(np.int32)
+    table = rng.integers(-32768, 32768, size=table_size).astype(np.int16) if table_size else None
+    m = espdl()
+    oracle.set_threads(16)
+    got = m.conv2d_s16_x8(to_dev(x), to_dev(f), to_dev(bias), to_dev(shift), k, stride, dil, pads,
+                          m.capi.RELU if relu else m.capi.LINEAR,
+                          m.capi.ROUND_HALF_EVEN if half_even else m.capi.ROUND_HALF_UP,
+                          None if table is None else to_dev(table))
+    want = oracle.conv2d_s16(x.astype(np.int16) * 256, f, bias, shift, k, stride, dil, pads,
+                             oracle.RELU if relu else oracle.LINEAR,
+                             oracle.ROUND_HALF_EVEN if half_even else oracle.ROUND_HALF_UP)
+    if table is not None:
+        want = oracle.lut_s16(want, table, p4_ties=half_even)
+    np.testing.assert_array_equal(to_host(got), want)
+
+
 @pytest.mark.parametrize("case", DW_TILE_CASES, ids=lambda c: c[0])
 def test_depthwise_s8_tiles(oracle, case):
     announce(f"depthwise_s8 tiles {case[0]}")
