@@ -36,7 +36,8 @@ public:
     /// The model does not take ownership of `fbs_model`.  `stream` is a hipStream_t (nullptr: the
     /// model creates its own).  `fuse` is a bit mask of graph fusions: FUSE_CONV_LUT folds a LUT that directly follows a Conv
     /// into its epilogue (int16: where the Conv also takes over a RequantizeLinear from int8 in front of it), FUSE_DW_PROJECT runs depthwise Conv -> 1x1 Conv [-> Add] as one kernel,
-    /// FUSE_CONV_ADD folds the Add behind a dense Conv into its epilogue, FUSE_CONV_GAP runs a 1x1 Conv and the
+    /// FUSE_CONV_ADD folds the Add behind a dense Conv into its epilogue and joins the RequantizeLinears in front of
+    /// an Add and a Concat that read the same tensor or the pieces of one Split, FUSE_CONV_GAP runs a 1x1 Conv and the
     /// GlobalAveragePool behind it as one kernel that writes the pooled tensor only, FUSE_CHANNEL_SLICES leaves the
     /// outputs of a Split along the last axis inside its input and lets dense 8-bit Convs write straight into the
     /// output of a Concat along the last axis (the modules stay in the plan and copy only what is not in place),
@@ -108,6 +109,7 @@ private:
     void fuse_conv_gap();
     void fuse_attention();
     void fuse_s16_input();
+    void merge_requantize();
     size_t plan_bytes();
     char *staging(size_t bytes);
 

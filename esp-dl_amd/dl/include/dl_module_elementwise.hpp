@@ -539,20 +539,61 @@ public:
     }
     std::vector<std::vector<int>> get_output_shape(std::vector<std::vector<int>> &input_shapes)
     {
-        return {input_shapes[0]};
+        return {input_shapes.begin(), input_shapes.begin() + m_outputs_index.size()};
+    }
+    /// Takes over another RequantizeLinear: its tensors become input and output `at` of this one.
+    /// The pieces of a tensor that a Split cut along the channels are then one pass where they lie side by side.
+    void join(RequantizeLinear *other, int at)
+    {
+        m_inputs_index.resize(m_outputs_index.size()); // (a scale or zero point behind the tensor is not read)
+        m_inputs_index.insert(m_inputs_index.begin() + at, other->m_inputs_index[0]);
+        m_outputs_index.insert(m_outputs_index.begin() + at, other->m_outputs_index[0]);
+        inplace = MODULE_NON_INPLACE;
     }
     void forward(ModelContext *context, runtime_mode_t mode = RUNTIME_MODE_AUTO)
     {
         (void)mode;
-        TensorBase *input = context->get_tensor(m_inputs_index[0]);
-        TensorBase *output = context->get_tensor(m_outputs_index[0]);
-        if (!on_device_all({input, output}) || !output->assign(input, context->stream))
-            DL_LOGE("RequantizeLinear", "%s: assign failed", name.c_str());
+        const size_t n = m_outputs_index.size();
+        for (size_t j = 0; j < n;) {
+            TensorBase *input = context->get_tensor(m_inputs_index[j]);
+            TensorBase *output = context->get_tensor(m_outputs_index[j]);
+            if (!on_device_all({input, output})) {
+                DL_LOGE("RequantizeLinear", "%s: assign failed", name.c_str());
+                return;
+            }
+            // pieces that lie side by side in the same rows on both sides go together
+            int c = input->shape.empty() ? 0 : input->shape.back();
+            const int8_t *const in = static_cast<const int8_t *>(input->data);
+            int8_t *const out = static_cast<int8_t *>(output->data);
+            size_t k = j + 1;
+            for (; k < n && input->channel_pitch > 0 && output->channel_pitch > 0; k++) {
+                TensorBase *ni = context->get_tensor(m_inputs_index[k]), *no = context->get_tensor(m_outputs_index[k]);
+                if (!on_device_all({ni, no}) || ni->channel_pitch != input->channel_pitch ||
+                    no->channel_pitch != output->channel_pitch || ni->data != in + c || no->data != out + c ||
+                    ni->exponent != input->exponent || no->exponent != output->exponent)
+                    break;
+                c += ni->shape.back();
+            }
+            const bool ok = k == j + 1 ?
+                output->assign(input, context->stream) :
+                espdl_hip_requantize_s8_rows(in, input->channel_pitch, out, output->channel_pitch, c,
+                                             input->get_size() / input->shape.back(), input->exponent, output->exponent,
+                                             context->stream) == ESPDL_HIP_OK;
+            if (!ok)
+                DL_LOGE("RequantizeLinear", "%s: assign failed", name.c_str());
+            j = k;
+        }
     }
     /// int8 -> int8 goes row by row when either side is a channel slice of a wider tensor; a model only makes such
     /// slices where both sides are int8 (TensorBase::assign handles nothing else with a pitch on the output).
-    bool reads_channel_slice(int slot) const { return slot == 0 && quant_type == QUANT_TYPE_SYMM_8BIT; }
-    bool writes_channel_slice(int slot) const { return slot == 0 && quant_type == QUANT_TYPE_SYMM_8BIT; }
+    bool reads_channel_slice(int slot) const
+    {
+        return slot < (int)m_outputs_index.size() && quant_type == QUANT_TYPE_SYMM_8BIT;
+    }
+    bool writes_channel_slice(int slot) const
+    {
+        return slot < (int)m_outputs_index.size() && quant_type == QUANT_TYPE_SYMM_8BIT;
+    }
     static Module *deserialize(fbs::FbsModel *fbs_model, std::string node_name)
     {
         quant_type_t quant_type = QUANT_TYPE_NONE;

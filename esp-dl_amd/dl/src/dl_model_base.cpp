@@ -250,6 +250,8 @@ esp_err_t Model::load(fbs::FbsModel *fbs_model)
         fuse_attention();
     if (ret == ESP_OK && (m_fuse & FUSE_CONV_LUT))
         fuse_s16_input();
+    if (ret == ESP_OK && (m_fuse & FUSE_CONV_ADD))
+        merge_requantize();
     return ret;
 }
 
@@ -946,6 +948,69 @@ void Model::fuse_s16_input()
         delete rq;
         m_execution_plan.erase(m_execution_plan.begin() + i);
         i--;
+    }
+}
+
+// RequantizeLinear in front of an Add and of a Concat.  Two of one tensor to one exponent hold the same bytes: the first
+// stays, the readers of the second read it.  Those of the pieces of one channel Split to one exponent become one module,
+// which is one pass where the pieces lie side by side.  int8 only.
+void Model::merge_requantize()
+{
+    std::set<std::string> pinned;
+    for (auto &n : m_fbs_model->get_graph_outputs())
+        pinned.insert(n);
+    for (auto &n : m_fbs_model->get_test_outputs_name())
+        pinned.insert(n);
+    const auto name_of = [&](int tensor) { return m_model_context->get_tensor_name(tensor); };
+    const auto is_s8 = [&](int tensor) {
+        return tensor < CONTEXT_PARAMETER_OFFSET && m_fbs_model->has_value_info(name_of(tensor)) &&
+            m_fbs_model->get_value_info_dtype(name_of(tensor)) == DATA_TYPE_INT8;
+    };
+    const auto requantize_at = [&](size_t i) -> dl::module::RequantizeLinear * {
+        dl::module::Module *m = m_execution_plan[i];
+        return typeid(*m) == typeid(dl::module::RequantizeLinear) && m->quant_type == QUANT_TYPE_SYMM_8BIT &&
+                is_s8(m->m_inputs_index[0]) && is_s8(m->m_outputs_index[0]) ?
+            static_cast<dl::module::RequantizeLinear *>(m) :
+            nullptr;
+    };
+    const auto exponent_of = [&](int tensor) { return m_fbs_model->get_value_info_exponent(name_of(tensor)); };
+    // the Split that leaves this tensor, nullptr if none does
+    const auto split_of = [&](int tensor) -> dl::module::Module * {
+        for (dl::module::Module *m : m_execution_plan)
+            if (dynamic_cast<dl::module::Split *>(m) &&
+                std::count(m->m_outputs_index.begin(), m->m_outputs_index.end(), tensor))
+                return m;
+        return nullptr;
+    };
+    for (size_t i = 0; i < m_execution_plan.size(); i++) {
+        auto *first = requantize_at(i);
+        if (!first)
+            continue;
+        const int src = first->m_inputs_index[0], dst = first->m_outputs_index[0], exponent = exponent_of(dst);
+        dl::module::Module *split = split_of(src);
+        for (size_t j = i + 1; j < m_execution_plan.size(); j++) {
+            auto *other = requantize_at(j);
+            if (!other || exponent_of(other->m_outputs_index[0]) != exponent)
+                continue;
+            const int from = other->m_inputs_index[0], to = other->m_outputs_index[0];
+            if (from == src && !pinned.count(name_of(to))) {
+                for (dl::module::Module *m : m_execution_plan)
+                    std::replace(m->m_inputs_index.begin(), m->m_inputs_index.end(), to, dst);
+            } else if (split && from != src && split_of(from) == split) {
+                // in the order of the Split's outputs
+                const std::vector<int> &pieces = split->m_outputs_index;
+                const auto place = [&](int v) { return std::find(pieces.begin(), pieces.end(), v) - pieces.begin(); };
+                int at = 0;
+                while (at < (int)first->m_outputs_index.size() && place(first->m_inputs_index[at]) <= place(from))
+                    at++;
+                first->join(other, at);
+            } else {
+                continue;
+            }
+            delete other;
+            m_execution_plan.erase(m_execution_plan.begin() + j);
+            j--;
+        }
     }
 }
 

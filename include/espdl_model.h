@@ -80,7 +80,8 @@ int espdl_graph_add_test_output(espdl_graph *g, const char *name, const int32_t 
  * fuse: bit mask of graph fusions, all exact: 1 folds Conv -> LUT pairs into the conv epilogue (int16
  * pairs together with a RequantizeLinear from int8 in front of them), 2 runs
  * depthwise Conv -> 1x1 Conv [-> Add] chains as one kernel, 4 folds the Add behind a dense Conv into the
- * conv epilogue, 8 runs a 1x1 Conv and the GlobalAveragePool behind it as one kernel, 16 keeps the outputs of a
+ * conv epilogue and joins the RequantizeLinears in front of Adds and Concats that read one tensor or the pieces of one
+ * Split, 8 runs a 1x1 Conv and the GlobalAveragePool behind it as one kernel, 16 keeps the outputs of a
  * Split along the last axis inside its input and lets dense 8-bit Convs write straight into the output of a
  * Concat along the last axis, so that neither copies, 32 runs an attention block between its convolutions as one
  * kernel (63 = all).  The graph must outlive the model. */

@@ -225,6 +225,32 @@ def test_first_block_with_requantized_residual_from_the_graph_input(oracle):
     mdl.close()
 
 
+@pytest.mark.parametrize("order", [(0, 1, 2), (1, 0, 2), (0, 2)], ids=["in_order", "swapped", "one_missing"])
+@pytest.mark.parametrize("channels", [32, 40, 6])
+def test_requantized_pieces_of_a_split(oracle, order, channels):
+    """The pieces of a Split requantized in front of an Add and a Concat: one module, whose pieces lie side by side
+    in the Concat's output, in another order there, or outside of it."""
+    announce(f"model requantized pieces order={order} channels={channels}")
+    _, zoo, _, _ = _mods()
+    g = zoo.GraphSpec("requantized_pieces")
+    b = zoo.Builder(g, 0xE5F2, per_channel=True, w_exp_range=None)
+    x = b.input("input", [1, 9, 13, 16], -6)
+    h = b.conv(x, 2 * channels, k=1, out_exp=-6, name="cv1")
+    p0, p1 = b.split(h, [channels, channels], name="split")
+    m = b.conv(p1, channels, k=3, out_exp=-5, name="m")
+    a = b.requantize(p1, -5, with_scale_input=True)
+    m = b.add(a, m, name="add")
+    parts = [b.requantize(p0, -5, with_scale_input=True), b.requantize(p1, -5), m]
+    b.output(b.conv(b.concat([parts[i] for i in order], name="cat"), 24, k=1, name="cv2"))
+    mdl, want, _ = _run_config(g, 3, 48)
+    # cv1, Split, the requantized pieces, m with its Add, Concat, cv2
+    assert sum(1 for n in g.nodes if n["op_type"] == "RequantizeLinear") == 3 and mdl.module_count() == 6
+    for rep in range(2):
+        np.testing.assert_array_equal(mdl.get_tensor(g.outputs[0]), want[g.outputs[0]])
+        mdl.run()
+    mdl.close()
+
+
 def test_channel_slices_every_case(oracle):
     """Split outputs left inside the Split's input and Concat inputs written in place, case by case: which
     tensors become slices (by their pitch), every tensor against the oracle, twice (the slices must survive a
