@@ -9,6 +9,7 @@
 // kernels on one HIP stream, and the launch-bound plan can be replayed from a HIP graph.
 #pragma once
 
+#include <atomic>
 #include <map>
 #include <mutex>
 #include <string>
@@ -63,6 +64,7 @@ public:
     /// Run segment `stage_index` of `stage_num` near-equal segments of the plan (dl_model_base.cpp:240-260).
     virtual void run(int stage_num, int stage_index, runtime_mode_t mode = RUNTIME_MODE_SINGLE_CORE);
     /// Enqueue only; pair with synchronize().  Uses the captured HIP graph when enable_graph() succeeded.
+    /// The launches of a pass stand together on the stream: passes of several threads follow one another, whole.
     void run_async(runtime_mode_t mode = RUNTIME_MODE_SINGLE_CORE);
     void synchronize();
     /// Capture the plan into a HIP graph (after one eager run has created every module's device state).  A short
@@ -130,9 +132,12 @@ private:
     char *m_staging = nullptr;    // pinned host memory of read_tensor / write_tensor
     size_t m_staging_bytes = 0;
     std::mutex m_staging_mutex;
+    // Held while a pass is enqueued.  All passes use one arena, whose blocks are used again inside a pass: the launches
+    // of two passes in turn would overwrite each other's tensors.
+    std::mutex m_pass_mutex;
     bool m_built = false;
-    bool m_failed = false;
-    long m_errors_at_start = 0;
+    std::atomic<bool> m_failed{false};
+    std::atomic<long> m_errors_at_start{0};
     void begin_pass()
     {
         m_failed = false;

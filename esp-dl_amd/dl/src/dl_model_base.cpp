@@ -1366,6 +1366,7 @@ esp_err_t Model::build(int batch)
 
 void Model::run_async(runtime_mode_t mode)
 {
+    std::lock_guard<std::mutex> pass(m_pass_mutex);
     begin_pass();
     if (!m_built) {
         m_failed = true;
@@ -1509,6 +1510,7 @@ void Model::run(int stage_num, int stage_index, runtime_mode_t mode)
         DL_LOGE(TAG, "Invalid stage_index(%d), it should be in range [0, %d).", stage_index, stage_num);
         return;
     }
+    std::lock_guard<std::mutex> pass(m_pass_mutex);
     begin_pass();
     const int start = stage_index * plan_size / stage_num;
     const int end = (stage_index + 1) * plan_size / stage_num;
@@ -1519,6 +1521,7 @@ void Model::run(int stage_num, int stage_index, runtime_mode_t mode)
 
 bool Model::enable_graph()
 {
+    std::lock_guard<std::mutex> pass(m_pass_mutex);
     if (!m_built || m_graph_exec)
         return m_graph_exec != nullptr;
     begin_pass();
@@ -1575,6 +1578,7 @@ size_t Model::plan_bytes()
 
 void Model::disable_graph()
 {
+    std::lock_guard<std::mutex> pass(m_pass_mutex);
     delete static_cast<LaunchList *>(m_launches);
     m_launches = nullptr;
     if (m_graph_exec) {
@@ -1592,6 +1596,7 @@ esp_err_t Model::test()
 {
     if (!m_built)
         return ESP_FAIL;
+    std::lock_guard<std::mutex> pass(m_pass_mutex);
     begin_pass();
     for (auto &kv : m_inputs) {
         TensorBase *test_input = m_fbs_model->get_test_input_tensor(kv.first);
@@ -1652,6 +1657,7 @@ std::vector<module_info> Model::get_module_info(int repeats)
     std::vector<module_info> info;
     if (!m_built)
         return info;
+    std::lock_guard<std::mutex> pass(m_pass_mutex);
     hipStream_t s = static_cast<hipStream_t>(m_stream);
     if (repeats < 1)
         repeats = 1;

@@ -91,7 +91,9 @@ void espdl_model_destroy(espdl_model *m);
  * that is not on the device, a shape a kernel refuses) can only log.  The model counts what is logged
  * during a pass: run / run_async / synchronize return -2 when a module of the current pass logged an
  * error or a HIP call failed; the tensors of such a pass are not valid results.  enable_graph refuses to
- * capture a plan with a failing module. */
+ * capture a plan with a failing module.
+ * Several threads may enqueue passes of one model: a pass is enqueued as a whole, in whatever order the threads come.
+ * The tensors are the model's own, so what one pass reads and leaves there is the callers' to agree on. */
 int espdl_model_run(espdl_model *m);       /* enqueue + wait */
 int espdl_model_run_async(espdl_model *m); /* enqueue only   */
 int espdl_model_synchronize(espdl_model *m);

@@ -1,0 +1,40 @@
+"""What the host side does around the kernels, looked at without a GPU: a stand-in for the HIP runtime (host_hip.py) logs
+the launches, allocations and graphs."""
+import pytest
+
+import host_hip
+
+
+@pytest.mark.parametrize("captured", [True, False], ids=["captured", "eager"])
+def test_passes_of_two_threads_do_not_interleave(captured):
+    """Every pass writes the same arena, so the launches of one run_async may not stand between those of another."""
+    host_hip.run('''
+    import threading
+    mdl = model.Model(model.Graph.from_spec(zoo.config2_mbv2_block()), 2)
+    mdl.run()
+    if %d:
+        assert mdl.enable_graph()
+    hip.host_hip_clear()
+    mdl.run_async()
+    one = [l["name"] for l in launches()]
+    assert len(one) > 1
+    hip.host_hip_clear()
+    hip.host_hip_delay(200)
+    start = threading.Barrier(2)
+
+    def passes():
+        start.wait()
+        for _ in range(40):
+            mdl.run_async()
+
+    threads = [threading.Thread(target=passes) for _ in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    log = launches()
+    assert len(log) == 80 * len(one) and len({l["thread"] for l in log}) == 2
+    for i in range(0, len(log), len(one)):
+        part = log[i:i + len(one)]
+        assert [l["name"] for l in part] == one and len({l["thread"] for l in part}) == 1, i
+    ''' % captured)
