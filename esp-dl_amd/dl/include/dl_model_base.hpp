@@ -71,7 +71,7 @@ public:
     /// chain of kernels that the host keeps ahead of is replayed as plain launches, anything else as the graph.
     bool enable_graph();
     void disable_graph();
-    bool graph_enabled() const { return m_graph_exec != nullptr; }
+    bool graph_enabled() const { return m_graph_exec != nullptr || m_launches != nullptr; }
     /// True when a module logged an error (a rejected kernel launch, a host tensor handed to a device
     /// module) or a HIP call failed since the last run / run_async / enable_graph / test began.  The
     /// tensors a failed pass leaves behind are not valid results.
@@ -127,8 +127,8 @@ private:
     void *m_stream = nullptr;
     bool m_own_stream = false;
     void *m_graph = nullptr;      // hipGraph_t
-    void *m_graph_exec = nullptr; // hipGraphExec_t
-    void *m_launches = nullptr;   // the captured kernels of a short plan, replayed without the graph
+    void *m_graph_exec = nullptr; // hipGraphExec_t, where the plan is replayed as a graph
+    void *m_launches = nullptr;   // the captured kernels of a short plan, replayed without a graph launch
     char *m_staging = nullptr;    // pinned host memory of read_tensor / write_tensor
     size_t m_staging_bytes = 0;
     std::mutex m_staging_mutex;

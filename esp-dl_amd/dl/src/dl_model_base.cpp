@@ -1522,8 +1522,8 @@ void Model::run(int stage_num, int stage_index, runtime_mode_t mode)
 bool Model::enable_graph()
 {
     std::lock_guard<std::mutex> pass(m_pass_mutex);
-    if (!m_built || m_graph_exec)
-        return m_graph_exec != nullptr;
+    if (!m_built || graph_enabled())
+        return graph_enabled();
     begin_pass();
     hipStream_t s = static_cast<hipStream_t>(m_stream);
     // one eager pass so that every module has uploaded its shifts / tables before capture starts; modules that
@@ -1547,19 +1547,19 @@ bool Model::enable_graph()
         (void)hipGraphDestroy(graph);
         return false;
     }
-    hipGraphExec_t exec = nullptr;
-    if (!hip_ok(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0), "hipGraphInstantiate")) {
-        (void)hipGraphDestroy(graph);
-        return false;
-    }
-    m_graph = graph;
-    m_graph_exec = exec;
     LaunchList *list = chain_of_kernels(graph);
     (void)hipGetLastError(); // a refused query must not surface as the error of a later launch
     if (list != nullptr && list->launches.size() > kDirectAlways && plan_bytes() < kDirectBytes * list->launches.size()) {
         delete list;
         list = nullptr;
     }
+    hipGraphExec_t exec = nullptr; // the list needs none: it is launched from the parameters that the graph holds
+    if (list == nullptr && !hip_ok(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0), "hipGraphInstantiate")) {
+        (void)hipGraphDestroy(graph);
+        return false;
+    }
+    m_graph = graph;
+    m_graph_exec = exec;
     m_launches = list;
     return true;
 }
@@ -1579,10 +1579,11 @@ size_t Model::plan_bytes()
 void Model::disable_graph()
 {
     std::lock_guard<std::mutex> pass(m_pass_mutex);
+    if (graph_enabled())
+        (void)hipStreamSynchronize(static_cast<hipStream_t>(m_stream));
     delete static_cast<LaunchList *>(m_launches);
     m_launches = nullptr;
     if (m_graph_exec) {
-        (void)hipStreamSynchronize(static_cast<hipStream_t>(m_stream));
         (void)hipGraphExecDestroy(static_cast<hipGraphExec_t>(m_graph_exec));
         m_graph_exec = nullptr;
     }

@@ -38,3 +38,27 @@ def test_passes_of_two_threads_do_not_interleave(captured):
         part = log[i:i + len(one)]
         assert [l["name"] for l in part] == one and len({l["thread"] for l in part}) == 1, i
     ''' % captured)
+
+
+def test_a_plan_replayed_as_launches_makes_no_graph_exec():
+    """enable_graph instantiates only what run_async launches: a short plan is replayed from its launch list, a plan of
+    many small launches as the graph."""
+    host_hip.run('''
+    def enabled(spec, batch):
+        mdl = model.Model(model.Graph.from_spec(spec), batch)
+        hip.host_hip_clear()
+        assert mdl.enable_graph() and mdl.enable_graph()  # (the second call finds it done)
+        made = hip.host_hip_calls(b"hipGraphInstantiate")
+        hip.host_hip_clear()
+        mdl.run()
+        replayed = hip.host_hip_launches(), hip.host_hip_calls(b"hipGraphLaunch")
+        mdl.disable_graph()
+        hip.host_hip_clear()
+        mdl.run()
+        return made, replayed, hip.host_hip_launches()
+
+    made, (plain, graphs), eager = enabled(zoo.config1_single_conv(), 1)
+    assert (made, plain, graphs, eager) == (0, 1, 0, 1)
+    made, (plain, graphs), eager = enabled(zoo.config3_mobilenetv2(resolution=96), 1)
+    assert (made, plain, graphs) == (1, 0, 1) and eager > 24
+    ''')
