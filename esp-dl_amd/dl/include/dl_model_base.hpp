@@ -81,6 +81,8 @@ public:
     esp_err_t test();
     std::vector<module_info> get_module_info(int repeats = 3);
     void profile(bool sort_module_by_latency = false);
+    /// Device: activation arena, parameters and the workspace of modules that run as several launches (it is there from
+    /// the first pass on).  Host: pinned memory that copies of whole tensors pass through (from the first such copy on).
     mem_info_t get_memory_info();
 
     /// Copy a whole dense device tensor from / to host memory on the model's stream; done on return.

@@ -1777,14 +1777,20 @@ void Model::profile(bool sort_module_by_latency)
                     m.latency_us > 0 ? m.bytes / m.latency_us * 1e-3 : 0.0);
     std::printf("total %.2f us for batch %d\n", total, m_batch);
     mem_info_t mem = get_memory_info();
-    std::printf("device memory: %zu bytes (activation arena + parameters)\n", mem.device);
+    std::printf("device memory: %zu bytes (activation arena + parameters + workspace)\n", mem.device);
+    std::printf("host memory: %zu bytes (pinned, for copies)\n", mem.host);
 }
 
 mem_info_t Model::get_memory_info()
 {
     mem_info_t m;
-    m.device = m_model_context->get_variable_memory_size() + m_model_context->get_parameter_memory_size();
-    m.host = 0;
+    {
+        std::lock_guard<std::mutex> pass(m_pass_mutex);
+        m.device = m_model_context->get_variable_memory_size() + m_model_context->get_parameter_memory_size() +
+            m_model_context->get_workspace_size();
+    }
+    std::lock_guard<std::mutex> lock(m_staging_mutex);
+    m.host = m_staging_bytes;
     return m;
 }
 

@@ -117,6 +117,7 @@ int espdl_model_tensor_exponent(espdl_model *m, const char *name, int32_t *expon
 int espdl_model_tensor_channel_pitch(espdl_model *m, const char *name);
 int espdl_model_set_input(espdl_model *m, const char *name, const void *host_data, int64_t bytes);
 int espdl_model_get_tensor(espdl_model *m, const char *name, void *host_data, int64_t bytes);
+/* Activation arena, parameters and, from the first pass on, the workspace of blocks that run as two launches. */
 int64_t espdl_model_device_bytes(espdl_model *m);
 void *espdl_model_stream(espdl_model *m);
 

@@ -62,3 +62,25 @@ def test_a_plan_replayed_as_launches_makes_no_graph_exec():
     made, (plain, graphs), eager = enabled(zoo.config3_mobilenetv2(resolution=96), 1)
     assert (made, plain, graphs) == (1, 0, 1) and eager > 24
     ''')
+
+
+def test_memory_queries_count_the_workspace_and_the_staging():
+    """A block run as two launches keeps its depthwise result in the model's workspace, and host copies pass through
+    pinned memory of the model's own: both are the model's memory."""
+    out = host_hip.run('''
+    spec = zoo.config2_mbv2_block()
+    mdl = model.Model(model.Graph.from_spec(spec), 2)
+    before = mdl.device_bytes()
+    mdl.run()
+    assert len(launches()) == 2
+    assert mdl.device_bytes() == before + 2 * 56 * 56 * 144, (before, mdl.device_bytes())
+    m.model.lib().espdl_model_print_profile(mdl.h)  # nothing was copied yet
+    mdl.get_tensor(spec.outputs[0])                 # too large for the staging
+    m.model.lib().espdl_model_print_profile(mdl.h)
+    spec = zoo.config3_mobilenetv2(resolution=96)
+    small = model.Model(model.Graph.from_spec(spec), 1)
+    small.get_tensor(spec.outputs[0])
+    m.model.lib().espdl_model_print_profile(small.h)
+    ''')
+    pinned = [int(line.split()[2]) for line in out.splitlines() if line.startswith("host memory:")]
+    assert pinned == [0, 0, 65536]
