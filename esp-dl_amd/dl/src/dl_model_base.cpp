@@ -392,6 +392,8 @@ void Model::fuse_dw_project()
         d.pad_left = dw->get_pads()[2];
         d.pad_right = dw->get_pads()[3];
         d.n_shift_expand = d.n_shift_dw = d.n_shift_project = 1;
+        // (what the kernels take depends on it: a Clip between the stages has no single launch in half-even mode)
+        d.round_mode = m_model_context->round_mode == ROUND_MODE_HALF_EVEN ? ESPDL_HIP_ROUND_HALF_EVEN : ESPDL_HIP_ROUND_HALF_UP;
         if (clip_d) {
             d.clip_dw = 1;
             d.clip_dw_min = clip_d->get_min();
@@ -405,7 +407,7 @@ void Model::fuse_dw_project()
         dl::module::Conv *ex = nullptr;
         dl::module::Clip *clip_e = nullptr;
         int ex_kernel[2] = {1, 1};
-        bool two_launches = false;
+        bool two_launches = false, only_two = false; // only_two: there is no single launch
         espdl_hip_mbconv_desc de = d; // the whole block, when a Conv in front joins
         {
             int dw_in = dw->m_inputs_index[0];
@@ -476,9 +478,11 @@ void Model::fuse_dw_project()
                     de.exp_pad_left = ex->get_pads()[2];
                     de.exp_pad_right = ex->get_pads()[3];
                 }
-                // one launch, or two (expand + depthwise, project) where that beats separate launches
+                // one launch, or two (expand + depthwise, project) where that beats separate launches; a Clip in half-even
+                // mode runs as two wherever that form exists (a stem in front, for one, leaves the modules separate)
                 if (espdl_hip_mbconv_s8_preferred(&de) != 1) {
-                    two_launches = espdl_hip_mbconv_s8_supported(&de) != 0 && espdl_hip_mbconv_s8_workspace(&de) > 0;
+                    only_two = de.round_mode == ESPDL_HIP_ROUND_HALF_EVEN && (de.clip_expand || de.clip_dw);
+                    two_launches = (only_two || espdl_hip_mbconv_s8_supported(&de) != 0) && espdl_hip_mbconv_s8_workspace(&de) > 0;
                     if (!two_launches)
                         ex = nullptr;
                 }
@@ -541,7 +545,7 @@ void Model::fuse_dw_project()
                 if (!m_fbs_model->has_value_info(src_name) || m_fbs_model->get_value_info_dtype(src_name) != DATA_TYPE_INT8 ||
                     m_fbs_model->get_value_info_dtype(res_name) != DATA_TYPE_INT8 ||
                     m_fbs_model->get_value_info_shape(src_name) != m_fbs_model->get_value_info_shape(res_name) || shift == 0 ||
-                    shift < -7 || shift > 7 || espdl_hip_mbconv_s8_preferred(&de) != 1)
+                    shift < -7 || shift > 7 || (only_two ? espdl_hip_mbconv_s8_workspace(&de) <= 0 : espdl_hip_mbconv_s8_preferred(&de) != 1))
                     rq = nullptr;
                 else
                     residual = rq->m_inputs_index[0];

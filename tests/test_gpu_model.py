@@ -225,6 +225,36 @@ def test_first_block_with_requantized_residual_from_the_graph_input(oracle):
     mdl.close()
 
 
+def clip_block(shape, exp_c, out_c, stride, stem):
+    """Conv -> Clip -> depthwise Conv -> Clip -> 1x1 Conv [-> Add]; `stem`: the first Conv is 3x3 at stride 2."""
+    _, zoo, _, _ = _mods()
+    g = zoo.GraphSpec("clip_block")
+    b = zoo.Builder(g, 0xE5F7, per_channel=True)
+    x = b.input("input", [1, *shape], -5)
+    e = b.clip(b.conv(x, exp_c, k=3 if stem else 1, stride=2 if stem else 1, name="expand"), 0, 90, name="clip_a")
+    d = b.clip(b.conv(e, None, k=3, stride=stride, depthwise=True, name="dw"), -3, 77, name="clip_b")
+    p = b.conv(d, out_c, k=1, name="project")
+    b.output(b.add(x, p, name="residual") if shape[2] == out_c and stride == 1 and not stem else p)
+    return g
+
+
+# (input shape, expanded and output channels, stride, stem, batch, modules in half-up and in half-even mode): one launch in
+# half-up mode and two in half-even mode, a shape without a single launch with Clips, which half-up leaves as separate
+# modules, and a stem, which half-even does
+@pytest.mark.parametrize("round_mode", [0, 1], ids=["half_up", "half_even"])
+@pytest.mark.parametrize("case", [((56, 56, 24), 144, 24, 1, False, 3, (1, 1)), ((28, 28, 32), 192, 64, 2, False, 4, (1, 1)),
+                                  ((14, 14, 64), 384, 64, 1, False, 3, (6, 1)), ((224, 224, 3), 32, 16, 1, True, 2, (1, 5)),
+                                  ((30, 37, 16), 96, 24, 2, False, 2, (1, 1))], ids=lambda c: "x".join(map(str, c[0])))
+def test_blocks_with_clips(oracle, case, round_mode):
+    announce(f"model block with Clips {case[0]} round mode {round_mode}")
+    shape, exp_c, out_c, stride, stem, batch, modules = case
+    spec = clip_block(shape, exp_c, out_c, stride, stem)
+    mdl, want, _ = _run_config(spec, batch, 49, round_mode=round_mode)
+    np.testing.assert_array_equal(mdl.get_tensor(spec.outputs[0]), want[spec.outputs[0]])
+    assert mdl.module_count() == modules[round_mode]
+    mdl.close()
+
+
 @pytest.mark.parametrize("order", [(0, 1, 2), (1, 0, 2), (0, 2)], ids=["in_order", "swapped", "one_missing"])
 @pytest.mark.parametrize("channels", [32, 40, 6])
 def test_requantized_pieces_of_a_split(oracle, order, channels):

@@ -84,3 +84,19 @@ def test_memory_queries_count_the_workspace_and_the_staging():
     ''')
     pinned = [int(line.split()[2]) for line in out.splitlines() if line.startswith("host memory:")]
     assert pinned == [0, 0, 65536]
+
+
+@pytest.mark.parametrize("round_mode", [0, 1], ids=["half_up", "half_even"])
+def test_fused_blocks_with_clips_have_a_kernel(round_mode):
+    """What fuse_dw_project joins must have a launch in the model's rounding mode: pointwise blocks with and without a single
+    launch, and a stem in front of the first block (the kernels are not run here)."""
+    host_hip.run("""
+    import test_gpu_model
+    for shape, exp, out, stride, stem, batch in [((56, 56, 24), 144, 24, 1, False, 2), ((56, 56, 24), 144, 24, 1, False, 256),
+                                                 ((28, 28, 32), 192, 64, 2, False, 4), ((14, 14, 64), 384, 64, 1, False, 3),
+                                                 ((224, 224, 3), 32, 16, 1, True, 2)]:
+        spec = test_gpu_model.clip_block(shape, exp, out, stride, stem)
+        mdl = model.Model(model.Graph.from_spec(spec), batch, round_mode=%d)
+        mdl.run()  # raises where a module's launch is refused
+        mdl.close()
+    """ % round_mode)
