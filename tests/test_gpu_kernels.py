@@ -488,9 +488,9 @@ def test_gemm_s8(oracle, m, k, n, has_bias, relu):
 @pytest.mark.parametrize("m,k,n,pad", [(1024, 16, 2049, 0), (1031, 17, 2303, 0), (1100, 64, 2305, 0), (5000, 65, 2055, 0),
                                        (1400, 128, 6625, 0), (40000, 120, 2119, 0), (1025, 33, 2064, 5)])
 @pytest.mark.parametrize("variant", ["per_channel", "per_tensor", "half_even", "wide_shifts"])
-def test_conv2d_s8_wide_rows(oracle, m, k, n, pad, variant):
+def test_conv2d_s8_wide_filters(oracle, m, k, n, pad, variant):
     import torch
-    announce(f"conv2d_s8 wide rows M={m} K={k} N={n} pad={pad} {variant}")
+    announce(f"conv2d_s8 wide filters M={m} K={k} N={n} pad={pad} {variant}")
     rng = np.random.default_rng(0xF5 + m + n)
     x, f = rng_int8(rng, (m, 1, 1, k)), rng_int8(rng, (n, 1, 1, k))
     bias = None if variant == "per_tensor" else rng.integers(-4096, 4097, size=n).astype(np.int32)
