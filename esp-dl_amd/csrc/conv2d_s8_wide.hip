@@ -14,6 +14,7 @@
 //
 // Restates conv2d_11cn (esp-dl/dl/base/dl_base_conv2d.cpp:9-33) with the n_wise epilogue
 // (esp-dl/dl/base/dl_base_activate_buffer.hpp:27-36, 61-72, 173-181, 201-210).
+#include <atomic>
 #include <type_traits>
 
 #include "conv_window.h"
@@ -27,6 +28,8 @@ typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;
 constexpr int kRow = 16 + 256; // a row of the output tile in LDS: the 16 bytes in front, then those of the step
+constexpr int kTileBytes = 64 * kRow + 16;
+constexpr int kMaxSteps = 12; // of a walk
 
 struct WideArgs {
     const int8_t *in, *w;
@@ -41,7 +44,7 @@ struct WideArgs {
 template <int KS>
 __global__ __launch_bounds__(kThreads, 2) void conv2d_s8_wide_kernel(const WideArgs a)
 {
-    __shared__ __align__(16) unsigned char tile[2][64 * kRow + 16];
+    __shared__ __align__(16) unsigned char tile[2][kTileBytes];
     extern __shared__ __align__(16) int cst[]; // per filter of the walk: start value | right shift | left shift
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int col = lane & 15, quad = lane >> 4;
@@ -227,6 +230,29 @@ __global__ __launch_bounds__(kThreads, 2) void conv2d_s8_wide_kernel(const WideA
         walk(std::integral_constant<int, 1>{});
 }
 
+// The tile and the constants of walks of 10 steps and more are past the 64 KB of LDS that a launch may have unasked
+// (twelve steps: 70 KB, two workgroups to a compute unit as before): the limit is raised once per device (bit d: done on
+// device d; two threads may both do it).
+template <int KS>
+hipError_t allow_lds(size_t dynamic)
+{
+    if (2 * kTileBytes + dynamic <= 64 * 1024)
+        return hipSuccess;
+    static std::atomic<unsigned long long> raised{0};
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess)
+        return e;
+    const unsigned long long bit = 1ull << (dev & 63);
+    if (dev < 64 && (raised.load(std::memory_order_relaxed) & bit))
+        return hipSuccess;
+    e = hipFuncSetAttribute(reinterpret_cast<const void *>(conv2d_s8_wide_kernel<KS>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            3 * (int)sizeof(int) * 256 * kMaxSteps);
+    if (e == hipSuccess && dev < 64)
+        raised.fetch_or(bit, std::memory_order_relaxed);
+    return e;
+}
+
 } // namespace
 
 // Rows of the result that are no multiple of 16 bytes long, which the other kernels write in pieces at odd addresses, and
@@ -263,12 +289,12 @@ hipError_t launch_conv2d_s8_wide(const ConvGeom &g, const int8_t *in, const int8
     if (a.M == 0)
         return hipSuccess;
     // Steps per walk: rounds of workgroups (two fit a compute unit) times a walk and its start, which costs about four
-    // steps; twelve steps' constants at most lie in LDS.
+    // steps; kMaxSteps steps' constants at most lie in LDS.
     const int tiles = (a.M + 63) / 64, steps = (a.N + 255) / 256;
     const long long slots = 2ll * std::max(1, cu_count);
     int per = 1;
     long long best = 0;
-    for (int p = 1; p <= std::min(steps, 12); p++) {
+    for (int p = 1; p <= std::min(steps, kMaxSteps); p++) {
         const long long cost = ((long long)tiles * ((steps + p - 1) / p) + slots - 1) / slots * (p + 4);
         if (p == 1 || cost < best) {
             best = cost;
@@ -278,6 +304,9 @@ hipError_t launch_conv2d_s8_wide(const ConvGeom &g, const int8_t *in, const int8
     a.per_walk = 256 * per;
     const dim3 grid((unsigned)tiles, (unsigned)((steps + per - 1) / per));
     const size_t lds = (size_t)3 * sizeof(int) * a.per_walk;
+    const hipError_t e = a.K <= 64 ? allow_lds<1>(lds) : allow_lds<2>(lds);
+    if (e != hipSuccess)
+        return e;
     if (a.K <= 64)
         hipLaunchKernelGGL(conv2d_s8_wide_kernel<1>, grid, dim3(kThreads), lds, stream, a);
     else

@@ -510,6 +510,32 @@ def test_conv2d_s8_wide_filters(oracle, m, k, n, pad, variant):
     assert (np.delete(got, np.s_[lo_c:lo_c + n], axis=3) == 77).all()
 
 
+# Walks of 10, 11 and 12 steps, whose constants take the kernel past 64 KB of LDS.
+@pytest.mark.parametrize("m,k,n", [(20003, 64, 2305), (20480, 17, 2563), (30000, 80, 2817)])
+def test_conv2d_s8_wide_filters_long_walks(oracle, m, k, n):
+    announce(f"conv2d_s8 wide filters, long walks M={m} K={k} N={n}")
+    rng = np.random.default_rng(0xF6 + n)
+    x, f = rng_int8(rng, (m, 1, 1, k)), rng_int8(rng, (n, 1, 1, k))
+    bias = rng.integers(-4096, 4097, size=n).astype(np.int32)
+    shift = rng.integers(6, 12, size=n).astype(np.int32)
+    oracle.set_threads(16)
+    got, want = _run_conv_s8(oracle, x, f, bias, shift, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True)
+    np.testing.assert_array_equal(got, want)
+
+
+# Walks of 10, 11 and 12 steps, whose constants take the kernel past 64 KB of LDS.
+@pytest.mark.parametrize("m,k,n", [(20003, 64, 2305), (20480, 17, 2563), (30000, 80, 2817)])
+def test_conv2d_s8_wide_filters_long_walks(oracle, m, k, n):
+    announce(f"conv2d_s8 wide filters, long walks M={m} K={k} N={n}")
+    rng = np.random.default_rng(0xF6 + n)
+    x, f = rng_int8(rng, (m, 1, 1, k)), rng_int8(rng, (n, 1, 1, k))
+    bias = rng.integers(-4096, 4097, size=n).astype(np.int32)
+    shift = rng.integers(6, 12, size=n).astype(np.int32)
+    oracle.set_threads(16)
+    got, want = _run_conv_s8(oracle, x, f, bias, shift, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True)
+    np.testing.assert_array_equal(got, want)
+
+
 # Products with so few rows that the tiled kernels would leave most of the device idle go to a kernel with one
 # wavefront per 16 x 16 tile: ragged row and filter counts, byte stores (N not a multiple of 4), one shift for all
 # filters, shifts outside 1..31, both roundings.

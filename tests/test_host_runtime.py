@@ -100,3 +100,18 @@ def test_fused_blocks_with_clips_have_a_kernel(round_mode):
         mdl.run()  # raises where a module's launch is refused
         mdl.close()
     """ % round_mode)
+
+
+def test_wide_filter_walks_ask_for_lds_that_the_kernel_may_have():
+    """A launch past 64 KB of LDS (34848 bytes of the kernel's own and the walk's constants) needs the kernel's limit raised;
+    walks of 9 to 12 steps."""
+    host_hip.run("""
+    for rows, filters, steps in [(20480, 6625, 9), (20003, 2305, 10), (20480, 2563, 11), (30000, 2817, 12)]:
+        desc = m.capi.make_desc((rows, 1, 1, 64), filters, (1, 1))
+        hip.host_hip_clear()
+        rc = m.lib().espdl_hip_conv2d(ctypes.byref(desc), 1 << 20, 1 << 30, None, 1 << 31, None, 1 << 32, None)
+        log = launches()
+        assert rc == 0 and len(log) == 1 and "conv2d_s8_wide" in log[0]["name"], (rc, log)
+        assert log[0]["lds"] == 3 * 4 * 256 * steps
+        assert 34848 + log[0]["lds"] <= 65536 or log[0]["limit"] >= log[0]["lds"], log
+    """)
