@@ -237,6 +237,29 @@ __global__ __launch_bounds__(kThreads) void depthwise_s8_strip_kernel(const Stri
     }
 }
 
+// Strips per image.  A strip of R rows turns R + 2 of them and starts once (2.5 rows' worth), and the rounds of wavefronts
+// (four fit a SIMD) should come out even; few rows where there are few wavefronts.  Within 10 % of the best of 1 to 56 rows
+// on sixteen layers from 8 to 300 MB.  Of the strip counts with the same number of rows only the smallest counts, which
+// leaves 2 sqrt(out_h) of them, and from where even rounds would cost more than the best found no later one is better: at
+// most some microseconds on a layer of a million rows (one count after the other: 5 ms).
+int strip_count(long long per_strip, int out_h, int cu_count)
+{
+    const double capacity = 64.0 * 4 * 4 * std::max(1, cu_count);
+    int strips = 1;
+    double best = 0;
+    for (int s = 1;;) {
+        const int rows = (out_h + s - 1) / s;
+        const double cost = std::ceil(per_strip * s / capacity) * (rows + 2.5);
+        if (s == 1 || cost < best) {
+            best = cost;
+            strips = s;
+        }
+        if (rows == 1 || per_strip / capacity * (out_h + 2.5 * s) > best)
+            return strips;
+        s = (out_h + rows - 2) / (rows - 1);
+    }
+}
+
 } // namespace
 
 bool depthwise_s8_strip_supports(const ConvGeom &g)
@@ -274,23 +297,8 @@ hipError_t launch_depthwise_s8_strip(const ConvGeom &g, const int8_t *in, const 
     const int most = (int)std::max(1ll, ((1ll << 30) - 64) / std::max(in_image, out_image));
     for (int n0 = 0; n0 < g.batch; n0 += most) {
         const int n = std::min(most, g.batch - n0);
-        // Rows per strip: a strip of R rows turns R + 2 of them and starts once (2.5 rows' worth), and the rounds of
-        // wavefronts (four fit a SIMD) should come out even; few rows where there are few wavefronts.  Within 10 % of the
-        // best of 1 to 56 rows on sixteen layers from 8 to 300 MB.
         const long long per_strip = (long long)n * xs * quads;
-        const double capacity = 64.0 * 4 * 4 * std::max(1, cu_count);
-        int strips = 1;
-        double best = 0;
-        for (int s = 1; s <= g.out_h; s++) {
-            const int rows = (g.out_h + s - 1) / s;
-            if ((g.out_h + rows - 1) / rows != s)
-                continue;
-            const double cost = std::ceil(per_strip * s / capacity) * (rows + 2.5);
-            if (s == 1 || cost < best) {
-                best = cost;
-                strips = s;
-            }
-        }
+        const int strips = strip_count(per_strip, g.out_h, cu_count);
         a.rows = (g.out_h + strips - 1) / strips;
         a.fd_ys = make_fastdiv((unsigned)strips);
         a.in = in + n0 * in_image;

@@ -115,3 +115,37 @@ def test_wide_filter_walks_ask_for_lds_that_the_kernel_may_have():
         assert log[0]["lds"] == 3 * 4 * 256 * steps
         assert 34848 + log[0]["lds"] <= 65536 or log[0]["limit"] >= log[0]["lds"], log
     """)
+
+
+def test_depthwise_strips_are_found_quickly():
+    """The strip count of the depthwise row walks is the cheapest of all (the plain search below), and finding it does not
+    take longer than the launch: a layer of a million rows."""
+    host_hip.run('''
+    import math, time
+
+    def launch(n, h, w, c, stride=1):
+        desc = m.capi.make_desc((n, h, w, c), c, (3, 3), (stride, stride), pads=(1, 1, 1, 1), group=c)
+        hip.host_hip_clear()
+        t = time.perf_counter()
+        rc = m.lib().espdl_hip_conv2d(ctypes.byref(desc), 1 << 20, 1 << 40, None, 1 << 41, None, 1 << 42, None)
+        t = time.perf_counter() - t
+        log = launches()
+        assert rc == 0 and len(log) == 1 and "strip" in log[0]["name"], (rc, log)
+        return log[0]["grid"][0], t
+
+    for n, h, w, c, stride in [(1, 1, 1, 4, 1), (1, 7, 7, 960, 1), (37, 14, 14, 384, 1), (256, 56, 56, 144, 1), (256, 112, 112, 96, 2),
+                               (3, 97, 55, 61, 2), (512, 20, 80, 24, 1), (1, 4096, 1, 20, 1), (2, 3001, 7, 5, 1), (1, 1009, 3, 4, 2)]:
+        out_h, out_w = (h - 1) // stride + 1, (w - 1) // stride + 1
+        per_strip, best = n * ((out_w + 3) // 4) * ((c + 3) // 4), None
+        for s in range(1, out_h + 1):
+            rows = -(-out_h // s)
+            cost = math.ceil(per_strip * s / (64 * 4 * 4 * 256)) * (rows + 2.5)
+            if -(-out_h // rows) == s and (best is None or cost < best[0]):
+                best = cost, s
+        blocks = -(-per_strip * best[1] // 256)
+        if n * h * w * c >= 64 << 20:
+            blocks = 8 * -(-blocks // 8)
+        assert launch(n, h, w, c, stride)[0] == blocks, (n, h, w, c, stride)
+    fastest = min(launch(1, 1 << 20, 1, 4)[1] for _ in range(5))
+    assert fastest < 1e-3, fastest
+    ''')
