@@ -187,6 +187,18 @@ def _stream(stream):
     return _current_raw_stream()
 
 
+_bits_of = None
+
+
+def _bits(x):
+    """S8 or S16 of an int8 or int16 tensor, None for any other."""
+    global _bits_of
+    if _bits_of is None:
+        import torch
+        _bits_of = {torch.int8: S8, torch.int16: S16}
+    return _bits_of.get(x.dtype)
+
+
 def _p(t):
     return None if t is None else t.data_ptr()
 
@@ -221,9 +233,11 @@ def conv2d(x, filt, bias, shift, k, stride=(1, 1), dilation=(1, 1), pads=(0, 0, 
     bias int32|int64 [OC] or None; shift int32 tensor with 1 or OC entries (device).  x, out and residual may be
     channel slices of wider NHWC tensors (wide[..., a:b]): they are read / written in place through the
     descriptor's pitches."""
+    bits = _bits(x)
+    if bits is None:
+        raise EspdlHipError(f"conv2d takes int8 or int16 tensors, not {x.dtype}")
     desc, out_shape = _conv_plan(x.shape, filt.numel(), tuple(k), tuple(stride), tuple(dilation), tuple(pads), bool(depthwise),
-                                 activation, round_mode, shift.numel(), S8 if x.element_size() == 1 else S16,
-                                 _channel_pitch(x), _channel_pitch(out), _channel_pitch(residual))
+                                 activation, round_mode, shift.numel(), bits, _channel_pitch(x), _channel_pitch(out), _channel_pitch(residual))
     if out is None:
         import torch
         out = torch.empty(out_shape, dtype=x.dtype, device=x.device)
@@ -518,7 +532,7 @@ def max_pool(x, kernel, strides=(1, 1), pads=(0, 0, 0, 0), out=None, stream=None
         oh = (h + pt + pb - kernel[0]) // strides[0] + 1
         ow = (w + pl + pr - kernel[1]) // strides[1] + 1
         out = torch.empty((n, max(oh, 0), max(ow, 0), c), dtype=x.dtype, device=x.device)
-    _check(lib().espdl_hip_max_pool_pitched(_p(x), S16 if x.element_size() == 2 else S8, n, h, w, c, kernel[0], kernel[1],
+    _check(lib().espdl_hip_max_pool_pitched(_p(x), _bits(x) or S8, n, h, w, c, kernel[0], kernel[1],
                                             strides[0], strides[1], pt, pb, pl, pr, _channel_pitch(x), _channel_pitch(out),
                                             _p(out), _stream(stream)))
     return out

@@ -52,3 +52,15 @@ def test_requantized_residual_is_refused_for_misaligned_operands():
     rc = m.lib().espdl_hip_mbconv_s8(C.byref(d), C.c_void_p(base + 4), C.byref(w), C.c_void_p(base * 9), C.c_void_p(base * 10), None)
     assert rc == -95, m.lib().espdl_hip_last_error()
     assert b"residual_shift" in m.lib().espdl_hip_last_error()
+
+
+def test_conv2d_refuses_other_types_than_int8_and_int16():
+    """The library would read the bytes of any other tensor as one of the two (no GPU needed: nothing is launched)."""
+    import importlib
+    import pytest
+    import torch
+    m = importlib.import_module("esp-dl_amd")
+    f, shift = torch.zeros(16 * 16, dtype=torch.int8), torch.zeros(1, dtype=torch.int32)
+    for dtype in (torch.uint8, torch.bool, torch.float16, torch.bfloat16, torch.int32, torch.float32):
+        with pytest.raises(m.EspdlHipError, match="int8 or int16"):
+            m.conv2d(torch.zeros((1, 4, 4, 16), dtype=dtype), f, None, shift, (1, 1), stream=0)
