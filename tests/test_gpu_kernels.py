@@ -1557,3 +1557,24 @@ def test_mbconv_s8_mixed_epilogues(oracle, general_stage, ce):
     dev = lambda t: tuple(to_dev(a) for a in t)  # noqa: E731
     got = m.mbconv_s8(to_dev(x), dev(ex), dev(dw), dev(pj), (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), (True, True, False))
     np.testing.assert_array_equal(to_host(got), want)
+
+
+@pytest.mark.parametrize("private", [True, False], ids=["raw_handle", "stream_object"])
+def test_calls_go_to_the_current_stream(monkeypatch, private):
+    """The stream a call is enqueued on is torch's current one, asked for through torch's own raw-handle functions where this
+    torch has them and through torch.cuda.current_stream() where it does not."""
+    import torch
+    capi = espdl().capi
+    announce(f"current stream private={private}")
+    if not private:
+        monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
+    monkeypatch.setattr(capi, "_current_raw_stream", None)
+    side = torch.cuda.Stream()
+    assert capi._stream(None) == torch.cuda.current_stream().cuda_stream
+    with torch.cuda.stream(side):
+        assert capi._stream(None) == side.cuda_stream != 0
+        x = torch.arange(-64, 64, dtype=torch.int8, device="cuda")
+        y = capi.relu_s8(x)
+    side.synchronize()
+    assert capi._stream(None) == torch.cuda.current_stream().cuda_stream and capi._stream(7) == 7
+    assert torch.equal(y, x.clamp(min=0))
