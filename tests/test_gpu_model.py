@@ -481,6 +481,69 @@ def test_attention_block_is_one_module(oracle):
     assert counts == [18, 5]
 
 
+# Tensors of the attention block's chain that somebody else wants: all of it then stays as separate modules.  The feature map
+# and v's own map are results of the one module and may be wanted.  (tensor, modules with it as an output, and with a Relu
+# that reads it)
+ATTENTION_TENSORS = [("qkv_nchw_out", 18, 19), ("qkv_heads_out", 18, 19), ("qkv_split_out0", 18, 19), ("qkv_split_out1", 18, 19),
+                     ("qkv_split_out2", 18, 19), ("q_t_out", 18, 19), ("qk_out", 18, 19), ("attn_scaled_out", 18, 19),
+                     ("attn_q_out", 18, 19), ("attn_t_out", 18, 19), ("av_out", 18, 19), ("o_map_out", 18, 19),
+                     ("v_map_out", 18, 19), ("qkv_out", 5, 6), ("o_nhwc_out", 5, 6), ("v_nhwc_out", 5, 6)]
+
+
+@pytest.mark.parametrize("use", ["output", "reader"])
+@pytest.mark.parametrize("tensor,as_output,with_reader", ATTENTION_TENSORS, ids=lambda v: v if isinstance(v, str) else "")
+def test_attention_block_with_a_wanted_tensor(oracle, tensor, as_output, with_reader, use):
+    announce(f"model attention_block {tensor} has another {use}")
+    _, zoo, _, _ = _mods()
+    spec = zoo.attention_block(hw=7, heads=2)
+    if use == "output":
+        spec.outputs.append(tensor)
+    else:
+        b = zoo.Builder(spec, 1)
+        b.output(b.relu(tensor, name="also"))
+    mdl, want, _ = _run_config(spec, 2, 37)
+    for name in spec.outputs:
+        np.testing.assert_array_equal(mdl.get_tensor(name).reshape(want[name].shape), want[name], err_msg=name)
+        assert want[name].min() < want[name].max()
+    assert mdl.module_count() == (as_output if use == "output" else with_reader)
+    mdl.close()
+
+
+# RequantizeLinear to int16 in front of an int16 Conv with a table behind it.  The Conv takes over the first where the int16
+# tensor is eight exponents finer than its int8 source and has no other reader, and the second where its table has at most
+# 4097 entries and nobody else reads the Conv's own result.  (exponents finer, table points, second reader, modules)
+S16_FOLDS = [(8, 2048, "", 2), (8, 4096, "", 2), (8, 8192, "", 3), (7, 2048, "", 4), (9, 2048, "", 4), (8, 2048, "requantized", 5),
+             (8, 2048, "requantized_output", 4), (8, 2048, "conv", 4), (8, 2048, "conv_output", 3)]
+
+
+@pytest.mark.parametrize("round_mode", [0, 1], ids=["half_up", "half_even"])
+@pytest.mark.parametrize("finer,points,other,modules", S16_FOLDS)
+def test_int16_conv_behind_requantize(oracle, finer, points, other, modules, round_mode):
+    announce(f"model int16 conv behind requantize finer={finer} points={points} other={other} round_mode={round_mode}")
+    _, zoo, _, _ = _mods()
+    g = zoo.GraphSpec("int16_conv_behind_requantize")
+    b = zoo.Builder(g, 0xE5F9, per_channel=True, w_exp_range=None)
+    x = b.input("input", [1, 9, 11, 16], -5)
+    h = b.conv(x, 24, k=3, name="c1")
+    h16 = "to_s16_out"
+    g.add_value(h16, g.shape(h), g.exponent(h) - finer, zoo.INT16)
+    g.add_node("to_s16", "RequantizeLinear", [h], [h16], quant_type="S16")
+    c2 = b.conv(h16, 40, k=3, s16=True, name="c2")
+    b.output(b.lut_s16(c2, zoo.silu, points=points, name="act"))
+    if other == "requantized":
+        b.output(b.lut_s16(h16, zoo.silu, points=64, name="also"))
+    elif other == "conv":
+        b.output(b.lut_s16(c2, zoo.silu, points=64, name="also"))
+    elif other:
+        b.output({"requantized_output": h16, "conv_output": c2}[other])
+    mdl, want, _ = _run_config(g, 3, 51, round_mode=round_mode)
+    for name in g.outputs:
+        np.testing.assert_array_equal(mdl.get_tensor(name, np.int16), want[name], err_msg=name)
+        assert want[name].min() < want[name].max()
+    assert mdl.module_count() == modules
+    mdl.close()
+
+
 @pytest.mark.parametrize("round_mode", [0, 1], ids=["half_up", "half_even"])
 def test_int16_tail(oracle, round_mode):
     """int16 table, Add, Mul by a constant, AveragePool and ReduceMean behind an int8 -> int16 requantize."""
