@@ -96,7 +96,7 @@ ZOO = [
     "models/human_face_detect/models/s3/human_face_detect_msr_s8_v1.espdl",
     "models/hand_gesture_recognition/models/p4/mobilenetv2_0_5_128_128_gesture.espdl",
 ]
-needs_reference = pytest.mark.skipif(not os.path.isdir(REF), reason="the reference tree is not on this machine")
+needs_reference = pytest.mark.skipif(not os.path.isdir(os.path.join(REF, "models")), reason="the reference tree is not on this machine")
 
 
 @needs_reference
