@@ -91,16 +91,18 @@ struct DwExpand {
     int n_shift, relu, c0;
 };
 
-// Depthwise with the input tile staged in LDS (contiguous global reads and writes) and the products
-// on the matrix pipe; same shape limits as the direct form.
-// conv2d_s8_wide.hip
+// Pointwise layers of at most 128 channels under thousands of filters, rows of the result no multiple of 16 bytes long
+// (conv2d_s8_wide.hip)
 bool conv2d_s8_wide_supports(const ConvGeom &g, const int8_t *lut, const int8_t *residual);
 hipError_t launch_conv2d_s8_wide(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,
                                  const int32_t *shift, int8_t *out, int cu_count, hipStream_t stream);
-// depthwise_s8_strip.hip
+// Depthwise 3 x 3 layers at dilation 1 as row walks on byte dot products, any channel count from 4 on
+// (depthwise_s8_strip.hip)
 bool depthwise_s8_strip_supports(const ConvGeom &g);
 hipError_t launch_depthwise_s8_strip(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,
                                      const int32_t *shift, const int8_t *lut, int8_t *out, int cu_count, hipStream_t stream);
+// Depthwise with the input tile staged in LDS (contiguous global reads and writes) and the products
+// on the matrix pipe; same shape limits as the direct form.
 bool depthwise_s8_lds_supports(const ConvGeom &g, const void *in, const void *out);
 hipError_t launch_depthwise_s8_lds(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,
                                    const int32_t *shift, const int8_t *lut, int8_t *out, int cu_count,
@@ -247,7 +249,7 @@ hipError_t launch_resize_nearest_s8(const int8_t *in, int batch, int h, int w, i
 hipError_t launch_max_pool(const void *in, int elem_size, int batch, int h, int w, int c, int k_h, int k_w, int stride_h,
                            int stride_w, int pad_top, int pad_left, int out_h, int out_w, long long in_pitch,
                            long long out_pitch, void *out, int cu_count, hipStream_t stream);
-// int8, square windows of 2 / 3 / 5 at stride 1, channels and pitches in multiples of 16 (max_pool_s8.hip)
+// int8, square windows of 2 / 3 / 5 at stride 1, any channel count from 8 on and any pitch (max_pool_s8.hip)
 bool max_pool_s8_window_supports(int h, int w, int c, int k_h, int k_w, int stride_h, int stride_w, int pad_top,
                                  int pad_left, int out_h, int out_w);
 hipError_t launch_max_pool_s8_window(const void *in, int batch, int h, int w, int c, int k, int pad_top, int pad_left,

@@ -88,7 +88,8 @@ __global__ __launch_bounds__(kBlock) void copy_rows_kernel(const RowCopyArgs a)
     }
 }
 
-inline int widest_access(const void *a, const void *b, long long p0, long long p1, long long n)
+// Accesses of rows too short for 16-byte pieces: dwords where both sides and the length allow, else bytes.
+inline int short_row_access(const void *a, const void *b, long long p0, long long p1, long long n)
 {
     const uintptr_t m = reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | (uintptr_t)p0 | (uintptr_t)p1 |
         (uintptr_t)n;
@@ -104,7 +105,7 @@ inline bool fill_seg(RowSeg &s, const void *src, long long src_pitch, void *dst,
     s.row_bytes = row_bytes;
     // 16 bytes at any address; the last access of a row that is no multiple of 16 long reaches back over bytes its
     // neighbour copies too
-    s.vec = row_bytes >= 16 ? 16 : widest_access(src, dst, src_pitch, dst_pitch, row_bytes);
+    s.vec = row_bytes >= 16 ? 16 : short_row_access(src, dst, src_pitch, dst_pitch, row_bytes);
     const long long per_row = (row_bytes + s.vec - 1) / s.vec;
     if (per_row > 0x7fffffffll)
         return false;
