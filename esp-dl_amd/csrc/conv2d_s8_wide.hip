@@ -9,8 +9,9 @@
 // 1.9 TB/s; so a step's bytes pass through LDS and leave as whole aligned 16-byte pieces of memory, cut out of the bytes
 // of this step and the last 16 of the step before, and only the two ends of a row's walk are written by the byte.
 //
-// 20480 pixels x 120 -> 6625 (136 MB written, 26 us at the copy rate): 50 us, where the kernel that keeps filters in LDS
-// took 75 us.  A third of that is the start of a walk (its pixels and constants), of which every compute unit does four.
+// 20480 pixels x 120 -> 6625 (136 MB written, 26 us at the copy rate): 51 us inside the recognizer, where the kernel that
+// keeps filters in LDS took 71 us; 50 against 69 us on one pair of tensors, 61 against 76 us on changing ones.  A third of
+// that is the start of a walk (its pixels and constants), of which every compute unit does four.
 //
 // Restates conv2d_11cn (esp-dl/dl/base/dl_base_conv2d.cpp:9-33) with the n_wise epilogue
 // (esp-dl/dl/base/dl_base_activate_buffer.hpp:27-36, 61-72, 173-181, 201-210).

@@ -10,10 +10,12 @@
 // neighbour has too; both write the same bytes.  Pixels outside the image are loads behind the descriptor's end (zeros),
 // outputs that do not exist stores behind it (dropped), so the walk has no branches.
 //
-// Bound by HBM on large layers: 256 images of 56 x 56 x 144 in 48 us (4.8 TB/s), where tiles staged through LDS for the
-// matrix cores took 60 us; by the launch on small ones: 56 x 56 x 144 in 4.5 us (10.3 us), most of which the staged form
-// spent on setting up its tile.  61 channels, which that form does not take: 27 us instead of 401 us.  Strips of few rows
-// and rounds of wavefronts lie between (14 x 14 x 384, 256 images: 13 us, 18 us before, 7 us at the copy rate).
+// Bound by memory on large layers: 256 images of 56 x 56 x 144 (231 MB in and out) take 59 us when the tensors come from HBM
+// (3.9 TB/s), as they do inside a program (61 us in a chain of operators), and 44 us when one pair of tensors, which the
+// last-level cache holds in part, is used again and again; tiles staged through LDS for the matrix cores took 60 (66 in
+// that chain) and 54 us.  So the gain is in what the staged form spends on its tiles: 256 images of 14 x 14 x 384 14.5 us (19 us
+// before, 7 us at the copy rate; strips of few rows and rounds of wavefronts lie between), one image of 56 x 56 x 144 4.8 us
+// (15 us), and 61 channels, which that form does not take, over 256 images of 28 x 28: 16 us (107 us).
 //
 // Restates depthwise_conv2d_33c1 (esp-dl/dl/base/dl_base_depthwise_conv2d.cpp:9-65) under dwconv_operation_shell's window
 // clipping (esp-dl/dl/base/dl_base.hpp:1852-2102); filter memory is [3][3][c].

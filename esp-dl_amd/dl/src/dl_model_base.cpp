@@ -38,13 +38,14 @@ dtype_t dtype_of(quant_type_t q)
 }
 
 // Which captured plans are replayed as plain kernel launches instead of as a HIP graph.  A graph replay costs the
-// stream about 8 us in which no kernel runs and the host 15 to 20 us, whatever the number of nodes (one 3x3
-// convolution at batch 1: 14.9 us per graph replay, 6.1 us per launch).  A plain launch costs the host 3 to 4 us and,
-// with its own release of the caches, the stream a few tenths of a microsecond more than a graph node does.  So a plan
-// of up to kDirectAlways launches is always replayed plainly, and one of up to kDirectLaunches when its modules
-// move kDirectBytes or more on average: such kernels take long enough for the host to stay ahead of the stream
-// (MobileNetV2 at batch 256, 19 launches of 33 us: 651 against 646 us; the attention block over 7 x 7 maps, 15 launches
-// of 3.6 us: 62 us as a graph, 63 us launched one by one; MobileNetV2 on one image: 348 against 354 us).
+// stream 4 to 5 us in which no kernel runs and the host 15 to 20 us, whatever the number of nodes (one 3x3
+// convolution at batch 1: 17.4 us per graph replay, 4.2 us per launch; the same layer at batch 256: 45.2 and 41.5 us).  A plain
+// launch costs the host 3 to 4 us and, with its own release of the caches, the stream a few tenths of a microsecond more
+// than a graph node does.  So a plan of up to kDirectAlways launches is always replayed plainly, and one of up to
+// kDirectLaunches when its modules move kDirectBytes or more on average: such kernels take long enough for the host to stay
+// ahead of the stream (MobileNetV2 at batch 256, 19 launches of 33 us: 649 against 644 us; the recognizer at 512 crops, 15
+// launches: 231 against 227 us; 15 launches of 3.6 us: 62 us as a graph, 63 us launched one by one; MobileNetV2 on one
+// image: 348 against 354 us).
 constexpr size_t kDirectAlways = 4;
 constexpr size_t kDirectLaunches = 24;
 constexpr size_t kDirectBytes = 1 << 20;
