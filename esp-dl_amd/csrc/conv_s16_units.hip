@@ -24,12 +24,12 @@
 // and its high bytes the int8 values themselves:  sum_k x w = 65536 sum x8 wh + 256 sum x8 l + 32768 sum x8 (l as above).
 // Two products per step instead of four, no cutting of pixels, half the input, no RequantizeLinear and no int16 copy.
 // They also take an int16 table behind the result (the nearest-entry LUT of esp-dl/dl/base/dl_base_lut.cpp:49-77).
-// 80 x 80 x 64 -> 64, 3 x 3, batch 64: 78 us where the three operators took 135 us.
+// 80 x 80 x 64 -> 64, 3 x 3, batch 64: 75 us where the three operators took 135 us.
 //
 // Two kernels, chosen by their measured cost (see the launch).  Against the one-wavefront-per-pixel-tile kernel
-// (conv_s16_mfma.hip) and the 64-bit multiply-add kernel (conv_s16.hip): 80 x 80 x 64 -> 64, 3 x 3, batch 64 98 -> 92 us,
-// batch 8 22 -> 17 us, one image 13.4 -> 8.4 us; 40 x 40 x 128 -> 128, batch 64 147 -> 89 us; 22 x 12 x 122 -> 252, 3 x 3,
-// batch 57 2764 -> 24 us.
+// (conv_s16_mfma.hip) and the 64-bit multiply-add kernel (conv_s16.hip): 80 x 80 x 64 -> 64, 3 x 3, batch 64 98 -> 90 us,
+// batch 8 22 -> 16 us, one image 13.4 -> 8.3 us; 40 x 40 x 128 -> 128, batch 64 147 -> 85 us; 22 x 12 x 122 -> 252, 3 x 3,
+// batch 57 2764 -> 31 us.
 //   * the tiled one: 64 PT pixels x 64 filters per workgroup, both operands global -> registers (two steps ahead) ->
 //     cut into bytes -> LDS (two buffers), so that a value is cut once per workgroup;
 //   * the narrow one for few outputs: 16 pixels x 16 NT filters per workgroup, its four wavefronts split the reduction

@@ -149,7 +149,7 @@ enum DenseRoute { DENSE_STEM, DENSE_NARROW, DENSE_UNITGEMM, DENSE_PWGEMM, DENSE_
 //   * strided windows of fewer than five reduction steps with many outputs: the direct kernel (320 x 320 x 16 -> 32 at
 //     stride 2, batch 32: 35.5 against 38.3 us).
 // A channel count that is not a multiple of 16 under a window has no other kernel worth taking: 31 x 101 x 61 -> 16,
-// 5 x 5, batch 142: 509 -> 111 us; 45 x 99 x 162 -> 87, 5 x 5 at stride 2, batch 3: 312 -> 33 us.
+// 5 x 5, batch 142: 509 -> 105 us; 45 x 99 x 162 -> 87, 5 x 5 at stride 2, batch 3: 312 -> 40 us.
 DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *filter, const void *residual, int cus)
 {
     const bool units = images_per_launch(g, espdl::conv2d_s8_units_support) > 0;
