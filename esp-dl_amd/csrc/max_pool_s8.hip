@@ -247,10 +247,8 @@ hipError_t launch_max_pool_s8_window(const void *in, int batch, int h, int w, in
     const double capacity = (double)(cu_count > 0 ? cu_count : 256) * 4 * 4;
     int best_strips = 1;
     double best_score = -1.0;
-    for (int strips = 1; strips <= out_h; strips++) {
+    for (int strips = 1;;) { // of the counts with one strip height only the smallest: 2 sqrt(out_h) of them
         const int rows = (out_h + strips - 1) / strips;
-        if ((out_h + rows - 1) / rows != strips)
-            continue; // the same strip height as a smaller count
         const double waves = (double)per_row * strips / 64.0;
         const double rounds = waves / capacity;
         const double fill = rounds / (double)(long long)(rounds + 0.999999);
@@ -259,6 +257,9 @@ hipError_t launch_max_pool_s8_window(const void *in, int batch, int h, int w, in
             best_score = score;
             best_strips = strips;
         }
+        if (rows <= 1)
+            break;
+        strips = (out_h + rows - 2) / (rows - 1);
     }
     a.strips = best_strips;
     a.rows = (out_h + best_strips - 1) / best_strips;

@@ -149,3 +149,35 @@ def test_depthwise_strips_are_found_quickly():
     fastest = min(launch(1, 1 << 20, 1, 4)[1] for _ in range(5))
     assert fastest < 1e-3, fastest
     ''')
+
+
+def test_pool_strips_are_found_quickly():
+    """The same for the strips of the stride-1 max pool."""
+    host_hip.run('''
+    import math, time
+
+    def launch(n, h, w, c, k):
+        hip.host_hip_clear()
+        t = time.perf_counter()
+        rc = m.lib().espdl_hip_max_pool_pitched(1 << 20, 8, n, h, w, c, k, k, 1, 1, k // 2, (k - 1) // 2, k // 2, (k - 1) // 2, 0, 0, 1 << 42, None)
+        t = time.perf_counter() - t
+        log = launches()
+        assert rc == 0 and len(log) == 1 and "max_pool_s8_window" in log[0]["name"], (rc, log)
+        return log[0]["grid"][0] * log[0]["block"][0], t
+
+    for n, h, w, c, k in [(1, 1, 1, 8, 3), (64, 20, 20, 128, 5), (327, 80, 80, 128, 5), (256, 56, 56, 144, 5), (128, 36, 8, 194, 5),
+                          (2, 3001, 7, 24, 3), (1, 4096, 1, 16, 2), (5, 97, 31, 9, 2)]:
+        vec = 16 if c >= 16 and c != 24 else 8
+        per_row, best, score = n * ((w + 1) // 2) * -(-c // vec), 1, -1.0
+        for s in range(1, h + 1):
+            rows = -(-h // s)
+            if -(-h // rows) != s:
+                continue
+            rounds = per_row * s / 64.0 / (256 * 4 * 4)
+            here = rounds / int(rounds + 0.999999) / (1.0 + 0.5 * (k - 1) / rows)
+            if here > score * 1.02:
+                score, best = here, s
+        assert launch(n, h, w, c, k)[0] == -(-per_row * best // 256) * 256, (n, h, w, c, k)
+    fastest = min(launch(1, 1 << 20, 1, 64, 5)[1] for _ in range(5))
+    assert fastest < 1e-3, fastest
+    ''')
