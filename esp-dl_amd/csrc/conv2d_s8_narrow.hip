@@ -205,6 +205,9 @@ static NarrowPlan narrow_plan(const ConvGeom &g, int cu_count)
 float conv2d_s8_narrow_us(const ConvGeom &g, const void *in, const void *filter, int cu_count)
 {
     const NarrowPlan p = narrow_plan(g, cu_count);
+    const long long tiles = ((long long)g.batch * g.out_h * g.out_w + 15) / 16;
+    if ((p.split ? tiles : (tiles + 3) / 4) * kThreads >= 1ll << 32) // more threads than a launch may have
+        return 1e30f;
     const float steps = (float)(p.split ? (p.ksteps + 3) / 4 : p.ksteps);
     const float waves = 4e-3f * (float)p.groups;
     if (window_aligned(g, in, filter))

@@ -181,3 +181,20 @@ def test_pool_strips_are_found_quickly():
     fastest = min(launch(1, 1 << 20, 1, 64, 5)[1] for _ in range(5))
     assert fastest < 1e-3, fastest
     ''')
+
+
+def test_narrow_kernels_stay_inside_the_grid_limit():
+    """A launch has fewer than 2^32 threads along x: layers with more pixels than that go to the kernel with larger tiles."""
+    host_hip.run('''
+    for dtype in (8, 16):
+        for n, h, w, c, oc, k in [(1500, 1000, 1000, 1, 8, (5, 1)), (700, 1000, 1000, 1, 8, (5, 1)), (1, 9, 9, 1, 8, (5, 1))]:
+            if dtype == 16 and n > 700:
+                continue
+            desc = m.capi.make_desc((n, h, w, c), oc, k, pads=(2, 2, 0, 0), dtype=dtype)
+            hip.host_hip_clear()
+            rc = m.lib().espdl_hip_conv2d(ctypes.byref(desc), 1 << 36, 1 << 37, None, 1 << 38, None, 1 << 39, None)
+            log = launches()
+            assert rc == 0 and log, (rc, n)
+            for l in log:
+                assert l["grid"][0] * l["block"][0] < 1 << 32, (dtype, n, l)
+    ''')
