@@ -2,6 +2,7 @@
 // validation, geometry derivation and kernel dispatch.  No allocation, no synchronization.
 #include "../../include/espdl_hip.h"
 
+#include <algorithm>
 #include <climits>
 #include <cstdarg>
 #include <cstdio>
@@ -133,11 +134,14 @@ int images_per_launch(const espdl::ConvGeom &g, bool (*supports)(const espdl::Co
     return supports(part) ? part.batch : 0;
 }
 
-enum DenseRoute { DENSE_STEM, DENSE_NARROW, DENSE_UNITGEMM, DENSE_PWGEMM, DENSE_TILED, DENSE_DIRECT };
+enum DenseRoute { DENSE_WALK, DENSE_STEM, DENSE_NARROW, DENSE_UNITGEMM, DENSE_PWGEMM, DENSE_TILED, DENSE_DIRECT };
 
 // Kernel of a dense int8 convolution.  The two kernels that read windows as 16-channel units take any layer; their
 // times, measured over 128 layers of 1 to 600 K output pixels, are straight lines in their work (within 15 %), so the
-// choice between them compares those lines.  Where the other kernels begin:
+// choice between them compares those lines.  The walking kernel takes what it has a build for where its expected time is
+// the smaller one: over 780 random layers of 16 to 256 channels (1 image to 260 MB) the kernels below take 1.14 times
+// as long in the geometric mean, twice and more from a hundred thousand pixels on; below some 4 us the narrow kernel is the
+// faster one (16 x 16 x 20 x 20, 3 x 3: 3.1 against 3.7 us).  Where the other kernels begin:
 //   * window rows of at most 16 bytes (RGB input): the first-layer kernel, which never takes less than 5.2 us;
 //   * 1x1 over flat rows: the pointwise GEMM kernel where it applies (two reads less address arithmetic), the direct
 //     kernel where pixels are many and channels few (its wavefronts keep their pixels in registers and write whole
@@ -150,7 +154,8 @@ enum DenseRoute { DENSE_STEM, DENSE_NARROW, DENSE_UNITGEMM, DENSE_PWGEMM, DENSE_
 //     stride 2, batch 32: 35.5 against 38.3 us).
 // A channel count that is not a multiple of 16 under a window has no other kernel worth taking: 31 x 101 x 61 -> 16,
 // 5 x 5, batch 142: 509 -> 105 us; 45 x 99 x 162 -> 87, 5 x 5 at stride 2, batch 3: 312 -> 40 us.
-DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *filter, const void *residual, int cus)
+DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *filter, const void *residual, const void *out,
+                          int cus)
 {
     const bool units = images_per_launch(g, espdl::conv2d_s8_units_support) > 0;
     float narrow = 0.f, gemm = 0.f;
@@ -158,6 +163,10 @@ DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *
     if (units) {
         narrow = espdl::conv2d_s8_narrow_us(g, in, filter, cus);
         gemm = espdl::conv2d_s8_unitgemm_us(g, in, filter, &tile_steps);
+        // (the larger routes below take up to twice the unit kernel's line; a quarter more puts no layer on the walk that
+        // is slower there by more than a fifth, and gives up 2 % of what the best choice of 780 random layers would)
+        if (espdl::conv2d_s8_walk_us(g, in, filter, residual, out, cus) < std::min(narrow, 1.25f * gemm))
+            return DENSE_WALK;
     }
     if (espdl::conv2d_s8_stem_supports(g, residual))
         return units && narrow < 5.2f ? DENSE_NARROW : DENSE_STEM;
@@ -274,7 +283,9 @@ int espdl_hip_conv2d_add(const espdl_hip_conv_desc *desc, const void *in, const 
         };
         if (espdl::conv2d_s8_wide_supports(g, lut, residual))
             return device_status(espdl::launch_conv2d_s8_wide(g, i8, f8, b32, shift, o8, cus, s), "conv2d_s8_wide");
-        switch (dense_s8_route(g, in, filter, residual, cus)) {
+        switch (dense_s8_route(g, in, filter, residual, out, cus)) {
+        case DENSE_WALK:
+            return run(espdl::launch_conv2d_s8_walk, "conv2d_s8_walk");
         case DENSE_STEM:
             return device_status(espdl::launch_conv2d_s8_stem(g, i8, f8, b32, shift, lut, o8, cus, s), "conv2d_s8_stem");
         case DENSE_NARROW:

@@ -51,6 +51,13 @@ float conv2d_s8_narrow_us(const ConvGeom &g, const void *in, const void *filter,
 hipError_t launch_conv2d_s8_narrow(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,
                                    const int32_t *shift, const int8_t *lut, const int8_t *residual, int8_t *out,
                                    int cu_count, hipStream_t stream);
+// Dense int8 convolution as a walk down the image, filters in registers (conv2d_s8_walk_kernel.h): square 1, 3 and 5 filters
+// at stride 1 and 2, channel counts that are multiples of 16, round half up.  Expected time; 1e30: no build takes it.
+float conv2d_s8_walk_us(const ConvGeom &g, const void *in, const void *filter, const void *residual, const void *out,
+                        int cu_count);
+hipError_t launch_conv2d_s8_walk(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,
+                                 const int32_t *shift, const int8_t *lut, const int8_t *residual, int8_t *out,
+                                 int cu_count, hipStream_t stream);
 // Dense int8 convolution with a window, input tile and filters staged in LDS (conv2d_s8_tiled.hip): channel
 // count a multiple of 16, 16-byte aligned input and filter.
 bool conv2d_s8_tiled_supports(const ConvGeom &g, const void *in, const void *filter, int cu_count);

@@ -190,3 +190,31 @@ def every_sum_image(h, w):
         x[0, :r, i] += 1
     assert x.min() >= -128 and x.max() <= 127
     return x.reshape(1, h, w, c).astype(np.int8)
+
+# Layers for the kernel that walks down the image with its filters in registers, batch first (the batch puts them where the
+# dispatcher takes it).  1 x 1 over pixel counts that end inside a workgroup's tile, one and several chunks of 16 to 128
+# filters, chunks that end early, every second pixel of odd extents; windows over images narrower than a tile, widths one
+# below and above a tile, many images in one tile, one-sided and missing padding, odd extents at stride 2, walks that start
+# and end inside an image, 16 to 256 input channels.
+WALK_CASES = [
+    (2, ("w1_16_16", (97, 131, 16), 16, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, True)),
+    (5, ("w1_64_176", (61, 67, 64), 176, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, True)),
+    (7, ("w1_112_48", (45, 83, 112), 48, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), False, True)),
+    (9, ("w1_256_256", (33, 31, 256), 256, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, False)),
+    (16, ("w1s2_96_64", (45, 83, 96), 64, (1, 1), (2, 2), (1, 1), (0, 0, 0, 0), True, True)),
+    (40, ("w3_16_16", (37, 53, 16), 16, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
+    (19, ("w3_32_32", (40, 81, 32), 32, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, False)),
+    (30, ("w3_48_48", (31, 33, 48), 48, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
+    (64, ("w3_64_64", (20, 20, 64), 64, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
+    (230, ("w3_64_32_narrow", (17, 7, 64), 32, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
+    (23, ("w3_128_64_nopad", (29, 18, 128), 64, (3, 3), (1, 1), (1, 1), (0, 0, 0, 0), False, True)),
+    (26, ("w3_64_80_tailpad", (25, 15, 64), 80, (3, 3), (1, 1), (1, 1), (0, 2, 0, 1), True, True)),
+    (33, ("w3_224_16", (23, 30, 224), 16, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
+    (1, ("w3_32_64_one_image", (150, 161, 32), 64, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
+    (90, ("w3s2_16_32_tailpad", (80, 112, 16), 32, (3, 3), (2, 2), (1, 1), (0, 1, 0, 1), True, True)),
+    (40, ("w3s2_64_64", (49, 51, 64), 64, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), True, True)),
+    (50, ("w3s2_128_64", (41, 30, 128), 64, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), True, False)),
+    (20, ("w5_16_16", (47, 65, 16), 16, (5, 5), (1, 1), (1, 1), (2, 2, 2, 2), True, True)),
+    (12, ("w5_64_32", (35, 40, 64), 32, (5, 5), (1, 1), (1, 1), (2, 2, 2, 2), True, True)),
+    (40, ("w5s2_64_48", (40, 43, 64), 48, (5, 5), (2, 2), (1, 1), (2, 2, 2, 2), True, True)),
+]

@@ -5,7 +5,7 @@ import ctypes
 import numpy as np
 import pytest
 
-from cases import CONFIG1, CONV_CASES, DW_CASES, GEMM_CASES, POINTWISE_MANY_PIXELS, WIDE_ROWS, WINDOW_GEMM_CASES, TILED_MANY_PIXELS, STEM_CASES, TILED_CASES, UNIT_CASES, every_sum_image, rng_int8, typical_shift
+from cases import CONFIG1, CONV_CASES, DW_CASES, GEMM_CASES, POINTWISE_MANY_PIXELS, WIDE_ROWS, WINDOW_GEMM_CASES, TILED_MANY_PIXELS, STEM_CASES, TILED_CASES, UNIT_CASES, WALK_CASES, every_sum_image, rng_int8, typical_shift
 from gpu_util import announce, espdl, to_dev, to_host
 
 pytestmark = pytest.mark.gpu
@@ -190,6 +190,49 @@ def test_conv2d_s8_channel_units(oracle, case, flavour):
     oracle.set_threads(16)
     got, want = _run_conv_s8(oracle, x, f, bias, shift, k, stride, dil, pads, relu, **kw)
     np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("case", WALK_CASES, ids=lambda c: c[1][0])
+@pytest.mark.parametrize("flavour", ["per_channel", "low_shifts", "lut_residual", "general_epilogue", "slices"])
+def test_conv2d_s8_walk(oracle, case, flavour):
+    """The kernel that walks down the image: right shifts and left shifts of the short epilogue, a table and a residual
+    operand, the general shift-and-round form, and operands that are channel slices of wider tensors (whose other
+    channels stay as they are)."""
+    import torch
+    announce(f"conv2d_s8 walk {case[1][0]} {flavour}")
+    x, f, bias, shift, k, stride, dil, pads, relu = _conv_inputs(case[1], 263, case[0], True)
+    kw = {}
+    if flavour == "low_shifts":
+        shift = (np.arange(shift.size) % 5 + 6).astype(np.int32)
+        f = (f >> 3).astype(np.int8)
+    if flavour == "lut_residual":
+        kw["lut"] = np.array([(i * 109 + 37) & 0xFF for i in range(256)], dtype=np.uint8).view(np.int8)
+        kw["residual_seed"] = 17
+        relu = False
+    if flavour == "general_epilogue":
+        shift = np.array(shift, dtype=np.int32)
+        shift[::3] = 0
+        shift[1::5] = 33
+    oracle.set_threads(16)
+    if flavour != "slices":
+        got, want = _run_conv_s8(oracle, x, f, bias, shift, k, stride, dil, pads, relu, **kw)
+        np.testing.assert_array_equal(got, want)
+        return
+    m = espdl()
+    c, oc = x.shape[3], f.shape[0]
+    want = oracle.conv2d_s8(x, f, bias, shift, k, stride, dil, pads, oracle.RELU if relu else oracle.LINEAR, oracle.ROUND_HALF_UP)
+    residual = rng_int8(np.random.default_rng(19), want.shape)
+    want = oracle.add_s8(want, residual)
+    wide_in = torch.full(x.shape[:3] + (c + 48,), 77, dtype=torch.int8, device="cuda")
+    wide_in[..., 16:16 + c] = to_dev(x)
+    wide_out = torch.full(want.shape[:3] + (oc + 32,), -9, dtype=torch.int8, device="cuda")
+    wide_res = torch.full(want.shape[:3] + (oc + 16,), 5, dtype=torch.int8, device="cuda")
+    wide_res[..., 16:] = to_dev(residual)
+    m.conv2d(wide_in[..., 16:16 + c], to_dev(f), to_dev(bias), to_dev(shift), k, stride, dil, pads,
+             activation=m.capi.RELU if relu else m.capi.LINEAR, residual=wide_res[..., 16:], out=wide_out[..., 16:16 + oc])
+    got = to_host(wide_out)
+    np.testing.assert_array_equal(got[..., 16:16 + oc], want)
+    assert (got[..., :16] == -9).all() and (got[..., 16 + oc:] == -9).all()
 
 
 @pytest.mark.parametrize("case", WINDOW_GEMM_CASES, ids=lambda c: c[0])
