@@ -1081,6 +1081,35 @@ static bool wave_before_group(const espdl::MbconvParams &p)
         !(espdl::mbconv_s8_group_supports(p) && espdl::mbconv_s8_group_has_fast_build(p));
 }
 
+// Expected time of the tile kernel that a block of kind 4 or 5 goes to.  The guarded builds take 0.6 to 2.4 times as long
+// as that, which their estimate leaves out.
+static float mbconv_tile_us(const espdl::MbconvParams &p, int kind, int cus)
+{
+    return kind == 5 ? espdl::mbconv_s8_group_us(p, cus) : espdl::mbconv_s8_wave_us(p);
+}
+
+// The walk down the image takes a block where its expected time is below the tile kernel's.  Up to 20 us (about one round
+// of tiles) that estimate lies a tenth high and the walk has to be below 0.9 of it.  160 random blocks of batch 1 to 256
+// gain a quarter on average, large ones without a guard-free build up to two thirds; the ones it would lose by more than
+// 2 us - single rounds, where a column strip is a longer chain than a tile - stay where they were.
+static bool mbconv_walks(const espdl::MbconvParams &p, int kind)
+{
+    const int cus = cu_count_cached();
+    const float tile = mbconv_tile_us(p, kind, cus);
+    return espdl::mbconv_s8_walk_us(p, cus) < (tile < 20.f ? 0.9f : 1.f) * tile;
+}
+
+// A block whose tile kernel is the one-wavefront-per-tile kernel (kind 4) or the workgroup-per-tile kernel (kind 5).
+static int launch_mbconv_single(const espdl::MbconvParams &p, int kind, void *stream)
+{
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    const int cus = cu_count_cached();
+    if (mbconv_walks(p, kind))
+        return device_status(espdl::launch_mbconv_s8_walk(p, cus, s), "mbconv_s8_walk");
+    return kind == 5 ? device_status(espdl::launch_mbconv_s8_group(p, cus, s), "mbconv_s8_group")
+                     : device_status(espdl::launch_mbconv_s8_wave(p, cus, s), "mbconv_s8_wave");
+}
+
 static int mbconv_kernel_choice(const espdl_hip_mbconv_desc *desc)
 {
     espdl::MbconvParams p = {};
@@ -1182,8 +1211,7 @@ int espdl_hip_mbconv_s8(const espdl_hip_mbconv_desc *desc, const int8_t *in, con
     if (espdl::mbconv_has_clip(p)) {
         if (!desc->has_expand || !espdl::mbconv_s8_wave_has_fast_build(p))
             return fail(ESPDL_HIP_ENOTSUP, "a Clip between the stages is covered for the block shapes with a guard-free build of the one-wavefront-per-tile kernel, round half up");
-        return device_status(espdl::launch_mbconv_s8_wave(p, cu_count_cached(), reinterpret_cast<hipStream_t>(stream)),
-                             "mbconv_s8_wave");
+        return launch_mbconv_single(p, 4, stream);
     }
     if (!desc->has_expand) {
         espdl::ConvGeom g;
@@ -1197,15 +1225,12 @@ int espdl_hip_mbconv_s8(const espdl_hip_mbconv_desc *desc, const int8_t *in, con
     if (desc->has_expand && !pointwise_expand(p)) {
         if (!espdl::mbconv_s8_wave_supports(p))
             return fail(ESPDL_HIP_ENOTSUP, "an expand stage with a window needs a 3x3 depthwise stage, at most 4 filter rows of at most 9 bytes (exp_k_w * in_c) and at most 64 project filters");
-        return device_status(espdl::launch_mbconv_s8_wave(p, cu_count_cached(), reinterpret_cast<hipStream_t>(stream)),
-                             "mbconv_s8_wave");
+        return launch_mbconv_single(p, 4, stream);
     }
     if (desc->has_expand && !wave_before_group(p) && espdl::mbconv_s8_group_supports(p))
-        return device_status(espdl::launch_mbconv_s8_group(p, cu_count_cached(), reinterpret_cast<hipStream_t>(stream)),
-                             "mbconv_s8_group");
+        return launch_mbconv_single(p, 5, stream);
     if (desc->has_expand && espdl::mbconv_s8_wave_supports(p))
-        return device_status(espdl::launch_mbconv_s8_wave(p, cu_count_cached(), reinterpret_cast<hipStream_t>(stream)),
-                             "mbconv_s8_wave");
+        return launch_mbconv_single(p, 4, stream);
     // Only the two kernels above requantize the residual operand.  The answer comes from the real pointers: a
     // block whose operands are merely 4-byte aligned can be refused by both although the shape alone passes.
     if (p.residual_shift != 0)
@@ -1278,7 +1303,7 @@ int64_t espdl_hip_mbconv_s8_workspace(const espdl_hip_mbconv_desc *desc)
     if (espdl_hip_mbconv_s8_supported(desc) == 0)
         other = 1e30f; // a Clip between the stages in half-even mode: no single launch
     else if (espdl_hip_mbconv_s8_preferred(desc) == 1)
-        other = espdl_hip_mbconv_s8_supported(desc) == 5 ? espdl::mbconv_s8_group_us(p, cus) : espdl::mbconv_s8_wave_us(p);
+        other = std::min(mbconv_tile_us(p, espdl_hip_mbconv_s8_supported(desc), cus), espdl::mbconv_s8_walk_us(p, cus));
     return expand_dw + project < other ? (int64_t)p.batch * p.out_h * p.out_w * p.exp_c : 0;
 }
 

@@ -163,6 +163,11 @@ inline bool mbconv_expand_is_pointwise(const MbconvParams &p)
 bool mbconv_s8_fused_supports(const MbconvParams &p);
 hipError_t launch_mbconv_s8_fused(const MbconvParams &p, int cu_count, hipStream_t stream);
 
+// The same block as a walk down the image (mbconv_s8_walk.hip): pointwise expand stage of at most 144 channels over 16 to
+// 48 block-input channels, 3x3 depthwise stage with stride 1 or 2.  Expected time; 1e30 where it does not apply.
+float mbconv_s8_walk_us(const MbconvParams &p, int cu_count);
+hipError_t launch_mbconv_s8_walk(const MbconvParams &p, int cu_count, hipStream_t stream);
+
 // The same block with one wavefront per output tile and no workgroup barriers (mbconv_s8_wave.hip): 3x3
 // depthwise stage with stride 1 or 2, at most 64 block-input channels and 64 project filters.
 bool mbconv_s8_wave_supports(const MbconvParams &p);

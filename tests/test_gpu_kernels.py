@@ -1355,6 +1355,64 @@ def test_mbconv_s8_guard_free_builds_ragged_tiles(oracle, case):
     np.testing.assert_array_equal(to_host(got), cur)
 
 
+# The block as a walk down the image: strips that cross images, odd heights (half a row pair at the end), images narrower
+# than a strip, fewer expanded channels than the build (one chunk, five, eight), input channels that end inside a unit,
+# both project builds, one-sided, missing and wide padding.
+# (name, (N, H, W, Cin), Ce, Cout, stride, residual, pads)
+MBCONV_WALK = [
+    ("114x115_16_96_16_res", (2, 114, 115, 16), 96, 16, 1, True, (1, 1, 1, 1)),
+    ("57x23_24_144_24_res", (11, 57, 23, 24), 144, 24, 1, True, (1, 1, 1, 1)),
+    ("33x9_32_16_32_res", (900, 33, 9, 32), 16, 32, 1, True, (1, 1, 1, 1)),
+    ("59x33_48_48_64", (9, 59, 33, 48), 48, 64, 1, False, (1, 1, 1, 1)),
+    ("45x31_20_80_8_tailpad", (20, 45, 31, 20), 80, 8, 1, False, (0, 2, 0, 2)),
+    ("200x5_28_128_32_nopad", (7, 200, 5, 28), 128, 32, 1, False, (0, 0, 0, 0)),
+    ("44x30_48_144_48_widepad", (9, 44, 30, 48), 144, 48, 1, False, (2, 0, 2, 1)),
+    ("77x112_16_96_24_s2", (150, 77, 112, 16), 96, 24, 2, False, (1, 1, 1, 1)),
+    ("82x47_44_128_48_s2_tailpad", (12, 82, 47, 44), 128, 48, 2, False, (0, 1, 0, 1)),
+    ("55x61_24_144_32_s2_nopad", (200, 55, 61, 24), 144, 32, 2, False, (0, 0, 0, 0)),
+    ("70x19_16_48_16_s2", (60, 70, 19, 16), 48, 16, 2, False, (1, 1, 1, 1)),
+]
+
+
+@pytest.mark.parametrize("flavour", ["high_shifts", "low_shifts", "half_even", "half_even_low", "general", "residual_shift"])
+@pytest.mark.parametrize("case", MBCONV_WALK, ids=lambda c: c[0])
+def test_mbconv_s8_walk(oracle, case, flavour):
+    announce(f"mbconv_s8 walk {case[0]} {flavour}")
+    name, (n, h, w, cin), ce, cout, stride, with_res, pads = case
+    if flavour == "residual_shift" and not with_res:
+        pytest.skip("no residual operand")
+    m = espdl()
+    half_even = flavour.startswith("half_even")
+    rng = np.random.default_rng(0x3A1 + len(name))
+    rm_o = oracle.ROUND_HALF_EVEN if half_even else oracle.ROUND_HALF_UP
+    oracle.set_threads(16)
+
+    def stage(oc, kk, fshape):
+        f, b = rng_int8(rng, fshape), rng.integers(-4096, 4097, size=oc).astype(np.int32)
+        s = np.maximum(typical_shift(kk) + rng.integers(-2, 3, size=oc), 8).astype(np.int32)
+        if flavour.endswith("low") or flavour == "low_shifts":
+            f, s = (f >> 4).astype(np.int8), np.maximum(s - 4, 1).astype(np.int32)
+            s[0] = 1
+        if flavour == "general":
+            s[::3], s[1::5] = 0, 33
+        return f, b, s
+
+    x = rng_int8(rng, (n, h, w, cin))
+    ex, dw, pj = stage(ce, cin, (ce, 1, 1, cin)), stage(ce, 9, (3, 3, ce)), stage(cout, ce, (cout, 1, 1, ce))
+    cur = oracle.conv2d_s8(x, ex[0], ex[1], ex[2], (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), oracle.RELU, rm_o)
+    cur = oracle.depthwise_s8(cur, dw[0], dw[1], dw[2], (3, 3), (stride, stride), (1, 1), pads, oracle.LINEAR, rm_o)
+    cur = oracle.conv2d_s8(cur, pj[0], pj[1], pj[2], (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), oracle.LINEAR, rm_o)
+    res, res_shift = None, -2 if flavour == "residual_shift" else 0
+    if with_res:
+        res = rng_int8(rng, cur.shape)
+        cur = oracle.add_s8(cur, oracle.requantize_s8(res, res_shift, 0) if res_shift else res)
+    dev = lambda t: tuple(to_dev(a) for a in t)  # noqa: E731
+    got = m.mbconv_s8(to_dev(x), dev(ex), dev(dw), dev(pj), (3, 3), (stride, stride), (1, 1), pads, (True, False, False),
+                      residual=to_dev(res), residual_shift=res_shift,
+                      round_mode=m.capi.ROUND_HALF_EVEN if half_even else m.capi.ROUND_HALF_UP)
+    np.testing.assert_array_equal(to_host(got), cur)
+
+
 # The block as two launches (expand + depthwise, then project): tiles of 7 x 14, 7 x 7 and, at stride 2, 4 x 7 outputs with
 # ragged last rows and columns, one to three reduction steps of block-input channels (also 4 and 20: units that end
 # inside a pixel), expanded channels that leave a group of 64 unfinished, Clips, a requantized residual operand, shifts
