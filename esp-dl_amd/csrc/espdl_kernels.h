@@ -167,6 +167,9 @@ hipError_t launch_mbconv_s8_fused(const MbconvParams &p, int cu_count, hipStream
 // 48 block-input channels, 3x3 depthwise stage with stride 1 or 2.  Expected time; 1e30 where it does not apply.
 float mbconv_s8_walk_us(const MbconvParams &p, int cu_count);
 hipError_t launch_mbconv_s8_walk(const MbconvParams &p, int cu_count, hipStream_t stream);
+// The same with an expand stage of at most 3 x 3 taps over the channels of an image (mbconv_s8_walk_stem.hip).
+bool mbconv_s8_walk_stem_supports(const MbconvParams &p, int cu_count);
+hipError_t launch_mbconv_s8_walk_stem(const MbconvParams &p, int cu_count, hipStream_t stream);
 
 // The same block with one wavefront per output tile and no workgroup barriers (mbconv_s8_wave.hip): 3x3
 // depthwise stage with stride 1 or 2, at most 64 block-input channels and 64 project filters.
@@ -175,6 +178,7 @@ bool mbconv_s8_wave_supports(const MbconvParams &p);
 // The guarded builds cover every supported shape but do not beat the separate launches.
 bool mbconv_s8_wave_has_fast_build(const MbconvParams &p);
 float mbconv_s8_wave_us(const MbconvParams &p); // expected time of a guard-free build
+float mbconv_s8_wave_rounds(const MbconvParams &p); // tiles per wavefront that the device holds
 hipError_t launch_mbconv_s8_wave(const MbconvParams &p, int cu_count, hipStream_t stream);
 
 // The same block for small images (output at most 16 pixels wide): a workgroup of eight wavefronts per tile

@@ -126,6 +126,147 @@ __device__ __forceinline__ int finish4(const v4i &acc, const v4i &shift, const B
     }
 }
 
+// Clamps of the three stages.
+struct Range {
+    int lo, hi;
+};
+__device__ __forceinline__ Range expand_range(const MbconvParams &p)
+{
+    return {max(p.relu_expand ? 0 : -128, p.clip_e ? p.clip_e_lo : -128), p.clip_e ? p.clip_e_hi : 127};
+}
+__device__ __forceinline__ Range depthwise_range(const MbconvParams &p)
+{
+    return {max(p.relu_dw ? 0 : -128, p.clip_d ? p.clip_d_lo : -128), p.clip_d ? p.clip_d_hi : 127};
+}
+__device__ __forceinline__ Range project_range(const MbconvParams &p)
+{
+    return {p.relu_project ? 0 : -128, 127};
+}
+__device__ __forceinline__ Band make_band(const Range &r, bool high)
+{
+    const auto pair = [](int v) { return (v & 0xffff) * 0x00010001; };
+    return high ? Band{r.lo, r.hi, pair(r.lo * 256), 0} : Band{r.lo, r.hi, pair(r.lo), pair(r.hi)};
+}
+
+// The set-up's loads all read inside their arrays and are selected afterwards: none waits for another.
+// Depthwise filters: row i of chunk j in the lane group of its four channels, dword kx holds the weight in its own channel's
+// byte.
+template <int CE, int WAVES>
+__device__ __forceinline__ void load_depthwise(const MbconvParams &p, v4i (*wd)[3][64], int wave, int lane)
+{
+    constexpr int N = (3 * CE + WAVES - 1) / WAVES;
+    const int col = lane & 15, quad = lane >> 4;
+    unsigned w[N][3];
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const int e = min(wave + i * WAVES, 3 * CE - 1), j = e / 3, ky = e - 3 * j;
+        const int8_t *src = p.w_dw + ky * 3 * p.exp_c + min(16 * j + col, p.exp_c - 1);
+#pragma unroll
+        for (int kx = 0; kx < 3; kx++)
+            w[i][kx] = (unsigned char)src[kx * p.exp_c];
+    }
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const int e = wave + i * WAVES, j = e / 3;
+        const bool own = quad == (col >> 2) && 16 * j < p.exp_c;
+        const int at = 8 * (col & 3);
+        if (e < 3 * CE)
+            wd[j][e - 3 * j][lane] = own ? v4i{(int)(w[i][0] << at), (int)(w[i][1] << at), (int)(w[i][2] << at), 0} : v4i{0, 0, 0, 0};
+    }
+}
+
+// Project filters: byte 4 jj + r of lane group q in step g is channel 16 (4 g + jj) + 4 q + r, as the depthwise results lie.
+template <int G, int RT, int WAVES>
+__device__ __forceinline__ void load_project(const MbconvParams &p, v4i (*wp)[64], int wave, int lane)
+{
+    constexpr int N = (G * RT + WAVES - 1) / WAVES;
+    const int col = lane & 15, quad = lane >> 4;
+    v4i w[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const int e = min(wave + i * WAVES, G * RT - 1), g = e / RT, t = e - g * RT;
+        const int oc = min(4 * RT * (col >> 2) + 4 * t + (col & 3), p.out_c - 1);
+#pragma unroll
+        for (int jj = 0; jj < 4; jj++)
+            w[i][jj] = *reinterpret_cast<const int *>(p.w_project + oc * p.exp_c + min(16 * (4 * g + jj), p.exp_c - 16) + 4 * quad);
+    }
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const int e = wave + i * WAVES, g = e / RT, t = e - g * RT;
+        const bool filter = 4 * RT * (col >> 2) + 4 * t + (col & 3) < p.out_c;
+#pragma unroll
+        for (int jj = 0; jj < 4; jj++)
+            w[i][jj] = filter && 16 * (4 * g + jj) < p.exp_c ? w[i][jj] : 0;
+        if (e < G * RT)
+            wp[e][lane] = w[i];
+    }
+}
+
+// Start values and shifts of all stages (expand, depthwise, project) in LDS, and what their ranges allow: one table entry
+// per thread of a whole workgroup.
+struct Tables {
+    bool fast; // start values with the rounding added, all of them within the folded form, and no sum overflows
+    bool high; // fast, every shift at least 8, and no stage but a ReLU clamps: MODE 0
+    int start; // of this thread's entry
+};
+template <int CE, int RT, bool HE, int THREADS>
+__device__ __forceinline__ Tables make_tables(const MbWalkArgs &a, int *start, int *shift, int tid)
+{
+    constexpr int NC = 16 * (2 * CE + RT), TD = 16 * CE, TP = 32 * CE;
+    static_assert(NC <= THREADS);
+    const MbconvParams &p = a.p;
+    const int c = tid, stage = c < TD ? 0 : (c < TP ? 1 : 2);
+    const int ch = c - (stage == 0 ? 0 : (stage == 1 ? TD : TP)), n = stage == 2 ? p.out_c : p.exp_c;
+    const int32_t *sp = stage == 0 ? p.s_expand : (stage == 1 ? p.s_dw : p.s_project);
+    const int32_t *bp = stage == 0 ? p.b_expand : (stage == 1 ? p.b_dw : p.b_project);
+    const bool one = (stage == 0 ? p.n_s_expand : (stage == 1 ? p.n_s_dw : p.n_s_project)) == 1;
+    const long long bound = stage == 0 ? a.bound_e : (stage == 1 ? a.bound_d : a.bound_p);
+    int s = 8, b = 0;
+    const Range re = expand_range(p), rd = depthwise_range(p);
+    int ok = re.lo <= 0 && re.hi >= 0, high = re.hi == 127 && rd.hi == 127;
+    if (c < NC && ch < n) {
+        s = sp[one ? 0 : ch];
+        b = bp ? bp[ch] : 0;
+        const long long st = (long long)b + (1ll << ((s - 1) & 31)), mag = st < 0 ? -st : st;
+        if (s < 1 || s > 31 || mag + bound >= (1ll << 31) || (stage == 0 && mag > 240000))
+            ok = 0;
+        if (s < 8)
+            high = 0;
+    }
+    Tables t;
+    t.fast = __syncthreads_and(ok) != 0;
+    t.high = __syncthreads_and(high) != 0 && t.fast;
+    t.start = t.fast ? b + (1 << ((s - 1) & 31)) - (HE ? 1 : 0) : b;
+    if (c < NC) {
+        start[c] = t.start;
+        shift[c] = t.high ? s - 8 : s;
+    }
+    return t;
+}
+
+// A start value b as d0 + 127 (d1 + .. + d15): operand A of sixteen products whose operand B is 1 and fifteen times 127 where
+// the pixel exists and zeros where it does not.
+__device__ __forceinline__ v4i start_digits(int b)
+{
+    int t = (b + (b < 0 ? -63 : 63)) / 127;
+    int d[16];
+    d[0] = b - 127 * t;
+#pragma unroll
+    for (int i = 1; i < 16; i++) {
+        d[i] = min(max(t, -127), 127);
+        t -= d[i];
+    }
+    v4i w;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        w[i] = pack4_s8(d[4 * i], d[4 * i + 1], d[4 * i + 2], d[4 * i + 3]);
+    return w;
+}
+__device__ __forceinline__ v4i start_factors(int mask)
+{
+    return v4i{mask & 0x7f7f7f01, mask & 0x7f7f7f7f, mask & 0x7f7f7f7f, mask & 0x7f7f7f7f};
+}
+
 template <int CE, int RT, int S, bool HE, bool RES>
 __global__ __launch_bounds__((64 * MbShape<CE, RT, S, RES>::W), 2) void mbconv_s8_walk_kernel(const MbWalkArgs a)
 {
@@ -202,133 +343,45 @@ __global__ __launch_bounds__((64 * MbShape<CE, RT, S, RES>::W), 2) void mbconv_s
             asm volatile("s_nop 4\n\tbuffer_store_byte %0, %0, %1, 0 offen" ::"v"(kParked), "s"(rsrc_of(p.out, 0)) : "memory");
     };
 
-    // ---- set-up: filters into LDS in operand order, tables
-    {
-        // expand: row i of chunk j is filter 16 j + i; unit u holds input channels min(16 u, c0 - 16) .. + 15, those that
-        // unit u - 1 holds already as zeros
-        for (int e = wave; e < CE; e += kWaves) {
-            v4i w = {0, 0, 0, 0};
-            if (quad < units && 16 * e < p.exp_c) {
-                const int first = min(16 * quad, c0 - 16);
-                w = *reinterpret_cast<const v4i_unaligned *>(p.w_expand + (16 * e + col) * c0 + first);
-                const int skip = (16 * quad - first) >> 2; // dwords
-#pragma unroll
-                for (int d = 0; d < 4; d++)
-                    w[d] = d < skip ? 0 : w[d];
-            }
-            we_l[e][lane] = w;
-        }
-        // depthwise: row i of chunk j in the lane group of its four channels: dword kx holds the weight in its own
-        // channel's byte
-        for (int e = wave; e < 3 * CE; e += kWaves) {
-            const int j = e / 3, ky = e - 3 * j;
-            v4i w = {0, 0, 0, 0};
-            if (quad == (col >> 2) && 16 * j < p.exp_c)
-#pragma unroll
-                for (int kx = 0; kx < 3; kx++)
-                    w[kx] = (int)((unsigned)(unsigned char)p.w_dw[(ky * 3 + kx) * p.exp_c + 16 * j + col] << (8 * (col & 3)));
-            wd_l[j][ky][lane] = w;
-        }
-        // project: byte 4 jj + r of lane group q in step g is channel 16 (4 g + jj) + 4 q + r, as the depthwise results lie
-        for (int e = wave; e < G * RT; e += kWaves) {
-            const int g = e / RT, t = e - g * RT;
-            const int oc = 4 * RT * (col >> 2) + 4 * t + (col & 3);
-            v4i w = {0, 0, 0, 0};
-#pragma unroll
-            for (int jj = 0; jj < 4; jj++)
-                if (16 * (4 * g + jj) < p.exp_c && oc < p.out_c)
-                    w[jj] = *reinterpret_cast<const int *>(p.w_project + oc * p.exp_c + 16 * (4 * g + jj) + 4 * quad);
-            wp_l[e][lane] = w;
-        }
-    }
-    const auto constants = [&](int c, int &s, int &b, long long &bound) { // of table entry c; false: no such channel
-        s = 8;
-        b = 0;
-        bound = 0;
-        if (c < TP && (c < TD ? c : c - TD) >= p.exp_c)
-            return false;
-        if (c < TD) {
-            s = p.s_expand[p.n_s_expand == 1 ? 0 : c];
-            b = p.b_expand ? p.b_expand[c] : 0;
-            bound = a.bound_e;
-        } else if (c < TP) {
-            s = p.s_dw[p.n_s_dw == 1 ? 0 : c - TD];
-            b = p.b_dw ? p.b_dw[c - TD] : 0;
-            bound = a.bound_d;
-        } else if (c - TP < p.out_c) {
-            s = p.s_project[p.n_s_project == 1 ? 0 : c - TP];
-            b = p.b_project ? p.b_project[c - TP] : 0;
-            bound = a.bound_p;
-        } else {
-            return false;
-        }
-        return true;
-    };
-    const int lo_e = max(p.relu_expand ? 0 : -128, p.clip_e ? p.clip_e_lo : -128), hi_e = p.clip_e ? p.clip_e_hi : 127;
-    const int lo_d = max(p.relu_dw ? 0 : -128, p.clip_d ? p.clip_d_lo : -128), hi_d = p.clip_d ? p.clip_d_hi : 127;
-    int ok = lo_e <= 0 && hi_e >= 0, high = hi_e == 127 && hi_d == 127;
-    for (int c = tid; c < NC; c += kThreads) {
-        int s, b;
-        long long bound;
-        if (constants(c, s, b, bound)) {
-            if (s < 1 || s > 31) {
-                ok = 0;
-            } else {
-                const long long st = (long long)b + (1ll << (s - 1)), mag = st < 0 ? -st : st;
-                if (mag + bound >= (1ll << 31) || (c < TD && mag > 240000))
-                    ok = 0;
-            }
-            if (s < 8)
-                high = 0;
-        }
-    }
-    const bool fast = __syncthreads_and(ok) != 0;             // the folded form holds every start value, the sums fit
-    const bool is_high = __syncthreads_and(high) != 0 && fast; // MODE 0
-    for (int c = tid; c < NC; c += kThreads) {
-        int s, b;
-        long long bound;
-        (void)constants(c, s, b, bound);
-        start_l[c] = fast ? b + (1 << (s - 1)) - (HE ? 1 : 0) : b;
-        shift_l[c] = is_high ? s - 8 : s;
-    }
-    if (fast) {
-        // the start value b of a filter as d0 + 127 (d1 + .. + d15): sixteen products of the reduction's last lane group,
-        // whose operand B is 1 and fifteen times 127 where the pixel exists and zeros where it does not
-        __syncthreads();
-        for (int c = tid; c < TD; c += kThreads) {
-            const int b = start_l[c];
-            int t = (b + (b < 0 ? -63 : 63)) / 127;
-            int d[16];
-            d[0] = b - 127 * t;
-#pragma unroll
-            for (int i = 1; i < 16; i++) {
-                d[i] = min(max(t, -127), 127);
-                t -= d[i];
-            }
-            v4i w;
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                w[i] = pack4_s8(d[4 * i], d[4 * i + 1], d[4 * i + 2], d[4 * i + 3]);
-            we_l[c >> 4][48 + (c & 15)] = w;
-        }
-    }
-    if (lane < 16)
-        one_l[wave][0][lane] = v4i{0, 0, 0, 0};
+    // ---- set-up: the first copies, filters into LDS in operand order, tables
 #pragma unroll
     for (int e = 0; e < ET; e++)
         vin[e] = kParked;
 #pragma unroll
     for (int i = 0; i <= AHEAD; i++) {
         feed();
-        if (i > 0)
-            no_stores();
+        no_stores();
     }
+    {
+        // expand: row i of chunk j is filter 16 j + i; unit u holds input channels min(16 u, c0 - 16) .. + 15, those that
+        // unit u - 1 holds already as zeros
+        constexpr int N = (CE + kWaves - 1) / kWaves;
+        const int first = min(16 * quad, c0 - 16), skip = (16 * quad - first) >> 2; // bytes, dwords
+        v4i w[N];
+#pragma unroll
+        for (int i = 0; i < N; i++)
+            w[i] = *reinterpret_cast<const v4i_unaligned *>(p.w_expand + min(16 * (wave + i * kWaves) + col, p.exp_c - 1) * c0 + first);
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const int e = wave + i * kWaves;
+#pragma unroll
+            for (int d = 0; d < 4; d++)
+                w[i][d] = d < skip || quad >= units || 16 * e >= p.exp_c ? 0 : w[i][d];
+            if (e < CE)
+                we_l[e][lane] = w[i];
+        }
+    }
+    load_depthwise<CE, kWaves>(p, wd_l, wave, lane);
+    load_project<G, RT, kWaves>(p, wp_l, wave, lane);
+    const Range range_e = expand_range(p), range_d = depthwise_range(p);
+    const Tables tab = make_tables<CE, RT, HE, kThreads>(a, start_l, shift_l, tid);
+    const bool fast = tab.fast, is_high = tab.high;
+    if (fast && tid < TD)
+        we_l[tid >> 4][48 + (tid & 15)] = start_digits(tab.start);
+    if (lane < 16)
+        one_l[wave][0][lane] = v4i{0, 0, 0, 0};
     __syncthreads();
-    const auto band = [&](int lo, int hi) {
-        const auto pair = [](int v) { return (v & 0xffff) * 0x00010001; };
-        return is_high ? Band{lo, hi, pair(lo * 256), 0} : Band{lo, hi, pair(lo), pair(hi)};
-    };
-    const Band band_e = band(lo_e, hi_e), band_d = band(lo_d, hi_d), band_p = band(p.relu_project ? 0 : -128, 127);
+    const Band band_e = make_band(range_e, is_high), band_d = make_band(range_d, is_high), band_p = make_band(project_range(p), is_high);
 
     const int c_of = 4 * quad; // of this lane's four channels of a chunk
     const Requant4 res_q = make_requant4(p.residual_shift);
@@ -372,7 +425,7 @@ __global__ __launch_bounds__((64 * MbShape<CE, RT, S, RES>::W), 2) void mbconv_s
             int n, x;
             emask[e] = in_pixel(v0, lane_now & 15, e, n, x) ? -1 : 0;
             if (lane < 16)
-                one_l[wave][1 + e][lane] = v4i{emask[e] & 0x7f7f7f01, emask[e] & 0x7f7f7f7f, emask[e] & 0x7f7f7f7f, emask[e] & 0x7f7f7f7f};
+                one_l[wave][1 + e][lane] = start_factors(emask[e]);
         }
         const int o = (lane_now & 15) - Shape::kFirst, v = v0 + max(o, 0);
         const int n = (int)fastdiv((unsigned)v, a.fd_po);
@@ -411,7 +464,7 @@ __global__ __launch_bounds__((64 * MbShape<CE, RT, S, RES>::W), 2) void mbconv_s
             if (c_left == 0)
                 segment();
             c_left--;
-            wait_copies<AHEAD * (kCopies + kStores)>(); // this step's input has arrived
+            wait_copies<AHEAD * (kCopies + kStores) + kStores>(); // this step's input has arrived
             read_x(c_row);
             const int out_y = ((c_row + p.pad_top) >> (S - 1)) - NR; // first output row this step finishes
             if constexpr (RES) { // asked for now, needed at the end of the step

@@ -1043,14 +1043,20 @@ bool mbconv_s8_wave_supports(const MbconvParams &p)
     return wave_plan(p).ok;
 }
 
+// Tiles per wavefront that the device holds (two workgroups per compute unit).
+float mbconv_s8_wave_rounds(const MbconvParams &p)
+{
+    const WavePlan plan = wave_plan(p);
+    return (float)((long long)p.batch * plan.a.tiles_y * plan.a.tiles_x) / (2.f * kPlanCus * kWavesPerGroup);
+}
+
 // A wavefront's chain over all expanded channels, whatever the batch, until the wavefronts fill the device at two per
 // SIMD; then rounds (MobileNetV2's blocks at batch 1 to 256, within 20 %).
 float mbconv_s8_wave_us(const MbconvParams &p)
 {
-    const WavePlan plan = wave_plan(p);
     const float n_sub = (float)(p.exp_c / 16);
     const float chain = (p.stride_h == 1 ? 7.f + 1.1f * n_sub : 5.5f + 0.9f * n_sub) * (p.half_even ? 1.2f : 1.f);
-    const float fill = (float)((long long)p.batch * plan.a.tiles_y * plan.a.tiles_x) / (2.f * kPlanCus * kWavesPerGroup);
+    const float fill = mbconv_s8_wave_rounds(p);
     return chain * (fill <= 1.f ? 1.f + 0.45f * fill : 1.45f * fill);
 }
 

@@ -1413,6 +1413,58 @@ def test_mbconv_s8_walk(oracle, case, flavour):
     np.testing.assert_array_equal(to_host(got), cur)
 
 
+# A windowed expand stage as a walk down the image, at batches where the tile kernel needs more than one round: one to three
+# expanded chunks, both project builds, windows that start at every byte of a dword, padding on every side and none, images
+# whose first and last pixels lie at the ends of the tensor.
+# (name, (N, H, W, Cin), expand (kernel, stride, pads), Ce, Cout, depthwise pads, Clip)
+STEM_WALK = [
+    ("rgb_64x60_s2_tailpad", (270, 64, 60, 3), ((3, 3), (2, 2), (0, 1, 0, 1)), 32, 16, (1, 1, 1, 1), False),
+    ("rgb_66x72_s2_clip", (270, 66, 72, 3), ((3, 3), (2, 2), (1, 1, 1, 1)), 32, 16, (1, 1, 1, 1), True),
+    ("rgb_95x120_s2_48_24", (130, 95, 120, 3), ((3, 3), (2, 2), (1, 0, 1, 0)), 48, 24, (0, 2, 0, 2), False),
+    ("rgb_61x64_s2_nopad_16_4", (270, 61, 64, 3), ((3, 3), (2, 2), (0, 0, 0, 0)), 16, 4, (0, 0, 0, 0), False),
+    ("gray_40x64_s2_16_8", (330, 40, 64, 1), ((3, 3), (2, 2), (2, 1, 2, 1)), 16, 8, (1, 1, 1, 1), False),
+    ("two_40x34_s1_32_32", (330, 40, 34, 2), ((2, 3), (1, 1), (1, 1, 1, 1)), 32, 32, (2, 0, 2, 1), False),
+    ("four_37x44_s1_32_12", (330, 37, 44, 4), ((3, 2), (1, 1), (1, 1, 0, 1)), 32, 12, (1, 1, 1, 1), False),
+]
+
+
+@pytest.mark.parametrize("flavour", ["high_shifts", "low_shifts", "half_even", "general"])
+@pytest.mark.parametrize("case", STEM_WALK, ids=lambda c: c[0])
+def test_mbconv_s8_walk_stem(oracle, case, flavour):
+    announce(f"mbconv_s8 walk with a windowed expand stage {case[0]} {flavour}")
+    name, (n, h, w, cin), (ek, es, ep), ce, cout, pads, clip = case
+    if clip and flavour == "half_even":
+        pytest.skip("a Clip between the stages: round half up")
+    m = espdl()
+    half_even = flavour == "half_even"
+    rm_o = oracle.ROUND_HALF_EVEN if half_even else oracle.ROUND_HALF_UP
+    rng = np.random.default_rng(0x57A1 + len(name))
+    oracle.set_threads(16)
+
+    def stage(oc, kk, fshape):
+        f, b = rng_int8(rng, fshape), rng.integers(-4096, 4097, size=oc).astype(np.int32)
+        s = np.maximum(typical_shift(kk) + rng.integers(-2, 3, size=oc), 8).astype(np.int32)
+        if flavour == "low_shifts":
+            f, s = (f >> 4).astype(np.int8), np.maximum(s - 4, 1).astype(np.int32)
+        if flavour == "general":
+            s[::3], s[1::5] = 0, 33
+        return f, b, s
+
+    x = rng_int8(rng, (n, h, w, cin))
+    x[:, 0, :, :], x[:, -1, :, :] = 127, 126   # make the borders count
+    x[:, :, 0, :], x[:, :, -1, :] = -128, -127
+    ex, dw, pj = stage(ce, ek[0] * ek[1] * cin, (ce, ek[0], ek[1], cin)), stage(ce, 9, (3, 3, ce)), stage(cout, ce, (cout, 1, 1, ce))
+    cur = oracle.conv2d_s8(x, ex[0], ex[1], ex[2], ek, es, (1, 1), ep, oracle.LINEAR, rm_o)
+    cur = oracle.clip_s8(cur, 5, 90, 0, 0) if clip else cur
+    cur = oracle.depthwise_s8(cur, dw[0], dw[1], dw[2], (3, 3), (1, 1), (1, 1), pads, oracle.RELU, rm_o)
+    cur = oracle.conv2d_s8(cur, pj[0], pj[1], pj[2], (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), oracle.LINEAR, rm_o)
+    dev = lambda t: tuple(to_dev(a) for a in t)  # noqa: E731
+    got = m.mbconv_s8(to_dev(x), dev(ex), dev(dw), dev(pj), (3, 3), (1, 1), (1, 1), pads, (False, True, False),
+                      round_mode=m.capi.ROUND_HALF_EVEN if half_even else m.capi.ROUND_HALF_UP,
+                      clip_expand=(5, 90) if clip else None, expand_conv=(ek, es, ep))
+    np.testing.assert_array_equal(to_host(got), cur)
+
+
 # The block as two launches (expand + depthwise, then project): tiles of 7 x 14, 7 x 7 and, at stride 2, 4 x 7 outputs with
 # ragged last rows and columns, one to three reduction steps of block-input channels (also 4 and 20: units that end
 # inside a pixel), expanded channels that leave a group of 64 unfinished, Clips, a requantized residual operand, shifts
