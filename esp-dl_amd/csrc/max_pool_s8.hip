@@ -14,11 +14,14 @@
 // The window is separable: a thread owns two neighbouring output columns and one 16-byte channel vector, walks
 // down a strip of output rows, takes the horizontal maxima of each input row once (K + 1 loaded pixels, K
 // maxima for the two columns since their windows share K - 1 pixels), keeps the last K of them in registers
-// (joined back into bytes, which halves their registers and lets a fourth wavefront onto each SIMD) and takes
-// the vertical maximum for each output row.  Pixels outside the image count as -128, which never wins against
-// a pixel inside (every window of a valid geometry holds at least one).  The walk is bound by the latency of
-// its loads (each pixel is requested by three threads), not by the arithmetic: 0.60 of the HBM rate on large
-// tensors against 0.10 for the byte-wise kernel.
+// (joined back into bytes, which halves their registers) and takes the vertical maximum for each output row.  A pixel
+// outside the image is replaced by the nearest one inside, which the same window holds (every window of a valid geometry
+// holds at least one): no load is conditional, and a row's loads are requested while the row before it is worked on.
+//
+// Bound by memory, and by how many rows are in flight at once: with conditional loads, none of them early, and four
+// wavefronts per SIMD 256 images of 56 x 56 x 144 took 69 us (3 x 3: 61), 100 of 80 x 80 x 96 44 us (37) and 64 of
+// 20 x 20 x 128 6.9 us; a row ahead 64, 41 and 5.8 us, and with two wavefronts per SIMD, whose longer strips read fewer rows
+// twice, 59 (55), 34 (31) and 6 us: 3.9 TB/s in and out, 4.2 at 3 x 3.
 // Input and output may be channel slices of wider tensors (pitches in bytes).  Where the channels are no multiple of
 // the vector, the last one of a pixel reaches back over its neighbour's channels and both write the same bytes: 36 x 8 x
 // 194, 128 images take 13.4 us, one byte per thread took 101 us.
@@ -125,45 +128,39 @@ __global__ __launch_bounds__(kThreads) void max_pool_s8_window_kernel(const Wind
     const char *img_in = a.in + (long long)n * a.h * a.w * a.in_pitch + c0;
     char *img_out = a.out + (long long)n * a.out_h * a.out_w * a.out_pitch + c0;
 
-    // the K + 1 input columns under the two windows
+    // The K + 1 input columns under the two windows.  A column or row outside the image is replaced by the nearest one inside:
+    // the window holds that one too, so its maximum stays the same and every load is unconditional.
     long long col_off[K + 1];
-    bool col_ok[K + 1];
 #pragma unroll
-    for (int c = 0; c <= K; c++) {
-        const int ix = x0 - a.pad_left + c;
-        col_ok[c] = ix >= 0 && ix < a.w;
-        col_off[c] = (long long)ix * a.in_pitch;
-    }
+    for (int c = 0; c <= K; c++)
+        col_off[c] = (long long)min(max(x0 - a.pad_left + c, 0), a.w - 1) * a.in_pitch;
     const bool second = x0 + 1 < a.out_w;
-    V outside;
-#pragma unroll
-    for (int i = 0; i < D; i++)
-        outside.d[i] = (int)0x80808080;
+    const long long row_pitch = (long long)a.w * a.in_pitch;
 
-    // the K + 1 pixels of input row `r` of the strip (rows and columns outside the image count as -128)
+    // the K + 1 pixels of input row `r` of the strip
     auto load_row = [&](int r, V (&px)[K + 1]) {
-        const int iy = y0 - a.pad_top + r;
-        const bool row_ok = iy >= 0 && iy < a.h;
-        const char *row = img_in + (long long)iy * a.w * a.in_pitch;
+        const char *row = img_in + min(max(y0 - a.pad_top + r, 0), a.h - 1) * row_pitch;
 #pragma unroll
         for (int c = 0; c <= K; c++)
-            px[c] = (row_ok && col_ok[c]) ? load_vec<D>(row + col_off[c]) : outside;
+            px[c] = load_vec<D>(row + col_off[c]);
     };
 
     // horizontal maxima of the last K input rows, as bytes again: [row][column of the pair]
     V hist[K][2];
     const int nrows = a.rows + K - 1;
+    V next[K + 1];
+    load_row(0, next);
     for (int base = 0; base < nrows; base += K) {
 #pragma unroll
         for (int j = 0; j < K; j++) {
             const int r = base + j;
             V odd[K + 1], even[K + 1];
-            load_row(r, odd);
 #pragma unroll
-            for (int c = 0; c <= K; c++)
-#pragma unroll
-                for (int i = 0; i < D; i++)
-                    even[c].d[i] = odd[c].d[i] << 8;
+            for (int c = 0; c <= K; c++) {
+                odd[c] = next[c];
+                even[c] = shifted(odd[c]);
+            }
+            load_row(r + 1, next); // (the last one is not used)
             // columns 1 .. K-1 are under both windows
             V both_odd = odd[1], both_even = even[1];
 #pragma unroll
@@ -238,13 +235,12 @@ hipError_t launch_max_pool_s8_window(const void *in, int batch, int h, int w, in
     a.in_pitch = in_pitch;
     a.out_pitch = out_pitch;
     a.xpairs = (out_w + 1) / 2;
-    // Strips per image.  Long strips read each input row once; a strip of `rows` rows reads k - 1 rows more
-    // (mostly from cache, but the horizontal maxima are taken again).  Short strips give small tensors enough
-    // wavefronts, and the count decides how evenly the last round of wavefronts fills the chip (about four
-    // wavefronts fit a SIMD).  Measured on 327 images of 80 x 80 x 128: 0.60 of the HBM rate at 5 strips (two
-    // full rounds), 0.57 at 4 (2.1 rounds in 3), 0.54 at 8.
+    // Strips per image.  Long strips read each input row once; a strip of `rows` rows reads k - 1 rows more (mostly from
+    // cache, but the horizontal maxima are taken again).  Short strips give small tensors enough wavefronts, and the count
+    // decides how evenly the last round of wavefronts fills the chip, two per SIMD: with four the strips are half as long,
+    // which loses on every layer from 30 MB on (5 to 20 %) and gains on none of fourteen from 50 kB on.
     const long long per_row = (long long)batch * a.xpairs * a.cv;
-    const double capacity = (double)(cu_count > 0 ? cu_count : 256) * 4 * 4;
+    const double capacity = (double)(cu_count > 0 ? cu_count : 256) * 4 * 2;
     int best_strips = 1;
     double best_score = -1.0;
     for (int strips = 1;;) { // of the counts with one strip height only the smallest: 2 sqrt(out_h) of them
