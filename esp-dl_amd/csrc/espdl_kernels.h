@@ -98,6 +98,12 @@ struct DwExpand {
     int n_shift, relu, c0;
 };
 
+// First layers as a walk down the image (conv2d_s8_walk_stem.hip): window rows of at most 13 bytes, up to four of them, image
+// rows of whole dwords, up to 64 filters.
+bool conv2d_s8_walk_stem_supports(const ConvGeom &g, const void *in, const void *out, const void *residual);
+hipError_t launch_conv2d_s8_walk_stem(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias, const int32_t *shift,
+                                      const int8_t *lut, const int8_t *residual, int8_t *out, int cu_count, hipStream_t stream);
+
 // Pointwise layers of at most 128 channels under thousands of filters, rows of the result no multiple of 16 bytes long
 // (conv2d_s8_wide.hip)
 bool conv2d_s8_wide_supports(const ConvGeom &g, const int8_t *lut, const int8_t *residual);

@@ -192,6 +192,56 @@ def test_conv2d_s8_channel_units(oracle, case, flavour):
     np.testing.assert_array_equal(got, want)
 
 
+# First layers as a walk down the image: image rows of whole 16-byte pieces; filter rows that begin at every byte of a dword,
+# one to four of them, both step heights, every count of filter tiles, ragged last strips and rows, padding on every side.
+# (batch, (name, (H, W, Cin), Cout, k, stride, dilation, pads, relu, bias))
+STEM_WALK_CONV = [
+    (3, ("rgb_k3s2_tailpad", (65, 112, 3), 16, (3, 3), (2, 2), (1, 1), (0, 1, 0, 1), True, True)),
+    (2, ("rgb_k3s2_32", (50, 80, 3), 32, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), True, True)),
+    (2, ("rgb_k3s2_64", (37, 96, 3), 64, (3, 3), (2, 2), (1, 1), (1, 0, 1, 0), False, True)),
+    (70, ("rgb_k3s2_nopad_narrow", (33, 16, 3), 16, (3, 3), (2, 2), (1, 1), (0, 0, 0, 0), True, False)),
+    (2, ("four_k3s1", (29, 40, 4), 16, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
+    (5, ("two_k4x5_s1", (23, 56, 2), 32, (4, 5), (1, 1), (1, 1), (3, 1, 2, 2), True, True)),
+    (4, ("gray_k4x7_s2", (40, 80, 1), 16, (4, 7), (2, 2), (1, 1), (2, 2, 3, 3), True, True)),
+    (9, ("rgb_k2_s4", (64, 64, 3), 64, (2, 2), (4, 4), (1, 1), (0, 0, 0, 0), False, True)),
+]
+
+
+@pytest.mark.parametrize("case", STEM_WALK_CONV, ids=lambda c: c[1][0])
+@pytest.mark.parametrize("flavour", ["per_channel", "low_shifts", "lut", "half_even", "general_epilogue", "out_slice"])
+def test_conv2d_s8_walk_stem(oracle, case, flavour):
+    """First layers as a walk: short epilogues with and without shifts below 8, a table, half even, the general form, and an
+    output that is a channel slice of a wider tensor."""
+    import torch
+    announce(f"conv2d_s8 walk stem {case[1][0]} {flavour}")
+    x, f, bias, shift, k, stride, dil, pads, relu = _conv_inputs(case[1], 271, case[0], True)
+    x[:, 0], x[:, -1], x[:, :, 0], x[:, :, -1] = 127, 126, -128, -127   # make the borders count
+    kw = {}
+    shift = np.maximum(np.array(shift, dtype=np.int32), 8)
+    if flavour == "low_shifts":
+        shift, f = (np.arange(shift.size) % 5 + 4).astype(np.int32), (f >> 3).astype(np.int8)
+    if flavour == "lut":
+        kw["lut"] = np.array([(i * 109 + 37) & 0xFF for i in range(256)], dtype=np.uint8).view(np.int8)
+    if flavour == "half_even":
+        kw["half_even"] = True
+    if flavour == "general_epilogue":
+        shift[::3], shift[1::5] = 0, 33
+    oracle.set_threads(16)
+    if flavour != "out_slice":
+        got, want = _run_conv_s8(oracle, x, f, bias, shift, k, stride, dil, pads, relu, **kw)
+        np.testing.assert_array_equal(got, want)
+        return
+    m = espdl()
+    oc = f.shape[0]
+    want = oracle.conv2d_s8(x, f, bias, shift, k, stride, dil, pads, oracle.RELU if relu else oracle.LINEAR, oracle.ROUND_HALF_UP)
+    wide = torch.full(want.shape[:3] + (oc + 20,), -9, dtype=torch.int8, device="cuda")
+    m.conv2d(to_dev(x), to_dev(f), to_dev(bias), to_dev(shift), k, stride, dil, pads,
+             activation=m.capi.RELU if relu else m.capi.LINEAR, out=wide[..., 4:4 + oc])
+    got = to_host(wide)
+    np.testing.assert_array_equal(got[..., 4:4 + oc], want)
+    assert (got[..., :4] == -9).all() and (got[..., 4 + oc:] == -9).all()
+
+
 @pytest.mark.parametrize("case", WALK_CASES, ids=lambda c: c[1][0])
 @pytest.mark.parametrize("flavour", ["per_channel", "low_shifts", "lut_residual", "general_epilogue", "slices"])
 def test_conv2d_s8_walk(oracle, case, flavour):
