@@ -9,8 +9,8 @@
 // 1.9 TB/s; so a step's bytes pass through LDS and leave as whole aligned 16-byte pieces of memory, cut out of the bytes
 // of this step and the last 16 of the step before, and only the two ends of a row's walk are written by the byte.
 //
-// 20480 pixels x 120 -> 6625 (136 MB written, 26 us at the copy rate): 51 us inside the recognizer, where the kernel that
-// keeps filters in LDS took 71 us; 50 against 69 us on one pair of tensors, 61 against 76 us on changing ones.  A third of
+// 20480 pixels x 120 -> 6625 (136 MB written, 26 us at the copy rate): 49 us inside the recognizer (51 where a shift is below
+// 8, which takes the epilogue with left shifts), where the kernel that keeps filters in LDS took 71 us.  A third of
 // that is the start of a walk (its pixels and constants), of which every compute unit does four.
 //
 // Restates conv2d_11cn (esp-dl/dl/base/dl_base_conv2d.cpp:9-33) with the n_wise epilogue
@@ -86,7 +86,7 @@ __global__ __launch_bounds__(kThreads, 2) void conv2d_s8_wide_kernel(const WideA
     v4i fa[4][KS];
     fetch(n_begin + 64 * wave, fa);
 
-    int ok = 1; // the short epilogue is exact
+    int ok = 1, low = 0; // the short epilogue is exact; some shift is below 8
     for (int i0 = tid; i0 < a.per_walk; i0 += 6 * kThreads) { // six at a time: their loads are in flight together
         int sh[6], bias[6];
 #pragma unroll
@@ -101,6 +101,8 @@ __global__ __launch_bounds__(kThreads, 2) void conv2d_s8_wide_kernel(const WideA
             const long long start = (long long)bias[u] + (1ll << (s - 1));
             if (sh[u] != s || (start < 0 ? -start : start) + (long long)a.K * 16384 >= 1ll << (31 - max(0, 8 - s)))
                 ok = 0;
+            if (s < 8)
+                low = 1;
             if (i < a.per_walk) {
                 c_start[i] = (int)start - (a.half_even ? 1 : 0);
                 c_rsh[i] = max(0, s - 8);
@@ -113,7 +115,7 @@ __global__ __launch_bounds__(kThreads, 2) void conv2d_s8_wide_kernel(const WideA
 #pragma unroll
         for (int k = 0; k < KS; k++)
             b[c][k] = mask_unit<false>(b[c][k], max(a.K - (64 * k + 16 * quad), 0));
-    const bool fast = __syncthreads_and(ok) != 0;
+    const bool fast = __syncthreads_and(ok) != 0, high = __syncthreads_or(low) == 0;
 
     const int floor_pk = a.relu ? 0 : (int)0x80008000u;
     // The walk's bytes of row r start lead(r) bytes into a 16-byte piece of memory.
@@ -163,7 +165,9 @@ __global__ __launch_bounds__(kThreads, 2) void conv2d_s8_wide_kernel(const WideA
 #pragma unroll
             for (int t = 0; t < 4; t++) {
                 const v4i rsh = *reinterpret_cast<const v4i *>(&c_rsh[at + 4 * t]);
-                const v4i lsh = *reinterpret_cast<const v4i *>(&c_lsh[at + 4 * t]);
+                v4i lsh = {0, 0, 0, 0};
+                if constexpr (MODE != 0 && MODE != 6)
+                    lsh = *reinterpret_cast<const v4i *>(&c_lsh[at + 4 * t]);
 #pragma unroll
                 for (int c = 0; c < 4; c++) {
                     if constexpr (MODE >= 0) {
@@ -226,9 +230,9 @@ __global__ __launch_bounds__(kThreads, 2) void conv2d_s8_wide_kernel(const WideA
     if (!fast)
         walk(std::integral_constant<int, -1>{});
     else if (a.half_even)
-        walk(std::integral_constant<int, 5>{});
+        high ? walk(std::integral_constant<int, 6>{}) : walk(std::integral_constant<int, 5>{});
     else
-        walk(std::integral_constant<int, 1>{});
+        high ? walk(std::integral_constant<int, 0>{}) : walk(std::integral_constant<int, 1>{});
 }
 
 // The tile and the constants of walks of 10 steps and more are past the 64 KB of LDS that a launch may have unasked

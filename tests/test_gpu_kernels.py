@@ -603,6 +603,20 @@ def test_conv2d_s8_wide_filters(oracle, m, k, n, pad, variant):
     assert (np.delete(got, np.s_[lo_c:lo_c + n], axis=3) == 77).all()
 
 
+@pytest.mark.parametrize("half_even", [False, True], ids=["half_up", "half_even"])
+@pytest.mark.parametrize("lo", [7, 8], ids=["some_below_8", "none_below_8"])
+def test_conv2d_s8_wide_filters_epilogues(oracle, lo, half_even):
+    """A walk whose shifts are all at least 8 takes the epilogue without left shifts."""
+    announce(f"conv2d_s8 wide filters epilogues lo={lo} half_even={half_even}")
+    rng = np.random.default_rng(0xF7)
+    x, f = rng_int8(rng, (1030, 1, 1, 120)), rng_int8(rng, (2307, 1, 1, 120))
+    shift = rng.integers(lo, 13, size=2307).astype(np.int32)
+    oracle.set_threads(16)
+    got, want = _run_conv_s8(oracle, x, f, rng.integers(-4096, 4097, size=2307).astype(np.int32), shift, (1, 1), (1, 1), (1, 1),
+                             (0, 0, 0, 0), False, half_even=half_even)
+    np.testing.assert_array_equal(got, want)
+
+
 # Walks of 10, 11 and 12 steps, whose constants take the kernel past 64 KB of LDS.
 @pytest.mark.parametrize("m,k,n", [(20003, 64, 2305), (20480, 17, 2563), (30000, 80, 2817)])
 def test_conv2d_s8_wide_filters_long_walks(oracle, m, k, n):
