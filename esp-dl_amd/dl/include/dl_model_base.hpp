@@ -35,8 +35,8 @@ enum { FUSE_CONV_LUT = 1, FUSE_DW_PROJECT = 2, FUSE_CONV_ADD = 4, FUSE_CONV_GAP 
 class Model {
 public:
     /// The model does not take ownership of `fbs_model`.  `stream` is a hipStream_t (nullptr: the
-    /// model creates its own).  `fuse` is a bit mask of graph fusions: FUSE_CONV_LUT folds a LUT that directly follows a Conv
-    /// into its epilogue (int16: where the Conv also takes over a RequantizeLinear from int8 in front of it), FUSE_DW_PROJECT runs depthwise Conv -> 1x1 Conv [-> Add] as one kernel,
+    /// model creates its own).  `fuse` is a bit mask of graph fusions: FUSE_CONV_LUT folds a LUT that directly follows a Conv,
+    /// a Gemm or a MatMul by a constant into its epilogue (int16: where the Conv also takes over a RequantizeLinear from int8 in front of it), FUSE_DW_PROJECT runs depthwise Conv -> 1x1 Conv [-> Add] as one kernel,
     /// FUSE_CONV_ADD folds the Add behind a dense Conv into its epilogue and joins the RequantizeLinears in front of
     /// an Add and a Concat that read the same tensor or the pieces of one Split, FUSE_CONV_GAP runs a 1x1 Conv and the
     /// GlobalAveragePool behind it as one kernel that writes the pooled tensor only, FUSE_CHANNEL_SLICES leaves the

@@ -34,14 +34,44 @@ inline std::vector<int32_t> conv_shifts(TensorBase *output, TensorBase *input, T
     return conv_shifts(output->exponent.get(), input, filter, out_c);
 }
 
-class Conv : public Module {
+/// Conv, Gemm and MatMul: a LUT that directly follows may run in the epilogue.
+class TableEpilogue {
+public:
+    virtual ~TableEpilogue() { delete m_fused_lut; }
+    /// Take ownership of a LUT (host or device tensor) to apply in the epilogue.
+    /// `table_in_exponent` is the exponent of the value the table is indexed with, i.e. of this
+    /// module's own (no longer materialized) output: the requantization shift is derived from it,
+    /// not from the exponent of the tensor the table's result is stored to.
+    void fuse_lut(TensorBase *table, int table_in_exponent)
+    {
+        delete m_fused_lut;
+        m_fused_lut = table;
+        m_lut_in_exponent = table_in_exponent;
+    }
+    bool has_fused_lut() const { return m_fused_lut != nullptr; }
+
+protected:
+    /// The table on the device, or nullptr.
+    const TensorBase *device_lut(ModelContext *context)
+    {
+        if (m_fused_lut && !m_fused_lut->on_device()) {
+            TensorBase *dev = m_fused_lut->to_device(context->stream);
+            delete m_fused_lut;
+            m_fused_lut = dev;
+        }
+        return m_fused_lut;
+    }
+    TensorBase *m_fused_lut = nullptr; ///< applied to the stored value (owned)
+    int m_lut_in_exponent = 0;         ///< exponent of the result that indexes it
+};
+
+class Conv : public Module, public TableEpilogue {
 private:
     activation_type_t activation;
     std::vector<int> m_pads;      ///< {top, bottom, left, right} (2-D) or {left, right} (1-D)
     std::vector<int> m_dilations; ///< {h, w} or {w}
     std::vector<int> m_strides;   ///< {h, w} or {w}
     int m_group;
-    TensorBase *m_fused_lut; ///< device int8[256] applied to the stored value, or nullptr (owned)
     DeviceInts m_shift;
     // A depthwise Conv may absorb the 1x1 Conv that follows it (and the Add after that): the three
     // run as one kernel and the depthwise result stays on chip.  The absorbed modules' parameter
@@ -49,7 +79,6 @@ private:
     bool m_has_project = false;
     activation_type_t m_project_activation = Linear;
     int m_mid_exponent = 0;      ///< exponent of the (no longer materialized) depthwise output
-    int m_lut_in_exponent = 0;   ///< exponent of the conv result that indexes a fused LUT
     int m_project_filter_pos = -1, m_project_bias_pos = -1, m_residual_pos = -1;
     int m_residual_shift = 0;
     bool m_x8 = false;           ///< int16 convolution on an int8 input
@@ -83,25 +112,12 @@ public:
         m_pads(pads),
         m_dilations(dilations),
         m_strides(strides),
-        m_group(group),
-        m_fused_lut(nullptr)
+        m_group(group)
     {
     }
-    ~Conv() { delete m_fused_lut; }
 
     int get_group() const { return m_group; }
     activation_type_t get_activation() const { return activation; }
-    /// Take ownership of a LUT (host or device tensor of 256 int8) to apply in the epilogue.
-    /// `table_in_exponent` is the exponent of the value the table is indexed with, i.e. of this
-    /// convolution's own (no longer materialized) output: the requantization shift is derived from it,
-    /// not from the exponent of the tensor the table's result is stored to.
-    void fuse_lut(TensorBase *table, int table_in_exponent)
-    {
-        delete m_fused_lut;
-        m_fused_lut = table;
-        m_lut_in_exponent = table_in_exponent;
-    }
-    bool has_fused_lut() const { return m_fused_lut != nullptr; }
     /// int16 only: take the int8 tensor that a RequantizeLinear multiplied by 256 (its output is eight exponents finer)
     /// as the input.  `in_exponent` is the exponent of the int16 tensor this convolution used to read.
     void fuse_requantize(int int8_index, int in_exponent)
@@ -359,16 +375,12 @@ public:
             conv_shifts(m_x8 ? out_exponent + input->exponent.get() - m_x8_in_exponent : out_exponent, input, filter, d.out_c);
         d.n_shift = (int32_t)shifts.size();
         const int32_t *shift_dev = m_shift.sync(shifts);
-        if (m_fused_lut && !m_fused_lut->on_device()) {
-            TensorBase *dev = m_fused_lut->to_device(context->stream);
-            delete m_fused_lut;
-            m_fused_lut = dev;
-        }
+        const TensorBase *lut = device_lut(context);
         if (m_x8) {
             const int rc = espdl_hip_conv2d_s16_x8(
                 &d, static_cast<const int8_t *>(input->data), static_cast<const int16_t *>(filter->data),
                 bias ? static_cast<const int64_t *>(bias->data) : nullptr, shift_dev,
-                m_fused_lut ? static_cast<const int16_t *>(m_fused_lut->data) : nullptr, m_fused_lut ? m_fused_lut->get_size() : 0,
+                lut ? static_cast<const int16_t *>(lut->data) : nullptr, lut ? lut->get_size() : 0,
                 static_cast<int16_t *>(output->data), context->stream);
             if (rc != ESPDL_HIP_OK)
                 DL_LOGE("Conv", "%s: %s", name.c_str(), espdl_hip_last_error());
@@ -381,7 +393,7 @@ public:
         }
         d.res_pitch = residual && !residual->is_dense() ? residual->channel_pitch : 0;
         const int rc = espdl_hip_conv2d_add(&d, input->data, filter->data, bias ? bias->data : nullptr, shift_dev,
-                                            m_fused_lut ? static_cast<const int8_t *>(m_fused_lut->data) : nullptr,
+                                            lut ? static_cast<const int8_t *>(lut->data) : nullptr,
                                             residual ? static_cast<const int8_t *>(residual->data) : nullptr, output->data,
                                             context->stream);
         if (rc != ESPDL_HIP_OK)

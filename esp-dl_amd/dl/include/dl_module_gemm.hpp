@@ -5,6 +5,7 @@
 // [1, 1, K, N] over N-major memory, and the 1x1 convolution kernel does the work.  Gemm carries a
 // bias and Linear/ReLU; MatMul has neither bias nor (in exported models) an activation other than
 // Linear.  MatMul is implemented for a constant right-hand side of rank 2 (the weight case).
+// A LUT behind one of them runs in the convolution's epilogue, as it does behind a Conv.
 #pragma once
 
 #include <cassert>
@@ -16,7 +17,7 @@ namespace module {
 
 inline void gemm_forward(const char *tag, const std::string &name, quant_type_t quant_type,
                          activation_type_t activation, ModelContext *context, TensorBase *input, TensorBase *filter,
-                         TensorBase *bias, TensorBase *output, DeviceInts &shift_cache)
+                         TensorBase *bias, TensorBase *output, DeviceInts &shift_cache, const TensorBase *lut, int own_exponent)
 {
     if (!input || !filter || !output || !input->on_device() || !filter->on_device() || !output->on_device() ||
         (bias && !bias->on_device())) {
@@ -37,16 +38,17 @@ inline void gemm_forward(const char *tag, const std::string &name, quant_type_t 
     d.group = 1;
     d.activation = activation == ReLU ? ESPDL_HIP_RELU : ESPDL_HIP_LINEAR;
     d.round_mode = context->round_mode == ROUND_MODE_HALF_EVEN ? ESPDL_HIP_ROUND_HALF_EVEN : ESPDL_HIP_ROUND_HALF_UP;
-    const std::vector<int32_t> shifts = conv_shifts(output, input, filter, n);
+    // (with a table the shifts lead to the value that indexes it, not to the one that is stored)
+    const std::vector<int32_t> shifts = conv_shifts(lut ? own_exponent : output->exponent.get(), input, filter, n);
     d.n_shift = (int32_t)shifts.size();
     const int32_t *shift_dev = shift_cache.sync(shifts);
-    const int rc = espdl_hip_conv2d(&d, input->data, filter->data, bias ? bias->data : nullptr, shift_dev, nullptr,
-                                    output->data, context->stream);
+    const int rc = espdl_hip_conv2d(&d, input->data, filter->data, bias ? bias->data : nullptr, shift_dev,
+                                    lut ? static_cast<const int8_t *>(lut->data) : nullptr, output->data, context->stream);
     if (rc != ESPDL_HIP_OK)
         DL_LOGE(tag, "%s: %s", name.c_str(), espdl_hip_last_error());
 }
 
-class Gemm : public Module {
+class Gemm : public Module, public TableEpilogue {
 private:
     activation_type_t activation;
     DeviceInts m_shift;
@@ -81,7 +83,8 @@ public:
         (void)mode;
         TensorBase *bias = m_inputs_index.size() == 3 ? context->get_tensor(m_inputs_index[2]) : nullptr;
         gemm_forward("Gemm", name, quant_type, activation, context, context->get_tensor(m_inputs_index[0]),
-                     context->get_tensor(m_inputs_index[1]), bias, context->get_tensor(m_outputs_index[0]), m_shift);
+                     context->get_tensor(m_inputs_index[1]), bias, context->get_tensor(m_outputs_index[0]), m_shift,
+                     device_lut(context), m_lut_in_exponent);
     }
 
     static Module *deserialize(fbs::FbsModel *fbs_model, std::string node_name)
@@ -109,7 +112,7 @@ public:
     }
 };
 
-class MatMul : public Module {
+class MatMul : public Module, public TableEpilogue {
 private:
     activation_type_t m_activation;
     DeviceInts m_shift;
@@ -179,8 +182,11 @@ public:
             return;
         }
         gemm_forward("MatMul", name, quant_type, m_activation, context, context->get_tensor(m_inputs_index[0]), rhs,
-                     nullptr, context->get_tensor(m_outputs_index[0]), m_shift);
+                     nullptr, context->get_tensor(m_outputs_index[0]), m_shift, device_lut(context), m_lut_in_exponent);
     }
+
+    /// The product with one constant matrix, which has the convolution's epilogue.
+    bool has_constant_rhs() const { return m_inputs_index[1] >= CONTEXT_PARAMETER_OFFSET; }
 
     /// True when the right-hand side is a stack of matrices (an activation), not one [K, N] matrix.
     static bool batched_rhs(const std::vector<int> &b)

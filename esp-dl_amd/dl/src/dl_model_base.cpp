@@ -265,8 +265,8 @@ static dl::module::Add *plain_add(dl::module::Module *m)
     return m && typeid(*m) == typeid(dl::module::Add) ? static_cast<dl::module::Add *>(m) : nullptr;
 }
 
-// Conv -> LUT with no other reader of the conv output: the table moves into the conv's epilogue and
-// the conv writes the LUT's output tensor directly.
+// Conv, Gemm or MatMul by a constant -> LUT with no other reader of the product: the table moves into its epilogue and
+// it writes the LUT's output tensor directly (a recognizer's two dense layers of 20480 rows: 10 us of launches less).
 void Model::fuse_conv_lut()
 {
     std::set<std::string> pinned; // tensors that must keep existing
@@ -275,8 +275,10 @@ void Model::fuse_conv_lut()
     for (auto &n : m_fbs_model->get_test_outputs_name())
         pinned.insert(n);
     for (size_t i = 0; i < m_execution_plan.size(); i++) {
-        auto *conv = dynamic_cast<dl::module::Conv *>(m_execution_plan[i]);
-        if (!conv || conv->quant_type != QUANT_TYPE_SYMM_8BIT || conv->has_fused_lut())
+        dl::module::Module *conv = m_execution_plan[i];
+        auto *epilogue = dynamic_cast<dl::module::TableEpilogue *>(conv);
+        auto *matmul = dynamic_cast<dl::module::MatMul *>(conv);
+        if (!epilogue || conv->quant_type != QUANT_TYPE_SYMM_8BIT || epilogue->has_fused_lut() || (matmul && !matmul->has_constant_rhs()))
             continue;
         const int mid = conv->m_outputs_index[0];
         if (pinned.count(m_model_context->get_tensor_name(mid)))
@@ -294,8 +296,8 @@ void Model::fuse_conv_lut()
         auto *lut = dynamic_cast<dl::module::LUT *>(m_execution_plan[lut_pos]);
         if (!lut || lut->quant_type != QUANT_TYPE_SYMM_8BIT || !lut->get_table() || lut->get_table()->get_size() != 256)
             continue;
-        conv->fuse_lut(lut->release_table(),
-                       m_fbs_model->get_value_info_exponent(m_model_context->get_tensor_name(mid)));
+        epilogue->fuse_lut(lut->release_table(),
+                           m_fbs_model->get_value_info_exponent(m_model_context->get_tensor_name(mid)));
         conv->m_outputs_index[0] = lut->m_outputs_index[0];
         delete lut;
         m_execution_plan.erase(m_execution_plan.begin() + lut_pos);

@@ -203,6 +203,31 @@ def test_config4_yolo_style(oracle, fuse):
     mdl.close()
 
 
+@pytest.mark.parametrize("round_mode", [0, 1], ids=["half_up", "half_even"])
+@pytest.mark.parametrize("rows,k,n,m", [(40, 120, 480, 120), (9, 33, 17, 5), (1, 16, 2100, 64)])
+def test_lut_behind_gemm_and_matmul(oracle, rows, k, n, m, round_mode):
+    """A table behind a Gemm or a MatMul by a constant runs in its epilogue, also where its result has another exponent; one
+    whose input is read twice or is a graph output stays a module."""
+    announce(f"model LUT behind Gemm and MatMul {rows} x {k} -> {n} -> {m} mode {round_mode}")
+    _, zoo, _, _ = _mods()
+    g = zoo.GraphSpec("gemm_lut")
+    b = zoo.Builder(g, 0xE5F7, per_channel=True, w_exp_range=None)
+    x = b.input("input", [1, rows, k], -5)
+    y = b.gemm(x, n, name="fc1")
+    y = b.lut(y, zoo.silu, "Swish", out_exp=g.exponent(y) + 1, name="fc1_act")
+    y = b.gemm(y, m, name="fc2", matmul=True)
+    y = b.lut(y, zoo.silu, "Swish", name="fc2_act")
+    z = b.gemm(y, 24, name="fc3")
+    b.output(b.lut(z, zoo.silu, "Swish", name="fc3_act"))
+    b.output(z)
+    mdl, want, _ = _run_config(g, 3, 21, round_mode=round_mode)
+    for name in g.outputs:
+        np.testing.assert_array_equal(mdl.get_tensor(name), want[name], err_msg=name)
+        assert want[name].min() < want[name].max()
+    assert mdl.module_count() == len(g.nodes) - 2
+    mdl.close()
+
+
 def test_first_block_with_requantized_residual_from_the_graph_input(oracle):
     """The very first modules of the plan form a block whose residual is the graph input behind a
     RequantizeLinear: absorbing that node must not end the scan, so the second block fuses as well."""
