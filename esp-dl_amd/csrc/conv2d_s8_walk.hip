@@ -10,9 +10,9 @@ using namespace walk;
 // Layer -> kernel arguments (without pointers).  False: a layer that no build takes.
 bool walk_layer(const ConvGeom &g, bool residual, WalkArgs *out, WalkLaunch *launch)
 {
-    if ((g.in_c & 15) || (g.out_c & 15) || g.in_c > 256 || (g.in_pitch & 15) || (g.out_pitch & 15) || g.half_even)
+    if ((g.in_c & 3) || g.in_c < 16 || g.out_c < 4 || g.in_c > 256 || (g.in_pitch & 3) || g.half_even)
         return false;
-    if (residual && ((g.res_pitch & 15) || g.res_shift != 0))
+    if (residual && ((g.out_c & 15) || (g.res_pitch & 15) || g.res_shift != 0))
         return false;
     if (g.k_h != g.k_w || (g.k_h != 1 && g.k_h != 3 && g.k_h != 5) || g.stride_h != g.stride_w || g.stride_w > 2 || g.dil_h != 1 ||
         g.dil_w != 1)
@@ -24,6 +24,7 @@ bool walk_layer(const ConvGeom &g, bool residual, WalkArgs *out, WalkLaunch *lau
         return false;
     WalkArgs a = {};
     a.in_bytes = (int)((px - 1) * g.in_pitch + g.in_c);
+    a.last = g.in_c - 16;
     a.w_len = g.k_h * g.k_w * g.in_c;
     a.w_bytes = (int)std::min<long long>((long long)g.out_c * a.w_len, most);
     if ((long long)g.out_c * a.w_len >= most)
@@ -91,7 +92,7 @@ bool walk_layer(const ConvGeom &g, bool residual, WalkArgs *out, WalkLaunch *lau
 
 hipError_t walk_launch(const ConvGeom &g, int nt, WalkArgs &a, const WalkLaunch &l)
 {
-    const int cu = g.in_c / 16;
+    const int cu = (g.in_c + 15) / 16;
     if (g.k_h == 1)
         return launch_1x1(cu, nt, a, l);
     if (g.k_h == 3)
@@ -106,6 +107,8 @@ int walk_tiles(const ConvGeom &g, const WalkArgs &args, WalkLaunch l, float *us)
     *us = 1e30f;
     for (int nt : {1, 2, 3, 4, 8}) {
         if (16 * nt >= 2 * g.out_c && nt > 1) // half of the filters would not exist
+            continue;
+        if (g.out_c < (nt == 8 ? 16 : 4 * nt)) // (a lane's channels)
             continue;
         if (nt == 3 && g.out_c % 48 != 0) // (a lane's twelve channels all exist or none do)
             continue;

@@ -152,7 +152,7 @@ enum DenseRoute { DENSE_WALK, DENSE_STEM, DENSE_NARROW, DENSE_UNITGEMM, DENSE_PW
 //     moves with the share of the last 64 filters in use;
 //   * strided windows of fewer than five reduction steps with many outputs: the direct kernel (320 x 320 x 16 -> 32 at
 //     stride 2, batch 32: 35.5 against 38.3 us).
-// A channel count that is not a multiple of 16 under a window has no other kernel worth taking: 31 x 101 x 61 -> 16,
+// A channel count that is not a multiple of 4 under a window has no other kernel worth taking: 31 x 101 x 61 -> 16,
 // 5 x 5, batch 142: 509 -> 105 us; 45 x 99 x 162 -> 87, 5 x 5 at stride 2, batch 3: 312 -> 40 us.
 DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *filter, const void *residual, const void *out,
                           int cus)
@@ -165,7 +165,10 @@ DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *
         gemm = espdl::conv2d_s8_unitgemm_us(g, in, filter, &tile_steps);
         // (the larger routes below take up to twice the unit kernel's line; a quarter more puts no layer on the walk that
         // is slower there by more than a fifth, and gives up 2 % of what the best choice of 780 random layers would)
-        if (espdl::conv2d_s8_walk_us(g, in, filter, residual, out, cus) < std::min(narrow, 1.25f * gemm))
+        // Channels that are no multiple of 16 cost it a further microsecond of set-up and partial lanes (60 random layers: 5 to
+        // 7 us where the others take 5, but 48 -> 13 us on 202 x 67 x 42 x 40 -> 13, 3 x 3, and 45 -> 13 us on 5 x 5 windows).
+        const float partial = ((g.in_c | g.out_c) & 15) != 0 ? 1.2f : 0.f;
+        if (espdl::conv2d_s8_walk_us(g, in, filter, residual, out, cus) + partial < std::min(narrow, 1.25f * gemm))
             return DENSE_WALK;
     }
     if (espdl::conv2d_s8_stem_supports(g, residual))

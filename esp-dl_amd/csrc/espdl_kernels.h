@@ -52,7 +52,7 @@ hipError_t launch_conv2d_s8_narrow(const ConvGeom &g, const int8_t *in, const in
                                    const int32_t *shift, const int8_t *lut, const int8_t *residual, int8_t *out,
                                    int cu_count, hipStream_t stream);
 // Dense int8 convolution as a walk down the image, filters in registers (conv2d_s8_walk_kernel.h): square 1, 3 and 5 filters
-// at stride 1 and 2, channel counts that are multiples of 16, round half up.  Expected time; 1e30: no build takes it.
+// at stride 1 and 2, 16 and more input channels in multiples of 4, round half up.  Expected time; 1e30: no build takes it.
 float conv2d_s8_walk_us(const ConvGeom &g, const void *in, const void *filter, const void *residual, const void *out,
                         int cu_count);
 hipError_t launch_conv2d_s8_walk(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,
@@ -98,8 +98,8 @@ struct DwExpand {
     int n_shift, relu, c0;
 };
 
-// First layers as a walk down the image (conv2d_s8_walk_stem.hip): window rows of at most 13 bytes, up to four of them, image
-// rows of whole dwords, up to 64 filters.
+// First layers as a walk down the image (conv2d_s8_walk_stem.hip): window rows of at most 12 bytes, up to four of them, image
+// rows of whole 16-byte pieces, 16, 32 or 64 filters.
 bool conv2d_s8_walk_stem_supports(const ConvGeom &g, const void *in, const void *out, const void *residual);
 hipError_t launch_conv2d_s8_walk_stem(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias, const int32_t *shift,
                                       const int8_t *lut, const int8_t *residual, int8_t *out, int cu_count, hipStream_t stream);

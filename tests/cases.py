@@ -217,4 +217,13 @@ WALK_CASES = [
     (20, ("w5_16_16", (47, 65, 16), 16, (5, 5), (1, 1), (1, 1), (2, 2, 2, 2), True, True)),
     (12, ("w5_64_32", (35, 40, 64), 32, (5, 5), (1, 1), (1, 1), (2, 2, 2, 2), True, True)),
     (40, ("w5s2_64_48", (40, 43, 64), 48, (5, 5), (2, 2), (1, 1), (2, 2, 2, 2), True, True)),
+    # channels that are no multiple of 16: last units that overlap, lanes whose channels exist in part
+    (1, ("w1_120_480_partial", (1, 20480, 120), 480, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, True)),
+    (60, ("w1_44_153_partial", (88, 20, 44), 153, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, True)),
+    (100, ("w1_44_36_partial", (40, 83, 44), 36, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), False, True)),
+    (40, ("w3_40_13_partial", (67, 42, 40), 13, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
+    (40, ("w3_200_18_partial", (19, 43, 200), 18, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
+    (40, ("w3_20_32_partial", (60, 51, 20), 32, (3, 3), (1, 1), (1, 1), (0, 2, 0, 1), True, True)),
+    (40, ("w3s2_44_98_partial", (49, 64, 44), 98, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), True, True)),
+    (40, ("w5_56_21_partial", (60, 17, 56), 21, (5, 5), (1, 1), (1, 1), (2, 2, 2, 2), True, True)),
 ]
