@@ -1,4 +1,4 @@
-// Depthwise 3 x 3 int8 convolution (stride 1 or 2 per axis, dilation 1) over any number of channels from 4 on, gfx950.
+// Depthwise 3 x 3 int8 convolution (stride 1 or 2 in x, any in y, dilation 1) over any number of channels from 4 on, gfx950.
 //
 // A thread owns four channels (one dword) of four neighbouring output columns and walks down a strip of output rows.
 // Of every input row it loads the six (stride 2: nine) pixels its columns see, one dword each, and turns them with byte
@@ -17,6 +17,10 @@
 // before, 7 us at the copy rate; strips of few rows and rounds of wavefronts lie between), one image of 56 x 56 x 144 4.8 us
 // (15 us), and 61 channels, which that form does not take, over 256 images of 28 x 28: 16 us (107 us).
 //
+// Strides of 3 and more in y (a recognizer that folds its last rows): three fresh rows per output row.  512 images of
+// 3 x 40 x 120 at stride (3, 1) 6.8 us (9.7 on the kernel without strips, 13.2 inside the recognizer), 256 of 28 x 28 x 192
+// 14.5 (18.4), one of 56 x 56 x 144 4.3 (9.3).
+//
 // Restates depthwise_conv2d_33c1 (esp-dl/dl/base/dl_base_depthwise_conv2d.cpp:9-65) under dwconv_operation_shell's window
 // clipping (esp-dl/dl/base/dl_base.hpp:1852-2102); filter memory is [3][3][c].
 #include "conv_window.h"
@@ -33,7 +37,7 @@ struct StripArgs {
     const int8_t *lut;
     int8_t *out;
     int in_bytes, out_bytes; // below 2^30
-    int in_h, in_w, c, out_h, out_w, pad_top, pad_left, n_shift, relu, half_even;
+    int in_h, in_w, c, out_h, out_w, stride_h, pad_top, pad_left, n_shift, relu, half_even;
     int rows; // output rows per strip
     FastDiv fd_cq, fd_xs, fd_ys;
     unsigned total;   // threads
@@ -81,6 +85,7 @@ __device__ __forceinline__ Row<SW> turn(const int (&px)[3 + 3 * SW])
     return r;
 }
 
+// SH: 1, 2, or 3 for every stride in y that leaves output rows no input row in common.
 template <int SH, int SW>
 __global__ __launch_bounds__(kThreads) void depthwise_s8_strip_kernel(const StripArgs a)
 {
@@ -119,10 +124,10 @@ __global__ __launch_bounds__(kThreads) void depthwise_s8_strip_kernel(const Stri
         for (int i = 0; i < kPx; i++)
             px[i] = __builtin_amdgcn_raw_buffer_load_b32(in, col[i] + row, 0, 0);
     };
-    int iy = oy0 * SH - a.pad_top;
+    int iy = oy0 * (SH == 3 ? a.stride_h : SH) - a.pad_top;
     int px[SH][kPx], first[2][kPx];
     load(iy, first[0]);
-    if constexpr (SH == 1)
+    if constexpr (SH != 2)
         load(iy + 1, first[1]);
 
     // filter rows per channel: bytes kx = 0, 1, 2 and a zero; requantization constants of the four channels
@@ -218,6 +223,23 @@ __global__ __launch_bounds__(kThreads) void depthwise_s8_strip_kernel(const Stri
                 }
             }
         }
+    } else if constexpr (SH == 3) {
+#pragma unroll
+        for (int i = 0; i < kPx; i++) {
+            px[0][i] = first[0][i];
+            px[1][i] = first[1][i];
+        }
+        load(iy + 2, px[2]);
+        for (int left = a.rows; left > 0; left--) {
+            Row<SW> r[3];
+            iy += a.stride_h;
+#pragma unroll
+            for (int ky = 0; ky < 3; ky++) {
+                r[ky] = turn<SW>(px[ky]);
+                load(iy + ky, px[ky]); // (the last three are not used)
+            }
+            finish(r[0], r[1], r[2]);
+        }
     } else {
         Row<SW> r[2];
         load(iy + 1, px[0]);
@@ -266,7 +288,7 @@ int strip_count(long long per_strip, int out_h, int cu_count)
 
 bool depthwise_s8_strip_supports(const ConvGeom &g)
 {
-    return g.k_h == 3 && g.k_w == 3 && g.dil_h == 1 && g.dil_w == 1 && g.in_c >= 4 && (g.stride_h == 1 || g.stride_h == 2) &&
+    return g.k_h == 3 && g.k_w == 3 && g.dil_h == 1 && g.dil_w == 1 && g.in_c >= 4 && g.stride_h < (1 << 20) &&
         (g.stride_w == 1 || g.stride_w == 2) && (long long)g.in_h * g.in_w * g.in_c < (1ll << 30) - 64 &&
         (long long)g.out_h * g.out_w * g.in_c < (1ll << 30) - 64;
 }
@@ -286,6 +308,7 @@ hipError_t launch_depthwise_s8_strip(const ConvGeom &g, const int8_t *in, const 
     a.in_w = g.in_w;
     a.c = g.in_c;
     a.out_h = g.out_h;
+    a.stride_h = g.stride_h;
     a.out_w = g.out_w;
     a.pad_top = g.pad_top;
     a.pad_left = g.pad_left;
@@ -317,7 +340,8 @@ hipError_t launch_depthwise_s8_strip(const ConvGeom &g, const int8_t *in, const 
         const dim3 grid(blocks);
         const auto kernel = g.stride_h == 1
             ? (g.stride_w == 1 ? depthwise_s8_strip_kernel<1, 1> : depthwise_s8_strip_kernel<1, 2>)
-            : (g.stride_w == 1 ? depthwise_s8_strip_kernel<2, 1> : depthwise_s8_strip_kernel<2, 2>);
+            : g.stride_h == 2 ? (g.stride_w == 1 ? depthwise_s8_strip_kernel<2, 1> : depthwise_s8_strip_kernel<2, 2>)
+                              : (g.stride_w == 1 ? depthwise_s8_strip_kernel<3, 1> : depthwise_s8_strip_kernel<3, 2>);
         hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, stream, a);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess)

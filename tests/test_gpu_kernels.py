@@ -893,6 +893,24 @@ def test_depthwise_s8_strips(oracle, case, half_even):
     np.testing.assert_array_equal(got, want)
 
 
+@pytest.mark.parametrize("half_even", [False, True], ids=["half_up", "half_even"])
+@pytest.mark.parametrize("case", [
+    # strides in y that leave output rows no input row in common: one row and many, skipped rows, padding above and below
+    ((20, 3, 40, 120), (3, 1), (1, 1, 1, 1), False), ((9, 61, 13, 18), (3, 2), (1, 1, 1, 1), True),
+    ((2, 50, 9, 7), (5, 1), (0, 2, 1, 0), False), ((1, 2, 5, 4), (4, 2), (1, 1, 0, 1), False), ((300, 31, 10, 33), (4, 1), (2, 0, 1, 1), True)],
+    ids=lambda c: "x".join(map(str, c[0])) + "_s%d%d" % c[1])
+def test_depthwise_s8_strips_without_shared_rows(oracle, case, half_even):
+    shape, stride, pads, with_lut = case
+    announce(f"depthwise_s8 strips {case} half_even={half_even}")
+    rng = np.random.default_rng(0xD8)
+    c = shape[3]
+    x, f = rng_int8(rng, shape), rng_int8(rng, (3, 3, c))
+    lut = np.array([(i * 109 + 37) & 0xFF for i in range(256)], dtype=np.uint8).view(np.int8) if with_lut else None
+    got, want = _run_conv_s8(oracle, x, f, rng.integers(-4096, 4097, size=c).astype(np.int32), rng.integers(5, 12, size=c).astype(np.int32),
+                             (3, 3), stride, (1, 1), pads, not with_lut, depthwise=True, half_even=half_even, lut=lut)
+    np.testing.assert_array_equal(got, want)
+
+
 def _run_conv_s16(oracle, x, f, bias, shift, k, stride, dil, pads, relu, depthwise):
     m = espdl()
     act = m.capi.RELU if relu else m.capi.LINEAR
