@@ -24,7 +24,8 @@
 // and its high bytes the int8 values themselves:  sum_k x w = 65536 sum x8 wh + 256 sum x8 l + 32768 sum x8 (l as above).
 // Two products per step instead of four, no cutting of pixels, half the input, no RequantizeLinear and no int16 copy.
 // They also take an int16 table behind the result (the nearest-entry LUT of esp-dl/dl/base/dl_base_lut.cpp:49-77).
-// 80 x 80 x 64 -> 64, 3 x 3, batch 64: 75 us where the three operators took 135 us.
+// 80 x 80 x 64 -> 64, 3 x 3, batch 64: 75 us where the three operators took 135 us (51 us as a walk down the image, which
+// takes the 3 x 3 layers that fill the device: conv2d_s16_x8_walk.hip).
 //
 // Two kernels, chosen by their measured cost (see the launch).  Against the one-wavefront-per-pixel-tile kernel
 // (conv_s16_mfma.hip) and the 64-bit multiply-add kernel (conv_s16.hip): 80 x 80 x 64 -> 64, 3 x 3, batch 64 98 -> 90 us,
@@ -34,6 +35,7 @@
 //     cut into bytes -> LDS (two buffers), so that a value is cut once per workgroup;
 //   * the narrow one for few outputs: 16 pixels x 16 NT filters per workgroup, its four wavefronts split the reduction
 //     axis and read both operands straight from memory in the matrix instruction's layout; the partial sums meet in LDS.
+#include <algorithm>
 #include <type_traits>
 
 #include "conv_window.h"
@@ -675,6 +677,12 @@ hipError_t launch_units(const ConvGeom &g, S16Args &a, const int64_t *bias, cons
     const float waves = 4e-3f * (float)tiles16 * (float)ny, own = (float)((a.ksteps + 3) / 4), nt = two ? 2.f : 1.f;
     const float narrow_us = aligned ? 3.15f + 0.09f * own + waves * (0.157f + 0.336f * own * nt)
                                     : 3.44f + 0.21f * own + waves * (0.51f + 0.277f * own * nt);
+    if constexpr (X8) { // 3 x 3 layers of whole units as a walk down the image, once their rows fill the device
+        const int8_t *in = static_cast<const int8_t *>(a.win.in);
+        if (1.1f * conv2d_s16_x8_walk_us(g, in, out, a.table_size, cus) < std::min(narrow_us, gemm_us)) // (56 x 56 x 16, batch 64: 11.9 against 10.6 us)
+            return launch_conv2d_s16_x8_walk(g, in, reinterpret_cast<const int16_t *>(a.win.w), bias, shift, a.table, a.table_size, a.table_shift,
+                                             out, cus, stream);
+    }
     if (narrow_us < gemm_us) {
         const dim3 grid(tiles16, ny);
         if (two && aligned)

@@ -220,6 +220,9 @@ bool conv2d_s16_units_supports(const ConvGeom &g);
 hipError_t launch_conv2d_s16_units(const ConvGeom &g, const int16_t *in, const int16_t *filter, const int64_t *bias,
                                    const int32_t *shift, int16_t *out, int cu_count, hipStream_t stream);
 // the same on an int8 input times 256, with an int16 table behind it (table_size 0: none)
+float conv2d_s16_x8_walk_us(const ConvGeom &g, const void *in, const void *out, int table_size, int cu_count); // 1e30: no build
+hipError_t launch_conv2d_s16_x8_walk(const ConvGeom &g, const int8_t *in, const int16_t *filter, const int64_t *bias, const int32_t *shift,
+                                     const int16_t *table, int table_size, int table_shift, int16_t *out, int cu_count, hipStream_t stream);
 bool conv2d_s16_x8_supports(const ConvGeom &g, int table_size);
 hipError_t launch_conv2d_s16_x8(const ConvGeom &g, const int8_t *in, const int16_t *filter, const int64_t *bias,
                                 const int32_t *shift, const int16_t *table, int table_size, int16_t *out, int cu_count,

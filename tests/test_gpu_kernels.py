@@ -855,6 +855,47 @@ def test_conv2d_s16_on_int8(oracle, case, table_size):
     np.testing.assert_array_equal(to_host(got), want)
 
 
+# 3 x 3 layers on an int8 input whose rows fill the device: every count of input units with a build, filter chunks that end in
+# the middle, strips across images, missing, one-sided and wide padding, sums at both ends of their range.
+# (name, (N, H, W, C), OC, pads, relu, half_even, lowest and highest shift, values)
+X8_WALK = [
+    ("16_16", (200, 40, 40, 16), 16, (1, 1, 1, 1), True, False, 24, 28, "random"),
+    ("32_24_nopad", (90, 44, 43, 32), 24, (0, 0, 0, 0), False, False, 20, 28, "random"),
+    ("48_40_tailpad_low", (60, 33, 47, 48), 40, (0, 2, 0, 1), True, False, 9, 20, "random"),
+    ("64_64", (110, 20, 41, 64), 64, (1, 1, 1, 1), True, False, 24, 28, "random"),
+    ("64_72_halfeven", (110, 40, 21, 64), 72, (2, 0, 2, 1), False, True, 24, 28, "random"),
+    ("64_64_general", (150, 31, 17, 64), 64, (1, 1, 1, 1), True, False, -3, 60, "random"),
+    ("64_32_min", (250, 24, 24, 64), 32, (1, 1, 1, 1), False, False, 24, 28, "min"),
+    ("96_20", (30, 40, 40, 96), 20, (1, 1, 1, 1), True, False, 24, 28, "random"),
+    ("128_132_max", (12, 40, 40, 128), 132, (1, 1, 1, 1), False, False, 1, 30, "max"),
+]
+
+
+@pytest.mark.parametrize("table_size", [0, 2049])
+@pytest.mark.parametrize("case", X8_WALK, ids=lambda c: c[0])
+def test_conv2d_s16_on_int8_walk(oracle, case, table_size):
+    announce(f"conv2d_s16_x8 walk {case[0]} table {table_size}")
+    name, (n, h, w, c), oc, pads, relu, half_even, s_lo, s_hi, values = case
+    rng = np.random.default_rng(0x519 + len(name))
+    lo, hi = {"min": (-128, -127), "max": (127, 128), "random": (-128, 128)}[values]
+    x = rng.integers(lo, hi, size=(n, h, w, c)).astype(np.int8)
+    f = rng.integers(256 * lo, 256 * hi, size=(oc, 3, 3, c)).astype(np.int16)
+    bias = rng.integers(-2**40, 2**40, size=oc).astype(np.int64)
+    shift = rng.integers(s_lo, s_hi + 1, size=oc).astype(np.int32)
+    table = rng.integers(-32768, 32768, size=table_size).astype(np.int16) if table_size else None
+    m = espdl()
+    oracle.set_threads(16)
+    got = m.conv2d_s16_x8(to_dev(x), to_dev(f), to_dev(bias), to_dev(shift), (3, 3), (1, 1), (1, 1), pads,
+                          m.capi.RELU if relu else m.capi.LINEAR,
+                          m.capi.ROUND_HALF_EVEN if half_even else m.capi.ROUND_HALF_UP,
+                          None if table is None else to_dev(table))
+    want = oracle.conv2d_s16(x.astype(np.int16) * 256, f, bias, shift, (3, 3), (1, 1), (1, 1), pads,
+                             oracle.RELU if relu else oracle.LINEAR, oracle.ROUND_HALF_EVEN if half_even else oracle.ROUND_HALF_UP)
+    if table is not None:
+        want = oracle.lut_s16(want, table, p4_ties=half_even)
+    np.testing.assert_array_equal(to_host(got), want)
+
+
 @pytest.mark.parametrize("case", DW_TILE_CASES, ids=lambda c: c[0])
 def test_depthwise_s8_tiles(oracle, case):
     announce(f"depthwise_s8 tiles {case[0]}")
