@@ -18,10 +18,9 @@
 // outside the image is replaced by the nearest one inside, which the same window holds (every window of a valid geometry
 // holds at least one): no load is conditional, and a row's loads are requested while the row before it is worked on.
 //
-// Bound by memory, and by how many rows are in flight at once: with conditional loads, none of them early, and four
-// wavefronts per SIMD 256 images of 56 x 56 x 144 took 69 us (3 x 3: 61), 100 of 80 x 80 x 96 44 us (37) and 64 of
-// 20 x 20 x 128 6.9 us; a row ahead 64, 41 and 5.8 us, and with two wavefronts per SIMD, whose longer strips read fewer rows
-// twice, 59 (55), 34 (31) and 6 us: 3.9 TB/s in and out, 4.2 at 3 x 3.
+// Bound by memory, at the number of rows in flight: with conditional loads, none of them early, 256 images of 56 x 56 x 144
+// took 69 us (3 x 3: 61), 100 of 80 x 80 x 96 44 us and 64 of 20 x 20 x 128 6.9 us; a row ahead 63 (61), 42 and 5.8 us,
+// 3.7 TB/s in and out.
 // Input and output may be channel slices of wider tensors (pitches in bytes).  Where the channels are no multiple of
 // the vector, the last one of a pixel reaches back over its neighbour's channels and both write the same bytes: 36 x 8 x
 // 194, 128 images take 13.4 us, one byte per thread took 101 us.
@@ -235,12 +234,12 @@ hipError_t launch_max_pool_s8_window(const void *in, int batch, int h, int w, in
     a.in_pitch = in_pitch;
     a.out_pitch = out_pitch;
     a.xpairs = (out_w + 1) / 2;
-    // Strips per image.  Long strips read each input row once; a strip of `rows` rows reads k - 1 rows more (mostly from
-    // cache, but the horizontal maxima are taken again).  Short strips give small tensors enough wavefronts, and the count
-    // decides how evenly the last round of wavefronts fills the chip, two per SIMD: with four the strips are half as long,
-    // which loses on every layer from 30 MB on (5 to 20 %) and gains on none of fourteen from 50 kB on.
+    // Strips per image.  Long strips read each input row once; a strip of `rows` rows reads k - 1 rows more
+    // (mostly from cache, but the horizontal maxima are taken again).  Short strips give small tensors enough
+    // wavefronts, and the count decides how evenly the last round of wavefronts fills the chip, counted at four
+    // wavefronts per SIMD.
     const long long per_row = (long long)batch * a.xpairs * a.cv;
-    const double capacity = (double)(cu_count > 0 ? cu_count : 256) * 4 * 2;
+    const double capacity = (double)(cu_count > 0 ? cu_count : 256) * 4 * 4;
     int best_strips = 1;
     double best_score = -1.0;
     for (int strips = 1;;) { // of the counts with one strip height only the smallest: 2 sqrt(out_h) of them
