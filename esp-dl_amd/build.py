@@ -27,7 +27,7 @@ HIP_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-fPIC", "-std=c++17", "-Wall", "-
 
 KERNEL_SOURCES = ["conv2d_s8_mfma.hip", "conv2d_s8_mfma_vec16.hip", "conv2d_s8_mfma_point.hip",
                   "conv2d_s8_mfma_gather.hip", "depthwise_s8.hip", "depthwise_s8_mfma.hip", "depthwise_s8_lds.hip", "depthwise_s8_strip.hip",
-                  "conv2d_s8_pwgemm.hip", "conv2d_s8_tiled.hip", "conv2d_s8_walk.hip", "conv2d_s8_walk_stem.hip", "conv2d_s8_walk_1x1.hip", "conv2d_s8_walk_3x3.hip", "conv2d_s8_walk_3x3_s2.hip", "conv2d_s8_walk_5x5.hip", "conv2d_s8_stem.hip", "conv2d_s8_narrow.hip", "conv2d_s8_wide.hip", "mbconv_s8_fused.hip", "mbconv_s8_staged.hip", "mbconv_s8_wave.hip", "mbconv_s8_walk.hip", "mbconv_s8_walk_stem.hip", "mbconv_s8_group.hip", "mbconv_s8_split.hip", "conv_s16.hip", "conv_s16_mfma.hip", "conv_s16_units.hip", "conv2d_s16_x8_walk.hip", "elementwise_s8.hip", "elementwise_s16.hip", "layout_ops.hip", "max_pool_s8.hip", "attention_ops.hip", "attention_s8.hip", "espdl_hip_api.hip"]
+                  "conv2d_s8_pwgemm.hip", "conv2d_s8_tiled.hip", "conv2d_s8_walk.hip", "conv2d_s8_walk_stem.hip", "conv2d_s8_walk_1x1.hip", "conv2d_s8_walk_3x3.hip", "conv2d_s8_walk_3x3_s2.hip", "conv2d_s8_walk_5x5.hip", "conv2d_s8_walk_raw_1x1.hip", "conv2d_s8_walk_raw_3x3.hip", "conv2d_s8_stem.hip", "conv2d_s8_narrow.hip", "conv2d_s8_wide.hip", "mbconv_s8_fused.hip", "mbconv_s8_staged.hip", "mbconv_s8_wave.hip", "mbconv_s8_walk.hip", "mbconv_s8_walk_stem.hip", "mbconv_s8_group.hip", "mbconv_s8_split.hip", "conv_s16.hip", "conv_s16_mfma.hip", "conv_s16_units.hip", "conv2d_s16_x8_walk.hip", "elementwise_s8.hip", "elementwise_s16.hip", "layout_ops.hip", "max_pool_s8.hip", "attention_ops.hip", "attention_s8.hip", "espdl_hip_api.hip"]
 
 
 def _run(cmd):

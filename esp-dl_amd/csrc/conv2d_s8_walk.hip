@@ -10,7 +10,7 @@ using namespace walk;
 // Layer -> kernel arguments (without pointers).  False: a layer that no build takes.
 bool walk_layer(const ConvGeom &g, bool residual, WalkArgs *out, WalkLaunch *launch)
 {
-    if ((g.in_c & 3) || g.in_c < 16 || g.out_c < 4 || g.in_c > 256 || (g.in_pitch & 3) || g.half_even)
+    if (g.in_c < 16 || g.out_c < 4 || g.in_c > 256 || g.half_even)
         return false;
     if (residual && ((g.out_c & 15) || (g.res_pitch & 15) || g.res_shift != 0))
         return false;
@@ -93,6 +93,10 @@ bool walk_layer(const ConvGeom &g, bool residual, WalkArgs *out, WalkLaunch *lau
 hipError_t walk_launch(const ConvGeom &g, int nt, WalkArgs &a, const WalkLaunch &l)
 {
     const int cu = (g.in_c + 15) / 16;
+    if ((g.in_c | g.in_pitch) & 3) // pieces that are no whole dwords of memory
+        return g.k_h == 1                   ? launch_raw_1x1(cu, nt, a, l)
+            : g.k_h == 3 && g.stride_w == 1 ? launch_raw_3x3(cu, nt, a, l)
+                                            : hipErrorInvalidValue;
     if (g.k_h == 1)
         return launch_1x1(cu, nt, a, l);
     if (g.k_h == 3)
@@ -110,7 +114,7 @@ int walk_tiles(const ConvGeom &g, const WalkArgs &args, WalkLaunch l, float *us)
             continue;
         if (g.out_c < (nt == 8 ? 16 : 4 * nt)) // (a lane's channels)
             continue;
-        if (nt == 3 && g.out_c % 48 != 0) // (a lane's twelve channels all exist or none do)
+        if (nt == 3 && g.out_c % 16 == 0 && g.out_c % 48 != 0) // (whole tiles: the other counts leave no lane with a part)
             continue;
         WalkArgs a = args;
         float t = 0.f;

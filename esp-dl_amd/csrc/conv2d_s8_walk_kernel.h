@@ -1,5 +1,5 @@
 // Dense int8 convolution as a walk down the image with the filters in registers: 1 x 1 at stride 1 and 2, 3 x 3 and
-// 5 x 5 at stride 1 and 2, 16 and more input channels in multiples of 4, any filter count from 4 on, round half up.
+// 5 x 5 at stride 1 and 2, 16 and more input channels, any filter count from 4 on, round half up.
 //
 // What it computes is conv2d_11cn / _33cn / _hwcn (esp-dl/dl/base/dl_base_conv2d.cpp:9-163) under
 // conv_operation_shell's window clipping (esp-dl/dl/base/dl_base.hpp:940-1191) with the n_wise epilogue
@@ -21,7 +21,9 @@
 //     regard to image borders: a 20-column image wastes 1 column in 21 and not 12 in 32;
 //   * a pixel whose channels are no multiple of 16 ends with a unit that reaches back over the one before; what both hold
 //     counts in the first and meets zeros in the filters of the second (20480 x 120 -> 480, 1 x 1: 12.8 -> 8.7 us;
-//     202 x 67 x 42 x 40 -> 13, 3 x 3: 48 -> 13 us, where units are loaded tap by tap from memory);
+//     202 x 67 x 42 x 40 -> 13, 3 x 3: 48 -> 13 us, where units are loaded tap by tap from memory).  Where they are no
+//     multiple of 4 either, pieces pass through registers on their way to LDS (120 x 73 x 30 x 77 -> 87, 3 x 3: 88 -> 31 us;
+//     200 x 19 x 23 x 22 -> 33 11.8 -> 10.8 us);
 //   * a workgroup's wavefronts take neighbouring tiles; each workgroup walks the same number of output rows, however
 //     many images those touch.
 // What bounds it: memory where the reduction is short (160 x 160 x 32 -> 64, 1 x 1, batch 64: 4.2 TB/s), else the matrix
@@ -94,6 +96,7 @@ struct WalkShape {
     static constexpr int kSwzSh = CU % 16 == 0 ? 0 : (CU % 8 == 0 ? 1 : 2);
     static constexpr int kSwzMask = CU % 16 == 0 ? 7 : (CU % 8 == 0 ? 3 : (CU % 4 == 0 ? 1 : 0));
     static constexpr int kHalf = (kCols + 1) / 2;
+    static constexpr int kHeld = kAcc == 2 ? 2 : 3; // steps in registers (RAW), a multiple of the accumulators' roles
     static constexpr int kLaneC = NT == 8 ? 16 : 4 * NT; // neighbouring channels that a lane stores at once
     static __device__ __forceinline__ int swz(int ip) { return ((ip >> kSwzSh) & kSwzMask) << 1; }
     static __device__ __forceinline__ int place(int i) { return S == 1 ? i : (i & 1) * kHalf + (i >> 1); }
@@ -129,9 +132,12 @@ __device__ __forceinline__ void wait_copies()
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N < 63 ? N : 63) : "memory"); // (six bits)
 }
 
-template <int KH, int S, int CU, int NT, bool RES>
+// RAW: channels or a pitch that are no multiple of 4.  The copies into LDS take whole dwords only, so the pieces pass through
+// registers: requested kHeld steps before they are written to the ring, that a step before their operands are read.
+template <int KH, int S, int CU, int NT, bool RES, bool RAW = false>
 __global__ __launch_bounds__((64 * WalkShape<KH, S, CU, NT, RES>::W), 2) void conv2d_s8_walk_kernel(const WalkArgs a)
 {
+    static_assert(!(RES && RAW));
     using Shape = WalkShape<KH, S, CU, NT, RES>;
     constexpr int KS = Shape::KS, PT = Shape::PT, AHEAD = Shape::AHEAD, kWaves = Shape::W;
     constexpr int LR = Shape::kRowLoads, RL = Shape::kResLoads, LAG = Shape::kLag, NACC = Shape::kAcc;
@@ -178,10 +184,24 @@ __global__ __launch_bounds__((64 * WalkShape<KH, S, CU, NT, RES>::W), 2) void co
         const __amdgpu_buffer_rsrc_t wr = rsrc_of(a.w, a.w_bytes);
         constexpr int units = KH * CU;
         const unsigned filt0 = (unsigned)reinterpret_cast<uintptr_t>(&filt_l[0][0]);
-        for (int e = wave; e < KH * KS * NT; e += kWaves) { // e = (ky * KS + s) * NT + t
+        const auto unit_at = [&](int e) { // e = (ky * KS + s) * NT + t
             const int t = e % NT, ks = e / NT, ky = ks / KS, u = 4 * (ks - ky * KS) + quad;
             const int oc = filter_of(Shape::channel(t, col)), tap = u / CU;
-            copy_to_lds(filt0 + e * 1024, oc < a.out_c && u < units ? oc * a.w_len + (ky * KH + tap) * (a.last + 16) + min(16 * (u - tap * CU), a.last) : kParked, wr);
+            return oc < a.out_c && u < units ? oc * a.w_len + (ky * KH + tap) * (a.last + 16) + min(16 * (u - tap * CU), a.last) : kParked;
+        };
+        constexpr int total = KH * KS * NT, N = (total + kWaves - 1) / kWaves;
+        if constexpr (RAW) {
+            v4i f[N];
+#pragma unroll
+            for (int i = 0; i < N; i++)
+                f[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, unit_at(min(wave + i * kWaves, total - 1)), 0, 0));
+#pragma unroll
+            for (int i = 0; i < N; i++)
+                if (wave + i * kWaves < total)
+                    filt_l[wave + i * kWaves][lane] = f[i];
+        } else {
+            for (int e = wave; e < total; e += kWaves)
+                copy_to_lds(filt0 + e * 1024, unit_at(e), wr);
         }
     }
 
@@ -229,19 +249,38 @@ __global__ __launch_bounds__((64 * WalkShape<KH, S, CU, NT, RES>::W), 2) void co
         if (units >= 64 || lane < units)
             copy_to_lds(lds, voff, rs);
     };
-    auto feed = [&]() { // one step; past the last one nothing is read (the counts stay the same)
+    constexpr int kHeld = Shape::kHeld;
+    [[maybe_unused]] v4i held[RAW ? kHeld : 1][RAW ? S : 1][RAW ? LR : 1];
+    [[maybe_unused]] unsigned w_slot = 0;
+    auto feed = [&](auto held_tag, bool write) __attribute__((always_inline)) { // one step; past the last one nothing is read (the counts stay the same)
+        [[maybe_unused]] constexpr int H = decltype(held_tag)::value % kHeld;
         if (f_left == 0 && f_r < r_end)
             feed_segment();
         const bool live = f_left > 0;
         const unsigned base = __builtin_amdgcn_readfirstlane(ring0 + f_slot);
+        if constexpr (RAW) {
+            if (write) {
+#pragma unroll
+                for (int s = 0; s < S; s++)
+#pragma unroll
+                    for (int j = 0; j < LR; j++)
+                        if (Shape::kRowUnits - 64 * j >= 64 || lane < Shape::kRowUnits - 64 * j)
+                            *reinterpret_cast<v4i *>(&ring[wave][0][0] + w_slot + s * Shape::kRowUnits * 16 + j * 1024 + 16 * lane) = held[H][s][j];
+                w_slot = w_slot + kSlot == kSlots * kSlot ? 0 : w_slot + kSlot;
+            }
+        }
 #pragma unroll
         for (int s = 0; s < S; s++) {
             const bool ok = live && (unsigned)(f_row + s) < (unsigned)a.in_h;
             const int off = __builtin_amdgcn_readfirstlane(ok ? (f_row + s) * a.in_row : 0);
             const __amdgpu_buffer_rsrc_t rs = rsrc_of(a.in + off, __builtin_amdgcn_readfirstlane(ok ? a.in_bytes - off : 0)); // rows outside the image arrive as zeros
 #pragma unroll
-            for (int j = 0; j < LR; j++)
-                copy(base + s * Shape::kRowUnits * 16 + j * 1024, vin[j], rs, Shape::kRowUnits - 64 * j);
+            for (int j = 0; j < LR; j++) {
+                if constexpr (RAW)
+                    held[H][s][j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rs, vin[j], 0, 0));
+                else
+                    copy(base + s * Shape::kRowUnits * 16 + j * 1024, vin[j], rs, Shape::kRowUnits - 64 * j);
+            }
         }
         if constexpr (RES) {
             const bool ok = live && f_res >= 0;
@@ -267,11 +306,20 @@ __global__ __launch_bounds__((64 * WalkShape<KH, S, CU, NT, RES>::W), 2) void co
         vin[j] = kParked;
     for (int j = 0; j < RL; j++)
         vres[j] = kParked;
+    if constexpr (RAW) { // steps 0 and 1 are in the ring behind it
+        feed(std::integral_constant<int, 0>{}, false);
+        feed(std::integral_constant<int, 1>{}, false);
+        if constexpr (kHeld == 3)
+            feed(std::integral_constant<int, 2>{}, false);
+        feed(std::integral_constant<int, kHeld>{}, true);
+        feed(std::integral_constant<int, kHeld + 1>{}, true);
+    } else {
 #pragma unroll
-    for (int i = 0; i <= AHEAD; i++) {
-        feed();
-        if (i > 0)
-            no_stores();
+        for (int i = 0; i <= AHEAD; i++) {
+            feed(std::integral_constant<int, 0>{}, false);
+            if (i > 0)
+                no_stores();
+        }
     }
 
     // ---- constants of the epilogue; short form when every shift of the chunk lies in 1 .. 31 and the sums fit (as in the
@@ -319,7 +367,8 @@ __global__ __launch_bounds__((64 * WalkShape<KH, S, CU, NT, RES>::W), 2) void co
         const int tap = u / CU, j = u - tap * CU, ip = Shape::place(col * S + tap);
         boff[s] = 16 * (ip * CU + (j ^ Shape::swz(ip)));
     }
-    wait_copies<(AHEAD + 1) * kCopies + AHEAD * kStores>(); // this wavefront's part of the filters
+    if constexpr (!RAW)
+        wait_copies<(AHEAD + 1) * kCopies + AHEAD * kStores>(); // this wavefront's part of the filters
     __syncthreads();
     v4i A[KH][KS][NT]; // operand A of the whole reduction, in registers for the life of the wavefront
 #pragma unroll
@@ -329,17 +378,20 @@ __global__ __launch_bounds__((64 * WalkShape<KH, S, CU, NT, RES>::W), 2) void co
 #pragma unroll
             for (int t = 0; t < NT; t++)
                 A[ky][s][t] = filt_l[(ky * KS + s) * NT + t][lane];
-    if (const int twice = (16 * CU - 16 - a.last) >> 2) // dwords of a last unit that the one before has: counted there
+    if (const int twice = 16 * CU - 16 - a.last) // bytes of a last unit that the one before has: counted there
 #pragma unroll
         for (int s = 0; s < KS; s++)
             if ((4 * s + quad) % CU == CU - 1)
 #pragma unroll
-                for (int ky = 0; ky < KH; ky++)
+                for (int d = 0; d < 4; d++) {
+                    const int cut = twice - 4 * d;
+                    const int mask = cut <= 0 ? -1 : (cut >= 4 ? 0 : (int)(0xffffffffu << (8 * cut)));
 #pragma unroll
-                    for (int t = 0; t < NT; t++)
+                    for (int ky = 0; ky < KH; ky++)
 #pragma unroll
-                        for (int d = 0; d < 4; d++)
-                            A[ky][s][t][d] = d < twice ? 0 : A[ky][s][t][d];
+                        for (int t = 0; t < NT; t++)
+                            A[ky][s][t][d] &= mask;
+                }
     const auto c_of = [&](int t) { return Shape::channel(t, 4 * quad); }; // first of this lane's four channels of a filter tile
     unsigned rsh[NT]; // right shifts of the lane's channels, a byte each
 #pragma unroll
@@ -358,7 +410,8 @@ __global__ __launch_bounds__((64 * WalkShape<KH, S, CU, NT, RES>::W), 2) void co
                 B[row][p][s] = *reinterpret_cast<const v4i *>(my_ring + (b_slot + boff[s]) + (row * Shape::kRowUnits * 16 + p * 256 * CU));
     };
     auto next_b = [&]() { b_slot = b_slot + kSlot == kSlots * kSlot ? 0 : b_slot + kSlot; };
-    wait_copies<AHEAD * (kCopies + kStores)>();
+    if constexpr (!RAW)
+        wait_copies<AHEAD * (kCopies + kStores)>();
 #pragma unroll
     for (int s = 0; s < KS; s++)
         read_b(s);
@@ -410,7 +463,7 @@ __global__ __launch_bounds__((64 * WalkShape<KH, S, CU, NT, RES>::W), 2) void co
 
     auto step = [&](auto tag) {
         constexpr int R = decltype(tag)::value;
-        constexpr int NEW = R % NACC, FIN = (R + NACC - LAG) % NACC;
+        constexpr int NEW = R % NACC, FIN = (R + LAG * (NACC - 1)) % NACC; // (LAG < NACC: LAG roles back)
         if (c_left == 0)
             segment();
         c_left--;
@@ -421,7 +474,8 @@ __global__ __launch_bounds__((64 * WalkShape<KH, S, CU, NT, RES>::W), 2) void co
             for (int p = 0; p < PT; p++)
                 acc[NEW][p][t] = st;
         }
-        wait_copies<(AHEAD - 1) * kCopies + AHEAD * kStores>(); // the next step's input has arrived
+        if constexpr (!RAW)
+            wait_copies<(AHEAD - 1) * kCopies + AHEAD * kStores>(); // the next step's input has arrived
         // residual words of the row that this step finishes sit in this step's slot, one in front of the next one's
         int resw[PT][NT];
         if constexpr (RES) {
@@ -448,7 +502,7 @@ __global__ __launch_bounds__((64 * WalkShape<KH, S, CU, NT, RES>::W), 2) void co
             read_b(s);
         }
         next_b();
-        feed(); // into the slot that this step's operands came from
+        feed(std::integral_constant<int, R + 2>{}, true); // into the slot that this step's operands came from
         if (c_y >= 0) {
             const __amdgpu_buffer_rsrc_t out_rs = rsrc_of(a.out + c_soff, a.out_bytes - c_soff);
 #pragma unroll
@@ -533,16 +587,17 @@ __global__ __launch_bounds__((64 * WalkShape<KH, S, CU, NT, RES>::W), 2) void co
         c_y++;
         c_soff += a.out_row;
     };
-    while (left > 0) { // the accumulators' roles rotate with the steps
+    constexpr int kRoles = RAW ? kHeld : NACC; // the accumulators' roles (and the held steps') rotate with the steps
+    while (left > 0) {
         step(std::integral_constant<int, 0>{});
         if (--left == 0)
             break;
-        if constexpr (NACC > 1) {
+        if constexpr (kRoles > 1) {
             step(std::integral_constant<int, 1>{});
             if (--left == 0)
                 break;
         }
-        if constexpr (NACC > 2) {
+        if constexpr (kRoles > 2) {
             step(std::integral_constant<int, 2>{});
             if (--left == 0)
                 break;
@@ -562,10 +617,12 @@ __global__ __launch_bounds__((64 * WalkShape<KH, S, CU, NT, RES>::W), 2) void co
 
 // Whether a build exists: filters and accumulators fit 256 registers with what else a wavefront holds, and its LDS leaves
 // a compute unit two wavefronts per SIMD.
-template <int KH, int S, int CU, int NT, bool RES>
+template <int KH, int S, int CU, int NT, bool RES, bool RAW>
 constexpr bool walk_fits()
 {
     using Shape = WalkShape<KH, S, CU, NT, RES>;
+    if (RAW && 4 * (KH * Shape::KS * NT + Shape::kAcc * NT * Shape::PT + S * Shape::PT * Shape::KS + Shape::kHeld * S * Shape::kRowLoads) > 204)
+        return false;
     return (NT != 8 || KH == 1) && (!RES || (S == 1 && KH <= 3)) &&
         4 * (KH * Shape::KS * NT + Shape::kAcc * NT * Shape::PT + S * Shape::PT * Shape::KS) <= (RES ? 200 : 208) &&
         (Shape::kTwo || Shape::W == 8 || (S == 2 && Shape::lds(4, 1) <= Shape::kCu));
@@ -630,10 +687,10 @@ float walk_us(const WalkArgs &a, const WalkLaunch &l)
     return us;
 }
 
-template <int KH, int S, int CU, int NT, bool RES>
+template <int KH, int S, int CU, int NT, bool RES, bool RAW = false>
 hipError_t launch_one(WalkArgs &a, const WalkLaunch &l)
 {
-    if constexpr (!walk_fits<KH, S, CU, NT, RES>()) {
+    if constexpr (!walk_fits<KH, S, CU, NT, RES, RAW>()) {
         return hipErrorInvalidValue;
     } else {
         using Shape = WalkShape<KH, S, CU, NT, RES>;
@@ -642,7 +699,7 @@ hipError_t launch_one(WalkArgs &a, const WalkLaunch &l)
             return hipSuccess;
         }
         constexpr int kThreads = 64 * Shape::W;
-        const auto kernel = conv2d_s8_walk_kernel<KH, S, CU, NT, RES>;
+        const auto kernel = conv2d_s8_walk_kernel<KH, S, CU, NT, RES, RAW>;
         const WalkCut c = walk_cut<KH, S, CU, NT, RES>(a, l, resident_workgroups_per_cu(kernel, kThreads, 0));
         if (l.flat) {
             a.in_w = a.out_w = c.width;
@@ -681,11 +738,29 @@ hipError_t launch_cu(int nt, WalkArgs &a, const WalkLaunch &l)
         return launch_nt<KH, S, CU, 1>(a, l);
     }
 }
+template <int KH, int S, int CU>
+hipError_t launch_raw(int nt, WalkArgs &a, const WalkLaunch &l)
+{
+    switch (a.res != nullptr ? 0 : nt) {
+    case 4:
+        return launch_one<KH, S, CU, 4, false, true>(a, l);
+    case 3:
+        return launch_one<KH, S, CU, 3, false, true>(a, l);
+    case 2:
+        return launch_one<KH, S, CU, 2, false, true>(a, l);
+    case 1:
+        return launch_one<KH, S, CU, 1, false, true>(a, l);
+    default:
+        return hipErrorInvalidValue;
+    }
+}
 // Per window entry points, each compiled in its own translation unit; hipErrorInvalidValue: no such build.
 hipError_t launch_1x1(int cu, int nt, WalkArgs &a, const WalkLaunch &l);
 hipError_t launch_3x3(int cu, int nt, WalkArgs &a, const WalkLaunch &l);
 hipError_t launch_3x3_s2(int cu, int nt, WalkArgs &a, const WalkLaunch &l);
 hipError_t launch_5x5(int cu, int stride, int nt, WalkArgs &a, const WalkLaunch &l);
+hipError_t launch_raw_1x1(int cu, int nt, WalkArgs &a, const WalkLaunch &l);
+hipError_t launch_raw_3x3(int cu, int nt, WalkArgs &a, const WalkLaunch &l);
 
 } // namespace walk
 } // namespace espdl

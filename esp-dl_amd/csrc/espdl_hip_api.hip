@@ -152,7 +152,7 @@ enum DenseRoute { DENSE_WALK, DENSE_STEM, DENSE_NARROW, DENSE_UNITGEMM, DENSE_PW
 //     moves with the share of the last 64 filters in use;
 //   * strided windows of fewer than five reduction steps with many outputs: the direct kernel (320 x 320 x 16 -> 32 at
 //     stride 2, batch 32: 35.5 against 38.3 us).
-// A channel count that is not a multiple of 4 under a window has no other kernel worth taking: 31 x 101 x 61 -> 16,
+// A channel count that is not a multiple of 16 under a window has no other kernel worth taking: 31 x 101 x 61 -> 16,
 // 5 x 5, batch 142: 509 -> 105 us; 45 x 99 x 162 -> 87, 5 x 5 at stride 2, batch 3: 312 -> 40 us.
 DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *filter, const void *residual, const void *out,
                           int cus)
@@ -167,8 +167,13 @@ DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *
         // is slower there by more than a fifth, and gives up 2 % of what the best choice of 780 random layers would)
         // Channels that are no multiple of 16 cost it a further microsecond of set-up and partial lanes (60 random layers: 5 to
         // 7 us where the others take 5, but 48 -> 13 us on 202 x 67 x 42 x 40 -> 13, 3 x 3, and 45 -> 13 us on 5 x 5 windows).
+        // No multiple of 4: pieces through registers, which the estimate does not know of: a 3 x 3 layer takes 1.2 to 1.5 times
+        // it, a 1 x 1 one 0.2 to 1.5 us more.  70 random layers gain a fifth in the geometric mean by this line, from 147 ->
+        // 45 us on 163 x 91 x 36 x 137 -> 30, 3 x 3; one is slower (222 x 84 x 18 x 67 -> 177, 1 x 1: 40 -> 44 us).
+        const float walk = espdl::conv2d_s8_walk_us(g, in, filter, residual, out, cus);
         const float partial = ((g.in_c | g.out_c) & 15) != 0 ? 1.2f : 0.f;
-        if (espdl::conv2d_s8_walk_us(g, in, filter, residual, out, cus) + partial < std::min(narrow, 1.25f * gemm))
+        const bool raw = ((g.in_c | g.in_pitch) & 3) != 0;
+        if (raw ? (g.k_h == 1 ? walk + 0.2f : 1.15f * walk + 0.6f) < std::min(narrow, gemm) : walk + partial < std::min(narrow, 1.25f * gemm))
             return DENSE_WALK;
     }
     if (espdl::conv2d_s8_stem_supports(g, residual))

@@ -52,7 +52,7 @@ hipError_t launch_conv2d_s8_narrow(const ConvGeom &g, const int8_t *in, const in
                                    const int32_t *shift, const int8_t *lut, const int8_t *residual, int8_t *out,
                                    int cu_count, hipStream_t stream);
 // Dense int8 convolution as a walk down the image, filters in registers (conv2d_s8_walk_kernel.h): square 1, 3 and 5 filters
-// at stride 1 and 2, 16 and more input channels in multiples of 4, round half up.  Expected time; 1e30: no build takes it.
+// at stride 1 and 2, 16 and more input channels, round half up.  Expected time; 1e30: no build takes it.
 float conv2d_s8_walk_us(const ConvGeom &g, const void *in, const void *filter, const void *residual, const void *out,
                         int cu_count);
 hipError_t launch_conv2d_s8_walk(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,

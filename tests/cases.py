@@ -225,5 +225,11 @@ WALK_CASES = [
     (40, ("w3_200_18_partial", (19, 43, 200), 18, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
     (40, ("w3_20_32_partial", (60, 51, 20), 32, (3, 3), (1, 1), (1, 1), (0, 2, 0, 1), True, True)),
     (40, ("w3s2_44_98_partial", (49, 64, 44), 98, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), True, True)),
+    (200, ("w3_22_33_raw", (19, 23, 22), 33, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
+    (60, ("w3_137_30_raw", (46, 36, 137), 30, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
+    (60, ("w3_50_28_raw_tailpad", (53, 43, 50), 28, (3, 3), (1, 1), (1, 1), (0, 2, 0, 1), False, True)),
+    (29, ("w1_21_24_raw", (90, 102, 21), 24, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, False)),
+    (84, ("w1_246_59_raw", (24, 21, 246), 59, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, True)),
+    (90, ("w1s2_49_185_raw", (31, 78, 49), 185, (1, 1), (2, 2), (1, 1), (0, 0, 0, 0), True, True)),
     (40, ("w5_56_21_partial", (60, 17, 56), 21, (5, 5), (1, 1), (1, 1), (2, 2, 2, 2), True, True)),
 ]
