@@ -23,7 +23,7 @@
 //     counts in the first and meets zeros in the filters of the second (20480 x 120 -> 480, 1 x 1: 12.8 -> 8.7 us;
 //     202 x 67 x 42 x 40 -> 13, 3 x 3: 48 -> 13 us, where units are loaded tap by tap from memory).  Where they are no
 //     multiple of 4 either, pieces pass through registers on their way to LDS (120 x 73 x 30 x 77 -> 87, 3 x 3: 88 -> 31 us;
-//     200 x 19 x 23 x 22 -> 33 11.8 -> 10.8 us);
+//     200 x 19 x 23 x 22 -> 33 11.0 -> 9.9 us);
 //   * a workgroup's wavefronts take neighbouring tiles; each workgroup walks the same number of output rows, however
 //     many images those touch.
 // What bounds it: memory where the reduction is short (160 x 160 x 32 -> 64, 1 x 1, batch 64: 4.2 TB/s), else the matrix

@@ -997,7 +997,7 @@ int mbconv_geometry(const espdl_hip_mbconv_desc *d, espdl::MbconvParams *p)
     return ESPDL_HIP_OK;
 }
 
-// Only the one-wavefront-per-tile kernel takes an expand stage with a window; every other form reads the
+// Only the one-wavefront-per-tile kernel and the stem's walk take an expand stage with a window; every other form reads the
 // block input as the depthwise stage's input grid.
 bool pointwise_expand(const espdl::MbconvParams &p)
 {

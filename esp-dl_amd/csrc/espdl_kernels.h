@@ -144,11 +144,11 @@ struct MbconvParams {
     // the block input, w_expand is [exp_c][ek_h][ek_w][in_c].  For the 1x1 expand img == in and ek == es == 1.
     int img_h, img_w, ek_h, ek_w, es_h, es_w, epad_top, epad_left;
     // The residual operand is requantized by 2^residual_shift (round half up, saturated) before the Add:
-    // a RequantizeLinear between two int8 exponents in front of the Add.  -7 .. 7; only the one-wavefront-per-tile
-    // and the workgroup-per-tile kernels take a value other than 0.
+    // a RequantizeLinear between two int8 exponents in front of the Add.  -7 .. 7; only the walking, the
+    // one-wavefront-per-tile and the workgroup-per-tile kernels take a value other than 0.
     int residual_shift;
     // Clamp of a stage's int8 result before the next stage reads it (a Clip with equal exponents between the
-    // stages); only the guard-free builds of the one-wavefront-per-tile kernel take it.
+    // stages); the walking kernel and the guard-free builds of the one-wavefront-per-tile kernel take it.
     int clip_e, clip_e_lo, clip_e_hi, clip_d, clip_d_lo, clip_d_hi;
 };
 inline bool mbconv_has_clip(const MbconvParams &p)

@@ -12,7 +12,7 @@
 //              first of the first row, the last ones of the last) are gathered byte by byte.
 //
 // Bound by issue: a step (two rows of 30 columns) of two chunks is 36 MFMAs at 16 cycles and 275 vector instructions at
-// 4, which fill 95 % of the cycles between them (180 of the 275 round and pack).  224 x 224 x 3, 3x3 stride 2 to 32, project
+// 4, which one after the other would fill 95 % of the launch's cycles (180 of the 275 round and pack).  224 x 224 x 3, 3x3 stride 2 to 32, project
 // to 16, batch 256: 62 us against 98 us on the tile kernel, which builds operand B from bytes; with 48 expanded channels at
 // 192 x 200, batch 64, 28 against 75.  Three wavefronts per SIMD instead of two: 62 us too, and coarser strips.
 //

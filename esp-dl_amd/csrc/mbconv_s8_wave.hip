@@ -907,7 +907,8 @@ hipError_t launch_one(const WavePlan &plan, hipStream_t stream)
         // a workgroup's set-up weighs on them.  Up to 16 rounds over the device the launch becomes one round of
         // resident workgroups that walk ceil(tiles / resident wavefronts) tiles each (measured on MobileNetV2's
         // stem at batch 256: 14 tiles per wavefront 0.742 ms per step, 7: 0.746, 10: 0.765, 1: 0.777); beyond
-        // that the rounds balance themselves and eight tiles per wavefront amortize the set-up.
+        // that the rounds balance themselves and eight tiles per wavefront amortize the set-up.  (Of more than one round
+        // only the stems come here that the walk down the image does not take.)
         const long long resident = (long long)plan.cus * resident_workgroups_per_cu(kernel, 64 * kWavesPerGroup, plan.lds) *
             kWavesPerGroup;
         const long long per_wave = (a.n_tiles + resident - 1) / resident;
