@@ -37,6 +37,7 @@ bool walk_layer(const ConvGeom &g, bool residual, WalkArgs *out, WalkLaunch *lau
     a.out_c = g.out_c;
     a.n_shift = g.n_shift;
     a.relu = g.relu;
+    a.through = writes_through((long long)po * g.out_c);
     a.mac_bound = (long long)g.k_h * g.k_w * g.in_c * 16384;
     WalkLaunch l = {};
     l.out_bytes = po * g.out_c;

@@ -56,6 +56,7 @@ struct WalkArgs {
     int out_h, out_w, out_pitch, out_row, out_img;
     int res_pitch, res_row, res_img;
     int batch, out_c, n_shift, relu;
+    int through; // results go through the L2 caches as they are stored
     int pad_top, pad_left;
     int w_len;    // bytes of one filter
     int last;     // first channel of a pixel's last unit, which overlaps the one before where channels are no multiple of 16
@@ -122,9 +123,33 @@ __device__ __forceinline__ void copy_to_lds(unsigned lds, int voff, __amdgpu_buf
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 typedef unsigned v3u __attribute__((ext_vector_type(3)));
 typedef unsigned v2u __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void store(const v4u &v, __amdgpu_buffer_rsrc_t rsrc, int voff)
+template <int AUX>
+__device__ __forceinline__ void store_as(const v4u &v, __amdgpu_buffer_rsrc_t rsrc, int voff)
 {
-    __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, voff, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, voff, 0, AUX);
+}
+template <int AUX>
+__device__ __forceinline__ void store_as(const v3u &v, __amdgpu_buffer_rsrc_t rsrc, int voff)
+{
+    __builtin_amdgcn_raw_buffer_store_b96(v, rsrc, voff, 0, AUX);
+}
+template <int AUX>
+__device__ __forceinline__ void store_as(const v2u &v, __amdgpu_buffer_rsrc_t rsrc, int voff)
+{
+    __builtin_amdgcn_raw_buffer_store_b64(v, rsrc, voff, 0, AUX);
+}
+template <int AUX>
+__device__ __forceinline__ void store_as(unsigned v, __amdgpu_buffer_rsrc_t rsrc, int voff)
+{
+    __builtin_amdgcn_raw_buffer_store_b32(v, rsrc, voff, 0, AUX);
+}
+template <typename T>
+__device__ __forceinline__ void store(const T &v, __amdgpu_buffer_rsrc_t rsrc, int voff, int through)
+{
+    if (through != 0) // uniform
+        store_as<kWriteThrough>(v, rsrc, voff);
+    else
+        store_as<0>(v, rsrc, voff);
 }
 template <int N>
 __device__ __forceinline__ void wait_copies()
@@ -171,6 +196,9 @@ __global__ __launch_bounds__((64 * WalkShape<KH, S, CU, NT, RES>::W), 2) void co
     // ---- requests of what the set-up needs: one filter's bias and shift per lane, the workgroup's filters straight into
     // LDS (a quarter per wavefront) in operand-A order
     const bool has_lut = a.lut != nullptr;
+    // (3 x 3 under four filter tiles, 56 x 56 x 64 -> 64 at batch 256: the choice alone costs 33.1 -> 34.9 us, its branches
+    // part the epilogue's instructions from the next step's; beyond 8 units registers spill)
+    const int through = KH == 1 || (KH == 3 && CU <= 8 && NT <= 2) ? a.through : 0;
     constexpr int kMine = (16 * NT + 63) / 64; // filters of a lane
     int my_shift[kMine], my_bias[kMine];
 #pragma unroll
@@ -569,16 +597,16 @@ __global__ __launch_bounds__((64 * WalkShape<KH, S, CU, NT, RES>::W), 2) void co
                     }
                 }
                 if constexpr (NT == 8) {
-                    store(v4u{(unsigned)words[0], (unsigned)words[1], (unsigned)words[2], (unsigned)words[3]}, out_rs, vout[p]);
-                    store(v4u{(unsigned)words[4 % NT], (unsigned)words[5 % NT], (unsigned)words[6 % NT], (unsigned)words[7 % NT]}, out_rs, vout[PT + p]);
+                    store(v4u{(unsigned)words[0], (unsigned)words[1], (unsigned)words[2], (unsigned)words[3]}, out_rs, vout[p], through);
+                    store(v4u{(unsigned)words[4 % NT], (unsigned)words[5 % NT], (unsigned)words[6 % NT], (unsigned)words[7 % NT]}, out_rs, vout[PT + p], through);
                 } else if constexpr (NT == 4) {
-                    store(v4u{(unsigned)words[0], (unsigned)words[1], (unsigned)words[2], (unsigned)words[3]}, out_rs, vout[p]);
+                    store(v4u{(unsigned)words[0], (unsigned)words[1], (unsigned)words[2], (unsigned)words[3]}, out_rs, vout[p], through);
                 } else if constexpr (NT == 3) {
-                    __builtin_amdgcn_raw_buffer_store_b96(v3u{(unsigned)words[0], (unsigned)words[1], (unsigned)words[2]}, out_rs, vout[p], 0, 0);
+                    store(v3u{(unsigned)words[0], (unsigned)words[1], (unsigned)words[2]}, out_rs, vout[p], through);
                 } else if constexpr (NT == 2) {
-                    __builtin_amdgcn_raw_buffer_store_b64(v2u{(unsigned)words[0], (unsigned)words[1]}, out_rs, vout[p], 0, 0);
+                    store(v2u{(unsigned)words[0], (unsigned)words[1]}, out_rs, vout[p], through);
                 } else {
-                    __builtin_amdgcn_raw_buffer_store_b32((unsigned)words[0], out_rs, vout[p], 0, 0);
+                    store((unsigned)words[0], out_rs, vout[p], through);
                 }
             }
         } else {

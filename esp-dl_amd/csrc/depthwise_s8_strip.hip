@@ -39,6 +39,7 @@ struct StripArgs {
     int in_bytes, out_bytes; // below 2^30
     int in_h, in_w, c, out_h, out_w, stride_h, pad_top, pad_left, n_shift, relu, half_even;
     int rows; // output rows per strip
+    int through; // results go through the L2 caches as they are stored
     FastDiv fd_cq, fd_xs, fd_ys;
     unsigned total;   // threads
     unsigned per_xcd; // workgroups of a contiguous part of the rows, 0: parts dealt to the XCDs in turn
@@ -201,7 +202,11 @@ __global__ __launch_bounds__(kThreads) void depthwise_s8_strip_kernel(const Stri
                 const unsigned i = (unsigned)word ^ 0x80808080u;
                 word = pack4_s8(table[i & 255], table[(i >> 8) & 255], table[(i >> 16) & 255], table[i >> 24]);
             }
-            __builtin_amdgcn_raw_buffer_store_b32(word, out, rows_left > 0 && x < cols ? to + x * a.c : window::kParked, 0, 0);
+            const int at = rows_left > 0 && x < cols ? to + x * a.c : window::kParked;
+            if (a.through) // uniform
+                __builtin_amdgcn_raw_buffer_store_b32(word, out, at, 0, kWriteThrough);
+            else
+                __builtin_amdgcn_raw_buffer_store_b32(word, out, at, 0, 0);
         }
         to += out_row;
         rows_left--;
@@ -300,6 +305,7 @@ hipError_t launch_depthwise_s8_strip(const ConvGeom &g, const int8_t *in, const 
     if (g.batch * out_image == 0)
         return hipSuccess;
     StripArgs a;
+    a.through = writes_through((long long)g.batch * g.out_h * g.out_w * g.out_c);
     a.w = filter;
     a.bias = bias;
     a.shift = shift;

@@ -14,6 +14,9 @@ namespace espdl {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
+// Cache policy of a buffer store (sc1): the line goes on to memory at once.  writes_through in espdl_kernels.h says when.
+constexpr int kWriteThrough = 16;
+
 // The same values at any byte address: gfx950 global loads and stores need no alignment, one instruction each.
 typedef v4i v4i_unaligned __attribute__((aligned(1)));
 typedef v2i v2i_unaligned __attribute__((aligned(1)));

@@ -16,6 +16,15 @@ namespace mbstage {
 
 constexpr int kDws = 80; // LDS pixel stride of a 64-channel depthwise result: 64 + 16 (odd number of 16-byte units)
 
+// Four results of a lane (writes_through in espdl_kernels.h); `p` is a multiple of 4 from the tensor's first byte.
+__device__ __forceinline__ void store_word(int8_t *p, int word, int through)
+{
+    if (through != 0) // uniform
+        __hip_atomic_store(reinterpret_cast<int *>(p), word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else
+        *reinterpret_cast<int *>(p) = word;
+}
+
 // 16 bytes at p + off of which the first `nvalid` exist (nvalid a multiple of 4, possibly <= 0); the rest
 // are zeros.  Branch-free: a piece that does not exist is read from offset 0 of `p` instead (always a valid
 // address) and replaced by zero, so that every lane issues the same loads and the wait counters of loads

@@ -65,6 +65,7 @@ constexpr int kRowRounds = 4; // ROWCONV guard-free builds: at most 64 * 4 16-by
 
 struct WaveArgs {
     MbconvParams p;
+    int through; // results go through the L2 caches as they are stored
     int th, tw, ph, pw;
     int n_xpt; // pixel tiles of 16 in the patch
     int tiles_x, tiles_y, n_tiles;
@@ -717,7 +718,7 @@ __global__ __launch_bounds__(64 * kWavesPerGroup, EXACT ? ((PACK > 1 && S == 2) 
                         word = wave_pack<MODE>(acc, cp, floor_p, p.relu_project != 0, HE);
                     }
                     if (live && t < th_real)
-                        *reinterpret_cast<int *>(out_img + (size_t)(off0 + (unsigned)(t * p.out_w * p.out_c + 16 * r))) = word;
+                        store_word(out_img + (size_t)(off0 + (unsigned)(t * p.out_w * p.out_c + 16 * r)), word, a.through);
                 }
             }
         }
@@ -810,6 +811,7 @@ WavePlan wave_plan(const MbconvParams &p)
     const int s = p.stride_h;
     WaveArgs a = {};
     a.p = p;
+    a.through = writes_through((long long)p.batch * p.out_h * p.out_w * p.out_c);
     // columns: the fewest column tiles and the narrowest tile that gives them (less halo to expand), or tiles of
     // 14 columns, the width every guard-free build is made for (patches of 16 columns at depthwise stride 1,
     // where the patch column of a lane does not change from pixel tile to pixel tile, and of 29 at stride 2).
