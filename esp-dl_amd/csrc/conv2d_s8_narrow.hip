@@ -34,6 +34,7 @@ struct NarrowArgs {
     int8_t *out;
     int n_pix, out_c, out_pitch, res_pitch;
     int ksteps, relu, half_even, n_shift, res_shift;
+    int through; // whole dwords that go through the L2 caches as they are stored
 };
 
 template <int NT, bool SPLIT, bool ALIGNED>
@@ -150,7 +151,11 @@ __global__ __launch_bounds__(kThreads) void conv2d_s8_narrow_kernel(const Narrow
             continue;
         int8_t *dst = a.out + (long long)m * a.out_pitch + f;
         if (f + 4 <= a.out_c) {
-            *reinterpret_cast<int_unaligned *>(dst) = pack4_s8(q[0], q[1], q[2], q[3]);
+            const int word = pack4_s8(q[0], q[1], q[2], q[3]);
+            if (a.through) // uniform
+                __hip_atomic_store(reinterpret_cast<int *>(dst), word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            else
+                *reinterpret_cast<int_unaligned *>(dst) = word;
         } else {
 #pragma unroll
             for (int r = 0; r < 4; r++)
@@ -220,6 +225,8 @@ hipError_t launch_conv2d_s8_narrow(const ConvGeom &g, const int8_t *in, const in
                                    int cu_count, hipStream_t stream)
 {
     NarrowArgs a;
+    a.through = ((reinterpret_cast<uintptr_t>(out) | (unsigned)g.out_pitch) & 3) == 0 &&
+        writes_through((long long)g.batch * g.out_h * g.out_w * g.out_c);
     a.win = window_args(g, in, filter);
     a.bias = bias;
     a.shift = shift;

@@ -35,6 +35,7 @@ constexpr int kThreads = 64 * kWaves;
 struct SplitArgs {
     MbconvParams p;
     int8_t *mid; // [batch][out_h][out_w][exp_c]
+    int through; // results go through the L2 caches as they are stored
     int tiles_x, tiles_y, n_tiles;
     int n_groups;    // groups of 64 expanded channels
     int per_wg;      // groups a workgroup walks
@@ -266,8 +267,7 @@ __global__ __launch_bounds__(kThreads, 4) void mbconv_s8_expand_dw_kernel(const 
             const int slot = u >> 2, q = u & 3;
             const int row = slot / T::TWP, x = slot % T::TWP;
             if (row < PT && x < TW && oy0 + row < p.out_h && ox0 + x < p.out_w && 64 * gi + 16 * q < p.exp_c)
-                *reinterpret_cast<v4i *>(dst + (row * p.out_w + x) * p.exp_c + 16 * q) =
-                    *reinterpret_cast<const v4i *>(dw_l + slot * kDws + 16 * q);
+                store16(dst, (row * p.out_w + x) * p.exp_c + 16 * q, *reinterpret_cast<const v4i *>(dw_l + slot * kDws + 16 * q), a.through);
         }
         cur = nxt;
     }
@@ -362,6 +362,7 @@ hipError_t launch_mbconv_s8_expand_dw(const MbconvParams &p, int8_t *mid, int cu
     SplitArgs a = {};
     a.p = p;
     a.mid = mid;
+    a.through = writes_through((long long)p.batch * p.out_h * p.out_w * p.exp_c);
     a.tiles_x = (p.out_w + plan.tw - 1) / plan.tw;
     a.tiles_y = (p.out_h + plan.pt - 1) / plan.pt;
     const long long tiles = (long long)p.batch * a.tiles_x * a.tiles_y;

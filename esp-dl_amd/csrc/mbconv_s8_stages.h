@@ -25,6 +25,17 @@ __device__ __forceinline__ void store_word(int8_t *p, int word, int through)
         *reinterpret_cast<int *>(p) = word;
 }
 
+// The same for 16 aligned bytes off (below 2^31) from `p`, which is the same in every lane.
+__device__ __forceinline__ void store16(int8_t *p, int off, const v4i &v, int through)
+{
+    typedef unsigned v4u __attribute__((ext_vector_type(4)));
+    if (through != 0) // uniform
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, v), __builtin_amdgcn_make_buffer_rsrc(p, (short)0, 0x7fffffff, 0x00020000),
+                                               off, 0, kWriteThrough);
+    else
+        *reinterpret_cast<v4i *>(p + off) = v;
+}
+
 // 16 bytes at p + off of which the first `nvalid` exist (nvalid a multiple of 4, possibly <= 0); the rest
 // are zeros.  Branch-free: a piece that does not exist is read from offset 0 of `p` instead (always a valid
 // address) and replaced by zero, so that every lane issues the same loads and the wait counters of loads
