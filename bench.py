@@ -40,9 +40,9 @@ MACHINE_BALANCE = PEAK_INT8_TOPS * 1e12 / (PEAK_HBM_GBS * 1e9)  # OP per byte
 # 256 MiB element-wise kernel of known traffic gave in the same runs).  Only valid for config 3 at
 # batch 256; any other workload reports null.
 MEASURED_TRAFFIC_BYTES_PER_LAUNCH = {
-    "mbconv_s8_wave": 38688657.0,   # 7 launches (the stem convolution rides in the first block's launch)
-    "mbconv_s8_group": 8491954.0,   # 10 launches
-    "conv2d_s8": 9459605.0,         # head convolution with GlobalAveragePool, classifier
+    "mbconv_s8_wave": 40991182.0,   # 7 launches (the stem convolution rides in the first block's launch)
+    "mbconv_s8_group": 11898185.0,   # 10 launches
+    "conv2d_s8": 9779723.0,         # head convolution with GlobalAveragePool, classifier
     "elementwise_s8": None,
 }
 
