@@ -197,8 +197,9 @@ __global__ __launch_bounds__((64 * WalkShape<KH, S, CU, NT, RES>::W), 2) void co
     // LDS (a quarter per wavefront) in operand-A order
     const bool has_lut = a.lut != nullptr;
     // (3 x 3 under four filter tiles, 56 x 56 x 64 -> 64 at batch 256: the choice alone costs 33.1 -> 34.9 us, its branches
-    // part the epilogue's instructions from the next step's; beyond 8 units registers spill)
-    const int through = KH == 1 || (KH == 3 && CU <= 8 && NT <= 2) ? a.through : 0;
+    // part the epilogue's instructions from the next step's; one unit, 62 x 104 x 16 -> 64 at batch 19: 7.8 -> 7.0 us all the
+    // same; beyond 8 units registers spill)
+    const int through = KH == 1 || (KH == 3 && CU <= 8 && (NT <= 2 || CU == 1)) ? a.through : 0;
     constexpr int kMine = (16 * NT + 63) / 64; // filters of a lane
     int my_shift[kMine], my_bias[kMine];
 #pragma unroll
