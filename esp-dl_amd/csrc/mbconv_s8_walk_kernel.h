@@ -62,6 +62,7 @@ struct MbShape {
     static constexpr int NR = S == 1 ? 2 : 1;     // output rows a step finishes
     static constexpr int kXTile = kUnits * 256;
     static constexpr int kSlot = 2 * ET * kXTile;
+    static constexpr int kOnes = (1 + ET) * 256; // what the start values are multiplied with, behind a wavefront's ring
     static constexpr int kResRow = RT * 256;
     static constexpr int kRes = RES ? NR * kResRow : 16; // the residual operand of the step
     static constexpr int kCopies = 2 * ET;
@@ -69,7 +70,7 @@ struct MbShape {
     static constexpr int kTabs = (2 * CE + RT) * 16 * 8;
     static constexpr long lds(int waves, int ahead)
     {
-        return (4 * CE + G * RT) * 1024l + kTabs + (long)waves * ((ahead + 2) * kSlot + kRes + (1 + ET) * 256) + 512;
+        return (4 * CE + G * RT) * 1024l + kTabs + (long)waves * ((ahead + 2) * kSlot + kOnes + kRes) + 512;
     }
     static constexpr int W = 8; // wavefronts
     static constexpr int AHEAD = lds(W, 2) <= kLdsLimit ? 2 : 1;
@@ -276,10 +277,12 @@ __global__ __launch_bounds__((64 * MbShape<CE, RT, S, RES>::W), 2) void mbconv_s
     constexpr int AHEAD = Shape::AHEAD, kSlot = Shape::kSlot, kSlots = AHEAD + 2, kCopies = Shape::kCopies, kStores = Shape::kStores;
     constexpr int NC = 16 * (2 * CE + RT); // channels of all tables: expand, depthwise, project
     constexpr int TE = 0, TD = 16 * CE, TP = 32 * CE;
-    __shared__ __align__(16) unsigned char ring[kWaves][kSlots][kSlot];
+    // The ring, and behind it [0: zeros, else expand tile][column] what the start values are multiplied with: a lane group reads
+    // one or the other by the same instruction, so both have to be one object to the compiler.
+    constexpr int kOnes = kSlots * kSlot;
+    __shared__ __align__(16) unsigned char ring[kWaves][kOnes + Shape::kOnes];
     __shared__ __align__(16) unsigned char res_l[kWaves][Shape::kRes];
     __shared__ v4i we_l[CE][64], wd_l[CE][3][64], wp_l[G * RT][64];
-    __shared__ v4i one_l[kWaves][1 + ET][16]; // [0: zeros, else expand tile][column]: what the start values are multiplied with
     __shared__ __align__(16) int start_l[NC], shift_l[NC];
 
     const MbconvParams &p = a.p;
@@ -291,7 +294,7 @@ __global__ __launch_bounds__((64 * MbShape<CE, RT, S, RES>::W), 2) void mbconv_s
     const int c0 = p.in_c, units = (c0 + 15) >> 4;
 
     // ---- copies, AHEAD steps in front of the computation
-    const unsigned ring0 = (unsigned)reinterpret_cast<uintptr_t>(&ring[wave][0][0]);
+    const unsigned ring0 = (unsigned)reinterpret_cast<uintptr_t>(&ring[wave][0]);
     int vin[ET];
     int f_r = r_begin, f_row = 0, f_left = 0;
     unsigned f_slot = 0;
@@ -379,7 +382,7 @@ __global__ __launch_bounds__((64 * MbShape<CE, RT, S, RES>::W), 2) void mbconv_s
     if (fast && tid < TD)
         we_l[tid >> 4][48 + (tid & 15)] = start_digits(tab.start);
     if (lane < 16)
-        one_l[wave][0][lane] = v4i{0, 0, 0, 0};
+        *reinterpret_cast<v4i *>(&ring[wave][kOnes + 16 * lane]) = v4i{0, 0, 0, 0};
     __syncthreads();
     const Band band_e = make_band(range_e, is_high), band_d = make_band(range_d, is_high), band_p = make_band(project_range(p), is_high);
 
@@ -388,11 +391,11 @@ __global__ __launch_bounds__((64 * MbShape<CE, RT, S, RES>::W), 2) void mbconv_s
 
     v4i X[2][ET];
     unsigned b_slot = 0;
-    const unsigned char *my_ring = &ring[wave][0][0];
+    const unsigned char *my_ring = &ring[wave][0];
     // lane groups past the last unit meet zero filters, or (folded start values, last group) the constant of the pixel
     const bool constant = fast && quad == 3;
     const int xoff = min(quad, kUnits - 1) * 256 + col * 16;
-    const int one_off = (int)(reinterpret_cast<const unsigned char *>(&one_l[wave][0][0]) - my_ring) + col * 16;
+    const int one_off = kOnes + col * 16;
     auto read_x = [&](int row) { // row: first input row of the step
 #pragma unroll
         for (int s = 0; s < 2; s++) {
@@ -425,7 +428,7 @@ __global__ __launch_bounds__((64 * MbShape<CE, RT, S, RES>::W), 2) void mbconv_s
             int n, x;
             emask[e] = in_pixel(v0, lane_now & 15, e, n, x) ? -1 : 0;
             if (lane < 16)
-                one_l[wave][1 + e][lane] = start_factors(emask[e]);
+                *reinterpret_cast<v4i *>(&ring[wave][kOnes + 256 * (1 + e) + 16 * lane]) = start_factors(emask[e]);
         }
         const int o = (lane_now & 15) - Shape::kFirst, v = v0 + max(o, 0);
         const int n = (int)fastdiv((unsigned)v, a.fd_po);

@@ -39,9 +39,11 @@ __global__ __launch_bounds__(64 * kStemWaves, kStemWaves / 4) void mbconv_s8_wal
     constexpr int kXTile = 768, kSlot = 4 * kXTile, kCopies = 4, kStores = 4;
     constexpr int NC = 16 * (2 * CE + RT), TE = 0, TD = 16 * CE, TP = 32 * CE;
     static_assert(CE <= 4);
-    __shared__ __align__(16) unsigned char ring[kWaves][kSlots][kSlot];
+    // The ring, and behind it [0: zeros, 1 / 2: even / odd tile][column] what the start values are multiplied with: a lane group
+    // reads one or the other by the same instruction, so both have to be one object to the compiler.
+    constexpr int kOnes = kSlots * kSlot;
+    __shared__ __align__(16) unsigned char ring[kWaves][kOnes + 3 * 256];
     __shared__ v4i we_l[CE][2][64], wd_l[CE][3][64], wp_l[RT][64];
-    __shared__ v4i one_l[kWaves][3][16]; // [0: zeros, 1 / 2: even / odd tile][column]: what the start values are multiplied with
     __shared__ __align__(16) int start_l[NC], shift_l[NC];
 
     const MbconvParams &p = a.p;
@@ -61,7 +63,7 @@ __global__ __launch_bounds__(64 * kStemWaves, kStemWaves / 4) void mbconv_s8_wal
     };
 
     // ---- copies, AHEAD steps in front of the computation
-    const unsigned ring0 = (unsigned)reinterpret_cast<uintptr_t>(&ring[wave][0][0]);
+    const unsigned ring0 = (unsigned)reinterpret_cast<uintptr_t>(&ring[wave][0]);
     int vin[2] = {kParked, kParked};
     int f_r = r_begin, f_row = 0, f_left = 0;
     unsigned f_slot = 0;
@@ -154,16 +156,16 @@ __global__ __launch_bounds__(64 * kStemWaves, kStemWaves / 4) void mbconv_s8_wal
     if (fast && tid < TD)
         we_l[tid >> 4][0][48 + (tid & 15)] = we_l[tid >> 4][1][48 + (tid & 15)] = start_digits(tab.start);
     if (lane < 16)
-        one_l[wave][0][lane] = v4i{0, 0, 0, 0};
+        *reinterpret_cast<v4i *>(&ring[wave][kOnes + 16 * lane]) = v4i{0, 0, 0, 0};
     __syncthreads();
     const Band band_e = make_band(range_e, tab.high), band_d = make_band(range_d, tab.high), band_p = make_band(project_range(p), tab.high);
 
     const int c_of = 4 * quad;
     unsigned b_slot = 0;
-    const unsigned char *my_ring = &ring[wave][0][0];
+    const unsigned char *my_ring = &ring[wave][0];
     const bool constant = fast && quad == 3;
     const int xoff = min(quad, 2) * 256 + col * 16;
-    const int one_off = (int)(reinterpret_cast<const unsigned char *>(&one_l[wave][0][0]) - my_ring) + col * 16;
+    const int one_off = kOnes + col * 16;
 
     int c_r = r_begin, c_left = 0, c_row = 0, c_k = 0, c_v0 = 0; // c_row: first expanded row of the step; c_k: output row it finishes first
     int vout[2] = {kParked, kParked};
@@ -189,7 +191,7 @@ __global__ __launch_bounds__(64 * kStemWaves, kStemWaves / 4) void mbconv_s8_wal
             const bool ok = mid_pixel(c_v0, m, e, n, x);
             emask[e] = ok ? -1 : 0;
             if (lane < 16)
-                one_l[wave][1 + e][lane] = start_factors(emask[e]);
+                *reinterpret_cast<v4i *>(&ring[wave][kOnes + 256 * (1 + e) + 16 * lane]) = start_factors(emask[e]);
             const int x0 = x * p.es_w - p.epad_left;               // image column of the filter's first
             const int lo = max(0, -x0) * p.in_c + skew_of(e);       // bytes [lo, hi) of the copied ones lie inside
             const int hi = (p.img_w - x0) * p.in_c + skew_of(e);
