@@ -295,6 +295,11 @@ __global__ __launch_bounds__((64 * WalkShape<KH, S, CU, NT, RES>::W), 2) void co
                     for (int j = 0; j < LR; j++)
                         if (Shape::kRowUnits - 64 * j >= 64 || lane < Shape::kRowUnits - 64 * j)
                             *reinterpret_cast<v4i *>(&ring[wave][0][0] + w_slot + s * Shape::kRowUnits * 16 + j * 1024 + 16 * lane) = held[H][s][j];
+                // Other lanes read these pieces in the next step, and what lay in the slot was read two steps ago at least: one
+                // fence a step orders both.  LDS executes a wavefront's instructions in order, so nothing is waited for.
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
                 w_slot = w_slot + kSlot == kSlots * kSlot ? 0 : w_slot + kSlot;
             }
         }
@@ -531,7 +536,9 @@ __global__ __launch_bounds__((64 * WalkShape<KH, S, CU, NT, RES>::W), 2) void co
             read_b(s);
         }
         next_b();
-        feed(std::integral_constant<int, R + 2>{}, true); // into the slot that this step's operands came from
+        // into the slot of the step before (the ring has AHEAD + 2: this step's residual words still lie in its own; RAW: the pieces
+        // of the step after the next, requested kHeld steps ago)
+        feed(std::integral_constant<int, R + 2>{}, true);
         if (c_y >= 0) {
             const __amdgpu_buffer_rsrc_t out_rs = rsrc_of(a.out + c_soff, a.out_bytes - c_soff);
 #pragma unroll
