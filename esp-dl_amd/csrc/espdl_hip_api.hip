@@ -1309,6 +1309,11 @@ int64_t espdl_hip_mbconv_s8_workspace(const espdl_hip_mbconv_desc *desc)
     static const int8_t *const aligned = reinterpret_cast<const int8_t *>(uintptr_t(256));
     p.in = aligned;
     p.w_expand = aligned;
+    // The descriptor does not say whether a residual operand follows.  A block that can have one counts as if it did: the walk
+    // is slower with it, or has no build, and the tile kernels take the same time (56 x 56 x 24 -> 144 -> 24 with an Add, batch 7:
+    // 10.9 us as two launches, 12.4 as the walk, which without the operand is expected to take less; half even, batch 8: 12.1, 15.3).
+    if (p.in_c == p.out_c && p.in_h == p.out_h && p.in_w == p.out_w)
+        p.residual = aligned;
     const espdl::ConvGeom g = project_geometry(p);
     if (!espdl::mbconv_s8_split_supports(p) || !espdl::conv2d_s8_units_support(g))
         return 0;

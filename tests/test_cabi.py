@@ -64,3 +64,18 @@ def test_conv2d_refuses_other_types_than_int8_and_int16():
     for dtype in (torch.uint8, torch.bool, torch.float16, torch.bfloat16, torch.int32, torch.float32):
         with pytest.raises(m.EspdlHipError, match="int8 or int16"):
             m.conv2d(torch.zeros((1, 4, 4, 16), dtype=dtype), f, None, shift, (1, 1), stream=0)
+
+
+def test_two_launches_are_weighed_against_the_launch_that_a_block_with_an_add_takes():
+    """The descriptor of a block has no residual operand, the launch has: where input and output have one shape the choice
+    between one and two launches has to count the kernel that takes the operand.  Each of these takes 14 to 65 % longer as one
+    launch (no GPU needed: the answer follows from estimates)."""
+    import ctypes as C
+    import importlib
+    m = importlib.import_module("esp-dl_amd")
+    for batch, hw, cin, ce, half_even in ((7, 56, 24, 144, 0), (8, 56, 24, 144, 1), (28, 28, 32, 96, 1), (14, 40, 32, 144, 1), (10, 28, 48, 144, 0)):
+        d = m.capi.MbconvDesc(batch, hw, hw, cin, ce, cin, 1, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 0, half_even, ce, ce, cin)
+        assert m.lib().espdl_hip_mbconv_s8_workspace(C.byref(d)) == batch * hw * hw * ce, (batch, hw, cin, ce, half_even)
+    # a depthwise stride takes the operand away, and with it the reason
+    d = m.capi.MbconvDesc(24, 56, 56, 24, 144, 24, 1, 3, 3, 2, 2, 1, 1, 1, 1, 1, 1, 1, 1, 0, 0, 144, 144, 24)
+    assert m.lib().espdl_hip_mbconv_s8_workspace(C.byref(d)) == 0
