@@ -40,7 +40,6 @@ constexpr int kMaxT = 7; // project pixel tiles per wavefront and row tile
 
 struct GroupArgs {
     MbconvParams p;
-    int through; // results go through the L2 caches as they are stored
     int th, tw, ph, pw;
     int twp;   // pixel slots per output row in the shared depthwise tile: 8 or 16
     int n_xpt; // pixel tiles of 16 in the patch
@@ -372,7 +371,7 @@ __global__ __launch_bounds__(kGroupThreads, (KSE == 1 && EXACT) ? 4 : 2) void mb
                         word = wave_pack<MODE>(acc, cp, floor_p, p.relu_project != 0, HE);
                     }
                     if (live[i])
-                        store_word(out_img + (size_t)off[i], word, a.through);
+                        store_word<true>(out_img + (size_t)off[i], word);
                 }
             };
             auto with_mode = [&](auto mode_tag) {
@@ -449,7 +448,6 @@ GroupPlan group_plan(const MbconvParams &p)
             continue; // nothing to round: the natural plan below is the same or better
         GroupArgs a = {};
         a.p = p;
-        a.through = writes_through((long long)p.batch * p.out_h * p.out_w * p.out_c);
         a.tw = rounded ? tw_class : p.out_w;
         a.pw = (a.tw - 1) * s + 3;
         a.twp = a.tw <= 8 ? 8 : 16;
