@@ -82,6 +82,8 @@ def lib():
         L.espdl_hip_conv2d.argtypes = [dp, vp, vp, vp, vp, vp, vp, vp]
         L.espdl_hip_conv2d_add.argtypes = [dp, vp, vp, vp, vp, vp, vp, vp, vp]
         L.espdl_hip_conv2d_add.restype = ctypes.c_int
+        L.espdl_hip_conv2d_s8_kernel.argtypes = [dp, vp, vp, vp, vp, vp]
+        L.espdl_hip_conv2d_s8_kernel.restype = ctypes.c_char_p
         L.espdl_hip_conv2d_gap_s8.argtypes = [dp, vp, vp, vp, vp, i32, i32, vp, vp]
         L.espdl_hip_conv2d_gap_s8.restype = ctypes.c_int
         L.espdl_hip_conv2d_gap_s8_supported.argtypes = [dp]
@@ -147,6 +149,8 @@ def lib():
         L.espdl_hip_mbconv_s8_staged.argtypes = L.espdl_hip_mbconv_s8.argtypes
         L.espdl_hip_mbconv_s8_ws.argtypes = [mp, vp, ctypes.POINTER(MbconvWeights), vp, vp, vp, vp]
         L.espdl_hip_mbconv_s8_ws.restype = ctypes.c_int
+        L.espdl_hip_mbconv_s8_kernel.argtypes = [mp, vp, ctypes.POINTER(MbconvWeights), vp, vp]
+        L.espdl_hip_mbconv_s8_kernel.restype = ctypes.c_char_p
         L.espdl_hip_mbconv_s8_workspace.argtypes = [mp]
         L.espdl_hip_mbconv_s8_workspace.restype = i64
         L.espdl_hip_mbconv_s8_preferred.argtypes = [mp]
@@ -246,6 +250,15 @@ def conv2d(x, filt, bias, shift, k, stride=(1, 1), dilation=(1, 1), pads=(0, 0, 
     return out
 
 
+def conv2d_s8_kernel(x, filt, shift, k, stride=(1, 1), dilation=(1, 1), pads=(0, 0, 0, 0), activation=LINEAR,
+                     round_mode=ROUND_HALF_UP, lut=None, out=None, residual=None):
+    """Name of the kernel that conv2d takes for these tensors of a dense int8 layer (out None: a dense output)."""
+    desc, _ = _conv_plan(x.shape, filt.numel(), tuple(k), tuple(stride), tuple(dilation), tuple(pads), False, activation, round_mode,
+                         shift.numel(), S8, _channel_pitch(x), _channel_pitch(out), _channel_pitch(residual))
+    name = lib().espdl_hip_conv2d_s8_kernel(desc, _p(x), _p(filt), _p(lut), _p(residual), 256 if out is None else _p(out))
+    return None if name is None else name.decode()
+
+
 def conv2d_s16_x8(x, filt, bias, shift, k, stride=(1, 1), dilation=(1, 1), pads=(0, 0, 0, 0), activation=LINEAR,
                   round_mode=ROUND_HALF_UP, table=None, stream=None):
     """int16 convolution of 256 * x for an int8 x, with an int16 table behind it (espdl_hip_conv2d_s16_x8)."""
@@ -295,6 +308,31 @@ def mbconv_s8(x, expand, dw, project, k, stride=(1, 1), dilation=(1, 1), pads=(0
     expand_conv = (kernel, stride, pads) makes the expand stage a dense convolution with a window over the
     block input (filter [E][kH][kW][C]); the depthwise stage then works on that convolution's output."""
     import torch
+    desc, wts, shape = _mbconv_plan(x, expand, dw, project, k, stride, dilation, pads, relus, round_mode, expand_conv,
+                                    residual_shift, clip_expand, clip_dw)
+    if out is None:
+        out = torch.empty(shape, dtype=torch.int8, device=x.device)
+    if workspace is not None:
+        _check(lib().espdl_hip_mbconv_s8_ws(ctypes.byref(desc), _p(x), ctypes.byref(wts), _p(residual), _p(workspace), _p(out),
+                                            _stream(stream)))
+        return out
+    fn = lib().espdl_hip_mbconv_s8_staged if staged else lib().espdl_hip_mbconv_s8
+    _check(fn(ctypes.byref(desc), _p(x), ctypes.byref(wts), _p(residual), _p(out), _stream(stream)))
+    return out
+
+
+def mbconv_s8_kernel(x, expand, dw, project, k, stride=(1, 1), dilation=(1, 1), pads=(0, 0, 0, 0), relus=(True, True, False),
+                     residual=None, round_mode=ROUND_HALF_UP, expand_conv=None, residual_shift=0, clip_expand=None,
+                     clip_dw=None):
+    """Name of the kernel that mbconv_s8 takes for these tensors as a single launch."""
+    desc, wts, _ = _mbconv_plan(x, expand, dw, project, k, stride, dilation, pads, relus, round_mode, expand_conv,
+                                residual_shift, clip_expand, clip_dw)
+    name = lib().espdl_hip_mbconv_s8_kernel(ctypes.byref(desc), _p(x), ctypes.byref(wts), _p(residual), 256)
+    return None if name is None else name.decode()
+
+
+def _mbconv_plan(x, expand, dw, project, k, stride, dilation, pads, relus, round_mode, expand_conv, residual_shift,
+                 clip_expand, clip_dw):
     n, h, w, c = x.shape
     wd, bd, sd = dw
     wp, bp, sp = project
@@ -316,16 +354,8 @@ def mbconv_s8(x, expand, dw, project, k, stride=(1, 1), dilation=(1, 1), pads=(0
         desc.clip_dw, desc.clip_dw_min, desc.clip_dw_max = 1, clip_dw[0], clip_dw[1]
     oh, ow = ctypes.c_int32(), ctypes.c_int32()
     _check(lib().espdl_hip_mbconv_out_shape(ctypes.byref(desc), ctypes.byref(oh), ctypes.byref(ow)))
-    if out is None:
-        out = torch.empty((n, oh.value, ow.value, out_c), dtype=torch.int8, device=x.device)
     wts = MbconvWeights(_p(we), _p(be), _p(se), _p(wd), _p(bd), _p(sd), _p(wp), _p(bp), _p(sp))
-    if workspace is not None:
-        _check(lib().espdl_hip_mbconv_s8_ws(ctypes.byref(desc), _p(x), ctypes.byref(wts), _p(residual), _p(workspace), _p(out),
-                                            _stream(stream)))
-        return out
-    fn = lib().espdl_hip_mbconv_s8_staged if staged else lib().espdl_hip_mbconv_s8
-    _check(fn(ctypes.byref(desc), _p(x), ctypes.byref(wts), _p(residual), _p(out), _stream(stream)))
-    return out
+    return desc, wts, (n, oh.value, ow.value, out_c)
 
 
 def lut_s8(x, table, out=None, stream=None):

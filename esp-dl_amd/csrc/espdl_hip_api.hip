@@ -134,7 +134,9 @@ int images_per_launch(const espdl::ConvGeom &g, bool (*supports)(const espdl::Co
     return supports(part) ? part.batch : 0;
 }
 
-enum DenseRoute { DENSE_WALK, DENSE_STEM, DENSE_NARROW, DENSE_UNITGEMM, DENSE_PWGEMM, DENSE_TILED, DENSE_DIRECT };
+enum DenseRoute { DENSE_WALK, DENSE_STEM, DENSE_NARROW, DENSE_UNITGEMM, DENSE_PWGEMM, DENSE_TILED, DENSE_DIRECT, DENSE_WALK_STEM, DENSE_WIDE };
+const char *const kDenseNames[] = {"conv2d_s8_walk", "conv2d_s8_stem", "conv2d_s8_narrow", "conv2d_s8_unitgemm", "conv2d_s8_pwgemm",
+                                   "conv2d_s8_tiled", "conv2d_s8", "conv2d_s8_walk_stem", "conv2d_s8_wide"};
 
 // Kernel of a dense int8 convolution.  The two kernels that read windows as 16-channel units take any layer; their
 // times, measured over 128 layers of 1 to 600 K output pixels, are straight lines in their work (within 15 %), so the
@@ -194,6 +196,17 @@ DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *
     if (units && (tile_steps <= unit_limit || (strided && g.k_h * g.k_w * g.in_c > 256) || g.k_h * g.k_w * g.in_c >= 2048))
         return few;
     return espdl::conv2d_s8_tiled_supports(g, in, filter, cus) ? DENSE_TILED : DENSE_DIRECT;
+}
+
+// The same with the kernels that take all layers that they apply to: the classifier's, and a walk of the first-layer kernel's
+// layers (one 416 x 416 image 5.1 us either way, 64 of 640 x 640 50 against 78 us).
+DenseRoute dense_s8_kernel(const espdl::ConvGeom &g, const void *in, const void *filter, const int8_t *lut, const int8_t *residual,
+                           const void *out, int cus)
+{
+    if (espdl::conv2d_s8_wide_supports(g, lut, residual))
+        return DENSE_WIDE;
+    const DenseRoute route = dense_s8_route(g, in, filter, residual, out, cus);
+    return route == DENSE_STEM && espdl::conv2d_s8_walk_stem_supports(g, in, out, residual) ? DENSE_WALK_STEM : route;
 }
 
 } // namespace
@@ -271,11 +284,13 @@ int espdl_hip_conv2d_add(const espdl_hip_conv_desc *desc, const void *in, const 
             return device_status(espdl::launch_depthwise_s8(g, i8, f8, b32, shift, lut, o8, s), "depthwise_s8");
         }
         const int cus = cu_count_cached();
-        const auto run = [&](auto launch, const char *name) {
+        const DenseRoute route = dense_s8_kernel(g, in, filter, lut, residual, out, cus);
+        const char *const name = kDenseNames[route];
+        const auto run = [&](auto launch) {
             return device_status(launch(g, i8, f8, b32, shift, lut, residual, o8, cus, s), name);
         };
         // in parts of the batch where the input is larger than a launch's offsets reach
-        const auto run_units = [&](auto launch, const char *name) {
+        const auto run_units = [&](auto launch) {
             espdl::ConvGeom part = g;
             const int most = images_per_launch(g, espdl::conv2d_s8_units_support);
             const size_t in_img = (size_t)g.in_h * g.in_w * g.in_pitch, out_pix = (size_t)g.out_h * g.out_w;
@@ -289,29 +304,27 @@ int espdl_hip_conv2d_add(const espdl_hip_conv_desc *desc, const void *in, const 
             }
             return (int)ESPDL_HIP_OK;
         };
-        if (espdl::conv2d_s8_wide_supports(g, lut, residual))
-            return device_status(espdl::launch_conv2d_s8_wide(g, i8, f8, b32, shift, o8, cus, s), "conv2d_s8_wide");
-        switch (dense_s8_route(g, in, filter, residual, out, cus)) {
+        switch (route) {
+        case DENSE_WIDE:
+            return device_status(espdl::launch_conv2d_s8_wide(g, i8, f8, b32, shift, o8, cus, s), name);
         case DENSE_WALK:
-            return run(espdl::launch_conv2d_s8_walk, "conv2d_s8_walk");
+            return run(espdl::launch_conv2d_s8_walk);
+        case DENSE_WALK_STEM:
+            return run(espdl::launch_conv2d_s8_walk_stem);
         case DENSE_STEM:
-            // (the walk is the faster one wherever it applies: one 416 x 416 image 5.1 us either way, 64 of 640 x 640 50
-            // against 78 us)
-            if (espdl::conv2d_s8_walk_stem_supports(g, in, out, residual))
-                return run(espdl::launch_conv2d_s8_walk_stem, "conv2d_s8_walk_stem");
-            return device_status(espdl::launch_conv2d_s8_stem(g, i8, f8, b32, shift, lut, o8, cus, s), "conv2d_s8_stem");
+            return device_status(espdl::launch_conv2d_s8_stem(g, i8, f8, b32, shift, lut, o8, cus, s), name);
         case DENSE_NARROW:
-            return run_units(espdl::launch_conv2d_s8_narrow, "conv2d_s8_narrow");
+            return run_units(espdl::launch_conv2d_s8_narrow);
         case DENSE_UNITGEMM:
-            return run_units(espdl::launch_conv2d_s8_unitgemm, "conv2d_s8_unitgemm");
+            return run_units(espdl::launch_conv2d_s8_unitgemm);
         case DENSE_PWGEMM:
-            return run(espdl::launch_conv2d_s8_pwgemm, "conv2d_s8_pwgemm");
+            return run(espdl::launch_conv2d_s8_pwgemm);
         case DENSE_TILED:
-            return run(espdl::launch_conv2d_s8_tiled, "conv2d_s8_tiled");
+            return run(espdl::launch_conv2d_s8_tiled);
         case DENSE_DIRECT:
             break;
         }
-        return run(espdl::launch_conv2d_s8_mfma, "conv2d_s8");
+        return run(espdl::launch_conv2d_s8_mfma);
     }
     if (lut != nullptr || residual != nullptr)
         return fail(ESPDL_HIP_ENOTSUP, "the fused LUT / residual epilogues exist for ESPDL_HIP_S8 only");
@@ -343,6 +356,15 @@ int espdl_hip_conv2d_add(const espdl_hip_conv_desc *desc, const void *in, const 
         return device_status(espdl::launch_conv2d_s16_mfma(g, i16, f16, b64, shift, o16, cu_count_cached(), s),
                              "conv2d_s16_mfma");
     return device_status(espdl::launch_conv2d_s16(g, i16, f16, b64, shift, o16, s), "conv2d_s16");
+}
+
+const char *espdl_hip_conv2d_s8_kernel(const espdl_hip_conv_desc *desc, const void *in, const void *filter, const int8_t *lut,
+                                       const int8_t *residual, const void *out)
+{
+    espdl::ConvGeom g;
+    if (derive_geometry(desc, &g) != ESPDL_HIP_OK || desc->dtype != ESPDL_HIP_S8 || desc->group != 1 || g.batch == 0)
+        return nullptr;
+    return kDenseNames[dense_s8_kernel(g, in, filter, lut, residual, out, cu_count_cached())];
 }
 
 static int check_exps(int32_t in_exp, int32_t out_exp);
@@ -1111,20 +1133,20 @@ static bool mbconv_walks(const espdl::MbconvParams &p, int kind)
     return espdl::mbconv_s8_walk_us(p, cus) < (tile < 20.f ? 0.9f : 1.f) * tile;
 }
 
+// The kernels of a block as one launch.
+enum BlockRoute { BLOCK_WALK_STEM, BLOCK_WALK, BLOCK_WAVE, BLOCK_GROUP, BLOCK_DW_PROJECT, BLOCK_EXPAND_DW_PROJECT, BLOCK_FUSED };
+static const char *const kBlockNames[] = {"mbconv_s8_walk_stem", "mbconv_s8_walk", "mbconv_s8_wave", "mbconv_s8_group",
+                                          "depthwise_project_s8", "expand_depthwise_project_s8", "mbconv_s8_fused"};
+
 // A block whose tile kernel is the one-wavefront-per-tile kernel (kind 4) or the workgroup-per-tile kernel (kind 5).
-static int launch_mbconv_single(const espdl::MbconvParams &p, int kind, void *stream)
+static BlockRoute mbconv_tile_route(const espdl::MbconvParams &p, int kind)
 {
-    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    const int cus = cu_count_cached();
     // A windowed expand stage walks once the tile kernel needs more than one round over the device: 224 x 224 images, batch 32
     // 20.5 -> 17.5 us, batch 256 98 -> 62 us; 160 x 160, batch 37 20.1 -> 18.3 us.  Below that a strip is the longer chain
     // (batch 8 at 224 x 224 11.0 against 13.5 us).
-    if (!pointwise_expand(p) && espdl::mbconv_s8_wave_rounds(p) > 1.f && espdl::mbconv_s8_walk_stem_supports(p, cus))
-        return device_status(espdl::launch_mbconv_s8_walk_stem(p, cus, s), "mbconv_s8_walk_stem");
-    if (mbconv_walks(p, kind))
-        return device_status(espdl::launch_mbconv_s8_walk(p, cus, s), "mbconv_s8_walk");
-    return kind == 5 ? device_status(espdl::launch_mbconv_s8_group(p, cus, s), "mbconv_s8_group")
-                     : device_status(espdl::launch_mbconv_s8_wave(p, cus, s), "mbconv_s8_wave");
+    if (!pointwise_expand(p) && espdl::mbconv_s8_wave_rounds(p) > 1.f && espdl::mbconv_s8_walk_stem_supports(p, cu_count_cached()))
+        return BLOCK_WALK_STEM;
+    return mbconv_walks(p, kind) ? BLOCK_WALK : (kind == 5 ? BLOCK_GROUP : BLOCK_WAVE);
 }
 
 static int mbconv_kernel_choice(const espdl_hip_mbconv_desc *desc)
@@ -1218,37 +1240,31 @@ static int mbconv_params(const espdl_hip_mbconv_desc *desc, const int8_t *in, co
     return ESPDL_HIP_OK;
 }
 
-int espdl_hip_mbconv_s8(const espdl_hip_mbconv_desc *desc, const int8_t *in, const espdl_hip_mbconv_weights *w,
-                        const int8_t *residual, int8_t *out, void *stream)
+// The kernel of a checked block.  Negative: the error it is refused with.
+static int mbconv_route(const espdl_hip_mbconv_desc *desc, const espdl::MbconvParams &p)
 {
-    espdl::MbconvParams p = {};
-    const int rc = mbconv_params(desc, in, w, residual, out, &p);
-    if (rc != ESPDL_HIP_OK || p.batch == 0)
-        return rc;
     if (espdl::mbconv_has_clip(p)) {
         if (!desc->has_expand || !espdl::mbconv_s8_wave_has_fast_build(p))
             return fail(ESPDL_HIP_ENOTSUP, "a Clip between the stages is covered for the block shapes with a guard-free build of the one-wavefront-per-tile kernel, round half up");
-        return launch_mbconv_single(p, 4, stream);
+        return mbconv_tile_route(p, 4);
     }
     if (!desc->has_expand) {
         espdl::ConvGeom g;
         espdl::DwProject pj;
         dwproject_from(p, &g, &pj);
         if (p.residual_shift == 0 && espdl::depthwise_project_s8_supports(g, p.in, pj))
-            return device_status(espdl::launch_depthwise_project_s8(g, p.in, p.w_dw, p.b_dw, p.s_dw, pj, cu_count_cached(),
-                                                                    reinterpret_cast<hipStream_t>(stream)),
-                                 "depthwise_project_s8");
+            return BLOCK_DW_PROJECT;
     }
     if (desc->has_expand && !pointwise_expand(p)) {
         if (!espdl::mbconv_s8_wave_supports(p))
             return fail(ESPDL_HIP_ENOTSUP, "an expand stage with a window needs a 3x3 depthwise stage, at most 4 filter rows of at most 9 bytes (exp_k_w * in_c) and at most 64 project filters");
-        return launch_mbconv_single(p, 4, stream);
+        return mbconv_tile_route(p, 4);
     }
     if (desc->has_expand && !wave_before_group(p) && espdl::mbconv_s8_group_supports(p))
-        return launch_mbconv_single(p, 5, stream);
+        return mbconv_tile_route(p, 5);
     if (desc->has_expand && espdl::mbconv_s8_wave_supports(p))
-        return launch_mbconv_single(p, 4, stream);
-    // Only the two kernels above requantize the residual operand.  The answer comes from the real pointers: a
+        return mbconv_tile_route(p, 4);
+    // Only the kernels above requantize the residual operand.  The answer comes from the real pointers: a
     // block whose operands are merely 4-byte aligned can be refused by both although the shape alone passes.
     if (p.residual_shift != 0)
         return fail(ESPDL_HIP_ENOTSUP, "a requantized residual operand (residual_shift %d) is not covered for this block shape and operand alignment",
@@ -1259,14 +1275,58 @@ int espdl_hip_mbconv_s8(const espdl_hip_mbconv_desc *desc, const int8_t *in, con
         espdl::DwExpand ex;
         expand_dwproject_from(p, &g, &pj, &ex);
         if (espdl::expand_depthwise_project_s8_supports(g, ex, pj))
-            return device_status(espdl::launch_expand_depthwise_project_s8(g, ex, p.w_dw, p.b_dw, p.s_dw, pj, cu_count_cached(),
-                                                                           reinterpret_cast<hipStream_t>(stream)),
-                                 "expand_depthwise_project_s8");
+            return BLOCK_EXPAND_DW_PROJECT;
     }
     if (!espdl::mbconv_s8_fused_supports(p))
         return fail(ESPDL_HIP_ENOTSUP, "this block shape is not covered by the fused kernel");
-    return device_status(espdl::launch_mbconv_s8_fused(p, cu_count_cached(), reinterpret_cast<hipStream_t>(stream)),
-                         "mbconv_s8_fused");
+    return BLOCK_FUSED;
+}
+
+static hipError_t launch_mbconv_route(const espdl::MbconvParams &p, int route, hipStream_t s)
+{
+    const int cus = cu_count_cached();
+    espdl::ConvGeom g;
+    espdl::DwProject pj;
+    espdl::DwExpand ex;
+    switch (route) {
+    case BLOCK_WALK_STEM:
+        return espdl::launch_mbconv_s8_walk_stem(p, cus, s);
+    case BLOCK_WALK:
+        return espdl::launch_mbconv_s8_walk(p, cus, s);
+    case BLOCK_WAVE:
+        return espdl::launch_mbconv_s8_wave(p, cus, s);
+    case BLOCK_GROUP:
+        return espdl::launch_mbconv_s8_group(p, cus, s);
+    case BLOCK_DW_PROJECT:
+        dwproject_from(p, &g, &pj);
+        return espdl::launch_depthwise_project_s8(g, p.in, p.w_dw, p.b_dw, p.s_dw, pj, cus, s);
+    case BLOCK_EXPAND_DW_PROJECT:
+        expand_dwproject_from(p, &g, &pj, &ex);
+        return espdl::launch_expand_depthwise_project_s8(g, ex, p.w_dw, p.b_dw, p.s_dw, pj, cus, s);
+    default:
+        return espdl::launch_mbconv_s8_fused(p, cus, s);
+    }
+}
+
+int espdl_hip_mbconv_s8(const espdl_hip_mbconv_desc *desc, const int8_t *in, const espdl_hip_mbconv_weights *w,
+                        const int8_t *residual, int8_t *out, void *stream)
+{
+    espdl::MbconvParams p = {};
+    const int rc = mbconv_params(desc, in, w, residual, out, &p);
+    if (rc != ESPDL_HIP_OK || p.batch == 0)
+        return rc;
+    const int route = mbconv_route(desc, p);
+    return route < 0 ? route : device_status(launch_mbconv_route(p, route, reinterpret_cast<hipStream_t>(stream)), kBlockNames[route]);
+}
+
+const char *espdl_hip_mbconv_s8_kernel(const espdl_hip_mbconv_desc *desc, const int8_t *in, const espdl_hip_mbconv_weights *w,
+                                       const int8_t *residual, int8_t *out)
+{
+    espdl::MbconvParams p = {};
+    if (mbconv_params(desc, in, w, residual, out, &p) != ESPDL_HIP_OK || p.batch == 0)
+        return nullptr;
+    const int route = mbconv_route(desc, p);
+    return route < 0 ? nullptr : kBlockNames[route];
 }
 
 // The project convolution of a block as a dense convolution over the depthwise result.

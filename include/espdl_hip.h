@@ -102,6 +102,11 @@ int espdl_hip_conv2d(const espdl_hip_conv_desc *desc, const void *in, const void
  */
 int espdl_hip_conv2d_add(const espdl_hip_conv_desc *desc, const void *in, const void *filter, const void *bias,
                          const int32_t *shift, const int8_t *lut, const int8_t *residual, void *out, void *stream);
+/* Name of the kernel that espdl_hip_conv2d_add() takes for these operands of a dense int8 layer, NULL for any other layer and
+ * where it refuses them.  Reads and launches nothing, the pointers count by being given and by their alignment.  For tests and
+ * measurements of one kernel. */
+const char *espdl_hip_conv2d_s8_kernel(const espdl_hip_conv_desc *desc, const void *in, const void *filter, const int8_t *lut,
+                                       const int8_t *residual, const void *out);
 
 /* base::lut_s8 (esp-dl/dl/base/dl_base_lut.cpp:10-48): out[i] = table[(uint8)in[i] ^ 0x80]. In-place allowed. */
 int espdl_hip_lut_s8(const int8_t *in, int64_t size, const int8_t *table, int8_t *out, void *stream);
@@ -473,6 +478,10 @@ int espdl_hip_mbconv_s8_supported(const espdl_hip_mbconv_desc *desc);
 int espdl_hip_mbconv_s8_preferred(const espdl_hip_mbconv_desc *desc);
 int espdl_hip_mbconv_s8(const espdl_hip_mbconv_desc *desc, const int8_t *in, const espdl_hip_mbconv_weights *weights,
                         const int8_t *residual, int8_t *out, void *stream);
+/* Name of the kernel that espdl_hip_mbconv_s8() takes for these operands, NULL where it refuses them.  Reads and launches
+ * nothing, the pointers count by being given and by their alignment.  For tests and measurements of one kernel. */
+const char *espdl_hip_mbconv_s8_kernel(const espdl_hip_mbconv_desc *desc, const int8_t *in, const espdl_hip_mbconv_weights *weights,
+                                       const int8_t *residual, int8_t *out);
 
 /*
  * The same block in one or two launches, whichever is expected to be faster: with few images (or few tiles) the single

@@ -79,3 +79,54 @@ def test_two_launches_are_weighed_against_the_launch_that_a_block_with_an_add_ta
     # a depthwise stride takes the operand away, and with it the reason
     d = m.capi.MbconvDesc(24, 56, 56, 24, 144, 24, 1, 3, 3, 2, 2, 1, 1, 1, 1, 1, 1, 1, 1, 0, 0, 144, 144, 24)
     assert m.lib().espdl_hip_mbconv_s8_workspace(C.byref(d)) == 0
+
+
+def _dense_kernel(m, shape, out_c, k, stride=1, pad=None, dilation=1, lut=None, residual=None, half_even=0, out_pitch=0, group=1, dtype=None):
+    import ctypes as C
+    pad = k // 2 * dilation if pad is None else pad
+    d = m.capi.make_desc(shape, out_c, (k, k), (stride, stride), (dilation, dilation), (pad,) * 4, group=group, round_mode=half_even,
+                         n_shift=out_c, dtype=m.capi.S8 if dtype is None else dtype)
+    d.out_pitch = out_pitch
+    return m.lib().espdl_hip_conv2d_s8_kernel(C.byref(d), 1 << 20, 2 << 20, lut, residual, 3 << 20)
+
+
+def test_dense_kernels_are_named_without_a_launch():
+    """One layer of each kernel of the dense dispatch, and the calls it refuses (no GPU needed)."""
+    import importlib
+    m = importlib.import_module("esp-dl_amd")
+    assert _dense_kernel(m, (256, 56, 56, 64), 64, 3) == b"conv2d_s8_walk"
+    assert _dense_kernel(m, (64, 640, 640, 3), 16, 3, 2) == b"conv2d_s8_walk_stem"
+    assert _dense_kernel(m, (64, 641, 641, 3), 16, 3, 2) == b"conv2d_s8_stem"
+    assert _dense_kernel(m, (1, 20, 20, 16), 16, 3) == b"conv2d_s8_narrow"
+    assert _dense_kernel(m, (80, 30, 31, 31), 64, 5, 2) == b"conv2d_s8_unitgemm"
+    assert _dense_kernel(m, (256, 14, 14, 576), 96, 1) == b"conv2d_s8_pwgemm"
+    assert _dense_kernel(m, (256, 56, 56, 64), 64, 3, half_even=1) == b"conv2d_s8_tiled"
+    assert _dense_kernel(m, (256, 80, 80, 32), 48, 1, half_even=1) == b"conv2d_s8"
+    assert _dense_kernel(m, (1, 1, 20480, 120), 6625, 1) == b"conv2d_s8_wide"
+    assert _dense_kernel(m, (1, 20, 20, 16), 16, 3, out_pitch=8) is None
+    assert _dense_kernel(m, (1, 20, 20, 16), 16, 3, group=16) is None
+    assert _dense_kernel(m, (1, 20, 20, 16), 16, 3, dtype=m.capi.S16) is None
+
+
+def test_block_kernels_are_named_without_a_launch():
+    import ctypes as C
+    import importlib
+    m = importlib.import_module("esp-dl_amd")
+    base = 1 << 20
+
+    def kernel(batch, hw, cin, ce, cout, stride=1, residual=False, shift=0, aligned=True, stem=False):
+        d = m.capi.MbconvDesc(batch, hw, hw, cin, ce, cout, 1, 3, 3, stride, stride, 1, 1, 1, 1, 1, 1, 1, 1, 0, 0, ce, ce, cout)
+        d.residual_shift = shift
+        if stem:
+            d.exp_k_h = d.exp_k_w = 3
+            d.exp_stride_h = d.exp_stride_w = 2
+            d.exp_pad_top = d.exp_pad_bottom = d.exp_pad_left = d.exp_pad_right = 1
+        w = m.capi.MbconvWeights(base * 3, None, base * 4, base * 5, None, base * 6, base * 7, None, base * 8)
+        return m.lib().espdl_hip_mbconv_s8_kernel(C.byref(d), base + (0 if aligned else 4), C.byref(w), base * 9 if residual else None, base * 10)
+
+    assert kernel(256, 56, 24, 144, 24, residual=True) == b"mbconv_s8_walk"
+    assert kernel(256, 28, 32, 192, 32, residual=True) == b"mbconv_s8_wave"
+    assert kernel(256, 14, 96, 576, 96, residual=True) == b"mbconv_s8_group"
+    assert kernel(256, 224, 3, 32, 16, stem=True) == b"mbconv_s8_walk_stem"
+    assert kernel(4, 224, 3, 32, 16, stem=True) == b"mbconv_s8_wave"
+    assert kernel(256, 14, 96, 576, 96, residual=True, shift=2, aligned=False) is None
