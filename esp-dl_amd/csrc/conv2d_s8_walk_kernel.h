@@ -703,7 +703,9 @@ WalkCut walk_cut(const WalkArgs &a, const WalkLaunch &l, int per_cu)
 // alike they add up in part.  The constants are a fit over 780 random layers of 1 to 260 MB (1641 builds, 8 % root mean
 // square).  Filter chunks of one pixel are written by different workgroups: past what the caches hold, their pieces of a
 // line reach memory one by one (188 x 63 x 88 x 32 -> 96, 1 x 1: 40 us as one chunk, 66 as pieces of 64 bytes, 81 of 32).
-template <int KH, int S, int CU, int NT, bool RES>
+// RAW builds under 3 x 3 pass their pieces through registers step by step, which takes a fifth longer; those of 11 and 12 units of
+// a pixel and the ones of 15 and 16 without RAW spill 24 to 35 registers besides (1600 and 60 layers).
+template <int KH, int S, int CU, int NT, bool RES, bool RAW>
 float walk_us(const WalkArgs &a, const WalkLaunch &l)
 {
     using Shape = WalkShape<KH, S, CU, NT, RES>;
@@ -720,7 +722,9 @@ float walk_us(const WalkArgs &a, const WalkLaunch &l)
         std::cbrt((walk * std::sqrt(walk) + memory * std::sqrt(memory)) * (walk * std::sqrt(walk) + memory * std::sqrt(memory)));
     if (c.chunks > 1 && l.out_bytes > 80000000)
         us += 12e-6f * (float)l.out_bytes / (float)(16 * NT);
-    return us;
+    if constexpr (RAW)
+        return KH == 1 ? us + 0.1f : us * (CU <= 3 ? 1.15f : (CU <= 10 ? 1.2f : 1.5f)) + 0.3f;
+    return KH == 3 && S == 1 && CU >= 15 ? 1.5f * us : us;
 }
 
 template <int KH, int S, int CU, int NT, bool RES, bool RAW = false>
@@ -731,7 +735,7 @@ hipError_t launch_one(WalkArgs &a, const WalkLaunch &l)
     } else {
         using Shape = WalkShape<KH, S, CU, NT, RES>;
         if (l.us != nullptr) {
-            *l.us = walk_us<KH, S, CU, NT, RES>(a, l);
+            *l.us = walk_us<KH, S, CU, NT, RES, RAW>(a, l);
             return hipSuccess;
         }
         constexpr int kThreads = 64 * Shape::W;

@@ -140,10 +140,7 @@ const char *const kDenseNames[] = {"conv2d_s8_walk", "conv2d_s8_stem", "conv2d_s
 
 // Kernel of a dense int8 convolution.  The two kernels that read windows as 16-channel units take any layer; their
 // times, measured over 128 layers of 1 to 600 K output pixels, are straight lines in their work (within 15 %), so the
-// choice between them compares those lines.  The walking kernel takes what it has a build for where its expected time is
-// the smaller one: over 780 random layers of 16 to 256 channels (1 image to 260 MB) the kernels below take 1.14 times
-// as long in the geometric mean, twice and more from a hundred thousand pixels on; below some 4 us the narrow kernel is the
-// faster one (16 x 16 x 20 x 20, 3 x 3: 3.1 against 3.7 us).  Where the other kernels begin:
+// choice between them compares those lines.  Where the other kernels begin, the walking kernel (dense_s8_walks) aside:
 //   * window rows of at most 16 bytes (RGB input): the first-layer kernel, which never takes less than 5.2 us;
 //   * 1x1 over flat rows: the pointwise GEMM kernel where it applies (two reads less address arithmetic), the direct
 //     kernel where pixels are many and channels few (its wavefronts keep their pixels in registers and write whole
@@ -156,28 +153,9 @@ const char *const kDenseNames[] = {"conv2d_s8_walk", "conv2d_s8_stem", "conv2d_s
 //     stride 2, batch 32: 35.5 against 38.3 us).
 // A channel count that is not a multiple of 16 under a window has no other kernel worth taking: 31 x 101 x 61 -> 16,
 // 5 x 5, batch 142: 509 -> 105 us; 45 x 99 x 162 -> 87, 5 x 5 at stride 2, batch 3: 312 -> 40 us.
-DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *filter, const void *residual, const void *out,
-                          int cus)
+DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *filter, const void *residual, bool units,
+                          float narrow, float gemm, long long tile_steps, int cus)
 {
-    const bool units = images_per_launch(g, espdl::conv2d_s8_units_support) > 0;
-    float narrow = 0.f, gemm = 0.f;
-    long long tile_steps = 0; // 64-pixel x 64-filter tiles times reduction steps
-    if (units) {
-        narrow = espdl::conv2d_s8_narrow_us(g, in, filter, cus);
-        gemm = espdl::conv2d_s8_unitgemm_us(g, in, filter, &tile_steps);
-        // (the larger routes below take up to twice the unit kernel's line; a quarter more puts no layer on the walk that
-        // is slower there by more than a fifth, and gives up 2 % of what the best choice of 780 random layers would)
-        // Channels that are no multiple of 16 cost it a further microsecond of set-up and partial lanes (60 random layers: 5 to
-        // 7 us where the others take 5, but 48 -> 13 us on 202 x 67 x 42 x 40 -> 13, 3 x 3, and 45 -> 13 us on 5 x 5 windows).
-        // No multiple of 4: pieces through registers, which the estimate does not know of: a 3 x 3 layer takes 1.2 to 1.5 times
-        // it, a 1 x 1 one 0.2 to 1.5 us more.  70 random layers gain a fifth in the geometric mean by this line, from 147 ->
-        // 45 us on 163 x 91 x 36 x 137 -> 30, 3 x 3; one is slower (222 x 84 x 18 x 67 -> 177, 1 x 1: 40 -> 44 us).
-        const float walk = espdl::conv2d_s8_walk_us(g, in, filter, residual, out, cus);
-        const float partial = ((g.in_c | g.out_c) & 15) != 0 ? 1.2f : 0.f;
-        const bool raw = ((g.in_c | g.in_pitch) & 3) != 0;
-        if (raw ? (g.k_h == 1 ? walk + 0.2f : 1.15f * walk + 0.6f) < std::min(narrow, gemm) : walk + partial < std::min(narrow, 1.25f * gemm))
-            return DENSE_WALK;
-    }
     if (espdl::conv2d_s8_stem_supports(g, residual))
         return units && narrow < 5.2f ? DENSE_NARROW : DENSE_STEM;
     const bool flat = g.k_h == 1 && g.k_w == 1 && g.stride_h == 1 && g.stride_w == 1 && g.pad_top == 0 &&
@@ -198,14 +176,40 @@ DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *
     return espdl::conv2d_s8_tiled_supports(g, in, filter, cus) ? DENSE_TILED : DENSE_DIRECT;
 }
 
-// The same with the kernels that take all layers that they apply to: the classifier's, and a walk of the first-layer kernel's
-// layers (one 416 x 416 image 5.1 us either way, 64 of 640 x 640 50 against 78 us).
+// The walking kernel takes what it has a build for where its expected time is the smaller one.  The estimates lie 8 to 10 %
+// off either way, and of two such the smaller one is more often the one that is too small, so 5 x 5 has to win by a margin;
+// the larger kernels take up to twice the unit kernel's line, the direct one three quarters of it where it writes long rows
+// that no other writes whole (channels that are no multiple of 4: 112 x 23 x 112 x 22 -> 158, 1 x 1, 23.1 against 31.8 us).  3076 random layers of 16 to 256
+// channels in 1 image to 400 MB, each timed on both sides with operands that change from launch to launch: 0.88 of the other
+// kernels' time in the geometric mean on channels that are a multiple of 4, 0.80 on others (the better one of each pair: 0.87,
+// 0.78); 1.7 % of all are slower by more than 5 % than on the other kernel, 0.9 % by more than 10.  (On operands that lie in the
+// L2 caches the other kernels gain more and a margin of 1.2 under 3 x 3 looks right; it costs a detector of 20 frames of 320 x 320
+// 8 % of its dense layers' time.)
+bool dense_s8_walks(const espdl::ConvGeom &g, DenseRoute other, float walk, float narrow, float gemm)
+{
+    const bool few = other == DENSE_NARROW || other == DENSE_UNITGEMM;
+    if (((g.in_c | g.in_pitch) & 3) != 0)
+        return walk < std::min(1.05f * narrow, gemm * (other == DENSE_PWGEMM ? 0.9f : (other == DENSE_DIRECT && g.out_c >= 96 ? 0.7f : 1.f)));
+    return walk * (g.k_h == 1 ? 1.f : (g.k_h == 3 ? 1.02f : 1.1f)) < std::min(narrow, gemm * (few ? 1.15f : 1.4f));
+}
+
+// Of all kernels.  Two take every layer that they apply to: the classifier's, and the walk of the first-layer kernel's layers
+// (one 416 x 416 image 5.1 us either way, 64 of 640 x 640 50 against 78 us).
 DenseRoute dense_s8_kernel(const espdl::ConvGeom &g, const void *in, const void *filter, const int8_t *lut, const int8_t *residual,
                            const void *out, int cus)
 {
     if (espdl::conv2d_s8_wide_supports(g, lut, residual))
         return DENSE_WIDE;
-    const DenseRoute route = dense_s8_route(g, in, filter, residual, out, cus);
+    const bool units = images_per_launch(g, espdl::conv2d_s8_units_support) > 0;
+    float narrow = 0.f, gemm = 0.f;
+    long long tile_steps = 0; // 64-pixel x 64-filter tiles times reduction steps
+    if (units) {
+        narrow = espdl::conv2d_s8_narrow_us(g, in, filter, cus);
+        gemm = espdl::conv2d_s8_unitgemm_us(g, in, filter, &tile_steps);
+    }
+    const DenseRoute route = dense_s8_route(g, in, filter, residual, units, narrow, gemm, tile_steps, cus);
+    if (units && dense_s8_walks(g, route, espdl::conv2d_s8_walk_us(g, in, filter, residual, out, cus), narrow, gemm))
+        return DENSE_WALK;
     return route == DENSE_STEM && espdl::conv2d_s8_walk_stem_supports(g, in, out, residual) ? DENSE_WALK_STEM : route;
 }
 

@@ -130,3 +130,23 @@ def test_block_kernels_are_named_without_a_launch():
     assert kernel(256, 224, 3, 32, 16, stem=True) == b"mbconv_s8_walk_stem"
     assert kernel(4, 224, 3, 32, 16, stem=True) == b"mbconv_s8_wave"
     assert kernel(256, 14, 96, 576, 96, residual=True, shift=2, aligned=False) is None
+
+
+def test_dense_layers_go_to_the_faster_kernel():
+    """Layers that one kernel takes less time for, most of them a tenth and more (measured with operands that change from
+    launch to launch; us there and on the other kernel)."""
+    import importlib
+    m = importlib.import_module("esp-dl_amd")
+    for shape, out_c, k, stride, kernel in (
+            ((194, 79, 72, 17), 202, 1, 1, b"conv2d_s8"),          # 120, 181
+            ((14, 35, 43, 16), 96, 5, 1, b"conv2d_s8_unitgemm"),   # 7.5, 10.6
+            ((43, 75, 11, 16), 240, 5, 2, b"conv2d_s8_unitgemm"),  # 7.8, 8.9
+            ((9, 13, 43, 16), 64, 3, 1, b"conv2d_s8_narrow"),      # 3.3, 3.9
+            ((1, 20, 20, 240), 16, 3, 1, b"conv2d_s8_narrow"),     # 3.9, 9.0
+            ((1, 56, 56, 64), 64, 3, 1, b"conv2d_s8_walk"),        # 4.1, 4.2
+            ((82, 15, 19, 16), 171, 1, 1, b"conv2d_s8_walk"),      # 4.9, 7.7
+            ((39, 8, 8, 116), 107, 1, 1, b"conv2d_s8_walk"),       # 3.2, 4.4
+            ((10, 18, 26, 43), 25, 3, 1, b"conv2d_s8_walk"),       # 4.4, 6.5
+            ((4, 44, 8, 125), 14, 1, 1, b"conv2d_s8_walk"),        # 3.0, 4.2
+            ((153, 12, 69, 240), 16, 3, 1, b"conv2d_s8_walk")):    # 17.6, 43
+        assert _dense_kernel(m, shape, out_c, k, stride) == kernel, (shape, out_c, k, stride)
