@@ -20,7 +20,10 @@
 //
 // Bound by memory, at the number of rows in flight: with conditional loads, none of them early, 256 images of 56 x 56 x 144
 // took 69 us (3 x 3: 61), 100 of 80 x 80 x 96 44 us and 64 of 20 x 20 x 128 6.9 us; a row ahead 63 (61), 42 and 5.8 us,
-// 3.7 TB/s in and out.
+// 3.7 TB/s in and out.  Pixels that are not whole dwords apart are taken apart by the memory pipeline, and there the up to five
+// rows that a strip requests and does not use cost more than a row ahead gives (17 x 14 x 198, 5 x 5, batch 144: 13.1 us with
+// conditional loads, 15.4 with them); the builds for those ask before every row, which costs the others (2 x 17 x 76 x 112,
+// 5 x 5: 4.05 -> 4.86).
 // Input and output may be channel slices of wider tensors (pitches in bytes).  Where the channels are no multiple of
 // the vector, the last one of a pixel reaches back over its neighbour's channels and both write the same bytes: 36 x 8 x
 // 194, 128 images take 13.4 us, one byte per thread took 101 us.
@@ -108,8 +111,8 @@ __device__ __forceinline__ Vec<D> join(const Vec<D> &odd, const Vec<D> &even)
     return r;
 }
 
-// K x K window, D dwords of channels per thread
-template <int K, int D>
+// K x K window, D dwords of channels per thread.  SHORT: rows that the strip does not use are not requested.
+template <int K, int D, bool SHORT>
 __global__ __launch_bounds__(kThreads) void max_pool_s8_window_kernel(const WindowPoolArgs a)
 {
     typedef Vec<D> V;
@@ -159,7 +162,8 @@ __global__ __launch_bounds__(kThreads) void max_pool_s8_window_kernel(const Wind
                 odd[c] = next[c];
                 even[c] = shifted(odd[c]);
             }
-            load_row(r + 1, next); // (the last one is not used)
+            if (!SHORT || r + 1 < nrows) // uniform
+                load_row(r + 1, next);
             // columns 1 .. K-1 are under both windows
             V both_odd = odd[1], both_even = even[1];
 #pragma unroll
@@ -187,14 +191,14 @@ __global__ __launch_bounds__(kThreads) void max_pool_s8_window_kernel(const Wind
     }
 }
 
-template <int K>
-hipError_t launch_window(const WindowPoolArgs &a, int dwords, hipStream_t stream)
+template <int K, int D>
+hipError_t launch_window(const WindowPoolArgs &a, bool whole, hipStream_t stream)
 {
     const dim3 grid((a.total + kThreads - 1) / kThreads);
-    if (dwords == 4)
-        hipLaunchKernelGGL((max_pool_s8_window_kernel<K, 4>), grid, dim3(kThreads), 0, stream, a);
+    if (whole)
+        hipLaunchKernelGGL((max_pool_s8_window_kernel<K, D, false>), grid, dim3(kThreads), 0, stream, a);
     else
-        hipLaunchKernelGGL((max_pool_s8_window_kernel<K, 2>), grid, dim3(kThreads), 0, stream, a);
+        hipLaunchKernelGGL((max_pool_s8_window_kernel<K, D, true>), grid, dim3(kThreads), 0, stream, a);
     return hipGetLastError();
 }
 
@@ -267,13 +271,16 @@ hipError_t launch_max_pool_s8_window(const void *in, int batch, int h, int w, in
     a.fd_cv = make_fastdiv((unsigned)a.cv);
     a.fd_xpairs = make_fastdiv((unsigned)a.xpairs);
     a.fd_strips = make_fastdiv((unsigned)a.strips);
+    // (2 x 2 reads a third more rows than it uses: up to some 3 MB 5 % less time all the same, above that 5 % more)
+    const bool whole = ((reinterpret_cast<uintptr_t>(in) | (uintptr_t)in_pitch | (uintptr_t)c) & 3) == 0 &&
+        (k != 2 || (long long)batch * h * w * c <= (3 << 20));
     switch (k) {
     case 2:
-        return launch_window<2>(a, dwords, stream);
+        return dwords == 4 ? launch_window<2, 4>(a, whole, stream) : launch_window<2, 2>(a, whole, stream);
     case 3:
-        return launch_window<3>(a, dwords, stream);
+        return dwords == 4 ? launch_window<3, 4>(a, whole, stream) : launch_window<3, 2>(a, whole, stream);
     default:
-        return launch_window<5>(a, dwords, stream);
+        return dwords == 4 ? launch_window<5, 4>(a, whole, stream) : launch_window<5, 2>(a, whole, stream);
     }
 }
 

@@ -198,6 +198,8 @@ def test_avg_pool_and_reduce_mean_s8_every_sum(oracle, hw):
     ((2, 12, 11, 32), 5, (0, 0, 0, 0)), ((2, 11, 12, 16), 3, (1, 1, 1, 1)), ((2, 8, 7, 64), 3, (0, 2, 2, 0)),
     ((3, 6, 5, 16), 2, (0, 1, 0, 1)), ((1, 80, 80, 16), 5, (2, 2, 2, 2)), ((70, 20, 20, 16), 5, (2, 2, 2, 2)),
     ((2, 9, 9, 8), 5, (2, 2, 2, 2)), ((2, 10, 7, 24), 3, (1, 1, 1, 1)),
+    # 2 x 2 above 3 MB, which requests no row that a strip does not use
+    ((2, 157, 170, 64), 2, (0, 1, 0, 1)), ((129, 31, 17, 48), 2, (1, 0, 1, 0)),
 ])
 @pytest.mark.parametrize("fill", ["random", "extremes", "low"])
 def test_max_pool_window_kernel(oracle, shape, k, pads, fill):
