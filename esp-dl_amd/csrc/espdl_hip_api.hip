@@ -276,7 +276,12 @@ int espdl_hip_conv2d_add(const espdl_hip_conv_desc *desc, const void *in, const 
         if (residual != nullptr && depthwise)
             return fail(ESPDL_HIP_ENOTSUP, "the fused residual Add exists for dense int8 convolutions only");
         if (depthwise) {
-            if (espdl::depthwise_s8_strip_supports(g))
+            // (strides of 3 and more in y share no rows between outputs, and what is left of the strips' gain comes with the work: on
+            // channels that are no multiple of 4 a byte per thread is the faster form up to some 200 K results, 320 K at stride 2 in x:
+            // 6 x 28 x 41 x 17 at stride (3, 2) 3.7 against 6.0 us; on multiples of 4 it takes 8 us, on 16 channels the others 5)
+            const bool few = g.stride_h > 2 && (g.in_c & 3) != 0 &&
+                (long long)g.batch * g.out_h * g.out_w * g.out_c < (g.stride_w == 1 ? 200000 : 320000);
+            if (!few && espdl::depthwise_s8_strip_supports(g))
                 return device_status(espdl::launch_depthwise_s8_strip(g, i8, f8, b32, shift, lut, o8, cu_count_cached(), s),
                                      "depthwise_s8_strip");
             if (espdl::depthwise_s8_lds_supports(g, in, out))

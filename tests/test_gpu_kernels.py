@@ -938,7 +938,9 @@ def test_depthwise_s8_strips(oracle, case, half_even):
 @pytest.mark.parametrize("case", [
     # strides in y that leave output rows no input row in common: one row and many, skipped rows, padding above and below
     ((20, 3, 40, 120), (3, 1), (1, 1, 1, 1), False), ((9, 61, 13, 18), (3, 2), (1, 1, 1, 1), True),
-    ((2, 50, 9, 7), (5, 1), (0, 2, 1, 0), False), ((1, 2, 5, 4), (4, 2), (1, 1, 0, 1), False), ((300, 31, 10, 33), (4, 1), (2, 0, 1, 1), True)],
+    ((2, 50, 9, 7), (5, 1), (0, 2, 1, 0), False), ((1, 2, 5, 4), (4, 2), (1, 1, 0, 1), False), ((300, 31, 10, 33), (4, 1), (2, 0, 1, 1), True),
+    # channels that are no multiple of 4 take the strips from 200 K results on, 320 K at stride 2 in x
+    ((400, 50, 9, 7), (5, 1), (0, 2, 1, 0), False), ((140, 61, 13, 18), (3, 2), (1, 1, 1, 1), True)],
     ids=lambda c: "x".join(map(str, c[0])) + "_s%d%d" % c[1])
 def test_depthwise_s8_strips_without_shared_rows(oracle, case, half_even):
     shape, stride, pads, with_lut = case
