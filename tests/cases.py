@@ -30,7 +30,7 @@ CONV_CASES = [
 ]
 
 # Convolutions whose window rows are at most 16 contiguous bytes (k_w * C <= 16) with at most 4 rows and 64 filters:
-# the first-layer kernel that does the whole reduction in one MFMA step.  RGB / grey / RGBA / 5 and 8 channels, a
+# the first-layer kernel's layers (few images: they go to the narrow one, OTHER_KERNELS has larger ones).  RGB / grey / RGBA / 5 and 8 channels, a
 # 1 x 2 window over 8 channels, 7 to 64 filters (1 to 4 filter tiles, ragged ones), strides 1 to 3, dilated
 # rows, padding on both / one / no side, rows longer than one 64-pixel unit, a one-row image.
 STEM_CASES = [
@@ -47,8 +47,9 @@ STEM_CASES = [
 ]
 
 # Pointwise products with at most 128 input channels over enough pixels to fill the device (3 x 80 x 80: the routes
-# the dispatcher takes for many pixels, which the small cases above never reach).  One and two reduction steps,
-# reductions that end inside a step (72, 100, 120), filter counts that are no multiple of 64 / 16 / 4, many filters.
+# the dispatcher takes for many pixels, which the small cases above never reach: the walk, in half even the GEMM kernels).  One
+# and two reduction steps, reductions that end inside a step (72, 100, 120), filter counts that are no multiple of 64 / 16 / 4,
+# many filters.
 POINTWISE_MANY_PIXELS = [
     ("p16_32", (80, 80, 16), 32, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, True),
     ("p32_64", (80, 80, 32), 64, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, False),
@@ -74,8 +75,8 @@ WIDE_ROWS = [
     ("w16_1900", (81, 81, 16), 1900, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, False),
 ]
 
-# Windowed convolutions whose channel count is a multiple of 16: the kernel that stages the input tile and the
-# filters in LDS.  Strides 1 to 3, dilation, reduction steps that span several taps (16, 32, 48 channels), several
+# Windowed convolutions whose channel count is a multiple of 16, on few images: the layers that the kernel with its input tile
+# and filters in LDS takes on more (OTHER_KERNELS), here on the narrow kernel and the walk.  Strides 1 to 3, dilation, reduction steps that span several taps (16, 32, 48 channels), several
 # groups of 64 filters in one and in several chunks, filter counts that are not a multiple of 64 / 16 / 4, images
 # wider than one column tile, ragged last tiles, padding on one side only, a window larger than the image.
 TILED_CASES = [
@@ -96,8 +97,7 @@ TILED_CASES = [
 ]
 
 # 1x56x56x64 -> 64, 3x3, s1, p1, bias, ReLU, shift 9
-# Strided windows over 64 channels or more on few pixels: rows gathered from under the window for the pointwise
-# GEMM kernel.  Strides 2, 3 and mixed, 3 x 3 / 5 x 5 / 2 x 4 windows, dilation, asymmetric padding, windows that
+# Strided windows over 64 channels or more on few pixels.  Strides 2, 3 and mixed, 3 x 3 / 5 x 5 / 2 x 4 windows, dilation, asymmetric padding, windows that
 # hang over every border, 64 / 128 / 192 / 320 channels, filter counts that are not a multiple of 64 / 16 / 4, pixel
 # counts that are not a multiple of 64 or 128.
 WINDOW_GEMM_CASES = [
@@ -112,16 +112,16 @@ WINDOW_GEMM_CASES = [
     ("g128_12x50_k24s21p0312_oc64", (12, 50, 128), 64, (2, 4), (2, 1), (1, 1), (0, 3, 1, 2), True, True),
 ]
 
-# Stride-1 windows over 64 and 128 channels on more than 128 K output pixels (with the batch the test gives them):
-# the shapes that stay with the LDS-tiled kernel when the few-pixel route takes the smaller ones.
+# Stride-1 windows over 64 and 128 channels on more than 128 K output pixels (with the batch the test gives them): the
+# LDS-tiled kernel in half even and dilated, the walk else.
 TILED_MANY_PIXELS = [
     ("tm64_56x56_k3p1_oc64", (56, 56, 64), 64, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True),
     ("tm128_40x44_k3p1_oc96", (40, 44, 128), 96, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, False),
     ("tm64_50x60_k3d2p2_oc72", (50, 60, 64), 72, (3, 3), (1, 1), (2, 2), (2, 2, 2, 2), False, True),
 ]
 
-# Windows over channel counts around the 16-channel units the two unit-reading kernels work in (one less, one more, a
-# single channel, several units), with the batch each needs to reach the one kernel or the other: (case, images).
+# Windows over channel counts around the 16-channel units the two unit-reading kernels and the walk work in (one less, one more, a
+# single channel, several units), on few and on many pixels: (case, images).
 UNIT_CASES = [
     (("u17_5x7_k3p1_oc1", (5, 7, 17), 1, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True), 1),
     (("u15_9x9_k3s2p1_oc31", (9, 9, 15), 31, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), True, False), 2),
@@ -195,14 +195,14 @@ def every_sum_image(h, w):
 # dispatcher takes it).  1 x 1 over pixel counts that end inside a workgroup's tile, one and several chunks of 16 to 128
 # filters, chunks that end early, every second pixel of odd extents; windows over images narrower than a tile, widths one
 # below and above a tile, many images in one tile, one-sided and missing padding, odd extents at stride 2, walks that start
-# and end inside an image, 16 to 256 input channels.
+# and end inside an image, 16 to 256 input channels.  The test checks that they go there.
 WALK_CASES = [
-    (2, ("w1_16_16", (97, 131, 16), 16, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, True)),
-    (5, ("w1_64_176", (61, 67, 64), 176, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, True)),
+    (6, ("w1_16_16", (97, 131, 16), 16, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, True)),
+    (20, ("w1_64_176", (61, 67, 64), 176, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, True)),
     (7, ("w1_112_48", (45, 83, 112), 48, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), False, True)),
     (9, ("w1_256_256", (33, 31, 256), 256, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, False)),
     (16, ("w1s2_96_64", (45, 83, 96), 64, (1, 1), (2, 2), (1, 1), (0, 0, 0, 0), True, True)),
-    (40, ("w3_16_16", (37, 53, 16), 16, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
+    (100, ("w3_16_16", (37, 53, 16), 16, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
     (19, ("w3_32_32", (40, 81, 32), 32, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, False)),
     (30, ("w3_48_48", (31, 33, 48), 48, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
     (64, ("w3_64_64", (20, 20, 64), 64, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
@@ -210,8 +210,8 @@ WALK_CASES = [
     (23, ("w3_128_64_nopad", (29, 18, 128), 64, (3, 3), (1, 1), (1, 1), (0, 0, 0, 0), False, True)),
     (26, ("w3_64_80_tailpad", (25, 15, 64), 80, (3, 3), (1, 1), (1, 1), (0, 2, 0, 1), True, True)),
     (33, ("w3_224_16", (23, 30, 224), 16, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
-    (1, ("w3_32_64_one_image", (150, 161, 32), 64, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
-    (90, ("w3s2_16_32_tailpad", (80, 112, 16), 32, (3, 3), (2, 2), (1, 1), (0, 1, 0, 1), True, True)),
+    (1, ("w3_32_64_one_image", (400, 261, 32), 64, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
+    (200, ("w3s2_16_32_tailpad", (80, 112, 16), 32, (3, 3), (2, 2), (1, 1), (0, 1, 0, 1), True, True)),
     (40, ("w3s2_64_64", (49, 51, 64), 64, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), True, True)),
     (50, ("w3s2_128_64", (41, 30, 128), 64, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), True, False)),
     (20, ("w5_16_16", (47, 65, 16), 16, (5, 5), (1, 1), (1, 1), (2, 2, 2, 2), True, True)),
@@ -232,4 +232,40 @@ WALK_CASES = [
     (84, ("w1_246_59_raw", (24, 21, 246), 59, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, True)),
     (90, ("w1s2_49_185_raw", (31, 78, 49), 185, (1, 1), (2, 2), (1, 1), (0, 0, 0, 0), True, True)),
     (40, ("w5_56_21_partial", (60, 17, 56), 21, (5, 5), (1, 1), (1, 1), (2, 2, 2, 2), True, True)),
+]
+
+# The ones whose residual operand the walk adds: whole filter tiles, 1 x 1 and stride-1 3 x 3 windows.
+WALK_RESIDUAL = [c for c in WALK_CASES if c[1][2] % 16 == 0 and c[1][1][2] % 4 == 0 and (c[1][3] == (1, 1) or (c[1][3] == (3, 3) and c[1][4] == (1, 1)))]
+# Channels that are a multiple of 4 at pixels that are not (the builds whose pieces pass through registers).
+WALK_ODD_PITCH = [c for c in WALK_CASES if c[1][0] in ("w1_64_176", "w1_256_256", "w1s2_96_64", "w3_32_32", "w3_64_64", "w3_128_64_nopad", "w3_64_80_tailpad",
+                                                       "w1_44_153_partial", "w3_40_13_partial", "w3_20_32_partial")]
+# Results above 16 MB, which leave by plain stores: whole and partial lanes, pieces through registers.
+WALK_LARGE = [
+    (110, ("w3_16_32_large", (75, 67, 16), 32, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
+    (100, ("w1_32_48_large", (63, 59, 32), 48, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, False)),
+    (150, ("w1_44_36_partial_large", (40, 83, 44), 36, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, True)),
+    (40, ("w3_20_36_partial_large", (110, 112, 20), 36, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), False, True)),
+    (90, ("w1_21_24_raw_large", (90, 102, 21), 24, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, False)),
+    (60, ("w3_18_30_raw_large", (97, 101, 18), 30, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
+]
+
+# Half-up layers that the walk has no build for or loses, for every other kernel of the dense dispatch: (kernel, images, case).
+# Dilated and non-square windows, strides of 3, more than 256 input channels, fewer than 16; the test checks the kernel.
+OTHER_KERNELS = [
+    ("conv2d_s8_stem", 20, ("stem_rgb_k3s2", (200, 203, 3), 16, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), True, True)),
+    ("conv2d_s8_stem", 30, ("stem_rgb_k3dh2", (61, 67, 3), 24, (3, 3), (1, 1), (2, 1), (2, 2, 1, 1), True, False)),
+    ("conv2d_s8_stem", 40, ("stem_5_k3_33", (51, 77, 5), 33, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), False, True)),
+    ("conv2d_s8_stem", 40, ("stem_8_k1x2_64", (60, 61, 8), 64, (1, 2), (1, 1), (1, 1), (0, 0, 0, 1), True, False)),
+    ("conv2d_s8_stem", 60, ("stem_1_k4s2", (81, 90, 1), 8, (4, 4), (2, 2), (1, 1), (1, 2, 1, 2), True, True)),
+    ("conv2d_s8_tiled", 45, ("tiled_64_72_d2", (50, 60, 64), 72, (3, 3), (1, 1), (2, 2), (2, 2, 2, 2), False, True)),
+    ("conv2d_s8_tiled", 40, ("tiled_48_130_d23", (40, 41, 48), 130, (3, 3), (1, 1), (2, 3), (2, 2, 3, 3), True, True)),
+    ("conv2d_s8_unitgemm", 40, ("unit_17_33_d2", (40, 41, 17), 33, (3, 3), (1, 1), (2, 2), (2, 2, 2, 2), True, True)),
+    ("conv2d_s8_unitgemm", 60, ("unit_64_130_s3", (30, 31, 64), 130, (3, 3), (3, 3), (1, 1), (0, 0, 0, 0), True, False)),
+    ("conv2d_s8_unitgemm", 40, ("unit_61_70_k2x5", (25, 27, 61), 70, (2, 5), (1, 1), (1, 1), (0, 1, 2, 2), False, True)),
+    ("conv2d_s8_pwgemm", 60, ("pw_320_96", (14, 14, 320), 96, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, True)),
+    ("conv2d_s8_pwgemm", 150, ("pw_960_163", (7, 7, 960), 163, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, False)),
+    ("conv2d_s8_pwgemm", 30, ("pw_300_257", (31, 17, 300), 257, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), False, True)),
+    ("conv2d_s8", 220, ("direct_16_32_s3", (80, 112, 16), 32, (3, 3), (3, 3), (1, 1), (1, 1, 1, 1), True, True)),
+    ("conv2d_s8", 60, ("direct_12_80", (80, 81, 12), 80, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, True)),
+    ("conv2d_s8", 60, ("direct_272_20", (60, 62, 272), 20, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True, False)),
 ]

@@ -5,14 +5,16 @@ import ctypes
 import numpy as np
 import pytest
 
-from cases import CONFIG1, CONV_CASES, DW_CASES, GEMM_CASES, POINTWISE_MANY_PIXELS, WIDE_ROWS, WINDOW_GEMM_CASES, TILED_MANY_PIXELS, STEM_CASES, TILED_CASES, UNIT_CASES, WALK_CASES, every_sum_image, rng_int8, typical_shift
+from cases import (CONFIG1, CONV_CASES, DW_CASES, GEMM_CASES, OTHER_KERNELS, POINTWISE_MANY_PIXELS, STEM_CASES, TILED_CASES,
+                   TILED_MANY_PIXELS, UNIT_CASES, WALK_CASES, WALK_LARGE, WALK_ODD_PITCH, WALK_RESIDUAL, WIDE_ROWS, WINDOW_GEMM_CASES,
+                   every_sum_image, rng_int8, typical_shift)
 from gpu_util import announce, espdl, to_dev, to_host
 
 pytestmark = pytest.mark.gpu
 
 
 def _run_conv_s8(oracle, x, f, bias, shift, k, stride, dil, pads, relu, depthwise=False, half_even=False, lut=None,
-                 residual_seed=None):
+                 residual_seed=None, kernel=None):
     m = espdl()
     act = m.capi.RELU if relu else m.capi.LINEAR
     rm = m.capi.ROUND_HALF_EVEN if half_even else m.capi.ROUND_HALF_UP
@@ -26,9 +28,39 @@ def _run_conv_s8(oracle, x, f, bias, shift, k, stride, dil, pads, relu, depthwis
     if residual_seed is not None:  # Conv -> Add in one launch
         residual = rng_int8(np.random.default_rng(residual_seed), want.shape)
         want = oracle.add_s8(want, residual)
-    got = m.conv2d(to_dev(x), to_dev(f), to_dev(bias), to_dev(shift), k, stride, dil, pads, depthwise=depthwise,
-                   activation=act, round_mode=rm, lut=to_dev(lut), residual=to_dev(residual))
+    x, f, shift, lut, residual = (to_dev(t) for t in (x, f, shift, lut, residual))
+    if kernel is not None:
+        assert m.capi.conv2d_s8_kernel(x, f, shift, k, stride, dil, pads, act, rm, lut, None, residual) == kernel
+    got = m.conv2d(x, f, to_dev(bias), shift, k, stride, dil, pads, depthwise=depthwise, activation=act, round_mode=rm, lut=lut,
+                   residual=residual)
     return to_host(got), want
+
+
+def _run_conv_slices(oracle, x, f, bias, shift, k, stride, dil, pads, relu, kernel, in_extra, lut=None, with_residual=False, half_even=False):
+    """Operands that are channel slices of wider tensors; the channels beside the result have to stay as they are."""
+    import torch
+    m = espdl()
+    c, oc = x.shape[3], f.shape[0]
+    act, rm = m.capi.RELU if relu else m.capi.LINEAR, m.capi.ROUND_HALF_EVEN if half_even else m.capi.ROUND_HALF_UP
+    want = oracle.conv2d_s8(x, f, bias, shift, k, stride, dil, pads, oracle.RELU if relu else oracle.LINEAR,
+                            oracle.ROUND_HALF_EVEN if half_even else oracle.ROUND_HALF_UP)
+    want = oracle.lut_s8(want, lut) if lut is not None else want
+    wide_in = torch.full(x.shape[:3] + (c + in_extra,), 77, dtype=torch.int8, device="cuda")
+    wide_in[..., 16:16 + c] = to_dev(x)
+    wide_out = torch.full(want.shape[:3] + (oc + 32,), -9, dtype=torch.int8, device="cuda")
+    residual = None
+    if with_residual:
+        values = rng_int8(np.random.default_rng(19), want.shape)
+        want = oracle.add_s8(want, values)
+        wide_res = torch.full(want.shape[:3] + (oc + 16,), 5, dtype=torch.int8, device="cuda")
+        wide_res[..., 16:] = to_dev(values)
+        residual = wide_res[..., 16:]
+    src, dst, f, shift, lut = wide_in[..., 16:16 + c], wide_out[..., 16:16 + oc], to_dev(f), to_dev(shift), to_dev(lut)
+    assert m.capi.conv2d_s8_kernel(src, f, shift, k, stride, dil, pads, act, rm, lut, dst, residual) == kernel
+    m.conv2d(src, f, to_dev(bias), shift, k, stride, dil, pads, activation=act, round_mode=rm, lut=lut, residual=residual, out=dst)
+    got = to_host(wide_out)
+    np.testing.assert_array_equal(got[..., 16:16 + oc], want)
+    assert (got[..., :16] == -9).all() and (got[..., 16 + oc:] == -9).all()
 
 
 def _conv_inputs(case, seed, n, per_channel):
@@ -242,47 +274,97 @@ def test_conv2d_s8_walk_stem(oracle, case, flavour):
     assert (got[..., :4] == -9).all() and (got[..., 4 + oc:] == -9).all()
 
 
+TABLE = np.array([(i * 109 + 37) & 0xFF for i in range(256)], dtype=np.uint8).view(np.int8)
+
+
 @pytest.mark.parametrize("case", WALK_CASES, ids=lambda c: c[1][0])
-@pytest.mark.parametrize("flavour", ["per_channel", "low_shifts", "lut_residual", "general_epilogue", "slices"])
+@pytest.mark.parametrize("flavour", ["per_channel", "low_shifts", "lut", "general_epilogue", "slices"])
 def test_conv2d_s8_walk(oracle, case, flavour):
-    """The kernel that walks down the image: right shifts and left shifts of the short epilogue, a table and a residual
-    operand, the general shift-and-round form, and operands that are channel slices of wider tensors (whose other
-    channels stay as they are)."""
-    import torch
+    """The kernel that walks down the image: right shifts and left shifts of the short epilogue, a table, the general
+    shift-and-round form, and operands that are channel slices of wider tensors (whose other channels stay as they are)."""
     announce(f"conv2d_s8 walk {case[1][0]} {flavour}")
     x, f, bias, shift, k, stride, dil, pads, relu = _conv_inputs(case[1], 263, case[0], True)
-    kw = {}
+    lut = None
     if flavour == "low_shifts":
         shift = (np.arange(shift.size) % 5 + 6).astype(np.int32)
         f = (f >> 3).astype(np.int8)
-    if flavour == "lut_residual":
-        kw["lut"] = np.array([(i * 109 + 37) & 0xFF for i in range(256)], dtype=np.uint8).view(np.int8)
-        kw["residual_seed"] = 17
-        relu = False
+    if flavour == "lut":
+        lut, relu = TABLE, False
     if flavour == "general_epilogue":
         shift = np.array(shift, dtype=np.int32)
         shift[::3] = 0
         shift[1::5] = 33
     oracle.set_threads(16)
-    if flavour != "slices":
-        got, want = _run_conv_s8(oracle, x, f, bias, shift, k, stride, dil, pads, relu, **kw)
-        np.testing.assert_array_equal(got, want)
+    if flavour == "slices":
+        _run_conv_slices(oracle, x, f, bias, shift, k, stride, dil, pads, relu, "conv2d_s8_walk", 48)
         return
-    m = espdl()
-    c, oc = x.shape[3], f.shape[0]
-    want = oracle.conv2d_s8(x, f, bias, shift, k, stride, dil, pads, oracle.RELU if relu else oracle.LINEAR, oracle.ROUND_HALF_UP)
-    residual = rng_int8(np.random.default_rng(19), want.shape)
-    want = oracle.add_s8(want, residual)
-    wide_in = torch.full(x.shape[:3] + (c + 48,), 77, dtype=torch.int8, device="cuda")
-    wide_in[..., 16:16 + c] = to_dev(x)
-    wide_out = torch.full(want.shape[:3] + (oc + 32,), -9, dtype=torch.int8, device="cuda")
-    wide_res = torch.full(want.shape[:3] + (oc + 16,), 5, dtype=torch.int8, device="cuda")
-    wide_res[..., 16:] = to_dev(residual)
-    m.conv2d(wide_in[..., 16:16 + c], to_dev(f), to_dev(bias), to_dev(shift), k, stride, dil, pads,
-             activation=m.capi.RELU if relu else m.capi.LINEAR, residual=wide_res[..., 16:], out=wide_out[..., 16:16 + oc])
-    got = to_host(wide_out)
-    np.testing.assert_array_equal(got[..., 16:16 + oc], want)
-    assert (got[..., :16] == -9).all() and (got[..., 16 + oc:] == -9).all()
+    got, want = _run_conv_s8(oracle, x, f, bias, shift, k, stride, dil, pads, relu, lut=lut, kernel="conv2d_s8_walk")
+    np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("case", WALK_RESIDUAL, ids=lambda c: c[1][0])
+@pytest.mark.parametrize("flavour", ["residual", "lut_residual", "slices"])
+def test_conv2d_s8_walk_residual(oracle, case, flavour):
+    announce(f"conv2d_s8 walk with a residual operand {case[1][0]} {flavour}")
+    x, f, bias, shift, k, stride, dil, pads, relu = _conv_inputs(case[1], 263, case[0], True)
+    oracle.set_threads(16)
+    if flavour == "slices":
+        _run_conv_slices(oracle, x, f, bias, shift, k, stride, dil, pads, relu, "conv2d_s8_walk", 48, with_residual=True)
+        return
+    lut = TABLE if flavour == "lut_residual" else None
+    got, want = _run_conv_s8(oracle, x, f, bias, shift, k, stride, dil, pads, relu and lut is None, lut=lut, residual_seed=17,
+                             kernel="conv2d_s8_walk")
+    np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("case", WALK_ODD_PITCH, ids=lambda c: c[1][0])
+@pytest.mark.parametrize("flavour", ["per_channel", "lut"])
+def test_conv2d_s8_walk_odd_pitch(oracle, case, flavour):
+    """Channels that are a multiple of 4 in pixels of an odd number of bytes."""
+    announce(f"conv2d_s8 walk odd pitch {case[1][0]} {flavour}")
+    x, f, bias, shift, k, stride, dil, pads, relu = _conv_inputs(case[1], 269, case[0], True)
+    oracle.set_threads(16)
+    _run_conv_slices(oracle, x, f, bias, shift, k, stride, dil, pads, relu, "conv2d_s8_walk", 21, lut=TABLE if flavour == "lut" else None)
+
+
+@pytest.mark.parametrize("case", WALK_LARGE, ids=lambda c: c[1][0])
+def test_conv2d_s8_walk_large_results(oracle, case):
+    announce(f"conv2d_s8 walk large {case[1][0]}")
+    x, f, bias, shift, k, stride, dil, pads, relu = _conv_inputs(case[1], 277, case[0], True)
+    oracle.set_threads(16)
+    got, want = _run_conv_s8(oracle, x, f, bias, shift, k, stride, dil, pads, relu, kernel="conv2d_s8_walk")
+    assert want.size > 16 << 20
+    np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("kernel,n,case", OTHER_KERNELS, ids=[c[2][0] for c in OTHER_KERNELS])
+@pytest.mark.parametrize("flavour", ["per_channel", "low_shifts", "lut", "lut_residual", "general_epilogue", "half_even", "slices"])
+def test_conv2d_s8_other_kernels(oracle, kernel, n, case, flavour):
+    """Each kernel beside the walk where it is the one that is taken: the short epilogue with and without left shifts, a table, a
+    table and a residual operand, the general form, half even, channel slices."""
+    announce(f"conv2d_s8 {kernel} {case[0]} {flavour}")
+    if kernel == "conv2d_s8_stem" and flavour in ("lut_residual", "slices"):
+        pytest.skip("a residual operand or slices take the layer to another kernel")
+    x, f, bias, shift, k, stride, dil, pads, relu = _conv_inputs(case, 283, n, True)
+    kw = {}
+    if flavour == "low_shifts":
+        shift = (np.arange(shift.size) % 5 + 6).astype(np.int32)
+        f = (f >> 3).astype(np.int8)
+    if flavour in ("lut", "lut_residual"):
+        kw["lut"], relu = TABLE, False
+    if flavour == "lut_residual":
+        kw["residual_seed"] = 17
+    if flavour == "general_epilogue":
+        shift[::3] = 0
+        shift[1::5] = 33
+    if flavour == "half_even":
+        kw["half_even"] = True
+    oracle.set_threads(16)
+    if flavour == "slices":
+        _run_conv_slices(oracle, x, f, bias, shift, k, stride, dil, pads, relu, kernel, 48)
+        return
+    got, want = _run_conv_s8(oracle, x, f, bias, shift, k, stride, dil, pads, relu, kernel=kernel, **kw)
+    np.testing.assert_array_equal(got, want)
 
 
 @pytest.mark.parametrize("case", WINDOW_GEMM_CASES, ids=lambda c: c[0])
