@@ -44,6 +44,7 @@ STEM_CASES = [
     ("s3_20x200_k3s2_nopad_oc16", (20, 200, 3), 16, (3, 3), (2, 2), (1, 1), (0, 0, 0, 0), True, True),
     ("s2_24x24_k3s3p2_oc7", (24, 24, 2), 7, (3, 3), (3, 3), (1, 1), (2, 2, 2, 2), True, False),
     ("s3_1x700_k3s2_oc16", (1, 700, 3), 16, (1, 3), (1, 2), (1, 1), (0, 0, 1, 1), True, True),
+    ("s3_64x64_k2s4_oc64", (64, 64, 3), 64, (2, 2), (4, 4), (1, 1), (0, 0, 0, 0), False, True),
 ]
 
 # Pointwise products with at most 128 input channels over enough pixels to fill the device (3 x 80 x 80: the routes

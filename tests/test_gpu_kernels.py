@@ -228,14 +228,16 @@ def test_conv2d_s8_channel_units(oracle, case, flavour):
 # one to four of them, both step heights, every count of filter tiles, ragged last strips and rows, padding on every side.
 # (batch, (name, (H, W, Cin), Cout, k, stride, dilation, pads, relu, bias))
 STEM_WALK_CONV = [
-    (3, ("rgb_k3s2_tailpad", (65, 112, 3), 16, (3, 3), (2, 2), (1, 1), (0, 1, 0, 1), True, True)),
-    (2, ("rgb_k3s2_32", (50, 80, 3), 32, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), True, True)),
-    (2, ("rgb_k3s2_64", (37, 96, 3), 64, (3, 3), (2, 2), (1, 1), (1, 0, 1, 0), False, True)),
-    (70, ("rgb_k3s2_nopad_narrow", (33, 16, 3), 16, (3, 3), (2, 2), (1, 1), (0, 0, 0, 0), True, False)),
-    (2, ("four_k3s1", (29, 40, 4), 16, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
-    (5, ("two_k4x5_s1", (23, 56, 2), 32, (4, 5), (1, 1), (1, 1), (3, 1, 2, 2), True, True)),
-    (4, ("gray_k4x7_s2", (40, 80, 1), 16, (4, 7), (2, 2), (1, 1), (2, 2, 3, 3), True, True)),
-    (9, ("rgb_k2_s4", (64, 64, 3), 64, (2, 2), (4, 4), (1, 1), (0, 0, 0, 0), False, True)),
+    (30, ("rgb_k3s2_tailpad", (65, 112, 3), 16, (3, 3), (2, 2), (1, 1), (0, 1, 0, 1), True, True)),
+    (30, ("rgb_k3s2_32", (50, 80, 3), 32, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), True, True)),
+    (30, ("rgb_k3s2_64", (37, 96, 3), 64, (3, 3), (2, 2), (1, 1), (1, 0, 1, 0), False, True)),
+    (400, ("rgb_k3s2_nopad_narrow", (33, 16, 3), 16, (3, 3), (2, 2), (1, 1), (0, 0, 0, 0), True, False)),
+    (50, ("four_k3s1", (29, 40, 4), 16, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
+    (9, ("two_k4x5_s1", (23, 56, 2), 32, (4, 5), (1, 1), (1, 1), (3, 1, 2, 2), True, True)),
+    (30, ("gray_k4x7_s2", (40, 80, 1), 16, (4, 7), (2, 2), (1, 1), (2, 2, 3, 3), True, True)),
+    (40, ("four_k3s2_64", (45, 52, 4), 64, (3, 3), (2, 2), (1, 1), (1, 1, 1, 1), False, True)),
+    (60, ("rgb_k3_s32_32", (70, 64, 3), 32, (3, 3), (3, 2), (1, 1), (1, 1, 1, 1), True, True)),
+    (90, ("two_k2x3_s2_16", (47, 72, 2), 16, (2, 3), (2, 2), (1, 1), (0, 1, 1, 0), True, False)),
 ]
 
 
@@ -260,15 +262,17 @@ def test_conv2d_s8_walk_stem(oracle, case, flavour):
         shift[::3], shift[1::5] = 0, 33
     oracle.set_threads(16)
     if flavour != "out_slice":
-        got, want = _run_conv_s8(oracle, x, f, bias, shift, k, stride, dil, pads, relu, **kw)
+        got, want = _run_conv_s8(oracle, x, f, bias, shift, k, stride, dil, pads, relu, kernel="conv2d_s8_walk_stem", **kw)
         np.testing.assert_array_equal(got, want)
         return
     m = espdl()
     oc = f.shape[0]
     want = oracle.conv2d_s8(x, f, bias, shift, k, stride, dil, pads, oracle.RELU if relu else oracle.LINEAR, oracle.ROUND_HALF_UP)
     wide = torch.full(want.shape[:3] + (oc + 20,), -9, dtype=torch.int8, device="cuda")
-    m.conv2d(to_dev(x), to_dev(f), to_dev(bias), to_dev(shift), k, stride, dil, pads,
-             activation=m.capi.RELU if relu else m.capi.LINEAR, out=wide[..., 4:4 + oc])
+    act = m.capi.RELU if relu else m.capi.LINEAR
+    x, f, shift, dst = to_dev(x), to_dev(f), to_dev(shift), wide[..., 4:4 + oc]
+    assert m.capi.conv2d_s8_kernel(x, f, shift, k, stride, dil, pads, act, out=dst) == "conv2d_s8_walk_stem"
+    m.conv2d(x, f, to_dev(bias), shift, k, stride, dil, pads, activation=act, out=dst)
     got = to_host(wide)
     np.testing.assert_array_equal(got[..., 4:4 + oc], want)
     assert (got[..., :4] == -9).all() and (got[..., 4 + oc:] == -9).all()
@@ -941,7 +945,7 @@ def test_conv2d_s16_on_int8(oracle, case, table_size):
 # the middle, strips across images, missing, one-sided and wide padding, sums at both ends of their range.
 # (name, (N, H, W, C), OC, pads, relu, half_even, lowest and highest shift, values)
 X8_WALK = [
-    ("16_16", (200, 40, 40, 16), 16, (1, 1, 1, 1), True, False, 24, 28, "random"),
+    ("16_16", (400, 40, 40, 16), 16, (1, 1, 1, 1), True, False, 24, 28, "random"),
     ("32_24_nopad", (90, 44, 43, 32), 24, (0, 0, 0, 0), False, False, 20, 28, "random"),
     ("48_40_tailpad_low", (60, 33, 47, 48), 40, (0, 2, 0, 1), True, False, 9, 20, "random"),
     ("64_64", (110, 20, 41, 64), 64, (1, 1, 1, 1), True, False, 24, 28, "random"),
@@ -1614,9 +1618,10 @@ def test_mbconv_s8_walk(oracle, case, flavour):
         res = rng_int8(rng, cur.shape)
         cur = oracle.add_s8(cur, oracle.requantize_s8(res, res_shift, 0) if res_shift else res)
     dev = lambda t: tuple(to_dev(a) for a in t)  # noqa: E731
-    got = m.mbconv_s8(to_dev(x), dev(ex), dev(dw), dev(pj), (3, 3), (stride, stride), (1, 1), pads, (True, False, False),
-                      residual=to_dev(res), residual_shift=res_shift,
-                      round_mode=m.capi.ROUND_HALF_EVEN if half_even else m.capi.ROUND_HALF_UP)
+    args = to_dev(x), dev(ex), dev(dw), dev(pj), (3, 3), (stride, stride), (1, 1), pads, (True, False, False)
+    kw = dict(residual=to_dev(res), residual_shift=res_shift, round_mode=m.capi.ROUND_HALF_EVEN if half_even else m.capi.ROUND_HALF_UP)
+    assert m.capi.mbconv_s8_kernel(*args, **kw) == "mbconv_s8_walk"
+    got = m.mbconv_s8(*args, **kw)
     np.testing.assert_array_equal(to_host(got), cur)
 
 
@@ -1666,9 +1671,11 @@ def test_mbconv_s8_walk_stem(oracle, case, flavour):
     cur = oracle.depthwise_s8(cur, dw[0], dw[1], dw[2], (3, 3), (1, 1), (1, 1), pads, oracle.RELU, rm_o)
     cur = oracle.conv2d_s8(cur, pj[0], pj[1], pj[2], (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), oracle.LINEAR, rm_o)
     dev = lambda t: tuple(to_dev(a) for a in t)  # noqa: E731
-    got = m.mbconv_s8(to_dev(x), dev(ex), dev(dw), dev(pj), (3, 3), (1, 1), (1, 1), pads, (False, True, False),
-                      round_mode=m.capi.ROUND_HALF_EVEN if half_even else m.capi.ROUND_HALF_UP,
-                      clip_expand=(5, 90) if clip else None, expand_conv=(ek, es, ep))
+    args = to_dev(x), dev(ex), dev(dw), dev(pj), (3, 3), (1, 1), (1, 1), pads, (False, True, False)
+    kw = dict(round_mode=m.capi.ROUND_HALF_EVEN if half_even else m.capi.ROUND_HALF_UP, clip_expand=(5, 90) if clip else None,
+              expand_conv=(ek, es, ep))
+    assert m.capi.mbconv_s8_kernel(*args, **kw) == "mbconv_s8_walk_stem"
+    got = m.mbconv_s8(*args, **kw)
     np.testing.assert_array_equal(to_host(got), cur)
 
 
