@@ -703,8 +703,14 @@ WalkCut walk_cut(const WalkArgs &a, const WalkLaunch &l, int per_cu)
 // alike they add up in part.  The constants are a fit over 780 random layers of 1 to 260 MB (1641 builds, 8 % root mean
 // square).  Filter chunks of one pixel are written by different workgroups: past what the caches hold, their pieces of a
 // line reach memory one by one (188 x 63 x 88 x 32 -> 96, 1 x 1: 40 us as one chunk, 66 as pieces of 64 bytes, 81 of 32).
+// Many chunks over few pixels: each has eight workgroups at least, idle ones among them, and every workgroup fetches its filters
+// before it starts, in as many turns as there are more workgroups than the CUs hold; the workgroups of the chunks beyond 16 cost
+// 1.5 ns each (120 channels of 40 pixels -> 6625, 1 x 1: 8.4 us, 4.7 on the pointwise GEMM kernel; 4 x 32 x 96 -> 6576, 3 x 3 at
+// stride 2, batch 2: 62, 8 on the narrow one; 1450 layers of 200 to 8192 filters: 0.16 root mean square, 0.21 before).
 // RAW builds under 3 x 3 pass their pieces through registers step by step, which takes a fifth longer; those of 11 and 12 units of
-// a pixel and the ones of 15 and 16 without RAW spill 24 to 35 registers besides (1600 and 60 layers).
+// a pixel and the ones of 15 and 16 without RAW spill 24 to 35 registers besides (1600 and 60 layers).  At stride 2 the builds of 6
+// units and more, 5 under 5 x 5, take more than 256 registers: one wavefront per SIMD, 1.4 and 2.3 us more whatever the layer's size
+// (52 layers of 5 to 82 us; 3 x 3 counts 1, for the unit kernel's line lies as far below its time at 128 channels).
 template <int KH, int S, int CU, int NT, bool RES, bool RAW>
 float walk_us(const WalkArgs &a, const WalkLaunch &l)
 {
@@ -717,13 +723,17 @@ float walk_us(const WalkArgs &a, const WalkLaunch &l)
     const int busy = (c.rows_total + c.per_group - 1) / c.per_group * c.chunks;
     const float waves = (float)(std::min(kPerCu, (busy + l.cus - 1) / l.cus) * Shape::W) * 0.25f; // of a SIMD
     const float cycles = waves * (14.4f * (KH * Shape::KS * NT * Shape::PT) + 86.f * (NT * Shape::PT) + 110.f + 1.95f * (Shape::kSlot / 16));
-    const float walk = steps * cycles * (1.f / 2100.f), memory = (float)((long long)a.in_bytes + l.out_bytes + a.res_bytes) * (1.f / 9e6f);
-    float us = 2.9f + 0.027f * Shape::kFilterUnits + (S == 2 ? 0.25f : 0.f) - (Shape::W == 8 ? 0.36f : 0.f) +
+    const float resident = (float)(l.cus * kPerCu);
+    const float walk = steps * cycles * (1.f / 2100.f) * std::max(1.f, (float)busy / resident), memory = (float)((long long)a.in_bytes + l.out_bytes + a.res_bytes) * (1.f / 9e6f);
+    const float set_up = 2.9f + 0.027f * Shape::kFilterUnits + (S == 2 ? 0.25f : 0.f) - (Shape::W == 8 ? 0.36f : 0.f);
+    float us = set_up * std::max(1.f, (float)(c.n_groups * c.chunks) / resident) + 1.5e-3f * (float)(c.n_groups * std::max(0, c.chunks - 16)) +
         std::cbrt((walk * std::sqrt(walk) + memory * std::sqrt(memory)) * (walk * std::sqrt(walk) + memory * std::sqrt(memory)));
     if (c.chunks > 1 && l.out_bytes > 80000000)
         us += 12e-6f * (float)l.out_bytes / (float)(16 * NT);
     if constexpr (RAW)
         return KH == 1 ? us + 0.1f : us * (CU <= 3 ? 1.15f : (CU <= 10 ? 1.2f : 1.5f)) + 0.3f;
+    if (S == 2 && ((KH == 3 && CU >= 6) || (KH == 5 && CU >= 5)))
+        us += KH == 3 ? 1.f : 2.3f;
     return KH == 3 && S == 1 && CU >= 15 ? 1.5f * us : us;
 }
 

@@ -178,8 +178,11 @@ DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *
 
 // The walking kernel takes what it has a build for where its expected time is the smaller one.  The estimates lie 8 to 10 %
 // off either way, and of two such the smaller one is more often the one that is too small, so 5 x 5 has to win by a margin;
-// the larger kernels take up to twice the unit kernel's line, the direct one three quarters of it where it writes long rows
-// that no other writes whole (channels that are no multiple of 4: 112 x 23 x 112 x 22 -> 158, 1 x 1, 23.1 against 31.8 us).  3076 random layers of 16 to 256
+// the direct kernel takes up to twice the unit kernel's line, the tiled one, which lost to the walk on 179 of 181 layers, any
+// multiple of it on small images (96 channels of 4 x 1 pixels -> 4969, 3 x 3, batch 286: 402 us, 30 by the walk, the line 15).
+// Where channels are no multiple of 4 the direct
+// kernel, which writes whole rows, takes less than the line: 112 x 23 x 112 x 22 -> 158, 1 x 1, 23.1 us against 31.8 by the walk;
+// beyond 256 filters (62 layers) the walk wins up to 0.85 of the line.  3076 random layers of 16 to 256
 // channels in 1 image to 400 MB, each timed on both sides with operands that change from launch to launch: 0.88 of the other
 // kernels' time in the geometric mean on channels that are a multiple of 4, 0.80 on others (the better one of each pair: 0.87,
 // 0.78); 1.7 % of all are slower by more than 5 % than on the other kernel, 0.9 % by more than 10.  (On operands that lie in the
@@ -187,10 +190,14 @@ DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *
 // 8 % of its dense layers' time.)
 bool dense_s8_walks(const espdl::ConvGeom &g, DenseRoute other, float walk, float narrow, float gemm)
 {
+    if (((g.in_c | g.in_pitch) & 3) != 0) {
+        const float direct = g.out_c < 96 ? 1.f : (g.out_c <= 256 ? 0.7f : 0.85f);
+        return walk < std::min(1.05f * narrow, gemm * (other == DENSE_PWGEMM ? 0.9f : (other == DENSE_DIRECT ? direct : 1.f)));
+    }
     const bool few = other == DENSE_NARROW || other == DENSE_UNITGEMM;
-    if (((g.in_c | g.in_pitch) & 3) != 0)
-        return walk < std::min(1.05f * narrow, gemm * (other == DENSE_PWGEMM ? 0.9f : (other == DENSE_DIRECT && g.out_c >= 96 ? 0.7f : 1.f)));
-    return walk * (g.k_h == 1 ? 1.f : (g.k_h == 3 ? 1.02f : 1.1f)) < std::min(narrow, gemm * (few ? 1.15f : 1.4f));
+    if (other == DENSE_TILED)
+        return walk < 1e30f; // (there is a build)
+    return walk * (g.k_h == 1 ? 1.f : (g.k_h == 3 ? 1.02f : 1.1f)) < std::min(narrow, gemm * (few ? 1.15f : 2.f));
 }
 
 // Of all kernels.  Two take every layer that they apply to: the classifier's, and the walk of the first-layer kernel's layers

@@ -143,6 +143,11 @@ def test_dense_layers_go_to_the_faster_kernel():
             ((43, 75, 11, 16), 240, 5, 2, b"conv2d_s8_unitgemm"),  # 7.8, 8.9
             ((9, 13, 43, 16), 64, 3, 1, b"conv2d_s8_narrow"),      # 3.3, 3.9
             ((1, 20, 20, 240), 16, 3, 1, b"conv2d_s8_narrow"),     # 3.9, 9.0
+            ((15, 42, 21, 84), 24, 3, 2, b"conv2d_s8_narrow"),     # 4.3, 6.3
+            ((1, 1, 40, 120), 6625, 1, 1, b"conv2d_s8_pwgemm"),    # 4.7, 8.4
+            ((2, 4, 32, 96), 6576, 3, 2, b"conv2d_s8_narrow"),     # 8.1, 62
+            ((286, 4, 1, 96), 4969, 3, 1, b"conv2d_s8_walk"),      # 30, 402
+            ((364, 5, 1, 16), 6078, 5, 1, b"conv2d_s8_walk"),      # 45, 340
             ((1, 56, 56, 64), 64, 3, 1, b"conv2d_s8_walk"),        # 4.1, 4.2
             ((82, 15, 19, 16), 171, 1, 1, b"conv2d_s8_walk"),      # 4.9, 7.7
             ((39, 8, 8, 116), 107, 1, 1, b"conv2d_s8_walk"),       # 3.2, 4.4
