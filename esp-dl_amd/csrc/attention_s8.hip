@@ -24,8 +24,8 @@
 //      on its way into LDS, and multiplied by the probabilities, a half of the head's channels per wavefront of a pair.
 //      A tile's operand-A row m is channel (m / 4) * 4 HT + 4 t + m % 4 of the head, so a lane ends with neighbouring
 //      channels of one position.
-// Bound by latency: the serial additions (12 cycles each) and the walk through LDS between the steps, two workgroups on
-// a compute unit at most.  400 positions, 64 images x heads of 32 + 32 + 64 channels take 15.4 us where the operators
+// Not bound by memory or the matrix pipe; two workgroups fit on a compute unit.  The serial additions, 12 cycles each, are 2 us of
+// a launch with 400 positions; how the rest divides between the steps and their walk through LDS has not been measured.  400 positions, 64 images x heads of 32 + 32 + 64 channels take 15.4 us where the operators
 // one by one took 117 us.  Four wavefronts that each owned 16 queries and re-read their scores from LDS took 18.3 us
 // (13.3 us for a single image, now 11.4 us), a ninth wavefront that only adds 17.7 us.
 #include "conv_window.h"

@@ -14,7 +14,8 @@
 // Bound by the matrix pipe and the epilogue, the table's lookups among it.  Against the tiled kernel, which cuts the filters
 // into bytes again in every workgroup and meets a barrier per 64 products: 80 x 80 x 64 -> 64 with a table, batch 64, 51
 // against 87 us, 40 x 40 21 against 27; 80 x 80 x 32 -> 32 without one 24 against 33; 40 x 40 x 128 -> 128, batch 32, 29
-// against 40.
+// against 40.  Half even takes the general epilogue, which the estimate does not know of: of 350 random layers two take more than
+// 5 % longer than on the tiled kernel.
 #include "conv2d_s8_walk_kernel.h"
 
 namespace espdl {

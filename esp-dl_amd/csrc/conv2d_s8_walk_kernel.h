@@ -31,7 +31,7 @@
 // the kernels such layers took before, us: 3 x 3 over 160 x 160 x 32 -> 32 47 -> 31, the same with a residual operand
 // 77 -> 41; 3 x 3 at stride 2 over 320 x 320 x 16 -> 32 61 -> 38, 160 x 160 x 64 -> 64 49 -> 35; 3 x 3 over
 // 80 x 80 x 64 -> 64 28 -> 22, 128 -> 128 90 -> 61; 1 x 1 over 160 x 160 x 32 -> 64 51 -> 37, 80 x 80 x 256 -> 256
-// 77 -> 51; 5 x 5 over 80 x 80 x 64 -> 64 58 -> 44; 56 x 56 x 64 -> 64, 3 x 3, batch 256 45 -> 39.
+// 77 -> 51; 5 x 5 over 80 x 80 x 64 -> 64 58 -> 44; 56 x 56 x 64 -> 64, 3 x 3, batch 256 42 -> 34.
 #pragma once
 
 #include <algorithm>
@@ -194,9 +194,10 @@ __global__ __launch_bounds__((64 * WalkShape<KH, S, CU, NT, RES>::W), 2) void co
     };
 
     // ---- requests of what the set-up needs: one filter's bias and shift per lane, the workgroup's filters straight into
-    // LDS (a quarter per wavefront) in operand-A order
+    // LDS (a part per wavefront) in operand-A order
     const bool has_lut = a.lut != nullptr;
-    // (3 x 3 under four filter tiles, 56 x 56 x 64 -> 64 at batch 256: the choice alone costs 33.1 -> 34.9 us, its branches
+    // (in 500 random 3 x 3 layers of 16 MB at most the choice under three and four filter tiles too gains 0.6 % in the mean, in 400 of one
+    // and two it gives 0.5 %; but 56 x 56 x 64 -> 64 at batch 256, whose results it does not concern, pays 33.1 -> 34.9 us, its branches
     // part the epilogue's instructions from the next step's; one unit, 62 x 104 x 16 -> 64 at batch 19: 7.8 -> 7.0 us all the
     // same; beyond 8 units registers spill)
     const int through = KH == 1 || (KH == 3 && CU <= 8 && (NT <= 2 || CU == 1)) ? a.through : 0;
@@ -724,7 +725,8 @@ float walk_us(const WalkArgs &a, const WalkLaunch &l)
     const float waves = (float)(std::min(kPerCu, (busy + l.cus - 1) / l.cus) * Shape::W) * 0.25f; // of a SIMD
     const float cycles = waves * (14.4f * (KH * Shape::KS * NT * Shape::PT) + 86.f * (NT * Shape::PT) + 110.f + 1.95f * (Shape::kSlot / 16));
     const float resident = (float)(l.cus * kPerCu);
-    const float walk = steps * cycles * (1.f / 2100.f) * std::max(1.f, (float)busy / resident), memory = (float)((long long)a.in_bytes + l.out_bytes + a.res_bytes) * (1.f / 9e6f);
+    const float walk = steps * cycles * (1.f / 2100.f) * std::max(1.f, (float)busy / resident);
+    const float memory = (float)((long long)a.in_bytes + l.out_bytes + a.res_bytes) * (1.f / 9e6f);
     const float set_up = 2.9f + 0.027f * Shape::kFilterUnits + (S == 2 ? 0.25f : 0.f) - (Shape::W == 8 ? 0.36f : 0.f);
     float us = set_up * std::max(1.f, (float)(c.n_groups * c.chunks) / resident) + 1.5e-3f * (float)(c.n_groups * std::max(0, c.chunks - 16)) +
         std::cbrt((walk * std::sqrt(walk) + memory * std::sqrt(memory)) * (walk * std::sqrt(walk) + memory * std::sqrt(memory)));

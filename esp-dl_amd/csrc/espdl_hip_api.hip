@@ -180,14 +180,13 @@ DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *
 // off either way, and of two such the smaller one is more often the one that is too small, so 5 x 5 has to win by a margin;
 // the direct kernel takes up to twice the unit kernel's line, the tiled one, which lost to the walk on 179 of 181 layers, any
 // multiple of it on small images (96 channels of 4 x 1 pixels -> 4969, 3 x 3, batch 286: 402 us, 30 by the walk, the line 15).
-// Where channels are no multiple of 4 the direct
-// kernel, which writes whole rows, takes less than the line: 112 x 23 x 112 x 22 -> 158, 1 x 1, 23.1 us against 31.8 by the walk;
-// beyond 256 filters (62 layers) the walk wins up to 0.85 of the line.  3076 random layers of 16 to 256
-// channels in 1 image to 400 MB, each timed on both sides with operands that change from launch to launch: 0.88 of the other
-// kernels' time in the geometric mean on channels that are a multiple of 4, 0.80 on others (the better one of each pair: 0.87,
-// 0.78); 1.7 % of all are slower by more than 5 % than on the other kernel, 0.9 % by more than 10.  (On operands that lie in the
-// L2 caches the other kernels gain more and a margin of 1.2 under 3 x 3 looks right; it costs a detector of 20 frames of 320 x 320
-// 8 % of its dense layers' time.)
+// Where channels are no multiple of 4 the direct kernel, which writes whole rows, takes less than the line: 112 x 23 x 112 x 22 ->
+// 158, 1 x 1, 23.1 us against 31.8 by the walk; beyond 256 filters (62 layers) the walk wins up to 0.85 of the line.
+// 3076 random layers of 16 to 256 channels in 1 image to 400 MB, each timed on both sides with operands that change from launch to
+// launch: 0.88 of the other kernels' time in the geometric mean on channels that are a multiple of 4, 0.80 on others (the better one of
+// each pair: 0.87, 0.78); 1.7 % of all are slower by more than 5 % than on the other kernel, 0.9 % by more than 10; 600 of 200 to 8192
+// filters 0.87, 2.8 % slower by more than 5 %.  (On operands that lie in the L2 caches the other kernels gain more and a margin of 1.2
+// under 3 x 3 looks right; it costs a detector of 20 frames of 320 x 320 8 % of its dense layers' time.)
 bool dense_s8_walks(const espdl::ConvGeom &g, DenseRoute other, float walk, float narrow, float gemm)
 {
     if (((g.in_c | g.in_pitch) & 3) != 0) {

@@ -24,8 +24,10 @@ struct ConvGeom {
 // Whether a kernel's results go through the L2 caches to memory as they are stored.  What lies in the caches when a kernel
 // ends is written back before the next one starts, with nothing else to do; up to half of the eight caches' 32 MB that is
 // most of what was stored.  480 x 6 x 120 x 64 -> 64, 1 x 1 (12 MB stored) 8.3 -> 5.7 us, the blocks on 28 x 28 and 14 x 14
-// images at batch 256 (3 to 6 MB) 4 to 14 % less; 26 MB between 2 % less and 5 % more, 52 MB into a slice 24.6 -> 28.1 us.  With it in the expand + depthwise launches and the narrow kernel
-// too, MobileNetV2 at 160 x 160 and 37 images takes 255 instead of 261 us.
+// images at batch 256 (3 to 6 MB) 4 to 14 % less; 26 MB between 2 % less and 5 % more, 52 MB into a slice 24.6 -> 28.1 us.  With
+// it in the expand + depthwise launches and the narrow kernel too, MobileNetV2 at 160 x 160 and 37 images takes 255 instead of 261 us.
+// The block tile kernels, whose results rarely are larger, have one store form per build and do not ask; the 5 x 5, first-layer, block
+// and int16 walks store plainly and were not measured otherwise.
 inline int writes_through(long long bytes)
 {
     return bytes <= (16ll << 20);
