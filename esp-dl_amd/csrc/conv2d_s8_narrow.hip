@@ -17,6 +17,13 @@
 // Measured against the kernels such layers took before, as nodes of a graph: 56 x 56 x 64 -> 64, 3 x 3, one image 6.0 ->
 // 4.1 us; 13 x 13 x 256 -> 64, 3 x 3 15.5 -> 5.0 us; 13 x 13 x 512 -> 256, 1 x 1 5.6 -> 3.3 us; 1 x 4096 -> 256 6.8 -> 4.7 us;
 // 17 x 27 x 74 -> 11, 3 x 3 at stride 2 31.2 -> 3.8 us.
+// In a chain of launches 1.2 us pass between a kernel's end and the next one's start; the rest is the instructions of ONE
+// wavefront, four cycles each and more, in front of its loads and behind them.  So a lane finds its units by additions (a
+// division takes six quarter-rate multiplications), layers of one tap have builds of their own, the epilogue's operands are
+// requested before the loads and prepared while those are on their way (start values, the vote on the short form), and what is
+// left behind the barrier is sums, a shift and a packed clamp.  14 x 14 x 64 -> 384 3.0 -> 2.4 us, 7 x 7 x 960 -> 160 3.1 -> 2.6,
+// 26 x 26 x 64 -> 64, 3 x 3 3.2 -> 2.8 (launch to launch, kernel itself 2.0 -> 1.5).  What did not help: a reduction split eight
+// ways (2 % at 36 steps, 9 % lost at 4: the loads of one compute unit's wavefronts take turns).
 #include "conv_window.h"
 
 namespace espdl {
@@ -34,10 +41,102 @@ struct NarrowArgs {
     int8_t *out;
     int n_pix, out_c, out_pitch, res_pitch;
     int ksteps, relu, half_even, n_shift, res_shift;
+    unsigned bound; // of a sum of products, see Short4
+    int dense_pixels; // output pixel m of a pointwise layer reads input pixel m
+    // From a lane's unit to its next one, where neither the channels nor the window's columns run out in between, and what
+    // is added where they do.
+    struct {
+        int units, channels, column, row, in, filter;
+        int tap_channels, in_tap, filter_tap;
+        int window_columns, in_row;
+    } step;
     int through; // whole dwords that go through the L2 caches as they are stored
 };
 
-template <int NT, bool SPLIT, bool ALIGNED>
+// The units of one lane in steps of the launch's stride, without a division per unit: where a unit lies follows from where
+// the one before it lay by additions, with one carry from channels to the tap's column and one from there to its row.
+template <bool ALIGNED, bool POINT>
+struct UnitWalk {
+    int u, j16;       // unit, its first channel
+    int ky, kx;       // row and column of its tap in the window, times the dilation
+    int in_off, w_off;
+    int base, iy, ix; // of the pixel's window
+    bool alive;       // the pixel exists
+
+    __device__ __forceinline__ void start(const NarrowArgs &a, int first, int m)
+    {
+        const WindowArgs &w = a.win;
+        alive = m < a.n_pix;
+        u = first;
+        if constexpr (POINT) {
+            // one tap: the window is the pixel
+            j16 = 16 * first;
+            base = (int)((unsigned)m * (unsigned)w.in_pitch);
+            if (a.dense_pixels == 0) { // uniform: a stride
+                const unsigned n = fastdiv((unsigned)m, w.fd_ohw), rem = (unsigned)m - n * w.fd_ohw.d;
+                const unsigned oy = fastdiv(rem, w.fd_ow), ox = rem - oy * w.fd_ow.d;
+                base = (((int)n * w.in_h + (int)oy * w.stride_h) * w.in_w + (int)ox * w.stride_w) * w.in_pitch;
+            }
+            w_off = 16 * first;
+            in_off = base + 16 * first;
+            ky = kx = iy = ix = 0;
+        } else {
+            const unsigned n = fastdiv((unsigned)m, w.fd_ohw), rem = (unsigned)m - n * w.fd_ohw.d;
+            const unsigned oy = fastdiv(rem, w.fd_ow), ox = rem - oy * w.fd_ow.d;
+            const unsigned tap = fastdiv((unsigned)first, w.fd_upt), row = fastdiv(tap, w.fd_kw);
+            j16 = 16 * (first - (int)(tap * w.fd_upt.d));
+            ky = (int)row * w.dil_h;
+            kx = (int)(tap - row * w.fd_kw.d) * w.dil_w;
+            iy = (int)oy * w.stride_h - w.pad_top;
+            ix = (int)ox * w.stride_w - w.pad_left;
+            base = (((int)n * w.in_h + iy) * w.in_w + ix) * w.in_pitch;
+            in_off = base + (ky * w.in_w + kx) * w.in_pitch + j16;
+            w_off = (int)tap * w.in_c + j16;
+        }
+    }
+    __device__ __forceinline__ void advance(const NarrowArgs &a)
+    {
+        u += a.step.units;
+        in_off += a.step.in;
+        w_off += a.step.filter;
+        if constexpr (POINT) {
+            j16 += 16 * a.step.units;
+        } else {
+            j16 += a.step.channels;
+            kx += a.step.column;
+            ky += a.step.row;
+            if (j16 >= a.step.tap_channels) {
+                j16 -= a.step.tap_channels;
+                kx += a.win.dil_w;
+                in_off += a.step.in_tap;
+                w_off += a.step.filter_tap;
+            }
+            if (kx >= a.step.window_columns) {
+                kx -= a.step.window_columns;
+                ky += a.win.dil_h;
+                in_off += a.step.in_row;
+            }
+        }
+    }
+    // Channels the unit holds (<= 0: it does not exist).
+    __device__ __forceinline__ int channels(const NarrowArgs &a) const
+    {
+        return u < a.win.n_units ? a.win.in_c - j16 : 0;
+    }
+    __device__ __forceinline__ v4i pixel(const NarrowArgs &a, __amdgpu_buffer_rsrc_t rsrc) const
+    {
+        bool ok = alive && u < a.win.n_units;
+        if constexpr (!POINT)
+            ok = ok && (unsigned)(iy + ky) < (unsigned)a.win.in_h && (unsigned)(ix + kx) < (unsigned)a.win.in_w;
+        return load16<ALIGNED>(rsrc, ok ? in_off : kParked, a.win.in_bytes);
+    }
+    __device__ __forceinline__ v4i filter(const NarrowArgs &a, __amdgpu_buffer_rsrc_t rsrc, int row) const
+    {
+        return load16<ALIGNED>(rsrc, u < a.win.n_units ? row + w_off : kParked, a.win.w_bytes);
+    }
+};
+
+template <int NT, bool SPLIT, bool ALIGNED, bool POINT>
 __global__ __launch_bounds__(kThreads) void conv2d_s8_narrow_kernel(const NarrowArgs a)
 {
     constexpr int G = NT >= 4 ? 2 : 4;
@@ -50,9 +149,40 @@ __global__ __launch_bounds__(kThreads) void conv2d_s8_narrow_kernel(const Narrow
     const int m = (SPLIT ? (int)blockIdx.x : (int)blockIdx.x * 4 + wave) * 16 + col;
     const int n0 = blockIdx.y * 16 * NT;
 
+    // What the epilogue needs is requested first, its addresses take no arithmetic: this wavefront's filter tiles.  Filters
+    // past the last one lie past the descriptors' ends and read as zeros.
+    const bool finisher = !SPLIT || wave < NT;
+    v4i bias[MINE], shift[MINE];
+    int res[MINE];
+    int lut = 0;
+    if (finisher) { // uniform
+        const __amdgpu_buffer_rsrc_t b_rsrc =
+            tensor_rsrc(reinterpret_cast<const int8_t *>(a.bias), a.bias != nullptr ? 4 * a.out_c : 0);
+        const __amdgpu_buffer_rsrc_t s_rsrc = tensor_rsrc(reinterpret_cast<const int8_t *>(a.shift), 4 * a.n_shift);
+#pragma unroll
+        for (int t = 0; t < MINE; t++) {
+            const int f = n0 + 4 * NT * quad + 4 * (SPLIT ? wave : t);
+            if ((a.out_c & 3) == 0) { // uniform
+                bias[t] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(b_rsrc, 4 * f, 0, 0));
+                shift[t] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(s_rsrc, 4 * f, 0, 0));
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    bias[t][r] = __builtin_amdgcn_raw_buffer_load_b32(b_rsrc, 4 * (f + r), 0, 0);
+                    shift[t][r] = __builtin_amdgcn_raw_buffer_load_b32(s_rsrc, 4 * (f + r), 0, 0);
+                }
+            }
+            if (a.n_shift == 1) { // uniform
+                const int s = __builtin_amdgcn_raw_buffer_load_b32(s_rsrc, 0, 0, 0);
+                shift[t] = v4i{s, s, s, s};
+            }
+        }
+    }
+    if (a.lut != nullptr)
+        lut = a.lut[tid];
+
     const __amdgpu_buffer_rsrc_t in_rsrc = tensor_rsrc(a.win.in, a.win.in_bytes);
     const __amdgpu_buffer_rsrc_t w_rsrc = tensor_rsrc(a.win.w, a.win.w_bytes);
-    const PixelWindow px = pixel_window(a.win, m, a.n_pix);
     int row[NT]; // a filter past the last one reads the last one again, its results are dropped
 #pragma unroll
     for (int t = 0; t < NT; t++)
@@ -62,65 +192,85 @@ __global__ __launch_bounds__(kThreads) void conv2d_s8_narrow_kernel(const Narrow
         v4i b[G], w[G][NT];
         int n[G];
     };
-    const int first = SPLIT ? wave : 0, stride = SPLIT ? 4 : 1;
-    auto request = [&](int s0, Batch &t) {
+    UnitWalk<ALIGNED, POINT> walk;
+    walk.start(a, 4 * (SPLIT ? wave : 0) + quad, m);
+    const int steps = SPLIT ? (a.ksteps - wave + 3) >> 2 : a.ksteps; // of this wavefront
+    auto request = [&](Batch &t) {
 #pragma unroll
         for (int i = 0; i < G; i++) {
-            const Unit u = locate_unit(a.win, 4 * (first + (s0 + i) * stride) + quad);
-            t.n[i] = u.n;
-            t.b[i] = load_pixel_unit<ALIGNED>(a.win, in_rsrc, px, u);
+            if constexpr (!ALIGNED)
+                t.n[i] = walk.channels(a);
+            t.b[i] = walk.pixel(a, in_rsrc);
 #pragma unroll
             for (int f = 0; f < NT; f++)
-                t.w[i][f] = load_filter_unit<ALIGNED>(a.win, w_rsrc, row[f], u);
+                t.w[i][f] = walk.filter(a, w_rsrc, row[f]);
+            walk.advance(a);
         }
     };
-    const int steps = SPLIT ? (a.ksteps - wave + 3) >> 2 : a.ksteps; // of this wavefront
     Batch cur, nxt;
-    request(0, cur);
-
-    // what the epilogue needs is requested before the products: this wavefront's filter tiles
-    const bool finisher = !SPLIT || wave < NT;
-    int bias[MINE][4], shift[MINE][4];
-    int res[MINE];
-    const int8_t *res_p = a.res != nullptr ? a.res + (long long)min(m, a.n_pix - 1) * a.res_pitch : nullptr;
+    request(cur);
+    // while the operands are on their way
+    const bool half_even = a.half_even != 0;
+    bool general = false;
+    Short4 consts[MINE];
+    int8_t *dst = nullptr;
+    if (finisher) { // uniform
+        dst = a.out + (long long)m * a.out_pitch;
+        if (a.res != nullptr) // uniform
 #pragma unroll
-    for (int t = 0; t < MINE; t++) {
-        const int f = n0 + 4 * NT * quad + 4 * (SPLIT ? wave : t);
-        res[t] = 0;
+            for (int t = 0; t < MINE; t++) {
+                const int f = n0 + 4 * NT * quad + 4 * (SPLIT ? wave : t);
+                const int8_t *p = a.res + (long long)min(m, a.n_pix - 1) * a.res_pitch;
+                res[t] = 0;
+                if (f + 4 <= a.out_c) {
+                    res[t] = *reinterpret_cast<const int_unaligned *>(p + f);
+                } else {
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int n = min(f + r, a.out_c - 1);
-            bias[t][r] = (finisher && a.bias != nullptr) ? a.bias[n] : 0;
-            shift[t][r] = finisher ? a.shift[a.n_shift == 1 ? 0 : n] : 0;
-            if (finisher && res_p != nullptr)
-                res[t] |= (int)(unsigned char)res_p[n] << (8 * r);
+                    for (int r = 0; r < 3; r++)
+                        if (f + r < a.out_c)
+                            res[t] |= (int)(unsigned char)p[f + r] << (8 * r);
+                }
+            }
+        bool bad = false;
+#pragma unroll
+        for (int t = 0; t < MINE; t++) {
+            const int f = n0 + 4 * NT * quad + 4 * (SPLIT ? wave : t);
+            if (a.out_c & 3) // uniform
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    shift[t][r] = f + r < a.out_c ? shift[t][r] : 1;
+            bad = bad || (f < a.out_c && !short4_ok(bias[t], shift[t], a.bound));
         }
+        general = __any(bad);
+#pragma unroll
+        for (int t = 0; t < MINE; t++)
+            consts[t] = make_short4(bias[t], shift[t], general, half_even);
     }
-    if (a.lut != nullptr)
-        lut_l[tid] = a.lut[tid];
 
     v4i acc[NT];
 #pragma unroll
     for (int t = 0; t < NT; t++)
         acc[t] = v4i{0, 0, 0, 0};
-    auto products = [&](const Batch &t, int left) {
+    // (steps past the last one have zeros on both sides)
+    auto products = [&](const Batch &t) {
 #pragma unroll
         for (int i = 0; i < G; i++)
-            if (i < left) // uniform
 #pragma unroll
-                for (int f = 0; f < NT; f++)
-                    acc[f] = __builtin_amdgcn_mfma_i32_16x16x64_i8(mask_unit<ALIGNED>(t.w[i][f], t.n[i]), t.b[i], acc[f], 0, 0, 0);
+            for (int f = 0; f < NT; f++)
+                acc[f] = __builtin_amdgcn_mfma_i32_16x16x64_i8(mask_unit<ALIGNED>(t.w[i][f], ALIGNED ? 16 : t.n[i]), t.b[i], acc[f], 0, 0, 0);
     };
     for (int s = 0; s < steps; s += 2 * G) {
         if (s + G < steps)
-            request(s + G, nxt);
-        products(cur, steps - s);
+            request(nxt);
+        products(cur);
         if (s + G < steps) {
             if (s + 2 * G < steps)
-                request(s + 2 * G, cur);
-            products(nxt, steps - s - G);
+                request(cur);
+            products(nxt);
         }
     }
+    if (a.lut != nullptr)
+        lut_l[tid] = (int8_t)lut;
     if constexpr (SPLIT) {
 #pragma unroll
         for (int t = 0; t < NT; t++)
@@ -130,54 +280,63 @@ __global__ __launch_bounds__(kThreads) void conv2d_s8_narrow_kernel(const Narrow
         __syncthreads();
     if (!finisher) // uniform
         return;
-    const bool relu = a.relu != 0, half_even = a.half_even != 0;
 #pragma unroll
     for (int t = 0; t < MINE; t++) {
-        v4i sum = acc[t];
-        if constexpr (SPLIT)
-            sum = part[0][wave][lane] + part[1][wave][lane] + part[2][wave][lane] + part[3][wave][lane];
-        const int f = n0 + 4 * NT * quad + 4 * (SPLIT ? wave : t);
-        int q[4];
-        const int word = a.res_shift != 0 ? requant4_s8(res[t], make_requant4(a.res_shift)) : res[t];
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            q[r] = requant_s8(sum[r] + bias[t][r], shift[t][r], relu, half_even);
-            if (a.lut != nullptr)
-                q[r] = lut_l[q[r] + 128];
-            if (a.res != nullptr)
-                q[r] = clamp_s8(q[r] + (int)(int8_t)(word >> (8 * r)));
+        v4i sum = acc[t] + consts[t].start;
+        if constexpr (SPLIT) {
+            sum = part[0][wave][lane] + part[1][wave][lane] + part[2][wave][lane] + part[3][wave][lane] + consts[t].start;
         }
+        const int f = n0 + 4 * NT * quad + 4 * (SPLIT ? wave : t);
+        int word;
+        if (general) // uniform, as are the next ones
+            word = finish_general4(sum, consts[t].shift, a.relu, a.half_even);
+        else
+            word = finish_short4(sum, consts[t].shift, a.relu != 0, half_even);
+        if (a.lut != nullptr) {
+            const int at = word ^ (int)0x80808080u;
+            word = (int)(unsigned char)lut_l[at & 255] | (int)(unsigned char)lut_l[(at >> 8) & 255] << 8 |
+                (int)(unsigned char)lut_l[(at >> 16) & 255] << 16 | (int)(unsigned char)lut_l[(unsigned)at >> 24] << 24;
+        }
+        if (a.res != nullptr)
+            word = sat_add4_pairs(word, a.res_shift != 0 ? requant4_s8(res[t], make_requant4(a.res_shift)) : res[t]);
         if (m >= a.n_pix || f >= a.out_c)
             continue;
-        int8_t *dst = a.out + (long long)m * a.out_pitch + f;
         if (f + 4 <= a.out_c) {
-            const int word = pack4_s8(q[0], q[1], q[2], q[3]);
             if (a.through) // uniform
-                __hip_atomic_store(reinterpret_cast<int *>(dst), word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(reinterpret_cast<int *>(dst + f), word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             else
-                *reinterpret_cast<int_unaligned *>(dst) = word;
+                *reinterpret_cast<int_unaligned *>(dst + f) = word;
         } else {
 #pragma unroll
-            for (int r = 0; r < 4; r++)
+            for (int r = 0; r < 3; r++)
                 if (f + r < a.out_c)
-                    dst[r] = (int8_t)q[r];
+                    dst[f + r] = (int8_t)(word >> (8 * r));
         }
     }
 }
 
-template <int NT>
-void launch_narrow(const NarrowArgs &a, bool split, bool aligned, hipStream_t stream)
+template <int NT, bool SPLIT>
+void launch_split(const NarrowArgs &a, bool aligned, bool point, hipStream_t stream)
 {
     const unsigned tiles = (unsigned)((a.n_pix + 15) / 16);
-    const dim3 grid(split ? tiles : (tiles + 3) / 4, (unsigned)((a.out_c + 16 * NT - 1) / (16 * NT)));
-    if (split && aligned)
-        hipLaunchKernelGGL((conv2d_s8_narrow_kernel<NT, true, true>), grid, dim3(kThreads), 0, stream, a);
-    else if (split)
-        hipLaunchKernelGGL((conv2d_s8_narrow_kernel<NT, true, false>), grid, dim3(kThreads), 0, stream, a);
+    const dim3 grid(SPLIT ? tiles : (tiles + 3) / 4, (unsigned)((a.out_c + 16 * NT - 1) / (16 * NT)));
+    if (aligned && point)
+        hipLaunchKernelGGL((conv2d_s8_narrow_kernel<NT, SPLIT, true, true>), grid, dim3(kThreads), 0, stream, a);
     else if (aligned)
-        hipLaunchKernelGGL((conv2d_s8_narrow_kernel<NT, false, true>), grid, dim3(kThreads), 0, stream, a);
+        hipLaunchKernelGGL((conv2d_s8_narrow_kernel<NT, SPLIT, true, false>), grid, dim3(kThreads), 0, stream, a);
+    else if (point)
+        hipLaunchKernelGGL((conv2d_s8_narrow_kernel<NT, SPLIT, false, true>), grid, dim3(kThreads), 0, stream, a);
     else
-        hipLaunchKernelGGL((conv2d_s8_narrow_kernel<NT, false, false>), grid, dim3(kThreads), 0, stream, a);
+        hipLaunchKernelGGL((conv2d_s8_narrow_kernel<NT, SPLIT, false, false>), grid, dim3(kThreads), 0, stream, a);
+}
+
+template <int NT>
+void launch_narrow(const NarrowArgs &a, bool split, bool aligned, bool point, hipStream_t stream)
+{
+    if (split)
+        launch_split<NT, true>(a, aligned, point, stream);
+    else
+        launch_split<NT, false>(a, aligned, point, stream);
 }
 
 } // namespace
@@ -206,7 +365,8 @@ static NarrowPlan narrow_plan(const ConvGeom &g, int cu_count)
     return p;
 }
 
-// Expected time (see dense_s8_route in espdl_hip_api.hip): launch, the steps of one wavefront, all steps in flight.
+// Expected time (see dense_s8_route in espdl_hip_api.hip): launch, the steps of one wavefront, all steps in flight.  Fitted to 2840
+// random layers on operands that change from launch to launch: 5 to 9 % off either way, 7 to 15 where channels are no whole units.
 float conv2d_s8_narrow_us(const ConvGeom &g, const void *in, const void *filter, int cu_count)
 {
     const NarrowPlan p = narrow_plan(g, cu_count);
@@ -215,9 +375,15 @@ float conv2d_s8_narrow_us(const ConvGeom &g, const void *in, const void *filter,
         return 1e30f;
     const float steps = (float)(p.split ? (p.ksteps + 3) / 4 : p.ksteps);
     const float waves = 4e-3f * (float)p.groups;
+    const float nt = (float)p.nt;
     if (window_aligned(g, in, filter))
-        return 2.7f + 0.12f * steps + waves * (0.25f + 0.077f * steps * (float)p.nt);
-    return 3.3f + waves * (0.12f + 0.264f * steps * (float)p.nt);
+        return p.split ? 2.23f + 0.11f * steps + waves * (0.14f + steps * (0.02f + 0.077f * nt))
+                       : 2.18f + 0.13f * steps + waves * nt * (g.k_h * g.k_w == 1 ? 0.36f + 0.075f * steps : 0.08f + 0.13f * steps);
+    if (((g.in_c | g.in_pitch) & 3) == 0) // units of whole dwords
+        return p.split ? 2.7f + 0.18f * steps + waves * (0.25f + nt * (0.06f + 0.082f * steps))
+                       : 2.95f + 0.05f * steps + waves * (0.55f * nt + 0.1f * steps);
+    return p.split ? 2.42f + 0.34f * steps + waves * (0.18f + steps * (0.085f + 0.206f * nt))
+                   : 2.78f + 0.23f * steps + waves * (0.39f * nt + steps * (0.123f + 0.165f * nt));
 }
 
 hipError_t launch_conv2d_s8_narrow(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,
@@ -246,12 +412,32 @@ hipError_t launch_conv2d_s8_narrow(const ConvGeom &g, const int8_t *in, const in
         return hipSuccess;
     const NarrowPlan p = narrow_plan(g, cu_count);
     const bool aligned = window_aligned(g, in, filter);
+    const bool point = g.k_h == 1 && g.k_w == 1 && g.pad_top == 0 && g.pad_left == 0 && (g.out_h - 1) * g.stride_h < g.in_h &&
+        (g.out_w - 1) * g.stride_w < g.in_w;
+    const long long products = 16384ll * a.win.w_len;
+    a.bound = products < 1ll << 30 ? (unsigned)products : 0x80000000u;
+    a.dense_pixels = g.out_h == g.in_h && g.out_w == g.in_w && g.stride_h == 1 && g.stride_w == 1;
+    a.step.units = p.split ? 16 : 4;
+    const int taps = a.step.units / a.win.upt, rows = taps / g.k_w, columns = taps % g.k_w;
+    a.step.channels = 16 * (a.step.units % a.win.upt);
+    a.step.column = columns * g.dil_w;
+    a.step.row = rows * g.dil_h;
+    a.step.in = (a.step.row * g.in_w + a.step.column) * g.in_pitch + a.step.channels;
+    a.step.filter = taps * g.in_c + a.step.channels;
+    a.step.tap_channels = 16 * a.win.upt;
+    a.step.in_tap = g.dil_w * g.in_pitch - a.step.tap_channels;
+    a.step.filter_tap = g.in_c - a.step.tap_channels;
+    a.step.window_columns = g.k_w * g.dil_w;
+    a.step.in_row = (g.dil_h * g.in_w - a.step.window_columns) * g.in_pitch;
+    if (point) { // channels past the tap's last one are no next tap
+        a.step.in = a.step.filter = 16 * a.step.units;
+    }
     if (p.nt == 4)
-        launch_narrow<4>(a, p.split, aligned, stream);
+        launch_narrow<4>(a, p.split, aligned, point, stream);
     else if (p.nt == 2)
-        launch_narrow<2>(a, p.split, aligned, stream);
+        launch_narrow<2>(a, p.split, aligned, point, stream);
     else
-        launch_narrow<1>(a, p.split, aligned, stream);
+        launch_narrow<1>(a, p.split, aligned, point, stream);
     return hipGetLastError();
 }
 

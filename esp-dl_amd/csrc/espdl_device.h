@@ -283,6 +283,61 @@ __device__ __forceinline__ int pack4_s8(int a, int b, int c, int d)
     return (a & 0xff) | ((b & 0xff) << 8) | ((c & 0xff) << 16) | ((d & 0xff) << 24);
 }
 
+// Four channels' requantization where a launch is too short for tables: the start value of a sum (bias and the rounding
+// constant) and the shifts, or, `general` (the whole wavefront alike), bias and shifts as they are for requant_s8.  Short where
+// every shift is in 1 .. 31 and no accumulator with its start value can pass int32: `bound` is the largest magnitude of the
+// sum of products, 2^31 where that is 2^30 or more.
+struct Short4 {
+    v4i start, shift;
+};
+__device__ __forceinline__ bool short4_ok(const v4i &bias, const v4i &shift, unsigned bound)
+{
+    const int s_lo = min(min(shift[0], shift[1]), min(shift[2], shift[3])), s_hi = max(max(shift[0], shift[1]), max(shift[2], shift[3]));
+    const int b_lo = min(min(bias[0], bias[1]), min(bias[2], bias[3])), b_hi = max(max(bias[0], bias[1]), max(bias[2], bias[3]));
+    const unsigned largest = max((unsigned)max(b_hi, 0), 0u - (unsigned)min(b_lo, 0));
+    const unsigned others = bound + (1u << ((s_hi - 1) & 31)); // at most 2^30 + 2^30 or 2^31 + 2^30
+    return s_lo >= 1 && s_hi <= 31 && others < 0x80000000u && largest < 0x80000000u - others;
+}
+__device__ __forceinline__ Short4 make_short4(const v4i &bias, const v4i &shift, bool general, bool half_even)
+{
+    Short4 c = {bias, shift};
+    if (!general)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            c.start[r] = bias[r] + (1 << (shift[r] - 1)) - (half_even ? 1 : 0);
+    return c;
+}
+// `acc` holds the start value.  The shifted values saturate to int16 in pairs, are clamped in pairs and lose their high bytes.
+__device__ __forceinline__ int finish_short4(v4i acc, const v4i &shift, bool relu, bool half_even)
+{
+    if (half_even)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            acc[r] = half_even_add(acc[r], shift[r]);
+    const v2s floor2 = __builtin_bit_cast(v2s, relu ? 0 : (int)0xff80ff80u), ceil2 = __builtin_bit_cast(v2s, 0x007f007f);
+    const v2s lo = __builtin_elementwise_min(
+        __builtin_elementwise_max(__builtin_amdgcn_cvt_pk_i16(acc[0] >> shift[0], acc[1] >> shift[1]), floor2), ceil2);
+    const v2s hi = __builtin_elementwise_min(
+        __builtin_elementwise_max(__builtin_amdgcn_cvt_pk_i16(acc[2] >> shift[2], acc[3] >> shift[3]), floor2), ceil2);
+    return (int)__builtin_amdgcn_perm((unsigned)__builtin_bit_cast(int, hi), (unsigned)__builtin_bit_cast(int, lo), 0x06040200u);
+}
+__device__ __forceinline__ int finish_general4(const v4i &acc, const v4i &shift, int relu, int half_even)
+{
+    int q[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+        q[r] = requant_s8(acc[r], shift[r], relu != 0, half_even != 0);
+    return pack4_s8(q[0], q[1], q[2], q[3]);
+}
+// int8 x 4 saturating add of two packed dwords on int16 pairs with the values in their high bytes.
+__device__ __forceinline__ int sat_add4_pairs(int x, int y)
+{
+    const auto spread = [](int w, unsigned sel) { return __builtin_bit_cast(v2s, (int)__builtin_amdgcn_perm(0u, (unsigned)w, sel)); };
+    const v2s lo = __builtin_elementwise_add_sat(spread(x, 0x010c000cu), spread(y, 0x010c000cu));
+    const v2s hi = __builtin_elementwise_add_sat(spread(x, 0x030c020cu), spread(y, 0x030c020cu));
+    return (int)__builtin_amdgcn_perm((unsigned)__builtin_bit_cast(int, hi), (unsigned)__builtin_bit_cast(int, lo), 0x07050301u);
+}
+
 // Tile sequence of one workgroup of a persistent grid.  The hardware deals workgroups to the eight
 // XCDs round-robin by their linear id, and every XCD has its own L2.  Striding tiles by gridDim.x
 // would therefore spread neighbouring tiles (which share input rows through the filter window) over

@@ -160,10 +160,13 @@ DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *
         return units && narrow < 5.2f ? DENSE_NARROW : DENSE_STEM;
     const bool flat = g.k_h == 1 && g.k_w == 1 && g.stride_h == 1 && g.stride_w == 1 && g.pad_top == 0 &&
         g.pad_left == 0 && g.out_h == g.in_h && g.out_w == g.in_w;
-    const DenseRoute few = narrow < gemm ? DENSE_NARROW : DENSE_UNITGEMM;
+    // (the tiled GEMM's line leaves out what channels that are no multiple of 4 cost it: 120 layers near the two lines took 1.06 to 1.16
+    // times the narrow kernel's time there)
+    const float uneven = ((g.in_c | g.in_pitch) & 3) != 0 ? 1.15f : 0.f;
+    const DenseRoute few = narrow < std::max(1.f, uneven) * gemm ? DENSE_NARROW : DENSE_UNITGEMM;
     if (flat) {
         if (espdl::conv2d_s8_pwgemm_supports(g, in, filter, cus))
-            return units && narrow < 0.97f * gemm ? DENSE_NARROW : DENSE_PWGEMM;
+            return units && narrow < std::max(0.97f, uneven) * gemm ? DENSE_NARROW : DENSE_PWGEMM;
         return units && tile_steps <= 3500 ? few : DENSE_DIRECT;
     }
     if (!espdl::conv2d_s8_units_aligned(g, in, filter))
@@ -185,18 +188,20 @@ DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *
 // 3076 random layers of 16 to 256 channels in 1 image to 400 MB, each timed on both sides with operands that change from launch to
 // launch: 0.88 of the other kernels' time in the geometric mean on channels that are a multiple of 4, 0.80 on others (the better one of
 // each pair: 0.87, 0.78); 1.7 % of all are slower by more than 5 % than on the other kernel, 0.9 % by more than 10; 600 of 200 to 8192
-// filters 0.87, 2.8 % slower by more than 5 %.  (On operands that lie in the L2 caches the other kernels gain more and a margin of 1.2
+// filters 0.87, 2.8 % slower by more than 5 %.  Pointwise layers on the two kernels' line, some 3 us either way, took 1 to 4 % longer on
+// the narrow one (RAW, or at stride 2), hence the factors on its line.  (On operands that lie in the L2 caches the other kernels gain more and a margin of 1.2
 // under 3 x 3 looks right; it costs a detector of 20 frames of 320 x 320 8 % of its dense layers' time.)
 bool dense_s8_walks(const espdl::ConvGeom &g, DenseRoute other, float walk, float narrow, float gemm)
 {
     if (((g.in_c | g.in_pitch) & 3) != 0) {
         const float direct = g.out_c < 96 ? 1.f : (g.out_c <= 256 ? 0.7f : 0.85f);
-        return walk < std::min(1.05f * narrow, gemm * (other == DENSE_PWGEMM ? 0.9f : (other == DENSE_DIRECT ? direct : 1.f)));
+        return walk < std::min(narrow * (g.k_h == 1 ? 1.06f : 1.f), gemm * (other == DENSE_PWGEMM ? 0.9f : (other == DENSE_DIRECT ? direct : 1.f)));
     }
     const bool few = other == DENSE_NARROW || other == DENSE_UNITGEMM;
     if (other == DENSE_TILED)
         return walk < 1e30f; // (there is a build)
-    return walk * (g.k_h == 1 ? 1.f : (g.k_h == 3 ? 1.02f : 1.1f)) < std::min(narrow, gemm * (few ? 1.15f : 2.f));
+    const float point = g.stride_h == 1 && g.stride_w == 1 ? 1.f : 1.08f;
+    return walk * (g.k_h == 1 ? 1.f : (g.k_h == 3 ? 1.02f : 1.1f)) < std::min(narrow * (g.k_h == 1 ? point : 1.f), gemm * (few ? 1.15f : 2.f));
 }
 
 // Of all kernels.  Two take every layer that they apply to: the classifier's, and the walk of the first-layer kernel's layers

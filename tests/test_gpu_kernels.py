@@ -872,6 +872,57 @@ def test_conv2d_s16_matrix_pipe(oracle, case):
     assert want.min() < want.max()
 
 
+# Few outputs: (name, (n, h, w, c), out_c, k, stride, dil, pads, shifts).  Steps of the split and of the whole reduction that
+# end inside a tap, at a row's end and past the window (1, 3 and 9 units a tap under windows of 3, 5 and 7 columns), pointwise
+# layers with a stride, a padding and a partial unit; filter counts around the tiles of 16 and the groups of 4; shifts the short
+# epilogue takes (1 .. 31), ones it does not, one shift for the layer.
+NARROW_EDGES = [
+    ("split_16_17", (1, 9, 11, 16), 17, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), (6, 10)),
+    ("split_48_64", (1, 7, 9, 48), 64, (5, 3), (2, 1), (1, 1), (2, 2, 1, 1), (1, 31)),
+    ("split_144_33", (2, 5, 6, 144), 33, (3, 3), (1, 1), (2, 2), (2, 2, 2, 2), (8, 12)),
+    ("split_16_66_wide_window", (1, 6, 12, 16), 66, (2, 7), (1, 2), (1, 1), (0, 1, 3, 3), (0, 32)),
+    ("whole_20_15", (1, 12, 13, 20), 15, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), (5, 9)),
+    ("whole_64_20_stride", (2, 13, 9, 64), 20, (1, 1), (2, 3), (1, 1), (0, 0, 0, 0), (6, 9)),
+    ("whole_48_36_padded", (1, 8, 9, 48), 36, (1, 1), (1, 1), (1, 1), (1, 1, 1, 1), (-3, 40)),
+    ("whole_16_70_window", (1, 9, 10, 16), 70, (2, 3), (1, 1), (1, 1), (0, 1, 1, 1), (6, 8)),
+    ("split_272_130", (1, 6, 7, 272), 130, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), (9, 9)),
+    ("split_1280_10_row", (1, 1, 1, 1280), 10, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), (10, 12)),
+]
+
+
+@pytest.mark.parametrize("half_even", [False, True], ids=["half_up", "half_even"])
+@pytest.mark.parametrize("behind", ["", "table", "add", "table+add"])
+@pytest.mark.parametrize("case", NARROW_EDGES, ids=lambda c: c[0])
+def test_conv2d_few_outputs(oracle, case, behind, half_even):
+    announce(f"few outputs {case[0]} {behind} {half_even}")
+    name, (n, h, w, c), oc, k, stride, dil, pads, (s_lo, s_hi) = case
+    rng = np.random.default_rng(0x6A0 + len(name))
+    x = rng.integers(-128, 128, size=(n, h, w, c)).astype(np.int8)
+    f = rng.integers(-128, 128, size=(oc, k[0], k[1], c)).astype(np.int8)
+    bias = rng.integers(-2**14, 2**14, size=oc).astype(np.int32)
+    if "66" in name:  # past what the short epilogue takes beside a shift of 31
+        bias[::5] = rng.choice([1 - 2**30, 2**30 - 1], size=len(bias[::5]))
+    # (half even is formed in 32 bits, shifts of 32 and more are not defined there)
+    shift = rng.integers(s_lo, min(s_hi, 31 if half_even else s_hi) + 1, size=1 if s_lo == s_hi else oc).astype(np.int32)
+    relu = "add" not in behind
+    rm_o = oracle.ROUND_HALF_EVEN if half_even else oracle.ROUND_HALF_UP
+    want = oracle.conv2d_s8(x, f, bias, shift, k, stride, dil, pads, oracle.RELU if relu else oracle.LINEAR, rm_o)
+    m = espdl()
+    kw = {"activation": m.capi.RELU if relu else m.capi.LINEAR, "round_mode": m.capi.ROUND_HALF_EVEN if half_even else m.capi.ROUND_HALF_UP}
+    if "table" in behind:
+        table = rng.integers(-128, 128, size=256).astype(np.int8)
+        want = table[want.astype(np.int32) + 128]
+        kw["lut"] = to_dev(table)
+    if "add" in behind:
+        res = rng.integers(-128, 128, size=want.shape).astype(np.int8)
+        want = oracle.add_s8(want, res)
+        kw["residual"] = to_dev(res)
+    args = (to_dev(x), to_dev(f), to_dev(bias), to_dev(shift), k, stride, dil, pads)
+    kernel = {a: v for a, v in kw.items() if a in ("activation", "round_mode", "lut", "residual")}
+    assert m.capi.conv2d_s8_kernel(args[0], args[1], args[3], *args[4:], **kernel) == "conv2d_s8_narrow"
+    np.testing.assert_array_equal(to_host(m.conv2d(*args, **kw)), want)
+
+
 S16_UNIT_CASES = [
     # (name, (n, h, w, c), out_c, k, stride, dil, pads, relu, half_even, lowest and highest shift, values): channel counts
     # around the 16-channel units, one to four filter tiles and tails of each, few pixels (narrow kernel) and many
