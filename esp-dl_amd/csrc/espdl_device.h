@@ -283,6 +283,15 @@ __device__ __forceinline__ int pack4_s8(int a, int b, int c, int d)
     return (a & 0xff) | ((b & 0xff) << 8) | ((c & 0xff) << 16) | ((d & 0xff) << 24);
 }
 
+// A workgroup barrier that orders LDS alone: loads and stores of global memory stay in flight across it (__syncthreads waits for
+// them, a memory round trip where the next operands have just been requested).
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Four channels' requantization where a launch is too short for tables: the start value of a sum (bias and the rounding
 // constant) and the shifts, or, `general` (the whole wavefront alike), bias and shifts as they are for requant_s8.  Short where
 // every shift is in 1 .. 31 and no accumulator with its start value can pass int32: `bound` is the largest magnitude of the

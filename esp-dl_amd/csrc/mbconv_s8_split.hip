@@ -17,6 +17,14 @@
 // next chunk a chunk ahead, builds the requantization constants of its own chunk in LDS (no workgroup tables, no votes
 // across wavefronts) and runs expand -> depthwise in a private LDS area.  The four chunks of a group meet in an LDS tile
 // [pixel][64 channels] that all wavefronts write out as 64-byte runs.
+//
+// On few images the launch is the life of one workgroup, instructions and round trips one behind the other (28 x 28, 32 -> 192, one image:
+// 0.4 us of arguments and addresses, 0.4 for the patch, 0.95 for constants and a barrier that waited for the next chunk's
+// loads, 0.55 expand, 0.85 depthwise, after 1.2 us between launches).  So there a tile has two output rows (one at stride 2)
+// instead of seven (four), a workgroup takes one group of 64 channels without a loop around it, barriers order LDS alone, and
+// all arguments are fetched at once: 4.6 -> 3.2 us; 7 x 7, 160 -> 960 5.0 -> 3.55; 37 images of 10 x 10, 64 -> 384 5.4 -> 4.8, of 20 x 20, 32 ->
+// 192 6.2 -> 5.6.  Requesting the patch before and placing it behind the constants' arithmetic held too many registers (spills from
+// 65 input channels on, 14 x 14, 96 -> 576 3.6 -> 4.0 us).
 #include <algorithm>
 #include <type_traits>
 
@@ -50,13 +58,21 @@ template <int PT, int TW, int S>
 struct Tile {
     static constexpr int PH = (PT - 1) * S + 3, PW = (TW - 1) * S + 3;
     static constexpr int NXPT = (PH * PW + 15) / 16;
+    // row of patch position p: p / PW in 24 bits (p below 1024, PW 9, 15 or 16)
+    static constexpr unsigned kPerPW = (65536u + PW - 1) / PW;
+    static __device__ __forceinline__ int patch_row(int p)
+    {
+        return (int)(__umul24((unsigned)p, kPerPW) >> 16);
+    }
     static constexpr int TWP = TW <= 8 ? 8 : 16; // pixel slots per output row in the LDS tile
     // the depthwise stage reads up to one row pair and three columns past the patch (zero weights meet those bytes)
     static constexpr int EXP_BYTES = std::max((PH + 1) * PW + 48, NXPT * 16) * 16;
     static constexpr int DW_BYTES = PT * TWP * kDws;
 };
 
-template <int PT, int TW, int S, int KSE, bool HE, bool CLIP>
+// LOOP: a workgroup walks several groups of 64 expanded channels.  Without it what the loop would keep over its turns (addresses, masks,
+// some 170 instructions and scalar spills ahead of the first product) does not exist.
+template <int PT, int TW, int S, int KSE, bool HE, bool CLIP, bool LOOP>
 __global__ __launch_bounds__(kThreads, 4) void mbconv_s8_expand_dw_kernel(const SplitArgs a)
 {
     using T = Tile<PT, TW, S>;
@@ -66,6 +82,9 @@ __global__ __launch_bounds__(kThreads, 4) void mbconv_s8_expand_dw_kernel(const 
     __shared__ __align__(16) int tab_l[kWaves][2][3 * 16]; // expand, depthwise: [start value | right shift | left shift]
     extern __shared__ __align__(16) unsigned char patch_l[]; // [NXPT * 16 pixels][pitch] + slack
     const MbconvParams &p = a.p;
+    if constexpr (!LOOP) // every argument on its way at once: one round trip of the scalar cache in front of everything
+        asm volatile("" ::"s"(p.relu_expand), "s"(p.out_h), "s"(p.out_w), "s"(p.pad_top), "s"(p.n_s_dw), "s"(a.mid), "s"(a.through),
+                     "s"(a.pitch), "s"(a.units), "s"(p.b_dw), "s"(p.s_dw));
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, quad = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
@@ -109,7 +128,7 @@ __global__ __launch_bounds__(kThreads, 4) void mbconv_s8_expand_dw_kernel(const 
         w.bias = b_src != nullptr ? b_src[(size_t)(unsigned)ch] : 0;
         w.shift = s_src[(size_t)(s_step * (unsigned)ch)];
     };
-    const int g_first = part * a.per_wg, g_end = min(g_first + a.per_wg, a.n_groups);
+    const int g_first = LOOP ? part * a.per_wg : part, g_end = LOOP ? min(g_first + a.per_wg, a.n_groups) : g_first + 1;
     Chunk cur;
     load_chunk(4 * g_first + wave, cur);
 
@@ -119,14 +138,16 @@ __global__ __launch_bounds__(kThreads, 4) void mbconv_s8_expand_dw_kernel(const 
         const __amdgpu_buffer_rsrc_t in_rsrc = window::tensor_rsrc(p.in, a.in_bytes);
         const int img = (int)n * p.in_h * p.in_w;
         const int n_pieces = T::PH * T::PW * a.units;
-        for (int u0 = tid; u0 < n_pieces; u0 += 4 * kThreads) {
+        for (int first = 0; first < n_pieces; first += 4 * kThreads) {
             v4i v[4];
             int at[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const int u = u0 + j * kThreads;
+                if (first + j * kThreads >= n_pieces) // uniform
+                    break;
+                const int u = first + j * kThreads + tid;
                 const int pp = (int)fastdiv((unsigned)u, a.fd_units), unit = u - pp * a.units;
-                const int prow = (int)fastdiv((unsigned)pp, a.fd_pw);
+                const int prow = T::patch_row(pp);
                 const int iy = iy0 + prow, ix = ix0 + pp - prow * T::PW;
                 const bool valid = u < n_pieces && (unsigned)iy < (unsigned)p.in_h && (unsigned)ix < (unsigned)p.in_w;
                 at[j] = pp * a.pitch + 16 * unit;
@@ -134,7 +155,7 @@ __global__ __launch_bounds__(kThreads, 4) void mbconv_s8_expand_dw_kernel(const 
             }
 #pragma unroll
             for (int j = 0; j < 4; j++)
-                if (u0 + j * kThreads < n_pieces)
+                if (first + j * kThreads + tid < n_pieces)
                     *reinterpret_cast<v4i *>(patch_l + at[j]) = v[j];
         }
     }
@@ -142,7 +163,7 @@ __global__ __launch_bounds__(kThreads, 4) void mbconv_s8_expand_dw_kernel(const 
 #pragma unroll
     for (int pt = 0; pt < NXPT; pt++) {
         const int pp = pt * 16 + col;
-        const int prow = T::PW == 16 ? pt : (int)fastdiv((unsigned)pp, a.fd_pw);
+        const int prow = T::patch_row(pp);
         const int iy = iy0 + prow, ix = ix0 + pp - prow * T::PW;
         xmask |= (unsigned)iy < (unsigned)p.in_h && (unsigned)ix < (unsigned)p.in_w ? 1u << pt : 0u;
     }
@@ -191,10 +212,12 @@ __global__ __launch_bounds__(kThreads, 4) void mbconv_s8_expand_dw_kernel(const 
     int *tab = tab_l[wave][0];
     const bool write_ok = col < TW;
 
-    for (int gi = g_first; gi < g_end; gi++) {
-        Chunk nxt;
+    int gi = g_first;
+    do {
+        Chunk nxt = cur;
         const int sub = 4 * gi + wave;
-        load_chunk(4 * min(gi + 1, g_end - 1) + wave, nxt);
+        if (LOOP && gi + 1 < g_end) // uniform
+            load_chunk(4 * (gi + 1) + wave, nxt);
         // constants of this chunk: the short form where every channel of the stage can take it (see mbconv_s8_stages.h)
         int mode_e, mode_d;
         {
@@ -216,14 +239,14 @@ __global__ __launch_bounds__(kThreads, 4) void mbconv_s8_expand_dw_kernel(const 
             }
         }
         wave_lds_sync();
-        if (gi == g_first)
-            __syncthreads(); // the patch is complete
         v4i aop[KSE];
 #pragma unroll
         for (int ks = 0; ks < KSE; ks++)
             aop[ks] = window::mask_unit<false>(cur.aop[ks], c0 - 64 * ks - 16 * quad);
+        const StageConsts ce = read_stage_table(tab, 16, 4 * quad, mode_e);
+        if (!LOOP || gi == g_first)
+            lds_barrier(); // the patch is complete
         {
-            const StageConsts ce = read_stage_table(tab, 16, 4 * quad, mode_e);
             if (!HE && ce.mode == 0)
                 expand(std::integral_constant<int, 0>{}, aop, ce, floor_e, ceil_e, exp_dst);
             else if (!HE && ce.mode == 1)
@@ -236,8 +259,8 @@ __global__ __launch_bounds__(kThreads, 4) void mbconv_s8_expand_dw_kernel(const 
                 expand(std::integral_constant<int, -1>{}, aop, ce, floor_e, ceil_e, exp_dst);
         }
         wave_lds_sync();
-        if (gi != g_first)
-            __syncthreads(); // the tile's previous group has been written out
+        if (LOOP && gi != g_first)
+            lds_barrier(); // the tile's previous group has been read
         if (16 * sub < p.exp_c) { // uniform
             v4i a0[3], a1[3];
 #pragma unroll
@@ -259,7 +282,7 @@ __global__ __launch_bounds__(kThreads, 4) void mbconv_s8_expand_dw_kernel(const 
             else
                 depthwise_chunk<-1, PT, S, true, false, CLIP>(exp_src, PT, T::PW, a0, a1, cd, floor_d, relu, HE, dw_dst, row_bytes, write_ok, ceil_d);
         }
-        __syncthreads(); // the group's tile is complete
+        lds_barrier(); // the group's tile is complete
         int8_t *dst = a.mid + (((long long)n * p.out_h + oy0) * p.out_w + ox0) * p.exp_c + 64 * gi;
 #pragma unroll
         for (int i = 0; i < (PT * T::TWP * 4 + kThreads - 1) / kThreads; i++) {
@@ -270,13 +293,32 @@ __global__ __launch_bounds__(kThreads, 4) void mbconv_s8_expand_dw_kernel(const 
                 store16(dst, (row * p.out_w + x) * p.exp_c + 16 * q, *reinterpret_cast<const v4i *>(dw_l + slot * kDws + 16 * q), a.through);
         }
         cur = nxt;
-    }
+    } while (LOOP && ++gi < g_end);
 }
 
 struct SplitPlan {
     bool ok;
     int pt, tw, kse;
+    float us; // expected time
 };
+
+// Expected time of tiles of `pt` rows: the launch and one workgroup's chain, which is shorter the fewer rows it has, then the work of
+// all workgroups, which grows with the halo (two rows of the patch at stride 1, one at stride 2).  Fitted to 846 launches of 14
+// blocks on 1 to 100 images, 3 to 4 % off; the tile it picks takes 0.7 % more than the best one in the mean, the largest one 11 %.
+float split_us(const MbconvParams &p, int kse, int tw, int pt)
+{
+    const long long tiles = (long long)p.batch * ((p.out_w + tw - 1) / tw) * ((p.out_h + pt - 1) / pt);
+    const float work = (float)(tiles * ((p.exp_c + 63) / 64)) * (1.f / 256.f), k = (float)(kse - 1), he = p.half_even ? 1.f : 0.f;
+    if (p.stride_h == 2)
+        return pt == 1 ? (2.91f + 0.25f * k + work * (0.453f + 0.022f * k)) * (1.f + 0.04f * he)
+            : pt == 2  ? (3.2f + 0.3f * k + work * (0.564f + 0.046f * k)) * (1.f + 0.05f * he)
+                       : (3.6f + 0.49f * k + work * (0.878f + 0.072f * k)) * (1.f + 0.06f * he);
+    if (pt == 2)
+        return (3.06f + 0.164f * k + work * (tw == 7 ? 0.587f : 0.534f + 0.036f * k)) * (1.f + 0.04f * he);
+    if (pt == 4)
+        return (3.42f + 0.166f * k + work * (tw == 7 ? 0.636f + 0.059f * k : 0.653f + 0.057f * k)) * (1.f + 0.05f * he);
+    return (4.02f + (tw == 7 ? 0.2f : 0.35f) * k + work * (tw == 7 ? 0.674f + 0.1f * k : 0.78f - 0.04f * k)) * (1.f + 0.06f * he);
+}
 
 SplitPlan split_plan(const MbconvParams &p)
 {
@@ -293,36 +335,52 @@ SplitPlan split_plan(const MbconvParams &p)
     plan.kse = (p.in_c + 63) / 64;
     // narrow images and strided blocks take tiles of seven columns (a patch of fifteen columns at stride 2), wide
     // images at stride 1 tiles of fourteen
-    if (p.stride_h == 1) {
-        plan.pt = 7;
-        plan.tw = p.out_w <= 7 ? 7 : 14;
-    } else {
-        plan.pt = 4;
-        plan.tw = 7;
+    plan.tw = p.stride_h == 1 && p.out_w > 7 ? 14 : 7;
+    // fewer rows while that leaves the launch shorter: few images
+    const int rows[2][3] = {{7, 4, 2}, {4, 2, 1}};
+    plan.us = 1e30f;
+    for (const int pt : rows[p.stride_h - 1]) {
+        const float us = split_us(p, plan.kse, plan.tw, pt);
+        if (us < plan.us) {
+            plan.us = us;
+            plan.pt = pt;
+        }
     }
     plan.ok = true;
     return plan;
 }
 
-template <int PT, int TW, int S, int KSE, bool HE>
+template <int PT, int TW, int S, int KSE, bool HE, bool LOOP>
 hipError_t launch_tile(const SplitArgs &a, hipStream_t stream)
 {
     const dim3 grid((unsigned)(a.n_tiles * a.parts));
     // (the last k step of the last pixel reads up to 64 bytes past its pixel)
     const size_t lds = (size_t)Tile<PT, TW, S>::NXPT * 16 * a.pitch + 256;
     if (a.p.clip_e || a.p.clip_d)
-        hipLaunchKernelGGL((mbconv_s8_expand_dw_kernel<PT, TW, S, KSE, HE, true>), grid, dim3(kThreads), lds, stream, a);
+        hipLaunchKernelGGL((mbconv_s8_expand_dw_kernel<PT, TW, S, KSE, HE, true, LOOP>), grid, dim3(kThreads), lds, stream, a);
     else
-        hipLaunchKernelGGL((mbconv_s8_expand_dw_kernel<PT, TW, S, KSE, HE, false>), grid, dim3(kThreads), lds, stream, a);
+        hipLaunchKernelGGL((mbconv_s8_expand_dw_kernel<PT, TW, S, KSE, HE, false, LOOP>), grid, dim3(kThreads), lds, stream, a);
     return hipGetLastError();
 }
 
 template <int KSE, bool HE>
 hipError_t launch_kse(const SplitPlan &plan, const SplitArgs &a, hipStream_t stream)
 {
+    if (a.per_wg > 1)
+        return a.p.stride_h == 2 ? launch_tile<4, 7, 2, KSE, HE, true>(a, stream)
+            : plan.tw == 7       ? launch_tile<7, 7, 1, KSE, HE, true>(a, stream)
+                                 : launch_tile<7, 14, 1, KSE, HE, true>(a, stream);
     if (a.p.stride_h == 2)
-        return launch_tile<4, 7, 2, KSE, HE>(a, stream);
-    return plan.tw == 7 ? launch_tile<7, 7, 1, KSE, HE>(a, stream) : launch_tile<7, 14, 1, KSE, HE>(a, stream);
+        return plan.pt == 1 ? launch_tile<1, 7, 2, KSE, HE, false>(a, stream)
+            : plan.pt == 2  ? launch_tile<2, 7, 2, KSE, HE, false>(a, stream)
+                            : launch_tile<4, 7, 2, KSE, HE, false>(a, stream);
+    if (plan.tw == 7)
+        return plan.pt == 2 ? launch_tile<2, 7, 1, KSE, HE, false>(a, stream)
+            : plan.pt == 4  ? launch_tile<4, 7, 1, KSE, HE, false>(a, stream)
+                            : launch_tile<7, 7, 1, KSE, HE, false>(a, stream);
+    return plan.pt == 2 ? launch_tile<2, 14, 1, KSE, HE, false>(a, stream)
+        : plan.pt == 4  ? launch_tile<4, 14, 1, KSE, HE, false>(a, stream)
+                        : launch_tile<7, 14, 1, KSE, HE, false>(a, stream);
 }
 
 template <bool HE>
@@ -345,13 +403,9 @@ bool mbconv_s8_split_supports(const MbconvParams &p)
     return split_plan(p).ok;
 }
 
-// Launch and one chunk's chain, then all chunks over the device (MobileNetV2's blocks at batch 1 to 256, within 15 %).
 float mbconv_s8_expand_dw_us(const MbconvParams &p)
 {
-    const SplitPlan plan = split_plan(p);
-    const float tiles = (float)((long long)p.batch * ((p.out_w + plan.tw - 1) / plan.tw) * ((p.out_h + plan.pt - 1) / plan.pt));
-    const float chunks = 1e-3f * tiles * (float)(p.exp_c / 16) * (p.half_even ? 1.2f : 1.f);
-    return (p.stride_h == 1 ? 4.3f + (plan.tw == 14 ? 1.9f : 1.3f) * chunks : 4.0f + 0.85f * chunks) * (1.f + 0.12f * (float)(plan.kse - 1));
+    return split_plan(p).us;
 }
 
 hipError_t launch_mbconv_s8_expand_dw(const MbconvParams &p, int8_t *mid, int cu_count, hipStream_t stream)
@@ -372,6 +426,8 @@ hipError_t launch_mbconv_s8_expand_dw(const MbconvParams &p, int8_t *mid, int cu
     // As many groups per workgroup as leave four workgroups per compute unit: the patch is loaded once for all of them.
     const long long cus = cu_count > 0 ? cu_count : 256;
     a.per_wg = (int)std::min<long long>(a.n_groups, std::max<long long>(1, tiles * a.n_groups / (4 * cus)));
+    if (plan.pt != (p.stride_h == 1 ? 7 : 4))
+        a.per_wg = 1;
     a.parts = (a.n_groups + a.per_wg - 1) / a.per_wg;
     a.per_wg = (a.n_groups + a.parts - 1) / a.parts;
     if (tiles * a.parts > 0x7fffffff)
