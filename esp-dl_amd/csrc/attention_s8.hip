@@ -20,14 +20,18 @@
 //   2. The registers become probabilities.  The exact result is an IEEE division, but only its rounding to int8 is
 //      kept: a product with the reciprocal decides it unless it lies within 2^-18 of a rounding boundary; there the lane
 //      divides.
-//   3. v is brought in 64 positions at a time by the whole workgroup, transposed in registers (4 x 4 bytes per lane)
-//      on its way into LDS, and multiplied by the probabilities, a half of the head's channels per wavefront of a pair.
-//      A tile's operand-A row m is channel (m / 4) * 4 HT + 4 t + m % 4 of the head, so a lane ends with neighbouring
-//      channels of one position.
-// Not bound by memory or the matrix pipe; two workgroups fit on a compute unit.  The serial additions, 12 cycles each, are 2 us of
-// a launch with 400 positions; how the rest divides between the steps and their walk through LDS has not been measured.  400 positions, 64 images x heads of 32 + 32 + 64 channels take 15.4 us where the operators
-// one by one took 117 us.  Four wavefronts that each owned 16 queries and re-read their scores from LDS took 18.3 us
-// (13.3 us for a single image, now 11.4 us), a ninth wavefront that only adds 17.7 us.
+//   3. v is brought in by the whole workgroup, as many positions as fit where the table values lay (512 of them at 64 channels),
+//      transposed in registers on its way into LDS, and multiplied by the probabilities, a half of the head's channels per
+//      wavefront of a pair.  A tile's operand-A row m is channel (m / 4) * 4 HT + 4 t + m % 4 of the head, so a lane ends with
+//      neighbouring channels of one position.
+// Not bound by memory or the matrix pipe; two workgroups fit on a compute unit.  Of 9.6 us with 400 positions and one image (two heads
+// of 32 + 32 + 64 channels) the scores take 4.2, in which one wavefront's additions and its next scores follow each other seven
+// times (without additions 3.1, without lookups either 2.5), the probabilities 1.1, v and its product 1.2; 64 heads 13.5, the operators
+// one by one 117 us.  With v a chunk of 64 and a barrier at a time, the epilogue's form chosen at run time and divisions out of line
+// one image took 10.7 us, eight 11.3 (10.6 now), 64 heads 14.3.  Tried: a wavefront that owns 16 queries and all keys, sums passed from
+// row to row by v_permlane swaps, k and v in LDS, no barriers (9.5 us for one image, 15 for 64 heads: four times the additions); three
+// chunks of k on their way (14.0); four wavefronts that each owned 16 queries and re-read their scores from LDS (18.3), a ninth
+// wavefront that only adds (17.7).
 #include "conv_window.h"
 
 namespace espdl {
@@ -35,48 +39,33 @@ namespace {
 
 constexpr int kThreads = 512, kQueries = 64;
 constexpr int kSumStride = 68; // floats per query row of the table values: 4 mod 64 banks, rows apart
-constexpr int kVStride = 80;   // bytes per channel row of transposed v: 16 rows of 16 bytes hit distinct banks
 
 struct Args {
     AttentionParams p;
     int prob_stride;  // bytes per row of probabilities: positions rounded up to 64, + 16 so that rows start in different banks
     int chunks;       // of 64 positions
-    int qk_mode, av_mode; // 0: short epilogue, half up; 1: short, half even; 2: general
+    int v_chunks;     // of v in LDS at a time
+    int v_stride;     // bytes per channel row of transposed v: 64 v_chunks + 16, 16 rows of 16 bytes hit distinct banks
+    int av_mode;      // of the second product's epilogue, see requant4
     FastDiv fd_n16;   // 16-byte pieces of a head's values
     float inv_scale;
     float table[256];
 };
 
-// Out of line: shifts no exported block has, from every step of an unrolled loop.
-__device__ __attribute__((noinline)) int requant4_any(v4i acc, int shift, int relu, int half_even)
+// Four accumulators requantized and packed.  MODE 0: short epilogue, half up; 1: short, half even; both hold 2^(s-1) (- 1) already;
+// 2: general.
+template <int MODE>
+__device__ __forceinline__ int requant4(const v4i &acc, int shift, int relu, int half_even)
 {
-    int q[4];
+    if constexpr (MODE == 2) {
+        int q[4];
 #pragma unroll
-    for (int e = 0; e < 4; e++)
-        q[e] = requant_s8(acc[e], shift, relu != 0, half_even != 0);
-    return pack4_s8(q[0], q[1], q[2], q[3]);
-}
-
-// N accumulators requantized, packed four to a dword.  Modes 0 and 1 hold 2^(s-1) (- 1) already.  The (uniform) choice
-// is made once for all of them, so that what follows is one run of independent instructions.
-template <int N>
-__device__ __forceinline__ void requant4(const v4i (&acc)[N], int (&out)[N], int mode, int shift, int relu, int half_even)
-{
-    const int l = max(0, 8 - shift), r = shift - 8 + l;
-    const v4i lsh = {l, l, l, l}, rsh = {r, r, r, r};
-    const int floor_pk = relu ? 0 : (int)0x80008000u;
-    if (mode == 0) {
-#pragma unroll
-        for (int t = 0; t < N; t++)
-            out[t] = pack_fast4<1>(acc[t], lsh, rsh, floor_pk);
-    } else if (mode == 1) {
-#pragma unroll
-        for (int t = 0; t < N; t++)
-            out[t] = pack_fast4<5>(acc[t], lsh, rsh, floor_pk);
+        for (int e = 0; e < 4; e++)
+            q[e] = requant_s8(acc[e], shift, relu != 0, half_even != 0);
+        return pack4_s8(q[0], q[1], q[2], q[3]);
     } else {
-#pragma unroll
-        for (int t = 0; t < N; t++)
-            out[t] = requant4_any(acc[t], shift, relu, half_even);
+        const int l = max(0, 8 - shift), r = shift - 8 + l;
+        return pack_fast4<MODE == 0 ? 1 : 5>(acc, v4i{l, l, l, l}, v4i{r, r, r, r}, relu ? 0 : (int)0x80008000u);
     }
 }
 __device__ __forceinline__ v4i start4(int mode, int shift)
@@ -85,8 +74,8 @@ __device__ __forceinline__ v4i start4(int mode, int shift)
     return v4i{v, v, v, v};
 }
 
-// QuantizeLinear of four elements of Softmax.  Out of line: rarely taken, from every step of an unrolled loop.
-__device__ __attribute__((noinline)) unsigned divide4(float4 e, float sum, float inv_scale)
+// QuantizeLinear of four elements of Softmax.
+__device__ __forceinline__ unsigned divide4(const float4 &e, float sum, float inv_scale)
 {
     const float v[4] = {e.x, e.y, e.z, e.w};
     int q[4];
@@ -100,7 +89,7 @@ __device__ __attribute__((noinline)) unsigned divide4(float4 e, float sum, float
 
 // HT: 16-channel tiles of a head's values (head_dim <= 16 HT, even).
 // CH: chunks whose table values a lane keeps in registers (positions <= 64 CH).
-template <int HT, int CH>
+template <int HT, int CH, int MODE>
 __global__ __launch_bounds__(kThreads) void attention_s8_kernel(const Args a)
 {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -146,7 +135,7 @@ __global__ __launch_bounds__(kThreads) void attention_s8_kernel(const Args a)
     v4i kf[2];
     kf[0] = load(32 * half + r, p.k_offset);
     kf[1] = load(32 * half + 16 + r, p.k_offset);
-    const v4i qk_start = start4(a.qk_mode, p.qk_shift);
+    const v4i qk_start = start4(MODE, p.qk_shift);
     float4 kept[CH][2]; // table values of the lane's keys 64 c + 32 half + 16 t + 4 g + (0 .. 3), query r
     __syncthreads();    // the table is there
 #pragma unroll
@@ -160,7 +149,9 @@ __global__ __launch_bounds__(kThreads) void attention_s8_kernel(const Args a)
             for (int t = 0; t < 2; t++) // (past the last chunk: zeros nobody reads)
                 kf[t] = load(64 * (c + 1) + 32 * half + 16 * t + r, p.k_offset);
             int s[2];
-            requant4<2>(acc, s, a.qk_mode, p.qk_shift, p.qk_relu, p.half_even);
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+                s[t] = requant4<MODE>(acc[t], p.qk_shift, p.qk_relu, p.half_even);
             const int n0 = L - (64 * c + 32 * half + 4 * g); // keys of the image from the lane's first on
             float *to = reinterpret_cast<float *>(scratch) + ((c & 1) * kQueries + pair * 16 + r) * kSumStride + 32 * half + 4 * g;
 #pragma unroll
@@ -200,21 +191,44 @@ __global__ __launch_bounds__(kThreads) void attention_s8_kernel(const Args a)
         }
     }
 
-    // the first 64 positions of v arrive while the last chunk is added and the probabilities are formed
-    constexpr int kBlocks = HT * 4 * 16;                        // 4 x 4 byte blocks of a chunk
-    constexpr int kPer = (kBlocks + kThreads - 1) / kThreads; // per lane
-    int vr[kPer][4];
-    auto load_values = [&](int c) {
+    // v, as much of it as fits where the table values lay: a piece is eight channels of four positions, transposed in registers on
+    // its way, two pieces a thread at a time.  The first ones arrive while the last chunk is added and the probabilities are formed.
+    constexpr int kPerChunk = 2 * HT * 16; // pieces of a chunk of 64 positions
+    const int v_at = tid % (2 * HT);       // the thread's eight channels
+    v2i vr[2][4];
+    const auto load_values = [&](int first, int end) {
 #pragma unroll
-        for (int b = 0; b < kPer; b++) {
-            const int at = tid + b * kThreads;
-            const int off = at < kBlocks ? (64 * c + 4 * (at / (4 * HT))) * C + ch0 + p.v_offset + 4 * (at % (4 * HT)) : window::kParked;
+        for (int j = 0; j < 2; j++) {
+            const int piece = first + j * kThreads;
+            const int off = 8 * v_at < p.head_dim && piece < end ? 4 * (piece / (2 * HT)) * C + ch0 + p.v_offset + 8 * v_at : window::kParked;
 #pragma unroll
             for (int e = 0; e < 4; e++)
-                vr[b][e] = __builtin_amdgcn_raw_buffer_load_b32(qkv, off + e * C, 0, 0);
+                vr[j][e] = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(qkv, off + e * C, 0, 0));
         }
     };
-    load_values(0);
+    const auto place_values = [&](int first, int end, int first_chunk) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int piece = first + j * kThreads;
+#pragma unroll
+            for (int d = 0; d < 2; d++) {
+                if (piece >= end)
+                    continue;
+                // channel 4 db + e of the head is row (db % HT) * 16 + (db / HT) * 4 + e
+                const int db = 2 * v_at + d;
+                unsigned char *const dst = scratch + ((db % HT) * 16 + (db / HT) * 4) * a.v_stride + 4 * (piece / (2 * HT)) - 64 * first_chunk;
+                const unsigned t0 = __builtin_amdgcn_perm((unsigned)vr[j][1][d], (unsigned)vr[j][0][d], 0x05010400u);
+                const unsigned t1 = __builtin_amdgcn_perm((unsigned)vr[j][1][d], (unsigned)vr[j][0][d], 0x07030602u);
+                const unsigned u0 = __builtin_amdgcn_perm((unsigned)vr[j][3][d], (unsigned)vr[j][2][d], 0x05010400u);
+                const unsigned u1 = __builtin_amdgcn_perm((unsigned)vr[j][3][d], (unsigned)vr[j][2][d], 0x07030602u);
+                *reinterpret_cast<unsigned *>(dst) = __builtin_amdgcn_perm(u0, t0, 0x05040100u);
+                *reinterpret_cast<unsigned *>(dst + a.v_stride) = __builtin_amdgcn_perm(u0, t0, 0x07060302u);
+                *reinterpret_cast<unsigned *>(dst + 2 * a.v_stride) = __builtin_amdgcn_perm(u1, t1, 0x05040100u);
+                *reinterpret_cast<unsigned *>(dst + 3 * a.v_stride) = __builtin_amdgcn_perm(u1, t1, 0x07060302u);
+            }
+        }
+    };
+    load_values(tid, min(a.v_chunks, a.chunks) * kPerChunk);
     __syncthreads(); // the sums are there, the table values are done with
 
     // Probabilities.  v_cvt_pk_u8_f32 rounds to nearest and saturates at 255; the two factors bracket the exact one by
@@ -227,6 +241,7 @@ __global__ __launch_bounds__(kThreads) void attention_s8_kernel(const Args a)
 #pragma unroll
     for (int c = 0; c < CH; c++) {
         if (c < a.chunks) {
+            unsigned w[2], differ = 0;
 #pragma unroll
             for (int t = 0; t < 2; t++) {
                 const float e[4] = {kept[c][t].x, kept[c][t].y, kept[c][t].z, kept[c][t].w};
@@ -237,11 +252,16 @@ __global__ __launch_bounds__(kThreads) void attention_s8_kernel(const Args a)
                     hi = __builtin_amdgcn_cvt_pk_u8_f32(e[b] * factor_hi, b, hi);
                 }
                 const unsigned over = lo & 0x80808080u; // 128 .. 255 become 127
-                unsigned w = (lo | (over - (over >> 7))) & 0x7f7f7f7fu;
-                if (lo != hi || !short_sum)
-                    w = divide4(kept[c][t], sum, a.inv_scale);
-                *reinterpret_cast<unsigned *>(prob_row + 64 * c + 32 * half + 16 * t + 4 * g) = w;
+                w[t] = (lo | (over - (over >> 7))) & 0x7f7f7f7fu;
+                differ |= lo ^ hi;
             }
+            if (differ != 0 || !short_sum)
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+                    w[t] = divide4(kept[c][t], sum, a.inv_scale);
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+                *reinterpret_cast<unsigned *>(prob_row + 64 * c + 32 * half + 16 * t + 4 * g) = w[t];
         }
     }
 
@@ -250,33 +270,26 @@ __global__ __launch_bounds__(kThreads) void attention_s8_kernel(const Args a)
 #pragma unroll
     for (int t = 0; t < HT / 2; t++)
         acc[t] = av_start;
-    for (int c = 0; c < a.chunks; c++) {
-        unsigned char *buf = scratch + (c & 1) * (16 * HT * kVStride);
-#pragma unroll
-        for (int b = 0; b < kPer; b++) {
-            const int at = tid + b * kThreads;
-            if (at >= kBlocks)
-                break;
-            const int db = at % (4 * HT);
-            // channel 4 db + e of the head is row (db % HT) * 16 + (db / HT) * 4 + e
-            unsigned char *dst = buf + ((db % HT) * 16 + (db / HT) * 4) * kVStride + 4 * (at / (4 * HT));
-            const unsigned t0 = __builtin_amdgcn_perm((unsigned)vr[b][1], (unsigned)vr[b][0], 0x05010400u);
-            const unsigned t1 = __builtin_amdgcn_perm((unsigned)vr[b][1], (unsigned)vr[b][0], 0x07030602u);
-            const unsigned u0 = __builtin_amdgcn_perm((unsigned)vr[b][3], (unsigned)vr[b][2], 0x05010400u);
-            const unsigned u1 = __builtin_amdgcn_perm((unsigned)vr[b][3], (unsigned)vr[b][2], 0x07030602u);
-            *reinterpret_cast<unsigned *>(dst) = __builtin_amdgcn_perm(u0, t0, 0x05040100u);
-            *reinterpret_cast<unsigned *>(dst + kVStride) = __builtin_amdgcn_perm(u0, t0, 0x07060302u);
-            *reinterpret_cast<unsigned *>(dst + 2 * kVStride) = __builtin_amdgcn_perm(u1, t1, 0x05040100u);
-            *reinterpret_cast<unsigned *>(dst + 3 * kVStride) = __builtin_amdgcn_perm(u1, t1, 0x07060302u);
+    for (int c0 = 0; c0 < a.chunks; c0 += a.v_chunks) {
+        const int c1 = min(c0 + a.v_chunks, a.chunks), end = c1 * kPerChunk;
+        if (c0 != 0) {
+            __syncthreads(); // the chunks before have been read
+            load_values(c0 * kPerChunk + tid, end);
         }
-        if (c + 1 < a.chunks)
-            load_values(c + 1);
-        __syncthreads(); // one barrier per chunk: the buffer written next was read before this one
-        const v4i pf = *reinterpret_cast<const v4i *>(prob_row + 64 * c + 16 * g);
+        for (int piece = c0 * kPerChunk + tid; piece - tid < end; piece += 2 * kThreads) {
+            place_values(piece, end, c0);
+            if (piece - tid + 2 * kThreads < end) // uniform
+                load_values(piece + 2 * kThreads, end);
+        }
+        __syncthreads();
+        const unsigned char *const row = scratch + (16 * half * (HT / 2) + r) * a.v_stride + 16 * g;
+        for (int c = c0; c < c1; c++) {
+            const v4i pf = *reinterpret_cast<const v4i *>(prob_row + 64 * c + 16 * g);
 #pragma unroll
-        for (int t = 0; t < HT / 2; t++) {
-            const v4i vf = *reinterpret_cast<const v4i *>(buf + (16 * (half * (HT / 2) + t) + r) * kVStride + 16 * g);
-            acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(vf, pf, acc[t], 0, 0, 0);
+            for (int t = 0; t < HT / 2; t++) {
+                const v4i vf = *reinterpret_cast<const v4i *>(row + 16 * t * a.v_stride + 64 * (c - c0));
+                acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(vf, pf, acc[t], 0, 0, 0);
+            }
         }
     }
     const int i = i0 + r;
@@ -284,7 +297,11 @@ __global__ __launch_bounds__(kThreads) void attention_s8_kernel(const Args a)
         const int d0 = g * 4 * HT + half * 2 * HT;
         int8_t *dst = p.out + ((long long)image * L + i) * (p.heads * p.head_dim) + head * p.head_dim + d0;
         int word[HT / 2];
-        requant4<HT / 2>(acc, word, a.av_mode, p.av_shift, p.av_relu, p.half_even);
+#pragma unroll
+        for (int t = 0; t < HT / 2; t++)
+            word[t] = a.av_mode == 0 ? requant4<0>(acc[t], p.av_shift, p.av_relu, 0) // (uniform)
+                : a.av_mode == 1     ? requant4<1>(acc[t], p.av_shift, p.av_relu, 1)
+                                     : requant4<2>(acc[t], p.av_shift, p.av_relu, p.half_even);
 #pragma unroll
         for (int t = 0; t < HT / 2; t++)
             if (d0 + 4 * t < p.head_dim)
@@ -292,11 +309,10 @@ __global__ __launch_bounds__(kThreads) void attention_s8_kernel(const Args a)
     }
 }
 
-size_t lds_bytes(int positions, int ht)
+// Bytes where the table values of two chunks lie, then v: more than that only where a single chunk of v needs it.
+size_t scratch_bytes(int ht)
 {
-    const size_t probs = (size_t)kQueries * ((positions + 63) / 64 * 64 + 16);
-    const size_t values = (size_t)2 * 16 * ht * kVStride, table_values = sizeof(float) * 2 * kQueries * kSumStride;
-    return (256 + kQueries) * sizeof(float) + probs + std::max(values, table_values);
+    return std::max((size_t)16 * ht * (64 + 16), sizeof(float) * 2 * kQueries * kSumStride);
 }
 int value_tiles(int head_dim)
 {
@@ -309,6 +325,14 @@ int epilogue_mode(int shift, int half_even, long long mac_bound)
     if (shift < 1 || shift > 31 || mac_bound + (1ll << (shift - 1)) >= 1ll << (31 - std::max(0, 8 - shift)))
         return 2;
     return half_even ? 1 : 0;
+}
+
+template <int HT>
+auto pick_kernel(int chunks, int mode)
+{
+    if (chunks <= 8)
+        return mode == 0 ? attention_s8_kernel<HT, 8, 0> : mode == 1 ? attention_s8_kernel<HT, 8, 1> : attention_s8_kernel<HT, 8, 2>;
+    return mode == 0 ? attention_s8_kernel<HT, 16, 0> : mode == 1 ? attention_s8_kernel<HT, 16, 1> : attention_s8_kernel<HT, 16, 2>;
 }
 
 } // namespace
@@ -330,7 +354,7 @@ hipError_t launch_attention_s8(const AttentionParams &params, hipStream_t stream
     a.p = params;
     a.prob_stride = (params.positions + 63) / 64 * 64 + 16;
     a.chunks = (params.positions + 63) / 64;
-    a.qk_mode = epilogue_mode(params.qk_shift, params.half_even, 128ll * 128 * params.key_dim);
+    const int qk_mode = epilogue_mode(params.qk_shift, params.half_even, 128ll * 128 * params.key_dim);
     a.av_mode = epilogue_mode(params.av_shift, params.half_even, 128ll * 128 * params.positions);
     a.fd_n16 = make_fastdiv((unsigned)(params.head_dim >> 4));
     a.inv_scale = dl_rescale(params.prob_exp);
@@ -338,11 +362,10 @@ hipError_t launch_attention_s8(const AttentionParams &params, hipStream_t stream
     for (int i = 0; i < 256; i++)
         a.table[i] = expf(scale * (float)(i - 128));
     const int ht = value_tiles(params.head_dim);
-    const size_t lds = lds_bytes(params.positions, ht);
-    const auto pick = [&](auto few, auto many) { return a.chunks <= 8 ? few : many; };
-    const auto kernel = ht == 2 ? pick(attention_s8_kernel<2, 8>, attention_s8_kernel<2, 16>)
-        : ht == 4               ? pick(attention_s8_kernel<4, 8>, attention_s8_kernel<4, 16>)
-                                : pick(attention_s8_kernel<8, 8>, attention_s8_kernel<8, 16>);
+    a.v_chunks = std::min(a.chunks, (int)((scratch_bytes(ht) / (16 * ht) - 16) / 64));
+    a.v_stride = 64 * a.v_chunks + 16;
+    const size_t lds = (256 + kQueries) * sizeof(float) + (size_t)kQueries * a.prob_stride + scratch_bytes(ht);
+    const auto kernel = ht == 2 ? pick_kernel<2>(a.chunks, qk_mode) : ht == 4 ? pick_kernel<4>(a.chunks, qk_mode) : pick_kernel<8>(a.chunks, qk_mode);
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     const int images = 65535 / params.heads; // per launch: grid.y is 16 bits wide
     const long long in_image = (long long)params.positions * params.channels;

@@ -302,6 +302,8 @@ ATTENTION_CASES = [
     (1, 19, 27, 1, 32, 16, 9, 7, -3, -8, 8, (0, 0)),       # one key past eight chunks
     (1, 1, 3, 2, 48, 32, 0, -1, -4, -7, -2, (0, 0)),       # left shifts: the general epilogue
     (1, 32, 32, 1, 16, 32, 5, 9, -2, -8, 3, (0, 0)),       # the longest row; small scores, quotients on ties
+    (2, 17, 20, 1, 32, 112, 9, 7, -3, -8, 8, (0, 0)),      # v in LDS in two parts, the second with a part of a chunk
+    (1, 24, 25, 2, 16, 64, 8, None, -4, -8, 7, (1, 1)),    # the same with the scores of more than eight chunks
 ]
 
 
