@@ -27,14 +27,28 @@ inline bool aligned16(const void *a, const void *b)
     return ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0;
 }
 
-// A per-byte functor applied over a flat tensor.
-template <typename F>
+// Vector i of an operand.  PAST: read for the last time, see reads_past_cache.
+template <bool PAST>
+__device__ __forceinline__ v4i load_vec(const int8_t *p, int64_t i)
+{
+    const v4i *v = reinterpret_cast<const v4i *>(p) + i;
+    if constexpr (PAST)
+        return __builtin_nontemporal_load(v);
+    else
+        return *v;
+}
+
+// A per-byte functor applied over a flat tensor.  The vector is requested before the functor's table, whose barrier it would
+// wait for (462 MB in and out: 80 -> 78 us).
+template <typename F, bool PAST>
 __global__ __launch_bounds__(kBlock) void map_s8_kernel(const int8_t *in, int8_t *out, int64_t size, int64_t vecs, F f)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    v4i v = {};
+    if (i < vecs)
+        v = load_vec<PAST>(in, i);
     f.prepare();
     if (i < vecs) {
-        const v4i v = reinterpret_cast<const v4i *>(in)[i];
         v4i r;
 #pragma unroll
         for (int w = 0; w < 4; w++) {
@@ -127,7 +141,8 @@ hipError_t launch_map(const int8_t *in, int8_t *out, int64_t size, F f, hipStrea
         return hipSuccess;
     int64_t vecs;
     const dim3 grid = grid_for(size, aligned16(in, out), &vecs);
-    hipLaunchKernelGGL(map_s8_kernel<F>, grid, dim3(kBlock), 0, stream, in, out, size, vecs, f);
+    const auto kernel = reads_past_cache(size) ? map_s8_kernel<F, true> : map_s8_kernel<F, false>;
+    hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, stream, in, out, size, vecs, f);
     return hipGetLastError();
 }
 
@@ -146,14 +161,14 @@ struct MulOp {
     __device__ __forceinline__ int apply(int a, int b) const { return requant_s8(a * b, shift, false, half_even); }
 };
 
-template <typename Op>
+template <typename Op, bool PAST>
 __global__ __launch_bounds__(kBlock) void binary_s8_dense_kernel(const int8_t *in0, const int8_t *in1, int8_t *out,
                                                                  int64_t size, int64_t vecs, Op op)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < vecs) {
-        const v4i a = reinterpret_cast<const v4i *>(in0)[i];
-        const v4i b = reinterpret_cast<const v4i *>(in1)[i];
+        const v4i a = load_vec<PAST>(in0, i);
+        const v4i b = load_vec<PAST>(in1, i);
         v4i r;
 #pragma unroll
         for (int w = 0; w < 4; w++) {
@@ -214,7 +229,8 @@ hipError_t launch_binary_s8(const int32_t dims[4], const int64_t s0[4], const in
         const bool vec_ok = aligned16(in0, in1) && aligned16(out, out);
         int64_t vecs;
         const dim3 grid = grid_for(size, vec_ok, &vecs);
-        hipLaunchKernelGGL(binary_s8_dense_kernel<Op>, grid, dim3(kBlock), 0, stream, in0, in1, out, size, vecs, op);
+        const auto kernel = reads_past_cache(size) ? binary_s8_dense_kernel<Op, true> : binary_s8_dense_kernel<Op, false>;
+        hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, stream, in0, in1, out, size, vecs, op);
     } else if (binary_vec::Args va; binary_vec::plan(dims, s0, s1, in0, in1, out, &va)) {
         // innermost axis dense or constant in each operand (a channel-wise scale, a per-row offset): 16 bytes per thread
         return binary_vec::launch(in0, in1, out, va, op, 0, stream);
@@ -318,6 +334,7 @@ namespace {
 // PReLU: 16 bytes of the flat tensor per thread.  Their slopes are 16 bytes of alpha at the first one's channel, at whatever
 // address that is; only where the channels start over among the 16 are they gathered one by one (36 x 8 x 194, 128
 // images: 5.8 us; with a 64-bit division per byte, as odd channel counts had before, 9.8 us).
+template <bool PAST>
 __global__ __launch_bounds__(kBlock) void prelu_s8_vec_kernel(const int8_t *in, const int8_t *alpha, int8_t *out, int64_t size,
                                                               int64_t vecs, int channels, int shift)
 {
@@ -325,7 +342,7 @@ __global__ __launch_bounds__(kBlock) void prelu_s8_vec_kernel(const int8_t *in, 
     const PreluFn f{alpha, channels, shift};
     if (i < vecs) {
         const int c = vecs <= (1ll << 27) ? (int)((unsigned)(i * 16) % (unsigned)channels) : (int)((uint64_t)(i * 16) % (unsigned)channels);
-        const v4i x = reinterpret_cast<const v4i *>(in)[i];
+        const v4i x = load_vec<PAST>(in, i);
         v4i s, r;
         if (c + 16 <= channels) {
             s = *reinterpret_cast<const v4i_unaligned *>(alpha + c);
@@ -365,7 +382,8 @@ hipError_t launch_prelu_s8(const int8_t *in, int64_t pixels, int channels, const
         return hipSuccess;
     int64_t vecs;
     const dim3 grid = grid_for(size, aligned16(in, out), &vecs);
-    hipLaunchKernelGGL(prelu_s8_vec_kernel, grid, dim3(kBlock), 0, stream, in, alpha, out, size, vecs, channels, shift);
+    const auto kernel = reads_past_cache(size) ? prelu_s8_vec_kernel<true> : prelu_s8_vec_kernel<false>;
+    hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, stream, in, alpha, out, size, vecs, channels, shift);
     return hipGetLastError();
 }
 
@@ -378,6 +396,7 @@ namespace {
 // Clip between equal exponents: the rescale factor is 1 and the operator is a clamp of the stored value.  Four
 // bytes per packed-int16 sequence: the bytes go to the high bytes of two int16 pairs (x * 256), one packed
 // maximum and minimum against (lo << 8) and (hi << 8) | 0xff, the high bytes are gathered again.
+template <bool PAST>
 __global__ __launch_bounds__(kBlock) void clamp_s8_kernel(const int8_t *in, int8_t *out, int64_t size, int64_t vecs, int lo,
                                                           int hi)
 {
@@ -385,7 +404,7 @@ __global__ __launch_bounds__(kBlock) void clamp_s8_kernel(const int8_t *in, int8
     const v2s lo2 = __builtin_bit_cast(v2s, ((lo << 8) & 0xffff) * 0x10001);
     const v2s hi2 = __builtin_bit_cast(v2s, (((hi << 8) | 0xff) & 0xffff) * 0x10001);
     if (i < vecs) {
-        const v4i v = reinterpret_cast<const v4i *>(in)[i];
+        const v4i v = load_vec<PAST>(in, i);
         v4i r;
 #pragma unroll
         for (int w = 0; w < 4; w++) {
@@ -413,7 +432,8 @@ hipError_t launch_clip_s8(const int8_t *in, int64_t size, int min_q, int max_q, 
         const int64_t work = std::max<int64_t>(vecs, size - vecs * 16);
         if (work <= 0)
             return hipSuccess;
-        hipLaunchKernelGGL(clamp_s8_kernel, dim3((unsigned)((work + kBlock - 1) / kBlock)), dim3(kBlock), 0, stream, in, out,
+        const auto kernel = reads_past_cache(size) ? clamp_s8_kernel<true> : clamp_s8_kernel<false>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((work + kBlock - 1) / kBlock)), dim3(kBlock), 0, stream, in, out,
                            size, vecs, min_q, max_q);
         return hipGetLastError();
     }
@@ -424,13 +444,14 @@ namespace {
 // int8 -> int8 between exponents at most 7 apart: four values per packed-int16 sequence (requant4_s8: round half
 // up of x * 2^d, saturated - what RequantFn computes in float, where both scales are powers of two and every step
 // is exact); bytes past the last 16-byte vector take RequantFn itself.
+template <bool PAST>
 __global__ __launch_bounds__(kBlock) void requantize_pow2_s8_kernel(const int8_t *in, int8_t *out, int64_t size, int64_t vecs,
                                                                     int d, RequantFn tail)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const Requant4 q = make_requant4(d);
     if (i < vecs) {
-        const v4i v = reinterpret_cast<const v4i *>(in)[i];
+        const v4i v = load_vec<PAST>(in, i);
         v4i r;
 #pragma unroll
         for (int w = 0; w < 4; w++)
@@ -456,7 +477,8 @@ hipError_t launch_requantize_s8(const int8_t *in, int64_t size, int in_exp, int 
     if (d >= -7 && d <= 7 && aligned16(in, out) && size >= 16) {
         int64_t vecs;
         const dim3 grid = grid_for(size, true, &vecs);
-        hipLaunchKernelGGL(requantize_pow2_s8_kernel, grid, dim3(kBlock), 0, stream, in, out, size, vecs, d,
+        const auto kernel = reads_past_cache(size) ? requantize_pow2_s8_kernel<true> : requantize_pow2_s8_kernel<false>;
+        hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, stream, in, out, size, vecs, d,
                            RequantFn{dl_scale(in_exp), inv});
         return hipGetLastError();
     }

@@ -32,6 +32,17 @@ inline int writes_through(long long bytes)
 {
     return bytes <= (16ll << 20);
 }
+// Whether an element-wise operator reads an operand of so many bytes with loads that leave no copy behind in the last-level
+// cache.  What an operator has read is mostly read for the last time, what it writes is read next: of large tensors the cache
+// (256 MB) then holds results instead of operands, and the next kernel finds its input there.  Depthwise 3 x 3, PReLU, Add, 5 x 5
+// pool, Concat and table activation in turn over 256 images of 56 x 56 x 144 (116 MB): Add 68 -> 51 us, the pool behind it
+// 65 -> 48, the table 80 -> 70, the chain 392 -> 358.  Operands of 39, 50 and 65 MB: the chain takes 4, 6 and 9 % less; below
+// that everything stays cached either way and such loads cost up to 5 % (4.5 to 16 MB), at 26 and 32 MB 1 to 2 %.  Windows (pool,
+// depthwise, 3 x 3 convolutions) read a pixel several times and lose by them: the pool 48 -> 105 us.
+inline bool reads_past_cache(long long bytes)
+{
+    return bytes > (36ll << 20);
+}
 inline bool conv_is_dense(const ConvGeom &g)
 {
     return g.in_pitch == g.in_c && g.out_pitch == g.out_c && g.res_pitch == g.out_c;

@@ -1170,6 +1170,30 @@ def test_prelu_s8(oracle, shift):
         np.testing.assert_array_equal(got, oracle.prelu_s8(x, alpha, shift))
 
 
+@pytest.mark.parametrize("extra", [0, 16, 16 * 256 + 5], ids=["at the line", "one vector more", "a part of a workgroup and a tail"])
+def test_elementwise_operands_that_leave_no_copy(oracle, extra):
+    """int8 operands around the size from which element-wise operators read past the last-level cache (36 MiB)."""
+    size = (36 << 20) + extra
+    announce(f"elementwise size={size}")
+    m = espdl()
+    rng = np.random.default_rng(extra)
+    a, b = rng_int8(rng, (size,)), rng_int8(rng, (size,))
+    ad, bd = to_dev(a), to_dev(b)
+    table = rng_int8(rng, (256,))
+    want = np.clip(a.astype(np.int16) + b.astype(np.int16), -128, 127).astype(np.int8)
+    np.testing.assert_array_equal(to_host(m.add_s8(ad, bd)), want)
+    np.testing.assert_array_equal(to_host(m.lut_s8(ad, to_dev(table))), oracle.lut_s8(a, table))
+    np.testing.assert_array_equal(to_host(m.clip_s8(ad, -3, 96, -5, -5)), oracle.clip_s8(a, -3, 96, -5, -5))
+    np.testing.assert_array_equal(to_host(m.requantize_s8(ad, -6, -4)), oracle.requantize_s8(a, -6, -4))
+    channels = 48 if size % 48 == 0 else 16 if size % 16 == 0 else 1
+    shape = (1, 1, size // channels, channels)
+    slope = rng_int8(rng, (channels,))
+    np.testing.assert_array_equal(to_host(m.prelu_s8(to_dev(a.reshape(shape)), to_dev(slope), 6)),
+                                  oracle.prelu_s8(a.reshape(shape), slope, 6))
+    m.add_s8(ad, bd, out=ad)  # in place
+    np.testing.assert_array_equal(to_host(ad), want)
+
+
 def test_relu_clip_requantize_s8(oracle):
     announce("relu/clip/requantize")
     m = espdl()

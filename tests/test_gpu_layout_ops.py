@@ -38,6 +38,16 @@ def test_concat(oracle, case, dtype):
     np.testing.assert_array_equal(got, oracle.concat(arrays, axis))
 
 
+@pytest.mark.parametrize("rows,widths", [(1023, [16]), (1024, [16]), (1025, [16]), (256, [33, 17]), (341, [16, 20]), (4097, [144, 144]), (1, [16, 16])])
+def test_concat_in_runs_of_1024_pieces(oracle, rows, widths):
+    """Counts of 16-byte pieces around a workgroup's 1024, with pieces that reach back over their neighbours'."""
+    announce(f"concat {rows} rows of {widths}")
+    rng = np.random.default_rng(rows)
+    arrays = [_rand(rng, (1, 1, rows, w), np.int8) for w in widths]
+    got = to_host(espdl().concat([to_dev(a) for a in arrays], 3))
+    np.testing.assert_array_equal(got, oracle.concat(arrays, 3))
+
+
 @pytest.mark.parametrize("dtype", [np.int8, np.int16])
 @pytest.mark.parametrize("shape,axis,sizes", [
     ((2, 20, 20, 128), 3, [64, 64]), ((2, 9, 9, 48), 3, [5, 20, 23]), ((4, 6, 5, 8), 1, [1, 2, 3]),
