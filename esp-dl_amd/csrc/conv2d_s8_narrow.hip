@@ -137,7 +137,7 @@ struct UnitWalk {
 };
 
 template <int NT, bool SPLIT, bool ALIGNED, bool POINT>
-__global__ __launch_bounds__(kThreads) void conv2d_s8_narrow_kernel(const NarrowArgs a)
+__device__ __forceinline__ void narrow_tile(const NarrowArgs &a, int bx, int by)
 {
     constexpr int G = NT >= 4 ? 2 : 4;
     constexpr int MINE = SPLIT ? 1 : NT; // filter tiles a wavefront finishes
@@ -146,8 +146,8 @@ __global__ __launch_bounds__(kThreads) void conv2d_s8_narrow_kernel(const Narrow
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 15, quad = lane >> 4;
-    const int m = (SPLIT ? (int)blockIdx.x : (int)blockIdx.x * 4 + wave) * 16 + col;
-    const int n0 = blockIdx.y * 16 * NT;
+    const int m = (SPLIT ? bx : bx * 4 + wave) * 16 + col;
+    const int n0 = by * 16 * NT;
 
     // What the epilogue needs is requested first, its addresses take no arithmetic: this wavefront's filter tiles.  Filters
     // past the last one lie past the descriptors' ends and read as zeros.
@@ -315,6 +315,33 @@ __global__ __launch_bounds__(kThreads) void conv2d_s8_narrow_kernel(const Narrow
     }
 }
 
+template <int NT, bool SPLIT, bool ALIGNED, bool POINT>
+__global__ __launch_bounds__(kThreads) void conv2d_s8_narrow_kernel(const NarrowArgs a)
+{
+    narrow_tile<NT, SPLIT, ALIGNED, POINT>(a, (int)blockIdx.x, (int)blockIdx.y);
+}
+
+// Several layers that do not depend on one another in one launch (the same level of a detector's heads): each is too small for
+// the device, and one after the other they pay a launch's 1.2 us and a wavefront's latency each (52, 26 and 13 pixels square, 64 ->
+// 80 with a table, 1 x 1: 11 us one by one, 3.6 together; 3 x 3 of 64, 128, 256 -> 64: 15 and 6).  One filter tile per wavefront
+// for all of them: what that costs a layer that took two by itself, workgroups of the others would have to wait for anyway.
+struct NarrowGroup {
+    NarrowArgs layer[kMostGrouped];
+    int first[kMostGrouped]; // first workgroup of a layer; past the last one: no workgroup reaches it
+    FastDiv columns[kMostGrouped]; // workgroups of a row of its grid
+};
+template <bool SPLIT, bool POINT>
+__global__ __launch_bounds__(kThreads) void conv2d_s8_narrow_group_kernel(const NarrowGroup g)
+{
+    int i = 0;
+#pragma unroll
+    for (int k = 1; k < kMostGrouped; k++)
+        i += (int)blockIdx.x >= g.first[k] ? 1 : 0;
+    const unsigned at = blockIdx.x - g.first[i];
+    const unsigned by = fastdiv(at, g.columns[i]);
+    narrow_tile<1, SPLIT, true, POINT>(g.layer[i], (int)(at - by * g.columns[i].d), (int)by);
+}
+
 template <int NT, bool SPLIT>
 void launch_split(const NarrowArgs &a, bool aligned, bool point, hipStream_t stream)
 {
@@ -338,6 +365,26 @@ void launch_narrow(const NarrowArgs &a, bool split, bool aligned, bool point, hi
     else
         launch_split<NT, false>(a, aligned, point, stream);
 }
+
+void launch_one(const NarrowArgs &a, int nt, bool split, bool aligned, bool point, hipStream_t stream)
+{
+    if (nt == 4)
+        launch_narrow<4>(a, split, aligned, point, stream);
+    else if (nt == 2)
+        launch_narrow<2>(a, split, aligned, point, stream);
+    else
+        launch_narrow<1>(a, split, aligned, point, stream);
+}
+
+// A launch held back in this thread's open group.
+struct Held {
+    NarrowArgs args;
+    int nt;
+    bool split, point;
+    hipStream_t stream;
+};
+thread_local Held held[kMostGrouped];
+thread_local int n_held = 0;
 
 } // namespace
 
@@ -432,13 +479,65 @@ hipError_t launch_conv2d_s8_narrow(const ConvGeom &g, const int8_t *in, const in
     if (point) { // channels past the tap's last one are no next tap
         a.step.in = a.step.filter = 16 * a.step.units;
     }
-    if (p.nt == 4)
-        launch_narrow<4>(a, p.split, aligned, point, stream);
-    else if (p.nt == 2)
-        launch_narrow<2>(a, p.split, aligned, point, stream);
-    else
-        launch_narrow<1>(a, p.split, aligned, point, stream);
+    if (group_open && aligned && p.nt <= 2 && n_held < kMostGrouped) {
+        held[n_held++] = Held{a, p.nt, p.split, point, stream};
+        return hipSuccess;
+    }
+    launch_one(a, p.nt, p.split, aligned, point, stream);
     return hipGetLastError();
+}
+
+// Which of a group's launches a layer takes (0: none), for tensors at aligned addresses.
+int conv2d_s8_narrow_group_kind(const ConvGeom &g, int cu_count)
+{
+    const NarrowPlan p = narrow_plan(g, cu_count);
+    if ((g.in_c & 15) != 0 || (g.in_pitch & 15) != 0 || p.nt > 2)
+        return 0;
+    return 1 + (p.split ? 2 : 0) + (g.k_h == 1 && g.k_w == 1 ? 1 : 0);
+}
+
+// The launches held back since the group was opened: those of one build together, in the order of the first of each.
+hipError_t flush_conv2d_s8_narrow()
+{
+    const int n = n_held;
+    n_held = 0;
+    bool done[kMostGrouped] = {};
+    for (int i = 0; i < n; i++) {
+        if (done[i])
+            continue;
+        const Held &h = held[i];
+        NarrowGroup group;
+        long long blocks = 0;
+        int members = 0;
+        for (int j = i; j < n; j++) {
+            const Held &o = held[j];
+            if (o.split != h.split || o.point != h.point || o.stream != h.stream)
+                continue;
+            const unsigned tiles = (unsigned)((o.args.n_pix + 15) / 16);
+            const unsigned columns = o.split ? tiles : (tiles + 3) / 4;
+            done[j] = true;
+            group.layer[members] = o.args;
+            group.first[members] = (int)blocks;
+            group.columns[members] = make_fastdiv(columns);
+            blocks += (long long)columns * ((o.args.out_c + 15) / 16);
+            members++;
+        }
+        if (members == 1 || blocks > 1 << 20) { // (a group's layers are small)
+            for (int j = i; j < n; j++)
+                if (held[j].split == h.split && held[j].point == h.point && held[j].stream == h.stream)
+                    launch_one(held[j].args, held[j].nt, h.split, true, h.point, h.stream);
+        } else {
+            for (int k = members; k < kMostGrouped; k++) {
+                group.layer[k] = group.layer[0];
+                group.first[k] = (int)blocks;
+                group.columns[k] = group.columns[0];
+            }
+            const auto kernel = h.split ? (h.point ? conv2d_s8_narrow_group_kernel<true, true> : conv2d_s8_narrow_group_kernel<true, false>)
+                                        : (h.point ? conv2d_s8_narrow_group_kernel<false, true> : conv2d_s8_narrow_group_kernel<false, false>);
+            hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kThreads), 0, h.stream, group);
+        }
+    }
+    return n > 0 ? hipGetLastError() : hipSuccess;
 }
 
 } // namespace espdl

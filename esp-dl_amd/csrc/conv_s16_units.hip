@@ -459,8 +459,8 @@ __global__ __launch_bounds__(kThreads) void conv2d_s16_gemm_kernel(const S16Args
     }
 }
 
-template <int NT, bool ALIGNED, bool X8 = false>
-__global__ __launch_bounds__(kThreads) void conv2d_s16_narrow_kernel(const S16Args a)
+template <int NT, bool ALIGNED, bool X8>
+__device__ __forceinline__ void narrow16_tile(const S16Args &a, int bx, int by)
 {
     constexpr int G = 2; // steps per batch of loads
     constexpr int kSums = X8 ? 2 : 3;
@@ -469,8 +469,8 @@ __global__ __launch_bounds__(kThreads) void conv2d_s16_narrow_kernel(const S16Ar
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 15, quad = lane >> 4;
-    const int m = blockIdx.x * 16 + col;
-    const int n0 = blockIdx.y * 16 * NT;
+    const int m = bx * 16 + col;
+    const int n0 = by * 16 * NT;
 
     const __amdgpu_buffer_rsrc_t in_rsrc = tensor_rsrc(a.win.in, a.win.in_bytes);
     const __amdgpu_buffer_rsrc_t w_rsrc = tensor_rsrc(a.win.w, a.win.w_bytes);
@@ -611,6 +611,45 @@ __global__ __launch_bounds__(kThreads) void conv2d_s16_narrow_kernel(const S16Ar
     }
 }
 
+template <int NT, bool ALIGNED, bool X8>
+__global__ __launch_bounds__(kThreads) void conv2d_s16_narrow_kernel(const S16Args a)
+{
+    narrow16_tile<NT, ALIGNED, X8>(a, (int)blockIdx.x, (int)blockIdx.y);
+}
+
+// Several layers that do not depend on one another in one launch, as in conv2d_s8_narrow.hip (64 -> 64 over 52, 26 and 13 pixels
+// square, 3 x 3 on int8 inputs: 18 us one by one, 9 together; 1 x 1: 16 and 7).
+struct S16Group {
+    S16Args layer[kMostGrouped];
+    int first[kMostGrouped];       // first workgroup of a layer
+    FastDiv columns[kMostGrouped]; // workgroups of a row of its grid
+};
+template <bool X8>
+__global__ __launch_bounds__(kThreads) void conv2d_s16_narrow_group_kernel(const S16Group g)
+{
+    int i = 0;
+#pragma unroll
+    for (int k = 1; k < kMostGrouped; k++)
+        i += (int)blockIdx.x >= g.first[k] ? 1 : 0;
+    const unsigned at = blockIdx.x - g.first[i];
+    const unsigned by = fastdiv(at, g.columns[i]);
+    narrow16_tile<1, true, X8>(g.layer[i], (int)(at - by * g.columns[i].d), (int)by);
+}
+
+template <bool X8>
+void launch_narrow16(const S16Args &a, bool two, bool aligned, hipStream_t stream)
+{
+    const dim3 grid((unsigned)((a.n_pix + 15) / 16), (unsigned)(two ? (a.out_c + 31) / 32 : (a.out_c + 15) / 16));
+    if (two && aligned)
+        hipLaunchKernelGGL((conv2d_s16_narrow_kernel<2, true, X8>), grid, dim3(kThreads), 0, stream, a);
+    else if (two)
+        hipLaunchKernelGGL((conv2d_s16_narrow_kernel<2, false, X8>), grid, dim3(kThreads), 0, stream, a);
+    else if (aligned)
+        hipLaunchKernelGGL((conv2d_s16_narrow_kernel<1, true, X8>), grid, dim3(kThreads), 0, stream, a);
+    else
+        hipLaunchKernelGGL((conv2d_s16_narrow_kernel<1, false, X8>), grid, dim3(kThreads), 0, stream, a);
+}
+
 template <int FT, bool X8>
 void launch_gemm(const S16Args &a, bool aligned, int cus, hipStream_t stream)
 {
@@ -642,6 +681,60 @@ int steps_of(const ConvGeom &g)
     return (g.k_h * g.k_w * ((g.in_c + 15) / 16) + 3) / 4;
 }
 
+// Expected times of the two kernels, straight lines in their work fitted to 97 layers of 56 to 720 K output pixels
+// (within 10 to 17 %): launch, the steps of one wavefront or workgroup, all of them over the device.
+struct S16Choice {
+    float gemm_us, narrow_us;
+    int ft;   // filter tiles of a workgroup of the GEMM form
+    bool two; // the narrow form's wavefronts take two
+    bool narrow() const { return narrow_us < gemm_us; }
+    // In a group of layers the narrow form saves the launch and the time between two.
+    bool groups() const { return narrow_us < gemm_us + 1.2f; }
+};
+S16Choice choose(const ConvGeom &g, bool aligned, int cus)
+{
+    S16Choice c;
+    const long long n_pix = (long long)g.batch * g.out_h * g.out_w;
+    c.ft = g.out_c <= 16 ? 1 : (g.out_c <= 32 ? 2 : 4);
+    const int ksteps = steps_of(g);
+    const float steps = (float)ksteps;
+    const float tiles = 1e-3f * (float)((n_pix + 63) / 64 * ((g.out_c + 16 * c.ft - 1) / (16 * c.ft)));
+    c.gemm_us = aligned ? 3.0f + 0.385f * steps + tiles * (0.227f * steps * (float)(1 + c.ft) + 0.644f * (float)(2 + c.ft))
+                        : 3.26f + 0.68f * steps + tiles * (0.158f * steps * (float)(1 + c.ft) + 1.05f * (float)(2 + c.ft));
+    const unsigned tiles16 = (unsigned)((n_pix + 15) / 16);
+    c.two = g.out_c > 16 && (long long)tiles16 * ((g.out_c + 31) / 32) >= 2ll * cus;
+    const unsigned ny = (unsigned)(c.two ? (g.out_c + 31) / 32 : (g.out_c + 15) / 16);
+    const float waves = 4e-3f * (float)tiles16 * (float)ny, own = (float)((ksteps + 3) / 4), nt = c.two ? 2.f : 1.f;
+    c.narrow_us = aligned ? 3.15f + 0.09f * own + waves * (0.157f + 0.336f * own * nt)
+                          : 3.44f + 0.21f * own + waves * (0.51f + 0.277f * own * nt);
+    return c;
+}
+
+// A layer's launch: the one that is expected to be faster.
+template <bool X8>
+void launch_one(const S16Args &a, const S16Choice &c, bool aligned, int cus, hipStream_t stream)
+{
+    if (c.narrow())
+        launch_narrow16<X8>(a, c.two, aligned, stream);
+    else if (c.ft == 1)
+        launch_gemm<1, X8>(a, aligned, cus, stream);
+    else if (c.ft == 2)
+        launch_gemm<2, X8>(a, aligned, cus, stream);
+    else
+        launch_gemm<4, X8>(a, aligned, cus, stream);
+}
+
+// A launch held back in this thread's open group.
+struct Held {
+    S16Args args;
+    S16Choice choice;
+    bool x8;
+    int cus;
+    hipStream_t stream;
+};
+thread_local Held held[kMostGrouped];
+thread_local int n_held = 0;
+
 // The kernel for a layer and its launch; a.win holds the input and the filter.
 template <bool X8>
 hipError_t launch_units(const ConvGeom &g, S16Args &a, const int64_t *bias, const int32_t *shift, int16_t *out, int cu_count,
@@ -664,42 +757,17 @@ hipError_t launch_units(const ConvGeom &g, S16Args &a, const int64_t *bias, cons
     const bool aligned = (g.in_c & 15) == 0 &&
         ((reinterpret_cast<uintptr_t>(a.win.in) | reinterpret_cast<uintptr_t>(a.win.w)) & 15) == 0;
     const int cus = cu_count > 0 ? cu_count : 256;
-    // Expected times of the two kernels, straight lines in their work fitted to 97 layers of 56 to 720 K output pixels
-    // (within 10 to 17 %): launch, the steps of one wavefront or workgroup, all of them over the device.
-    const int ft = g.out_c <= 16 ? 1 : (g.out_c <= 32 ? 2 : 4);
-    const float steps = (float)a.ksteps;
-    const float tiles = 1e-3f * (float)(((long long)a.n_pix + 63) / 64 * ((g.out_c + 16 * ft - 1) / (16 * ft)));
-    const float gemm_us = aligned ? 3.0f + 0.385f * steps + tiles * (0.227f * steps * (float)(1 + ft) + 0.644f * (float)(2 + ft))
-                                  : 3.26f + 0.68f * steps + tiles * (0.158f * steps * (float)(1 + ft) + 1.05f * (float)(2 + ft));
-    const unsigned tiles16 = (unsigned)((a.n_pix + 15) / 16);
-    const bool two = g.out_c > 16 && (long long)tiles16 * ((g.out_c + 31) / 32) >= 2ll * cus;
-    const unsigned ny = (unsigned)(two ? (g.out_c + 31) / 32 : (g.out_c + 15) / 16);
-    const float waves = 4e-3f * (float)tiles16 * (float)ny, own = (float)((a.ksteps + 3) / 4), nt = two ? 2.f : 1.f;
-    const float narrow_us = aligned ? 3.15f + 0.09f * own + waves * (0.157f + 0.336f * own * nt)
-                                    : 3.44f + 0.21f * own + waves * (0.51f + 0.277f * own * nt);
+    const S16Choice c = choose(g, aligned, cus);
     if constexpr (X8) { // 3 x 3 layers of whole units as a walk down the image, once their rows fill the device
         const int8_t *in = static_cast<const int8_t *>(a.win.in);
-        if (1.1f * conv2d_s16_x8_walk_us(g, in, out, a.table_size, cus) < std::min(narrow_us, gemm_us)) // (56 x 56 x 16, batch 64: 11.9 against 10.6 us)
+        if (1.1f * conv2d_s16_x8_walk_us(g, in, out, a.table_size, cus) < std::min(c.narrow_us, c.gemm_us)) // (56 x 56 x 16, batch 64: 11.9 against 10.6 us)
             return launch_conv2d_s16_x8_walk(g, in, reinterpret_cast<const int16_t *>(a.win.w), bias, shift, a.table, a.table_size, a.table_shift,
                                              out, cus, stream);
     }
-    if (narrow_us < gemm_us) {
-        const dim3 grid(tiles16, ny);
-        if (two && aligned)
-            hipLaunchKernelGGL((conv2d_s16_narrow_kernel<2, true, X8>), grid, dim3(kThreads), 0, stream, a);
-        else if (two)
-            hipLaunchKernelGGL((conv2d_s16_narrow_kernel<2, false, X8>), grid, dim3(kThreads), 0, stream, a);
-        else if (aligned)
-            hipLaunchKernelGGL((conv2d_s16_narrow_kernel<1, true, X8>), grid, dim3(kThreads), 0, stream, a);
-        else
-            hipLaunchKernelGGL((conv2d_s16_narrow_kernel<1, false, X8>), grid, dim3(kThreads), 0, stream, a);
-    } else if (ft == 1) {
-        launch_gemm<1, X8>(a, aligned, cus, stream);
-    } else if (ft == 2) {
-        launch_gemm<2, X8>(a, aligned, cus, stream);
-    } else {
-        launch_gemm<4, X8>(a, aligned, cus, stream);
-    }
+    if (group_open && aligned && c.groups() && n_held < kMostGrouped)
+        held[n_held++] = Held{a, c, X8, cus, stream};
+    else
+        launch_one<X8>(a, c, aligned, cus, stream);
     return hipGetLastError();
 }
 
@@ -736,6 +804,63 @@ hipError_t launch_conv2d_s16_x8(const ConvGeom &g, const int8_t *in, const int16
     for (a.table_shift = 0; table != nullptr && ((table_size - 1) << a.table_shift) < 65536;)
         a.table_shift++;
     return launch_units<true>(g, a, bias, shift, out, cu_count, stream);
+}
+
+// Which of a group's launches a layer takes (0: none), for tensors at aligned addresses.
+int conv2d_s16_group_kind(const ConvGeom &g, bool x8, int table_size, int cu_count)
+{
+    const S16Choice c = choose(g, true, cu_count > 0 ? cu_count : 256);
+    const void *aligned = reinterpret_cast<const void *>(uintptr_t(256));
+    if ((g.in_c & 15) != 0 || !c.groups() ||
+        (x8 && 1.1f * conv2d_s16_x8_walk_us(g, aligned, aligned, table_size, cu_count > 0 ? cu_count : 256) < std::min(c.narrow_us, c.gemm_us)))
+        return 0;
+    return x8 ? 6 : 5;
+}
+
+// The launches held back since the group was opened: those of one build together.
+hipError_t flush_conv2d_s16_units()
+{
+    const int n = n_held;
+    n_held = 0;
+    bool done[kMostGrouped] = {};
+    for (int i = 0; i < n; i++) {
+        if (done[i])
+            continue;
+        const Held &h = held[i];
+        S16Group group;
+        long long blocks = 0;
+        int members = 0;
+        for (int j = i; j < n; j++) {
+            const Held &o = held[j];
+            if (o.x8 != h.x8 || o.stream != h.stream)
+                continue;
+            const unsigned columns = (unsigned)((o.args.n_pix + 15) / 16);
+            done[j] = true;
+            group.layer[members] = o.args;
+            group.first[members] = (int)blocks;
+            group.columns[members] = make_fastdiv(columns);
+            blocks += (long long)columns * ((o.args.out_c + 15) / 16);
+            members++;
+        }
+        if (members == 1 || blocks > 1 << 20) { // (a group's layers are small)
+            for (int j = i; j < n; j++)
+                if (held[j].x8 == h.x8 && held[j].stream == h.stream) {
+                    if (h.x8)
+                        launch_one<true>(held[j].args, held[j].choice, true, held[j].cus, h.stream);
+                    else
+                        launch_one<false>(held[j].args, held[j].choice, true, held[j].cus, h.stream);
+                }
+        } else {
+            for (int k = members; k < kMostGrouped; k++) {
+                group.layer[k] = group.layer[0];
+                group.first[k] = (int)blocks;
+                group.columns[k] = group.columns[0];
+            }
+            const auto kernel = h.x8 ? conv2d_s16_narrow_group_kernel<true> : conv2d_s16_narrow_group_kernel<false>;
+            hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kThreads), 0, h.stream, group);
+        }
+    }
+    return n > 0 ? hipGetLastError() : hipSuccess;
 }
 
 } // namespace espdl

@@ -378,6 +378,45 @@ int espdl_hip_conv2d_add(const espdl_hip_conv_desc *desc, const void *in, const 
     return device_status(espdl::launch_conv2d_s16(g, i16, f16, b64, shift, o16, s), "conv2d_s16");
 }
 
+static bool x8_layer(const espdl::ConvGeom &g);
+
+int espdl_hip_conv2d_group_kind(const espdl_hip_conv_desc *desc, int has_lut, int has_residual, int x8, int32_t table_size)
+{
+    espdl::ConvGeom g;
+    if (derive_geometry(desc, &g) != ESPDL_HIP_OK || desc->group != 1 || g.batch == 0)
+        return 0;
+    const int cus = cu_count_cached();
+    static int8_t *const aligned = reinterpret_cast<int8_t *>(uintptr_t(256));
+    if (desc->dtype == ESPDL_HIP_S8) {
+        if (x8 || dense_s8_kernel(g, aligned, aligned, has_lut ? aligned : nullptr, has_residual ? aligned : nullptr, aligned, cus) != DENSE_NARROW)
+            return 0;
+        return images_per_launch(g, espdl::conv2d_s8_units_support) >= g.batch ? espdl::conv2d_s8_narrow_group_kind(g, cus) : 0;
+    }
+    if (has_lut || has_residual || !espdl::conv_is_dense(g))
+        return 0;
+    if (x8 ? !espdl_hip_conv2d_s16_x8_supported(desc, table_size) || images_per_launch(g, x8_layer) < g.batch
+           : images_per_launch(g, espdl::conv2d_s16_units_supports) < g.batch)
+        return 0;
+    return espdl::conv2d_s16_group_kind(g, x8 != 0, table_size, cus);
+}
+
+int espdl_hip_conv2d_group_begin(void)
+{
+    if (espdl::group_open)
+        return fail(ESPDL_HIP_EINVAL, "a group of convolutions is open on this thread");
+    espdl::group_open = true;
+    return ESPDL_HIP_OK;
+}
+
+int espdl_hip_conv2d_group_end(void)
+{
+    if (!espdl::group_open)
+        return fail(ESPDL_HIP_EINVAL, "no group of convolutions is open on this thread");
+    espdl::group_open = false;
+    const hipError_t s8 = espdl::flush_conv2d_s8_narrow(), s16 = espdl::flush_conv2d_s16_units();
+    return device_status(s8 != hipSuccess ? s8 : s16, "grouped convolutions");
+}
+
 const char *espdl_hip_conv2d_s8_kernel(const espdl_hip_conv_desc *desc, const void *in, const void *filter, const int8_t *lut,
                                        const int8_t *residual, const void *out)
 {

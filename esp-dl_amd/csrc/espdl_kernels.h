@@ -48,6 +48,14 @@ inline bool conv_is_dense(const ConvGeom &g)
     return g.in_pitch == g.in_c && g.out_pitch == g.out_c && g.res_pitch == g.out_c;
 }
 
+// Between espdl_hip_conv2d_group_begin and _end a thread's launches that can share one are held back; _end sends them out.
+constexpr int kMostGrouped = 4;
+inline thread_local bool group_open = false;
+int conv2d_s8_narrow_group_kind(const ConvGeom &g, int cu_count);
+int conv2d_s16_group_kind(const ConvGeom &g, bool x8, int table_size, int cu_count);
+hipError_t flush_conv2d_s8_narrow();
+hipError_t flush_conv2d_s16_units();
+
 // Dense int8 convolution / Gemm as an implicit GEMM on v_mfma_i32_16x16x64_i8.
 hipError_t launch_conv2d_s8_mfma(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,
                                  const int32_t *shift, const int8_t *lut, const int8_t *residual, int8_t *out,

@@ -115,10 +115,14 @@ private:
     void fuse_s16_input();
     void merge_requantize();
     size_t plan_bytes();
+    void enqueue(runtime_mode_t mode);
     char *staging(size_t bytes);
 
     fbs::FbsModel *m_fbs_model = nullptr;
     std::vector<dl::module::Module *> m_execution_plan;
+    // What a pass enqueues, as positions in m_execution_plan: the plan in its order, except that convolutions too small for
+    // the device which do not depend on one another share the launch of the first of them.
+    std::vector<std::vector<int>> m_schedule;
     ModelContext *m_model_context = nullptr;
     std::map<std::string, TensorBase *> m_inputs, m_outputs;
     std::string m_name, m_doc_string;

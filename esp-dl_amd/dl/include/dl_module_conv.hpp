@@ -295,6 +295,66 @@ public:
         return pixels * out.back() * taps * in_c;
     }
 
+    /// The layer's geometry for tensors of these shapes; false: not a shape that a convolution takes.
+    bool describe(const std::vector<int> &in, const std::vector<int> &filter, const std::vector<int> &out,
+                  espdl_hip_conv_desc *d) const
+    {
+        *d = {};
+        d->dtype = quant_type == QUANT_TYPE_SYMM_16BIT ? ESPDL_HIP_S16 : ESPDL_HIP_S8;
+        d->batch = in[0];
+        if (in.size() == 3) {
+            d->in_h = 1;
+            d->in_w = in[1];
+            d->in_c = in[2];
+            d->out_c = out[2];
+            d->k_h = 1;
+            d->k_w = filter[0];
+            d->stride_h = 1;
+            d->stride_w = m_strides[0];
+            d->dil_h = 1;
+            d->dil_w = m_dilations[0];
+            d->pad_left = m_pads[0];
+            d->pad_right = m_pads[1];
+        } else if (in.size() == 4) {
+            d->in_h = in[1];
+            d->in_w = in[2];
+            d->in_c = in[3];
+            d->out_c = out[3];
+            d->k_h = filter[0];
+            d->k_w = filter[1];
+            d->stride_h = m_strides[0];
+            d->stride_w = m_strides[1];
+            d->dil_h = m_dilations[0];
+            d->dil_w = m_dilations[1];
+            d->pad_top = m_pads[0];
+            d->pad_bottom = m_pads[1];
+            d->pad_left = m_pads[2];
+            d->pad_right = m_pads[3];
+        } else {
+            return false;
+        }
+        d->group = m_group == 1 ? 1 : d->in_c;
+        return true;
+    }
+    /// Which other convolutions this one may share a launch with (espdl_hip_conv2d_group_kind), 0 for none.  Pitches in
+    /// channels, 0 for dense tensors.
+    int group_kind(const std::vector<int> &in, const std::vector<int> &filter, const std::vector<int> &out, int in_pitch,
+                   int out_pitch, int res_pitch, bool half_even) const
+    {
+        espdl_hip_conv_desc d;
+        if (m_group != 1 || m_has_project || m_has_gap || !describe(in, filter, out, &d))
+            return 0;
+        d.in_pitch = in_pitch;
+        d.out_pitch = out_pitch;
+        d.res_pitch = res_pitch;
+        d.activation = activation == ReLU ? ESPDL_HIP_RELU : ESPDL_HIP_LINEAR;
+        d.round_mode = half_even ? ESPDL_HIP_ROUND_HALF_EVEN : ESPDL_HIP_ROUND_HALF_UP;
+        d.n_shift = 1;
+        return espdl_hip_conv2d_group_kind(&d, m_fused_lut != nullptr && !m_x8, m_residual_pos >= 0, m_x8,
+                                           m_x8 && m_fused_lut ? m_fused_lut->get_size() : 0);
+    }
+    int residual_pos() const { return m_residual_pos; }
+
     void forward(ModelContext *context, runtime_mode_t mode = RUNTIME_MODE_AUTO)
     {
         (void)mode;
@@ -312,42 +372,11 @@ public:
             return;
         }
 
-        espdl_hip_conv_desc d = {};
-        d.dtype = quant_type == QUANT_TYPE_SYMM_16BIT ? ESPDL_HIP_S16 : ESPDL_HIP_S8;
-        d.batch = input->shape[0];
-        if (input->shape.size() == 3) {
-            d.in_h = 1;
-            d.in_w = input->shape[1];
-            d.in_c = input->shape[2];
-            d.out_c = output->shape[2];
-            d.k_h = 1;
-            d.k_w = filter->shape[0];
-            d.stride_h = 1;
-            d.stride_w = m_strides[0];
-            d.dil_h = 1;
-            d.dil_w = m_dilations[0];
-            d.pad_left = m_pads[0];
-            d.pad_right = m_pads[1];
-        } else if (input->shape.size() == 4) {
-            d.in_h = input->shape[1];
-            d.in_w = input->shape[2];
-            d.in_c = input->shape[3];
-            d.out_c = output->shape[3];
-            d.k_h = filter->shape[0];
-            d.k_w = filter->shape[1];
-            d.stride_h = m_strides[0];
-            d.stride_w = m_strides[1];
-            d.dil_h = m_dilations[0];
-            d.dil_w = m_dilations[1];
-            d.pad_top = m_pads[0];
-            d.pad_bottom = m_pads[1];
-            d.pad_left = m_pads[2];
-            d.pad_right = m_pads[3];
-        } else {
+        espdl_hip_conv_desc d;
+        if (!describe(input->shape, filter->shape, output->shape, &d)) {
             DL_LOGE("Conv", "Do not support input shape.");
             return;
         }
-        d.group = m_group == 1 ? 1 : d.in_c;
         d.in_pitch = input->is_dense() ? 0 : input->channel_pitch;
         d.out_pitch = output->is_dense() ? 0 : output->channel_pitch;
         d.activation = activation == ReLU ? ESPDL_HIP_RELU : ESPDL_HIP_LINEAR;

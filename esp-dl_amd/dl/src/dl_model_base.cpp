@@ -1275,6 +1275,56 @@ esp_err_t Model::build(int batch)
     for (int i = n_var - 1; i >= 1; i--)
         if (vars[i].alias_of >= 0)
             vars[vars[i].alias_of].last = std::max(vars[vars[i].alias_of].last, vars[i].last);
+    // 1c. convolutions that share a launch.  A small one takes along later ones of its kind whose inputs are there by then: the
+    // heads of a detector, level by level, where one launch after the other costs 1.2 us between them and a wavefront's latency each
+    // (416 x 416, one frame: 56 launches and 193 us, 46 and 167; 640 x 640, two frames 272 and 256; 512 x 512, twelve, whose layers
+    // mostly fill the device and have kind 0: 379 both ways).  Results, the plan and its order stay as they are: a module that
+    // runs early has its output placed then and its inputs kept until its own place, so that a pass module by module (test,
+    // get_module_info, a stage) finds the same tensors.
+    std::vector<std::vector<int>> with(plan_size); // the later modules that run with this one
+    {
+        auto pitch = [&](int v) { return vars[v].slice_of >= 0 ? vars[vars[v].slice_of].shape.back() : 0; };
+        auto kind_of = [&](int i) {
+            auto *conv = dynamic_cast<dl::module::Conv *>(m_execution_plan[i]);
+            if (!conv || conv->inplace != MODULE_NON_INPLACE || conv->m_outputs_index.size() != 1)
+                return 0;
+            const int in = conv->m_inputs_index[0], out = conv->m_outputs_index[0];
+            const int res = conv->residual_pos() >= 0 ? conv->m_inputs_index[conv->residual_pos()] : 0;
+            TensorBase *filter = conv->m_inputs_index[1] >= CONTEXT_PARAMETER_OFFSET ? ctx->get_tensor(conv->m_inputs_index[1]) : nullptr;
+            if (in <= 0 || in >= CONTEXT_PARAMETER_OFFSET || res < 0 || res >= CONTEXT_PARAMETER_OFFSET || !filter || vars[out].alias_of >= 0)
+                return 0;
+            return conv->group_kind(vars[in].shape, filter->shape, vars[out].shape, pitch(in), pitch(out), res > 0 ? pitch(res) : 0,
+                                    ctx->round_mode == ROUND_MODE_HALF_EVEN);
+        };
+        std::vector<int> kind(plan_size);
+        for (int i = 0; i < plan_size; i++)
+            kind[i] = kind_of(i);
+        std::vector<bool> there(n_var, false), scheduled(plan_size, false);
+        for (const std::string &name : m_fbs_model->get_graph_inputs())
+            there[ctx->get_variable_index(name)] = true;
+        m_schedule.clear();
+        for (int i = 0; i < plan_size; i++) {
+            if (scheduled[i])
+                continue;
+            std::vector<int> part = {i};
+            for (int j = i + 1; kind[i] != 0 && j < plan_size && part.size() < 4; j++) {
+                if (scheduled[j] || kind[j] != kind[i])
+                    continue;
+                bool ready = true;
+                for (int idx : m_execution_plan[j]->m_inputs_index)
+                    ready = ready && (idx <= 0 || idx >= CONTEXT_PARAMETER_OFFSET || there[idx]);
+                if (ready)
+                    part.push_back(j);
+            }
+            for (int j : part) {
+                scheduled[j] = true;
+                for (int idx : m_execution_plan[j]->m_outputs_index)
+                    there[idx] = true;
+            }
+            with[i].assign(part.begin() + 1, part.end());
+            m_schedule.push_back(part);
+        }
+    }
     // 2. placement
     auto bytes_of = [&](const VarInfo &v) {
         size_t n = dtype_sizeof(v.dtype);
@@ -1301,7 +1351,7 @@ esp_err_t Model::build(int batch)
                 vars[v].last = -2;
             }
     };
-    for (int i = 0; i < plan_size; i++) {
+    auto place_outputs = [&](int i) {
         dl::module::Module *m = m_execution_plan[i];
         for (size_t j = 0; j < m->m_outputs_index.size(); j++) {
             const int idx = m->m_outputs_index[j];
@@ -1311,7 +1361,7 @@ esp_err_t Model::build(int batch)
                 continue;
             }
             if (placed[idx])
-                continue; // the output of a Concat that an earlier producer already writes into
+                continue; // the output of a Concat that an earlier producer already writes into, or of a module that runs early
             if (v.slice_of >= 0) {
                 // lives inside the wider tensor, which is placed when its first slice is written
                 const int w = v.slice_of;
@@ -1341,6 +1391,11 @@ esp_err_t Model::build(int batch)
             offset[idx] = arena.alloc(bytes_of(v));
             placed[idx] = true;
         }
+    };
+    for (int i = 0; i < plan_size; i++) {
+        place_outputs(i);
+        for (int j : with[i])
+            place_outputs(j);
         release_dead(i);
     }
 
@@ -1396,8 +1451,18 @@ void Model::run_async(runtime_mode_t mode)
                      "hipGraphLaunch");
         return;
     }
-    for (auto *module : m_execution_plan)
-        module->forward(m_model_context, mode);
+    enqueue(mode);
+}
+
+void Model::enqueue(runtime_mode_t mode)
+{
+    for (const std::vector<int> &part : m_schedule) {
+        const bool group = part.size() > 1 && espdl_hip_conv2d_group_begin() == ESPDL_HIP_OK; // (else one by one)
+        for (int i : part)
+            m_execution_plan[i]->forward(m_model_context, mode);
+        if (group && espdl_hip_conv2d_group_end() != ESPDL_HIP_OK)
+            DL_LOGE(TAG, "%s", espdl_hip_last_error());
+    }
 }
 
 void Model::synchronize()
@@ -1539,16 +1604,14 @@ bool Model::enable_graph()
     // carry data between passes (StreamingCache) get it back afterwards, the pass counts for nothing
     for (auto *module : m_execution_plan)
         module->hold_state(m_stream);
-    for (auto *module : m_execution_plan)
-        module->forward(m_model_context, RUNTIME_MODE_AUTO);
+    enqueue(RUNTIME_MODE_AUTO);
     for (auto *module : m_execution_plan)
         module->restore_state(m_stream);
     if (!hip_ok(hipStreamSynchronize(s), "hipStreamSynchronize") || last_run_failed())
         return false; // a plan with a rejected module must not be captured: the graph would miss its kernels
     if (!hip_ok(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture"))
         return false;
-    for (auto *module : m_execution_plan)
-        module->forward(m_model_context, RUNTIME_MODE_AUTO);
+    enqueue(RUNTIME_MODE_AUTO);
     hipGraph_t graph = nullptr;
     if (!hip_ok(hipStreamEndCapture(s, &graph), "hipStreamEndCapture") || !graph)
         return false;

@@ -108,6 +108,17 @@ int espdl_hip_conv2d_add(const espdl_hip_conv_desc *desc, const void *in, const 
 const char *espdl_hip_conv2d_s8_kernel(const espdl_hip_conv_desc *desc, const void *in, const void *filter, const int8_t *lut,
                                        const int8_t *residual, const void *out);
 
+/*
+ * Convolutions that do not depend on one another in one launch.  Between the two calls a thread makes up to four calls of
+ * espdl_hip_conv2d, _conv2d_add or _conv2d_s16_x8 (and no others) on one stream, none of which reads or overwrites what another one
+ * writes; launches of one build are held back and leave together in _end, on that stream, the others at once.  Which layers share
+ * a launch: those of one kind, 0 for a layer that takes another kernel.  `x8`: espdl_hip_conv2d_s16_x8 with a table of that many
+ * entries (0: none).  Groups do not nest: _begin fails (ESPDL_HIP_EINVAL) where one is open, _end where none is.
+ */
+int espdl_hip_conv2d_group_kind(const espdl_hip_conv_desc *desc, int has_lut, int has_residual, int x8, int32_t table_size);
+int espdl_hip_conv2d_group_begin(void);
+int espdl_hip_conv2d_group_end(void);
+
 /* base::lut_s8 (esp-dl/dl/base/dl_base_lut.cpp:10-48): out[i] = table[(uint8)in[i] ^ 0x80]. In-place allowed. */
 int espdl_hip_lut_s8(const int8_t *in, int64_t size, const int8_t *table, int8_t *out, void *stream);
 

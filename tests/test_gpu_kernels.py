@@ -923,6 +923,78 @@ def test_conv2d_few_outputs(oracle, case, behind, half_even):
     np.testing.assert_array_equal(to_host(m.conv2d(*args, **kw)), want)
 
 
+GROUPED = {
+    # layers (input shape, filters, window, stride, padding, int16 input / int8 input of an int16 layer, table, residual)
+    "one level of three heads": [((1, 20, 20, 64), 64, 3, 1, 1, "s8", True, False), ((1, 10, 10, 128), 64, 3, 1, 1, "s8", True, False),
+                                 ((1, 5, 5, 256), 64, 3, 1, 1, "s8", False, False)],
+    "every build": [((1, 13, 7, 64), 33, 3, 1, 1, "s8", False, False), ((1, 5, 3, 512), 20, 1, 1, 0, "s8", True, False),
+                    ((1, 9, 9, 16), 80, 1, 2, 0, "s8", False, False), ((1, 6, 11, 16), 17, 2, 1, 1, "s8", False, True)],
+    "edges of tiles": [((1, 1, 1, 64), 4, 1, 1, 0, "s8", False, False), ((1, 1, 65, 64), 80, 1, 1, 0, "s8", False, True),
+                       ((1, 8, 8, 64), 5, 1, 1, 0, "s8", True, False), ((3, 1, 17, 32), 16, 1, 1, 0, "s8", False, False)],
+    "with layers that leave at once": [((1, 7, 7, 20), 9, 3, 1, 1, "s8", False, False), ((1, 9, 9, 48), 48, 3, 1, 1, "s8", False, False),
+                                       ((8, 28, 28, 64), 64, 3, 1, 1, "s8", False, False), ((1, 5, 9, 48), 30, 3, 1, 1, "s8", False, False)],
+    "int16 layers": [((1, 20, 20, 64), 64, 1, 1, 0, "s16", False, False), ((1, 10, 10, 64), 64, 1, 1, 0, "s16", False, False),
+                     ((1, 5, 5, 64), 33, 1, 1, 0, "s16", False, False), ((1, 5, 4, 128), 17, 3, 1, 1, "s16", False, False)],
+    "int16 layers on int8 inputs": [((1, 20, 20, 64), 64, 3, 1, 1, "x8", False, False), ((1, 10, 9, 64), 64, 3, 1, 1, "x8", True, False),
+                                    ((1, 5, 5, 64), 20, 3, 1, 1, "x8", True, False), ((1, 9, 9, 64), 64, 3, 1, 1, "s8", False, False)],
+    "one alone": [((1, 10, 10, 64), 64, 1, 1, 0, "s16", False, False)],
+}
+
+
+@pytest.mark.parametrize("half_even", [False, True], ids=["half_up", "half_even"])
+@pytest.mark.parametrize("group", list(GROUPED))
+def test_grouped_convolutions(oracle, group, half_even):
+    """Independent convolutions in one launch give what each gives by itself."""
+    announce(f"grouped convolutions: {group} {half_even}")
+    m, L = espdl(), espdl().lib()
+    rm_o = oracle.ROUND_HALF_EVEN if half_even else oracle.ROUND_HALF_UP
+    rm = m.capi.ROUND_HALF_EVEN if half_even else m.capi.ROUND_HALF_UP
+    rng = np.random.default_rng(0x6B0)
+    calls, want = [], []
+    for shape, oc, k, stride, pad, kind, has_table, has_res in GROUPED[group]:
+        geometry = ((k, k), (stride, stride), (1, 1), (pad,) * 4)
+        relu, act = m.capi.RELU, oracle.RELU
+        if kind == "s8":
+            x = rng_int8(rng, shape)
+            f = rng_int8(rng, (oc, k, k, shape[3]))
+            bias = rng.integers(-2**14, 2**14, size=oc).astype(np.int32)
+            shift = rng.integers(7, 13, size=oc).astype(np.int32)
+            w = oracle.conv2d_s8(x, f, bias, shift, *geometry, act, rm_o)
+            kw = {}
+            if has_table:
+                table = rng_int8(rng, (256,))
+                w = table[w.astype(np.int32) + 128]
+                kw["lut"] = to_dev(table)
+            if has_res:
+                res = rng_int8(rng, w.shape)
+                w = oracle.add_s8(w, res)
+                kw["residual"] = to_dev(res)
+            args = (to_dev(x), to_dev(f), to_dev(bias), to_dev(shift), *geometry)
+            calls.append(lambda a=args, kw=kw: m.conv2d(*a, activation=relu, round_mode=rm, **kw))
+        else:
+            f = rng.integers(-32768, 32768, size=(oc, k, k, shape[3])).astype(np.int16)
+            bias = rng.integers(-2**30, 2**30, size=oc).astype(np.int64)
+            shift = rng.integers(20, 26, size=oc).astype(np.int32)
+            table = rng.integers(-32768, 32768, size=257).astype(np.int16) if has_table else None
+            x = rng_int8(rng, shape) if kind == "x8" else rng.integers(-32768, 32768, size=shape).astype(np.int16)
+            args = (to_dev(x), to_dev(f), to_dev(bias), to_dev(shift), *geometry)
+            if kind == "x8":
+                tab = None if table is None else to_dev(table)
+                calls.append(lambda a=args, tab=tab: m.capi.conv2d_s16_x8(*a, activation=relu, round_mode=rm, table=tab))
+                w = to_host(calls[-1]()) if has_table else oracle.conv2d_s16((x.astype(np.int16) * 256), f, bias, shift, *geometry, act, rm_o)
+            else:
+                calls.append(lambda a=args: m.conv2d(*a, activation=relu, round_mode=rm))
+                w = oracle.conv2d_s16(x, f, bias, shift, *geometry, act, rm_o)
+        want.append(w)
+    assert L.espdl_hip_conv2d_group_begin() == 0
+    got = [call() for call in calls]
+    assert L.espdl_hip_conv2d_group_begin() != 0  # groups do not nest
+    assert L.espdl_hip_conv2d_group_end() == 0
+    assert L.espdl_hip_conv2d_group_end() != 0
+    for i, (g, w) in enumerate(zip(got, want)):
+        np.testing.assert_array_equal(to_host(g), w, err_msg=f"layer {i}")
+
+
 S16_UNIT_CASES = [
     # (name, (n, h, w, c), out_c, k, stride, dil, pads, relu, half_even, lowest and highest shift, values): channel counts
     # around the 16-channel units, one to four filter tiles and tails of each, few pixels (narrow kernel) and many

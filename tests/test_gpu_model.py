@@ -203,6 +203,35 @@ def test_config4_yolo_style(oracle, fuse):
     mdl.close()
 
 
+@pytest.mark.parametrize("resolution,batch", [(96, 1), (160, 3)])
+def test_convolutions_that_share_a_launch(oracle, resolution, batch):
+    """The heads of a small detector run level by level: the outputs are those of the oracle, of a pass module by module and of
+    every replay, with passes of another input in between."""
+    announce(f"model config4 {resolution}px batch {batch}: shared launches")
+    _, zoo, _, _ = _mods()
+    spec = zoo.config4_yolo_style(resolution=resolution)
+    mdl, want, x = _run_config(spec, batch, 9)
+    name = spec.inputs[0]
+
+    def check():
+        for out in spec.outputs:
+            np.testing.assert_array_equal(mdl.get_tensor(out, _np_dtype(spec, out)), want[out], err_msg=out)
+
+    check()
+    for replay in (False, True, True):
+        if replay:
+            assert mdl.enable_graph()
+        mdl.set_input(name, np.flip(x, axis=1).copy())
+        mdl.run()
+        mdl.set_input(name, x)
+        mdl.run()
+        check()
+        mdl.set_input(name, x)
+        mdl.profile(1)  # module by module, in the plan's order
+        check()
+    mdl.close()
+
+
 @pytest.mark.parametrize("round_mode", [0, 1], ids=["half_up", "half_even"])
 @pytest.mark.parametrize("rows,k,n,m", [(40, 120, 480, 120), (9, 33, 17, 5), (1, 16, 2100, 64)])
 def test_lut_behind_gemm_and_matmul(oracle, rows, k, n, m, round_mode):
