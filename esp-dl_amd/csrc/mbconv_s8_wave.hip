@@ -819,7 +819,9 @@ WavePlan wave_plan(const MbconvParams &p)
     // dropped) and still takes a third of the time of a guarded build.
     // rows: cheapest total of expand tiles (x 1.5: MFMA + the longer epilogue) and depthwise MFMAs.  A launch
     // that does not fill the device once (two resident workgroups per compute unit) takes one tile's time
-    // whatever its tile count, so there a lower tile that brings more workgroups wins.  Heights whose plan has a
+    // whatever its tile count, so there a lower tile that brings more workgroups wins (the stem and first block of
+    // MobileNetV2 on one image of 224 x 224, eight rows and 28 workgroups against two and 112: 12.1 -> 9.0 us; its second
+    // block on 18 images 14.6 -> 11.2, on 37 of 160 x 160, half even, 19.1 -> 15.9).  Heights whose plan has a
     // guard-free build come first: the guarded builds take about three times as long per tile, and a caller
     // that fuses by espdl_hip_mbconv_s8_preferred gets the same answer at every batch size.
     const int nxpt_limit = 17;
@@ -848,7 +850,9 @@ WavePlan wave_plan(const MbconvParams &p)
             size_t lds_unused;
             wave_layout(a, &lds_unused); // (the guard-free build of a windowed expand stage asks for its row copy)
             const bool exact = wave_plan_has_exact_build(a);
-            const double tile_cost = 1.5 * a.n_xpt + 3.0 * th + 2.0;
+            // (a guard-free tile of two rows costs a wavefront's start beside it: 30 images of 56 x 56, 16 -> 96 -> 24 at stride 2,
+            // 1.6 rounds of them, 17.7 us, 16.5 as tiles of four)
+            const double tile_cost = 1.5 * a.n_xpt + 3.0 * th + (exact && th <= 2 ? 6.0 : 2.0);
             const double groups = std::ceil((double)std::max(1, p.batch) * a.tiles_y * a.tiles_x / kWavesPerGroup);
             const double rounds = groups / slots;
             const double cost = tile_cost * std::max(1.0, rounds);
@@ -959,6 +963,8 @@ bool launch_exact(const WavePlan &plan, hipStream_t stream, bool dry, hipError_t
         // expand stage with a window: the stem + first block of MobileNetV2 at 224 x 224
         if (a.n_xpt == 10 && a.pw == 16 && a.rt == 1 && a.th == 8 && s == 1 && a.rows_n > 0)
             ESPDL_WAVE_EXACT(10, 1, 8, 1, false, true);
+        if (a.n_xpt == 4 && a.pw == 16 && a.rt == 1 && a.th == 2 && s == 1 && a.rows_n > 0)
+            ESPDL_WAVE_EXACT(4, 1, 2, 1, false, true);
         return false;
     }
     const auto is = [&](int nxpt, int rt, int th, int stride, bool v) {
@@ -981,6 +987,8 @@ bool launch_exact(const WavePlan &plan, hipStream_t stream, bool dry, hipError_t
     const int c0 = a.p.in_c;
     if (is(17, 2, 4, 2, true) && c0 == 16)
         ESPDL_WAVE_PACKED(17, 2, 4, 2, true, 4);
+    if (is(10, 2, 2, 2, true) && c0 == 16)
+        ESPDL_WAVE_PACKED(10, 2, 2, 2, true, 4);
     if (is(17, 2, 4, 2, false) && c0 <= 32)
         ESPDL_WAVE_PACKED(17, 2, 4, 2, false, 2);
     if (is(10, 2, 8, 1, false) && c0 <= 32)
@@ -1060,6 +1068,11 @@ float mbconv_s8_wave_us(const MbconvParams &p)
     const float n_sub = (float)(p.exp_c / 16);
     const float chain = (p.stride_h == 1 ? 7.f + 1.1f * n_sub : 5.5f + 0.9f * n_sub) * (p.half_even ? 1.2f : 1.f);
     const float fill = mbconv_s8_wave_rounds(p);
+    if (p.stride_h == 2 && p.in_c == 16) { // the low tiles of few images (9 to 37 of 56 x 56 and 40 x 40, within 10 %)
+        const WavePlan plan = wave_plan(p);
+        if (plan.a.th <= 2 && wave_plan_has_exact_build(plan.a))
+            return 0.77f * chain * (fill <= 1.f ? 1.f + 0.35f * fill : 1.35f * fill);
+    }
     return chain * (fill <= 1.f ? 1.f + 0.45f * fill : 1.45f * fill);
 }
 

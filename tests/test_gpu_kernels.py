@@ -1826,6 +1826,58 @@ def test_mbconv_s8_walk_stem(oracle, case, flavour):
     np.testing.assert_array_equal(to_host(got), cur)
 
 
+# Few images, where the tile kernel takes tiles of two rows: a windowed expand stage and blocks of 16 input channels at stride 2, odd
+# heights and widths, the last tile of a row and a column in part outside.
+# (name, (N, H, W, Cin), expand window (kernel, stride, pads) or None, Ce, Cout, stride, Clip)
+LOW_TILES = [
+    ("rgb_63x61_s2", (2, 63, 61, 3), ((3, 3), (2, 2), (0, 1, 0, 1)), 32, 16, 1, False),
+    ("rgb_34x58_s2_clip", (1, 34, 58, 3), ((3, 3), (2, 2), (1, 1, 1, 1)), 32, 16, 1, True),
+    ("gray_17x40_s2_16_4", (3, 17, 40, 1), ((3, 3), (2, 2), (1, 0, 1, 0)), 16, 4, 1, False),
+    ("rgb_3x40_s1_48_12", (1, 3, 40, 3), ((2, 3), (1, 1), (1, 1, 1, 1)), 48, 12, 1, False),
+    ("block_31x57_96_24", (2, 31, 57, 16), None, 96, 24, 2, False),
+    ("block_80x80_96_24_clip", (5, 80, 80, 16), None, 96, 24, 2, True),
+    ("block_5x28_112_32", (1, 5, 28, 16), None, 112, 32, 2, False),
+    ("block_2x29_16_20", (4, 2, 29, 16), None, 16, 20, 2, False),
+]
+
+
+@pytest.mark.parametrize("flavour", ["half_up", "half_even", "general"])
+@pytest.mark.parametrize("case", LOW_TILES, ids=lambda c: c[0])
+def test_mbconv_s8_low_tiles(oracle, case, flavour):
+    announce(f"mbconv_s8 low tiles {case[0]} {flavour}")
+    name, (n, h, w, cin), window, ce, cout, stride, clip = case
+    if clip and flavour == "half_even":
+        pytest.skip("a Clip between the stages: round half up")
+    m = espdl()
+    half_even = flavour == "half_even"
+    rm_o = oracle.ROUND_HALF_EVEN if half_even else oracle.ROUND_HALF_UP
+    rng = np.random.default_rng(0x10A + len(name))
+    ek, es, ep = window or ((1, 1), (1, 1), (0, 0, 0, 0))
+
+    def stage(oc, kk, fshape):
+        shift = (typical_shift(kk) + rng.integers(-2, 3, size=oc)).astype(np.int32)
+        if flavour == "general":
+            shift[::5] = 0
+        return rng_int8(rng, fshape), rng.integers(-4096, 4097, size=oc).astype(np.int32), shift
+
+    x = rng_int8(rng, (n, h, w, cin))
+    x[:, 0, :, :], x[:, -1, :, :] = 127, 126   # make the borders count
+    x[:, :, 0, :], x[:, :, -1, :] = -128, -127
+    ex, dw, pj = stage(ce, ek[0] * ek[1] * cin, (ce, ek[0], ek[1], cin)), stage(ce, 9, (3, 3, ce)), stage(cout, ce, (cout, 1, 1, ce))
+    pads = (1, 1, 1, 1)
+    cur = oracle.conv2d_s8(x, ex[0], ex[1], ex[2], ek, es, (1, 1), ep, oracle.LINEAR if clip else oracle.RELU, rm_o)
+    cur = oracle.clip_s8(cur, 5, 90, 0, 0) if clip else cur
+    cur = oracle.depthwise_s8(cur, dw[0], dw[1], dw[2], (3, 3), (stride, stride), (1, 1), pads, oracle.RELU, rm_o)
+    cur = oracle.conv2d_s8(cur, pj[0], pj[1], pj[2], (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), oracle.LINEAR, rm_o)
+    dev = lambda t: tuple(to_dev(a) for a in t)  # noqa: E731
+    args = to_dev(x), dev(ex), dev(dw), dev(pj), (3, 3), (stride, stride), (1, 1), pads, (not clip, True, False)
+    kw = dict(round_mode=m.capi.ROUND_HALF_EVEN if half_even else m.capi.ROUND_HALF_UP, clip_expand=(5, 90) if clip else None)
+    if window:
+        kw["expand_conv"] = window
+    assert m.capi.mbconv_s8_kernel(*args, **kw) == "mbconv_s8_wave"
+    np.testing.assert_array_equal(to_host(m.mbconv_s8(*args, **kw)), cur)
+
+
 # The block as two launches (expand + depthwise, then project): tiles of 7 x 14, 7 x 7 and, at stride 2, 4 x 7 outputs with
 # ragged last rows and columns, one to three reduction steps of block-input channels (also 4 and 20: units that end
 # inside a pixel), expanded channels that leave a group of 64 unfinished, Clips, a requantized residual operand, shifts
