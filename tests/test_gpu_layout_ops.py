@@ -118,6 +118,18 @@ def test_max_pool(oracle, shape, kernel, strides, pads, dtype):
     np.testing.assert_array_equal(got, oracle.max_pool(x, kernel, strides, pads))
 
 
+@pytest.mark.parametrize("k", [2, 3, 5])
+@pytest.mark.parametrize("shape", [(1, 1, 1, 16), (1, 1, 2, 9), (2, 3, 5, 61), (1, 13, 13, 128), (80, 33, 31, 144), (80, 35, 30, 146)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_max_pool_one_row_and_strips(oracle, shape, k):
+    """Few outputs, a row each (all rows of a window at once), and enough of them for strips of several rows, whole dwords or not."""
+    announce(f"max_pool rows and strips {shape} k{k}")
+    x = _rand(np.random.default_rng(k), shape)
+    for pads in ((k // 2,) * 4 if k % 2 else (0, 1, 0, 1), (0, k - 1, k - 1, 0)):
+        got = to_host(espdl().max_pool(to_dev(x), (k, k), (1, 1), pads))
+        np.testing.assert_array_equal(got, oracle.max_pool(x, (k, k), (1, 1), pads))
+
+
 @pytest.mark.parametrize("shape,kernel,strides,pads,exps", [
     ((2, 1, 24, 32), (1, 3), (1, 1), (0, 0, 2, 0), (-6, -7)), ((2, 14, 14, 64), (3, 3), (1, 1), (1, 1, 1, 1), (-5, -5)),
     ((3, 16, 16, 24), (2, 2), (2, 2), (0, 0, 0, 0), (-4, -5)), ((2, 7, 7, 1280), (7, 7), (1, 1), (0, 0, 0, 0), (-3, -4)),
