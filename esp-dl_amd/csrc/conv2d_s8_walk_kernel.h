@@ -653,7 +653,9 @@ __global__ __launch_bounds__((64 * WalkShape<KH, S, CU, NT, RES>::W), 2) void co
 }
 
 // Whether a build exists: filters and accumulators fit 256 registers with what else a wavefront holds, and its LDS leaves
-// a compute unit two wavefronts per SIMD.
+// a compute unit two wavefronts per SIMD.  With a residual operand 204 fit for four units and four filter tiles (80 x 80 x 64 -> 64,
+// 3 x 3, batch 64, input and results slices of wider tensors: 38.1 us as two chunks of 32 filters, 29.8 as one); 15 and 16 units spill
+// 49 registers at that.
 template <int KH, int S, int CU, int NT, bool RES, bool RAW>
 constexpr bool walk_fits()
 {
@@ -661,7 +663,7 @@ constexpr bool walk_fits()
     if (RAW && 4 * (KH * Shape::KS * NT + Shape::kAcc * NT * Shape::PT + S * Shape::PT * Shape::KS + Shape::kHeld * S * Shape::kRowLoads) > 204)
         return false;
     return (NT != 8 || KH == 1) && (!RES || (S == 1 && KH <= 3)) &&
-        4 * (KH * Shape::KS * NT + Shape::kAcc * NT * Shape::PT + S * Shape::PT * Shape::KS) <= (RES ? 200 : 208) &&
+        4 * (KH * Shape::KS * NT + Shape::kAcc * NT * Shape::PT + S * Shape::PT * Shape::KS) <= (RES ? (CU == 4 ? 204 : 200) : 208) &&
         (Shape::kTwo || Shape::W == 8 || (S == 2 && Shape::lds(4, 1) <= Shape::kCu));
 }
 

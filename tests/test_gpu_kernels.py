@@ -321,6 +321,24 @@ def test_conv2d_s8_walk_residual(oracle, case, flavour):
     np.testing.assert_array_equal(got, want)
 
 
+@pytest.mark.parametrize("flavour", ["residual", "lut_residual", "slices"])
+@pytest.mark.parametrize("case", [(64, ("64_64", (41, 37, 64), 64, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
+                                  (50, ("52_128_tailpad", (37, 45, 52), 128, (3, 3), (1, 1), (1, 1), (0, 1, 0, 1), True, True))],
+                         ids=lambda c: c[1][0])
+def test_conv2d_s8_walk_residual_four_units(oracle, case, flavour):
+    """Four units of input channels under four filter tiles with a residual operand: all of a wavefront's registers."""
+    announce(f"conv2d_s8 walk with a residual operand, four units {case[1][0]} {flavour}")
+    x, f, bias, shift, k, stride, dil, pads, relu = _conv_inputs(case[1], 281, case[0], True)
+    oracle.set_threads(16)
+    if flavour == "slices":
+        _run_conv_slices(oracle, x, f, bias, shift, k, stride, dil, pads, relu, "conv2d_s8_walk", 48, with_residual=True)
+        return
+    lut = TABLE if flavour == "lut_residual" else None
+    got, want = _run_conv_s8(oracle, x, f, bias, shift, k, stride, dil, pads, relu and lut is None, lut=lut, residual_seed=19,
+                             kernel="conv2d_s8_walk")
+    np.testing.assert_array_equal(got, want)
+
+
 @pytest.mark.parametrize("case", WALK_ODD_PITCH, ids=lambda c: c[1][0])
 @pytest.mark.parametrize("flavour", ["per_channel", "lut"])
 def test_conv2d_s8_walk_odd_pitch(oracle, case, flavour):
