@@ -321,24 +321,21 @@ hipError_t launch_conv2d_s8_wide(const ConvGeom &g, const int8_t *in, const int8
     a.n_shift = g.n_shift;
     if (a.M == 0)
         return hipSuccess;
-    // Steps per walk and walks of a workgroup, each over other pixels: as many workgroups as fit the device (two to a compute unit)
-    // share the walks of their filters evenly.  The start (constants of the filters) counts as four steps, a further walk's as one;
-    // kMaxSteps steps' constants at most lie in LDS.
+    // Steps per walk: rounds of workgroups (two fit a compute unit) times a walk and its start, which costs about four
+    // steps; kMaxSteps steps' constants at most lie in LDS.  More rounds than one become walks of the same workgroups.
     const int tiles = (a.M + 63) / 64, steps = (a.N + 255) / 256;
     const long long slots = 2ll * std::max(1, cu_count);
-    int per = 1, walks = 1;
+    int per = 1;
     long long best = 0;
     for (int p = 1; p <= std::min(steps, kMaxSteps); p++) {
-        const long long chunks = (steps + p - 1) / p, groups = std::max(1ll, slots / chunks);
-        const long long of_one = (tiles + groups - 1) / groups;
-        const long long rounds = (chunks + slots - 1) / slots; // of workgroups, where the chunks alone are more than fit
-        const long long cost = rounds * (of_one * (p + 1) + 3);
+        const long long cost = ((long long)tiles * ((steps + p - 1) / p) + slots - 1) / slots * (p + 4);
         if (p == 1 || cost < best) {
             best = cost;
             per = p;
-            walks = (int)of_one;
         }
     }
+    const long long groups = std::max(1ll, slots / ((steps + per - 1) / per)); // that take the same filters
+    const int walks = (int)((tiles + groups - 1) / groups);
     a.per_walk = 256 * per;
     const dim3 grid((unsigned)((tiles + walks - 1) / walks), (unsigned)((steps + per - 1) / per));
     const size_t lds = (size_t)3 * sizeof(int) * a.per_walk;
