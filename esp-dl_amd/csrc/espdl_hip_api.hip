@@ -1418,7 +1418,7 @@ static auto project_launch(const espdl::ConvGeom &g, const void *in, const void 
 
 // The single launch is a chain of 10 to 25 us through all expanded channels of a tile, whatever the batch, until the
 // device is full; the two launches start at 7 us and grow with the work (MobileNetV2 at 224 x 224: one image 282 -> 155 us,
-// 16 images 296 -> 221 us; the blocks of batch 256 stay single launches).  Where no single-launch kernel has a fast build
+// 16 images 296 -> 221 us, with the launches of then, 133 and 200 us now; the blocks of batch 256 stay single launches).  Where no single-launch kernel has a fast build
 // the alternative is three launches, of which the depthwise one alone takes 9 us.
 int64_t espdl_hip_mbconv_s8_workspace(const espdl_hip_mbconv_desc *desc)
 {

@@ -46,8 +46,8 @@ dtype_t dtype_of(quant_type_t q)
 // ahead of the stream (MobileNetV2 at batch 256, 19 launches of 33 us: 649 against 644 us; the recognizer at 512 crops, 15
 // launches: 231 against 227 us; 15 launches of 3.6 us: 62 us as a graph, 63 us launched one by one).  Longer plans stay
 // graphs for the host's sake, which a plain replay keeps busy for most of the pass: the pass itself is about as long either
-// way (MobileNetV2 at 160 x 160, 37 images: 269 us as a graph, 262 us plainly; a detector on one frame, some 60 launches:
-// 234 and 230 us; MobileNetV2 on one image between host copies: 214 us both ways).
+// way (with longer launches than now: MobileNetV2 at 160 x 160, 37 images: 269 us as a graph, 262 us plainly; a detector on one
+// frame, then some 60 launches: 234 and 230 us; MobileNetV2 on one image between host copies: 214 us both ways).
 constexpr size_t kDirectAlways = 4;
 constexpr size_t kDirectLaunches = 24;
 constexpr size_t kDirectBytes = 1 << 20;
