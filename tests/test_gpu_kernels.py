@@ -1260,6 +1260,20 @@ def test_prelu_s8(oracle, shift):
         np.testing.assert_array_equal(got, oracle.prelu_s8(x, alpha, shift))
 
 
+@pytest.mark.parametrize("shift", [1, 7, 14, 15, 16, 24])
+def test_prelu_s8_every_product(oracle, shift):
+    """Every value under every slope, in 16-byte pieces whose channels start over at every place, at right shifts up to past 15."""
+    announce(f"prelu_s8 every product shift={shift}")
+    m = espdl()
+    x = np.repeat(np.arange(-128, 128).astype(np.int8)[:, None], 256, axis=1).reshape(1, 16, 16, 256)
+    alpha = np.arange(-128, 128).astype(np.int8)
+    np.testing.assert_array_equal(to_host(m.prelu_s8(to_dev(x), to_dev(alpha), shift)), oracle.prelu_s8(x, alpha, shift))
+    rng = np.random.default_rng(shift)
+    for channels in (1, 3, 17, 40):
+        x, alpha = rng_int8(rng, (1, 5, 32, channels)), rng_int8(rng, (channels,))
+        np.testing.assert_array_equal(to_host(m.prelu_s8(to_dev(x), to_dev(alpha), shift)), oracle.prelu_s8(x, alpha, shift))
+
+
 @pytest.mark.parametrize("extra", [0, 16, 16 * 256 + 5], ids=["at the line", "one vector more", "a part of a workgroup and a tail"])
 def test_elementwise_operands_that_leave_no_copy(oracle, extra):
     """int8 operands around the size from which element-wise operators read past the last-level cache (36 MiB)."""
