@@ -192,14 +192,14 @@ __global__ __launch_bounds__(kThreads) void max_pool_s8_window_kernel(const Wind
 }
 
 // Strips of one row, which is what few outputs are cut into: all rows of the window are requested at once, where the walk waits
-// for one after the other.  One wavefront to a workgroup, for the loads of a compute unit's wavefronts take turns (30 of 16 bytes
-// each).  5 x 5, launch to launch in a graph: 13 x 13 x 128, one image, 3.2 -> 2.9 us, 30 x 30 x 198 4.8 -> 2.9, 17 x 14 x 61, three
+// for one after the other.  One wavefront to a workgroup while that leaves none to share a compute unit, for the loads of its
+// wavefronts take turns (30 of 16 bytes each); beyond that wavefronts side by side, whose windows overlap, stay in one workgroup.  5 x 5, launch to launch in a graph: 13 x 13 x 128, one image, 3.2 -> 2.9 us, 30 x 30 x 198 4.8 -> 2.9, 17 x 14 x 61, three
 // images, 5.4 -> 3.0, 20 x 20 x 128, 64 images, 4.8 -> 4.4; images of one row, 512 of 40 x 480, 9.5 -> 8.9; 3 x 3 and 2 x 2 as much.
 template <int K, int D>
-__global__ __launch_bounds__(64) void max_pool_s8_window_row_kernel(const WindowPoolArgs a)
+__global__ __launch_bounds__(kThreads) void max_pool_s8_window_row_kernel(const WindowPoolArgs a)
 {
     typedef Vec<D> V;
-    const unsigned tid = blockIdx.x * 64 + threadIdx.x;
+    const unsigned tid = blockIdx.x * blockDim.x + threadIdx.x;
     if (tid >= a.total)
         return;
     const unsigned q0 = fastdiv(tid, a.fd_cv);
@@ -246,8 +246,10 @@ template <int K, int D>
 hipError_t launch_window(const WindowPoolArgs &a, bool whole, hipStream_t stream)
 {
     const dim3 grid((a.total + kThreads - 1) / kThreads);
-    if (a.rows == 1)
+    if (a.rows == 1 && grid.x <= 256)
         hipLaunchKernelGGL((max_pool_s8_window_row_kernel<K, D>), dim3(grid.x * (kThreads / 64)), dim3(64), 0, stream, a);
+    else if (a.rows == 1)
+        hipLaunchKernelGGL((max_pool_s8_window_row_kernel<K, D>), grid, dim3(kThreads), 0, stream, a);
     else if (whole)
         hipLaunchKernelGGL((max_pool_s8_window_kernel<K, D, false>), grid, dim3(kThreads), 0, stream, a);
     else
