@@ -440,6 +440,7 @@ int espdl_hip_conv2d_gap_s8_supported(const espdl_hip_conv_desc *desc)
 int espdl_hip_conv2d_gap_s8(const espdl_hip_conv_desc *desc, const int8_t *in, const int8_t *filter, const int32_t *bias,
                             const int32_t *shift, int32_t conv_out_exp, int32_t pool_out_exp, int8_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     espdl::ConvGeom g;
     const int rc = derive_geometry(desc, &g);
     if (rc != ESPDL_HIP_OK)
@@ -464,6 +465,7 @@ int espdl_hip_conv2d_gap_s8(const espdl_hip_conv_desc *desc, const int8_t *in, c
 
 int espdl_hip_lut_s8(const int8_t *in, int64_t size, const int8_t *table, int8_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (size < 0)
         return fail(ESPDL_HIP_EINVAL, "negative size");
     if (size == 0)
@@ -476,6 +478,7 @@ int espdl_hip_lut_s8(const int8_t *in, int64_t size, const int8_t *table, int8_t
 int espdl_hip_prelu_s8(const int8_t *in, int64_t pixels, int32_t channels, const int8_t *alpha, int32_t shift,
                        int8_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (pixels < 0 || channels <= 0)
         return fail(ESPDL_HIP_EINVAL, "bad extents: pixels %lld channels %d", (long long)pixels, channels);
     if (pixels == 0)
@@ -498,6 +501,7 @@ static int check_exps(int32_t in_exp, int32_t out_exp)
 
 int espdl_hip_relu_s8(const int8_t *in, int64_t size, int32_t in_exp, int32_t out_exp, int8_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (size < 0)
         return fail(ESPDL_HIP_EINVAL, "negative size");
     if (check_exps(in_exp, out_exp) != ESPDL_HIP_OK)
@@ -513,6 +517,7 @@ int espdl_hip_relu_s8(const int8_t *in, int64_t size, int32_t in_exp, int32_t ou
 int espdl_hip_clip_s8(const int8_t *in, int64_t size, int32_t min_q, int32_t max_q, int32_t in_exp, int32_t out_exp,
                       int8_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (size < 0)
         return fail(ESPDL_HIP_EINVAL, "negative size");
     if (min_q < -128 || max_q > 127)
@@ -531,6 +536,7 @@ int espdl_hip_clip_s8(const int8_t *in, int64_t size, int32_t min_q, int32_t max
 int espdl_hip_add_s8(const int32_t out_dims[4], const int64_t in0_strides[4], const int64_t in1_strides[4],
                      const int8_t *in0, const int8_t *in1, int8_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (out_dims == nullptr || in0_strides == nullptr || in1_strides == nullptr)
         return fail(ESPDL_HIP_EINVAL, "dims and strides must not be NULL");
     long long size = 1;
@@ -554,6 +560,7 @@ int espdl_hip_mul_s8(const int32_t out_dims[4], const int64_t in0_strides[4], co
                      const int8_t *in0, const int8_t *in1, int32_t mul_shift, int32_t round_mode, int8_t *out,
                      void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (out_dims == nullptr || in0_strides == nullptr || in1_strides == nullptr)
         return fail(ESPDL_HIP_EINVAL, "dims and strides must not be NULL");
     if (mul_shift < -60 || mul_shift > 60)
@@ -581,6 +588,7 @@ int espdl_hip_mul_s8(const int32_t out_dims[4], const int64_t in0_strides[4], co
 int espdl_hip_global_avg_pool_s8(const int8_t *in, int32_t batch, int32_t h, int32_t w, int32_t c, int32_t in_exp,
                                  int32_t out_exp, int8_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (batch < 0 || h <= 0 || w <= 0 || c <= 0 || (long long)h * w > (1 << 23) || batch > 65535)
         return fail(ESPDL_HIP_EINVAL, "bad extents: batch %d, %dx%dx%d", batch, h, w, c);
     if (check_exps(in_exp, out_exp) != ESPDL_HIP_OK)
@@ -597,6 +605,7 @@ int espdl_hip_global_avg_pool_s8(const int8_t *in, int32_t batch, int32_t h, int
 int espdl_hip_requantize_s8(const int8_t *in, int64_t size, int32_t in_exp, int32_t out_exp, int8_t *out,
                             void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (size < 0)
         return fail(ESPDL_HIP_EINVAL, "negative size");
     if (check_exps(in_exp, out_exp) != ESPDL_HIP_OK)
@@ -613,6 +622,7 @@ int espdl_hip_requantize_s8(const int8_t *in, int64_t size, int32_t in_exp, int3
 int espdl_hip_requantize_s8_rows(const int8_t *in, int64_t in_pitch, int8_t *out, int64_t out_pitch, int64_t row_bytes,
                                  int64_t rows, int32_t in_exp, int32_t out_exp, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (rows < 0 || row_bytes < 0 || in_pitch < row_bytes || out_pitch < row_bytes)
         return fail(ESPDL_HIP_EINVAL, "rows of %lld bytes need pitches of at least that (got %lld / %lld) and a count >= 0",
                     (long long)row_bytes, (long long)in_pitch, (long long)out_pitch);
@@ -632,6 +642,7 @@ int espdl_hip_requantize_s8_rows(const int8_t *in, int64_t in_pitch, int8_t *out
 int espdl_hip_requantize(const void *in, int32_t in_dtype, int64_t size, int32_t in_exp, int32_t out_exp, void *out,
                          int32_t out_dtype, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (size < 0)
         return fail(ESPDL_HIP_EINVAL, "negative size");
     if ((in_dtype != ESPDL_HIP_S8 && in_dtype != ESPDL_HIP_S16) || (out_dtype != ESPDL_HIP_S8 && out_dtype != ESPDL_HIP_S16))
@@ -655,6 +666,7 @@ int espdl_hip_requantize(const void *in, int32_t in_dtype, int64_t size, int32_t
 int espdl_hip_concat(int32_t n_inputs, const void *const *inputs, const int64_t *copy_bytes, int64_t loop_times,
                      void *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (n_inputs < 0 || loop_times < 0 || (n_inputs > 0 && (inputs == nullptr || copy_bytes == nullptr)))
         return fail(ESPDL_HIP_EINVAL, "bad concat arguments");
     std::vector<long long> bytes((size_t)n_inputs);
@@ -677,6 +689,7 @@ int espdl_hip_concat(int32_t n_inputs, const void *const *inputs, const int64_t 
 int espdl_hip_copy_rows(const void *src, int64_t src_pitch, void *dst, int64_t dst_pitch, int64_t row_bytes,
                         int64_t rows, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (rows < 0 || row_bytes < 0 || src_pitch < 0 || dst_pitch < 0)
         return fail(ESPDL_HIP_EINVAL, "negative size or pitch");
     if (rows == 0 || row_bytes == 0)
@@ -693,6 +706,7 @@ int espdl_hip_copy_rows(const void *src, int64_t src_pitch, void *dst, int64_t d
 int espdl_hip_split(const void *in, int64_t in_pitch, int32_t n_outputs, void *const *outputs, const int64_t *copy_bytes,
                     int64_t rows, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (n_outputs < 1 || outputs == nullptr || copy_bytes == nullptr || rows < 0 || in_pitch < 0)
         return fail(ESPDL_HIP_EINVAL, "split needs at least one output, sizes and a row count >= 0");
     long long total = 0;
@@ -718,6 +732,7 @@ int espdl_hip_split(const void *in, int64_t in_pitch, int32_t n_outputs, void *c
 int espdl_hip_transpose(const void *in, const int32_t *shape, int32_t dims, const int32_t *perm, int32_t n_perm,
                         int32_t elem_size, void *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (dims < 1 || dims > 8 || shape == nullptr)
         return fail(ESPDL_HIP_EINVAL, "transpose handles 1..8 dims");
     if (elem_size != 1 && elem_size != 2 && elem_size != 4)
@@ -755,6 +770,7 @@ int espdl_hip_resize_nearest_s8_pitched(const int8_t *in, int32_t batch, int32_t
                                         int32_t out_w, float scale_h, float scale_w, int32_t in_exp, int32_t out_exp,
                                         int32_t in_pitch, int32_t out_pitch, int8_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (batch < 0 || h <= 0 || w <= 0 || c <= 0 || out_h < 0 || out_w < 0 || !(scale_h > 0) || !(scale_w > 0))
         return fail(ESPDL_HIP_EINVAL, "bad resize geometry");
     if (check_exps(in_exp, out_exp) != ESPDL_HIP_OK)
@@ -778,6 +794,7 @@ int espdl_hip_resize_nearest_s8(const int8_t *in, int32_t batch, int32_t h, int3
                                 int32_t out_w, float scale_h, float scale_w, int32_t in_exp, int32_t out_exp,
                                 int8_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     return espdl_hip_resize_nearest_s8_pitched(in, batch, h, w, c, out_h, out_w, scale_h, scale_w, in_exp, out_exp, 0, 0, out,
                                                stream);
 }
@@ -787,6 +804,7 @@ int espdl_hip_max_pool_pitched(const void *in, int32_t dtype, int32_t batch, int
                                int32_t pad_left, int32_t pad_right, int32_t in_pitch, int32_t out_pitch, void *out,
                                void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (dtype != ESPDL_HIP_S8 && dtype != ESPDL_HIP_S16)
         return fail(ESPDL_HIP_EINVAL, "dtype must be ESPDL_HIP_S8 or ESPDL_HIP_S16");
     if (batch < 0 || h <= 0 || w <= 0 || c <= 0 || k_h <= 0 || k_w <= 0 || stride_h <= 0 || stride_w <= 0 || pad_top < 0 ||
@@ -815,6 +833,7 @@ int espdl_hip_max_pool(const void *in, int32_t dtype, int32_t batch, int32_t h, 
                        int32_t k_w, int32_t stride_h, int32_t stride_w, int32_t pad_top, int32_t pad_bottom,
                        int32_t pad_left, int32_t pad_right, void *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     return espdl_hip_max_pool_pitched(in, dtype, batch, h, w, c, k_h, k_w, stride_h, stride_w, pad_top, pad_bottom, pad_left,
                                       pad_right, 0, 0, out, stream);
 }
@@ -823,6 +842,7 @@ int espdl_hip_avg_pool_s8(const int8_t *in, int32_t batch, int32_t h, int32_t w,
                           int32_t stride_h, int32_t stride_w, int32_t pad_top, int32_t pad_bottom, int32_t pad_left,
                           int32_t pad_right, int32_t in_exp, int32_t out_exp, int8_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (batch < 0 || h <= 0 || w <= 0 || c <= 0 || k_h <= 0 || k_w <= 0 || stride_h <= 0 || stride_w <= 0 || pad_top < 0 ||
         pad_bottom < 0 || pad_left < 0 || pad_right < 0 || (long long)k_h * k_w > (1 << 23))
         return fail(ESPDL_HIP_EINVAL, "bad avg_pool geometry");
@@ -844,6 +864,7 @@ int espdl_hip_avg_pool_s8(const int8_t *in, int32_t batch, int32_t h, int32_t w,
 int espdl_hip_slice(const void *in, const int32_t *shape, int32_t dims, const int32_t *start, const int32_t *step,
                     const int32_t *out_shape, int32_t elem_size, void *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (dims < 1 || dims > 8 || shape == nullptr || start == nullptr || step == nullptr || out_shape == nullptr)
         return fail(ESPDL_HIP_EINVAL, "slice handles 1..8 dims");
     if (elem_size != 1 && elem_size != 2 && elem_size != 4)
@@ -875,6 +896,7 @@ int espdl_hip_slice(const void *in, const int32_t *shape, int32_t dims, const in
 int espdl_hip_reduce_int(const void *in, int32_t dtype, const int32_t *shape, int32_t dims, const int32_t *reduce_flag,
                          int32_t op, int32_t shift, int32_t round_mode, void *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (dtype != ESPDL_HIP_S8 && dtype != ESPDL_HIP_S16)
         return fail(ESPDL_HIP_EINVAL, "dtype must be ESPDL_HIP_S8 or ESPDL_HIP_S16");
     if (dims < 1 || dims > 8 || shape == nullptr || reduce_flag == nullptr)
@@ -917,6 +939,7 @@ int espdl_hip_reduce_int(const void *in, int32_t dtype, const int32_t *shape, in
 int espdl_hip_pad(const void *in, const int32_t *shape, int32_t dims, const int32_t *pads, int32_t mode,
                   int32_t constant_value, int32_t elem_size, void *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (dims < 1 || dims > 8 || shape == nullptr || pads == nullptr)
         return fail(ESPDL_HIP_EINVAL, "pad handles 1..8 dims");
     if (elem_size != 1 && elem_size != 2 && elem_size != 4)
@@ -957,6 +980,7 @@ int espdl_hip_pad(const void *in, const int32_t *shape, int32_t dims, const int3
 int espdl_hip_reduce_mean_s8(const int8_t *in, const int32_t *shape, int32_t dims, const int32_t *reduce_flag,
                              int32_t in_exp, int32_t out_exp, int8_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (dims < 1 || dims > 8 || shape == nullptr || reduce_flag == nullptr)
         return fail(ESPDL_HIP_EINVAL, "reduce_mean handles 1..8 dims");
     if (check_exps(in_exp, out_exp) != ESPDL_HIP_OK)
@@ -1370,6 +1394,7 @@ static hipError_t launch_mbconv_route(const espdl::MbconvParams &p, int route, h
 int espdl_hip_mbconv_s8(const espdl_hip_mbconv_desc *desc, const int8_t *in, const espdl_hip_mbconv_weights *w,
                         const int8_t *residual, int8_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     espdl::MbconvParams p = {};
     const int rc = mbconv_params(desc, in, w, residual, out, &p);
     if (rc != ESPDL_HIP_OK || p.batch == 0)
@@ -1457,6 +1482,7 @@ int64_t espdl_hip_mbconv_s8_workspace(const espdl_hip_mbconv_desc *desc)
 int espdl_hip_mbconv_s8_ws(const espdl_hip_mbconv_desc *desc, const int8_t *in, const espdl_hip_mbconv_weights *w,
                            const int8_t *residual, void *workspace, int8_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (workspace == nullptr)
         return espdl_hip_mbconv_s8(desc, in, w, residual, out, stream);
     espdl::MbconvParams p = {};
@@ -1510,6 +1536,7 @@ static int binary_s16(int op, const int32_t out_dims[4], const int64_t in0_strid
 int espdl_hip_add_s16(const int32_t out_dims[4], const int64_t in0_strides[4], const int64_t in1_strides[4],
                       const int16_t *in0, const int16_t *in1, int16_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     return binary_s16(0, out_dims, in0_strides, in1_strides, in0, in1, 0, ESPDL_HIP_ROUND_HALF_UP, out, stream);
 }
 
@@ -1517,18 +1544,21 @@ int espdl_hip_mul_s16(const int32_t out_dims[4], const int64_t in0_strides[4], c
                       const int16_t *in0, const int16_t *in1, int32_t mul_shift, int32_t round_mode, int16_t *out,
                       void *stream)
 {
+    REFUSE_IN_A_GROUP();
     return binary_s16(1, out_dims, in0_strides, in1_strides, in0, in1, mul_shift, round_mode, out, stream);
 }
 
 int espdl_hip_sub_s16(const int32_t out_dims[4], const int64_t in0_strides[4], const int64_t in1_strides[4],
                       const int16_t *in0, const int16_t *in1, int16_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     return binary_s16(2, out_dims, in0_strides, in1_strides, in0, in1, 0, ESPDL_HIP_ROUND_HALF_UP, out, stream);
 }
 
 int espdl_hip_div_s16(const int32_t out_dims[4], const int64_t in0_strides[4], const int64_t in1_strides[4],
                       const int16_t *in0, const int16_t *in1, int32_t div_shift, int16_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     return binary_s16(3, out_dims, in0_strides, in1_strides, in0, in1, div_shift, ESPDL_HIP_ROUND_HALF_UP, out, stream);
 }
 
@@ -1559,12 +1589,14 @@ static int subdiv_s8(bool div, const int32_t out_dims[4], const int64_t in0_stri
 int espdl_hip_sub_s8(const int32_t out_dims[4], const int64_t in0_strides[4], const int64_t in1_strides[4],
                      const int8_t *in0, const int8_t *in1, int8_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     return subdiv_s8(false, out_dims, in0_strides, in1_strides, in0, in1, 0, out, stream);
 }
 
 int espdl_hip_div_s8(const int32_t out_dims[4], const int64_t in0_strides[4], const int64_t in1_strides[4],
                      const int8_t *in0, const int8_t *in1, int32_t div_shift, int8_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     return subdiv_s8(true, out_dims, in0_strides, in1_strides, in0, in1, div_shift, out, stream);
 }
 
@@ -1572,6 +1604,7 @@ int espdl_hip_avg_pool_s16(const int16_t *in, int32_t batch, int32_t h, int32_t 
                            int32_t stride_h, int32_t stride_w, int32_t pad_top, int32_t pad_bottom, int32_t pad_left,
                            int32_t pad_right, int32_t in_exp, int32_t out_exp, int16_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (batch < 0 || h <= 0 || w <= 0 || c <= 0 || k_h <= 0 || k_w <= 0 || stride_h <= 0 || stride_w <= 0 || pad_top < 0 ||
         pad_bottom < 0 || pad_left < 0 || pad_right < 0 || (long long)k_h * k_w > (1 << 15))
         return fail(ESPDL_HIP_EINVAL, "bad avg_pool geometry");
@@ -1593,6 +1626,7 @@ int espdl_hip_avg_pool_s16(const int16_t *in, int32_t batch, int32_t h, int32_t 
 int espdl_hip_reduce_mean_s16(const int16_t *in, const int32_t *shape, int32_t dims, const int32_t *reduce_flag,
                               int32_t in_exp, int32_t out_exp, int16_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (dims < 1 || dims > 8 || shape == nullptr || reduce_flag == nullptr)
         return fail(ESPDL_HIP_EINVAL, "reduce_mean handles 1..8 dims");
     if (check_exps(in_exp, out_exp) != ESPDL_HIP_OK)
@@ -1621,6 +1655,7 @@ int espdl_hip_insert_zeros(const void *in, int32_t elem_size, int32_t batch, int
                            int32_t stride_h, int32_t stride_w, int32_t output_padding_h, int32_t output_padding_w,
                            void *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (elem_size != 1 && elem_size != 2 && elem_size != 4)
         return fail(ESPDL_HIP_EINVAL, "elem_size must be 1, 2 or 4");
     if (batch < 0 || h < 0 || w < 0 || c < 0)
@@ -1655,6 +1690,7 @@ static int table_step(int32_t table_size)
 int espdl_hip_lut_s16(const int16_t *in, int64_t size, const int16_t *table, int32_t table_size, int32_t round_mode,
                       int16_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (size < 0)
         return fail(ESPDL_HIP_EINVAL, "negative size");
     if (round_mode != ESPDL_HIP_ROUND_HALF_UP && round_mode != ESPDL_HIP_ROUND_HALF_EVEN)
@@ -1721,6 +1757,7 @@ int espdl_hip_conv2d_s16_x8(const espdl_hip_conv_desc *desc, const int8_t *in, c
 int espdl_hip_softmax_s8(const int8_t *in, int64_t outer, int64_t len, int64_t inner, int32_t in_exp, float *out,
                          void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (outer < 0 || len < 0 || inner < 0)
         return fail(ESPDL_HIP_EINVAL, "negative extent");
     if (check_exps(in_exp, 0) != ESPDL_HIP_OK)
@@ -1738,6 +1775,7 @@ int espdl_hip_softmax_s8(const int8_t *in, int64_t outer, int64_t len, int64_t i
 
 int espdl_hip_quantize_f32(const float *in, int64_t size, int32_t out_exp, int32_t elem_size, void *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (size < 0)
         return fail(ESPDL_HIP_EINVAL, "negative size");
     if (elem_size != 1 && elem_size != 2)
@@ -1755,6 +1793,7 @@ int espdl_hip_quantize_f32(const float *in, int64_t size, int32_t out_exp, int32
 
 int espdl_hip_dequantize_f32(const void *in, int64_t size, int32_t in_exp, int32_t elem_size, float *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (size < 0)
         return fail(ESPDL_HIP_EINVAL, "negative size");
     if (elem_size != 1 && elem_size != 2)
@@ -1774,6 +1813,7 @@ int espdl_hip_matmul_s8(const int8_t *a, const int8_t *b, int32_t m, int32_t k, 
                         const int64_t a_stride[2], const int64_t b_stride[2], int32_t shift, int32_t activation,
                         int32_t round_mode, int8_t *out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (lead == nullptr || a_stride == nullptr || b_stride == nullptr)
         return fail(ESPDL_HIP_EINVAL, "lead, a_stride and b_stride must not be NULL");
     if (m < 0 || k < 0 || n < 0 || lead[0] < 0 || lead[1] < 0 || a_stride[0] < 0 || a_stride[1] < 0 || b_stride[0] < 0 ||
@@ -1836,6 +1876,7 @@ int espdl_hip_attention_s8_supported(const espdl_hip_attention_desc *desc)
 int espdl_hip_attention_s8(const espdl_hip_attention_desc *desc, const int8_t *qkv, const int8_t *mul_constant, int8_t *out,
                            int8_t *v_out, void *stream)
 {
+    REFUSE_IN_A_GROUP();
     if (desc == nullptr)
         return fail(ESPDL_HIP_EINVAL, "desc must not be NULL");
     const espdl_hip_attention_desc &d = *desc;

@@ -48,9 +48,16 @@ inline bool conv_is_dense(const ConvGeom &g)
     return g.in_pitch == g.in_c && g.out_pitch == g.out_c && g.res_pitch == g.out_c;
 }
 
-// Between espdl_hip_conv2d_group_begin and _end a thread's launches that can share one are held back; _end sends them out.
+// Between espdl_hip_conv2d_group_begin and _end a thread's launches that can share one are held back; _end sends them out.  Only
+// the three calls that a group is made of get that far: every other entry point that launches refuses while one is open, for it
+// might read what has not been sent yet.
 constexpr int kMostGrouped = 4;
 inline thread_local bool group_open = false;
+#define REFUSE_IN_A_GROUP()                                                                                             \
+    do {                                                                                                                \
+        if (espdl::group_open)                                                                                          \
+            return espdl::set_error(ESPDL_HIP_EINVAL, "%s in an open group of convolutions", __func__);                 \
+    } while (0)
 int conv2d_s8_narrow_group_kind(const ConvGeom &g, int cu_count);
 int conv2d_s16_group_kind(const ConvGeom &g, bool x8, int table_size, int cu_count);
 hipError_t flush_conv2d_s8_narrow();

@@ -57,6 +57,7 @@ extern "C" int espdl_hip_mbconv_s8_staged(const espdl_hip_mbconv_desc *d, const 
                                            const espdl_hip_mbconv_weights *w, const int8_t *residual, int8_t *out,
                                            void *stream)
 {
+    REFUSE_IN_A_GROUP();
     int32_t out_h = 0, out_w = 0;
     int rc = espdl_hip_mbconv_out_shape(d, &out_h, &out_w); // validates the descriptor
     if (rc != ESPDL_HIP_OK)

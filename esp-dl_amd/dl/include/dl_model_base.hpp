@@ -64,7 +64,8 @@ public:
     /// Run segment `stage_index` of `stage_num` near-equal segments of the plan (dl_model_base.cpp:240-260).
     virtual void run(int stage_num, int stage_index, runtime_mode_t mode = RUNTIME_MODE_SINGLE_CORE);
     /// Enqueue only; pair with synchronize().  Uses the captured HIP graph when enable_graph() succeeded.
-    /// The launches of a pass stand together on the stream: passes of several threads follow one another, whole.
+    /// The launches of a pass stand together on the stream: passes of several threads follow one another, whole.  A pass is
+    /// no part of a group of convolutions (espdl_hip_conv2d_group_begin): with one open on the thread it fails.
     void run_async(runtime_mode_t mode = RUNTIME_MODE_SINGLE_CORE);
     void synchronize();
     /// Capture the plan into a HIP graph (after one eager run has created every module's device state).  A short
@@ -115,6 +116,7 @@ private:
     void fuse_s16_input();
     void merge_requantize();
     size_t plan_bytes();
+    bool in_a_group();
     void enqueue(runtime_mode_t mode);
     char *staging(size_t bytes);
 

@@ -1436,6 +1436,8 @@ void Model::run_async(runtime_mode_t mode)
         m_failed = true;
         return;
     }
+    if (in_a_group())
+        return;
     if (m_launches) {
         for (const hipKernelNodeParams &p : static_cast<LaunchList *>(m_launches)->launches)
             if (!hip_ok(hipLaunchKernel(p.func, p.gridDim, p.blockDim, p.kernelParams, p.sharedMemBytes,
@@ -1454,14 +1456,35 @@ void Model::run_async(runtime_mode_t mode)
     enqueue(mode);
 }
 
+// In a group of convolutions that the caller has open on this thread a pass's own would be held back, and the modules that read
+// them enqueued in front of them: such a pass fails with nothing enqueued, also one whose plan shares no launch.
+bool Model::in_a_group()
+{
+    if (espdl_hip_conv2d_group_begin() == ESPDL_HIP_OK && espdl_hip_conv2d_group_end() == ESPDL_HIP_OK)
+        return false;
+    DL_LOGE(TAG, "A pass of a model cannot be part of a group of convolutions: %s", espdl_hip_last_error());
+    return true;
+}
+
 void Model::enqueue(runtime_mode_t mode)
 {
+    // ends the group however its modules are left: one that stayed open would hold back what the thread launches next
+    struct Group {
+        bool open;
+        ~Group()
+        {
+            if (open && espdl_hip_conv2d_group_end() != ESPDL_HIP_OK)
+                DL_LOGE(TAG, "%s", espdl_hip_last_error());
+        }
+    };
     for (const std::vector<int> &part : m_schedule) {
-        const bool group = part.size() > 1 && espdl_hip_conv2d_group_begin() == ESPDL_HIP_OK; // (else one by one)
+        const Group group{part.size() > 1 && espdl_hip_conv2d_group_begin() == ESPDL_HIP_OK};
+        if (part.size() > 1 && !group.open) {
+            DL_LOGE(TAG, "%s", espdl_hip_last_error());
+            return;
+        }
         for (int i : part)
             m_execution_plan[i]->forward(m_model_context, mode);
-        if (group && espdl_hip_conv2d_group_end() != ESPDL_HIP_OK)
-            DL_LOGE(TAG, "%s", espdl_hip_last_error());
     }
 }
 
@@ -1586,6 +1609,8 @@ void Model::run(int stage_num, int stage_index, runtime_mode_t mode)
     }
     std::lock_guard<std::mutex> pass(m_pass_mutex);
     begin_pass();
+    if (in_a_group())
+        return;
     const int start = stage_index * plan_size / stage_num;
     const int end = (stage_index + 1) * plan_size / stage_num;
     for (int i = start; i < end; i++)
@@ -1599,6 +1624,8 @@ bool Model::enable_graph()
     if (!m_built || graph_enabled())
         return graph_enabled();
     begin_pass();
+    if (in_a_group())
+        return false;
     hipStream_t s = static_cast<hipStream_t>(m_stream);
     // one eager pass so that every module has uploaded its shifts / tables before capture starts; modules that
     // carry data between passes (StreamingCache) get it back afterwards, the pass counts for nothing
@@ -1671,6 +1698,8 @@ esp_err_t Model::test()
         return ESP_FAIL;
     std::lock_guard<std::mutex> pass(m_pass_mutex);
     begin_pass();
+    if (in_a_group())
+        return ESP_FAIL;
     for (auto &kv : m_inputs) {
         TensorBase *test_input = m_fbs_model->get_test_input_tensor(kv.first);
         if (!test_input) {
@@ -1731,6 +1760,8 @@ std::vector<module_info> Model::get_module_info(int repeats)
     if (!m_built)
         return info;
     std::lock_guard<std::mutex> pass(m_pass_mutex);
+    if (in_a_group())
+        return info;
     hipStream_t s = static_cast<hipStream_t>(m_stream);
     if (repeats < 1)
         repeats = 1;

@@ -110,8 +110,11 @@ const char *espdl_hip_conv2d_s8_kernel(const espdl_hip_conv_desc *desc, const vo
 
 /*
  * Convolutions that do not depend on one another in one launch.  Between the two calls a thread makes up to four calls of
- * espdl_hip_conv2d, _conv2d_add or _conv2d_s16_x8 (and no others) on one stream, none of which reads or overwrites what another one
- * writes; launches of one build are held back and leave together in _end, on that stream, the others at once.  Which layers share
+ * espdl_hip_conv2d, _conv2d_add or _conv2d_s16_x8 on one stream, none of which reads or overwrites what another one
+ * writes; launches of one build are held back and leave together in _end, on that stream, the others at once.  So until _end
+ * such a call returns ESPDL_HIP_OK with nothing on the stream: an event recorded or a copy enqueued behind it by other means
+ * comes in front of it.  The group belongs to the thread.  Every other call of this header that takes a stream fails
+ * (ESPDL_HIP_EINVAL) on a thread with an open group, and so does a pass of a dl::Model.  Which layers share
  * a launch: those of one kind, 0 for a layer that takes another kernel.  `x8`: espdl_hip_conv2d_s16_x8 with a table of that many
  * entries (0: none).  Groups do not nest: _begin fails (ESPDL_HIP_EINVAL) where one is open, _end where none is.
  */

@@ -198,3 +198,89 @@ def test_narrow_kernels_stay_inside_the_grid_limit():
             for l in log:
                 assert l["grid"][0] * l["block"][0] < 1 << 32, (dtype, n, l)
     ''')
+
+
+@pytest.mark.parametrize("spec,batch", [("config4_yolo_style(resolution=96)", 1), ("config1_single_conv()", 1),
+                                        ("config2_mbv2_block()", 2)], ids=["shared launches", "one convolution", "block"])
+def test_a_pass_in_an_open_group_of_convolutions_fails(spec, batch):
+    """The group would hold back the pass's convolutions while the modules that read them run: every way to run the plan fails
+    and launches nothing, and works again behind the group."""
+    host_hip.run('''
+    L, spec = m.lib(), zoo.%s
+    mdl = model.Model(model.Graph.from_spec(spec), %d)
+
+    def passes():
+        ways = {"run": mdl.run, "run_async": mdl.run_async, "enable_graph": mdl.enable_graph, "profile": lambda: mdl.profile(1)}
+        for name, way in ways.items():
+            hip.host_hip_clear()
+            try:
+                done = way()
+                done = len(done) > 0 if name == "profile" else done in (None, True)
+            except model.EspdlModelError:
+                done = False
+            yield name, done, hip.host_hip_launches(), hip.host_hip_calls(b"hipGraphLaunch")
+            if name == "enable_graph":
+                mdl.disable_graph()
+
+    def replay():
+        hip.host_hip_clear()
+        try:
+            mdl.run()
+        except model.EspdlModelError:
+            return False, hip.host_hip_launches(), hip.host_hip_calls(b"hipGraphLaunch")
+        return True, hip.host_hip_launches(), hip.host_hip_calls(b"hipGraphLaunch")
+
+    mdl.run()
+    assert L.espdl_hip_conv2d_group_begin() == 0
+    for name, done, n, graphs in passes():
+        assert not done and n == 0 and graphs == 0, (name, done, n)
+    hip.host_hip_clear()
+    assert L.espdl_hip_conv2d_group_end() == 0 and hip.host_hip_launches() == 0  # nothing was held back either
+    for name, done, n, graphs in passes():
+        assert done and n + graphs > 0, (name, done, n)
+    assert mdl.enable_graph() and replay()[0]
+    assert L.espdl_hip_conv2d_group_begin() == 0
+    assert replay() == (False, 0, 0)
+    assert L.espdl_hip_conv2d_group_end() == 0
+    assert replay()[0]
+    ''' % (spec, batch))
+
+
+def test_other_calls_refuse_in_an_open_group():
+    """What a group holds back may be read by any other launch: every call of the header that takes a stream, but the three
+    that a group is made of, fails before it looks at its arguments."""
+    host_hip.run('''
+    import re
+    text = re.sub(r"/\\*.*?\\*/", "", open(sys.path[0] + "/include/espdl_hip.h").read(), flags=re.S)
+    calls = {name: args.count(",") + 1 for name, args in re.findall(r"\\bint (espdl_hip_\\w+)\\(([^)]*)\\)", text) if "void *stream" in args}
+    members = {"espdl_hip_conv2d", "espdl_hip_conv2d_add", "espdl_hip_conv2d_s16_x8"}
+    assert len(calls) > 40 and members < set(calls)
+    L = m.lib()
+    message = L.espdl_hip_last_error
+    assert L.espdl_hip_conv2d_group_begin() == 0
+    for name, n in calls.items():
+        call = getattr(ctypes.CDLL(m.capi.LIB_PATH), name)  # (a handle without argument types)
+        assert call(*[ctypes.c_void_p(0)] * n) == -22, name
+        assert (name.encode() + b" in an open group" in message()) == (name not in members), (name, message())
+    assert hip.host_hip_launches() == 0
+    assert L.espdl_hip_conv2d_group_end() == 0
+    for name, n in calls.items():
+        getattr(ctypes.CDLL(m.capi.LIB_PATH), name)(*[ctypes.c_void_p(0)] * n)
+        assert b"in an open group" not in message(), (name, message())
+    ''')
+
+
+def test_a_block_in_an_open_group_is_refused():
+    """Its project layer is a narrow convolution: the group would keep it."""
+    host_hip.run('''
+    d = m.capi.MbconvDesc(1, 14, 14, 64, 384, 64, 1, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 0, 0, 1, 1, 1)
+    base = 1 << 30
+    w = m.capi.MbconvWeights(base * 3, None, base * 4, base * 5, None, base * 6, base * 7, None, base * 8)
+    call = lambda: m.lib().espdl_hip_mbconv_s8_ws(ctypes.byref(d), base, ctypes.byref(w), None, base * 2, base * 10, None)
+    assert m.lib().espdl_hip_mbconv_s8_workspace(ctypes.byref(d)) > 0
+    assert call() == 0 and len(launches()) == 2
+    hip.host_hip_clear()
+    assert m.lib().espdl_hip_conv2d_group_begin() == 0
+    assert call() == -22 and len(launches()) == 0
+    assert m.lib().espdl_hip_conv2d_group_end() == 0 and len(launches()) == 0
+    ''')
