@@ -1444,7 +1444,10 @@ static auto project_launch(const espdl::ConvGeom &g, const void *in, const void 
 // The single launch is a chain of 10 to 25 us through all expanded channels of a tile, whatever the batch, until the
 // device is full; the two launches start at 7 us and grow with the work (MobileNetV2 at 224 x 224: one image 282 -> 155 us,
 // 16 images 296 -> 221 us, with the launches of then, 133 and 200 us now; the blocks of batch 256 stay single launches).
-// Where no single-launch kernel has a fast build the alternative is three launches, of which the depthwise one alone takes 9 us.
+// Where no single-launch kernel has a fast build the alternative is the convolutions by themselves, of which the depthwise one
+// alone takes 9 us and which write and read the expanded tensor too: 66 such blocks with 8 to 260 MB between the launches took 1.25
+// times the two launches' time in the geometric mean (56 x 56 x 64 -> 384 -> 64, 226 images: 327 and 228 us; 0.8 to 1.0 of it where the
+// parts still fit the last-level cache and the reduction is long: 204 images of 20 x 20 x 128 -> 512 -> 128, 62 and 79 us).
 int64_t espdl_hip_mbconv_s8_workspace(const espdl_hip_mbconv_desc *desc)
 {
     espdl::MbconvParams p = {};
@@ -1465,18 +1468,14 @@ int64_t espdl_hip_mbconv_s8_workspace(const espdl_hip_mbconv_desc *desc)
     float project = 0.f;
     (void)project_launch(g, aligned, aligned, cus, &project);
     const int64_t between = (int64_t)p.batch * p.out_h * p.out_w * p.exp_c;
-    // A quarter more with Clips between the stages (18 images of 56 x 56 x 24 -> 144 -> 24: 20.2 us as two launches, 19.1 as one) and,
-    // half even, on more than the estimate was fitted to (256 of 12 x 12 x 96 -> 576 -> 96: 45 and 34 us).
-    const bool clip = p.clip_e || p.clip_d;
-    const float expand_dw = espdl::mbconv_s8_expand_dw_us(p) * (clip || (p.half_even && between > (16ll << 20)) ? 1.25f : 1.f);
-    float other = 9.f + 1.25f * expand_dw + project;
-    if (espdl_hip_mbconv_s8_supported(desc) == 0)
-        other = 1e30f; // a Clip between the stages in half-even mode: no single launch
-    else if (espdl_hip_mbconv_s8_preferred(desc) == 1)
-        other = std::min(mbconv_tile_us(p, espdl_hip_mbconv_s8_supported(desc), cus), espdl::mbconv_s8_walk_us(p, cus));
-    // 0.2 us a megabyte for the tensor between the launches, which one of them writes and the other reads back.  The choice takes
-    // 0.3 % more time than the better one of the two in the mean of 1089 blocks on 1 to 256 images, 2 % of them 5 % more and over.
-    return expand_dw + project + 0.2e-6f * (float)between < other ? between : 0;
+    // no single launch at all (a Clip between the stages in half-even mode), or none that the convolutions would be left for
+    if (espdl_hip_mbconv_s8_supported(desc) == 0 || espdl_hip_mbconv_s8_preferred(desc) != 1)
+        return between;
+    const float one = std::min(mbconv_tile_us(p, espdl_hip_mbconv_s8_supported(desc), cus), espdl::mbconv_s8_walk_us(p, cus));
+    // 0.3 us a megabyte for the tensor between the launches, which one of them writes and the other reads back, and which the projection's
+    // estimate leaves out.  Of 2368 blocks on 2 to 256 images, with and without Clips, in both rounding modes, the choice takes 0.6 % more
+    // time than the better one of the two in the mean, 4 % of them 5 % more and over.
+    return espdl::mbconv_s8_expand_dw_us(p) + project + 0.3e-6f * (float)between < one ? between : 0;
 }
 
 int espdl_hip_mbconv_s8_ws(const espdl_hip_mbconv_desc *desc, const int8_t *in, const espdl_hip_mbconv_weights *w,

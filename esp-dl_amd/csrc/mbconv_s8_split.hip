@@ -143,7 +143,7 @@ __global__ __launch_bounds__(kThreads, 4) void mbconv_s8_expand_dw_kernel(const 
             int at[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                if (first + j * kThreads >= n_pieces) // uniform
+                if (!LOOP && first + j * kThreads >= n_pieces) // uniform
                     break;
                 const int u = first + j * kThreads + tid;
                 const int pp = (int)fastdiv((unsigned)u, a.fd_units), unit = u - pp * a.units;
@@ -216,8 +216,8 @@ __global__ __launch_bounds__(kThreads, 4) void mbconv_s8_expand_dw_kernel(const 
     do {
         Chunk nxt = cur;
         const int sub = 4 * gi + wave;
-        if (LOOP && gi + 1 < g_end) // uniform
-            load_chunk(4 * (gi + 1) + wave, nxt);
+        if constexpr (LOOP) // (the last one again in the last turn: a branch here costs 3 %, 4 % on 80 -> 480 at stride 2)
+            load_chunk(4 * min(gi + 1, g_end - 1) + wave, nxt);
         // constants of this chunk: the short form where every channel of the stage can take it (see mbconv_s8_stages.h)
         int mode_e, mode_d;
         {
@@ -303,21 +303,29 @@ struct SplitPlan {
 };
 
 // Expected time of tiles of `pt` rows: the launch and one workgroup's chain, which is shorter the fewer rows it has, then the work of
-// all workgroups, which grows with the halo (two rows of the patch at stride 1, one at stride 2).  Fitted to 846 launches of 14
-// blocks on 1 to 100 images, 3 to 4 % off; the tile it picks takes 0.7 % more than the best one in the mean, the largest one 11 %.
+// all workgroups, which grows with the halo (two rows of the patch at stride 1, one at stride 2); the highest tiles lose 2 to 4 us
+// where workgroups walk several groups, of which there are fewer and longer ones then.  Fitted to 6700 launches on 1 to 400
+// images and 1 KB to 300 MB of results, each tile forced in turn: 4 to 8 % off; the tile it picks takes 0.5 % more than the best one in
+// the mean, the largest one 26 %.  (A fit to 1 to 100 images, most of them below 4 MB, had the highest tiles at stride 1 half as expensive
+// again as expected beyond that: 48 images of 40 x 40, 24 -> 144, 12.6 us expected, 24.5 measured.)
 float split_us(const MbconvParams &p, int kse, int tw, int pt)
 {
     const long long tiles = (long long)p.batch * ((p.out_w + tw - 1) / tw) * ((p.out_h + pt - 1) / pt);
-    const float work = (float)(tiles * ((p.exp_c + 63) / 64)) * (1.f / 256.f), k = (float)(kse - 1), he = p.half_even ? 1.f : 0.f;
+    const long long groups = (p.exp_c + 63) / 64;
+    const float work = (float)(tiles * groups) * (1.f / 256.f), k = (float)(kse - 1), he = p.half_even ? 1.f : 0.f;
+    const float walks = groups > 1 && tiles * groups >= 2048 ? 1.f : 0.f; // several groups to a workgroup of the highest tiles
     if (p.stride_h == 2)
-        return pt == 1 ? (2.91f + 0.25f * k + work * (0.453f + 0.022f * k)) * (1.f + 0.04f * he)
-            : pt == 2  ? (3.2f + 0.3f * k + work * (0.564f + 0.046f * k)) * (1.f + 0.05f * he)
-                       : (3.6f + 0.49f * k + work * (0.878f + 0.072f * k)) * (1.f + 0.06f * he);
-    if (pt == 2)
-        return (3.06f + 0.164f * k + work * (tw == 7 ? 0.587f : 0.534f + 0.036f * k)) * (1.f + 0.04f * he);
-    if (pt == 4)
-        return (3.42f + 0.166f * k + work * (tw == 7 ? 0.636f + 0.059f * k : 0.653f + 0.057f * k)) * (1.f + 0.05f * he);
-    return (4.02f + (tw == 7 ? 0.2f : 0.35f) * k + work * (tw == 7 ? 0.674f + 0.1f * k : 0.78f - 0.04f * k)) * (1.f + 0.06f * he);
+        return pt == 1 ? (3.2f + 0.18f * k + work * (0.431f + 0.04f * k)) * (1.f + 0.056f * he)
+            : pt == 2  ? (3.41f + 0.21f * k + work * (0.54f + 0.091f * k)) * (1.f + 0.069f * he)
+                       : (3.95f + 0.35f * k + work * (0.696f + 0.208f * k) + 2.3f * walks) * (1.f + 0.077f * he);
+    if (tw == 7)
+        return pt == 2 ? (3.46f + 0.087f * k + work * (0.476f + 0.054f * k)) * (1.f + 0.017f * he)
+            : pt == 4  ? (3.68f + 0.098f * k + work * (0.563f + 0.09f * k)) * (1.f + 0.042f * he)
+                       : (4.11f + 0.133f * k + work * (0.661f + 0.158f * k) + 3.5f * walks) * (1.f + 0.062f * he);
+    const float wide_pixel = kse == 3 ? 0.21f : 0.f; // its patch leaves a compute unit fewer workgroups
+    return pt == 2 ? (3.34f + 0.135f * k + work * (0.513f + 0.071f * k)) * (1.f + 0.058f * he)
+        : pt == 4  ? (3.59f + 0.106f * k + work * (0.667f + 0.17f * k)) * (1.f + 0.07f * he)
+                   : (4.07f + 0.24f * k + work * (0.867f + 0.213f * k + wide_pixel) + 3.5f * walks) * (1.f + 0.096f * he);
 }
 
 SplitPlan split_plan(const MbconvParams &p)

@@ -81,6 +81,29 @@ def test_two_launches_are_weighed_against_the_launch_that_a_block_with_an_add_ta
     assert m.lib().espdl_hip_mbconv_s8_workspace(C.byref(d)) == 0
 
 
+def test_one_or_two_launches_of_a_block_by_what_each_takes():
+    """Blocks that one form takes a tenth less time for and more (us as two launches, and as one or as separate
+    convolutions): large ones that no single launch has a fast build for, and ones on either side of the line."""
+    import ctypes as C
+    import importlib
+    m = importlib.import_module("esp-dl_amd")
+    for batch, hw, cin, ce, cout, half_even, two in (
+            (226, 56, 64, 384, 64, 0, True),     # 228, 327 as convolutions
+            (362, 56, 40, 240, 40, 0, True),     # 274, 316
+            (452, 56, 48, 192, 48, 0, True),     # 255, 323
+            (177, 80, 40, 240, 40, 0, True),     # 285, 317
+            (905, 28, 64, 384, 64, 0, True),     # 227, 329
+            (215, 112, 48, 288, 48, 1, True),    # 787, 921
+            (63, 32, 24, 144, 24, 1, False),     # 32.1, 19.5 as one launch
+            (17, 64, 24, 144, 24, 1, False),     # 31.6, 19.9
+            (122, 28, 32, 192, 32, 1, False),    # 36.2, 23.1
+            (128, 14, 96, 576, 96, 0, False),    # 31.9, 16.5
+            (40, 10, 96, 576, 96, 0, True),      # 11.5, 15.1
+            (6, 7, 160, 960, 160, 1, True)):     # 7.2, 24.6
+        d = m.capi.MbconvDesc(batch, hw, hw, cin, ce, cout, 1, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 0, half_even, ce, ce, cout)
+        assert m.lib().espdl_hip_mbconv_s8_workspace(C.byref(d)) == (batch * hw * hw * ce if two else 0), (batch, hw, cin, ce, cout, half_even)
+
+
 def _dense_kernel(m, shape, out_c, k, stride=1, pad=None, dilation=1, lut=None, residual=None, half_even=0, out_pitch=0, group=1, dtype=None):
     import ctypes as C
     pad = k // 2 * dilation if pad is None else pad
