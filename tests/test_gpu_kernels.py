@@ -1933,24 +1933,33 @@ TWO_LAUNCHES = [
 
 
 # Images enough for each tile of the first launch: 2, 4 and 7 rows at stride 1 (14 and 7 columns), 1, 2 and 4 at stride 2, the largest
-# both with one group of 64 expanded channels per workgroup and with several; last rows and columns that are not full.
+# both with one group of 64 expanded channels per workgroup and with several (loop); last rows and columns that are not full.  The
+# names say which tile a case takes; test_host_runtime.py looks at the launches.
 TWO_LAUNCH_TILES = [
     ("2_rows_14", (9, 9, 23, 48), 208, 20, 1, False, False, ""),
+    ("2_rows_14_three_steps", (30, 9, 20, 132), 144, 8, 1, False, False, "general"),
     ("4_rows_14", (40, 9, 15, 24), 144, 24, 1, True, False, ""),
     ("4_rows_14_halfeven_clips", (40, 9, 15, 24), 144, 24, 1, True, True, "clip"),
-    ("4_rows_14_three_steps", (30, 9, 20, 132), 144, 8, 1, False, False, "general"),
+    ("4_rows_14_three_steps", (16, 11, 20, 132), 144, 8, 1, False, False, "general"),
+    ("4_rows_14_halfeven_many", (150, 10, 9, 24), 208, 8, 1, False, True, ""),
+    ("4_rows_14_many", (260, 11, 20, 20), 144, 4, 1, False, False, ""),
     ("7_rows_14", (150, 10, 9, 24), 208, 8, 1, False, False, ""),
-    ("7_rows_14_halfeven", (150, 10, 9, 24), 208, 8, 1, False, True, ""),
-    ("7_rows_14_loop", (260, 11, 20, 20), 144, 4, 1, False, False, ""),
+    ("7_rows_14_halfeven", (80, 13, 9, 24), 208, 8, 1, False, True, ""),
+    ("7_rows_14_loop", (260, 13, 20, 20), 144, 4, 1, False, False, ""),
+    ("7_rows_14_loop_halfeven_three_steps", (200, 13, 20, 132), 144, 4, 1, False, True, "clip"),
     ("2_rows_7", (4, 9, 7, 160), 960, 16, 1, False, False, ""),
     ("4_rows_7", (30, 9, 7, 72), 320, 16, 1, False, False, "clip"),
+    ("4_rows_7_many", (220, 9, 7, 136), 528, 8, 1, False, False, "general"),
     ("7_rows_7_halfeven", (60, 9, 5, 16), 528, 16, 1, True, True, ""),
-    ("7_rows_7_loop", (220, 9, 7, 136), 528, 8, 1, False, False, "general"),
-    ("1_row_s2", (6, 19, 27, 40), 144, 24, 2, False, False, "clip"),
-    ("2_rows_s2", (12, 19, 27, 40), 144, 24, 2, False, False, ""),
-    ("2_rows_s2_halfeven", (40, 19, 27, 132), 144, 8, 2, False, True, ""),
-    ("4_rows_s2", (100, 16, 14, 40), 144, 8, 2, False, False, "general"),
-    ("4_rows_s2_loop", (130, 19, 27, 40), 144, 8, 2, False, False, ""),
+    ("7_rows_7_loop", (230, 13, 5, 136), 528, 8, 1, False, False, "general"),
+    ("1_rows_7_s2", (4, 19, 27, 40), 144, 24, 2, False, False, "clip"),
+    ("2_rows_7_s2_clips", (6, 19, 27, 40), 144, 24, 2, False, False, "clip"),
+    ("2_rows_7_s2", (12, 19, 27, 40), 144, 24, 2, False, False, ""),
+    ("2_rows_7_s2_halfeven", (40, 19, 27, 132), 144, 8, 2, False, True, ""),
+    ("2_rows_7_s2_many", (130, 19, 27, 40), 144, 8, 2, False, False, ""),
+    ("4_rows_7_s2", (100, 16, 14, 40), 144, 8, 2, False, False, "general"),
+    ("4_rows_7_s2_loop", (130, 23, 27, 40), 144, 8, 2, False, False, ""),
+    ("4_rows_7_s2_loop_halfeven_two_steps", (200, 13, 27, 72), 144, 8, 2, False, True, ""),
 ]
 
 

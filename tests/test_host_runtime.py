@@ -284,3 +284,27 @@ def test_a_block_in_an_open_group_is_refused():
     assert call() == -22 and len(launches()) == 0
     assert m.lib().espdl_hip_conv2d_group_end() == 0 and len(launches()) == 0
     ''')
+
+
+def test_two_launch_cases_take_the_tile_of_their_name():
+    """The builds of the expand + depthwise launch that test_gpu_kernels.py means to run."""
+    host_hip.run('''
+    import re
+    import test_gpu_kernels
+    taken = set()
+    for name, (n, h, w, cin), ce, cout, stride, res, half_even, extra in test_gpu_kernels.TWO_LAUNCH_TILES:
+        d = m.capi.MbconvDesc(n, h, w, cin, ce, cout, 1, 3, 3, stride, stride, 1, 1, 1, 1, 1, 1, 1, 1, 0, int(half_even), ce, ce, cout)
+        if extra == "clip":
+            d.clip_expand = d.clip_dw = 1
+            d.clip_expand_max = d.clip_dw_max = 90
+        base = 1 << 30
+        weights = m.capi.MbconvWeights(base * 3, None, base * 4, base * 5, None, base * 6, base * 7, None, base * 8)
+        hip.host_hip_clear()
+        assert m.lib().espdl_hip_mbconv_s8_ws(ctypes.byref(d), base, ctypes.byref(weights), base * 9 if res else None, base * 2, base * 10, None) == 0
+        build = re.search("kernelILi(.*?)ELi(.*?)ELi(.*?)ELi(.*?)ELb(.)ELb(.)ELb(.)E", launches()[0]["name"]).groups()
+        rows, columns = re.match("([0-9]+)_rows_([0-9]+)", name).groups()
+        want = rows, columns, "2" if "_s2" in name else "1", str(-(-cin // 64)), str(int(half_even)), str(int(extra == "clip")), str(int("loop" in name))
+        assert build == want, (name, build)
+        taken.add((build[0], build[1], build[2], build[6]))
+    assert len(taken) == 12, taken  # nine tiles, three of them with the loop too
+    ''')
