@@ -9,11 +9,11 @@
 // 1.9 TB/s; so a step's bytes pass through LDS and leave as whole aligned 16-byte pieces of memory, cut out of the bytes
 // of this step and the last 16 of the step before, and only the two ends of a row's walk are written by the byte.
 //
-// 20480 pixels x 120 -> 6625 (136 MB written, 26 us at the copy rate): 48 us inside the recognizer, where the kernel that keeps
+// 20480 pixels x 120 -> 6625 (136 MB written, 26 us at the copy rate): 43 us inside the recognizer, where the kernel that keeps
 // filters in LDS took 71 us.  A step is what bounds it: 330 vector and 32 matrix instructions of each of two wavefronts of a SIMD
-// and a barrier, 2.3 us for 32 KB per compute unit.  A workgroup has several walks, over other pixels under the same filters, so
-// that the filters' constants are brought in once (two walks: 178.5 -> 172.8 us for the recognizer on 512 crops; one start each: 50
-// us).  Reading the pieces from LDS with one unaligned instruction instead of five words and shifts costs 4 us.
+// and a barrier, 2.3 us for 32 KB per compute unit.  A workgroup may have several walks, over other pixels under the same filters, so
+// that the filters' constants are brought in once (two walks 42.4 us, one each 46.6; where some shift is below 8 46.1 and 49.9).
+// Reading the pieces from LDS with one unaligned instruction instead of five words and shifts costs 4 us.
 //
 // Restates conv2d_11cn (esp-dl/dl/base/dl_base_conv2d.cpp:9-33) with the n_wise epilogue
 // (esp-dl/dl/base/dl_base_activate_buffer.hpp:27-36, 61-72, 173-181, 201-210).
@@ -44,8 +44,10 @@ struct WideArgs {
     int relu, half_even, n_shift;
 };
 
-// WALKS: a workgroup may have several walks.  (A build of its own: registers are short, and 68 bytes of it lie in scratch, which
-// costs a launch of one walk each 2 us.)
+// WALKS: a workgroup may have several walks, each of which requests its operands itself.  (A build of its own, for with one walk
+// they are on their way while the constants are prepared.  Requested there for the first walk and in the loop for the others they
+// were live across all five epilogues, and 37 registers of KS 2 spilled: 44.1 instead of 42.4 us, with shifts below 8 51.4 instead of
+// 46.1, which was longer than one walk each.)
 template <int KS, bool WALKS>
 __global__ __launch_bounds__(kThreads, 2) void conv2d_s8_wide_kernel(const WideArgs a)
 {
@@ -75,7 +77,8 @@ __global__ __launch_bounds__(kThreads, 2) void conv2d_s8_wide_kernel(const WideA
             for (int k = 0; k < KS; k++)
                 b[c][k] = mask_unit<false>(b[c][k], max(a.K - (64 * k + 16 * quad), 0));
     };
-    pixels(blockIdx.x * 64, col, quad);
+    if constexpr (!WALKS)
+        pixels(blockIdx.x * 64, col, quad);
     // Operand A of step n: rows in lane order, a filter past the last one reads the last one again.  Away from the last
     // filters every piece is whole and the lane's one offset serves all of them.
     const auto fetch = [&](int n, v4i (&p)[4][KS], int col, int quad) {
@@ -98,7 +101,8 @@ __global__ __launch_bounds__(kThreads, 2) void conv2d_s8_wide_kernel(const WideA
         }
     };
     v4i fa[4][KS];
-    fetch(n_begin + 64 * wave, fa, col, quad);
+    if constexpr (!WALKS)
+        fetch(n_begin + 64 * wave, fa, col, quad);
 
     int ok = 1, low = 0; // the short epilogue is exact; some shift is below 8
     for (int i0 = tid; i0 < a.per_walk; i0 += 6 * kThreads) { // six at a time: their loads are in flight together
@@ -124,7 +128,8 @@ __global__ __launch_bounds__(kThreads, 2) void conv2d_s8_wide_kernel(const WideA
             }
         }
     }
-    mask(quad);
+    if constexpr (!WALKS)
+        mask(quad);
     const bool fast = __syncthreads_and(ok) != 0, high = __syncthreads_or(low) == 0;
 
     const int floor_pk = a.relu ? 0 : (int)0x80008000u;
@@ -137,7 +142,7 @@ __global__ __launch_bounds__(kThreads, 2) void conv2d_s8_wide_kernel(const WideA
             if constexpr (WALKS) // (through an empty asm statement: nothing that follows from it is kept from walk to walk)
                 asm volatile("" : "+v"(tid));
             const int col = tid & 15, quad = (tid & 63) >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-            if (WALKS && m0 != 64 * (int)blockIdx.x) {
+            if constexpr (WALKS) {
                 pixels(m0, col, quad);
                 fetch(n_begin + 64 * wave, fa, col, quad);
                 mask(quad);
@@ -250,7 +255,6 @@ __global__ __launch_bounds__(kThreads, 2) void conv2d_s8_wide_kernel(const WideA
                 if (tid < 64) // what the next step's first pieces start with
                     *reinterpret_cast<v4i *>(next + tid * kRow) = *reinterpret_cast<const v4i *>(buf + tid * kRow + 256);
             }
-        
             if constexpr (!WALKS)
                 break;
         }
@@ -322,7 +326,7 @@ hipError_t launch_conv2d_s8_wide(const ConvGeom &g, const int8_t *in, const int8
     if (a.M == 0)
         return hipSuccess;
     // Steps per walk: rounds of workgroups (two fit a compute unit) times a walk and its start, which costs about four
-    // steps; kMaxSteps steps' constants at most lie in LDS.  More rounds than one become walks of the same workgroups.
+    // steps; kMaxSteps steps' constants at most lie in LDS.
     const int tiles = (a.M + 63) / 64, steps = (a.N + 255) / 256;
     const long long slots = 2ll * std::max(1, cu_count);
     int per = 1;
@@ -335,7 +339,14 @@ hipError_t launch_conv2d_s8_wide(const ConvGeom &g, const int8_t *in, const int8
         }
     }
     const long long groups = std::max(1ll, slots / ((steps + per - 1) / per)); // that take the same filters
-    const int walks = (int)((tiles + groups - 1) / groups);
+    // More rounds than one become walks of the same workgroups.  Beyond 64 channels, where a step is matrix work too, only if that leaves
+    // the busiest compute unit no more tiles than it had, and at most 1.3 times an even share of all steps: 250 random layers 0.87 to
+    // 1.06 of the time of a workgroup per walk, 0.95 in the mean; the other 84 up to 1.25.  (Up to 64 channels 59 layers 0.82 to 1.03.)
+    int walks = (int)((tiles + groups - 1) / groups);
+    const long long cus = std::max(1, cu_count), columns = (steps + per - 1) / per;
+    const long long share = ((tiles + walks - 1) / walks * columns + cus - 1) / cus * walks; // walks of the busiest compute unit
+    if (a.K > 64 && (share > (tiles * columns + cus - 1) / cus || 10 * share * per * cus > 13ll * tiles * steps))
+        walks = 1;
     a.per_walk = 256 * per;
     const dim3 grid((unsigned)((tiles + walks - 1) / walks), (unsigned)((steps + per - 1) / per));
     const size_t lds = (size_t)3 * sizeof(int) * a.per_walk;

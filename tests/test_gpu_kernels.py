@@ -734,17 +734,26 @@ def test_conv2d_s8_wide_filters_long_walks(oracle, m, k, n):
     np.testing.assert_array_equal(got, want)
 
 
-# Walks of 10, 11 and 12 steps, whose constants take the kernel past 64 KB of LDS.
-@pytest.mark.parametrize("m,k,n", [(20003, 64, 2305), (20480, 17, 2563), (30000, 80, 2817)])
-def test_conv2d_s8_wide_filters_long_walks(oracle, m, k, n):
-    announce(f"conv2d_s8 wide filters, long walks M={m} K={k} N={n}")
-    rng = np.random.default_rng(0xF6 + n)
+# Several walks to a workgroup (321 tiles of 64 rows under nine steps of filters, the last tile a part of one; test_host_runtime.py looks
+# at the launch): every epilogue, one and two k steps.  The oracle computes a row of every tile, another one in each, and the last tile.
+@pytest.mark.parametrize("variant", ["some_below_8", "none_below_8", "half_even_some_below_8", "half_even_none_below_8", "wide_shifts"])
+@pytest.mark.parametrize("k", [64, 120])
+def test_conv2d_s8_wide_filters_several_walks(oracle, k, variant):
+    announce(f"conv2d_s8 wide filters, several walks K={k} {variant}")
+    m, n = 20493, 6625
+    rng = np.random.default_rng(0xF8 + k)
     x, f = rng_int8(rng, (m, 1, 1, k)), rng_int8(rng, (n, 1, 1, k))
     bias = rng.integers(-4096, 4097, size=n).astype(np.int32)
-    shift = rng.integers(6, 12, size=n).astype(np.int32)
+    lo, hi = (-2, 34) if variant == "wide_shifts" else (7 if "some" in variant else 8, 13)
+    shift, even = rng.integers(lo, hi, size=n).astype(np.int32), "half_even" in variant
+    mod = espdl()
+    got = to_host(mod.conv2d(to_dev(x), to_dev(f), to_dev(bias), to_dev(shift), (1, 1), activation=mod.capi.RELU,
+                             round_mode=mod.capi.ROUND_HALF_EVEN if even else mod.capi.ROUND_HALF_UP))
+    rows = np.array([64 * t + 7 * t % 64 for t in range(m // 64)] + list(range(m // 64 * 64, m)))
     oracle.set_threads(16)
-    got, want = _run_conv_s8(oracle, x, f, bias, shift, (1, 1), (1, 1), (1, 1), (0, 0, 0, 0), True)
-    np.testing.assert_array_equal(got, want)
+    want = oracle.conv2d_s8(x[rows], f, bias, shift, (1, 1), activation=oracle.RELU,
+                            round_mode=oracle.ROUND_HALF_EVEN if even else oracle.ROUND_HALF_UP)
+    np.testing.assert_array_equal(got[rows], want)
 
 
 # Products with so few rows that the tiled kernels would leave most of the device idle go to a kernel with one

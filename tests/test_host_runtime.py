@@ -117,6 +117,27 @@ def test_wide_filter_walks_ask_for_lds_that_the_kernel_may_have():
     """)
 
 
+def test_wide_filters_walk_several_times_where_the_shares_stay_even():
+    """The layers that take longer with several walks to a workgroup keep a workgroup per walk (us: several, one): one compute
+    unit would get more tiles than before, or the last filters leave too many of them idle."""
+    host_hip.run("""
+    for rows, channels, filters, several in [(20480, 120, 6625, True),   # 42.4, 46.6
+                                             (20480, 128, 6625, True),   # 52.6, 55.5
+                                             (20493, 120, 6625, True), (20493, 64, 6625, True), (33000, 64, 4509, True),
+                                             (11520, 72, 6625, False),   # 34.7, 31.7
+                                             (17602, 91, 3327, False),   # 43.5, 40.5
+                                             (10944, 125, 6909, False),  # 86.1, 79.5
+                                             (1024, 48, 6625, False)]:   # one round
+        desc = m.capi.make_desc((rows, 1, 1, channels), filters, (1, 1))
+        hip.host_hip_clear()
+        rc = m.lib().espdl_hip_conv2d(ctypes.byref(desc), 1 << 20, 1 << 30, None, 1 << 31, None, 1 << 32, None)
+        log = launches()
+        build = "conv2d_s8_wide_kernelILi%dELb%dE" % (1 if channels <= 64 else 2, several)
+        assert rc == 0 and len(log) == 1 and build in log[0]["name"], (rows, channels, log)
+        assert (log[0]["grid"][0] < (rows + 63) // 64) == several, (rows, channels, log)
+    """)
+
+
 def test_depthwise_strips_are_found_quickly():
     """The strip count of the depthwise row walks is the cheapest of all (the plain search below), and finding it does not
     take longer than the launch: a layer of a million rows."""
