@@ -192,9 +192,8 @@ __global__ __launch_bounds__(kThreads) void max_pool_s8_window_kernel(const Wind
 }
 
 // Strips of one row, which is what few outputs are cut into: all rows of the window are requested at once, where the walk waits
-// for one after the other.  One wavefront to a workgroup while that leaves none to share a compute unit, for the loads of its
-// wavefronts take turns (30 of 16 bytes each); beyond that wavefronts side by side, whose windows overlap, stay in one workgroup.  5 x 5, launch to launch in a graph: 13 x 13 x 128, one image, 3.2 -> 2.9 us, 30 x 30 x 198 4.8 -> 2.9, 17 x 14 x 61, three
-// images, 5.4 -> 3.0, 20 x 20 x 128, 64 images, 4.8 -> 4.4; images of one row, 512 of 40 x 480, 9.5 -> 8.9; 3 x 3 and 2 x 2 as much.
+// for one after the other.  5 x 5, launch to launch in a graph: 13 x 13 x 128, one image, 3.2 -> 2.9 us, 30 x 30 x 198 4.8 -> 2.9, 17 x 14 x 61,
+// three images, 5.4 -> 3.0, 20 x 20 x 128, 64 images, 4.8 -> 4.4; images of one row, 512 of 40 x 480, 9.5 -> 8.9; 3 x 3 and 2 x 2 as much.
 template <int K, int D>
 __global__ __launch_bounds__(kThreads) void max_pool_s8_window_row_kernel(const WindowPoolArgs a)
 {
@@ -243,10 +242,14 @@ __global__ __launch_bounds__(kThreads) void max_pool_s8_window_row_kernel(const 
 }
 
 template <int K, int D>
-hipError_t launch_window(const WindowPoolArgs &a, bool whole, hipStream_t stream)
+hipError_t launch_window(const WindowPoolArgs &a, bool whole, int cus, hipStream_t stream)
 {
     const dim3 grid((a.total + kThreads - 1) / kThreads);
-    if (a.rows == 1 && grid.x <= 256)
+    // One wavefront to a workgroup up to two of them per compute unit, for the loads of a compute unit's wavefronts take turns (30 of
+    // 16 bytes each); beyond that wavefronts side by side, whose windows overlap, stay in one workgroup and on one XCD.  Of 1200 pools
+    // on the row kernel single wavefronts take 0.51 to 1.06 of the time of four to a workgroup up to 64 workgroups of four, 0.72 to 1.18
+    // up to 128, from there 0.87 to 1.34 (12 images of 96 x 54 x 32, 3 x 3: 4.67 and 3.6 us, the walk 3.7).
+    if (a.rows == 1 && 2 * (long long)grid.x <= cus)
         hipLaunchKernelGGL((max_pool_s8_window_row_kernel<K, D>), dim3(grid.x * (kThreads / 64)), dim3(64), 0, stream, a);
     else if (a.rows == 1)
         hipLaunchKernelGGL((max_pool_s8_window_row_kernel<K, D>), grid, dim3(kThreads), 0, stream, a);
@@ -298,7 +301,8 @@ hipError_t launch_max_pool_s8_window(const void *in, int batch, int h, int w, in
     // wavefronts, and the count decides how evenly the last round of wavefronts fills the chip, counted at four
     // wavefronts per SIMD.
     const long long per_row = (long long)batch * a.xpairs * a.cv;
-    const double capacity = (double)(cu_count > 0 ? cu_count : 256) * 4 * 4;
+    const int cus = cu_count > 0 ? cu_count : 256;
+    const double capacity = (double)cus * 4 * 4;
     int best_strips = 1;
     double best_score = -1.0;
     for (int strips = 1;;) { // of the counts with one strip height only the smallest: 2 sqrt(out_h) of them
@@ -331,11 +335,11 @@ hipError_t launch_max_pool_s8_window(const void *in, int batch, int h, int w, in
         (k != 2 || (long long)batch * h * w * c <= (3 << 20));
     switch (k) {
     case 2:
-        return dwords == 4 ? launch_window<2, 4>(a, whole, stream) : launch_window<2, 2>(a, whole, stream);
+        return dwords == 4 ? launch_window<2, 4>(a, whole, cus, stream) : launch_window<2, 2>(a, whole, cus, stream);
     case 3:
-        return dwords == 4 ? launch_window<3, 4>(a, whole, stream) : launch_window<3, 2>(a, whole, stream);
+        return dwords == 4 ? launch_window<3, 4>(a, whole, cus, stream) : launch_window<3, 2>(a, whole, cus, stream);
     default:
-        return dwords == 4 ? launch_window<5, 4>(a, whole, stream) : launch_window<5, 2>(a, whole, stream);
+        return dwords == 4 ? launch_window<5, 4>(a, whole, cus, stream) : launch_window<5, 2>(a, whole, cus, stream);
     }
 }
 

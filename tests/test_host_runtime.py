@@ -204,6 +204,23 @@ def test_pool_strips_are_found_quickly():
     ''')
 
 
+def test_pools_of_one_row_keep_neighbouring_wavefronts_together():
+    """Strips of one row: single wavefronts only while the device has two of them per compute unit (us with single wavefronts
+    and with four to a workgroup)."""
+    host_hip.run('''
+    for n, h, w, c, k, threads in [(1, 13, 13, 128, 5, 64),   # 2.9, 3.2
+                                   (1, 30, 30, 198, 5, 64),
+                                   (12, 96, 54, 32, 3, 256),  # 4.67, 3.6
+                                   (7, 72, 24, 128, 3, 256),  # 4.40, 3.5
+                                   (87, 12, 18, 80, 3, 256)]:
+        hip.host_hip_clear()
+        rc = m.lib().espdl_hip_max_pool_pitched(1 << 20, 8, n, h, w, c, k, k, 1, 1, k // 2, (k - 1) // 2, k // 2, (k - 1) // 2, 0, 0, 1 << 42, None)
+        log = launches()
+        assert rc == 0 and len(log) == 1 and "max_pool_s8_window_row" in log[0]["name"], (rc, log)
+        assert log[0]["block"][0] == threads and log[0]["grid"][0] * threads <= (32768 if threads == 64 else 1 << 30), (n, h, w, c, k, log)
+    ''')
+
+
 def test_narrow_kernels_stay_inside_the_grid_limit():
     """A launch has fewer than 2^32 threads along x: layers with more pixels than that go to the kernel with larger tiles."""
     host_hip.run('''
