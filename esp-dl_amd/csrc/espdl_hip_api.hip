@@ -1469,13 +1469,16 @@ int64_t espdl_hip_mbconv_s8_workspace(const espdl_hip_mbconv_desc *desc)
     (void)project_launch(g, aligned, aligned, cus, &project);
     const int64_t between = (int64_t)p.batch * p.out_h * p.out_w * p.exp_c;
     // no single launch at all (a Clip between the stages in half-even mode), or none that the convolutions would be left for
-    if (espdl_hip_mbconv_s8_supported(desc) == 0 || espdl_hip_mbconv_s8_preferred(desc) != 1)
+    const int kind = espdl_hip_mbconv_s8_supported(desc);
+    if (kind == 0 || espdl_hip_mbconv_s8_preferred(desc) != 1)
         return between;
-    const float one = std::min(mbconv_tile_us(p, espdl_hip_mbconv_s8_supported(desc), cus), espdl::mbconv_s8_walk_us(p, cus));
-    // 0.3 us a megabyte for the tensor between the launches, which one of them writes and the other reads back, and which the projection's
-    // estimate leaves out.  Of 2368 blocks on 2 to 256 images, with and without Clips, in both rounding modes, the choice takes 0.6 % more
-    // time than the better one of the two in the mean, 4 % of them 5 % more and over.
-    return espdl::mbconv_s8_expand_dw_us(p) + project + 0.3e-6f * (float)between < one ? between : 0;
+    const float one = mbconv_walks(p, kind) ? espdl::mbconv_s8_walk_us(p, cus)
+        : kind == 5                         ? espdl::mbconv_s8_group_us(p, cus)
+                                            : espdl::mbconv_s8_wave_launch_us(p);
+    // 0.2 us a megabyte for the tensor between the launches, which one of them writes and the other reads back, and which the projection's
+    // estimate leaves out.  Of 12700 blocks on 1 to 300 images, with and without Clips, in both rounding modes, the choice takes 0.3 % more
+    // time than the better one of the two in the mean, 2 % of them 5 % more and over.
+    return espdl::mbconv_s8_expand_dw_us(p) + project + 0.2e-6f * (float)between < one ? between : 0;
 }
 
 int espdl_hip_mbconv_s8_ws(const espdl_hip_mbconv_desc *desc, const int8_t *in, const espdl_hip_mbconv_weights *w,

@@ -221,6 +221,7 @@ bool mbconv_s8_wave_supports(const MbconvParams &p);
 // The guarded builds cover every supported shape but do not beat the separate launches.
 bool mbconv_s8_wave_has_fast_build(const MbconvParams &p);
 float mbconv_s8_wave_us(const MbconvParams &p); // expected time of a guard-free build
+float mbconv_s8_wave_launch_us(const MbconvParams &p); // the same by the workgroups that a compute unit holds
 float mbconv_s8_wave_rounds(const MbconvParams &p); // tiles per wavefront that the device holds
 hipError_t launch_mbconv_s8_wave(const MbconvParams &p, int cu_count, hipStream_t stream);
 

@@ -1076,6 +1076,22 @@ float mbconv_s8_wave_us(const MbconvParams &p)
     return chain * (fill <= 1.f ? 1.f + 0.45f * fill : 1.45f * fill);
 }
 
+// The same by what a compute unit holds, for the choice between one and two launches: a wavefront's chain, and for every second and
+// every third workgroup of a compute unit as much again as that adds.  8400 launches of guard-free builds on 1 to 300 images within
+// 5 % (the line above, against which the walk's margins are set, 13 %: flat up to half a round, where it rises, and a step there,
+// where it goes on).  The low tiles at stride 2 have the line above alone.
+float mbconv_s8_wave_launch_us(const MbconvParams &p)
+{
+    const bool s1 = p.stride_h == 1;
+    if (!s1 && p.in_c == 16)
+        return mbconv_s8_wave_us(p);
+    const bool vec = p.in_c % 16 == 0;
+    const float per_sub = (vec ? (s1 ? 1.09f : 0.85f) : (s1 ? 1.24f : 1.26f)) * (p.half_even ? 1.2f : 1.f);
+    const float chain = 5.35f + (p.half_even ? 0.25f : 0.f) + per_sub * (float)(p.exp_c / 16);
+    const int more = std::max(1, (int)std::ceil(2.f * mbconv_s8_wave_rounds(p))) - 1; // workgroups of a compute unit beyond the first
+    return chain * (1.02f + (s1 ? 1.15f : 1.f) * (float)(more / 2) + (s1 ? 0.42f : 0.4f) * (float)(more % 2));
+}
+
 bool mbconv_s8_wave_has_fast_build(const MbconvParams &p)
 {
     const WavePlan plan = wave_plan(p);
