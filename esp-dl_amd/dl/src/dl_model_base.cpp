@@ -1332,75 +1332,97 @@ esp_err_t Model::build(int batch)
             n *= (size_t)d;
         return n;
     };
-    std::vector<size_t> offset(n_var, 0);
-    std::vector<bool> placed(n_var, false);
-    ArenaPlanner arena;
     std::set<int> graph_io;
     for (const std::string &name : m_fbs_model->get_graph_inputs())
         graph_io.insert(ctx->get_variable_index(name));
-    for (int idx : graph_io) {
-        offset[idx] = arena.alloc(bytes_of(vars[idx]));
-        placed[idx] = true;
-    }
-    auto release_dead = [&](int step) {
-        for (int v = 1; v < n_var; v++)
-            if (placed[v] && vars[v].alias_of < 0 && vars[v].last == step && !graph_io.count(v)) {
-                // views that share the block die no later than their source (made sure above)
-                arena.release(offset[v], bytes_of(vars[v]));
-                placed[v] = false;
-                vars[v].last = -2;
-            }
-    };
-    auto place_outputs = [&](int i) {
-        dl::module::Module *m = m_execution_plan[i];
-        for (size_t j = 0; j < m->m_outputs_index.size(); j++) {
-            const int idx = m->m_outputs_index[j];
-            VarInfo &v = vars[idx];
-            if (v.alias_of >= 0) {
-                offset[idx] = offset[v.alias_of];
-                continue;
-            }
-            if (placed[idx])
-                continue; // the output of a Concat that an earlier producer already writes into, or of a module that runs early
-            if (v.slice_of >= 0) {
-                // lives inside the wider tensor, which is placed when its first slice is written
-                const int w = v.slice_of;
-                if (!placed[w]) {
-                    offset[w] = arena.alloc(bytes_of(vars[w]));
-                    placed[w] = true;
-                }
-                continue;
-            }
-            // an in-place module may overwrite its first input when nobody reads that input later
-            const int in0 = m->m_inputs_index.empty() ? -1 : m->m_inputs_index[0];
-            if (m->inplace == MODULE_INPLACE_CHANGED_BUFFER && j == 0 && in0 > 0 && in0 < CONTEXT_PARAMETER_OFFSET &&
-                placed[in0] && vars[in0].alias_of < 0 && vars[in0].last == i && !graph_io.count(in0) &&
-                bytes_of(vars[in0]) == bytes_of(v)) {
-                bool aliased_elsewhere = false;
-                for (int k = 1; k < n_var; k++)
-                    if (vars[k].alias_of == in0 || vars[k].slice_of == in0)
-                        aliased_elsewhere = true;
-                if (!aliased_elsewhere) {
-                    offset[idx] = offset[in0];
-                    placed[idx] = true;
-                    placed[in0] = false;
-                    vars[in0].last = -2;
-                    continue;
-                }
-            }
-            offset[idx] = arena.alloc(bytes_of(v));
+    // `early`: modules that run with module i, in front of their own place
+    auto place = [&](const std::vector<std::vector<int>> &early, std::vector<size_t> &offset) {
+        offset.assign(n_var, 0);
+        std::vector<bool> placed(n_var, false);
+        std::vector<int> last(n_var);
+        for (int v = 0; v < n_var; v++)
+            last[v] = vars[v].last;
+        ArenaPlanner arena;
+        for (int idx : graph_io) {
+            offset[idx] = arena.alloc(bytes_of(vars[idx]));
             placed[idx] = true;
         }
+        auto release_dead = [&](int step) {
+            for (int v = 1; v < n_var; v++)
+                if (placed[v] && vars[v].alias_of < 0 && last[v] == step && !graph_io.count(v)) {
+                    // views that share the block die no later than their source (made sure above)
+                    arena.release(offset[v], bytes_of(vars[v]));
+                    placed[v] = false;
+                    last[v] = -2;
+                }
+        };
+        auto place_outputs = [&](int i) {
+            dl::module::Module *m = m_execution_plan[i];
+            for (size_t j = 0; j < m->m_outputs_index.size(); j++) {
+                const int idx = m->m_outputs_index[j];
+                VarInfo &v = vars[idx];
+                if (v.alias_of >= 0) {
+                    offset[idx] = offset[v.alias_of];
+                    continue;
+                }
+                if (placed[idx])
+                    continue; // the output of a Concat that an earlier producer already writes into, or of a module that runs early
+                if (v.slice_of >= 0) {
+                    // lives inside the wider tensor, which is placed when its first slice is written
+                    const int w = v.slice_of;
+                    if (!placed[w]) {
+                        offset[w] = arena.alloc(bytes_of(vars[w]));
+                        placed[w] = true;
+                    }
+                    continue;
+                }
+                // an in-place module may overwrite its first input when nobody reads that input later
+                const int in0 = m->m_inputs_index.empty() ? -1 : m->m_inputs_index[0];
+                if (m->inplace == MODULE_INPLACE_CHANGED_BUFFER && j == 0 && in0 > 0 && in0 < CONTEXT_PARAMETER_OFFSET &&
+                    placed[in0] && vars[in0].alias_of < 0 && last[in0] == i && !graph_io.count(in0) &&
+                    bytes_of(vars[in0]) == bytes_of(v)) {
+                    bool aliased_elsewhere = false;
+                    for (int k = 1; k < n_var; k++)
+                        if (vars[k].alias_of == in0 || vars[k].slice_of == in0)
+                            aliased_elsewhere = true;
+                    if (!aliased_elsewhere) {
+                        offset[idx] = offset[in0];
+                        placed[idx] = true;
+                        placed[in0] = false;
+                        last[in0] = -2;
+                        continue;
+                    }
+                }
+                offset[idx] = arena.alloc(bytes_of(v));
+                placed[idx] = true;
+            }
+        };
+        for (int i = 0; i < plan_size; i++) {
+            place_outputs(i);
+            for (int j : early[i])
+                place_outputs(j);
+            release_dead(i);
+        }
+        return arena.top();
     };
-    for (int i = 0; i < plan_size; i++) {
-        place_outputs(i);
-        for (int j : with[i])
-            place_outputs(j);
-        release_dead(i);
+    std::vector<size_t> offset;
+    size_t arena_bytes = place(with, offset);
+    if ((int)m_schedule.size() != plan_size) {
+        // What runs early keeps its output from then on: small tensors, but any number of them.  Up to a sixteenth of the arena for it
+        // and 4 MB (a detector at 96 to 640 pixels square needs nothing, a block of gated branches half a percent), else the plan's order.
+        std::vector<size_t> in_order;
+        const size_t bytes = place(std::vector<std::vector<int>>(plan_size), in_order);
+        if (arena_bytes > bytes + bytes / 16 + (4 << 20)) {
+            arena_bytes = bytes;
+            offset = in_order;
+            m_schedule.clear();
+            for (int i = 0; i < plan_size; i++)
+                m_schedule.push_back({i});
+        }
     }
 
     // 3. materialize
-    if (!ctx->root_alloc(arena.top()))
+    if (!ctx->root_alloc(arena_bytes))
         return ESP_FAIL;
     char *root = static_cast<char *>(ctx->get_device_root());
     for (int i = 1; i < n_var; i++) {

@@ -232,6 +232,43 @@ def test_convolutions_that_share_a_launch(oracle, resolution, batch):
     mdl.close()
 
 
+def shared_launch_graph(kind, side=3):
+    """Two convolutions of one tensor, of which the later one runs with the first: with an in-place operator on the first one's
+    result in between; the later one between channel slices (it reads a Split's piece and writes into a Concat that comes
+    later); with a residual operand; read by nobody.  "side": a chain of small layers and `side` layers behind it, each read at
+    once, that could all run with the chain."""
+    _, zoo, _, _ = _mods()
+    g = zoo.GraphSpec("shared_launch_" + kind)
+    b = zoo.Builder(g, 0xE5F8, per_channel=True, w_exp_range=None)
+    x = b.input("input", [1, 20, 20, 64], -5)
+    t = b.conv(x, 64, k=3, relu=True, out_exp=-4, name="trunk")
+    if kind == "in_place":
+        p = b.prelu(b.conv(t, 48, k=3, out_exp=-4, name="first"), name="in_between")
+        c = b.conv(t, 48, k=3, out_exp=-4, name="early")
+        b.output(b.mul(p, c, out_exp=-2, name="behind"))
+    elif kind == "slices":
+        u, v = b.split(t, [32, 32], name="pieces")
+        m = b.max_pool(b.conv(u, 32, k=3, out_exp=-4, name="first"), 3, name="in_between")
+        c = b.conv(v, 32, k=3, out_exp=-4, name="early")
+        b.output(b.conv(b.concat([m, c], name="behind"), 16, k=1, name="last"))
+    elif kind == "residual":
+        m = b.max_pool(b.conv(t, 64, k=3, out_exp=-4, name="first"), 3, name="in_between")
+        b.output(m)
+        b.output(b.add(t, b.conv(t, 64, k=3, out_exp=-4, name="early"), name="behind"))
+    elif kind == "unread":
+        r = b.max_pool(b.conv(t, 32, k=3, name="first"), 3, name="in_between")
+        b.conv(t, 32, k=3, name="early")
+        b.output(b.conv(r, 32, k=3, name="last"))
+    else:
+        h = t
+        for i in range((side + 2) // 3 + 1):
+            h = b.conv(h, 64, k=3, out_exp=-4, name="chain%d" % i)
+        b.output(h)
+        for i in range(side):
+            b.output(b.global_avg_pool(b.conv(t, 64, k=3, out_exp=-4, name="side%d" % i), name="read%d" % i))
+    return g
+
+
 @pytest.mark.parametrize("round_mode", [0, 1], ids=["half_up", "half_even"])
 @pytest.mark.parametrize("rows,k,n,m", [(40, 120, 480, 120), (9, 33, 17, 5), (1, 16, 2100, 64)])
 def test_lut_behind_gemm_and_matmul(oracle, rows, k, n, m, round_mode):

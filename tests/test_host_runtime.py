@@ -346,3 +346,27 @@ def test_two_launch_cases_take_the_tile_of_their_name():
         taken.add((build[0], build[1], build[2], build[6]))
     assert len(taken) == 12, taken  # nine tiles, three of them with the loop too
     ''')
+
+
+def test_layers_run_early_only_while_the_arena_stays_small():
+    """A layer that runs in front of its place keeps its output until there: up to a sixteenth of the arena and 4 MB."""
+    host_hip.run('''
+    import test_gpu_model
+    output = 4 * 20 * 20 * 64  # of a side layer
+
+    def plan(side):
+        spec = test_gpu_model.shared_launch_graph("side", side)
+        mdl = model.Model(model.Graph.from_spec(spec), 4)
+        parameters = sum(data.nbytes for _, _, data, _ in spec.initializers.values())
+        hip.host_hip_clear()
+        mdl.run()
+        shared = any("narrow_group" in l["name"] for l in launches())
+        arena = mdl.device_bytes() - parameters
+        mdl.close()
+        return shared, arena
+
+    shared, few = plan(30)
+    assert shared and few > 20 * output
+    shared, many = plan(90)
+    assert not shared and many < 20 * output, many
+    ''')
