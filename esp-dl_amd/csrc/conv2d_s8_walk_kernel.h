@@ -653,9 +653,9 @@ __global__ __launch_bounds__((64 * WalkShape<KH, S, CU, NT, RES>::W), 2) void co
 }
 
 // Whether a build exists: filters and accumulators fit 256 registers with what else a wavefront holds, and its LDS leaves
-// a compute unit two wavefronts per SIMD.  With a residual operand 204 fit for four units and four filter tiles (80 x 80 x 64 -> 64,
-// 3 x 3, batch 64, input and results slices of wider tensors: 38.1 us as two chunks of 32 filters, 29.8 as one); 15 and 16 units spill
-// 49 registers at that.
+// a compute unit two wavefronts per SIMD.  With a residual operand 204 fit beside four filter tiles (3 and 4 units; 80 x 80 x 64 -> 64,
+// 3 x 3, batch 64, input and results slices of wider tensors: 38.1 us as two chunks of 32 filters, 29.8 as one); beside one tile,
+// 15 and 16 units spill 49 registers at that: a row of the input then takes several more loads, each with an address.
 template <int KH, int S, int CU, int NT, bool RES, bool RAW>
 constexpr bool walk_fits()
 {
@@ -663,7 +663,7 @@ constexpr bool walk_fits()
     if (RAW && 4 * (KH * Shape::KS * NT + Shape::kAcc * NT * Shape::PT + S * Shape::PT * Shape::KS + Shape::kHeld * S * Shape::kRowLoads) > 204)
         return false;
     return (NT != 8 || KH == 1) && (!RES || (S == 1 && KH <= 3)) &&
-        4 * (KH * Shape::KS * NT + Shape::kAcc * NT * Shape::PT + S * Shape::PT * Shape::KS) <= (RES ? (CU == 4 ? 204 : 200) : 208) &&
+        4 * (KH * Shape::KS * NT + Shape::kAcc * NT * Shape::PT + S * Shape::PT * Shape::KS) <= (RES ? (NT == 4 ? 204 : 200) : 208) &&
         (Shape::kTwo || Shape::W == 8 || (S == 2 && Shape::lds(4, 1) <= Shape::kCu));
 }
 
@@ -713,7 +713,11 @@ WalkCut walk_cut(const WalkArgs &a, const WalkLaunch &l, int per_cu)
 // RAW builds under 3 x 3 pass their pieces through registers step by step, which takes a fifth longer; those of 11 and 12 units of
 // a pixel and the ones of 15 and 16 without RAW spill 24 to 35 registers besides (1600 and 60 layers).  At stride 2 the builds of 6
 // units and more, 5 under 5 x 5, take more than 256 registers: one wavefront per SIMD, 1.4 and 2.3 us more whatever the layer's size
-// (52 layers of 5 to 82 us; 3 x 3 counts 1, for the unit kernel's line lies as far below its time at 128 channels).
+// (52 layers of 5 to 82 us; 3 x 3 counts 1, for the unit kernel's line lies as far below its time at 128 channels).  Four filter tiles
+// beside a residual operand on 3 and 4 units, the builds that take all registers: of two chunks of 32 filters and one of 64 the smaller
+// expected time is more often the one that is too small.  With 4 % and 0.6 us in favour of the two, 1 of 3500 layers of 33 to 64 channels
+// is slower by more than 5 % than without the build, at 0.967 of that time in the mean (111 layers and 0.963 without the margin:
+// 40 x 40 x 64 -> 128, batch 58, 14.2 us as two chunks and 17.4 as one).
 template <int KH, int S, int CU, int NT, bool RES, bool RAW>
 float walk_us(const WalkArgs &a, const WalkLaunch &l)
 {
@@ -738,6 +742,8 @@ float walk_us(const WalkArgs &a, const WalkLaunch &l)
         return KH == 1 ? us + 0.1f : us * (CU <= 3 ? 1.15f : (CU <= 10 ? 1.2f : 1.5f)) + 0.3f;
     if (S == 2 && ((KH == 3 && CU >= 6) || (KH == 5 && CU >= 5)))
         us += KH == 3 ? 1.f : 2.3f;
+    if (RES && kRegs > 244)
+        us = 1.04f * us + 0.6f;
     return KH == 3 && S == 1 && CU >= 15 ? 1.5f * us : us;
 }
 

@@ -321,12 +321,14 @@ def test_conv2d_s8_walk_residual(oracle, case, flavour):
     np.testing.assert_array_equal(got, want)
 
 
+# (their tiles: test_host_runtime.py)
 @pytest.mark.parametrize("flavour", ["residual", "lut_residual", "slices"])
-@pytest.mark.parametrize("case", [(64, ("64_64", (41, 37, 64), 64, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
-                                  (50, ("52_128_tailpad", (37, 45, 52), 128, (3, 3), (1, 1), (1, 1), (0, 1, 0, 1), True, True))],
+@pytest.mark.parametrize("case", [(244, ("64_64", (41, 37, 64), 64, (3, 3), (1, 1), (1, 1), (1, 1, 1, 1), True, True)),
+                                  (130, ("52_128_tailpad", (37, 45, 52), 128, (3, 3), (1, 1), (1, 1), (0, 1, 0, 1), True, True)),
+                                  (256, ("44_64_wide_pad", (39, 43, 44), 64, (3, 3), (1, 1), (1, 1), (2, 0, 2, 1), True, True))],
                          ids=lambda c: c[1][0])
 def test_conv2d_s8_walk_residual_four_units(oracle, case, flavour):
-    """Four units of input channels under four filter tiles with a residual operand: all of a wavefront's registers."""
+    """Three and four units of input channels under four filter tiles with a residual operand: all of a wavefront's registers."""
     announce(f"conv2d_s8 walk with a residual operand, four units {case[1][0]} {flavour}")
     x, f, bias, shift, k, stride, dil, pads, relu = _conv_inputs(case[1], 281, case[0], True)
     oracle.set_threads(16)

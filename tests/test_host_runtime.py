@@ -370,3 +370,21 @@ def test_layers_run_early_only_while_the_arena_stays_small():
     shared, many = plan(90)
     assert not shared and many < 20 * output, many
     ''')
+
+
+def test_residual_walks_take_four_filter_tiles_only_where_they_gain():
+    """Filter tiles of the walking kernel's build for 3 x 3 layers with a residual operand (in microseconds: two tiles, four)."""
+    host_hip.run('''
+    for shape, oc, tiles in [((58, 40, 40, 64), 128, 2),   # 14.2, 17.4
+                             ((110, 40, 40, 40), 64, 2),   # 13.5, 16.3
+                             ((64, 80, 80, 64), 64, 4),    # 38, 30
+                             ((216, 104, 104, 48), 64, 4),
+                             ((244, 41, 37, 64), 64, 4), ((130, 37, 45, 52), 128, 4), ((256, 39, 43, 44), 64, 4)]:
+        pads = {45: (0, 1, 0, 1), 43: (2, 0, 2, 1)}.get(shape[2], (1, 1, 1, 1))
+        desc = m.capi.make_desc(shape, oc, (3, 3), pads=pads, n_shift=oc)
+        hip.host_hip_clear()
+        rc = m.lib().espdl_hip_conv2d_add(ctypes.byref(desc), 1 << 36, 1 << 37, None, 1 << 38, None, 1 << 39, 1 << 40, None)
+        names = [l["name"] for l in launches()]
+        assert rc == 0 and len(names) == 1, (shape, names)
+        assert "conv2d_s8_walk_kernelILi3ELi1ELi%dELi%dELb1E" % ((shape[3] + 15) // 16, tiles) in names[0], (shape, names)
+    ''')
