@@ -160,13 +160,15 @@ DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *
         return units && narrow < 5.2f ? DENSE_NARROW : DENSE_STEM;
     const bool flat = g.k_h == 1 && g.k_w == 1 && g.stride_h == 1 && g.stride_w == 1 && g.pad_top == 0 &&
         g.pad_left == 0 && g.out_h == g.in_h && g.out_w == g.in_w;
-    // (the tiled GEMM's line leaves out what channels that are no multiple of 4 cost it: 120 layers near the two lines took 1.06 to 1.16
-    // times the narrow kernel's time there)
-    const float uneven = ((g.in_c | g.in_pitch) & 3) != 0 ? 1.15f : 0.f;
-    const DenseRoute few = narrow < std::max(1.f, uneven) * gemm ? DENSE_NARROW : DENSE_UNITGEMM;
+    // The GEMMs' lines leave out part of what channels that are no multiple of 4 cost them.  Over 5500 random layers of those on both
+    // kernels the better line is slower than the better kernel by 0.57 % in the geometric mean, by 0.52 % with 1.1 under 1 x 1, and by
+    // 1.15 % with 1.15 under any window: there the narrow kernel's line leaves out as much (14 x 14 x 87 -> 444, 5 x 5 at stride 2,
+    // batch 19: 41 us against 20).
+    const bool uneven = ((g.in_c | g.in_pitch) & 3) != 0;
+    const DenseRoute few = narrow < (uneven && g.k_h * g.k_w == 1 ? 1.1f : 1.f) * gemm ? DENSE_NARROW : DENSE_UNITGEMM;
     if (flat) {
         if (espdl::conv2d_s8_pwgemm_supports(g, in, filter, cus))
-            return units && narrow < std::max(0.97f, uneven) * gemm ? DENSE_NARROW : DENSE_PWGEMM;
+            return units && narrow < (uneven ? 1.15f : 0.97f) * gemm ? DENSE_NARROW : DENSE_PWGEMM;
         return units && tile_steps <= 3500 ? few : DENSE_DIRECT;
     }
     if (!espdl::conv2d_s8_units_aligned(g, in, filter))

@@ -388,3 +388,21 @@ def test_residual_walks_take_four_filter_tiles_only_where_they_gain():
         assert rc == 0 and len(names) == 1, (shape, names)
         assert "conv2d_s8_walk_kernelILi3ELi1ELi%dELi%dELb1E" % ((shape[3] + 15) // 16, tiles) in names[0], (shape, names)
     ''')
+
+
+def test_windows_over_channels_that_are_no_multiple_of_four_go_to_the_faster_kernel():
+    """The kernel of a few pixels against the tiled GEMM (their microseconds beside the layer)."""
+    host_hip.run('''
+    L = m.lib()
+    L.espdl_hip_conv2d_s8_kernel.restype = ctypes.c_char_p
+    at = ctypes.c_void_p(256)
+    for shape, oc, k, stride, residual, kernel in [((19, 14, 14, 87), 444, 5, 2, None, b"unitgemm"),   # 41, 20
+                                                   ((16, 20, 20, 258), 64, 3, 1, None, b"unitgemm"),   # 32, 21
+                                                   ((4, 40, 40, 94), 64, 5, 1, at, b"unitgemm"),       # 29, 21
+                                                   ((10, 26, 26, 33), 64, 3, 1, at, b"unitgemm"),      # 8.9, 6.8
+                                                   ((7, 52, 52, 221), 35, 1, 2, at, b"narrow"),        # 6.2, 6.5
+                                                   ((1, 13, 13, 33), 64, 3, 1, None, b"narrow")]:
+        desc = m.capi.make_desc(shape, oc, (k, k), (stride, stride), pads=(k // 2,) * 4, n_shift=oc)
+        name = L.espdl_hip_conv2d_s8_kernel(ctypes.byref(desc), at, at, None, residual, at)
+        assert name == b"conv2d_s8_" + kernel, (shape, name)
+    ''')
