@@ -967,6 +967,16 @@ GROUPED = {
     "int16 layers on int8 inputs": [((1, 20, 20, 64), 64, 3, 1, 1, "x8", False, False), ((1, 10, 9, 64), 64, 3, 1, 1, "x8", True, False),
                                     ((1, 5, 5, 64), 20, 3, 1, 1, "x8", True, False), ((1, 9, 9, 64), 64, 3, 1, 1, "s8", False, False)],
     "one alone": [((1, 10, 10, 64), 64, 1, 1, 0, "s16", False, False)],
+    "two each of two builds": [((1, 6, 11, 16), 17, 2, 1, 1, "s8", False, True), ((1, 5, 3, 512), 20, 1, 1, 0, "s8", True, False),
+                               ((2, 5, 7, 16), 30, 2, 1, 1, "s8", True, False), ((1, 4, 5, 512), 33, 1, 1, 0, "s8", False, True)],
+}
+
+# Which layers of a group share a launch: those of one number.  A layer of 0 leaves at once: 20 channels are no whole units, and the
+# 28 x 28 images go to the walk.
+GROUPED_KINDS = {
+    "one level of three heads": [3, 3, 3], "every build": [3, 4, 2, 1], "edges of tiles": [2, 2, 2, 2],
+    "with layers that leave at once": [0, 3, 0, 3], "int16 layers": [5, 5, 5, 5], "int16 layers on int8 inputs": [6, 6, 6, 3],
+    "one alone": [5], "two each of two builds": [1, 4, 1, 4],
 }
 
 
@@ -979,10 +989,13 @@ def test_grouped_convolutions(oracle, group, half_even):
     rm_o = oracle.ROUND_HALF_EVEN if half_even else oracle.ROUND_HALF_UP
     rm = m.capi.ROUND_HALF_EVEN if half_even else m.capi.ROUND_HALF_UP
     rng = np.random.default_rng(0x6B0)
-    calls, want = [], []
+    calls, want, kinds = [], [], []
     for shape, oc, k, stride, pad, kind, has_table, has_res in GROUPED[group]:
         geometry = ((k, k), (stride, stride), (1, 1), (pad,) * 4)
         relu, act = m.capi.RELU, oracle.RELU
+        desc = m.capi.make_desc(shape, oc, *geometry, 1, relu, rm, oc, m.capi.S8 if kind == "s8" else m.capi.S16)
+        kinds.append(L.espdl_hip_conv2d_group_kind(ctypes.byref(desc), kind == "s8" and has_table, has_res, kind == "x8",
+                                                   257 if has_table and kind == "x8" else 0))
         if kind == "s8":
             x = rng_int8(rng, shape)
             f = rng_int8(rng, (oc, k, k, shape[3]))
@@ -1010,11 +1023,14 @@ def test_grouped_convolutions(oracle, group, half_even):
             if kind == "x8":
                 tab = None if table is None else to_dev(table)
                 calls.append(lambda a=args, tab=tab: m.capi.conv2d_s16_x8(*a, activation=relu, round_mode=rm, table=tab))
-                w = to_host(calls[-1]()) if has_table else oracle.conv2d_s16((x.astype(np.int16) * 256), f, bias, shift, *geometry, act, rm_o)
+                w = oracle.conv2d_s16(x.astype(np.int16) * 256, f, bias, shift, *geometry, act, rm_o)
+                w = w if table is None else oracle.lut_s16(w, table, p4_ties=half_even)
             else:
                 calls.append(lambda a=args: m.conv2d(*a, activation=relu, round_mode=rm))
                 w = oracle.conv2d_s16(x, f, bias, shift, *geometry, act, rm_o)
         want.append(w)
+    if not (group == "with layers that leave at once" and half_even):  # the walk over 28 x 28 images has no half-even build
+        assert kinds == GROUPED_KINDS[group]
     assert L.espdl_hip_conv2d_group_begin() == 0
     got = [call() for call in calls]
     assert L.espdl_hip_conv2d_group_begin() != 0  # groups do not nest

@@ -270,6 +270,40 @@ def shared_launch_graph(kind, side=3):
 
 
 @pytest.mark.parametrize("round_mode", [0, 1], ids=["half_up", "half_even"])
+@pytest.mark.parametrize("kind", ["in_place", "slices", "residual", "unread", "side"])
+def test_layers_that_run_in_front_of_their_place(oracle, kind, round_mode):
+    """The outputs are the oracle's eagerly, as a replay, in a pass module by module, and compared module by module with every
+    tensor that the plan has, with passes of another input in between.  (test_host_runtime.py looks at the launches.)"""
+    announce(f"model shared launch graph {kind} round mode {round_mode}")
+    _, _, model, _ = _mods()
+    spec = shared_launch_graph(kind, 7)
+    batch = 2
+    mdl, want, x = _run_config(spec, batch, 51, round_mode=round_mode)
+
+    def check():
+        for out in spec.outputs:
+            np.testing.assert_array_equal(mdl.get_tensor(out), want[out], err_msg=out)
+            assert want[out].min() < want[out].max()
+
+    check()
+    for replay in (False, True, True):
+        if replay:
+            assert mdl.enable_graph()
+        for values in (np.flip(x, axis=1).copy(), x):
+            mdl.set_input("input", values)
+            mdl.run()
+        check()
+        mdl.set_input("input", x)
+        mdl.profile(1)
+        check()
+    mdl.close()
+    tensors = {name: ref for name, ref in want.items() if name in spec.outputs or name.startswith(("first", "early", "in_between"))}
+    tested = model.Model(model.Graph.from_spec(spec, {"input": x[:1]}, {n: r[:1] for n, r in tensors.items()}), 1, round_mode=round_mode)
+    assert tested.test()
+    tested.close()
+
+
+@pytest.mark.parametrize("round_mode", [0, 1], ids=["half_up", "half_even"])
 @pytest.mark.parametrize("rows,k,n,m", [(40, 120, 480, 120), (9, 33, 17, 5), (1, 16, 2100, 64)])
 def test_lut_behind_gemm_and_matmul(oracle, rows, k, n, m, round_mode):
     """A table behind a Gemm or a MatMul by a constant runs in its epilogue, also where its result has another exponent; one

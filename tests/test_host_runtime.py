@@ -348,6 +348,27 @@ def test_two_launch_cases_take_the_tile_of_their_name():
     ''')
 
 
+def test_layers_that_share_a_launch():
+    """What a pass of small graphs launches: the early layer goes out with the first one, and a pass module by module with its own
+    place's neighbours."""
+    host_hip.run('''
+    import test_gpu_model
+    expected = {"in_place": 4, "slices": 4, "residual": 3, "unread": 4}
+    for kind, launched in expected.items():
+        mdl = model.Model(model.Graph.from_spec(test_gpu_model.shared_launch_graph(kind)), 2)
+        hip.host_hip_clear()
+        mdl.run()
+        names = [l["name"] for l in launches()]
+        assert len(names) == launched and sum("narrow_group" in n for n in names) == 1, (kind, names)
+        assert "narrow_group" in names[1], (kind, names)  # behind the trunk
+        hip.host_hip_clear()
+        mdl.profile(1)  # four passes of it
+        names = [l["name"] for l in launches()]
+        assert not any("narrow_group" in n for n in names) and len(names) == 4 * (launched + 1), (kind, names)
+        mdl.close()
+    ''')
+
+
 def test_layers_run_early_only_while_the_arena_stays_small():
     """A layer that runs in front of its place keeps its output until there: up to a sixteenth of the arena and 4 MB."""
     host_hip.run('''
