@@ -50,7 +50,7 @@ struct SplitArgs {
     int parts;       // workgroups per tile
     int in_bytes;
     int units, pitch; // 16-byte pieces of a patch pixel, LDS bytes from pixel to pixel (twice an odd number of pieces)
-    FastDiv fd_units, fd_pw, fd_tiles_x, fd_tiles_yx, fd_parts;
+    FastDiv fd_units, fd_tiles_x, fd_tiles_yx, fd_parts;
 };
 
 // Tile of PT x TW output pixels; patch of ((PT - 1) S + 3) x ((TW - 1) S + 3) block-input pixels.
@@ -448,7 +448,6 @@ hipError_t launch_mbconv_s8_expand_dw(const MbconvParams &p, int8_t *mid, int cu
         pitch_units++;
     a.pitch = 16 * pitch_units;
     a.fd_units = make_fastdiv((unsigned)a.units);
-    a.fd_pw = make_fastdiv((unsigned)((plan.tw - 1) * p.stride_h + 3));
     a.fd_tiles_x = make_fastdiv((unsigned)a.tiles_x);
     a.fd_tiles_yx = make_fastdiv((unsigned)(a.tiles_x * a.tiles_y));
     a.fd_parts = make_fastdiv((unsigned)a.parts);
