@@ -715,9 +715,10 @@ WalkCut walk_cut(const WalkArgs &a, const WalkLaunch &l, int per_cu)
 // units and more, 5 under 5 x 5, take more than 256 registers: one wavefront per SIMD, 1.4 and 2.3 us more whatever the layer's size
 // (52 layers of 5 to 82 us; 3 x 3 counts 1, for the unit kernel's line lies as far below its time at 128 channels).  Four filter tiles
 // beside a residual operand on 3 and 4 units, the builds that take all registers: of two chunks of 32 filters and one of 64 the smaller
-// expected time is more often the one that is too small.  With 4 % and 0.6 us in favour of the two, 1 of 3500 layers of 33 to 64 channels
-// is slower by more than 5 % than without the build, at 0.967 of that time in the mean (111 layers and 0.963 without the margin:
-// 40 x 40 x 64 -> 128, batch 58, 14.2 us as two chunks and 17.4 as one).
+// expected time is more often the one that is too small, and two chunks read a layer's input twice and write halves of its pixels.  With
+// 1.2 us in favour of the two and a tenth of the memory's time in favour of the one, 5 of 4000 layers of 33 to 64 channels, slices of wider
+// tensors among them, are slower by more than 5 % than without the builds, at 0.963 of that time in the mean (119 layers and 0.961 by the
+// expected time alone: 40 x 40 x 64 -> 128, batch 58, 14.2 us as two chunks and 17.4 as one).
 template <int KH, int S, int CU, int NT, bool RES, bool RAW>
 float walk_us(const WalkArgs &a, const WalkLaunch &l)
 {
@@ -743,7 +744,7 @@ float walk_us(const WalkArgs &a, const WalkLaunch &l)
     if (S == 2 && ((KH == 3 && CU >= 6) || (KH == 5 && CU >= 5)))
         us += KH == 3 ? 1.f : 2.3f;
     if (RES && kRegs > 244)
-        us = 1.04f * us + 0.6f;
+        us += 1.2f - 0.1f * memory;
     return KH == 3 && S == 1 && CU >= 15 ? 1.5f * us : us;
 }
 

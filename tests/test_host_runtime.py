@@ -403,11 +403,15 @@ def test_residual_walks_take_four_filter_tiles_only_where_they_gain():
                              ((244, 41, 37, 64), 64, 4), ((130, 37, 45, 52), 128, 4), ((256, 39, 43, 44), 64, 4)]:
         pads = {45: (0, 1, 0, 1), 43: (2, 0, 2, 1)}.get(shape[2], (1, 1, 1, 1))
         desc = m.capi.make_desc(shape, oc, (3, 3), pads=pads, n_shift=oc)
-        hip.host_hip_clear()
-        rc = m.lib().espdl_hip_conv2d_add(ctypes.byref(desc), 1 << 36, 1 << 37, None, 1 << 38, None, 1 << 39, 1 << 40, None)
-        names = [l["name"] for l in launches()]
-        assert rc == 0 and len(names) == 1, (shape, names)
-        assert "conv2d_s8_walk_kernelILi3ELi1ELi%dELi%dELb1E" % ((shape[3] + 15) // 16, tiles) in names[0], (shape, names)
+        for pitches in ((0, 0, 0), (192, 192, 192)):  # slices of wider tensors
+            if pitches[0] and shape[1:] != (80, 80, 64):
+                continue
+            desc.in_pitch, desc.out_pitch, desc.res_pitch = pitches
+            hip.host_hip_clear()
+            rc = m.lib().espdl_hip_conv2d_add(ctypes.byref(desc), 1 << 36, 1 << 37, None, 1 << 38, None, 1 << 39, 1 << 40, None)
+            names = [l["name"] for l in launches()]
+            assert rc == 0 and len(names) == 1, (shape, names)
+            assert "conv2d_s8_walk_kernelILi3ELi1ELi%dELi%dELb1E" % ((shape[3] + 15) // 16, tiles) in names[0], (shape, pitches, names)
     ''')
 
 
