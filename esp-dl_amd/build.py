@@ -2,7 +2,7 @@
 
   python esp-dl_amd/build.py            # libespdl_hip.so (kernels + C ABI)
 
-The GPU box runs the prebuilt .so files that travel with the tree; nothing is compiled there.
+The machine with the GPU runs the prebuilt .so files that travel with the tree; nothing is compiled there.
 """
 import concurrent.futures
 import os

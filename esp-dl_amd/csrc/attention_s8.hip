@@ -26,8 +26,8 @@
 //      neighbouring channels of one position.
 // Not bound by memory or the matrix pipe; two workgroups fit on a compute unit.  Of 9.6 us with 400 positions and one image (two heads
 // of 32 + 32 + 64 channels) the scores take 4.2, in which one wavefront's additions and its next scores follow each other seven
-// times (without additions 3.1, without lookups either 2.5), the probabilities 1.1, v and its product 1.2; 64 heads 13.5, the operators
-// one by one 117 us.  With v a chunk of 64 and a barrier at a time, the epilogue's form chosen at run time and divisions out of line
+// times (without additions 3.1, without lookups either 2.5), the probabilities 1.1, v and its product 1.2; 64 heads 13.5 (launch to
+// launch one image takes 10.4, eight 11.2, 64 heads 14.9, 15.3 on inputs that change), the operators one by one 117 us.  With v a chunk of 64 and a barrier at a time, the epilogue's form chosen at run time and divisions out of line
 // one image took 10.7 us, eight 11.3 (10.6 now), 64 heads 14.3.  Tried: a wavefront that owns 16 queries and all keys, sums passed from
 // row to row by v_permlane swaps, k and v in LDS, no barriers (9.5 us for one image, 15 for 64 heads: four times the additions); three
 // chunks of k on their way (14.0); four wavefronts that each owned 16 queries and re-read their scores from LDS (18.3), a ninth

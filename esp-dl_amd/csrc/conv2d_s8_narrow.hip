@@ -14,9 +14,8 @@
 // For reductions of under four steps (not SPLIT) the wavefronts take neighbouring pixel tiles instead.
 // Lane (col, quad) holds unit 4 step + quad of pixel col (operand B) and of filter row col (operand A); filter rows
 // are permuted (row i of tile t is filter 4 NT (i / 4) + 4 t + i % 4) so that a lane's results are 4 NT neighbours.
-// Measured against the kernels such layers took before, as nodes of a graph: 56 x 56 x 64 -> 64, 3 x 3, one image 6.0 ->
-// 4.1 us; 13 x 13 x 256 -> 64, 3 x 3 15.5 -> 5.0 us; 13 x 13 x 512 -> 256, 1 x 1 5.6 -> 3.3 us; 1 x 4096 -> 256 6.8 -> 4.7 us;
-// 17 x 27 x 74 -> 11, 3 x 3 at stride 2 31.2 -> 3.8 us.
+// Measured against the kernels such layers took before, as nodes of a graph: 13 x 13 x 256 -> 64, 3 x 3 15.5 -> 5.0 us;
+// 13 x 13 x 512 -> 256, 1 x 1 5.6 -> 3.3 us; 1 x 4096 -> 256 6.8 -> 4.7 us; 17 x 27 x 74 -> 11, 3 x 3 at stride 2 31.2 -> 3.8 us.
 // In a chain of launches 1.2 us pass between a kernel's end and the next one's start; the rest is the instructions of ONE
 // wavefront, four cycles each and more, in front of its loads and behind them.  So a lane finds its units by additions (a
 // division takes six quarter-rate multiplications), layers of one tap have builds of their own, the epilogue's operands are
@@ -413,7 +412,9 @@ static NarrowPlan narrow_plan(const ConvGeom &g, int cu_count)
 }
 
 // Expected time (see dense_s8_route in espdl_hip_api.hip): launch, the steps of one wavefront, all steps in flight.  Fitted to 2840
-// random layers on operands that change from launch to launch: 5 to 9 % off either way, 7 to 15 where channels are no whole units.
+// random layers on operands that change from launch to launch: 5 to 9 % off either way, 7 to 15 where channels are no whole units (over
+// 5500 others, no multiple of 4: 6 to 9 % too small in the mean, 12 to 18 off around that, and up to 1.7 times too small where the
+// launch takes several times the tiled GEMM's time; lines of their own for odd channels choose no better).
 float conv2d_s8_narrow_us(const ConvGeom &g, const void *in, const void *filter, int cu_count)
 {
     const NarrowPlan p = narrow_plan(g, cu_count);

@@ -9,7 +9,7 @@
 // 1.9 TB/s; so a step's bytes pass through LDS and leave as whole aligned 16-byte pieces of memory, cut out of the bytes
 // of this step and the last 16 of the step before, and only the two ends of a row's walk are written by the byte.
 //
-// 20480 pixels x 120 -> 6625 (136 MB written, 26 us at the copy rate): 43 us inside the recognizer, where the kernel that keeps
+// 20480 pixels x 120 -> 6625 (136 MB written, 26 us at the copy rate): 44 us inside the recognizer, where the kernel that keeps
 // filters in LDS took 71 us.  A step is what bounds it: 330 vector and 32 matrix instructions of each of two wavefronts of a SIMD
 // and a barrier, 2.3 us for 32 KB per compute unit.  A workgroup may have several walks, over other pixels under the same filters, so
 // that the filters' constants are brought in once (two walks 42.4 us, one each 46.6; where some shift is below 8 46.1 and 49.9).

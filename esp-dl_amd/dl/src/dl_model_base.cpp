@@ -1277,8 +1277,8 @@ esp_err_t Model::build(int batch)
             vars[vars[i].alias_of].last = std::max(vars[vars[i].alias_of].last, vars[i].last);
     // 1c. convolutions that share a launch.  A small one takes along later ones of its kind whose inputs are there by then: the
     // heads of a detector, level by level, where one launch after the other costs 1.2 us between them and a wavefront's latency each
-    // (416 x 416, one frame: 56 launches and 193 us, 46 and 167; 640 x 640, two frames 272 and 256; 512 x 512, twelve, whose layers
-    // mostly fill the device and have kind 0: 379 both ways).  Results, the plan and its order stay as they are: a module that
+    // (416 x 416, one frame: 55 launches and 176 us as a graph, 45 and 150; 640 x 640, two frames 265 and 252; 512 x 512, twelve, whose
+    // layers all fill the device and have kind 0: 380 either way).  Results, the plan and its order stay as they are: a module that
     // runs early has its output placed then and its inputs kept until its own place, so that a pass module by module (test,
     // get_module_info, a stage) finds the same tensors.
     std::vector<std::vector<int>> with(plan_size); // the later modules that run with this one

@@ -1,5 +1,5 @@
 """Copies the small `.espdl` DATA files that the reference's own tests and examples hold, each with
-embedded test inputs and expected outputs, into tests/golden/espdl/ so that the GPU box (which has no
+embedded test inputs and expected outputs, into tests/golden/espdl/ so that the machine with the GPU (which has no
 copy of the reference) can load them.  They are model containers (weights + known-answer vectors), not
 source code.  Run in the development container:  python tests/golden/copy_espdl_fixtures.py
 
