@@ -459,8 +459,10 @@ __global__ __launch_bounds__(kThreads) void conv2d_s16_gemm_kernel(const S16Args
     }
 }
 
+// (The arguments by value: by reference the compiler fetches some of them behind the loop's branches, 50 instructions more; 5 x 5 over 160
+// channels and 228 pixels -> 16 6.0 -> 6.5 us, 900 layers 0.9 % longer.)
 template <int NT, bool ALIGNED, bool X8>
-__device__ __forceinline__ void narrow16_tile(const S16Args &a, int bx, int by)
+__device__ __forceinline__ void narrow16_tile(const S16Args a, int bx, int by)
 {
     constexpr int G = 2; // steps per batch of loads
     constexpr int kSums = X8 ? 2 : 3;
