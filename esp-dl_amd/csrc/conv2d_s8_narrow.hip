@@ -430,8 +430,10 @@ float conv2d_s8_narrow_us(const ConvGeom &g, const void *in, const void *filter,
     if (((g.in_c | g.in_pitch) & 3) == 0) // units of whole dwords
         return p.split ? 2.7f + 0.18f * steps + waves * (0.25f + nt * (0.06f + 0.082f * steps))
                        : 2.95f + 0.05f * steps + waves * (0.55f * nt + 0.1f * steps);
-    return p.split ? 2.42f + 0.34f * steps + waves * (0.18f + steps * (0.085f + 0.206f * nt))
-                   : 2.78f + 0.23f * steps + waves * (0.39f * nt + steps * (0.123f + 0.165f * nt));
+    if (p.split)
+        return 2.42f + 0.34f * steps + waves * (0.18f + steps * (0.085f + 0.206f * nt));
+    // (under 16 channels neighbouring pixels' units are bytes of the same lines: 0.65 to 0.85 of what more channels take, 450 layers)
+    return 2.78f + 0.23f * steps + (g.in_c < 16 ? 0.65f : 1.f) * waves * (0.39f * nt + steps * (0.123f + 0.165f * nt));
 }
 
 hipError_t launch_conv2d_s8_narrow(const ConvGeom &g, const int8_t *in, const int8_t *filter, const int32_t *bias,

@@ -160,12 +160,13 @@ DenseRoute dense_s8_route(const espdl::ConvGeom &g, const void *in, const void *
         return units && narrow < 5.2f ? DENSE_NARROW : DENSE_STEM;
     const bool flat = g.k_h == 1 && g.k_w == 1 && g.stride_h == 1 && g.stride_w == 1 && g.pad_top == 0 &&
         g.pad_left == 0 && g.out_h == g.in_h && g.out_w == g.in_w;
-    // The GEMMs' lines leave out part of what channels that are no multiple of 4 cost them.  Over 5500 random layers of those on both
-    // kernels the better line is slower than the better kernel by 0.57 % in the geometric mean, by 0.52 % with 1.1 under 1 x 1, and by
-    // 1.15 % with 1.15 under any window: there the narrow kernel's line leaves out as much (14 x 14 x 87 -> 444, 5 x 5 at stride 2,
-    // batch 19: 41 us against 20).
+    // The GEMMs' lines leave out part of what channels that are no multiple of 4 cost them, and so does the narrow kernel's under a
+    // window.  Distance of the better line from the better kernel, geometric means over random layers of those on both: 16 channels and
+    // more (5500 layers) 0.57 % by the lines alone, 0.52 % with 1.1 under 1 x 1, 1.15 % with 1.15 under any window (14 x 14 x 87 -> 444,
+    // 5 x 5 at stride 2, batch 19: 41 us against 20); under 16 channels (1600) 0.27 % by the lines, 0.18 % with 1.05.
     const bool uneven = ((g.in_c | g.in_pitch) & 3) != 0;
-    const DenseRoute few = narrow < (uneven && g.k_h * g.k_w == 1 ? 1.1f : 1.f) * gemm ? DENSE_NARROW : DENSE_UNITGEMM;
+    const float favour = !uneven ? 1.f : (g.in_c < 16 ? 1.05f : (g.k_h * g.k_w == 1 ? 1.1f : 1.f));
+    const DenseRoute few = narrow < favour * gemm ? DENSE_NARROW : DENSE_UNITGEMM;
     if (flat) {
         if (espdl::conv2d_s8_pwgemm_supports(g, in, filter, cus))
             return units && narrow < (uneven ? 1.15f : 0.97f) * gemm ? DENSE_NARROW : DENSE_PWGEMM;
@@ -223,7 +224,13 @@ DenseRoute dense_s8_kernel(const espdl::ConvGeom &g, const void *in, const void 
     const DenseRoute route = dense_s8_route(g, in, filter, residual, units, narrow, gemm, tile_steps, cus);
     if (units && dense_s8_walks(g, route, espdl::conv2d_s8_walk_us(g, in, filter, residual, out, cus), narrow, gemm))
         return DENSE_WALK;
-    return route == DENSE_STEM && espdl::conv2d_s8_walk_stem_supports(g, in, out, residual) ? DENSE_WALK_STEM : route;
+    if (route != DENSE_STEM)
+        return route;
+    if (espdl::conv2d_s8_walk_stem_supports(g, in, out, residual))
+        return DENSE_WALK_STEM;
+    // (the first-layer kernel's least time grows with the filters: 7 x 47 x 86 x 5 -> 7, 3 x 3, 7.7 us against 4.8 by the narrow one, at
+    // stride 2 6 x 104 x 104 x 4 -> 41 11.3 against 4.8; 19 x 52 x 52 x 2 -> 8 5.7 either way at a line of 6.1)
+    return units && narrow < 6.f ? DENSE_NARROW : DENSE_STEM;
 }
 
 } // namespace

@@ -416,7 +416,7 @@ def test_residual_walks_take_four_filter_tiles_only_where_they_gain():
 
 
 def test_windows_over_channels_that_are_no_multiple_of_four_go_to_the_faster_kernel():
-    """The kernel of a few pixels against the tiled GEMM (their microseconds beside the layer)."""
+    """The kernel of a few pixels against the tiled GEMM and the first-layer kernel (their microseconds beside the layer)."""
     host_hip.run('''
     L = m.lib()
     L.espdl_hip_conv2d_s8_kernel.restype = ctypes.c_char_p
@@ -426,6 +426,11 @@ def test_windows_over_channels_that_are_no_multiple_of_four_go_to_the_faster_ker
                                                    ((4, 40, 40, 94), 64, 5, 1, at, b"unitgemm"),       # 29, 21
                                                    ((10, 26, 26, 33), 64, 3, 1, at, b"unitgemm"),      # 8.9, 6.8
                                                    ((7, 52, 52, 221), 35, 1, 2, at, b"narrow"),        # 6.2, 6.5
+                                                   ((205, 4, 41, 7), 6, 3, 1, None, b"narrow"),        # 5.7, 7.2
+                                                   ((91, 40, 40, 13), 14, 3, 1, None, b"narrow"),      # 12.2, 15.4
+                                                   ((7, 47, 86, 5), 7, 3, 1, None, b"narrow"),         # 4.8, the first-layer kernel 7.7
+                                                   ((6, 104, 104, 4), 41, 3, 2, None, b"narrow"),      # 4.8, 11.3
+                                                   ((19, 52, 52, 2), 8, 3, 1, None, b"stem"),          # 5.7, 5.7
                                                    ((1, 13, 13, 33), 64, 3, 1, None, b"narrow")]:
         desc = m.capi.make_desc(shape, oc, (k, k), (stride, stride), pads=(k // 2,) * 4, n_shift=oc)
         name = L.espdl_hip_conv2d_s8_kernel(ctypes.byref(desc), at, at, None, residual, at)
